@@ -85,6 +85,24 @@ def test_linear_generic(dtype, m, n, k):
         torch.testing.assert_close(one, out[:1], rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 8, 9, 16, 17, 33, 515])
+@pytest.mark.parametrize("n,k", [(1, 4), (7, 2052), (33, 60), (130, 64), (700, 516), (4100, 576)])
+def test_linear_f32_forms(m, n, k):
+    """32-bit products of few and of many rows at the edges of their tiles (8 rows or columns, 16, 32), of a stage of 64 k and of
+    the stages that are in flight; rows of x and of the result with a stride of their own."""
+    ops = _ops()
+    torch.manual_seed(m + n + k)
+    wide = torch.randn(m, k + 12, device=DEV)
+    x, w, out = wide[:, 4 : 4 + k], torch.randn(n, k, device=DEV), torch.full((m, n + 3), 7.0, device=DEV)
+    ref = x.cpu().double() @ w.cpu().double().T
+    bound = 2.0 ** -20 * (x.cpu().double().abs() @ w.cpu().double().abs().T)  # as above
+    ops.linear_generic(x, w, out=out[:, :n])
+    assert ((out[:, :n].cpu().double() - ref).abs() <= bound).all()
+    assert bool((out[:, n:] == 7).all())
+    rows = 1 if m <= 8 else 9
+    assert torch.equal(ops.linear_generic(x[:rows], w), out[:rows, :n])
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("n,k", [(48, 64), (130, 200), (1000, 4096), (257, 1064), (16, 8), (4096, 14336)])
 def test_linear_tiled(m, n, k):

@@ -696,6 +696,49 @@ def attention_generic(q, out, k_cache, v_cache, token_req, positions, block_tabl
     return out
 
 
+F32_ATTENTION_MAX_RANGES = 64
+
+
+def f32_attention_takes(dtype, head_dim: int, v_dim: int, page_size: int) -> bool:
+    return dtype == torch.float32 and v_dim == head_dim and head_dim % 16 == 0 and 16 <= head_dim <= 128 and page_size >= 4 and page_size & (page_size - 1) == 0
+
+
+def attention_f32(q, out, k_cache, v_cache, tiles, block_table, heads: int, kv_heads: int, head_dim: int, scale: float, rows: bool,
+                  splits: int = 1, range_keys: int = 0, workspace: tuple[torch.Tensor, torch.Tensor] | None = None, window: int = 0, chunk: int = 0,
+                  cap: float = 0.0, sink: bool = False, slope_exp: float = 0.0, sink_logits: torch.Tensor | None = None) -> torch.Tensor:
+    """32-bit attention on the matrix cores for the tiles described in ``tiles`` (as for ``attention_mfma``): single tokens
+    (``rows``) whose keys go in ``splits`` ranges of ``range_keys`` (a multiple of 16; the ranges start at multiples of it, and the first is
+    the one with the first key that the token sees, so ``splits`` of them have to reach the last key), or up to 32 tokens of a
+    request whose keys are cut into ``splits`` equal ranges.  ``splits`` > 1 needs ``workspace`` = (part_o, part_ml) float32 tensors.  The other
+    arguments: as for ``attention_generic``."""
+    page = _check_attn(q, out, k_cache, v_cache, heads, kv_heads, head_dim)
+    if sink_logits is not None and _f32(sink_logits, "sink_logits").numel() != heads:
+        raise KernelRefused(f"attention_f32: sink_logits holds one float32 value for each of the {heads} heads")
+    if not f32_attention_takes(q.dtype, head_dim, head_dim, page) or q.stride(0) % 4 or any(t.data_ptr() % 16 for t in (q, out, k_cache, v_cache)):
+        raise KernelRefused(f"attention_f32 takes float32 in 16-byte pieces, head sizes that are multiples of 16 up to 128 and page sizes that are "
+                            f"powers of two from 4; got {q.dtype}, head size {head_dim}, page {page}, rows {q.stride(0)} apart")
+    _gpu(tiles, block_table)
+    _i32(tiles, "tiles"), _i32(block_table, "block_table")
+    if tiles.dim() != 2 or tiles.shape[1] != TILE_INTS:
+        raise KernelRefused(f"attention_f32: tiles must be int32 [n_tiles, {TILE_INTS}]")
+    if rows and (range_keys < 16 or range_keys % 16):
+        raise KernelRefused("attention_f32: a range of a single token's keys is a multiple of 16 keys")
+    po = pm = None
+    if splits > 1:
+        if workspace is None or splits > F32_ATTENTION_MAX_RANGES:
+            raise KernelRefused(f"attention_f32: 2 to {F32_ATTENTION_MAX_RANGES} key ranges are taken, with a workspace")
+        po, pm = workspace
+        cols = tiles.shape[0] * (1 if rows else 32) * heads
+        if po.dtype != torch.float32 or pm.dtype != torch.float32 or po.numel() < cols * splits * head_dim or pm.numel() < cols * splits * 2 or po.data_ptr() % 16:
+            raise KernelRefused("attention_f32: workspace too small")
+    _check(build.core().ns_attn_f32(_ptr(out), _ptr(po), _ptr(pm), _ptr(q), c_int(q.stride(0)), _ptr(k_cache), _ptr(v_cache), _ptr(tiles),
+                                    _ptr(block_table), c_int(block_table.stride(0)), c_int(tiles.shape[0]), c_int(heads), c_int(kv_heads),
+                                    c_int(head_dim), c_int(page), c_int(1 if rows else 0), c_int(splits), c_int(range_keys // 16 if rows else 1),
+                                    c_float(scale), c_int(window), c_int(chunk), c_float(cap), c_int(1 if sink else 0), _ptr(sink_logits),
+                                    c_float(slope_exp), _stream()), "attention_f32")
+    return out
+
+
 def unit_kv_write(qkv: torch.Tensor, positions, token_req, block_table, k_cache, v_cache, heads: int, kv_heads: int, head_dim: int,
                   v_dim: int, eps: float | None, own_kv: bool = True) -> None:
     """For attention without rotation.  A row of ``qkv`` is q [heads, head_dim] and, with ``own_kv``, k [kv_heads, head_dim]

@@ -3,8 +3,8 @@ model/attention.py).
 
 Per step: one product for q, k and v together (the three checkpoint matrices are stacked at load
 time), rotation of q and k fused with the write of k and v into the pages, attention of every token
-over its request's pages, output projection.  float32 runs the plain attention kernel; bfloat16 runs
-the matrix-core kernel: prompt portions as tiles of 16 tokens of one head, decode rows as tiles of
+over its request's pages, output projection.  float32 runs the 32-bit matrix-core kernels (or, for other sizes, the plain
+attention kernel); bfloat16 runs the matrix-core kernel: prompt portions as tiles of 16 tokens of one head, decode rows as tiles of
 all heads of a group with the keys cut into ranges that are joined afterwards.
 """
 
@@ -25,6 +25,8 @@ PORTION_RANGE_BLOCKS = 16  # the fewest 32-key blocks that a range of a prompt p
 PORTION_SINGLE_SET_BLOCKS = 128  # 32-key blocks of the longest row from which a workgroup is one set of waves instead of two
 DECODE_WAVES_PER_UNIT = 4  # decode rows' keys are cut into ranges until about this many waves per compute unit are at work
 LONG_ROW_KEYS = 8192  # rows that may reach this many keys get up to 32 ranges instead of 16
+F32_RANGE_KEYS = 128  # keys of a range of a single token's row in 32-bit: two tiles of 16 for each wave of its workgroup
+F32_PORTION_RANGE_BLOCKS = 4  # the fewest 64-key blocks that a range of a portion's keys is worth a workgroup of its own in 32-bit
 QKV_JOIN_MAX_RANGES = 4  # 17 to 128 rows: the kernel that joins the ranges of the q/k/v product, rotates and writes the cache reads
 #                          every range, so more of them cost it what they gain the product
 
@@ -172,6 +174,36 @@ def wide_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_di
             ws = (take((cols * splits * v_dim,), torch.float32), take((cols * splits * 2,), torch.float32))
         ops.attention_wide(q, out, cache.k, cache.v, decode_tiles, table, heads, kv_heads, head_dim, v_dim, scale, window=window, hp=hp,
                            splits=splits, workspace=ws, qt=1, slope_exp=slope_exp, sink_logits=sink_logits)
+    return out
+
+
+def f32_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_dim: int, scale: float, window: int = 0, chunk: int = 0,
+                  **options) -> torch.Tensor:
+    """32-bit attention of the batch's portion tiles and single tokens on the matrix cores (sizes: ``ops.f32_attention_takes``).
+    A single token's keys go in ranges of ``F32_RANGE_KEYS`` from key 0 whatever else is in the batch, so its result does not
+    depend on it; a portion's are cut only where its tiles leave the GPU idle."""
+    chunk_tiles, decode_tiles = TilePlan.views(ctx)
+    units = ops.compute_units(ctx.token_ids.device)
+    span = min(n for n in (window, chunk, 1 << 30) if n)
+    group, take = heads // kv_heads, ctx.arena.take
+
+    def launch(tiles, rows: bool, splits: int, range_keys: int = 0) -> None:
+        cols = tiles.shape[0] * (1 if rows else TilePlan.TOKENS) * heads
+        ws = (take((cols * splits * head_dim,), torch.float32), take((cols * splits * 2,), torch.float32)) if splits > 1 else None
+        ops.attention_f32(q, out, cache.k, cache.v, tiles, table, heads, kv_heads, head_dim, scale, rows=rows, splits=splits, range_keys=range_keys,
+                          workspace=ws, window=window, chunk=chunk, **options)
+
+    if chunk_tiles.shape[0]:
+        wgs = chunk_tiles.shape[0] * kv_heads * -(-group // 2)
+        blocks = -(-min(ctx.max_chunk_kv, span + TilePlan.TOKENS) // 64)
+        launch(chunk_tiles, False, max(1, min(16, 2 * units // wgs, blocks // F32_PORTION_RANGE_BLOCKS)))
+    if decode_tiles.shape[0]:
+        # (a span of keys may begin anywhere in its first range)
+        longest, edge = (ctx.max_kv_len, 0) if ctx.max_kv_len <= span else (span, 1)
+        range_keys = F32_RANGE_KEYS
+        while -(-longest // range_keys) + edge > ops.F32_ATTENTION_MAX_RANGES:
+            range_keys *= 2
+        launch(decode_tiles, True, -(-longest // range_keys) + edge, range_keys)
     return out
 
 
@@ -362,6 +394,8 @@ class Attention:
                 ops.attention_mfma(qkv, att, cache.k, cache.v, plan.tiles, table, s.heads, s.kv_heads, s.head_dim,
                                    s.softmax_scale, window=s.window, hp=plan.hp, splits=plan.splits, workspace=plan.workspace,
                                    qt=plan.qt, coop=plan.coop)
+        elif ops.f32_attention_takes(x.dtype, s.head_dim, s.head_dim, page):
+            f32_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.softmax_scale, window=s.window)
         else:
             ops.attention_generic(qkv, att, cache.k, cache.v, ctx.token_req, ctx.positions, table, s.heads, s.kv_heads,
                                   s.head_dim, s.softmax_scale, window=s.window)
@@ -427,6 +461,9 @@ class Attention:
             # bfloat16, values of another size than the keys or a bias by distance: the two-size matrix-core kernel
             wide_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.v_dim, s.softmax_scale, window=s.window,
                            slope_exp=s.slope_exp, sink_logits=self.sink_logits)
+        elif ops.f32_attention_takes(x.dtype, s.head_dim, s.v_dim, cache.k.shape[2]) and qkv.stride(0) % 4 == 0:
+            f32_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.softmax_scale, window=s.window, chunk=s.chunk,
+                          cap=s.score_cap, sink=s.sink, slope_exp=s.slope_exp, sink_logits=self.sink_logits)
         else:
             ops.attention_generic(qkv, att, cache.k, cache.v, ctx.token_req, ctx.positions, table, s.heads, s.kv_heads, s.head_dim,
                                   s.softmax_scale, window=s.window, v_dim=s.v_dim, chunk=s.chunk, cap=s.score_cap, sink=s.sink,

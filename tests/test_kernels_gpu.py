@@ -1001,3 +1001,96 @@ def test_products_at_the_largest_feed_forward_sizes(n, k):
     piece = torch.empty((n, 7168 if k > 8192 else 2048), dtype=torch.bfloat16, device=DEV)
     width = piece.shape[1]
     assert torch.equal(ops.untile(wt, piece, width, 2 * width), w[:, width : 2 * width])
+
+
+F32_OPTIONS = {
+    "plain": {},
+    "window": dict(window=70),
+    "chunk": dict(chunk=96),
+    "cap_sink": dict(cap=2.0, sink=True),
+    "slope_learned_sink": dict(slope_exp=8.0, sink_logits=True),
+}
+
+
+@pytest.mark.parametrize("option", list(F32_OPTIONS))
+@pytest.mark.parametrize("case", ["append6", "mixed", "long", "beyond64pages"])
+@pytest.mark.parametrize("heads,kvh,hd,page", [(8, 2, 128, 16), (6, 1, 48, 4), (3, 3, 16, 8), (32, 8, 64, 16), (40, 2, 32, 64)])
+def test_attention_f32(case, option, heads, kvh, hd, page):
+    """The 32-bit matrix-core kernels against the plain kernel: tiles and single tokens, whole and cut into ranges, every option, and
+    pages that a window has let go.  Both sum 32-bit products in orders of their own: a few units in the last place of a row's scale."""
+    ops = _ops()
+    starts, lens = CASES[case]
+    torch.manual_seed(11)
+    total = [s + l for s, l in zip(starts, lens)]
+    pages = sum(-(-t // page) for t in total) + 3
+    table = scattered_tables(total, page, pages, seed=4)
+    opt = dict(F32_OPTIONS[option])
+    if opt.get("window"):
+        for b, s in enumerate(starts):
+            table[b, : max(0, s - opt["window"] + 1) // page] = -1
+    k, v = make_cache(pages, page, kvh, hd, torch.float32)
+    k.normal_(), v.normal_()
+    if opt.get("sink_logits"):
+        opt["sink_logits"] = torch.randn(heads, device=DEV)
+    n = sum(lens)
+    wide = torch.randn(n, heads * hd + 8, device=DEV)
+    q = wide[:, : heads * hd]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    positions, token_req = i32([s + i for s, l in zip(starts, lens) for i in range(l)]), i32([b for b, l in enumerate(lens) for _ in range(l)])
+    scale = 1 / math.sqrt(hd)
+    want = torch.empty(n, heads * hd, device=DEV)
+    ops.attention_generic(q, want, k, v, token_req, positions, table.to(DEV), heads, kvh, hd, scale, **opt)
+    first = [sum(lens[:b]) for b in range(len(lens))]
+    ct = [(b, t, first[b], l, total[b], 0, 0, 0) for b, l in enumerate(lens) if l > 1 for t in range(0, l, 32)] + [(0, 0, 0, 0, 0, 0, 0, 0)]
+    dt = [(b, 0, first[b], 1, total[b], 0, 0, 0) for b, l in enumerate(lens) if l == 1] + [(0, 0, 0, 0, 0, 0, 0, 0)]
+    longest = max(total)
+    span = opt.get("window") or opt.get("chunk") or longest
+    outs = []
+    for splits, range_keys in ((1, -(-longest // 16) * 16), (3, 128), (16, 48)):
+        out = torch.full((n, heads * hd), 7.0, device=DEV)
+        for tiles, rows in ((ct, False), (dt, True)):
+            s = -(-min(span, longest) // range_keys) + 1 if rows else splits
+            cols = len(tiles) * (1 if rows else 32) * heads
+            ws = tuple(torch.full((cols * s * m,), float("nan"), device=DEV) for m in (hd, 2)) if s > 1 else None
+            if s <= ops.F32_ATTENTION_MAX_RANGES:
+                ops.attention_f32(q, out, k, v, i32(tiles), table.to(DEV), heads, kvh, hd, scale, rows=rows, splits=s, range_keys=range_keys if rows else 0,
+                                  workspace=ws, **opt)
+        outs.append(out)
+        # 1,300 weights of a row, each off by a few 2^-24 of its score's scale, and their sum
+        torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-5)
+    rows = torch.tensor([i for b, l in enumerate(lens) if l > 1 for i in range(first[b], first[b] + l)], device=DEV)
+    # a row by itself in its tile, beside what its tile holds here: the same sums
+    b = next(b for b, l in enumerate(lens) if l > 1)
+    last = [(b, lens[b] - 1, first[b], lens[b], total[b], 0, 0, 0)]
+    alone = torch.full((n, heads * hd), 7.0, device=DEV)
+    ops.attention_f32(q, alone, k, v, i32(last), table.to(DEV), heads, kvh, hd, scale, rows=False, **opt)
+    assert torch.equal(alone[first[b] + lens[b] - 1], outs[0][first[b] + lens[b] - 1])
+    assert rows.numel() and bool((alone[: first[b] + lens[b] - 1] == 7).all())
+
+
+def test_attention_f32_keeps_infinities_to_the_rows_that_see_them():
+    """A value that is infinite or no number belongs to the tokens at its position and behind; the others' results are what they
+    would be without it.  The same for keys, and for what earlier owners left in a page behind the last key."""
+    ops = _ops()
+    torch.manual_seed(5)
+    heads, kvh, hd, page, n = 4, 2, 32, 16, 50
+    table = torch.arange(4, dtype=torch.int32, device=DEV).view(1, 4)
+    q = torch.randn(n, heads * hd, device=DEV)
+    tiles = torch.tensor([(0, t, 0, n, n, 0, 0, 0) for t in range(0, n, 32)], dtype=torch.int32, device=DEV)
+    k, v = (torch.randn(4, kvh, page, hd, device=DEV), torch.randn(4, kvh, hd, page, device=DEV))
+    k[3, :, 2:], v[3, :, :, 2:] = float("nan"), float("nan")  # positions 50 to 63 are nobody's
+    run = lambda: ops.attention_f32(q, torch.zeros(n, heads * hd, device=DEV), k, v, tiles, table, heads, kvh, hd, 0.2, rows=False)
+    clean = run()
+    assert torch.isfinite(clean).all()
+    for bad in (float("inf"), float("nan")):
+        for what, cache in (("v", v[2, :, 3, 5]), ("k", k[2, :, 5, 3])):  # position 37
+            kept = cache.clone()
+            cache.fill_(bad)
+            out = run()
+            cache.copy_(kept)
+            torch.testing.assert_close(out[:37], clean[:37], rtol=1e-5, atol=1e-6)
+            if what == "v" or bad != bad:  # (an infinite key may make a score of minus infinity: a weight of zero)
+                assert not torch.isfinite(out[37:]).all(dim=1).any()
+    one = torch.tensor([(0, 0, 0, 1, n, 0, 0, 0)], dtype=torch.int32, device=DEV)
+    out = ops.attention_f32(q[:1], torch.zeros(1, heads * hd, device=DEV), k, v, one, table, heads, kvh, hd, 0.2, rows=True, range_keys=64)
+    assert torch.isfinite(out).all()

@@ -348,10 +348,14 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 
 // ------------------------------------------------------------------------------------------------ many rows
 // Steps of many rows (bfloat16): the (token, chosen expert) pairs are sorted by expert on the device, and every expert's
-// pairs are cut into tiles of 128 rows.  A workgroup takes one tile and 128 output channels and multiplies on the matrix
-// cores (v_mfma_f32_16x16x32_bf16): its four waves own 64 x 64 each, operands come through LDS in pieces of 64 along K,
-// the next piece is fetched into registers while the current one is multiplied.  The host never learns which experts were
-// chosen: the launch has as many tiles as any choice can need (pairs / 128 + experts), and a tile without rows returns.
+// pairs are cut into even tiles of at most 128 rows (16 where the experts see few; ``moe_tile_cap``).  A workgroup takes one tile
+// and 128 output channels and multiplies on the matrix cores (v_mfma_f32_16x16x32_bf16): its four waves own 64 x 64 each
+// (every second block of 16 rows), operands come through LDS in pieces of 64 along K, the next piece is fetched into registers
+// while the current one is multiplied.  The host never learns which experts were chosen: the launch has as many tiles as any
+// choice can need (pairs / 128 + experts), and a tile without rows returns.
+// Bound by the matrices' bytes up to some hundred tokens (300: 104 us of which the 403 MB take 82 at a large copy's rate), by what
+// a compute unit takes in from L2 beyond.  32 experts of 1,024, width 2,048, four a token, sorting included: 1,024 tokens 212 -> 146 us,
+// 2,048 tokens 311 -> 238 us (even tiles, blocks without rows skipped, LDS rows without bank conflicts, the sort's scan).
 //   first:  rows gathered from h by the sorted pairs; gate (if there is one: DUAL) and up matrices in the same pass; act [pairs
 //           sorted][ff] in bfloat16
 //   second: act times the down matrix; out [tokens][top][W] in 32-bit, each row back at its pair and times its weight
@@ -361,41 +365,131 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 #define MG_TM 128
 #define MG_TN 128
 #define MG_KC 64
-#define MG_LD (MG_KC + 8)  // bfloat16 values between two rows of a staged tile (padded: neighbouring rows start in other banks)
+// bfloat16 values between two rows of a staged tile: 32 bytes more than its data, so that the lanes 0-7 and 16-23 that a 16-byte read serves together
+// touch all banks once (with 16 bytes more the eighth row's second piece meets the first row's first)
+#define MG_LD (MG_KC + 16)
 #define MG_RI (MG_TM / 32)  // 16-row blocks of a wave's 64 x 64 (the four waves are 2 x 2)
 #define MG_CJ (MG_TN / 32)
 #define MG_FA (MG_TM / 32)  // pieces of 8 values that a thread fetches of a staged tile of MG_TM rows (256 threads, 8 pieces a row)
 #define MG_FB (MG_TN / 32)
 
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ sel, int pairs, int experts, int* __restrict__ perm,
+// Pairs sorted by expert and every expert's pairs cut into the fewest tiles of at most ``cap`` rows, as even as whole blocks of
+// 16 rows allow (an expert with a few rows more than ``cap`` makes two tiles of about half, not a full one and a sliver).  The counts
+// are taken and the places dealt with LDS atomics by all threads; the experts' places come from a scan over the lanes.
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ sel, int pairs, int experts, int cap, int* __restrict__ perm,
                                                         int* __restrict__ tile_e, int* __restrict__ tile_r0, int* __restrict__ tile_rows,
                                                         int max_tiles) {
-  __shared__ int cnt[MOE_MAX_EXPERTS], off[MOE_MAX_EXPERTS], cur[MOE_MAX_EXPERTS];
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) cnt[e] = 0, cur[e] = 0;
+  __shared__ int cnt[MOE_MAX_EXPERTS], cur[MOE_MAX_EXPERTS], tiles_of[MOE_MAX_EXPERTS], used;
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x)
-    if (sel[p] < experts) atomicAdd(&cnt[sel[p]], 1);  // (pairs of identity experts have no place)
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, tiles = 0;
-    for (int e = 0; e < experts; ++e) {
-      off[e] = at;
-      for (int r = 0; r < cnt[e] && tiles < max_tiles; r += MG_TM, ++tiles)
-        tile_e[tiles] = e, tile_r0[tiles] = at + r, tile_rows[tiles] = min(MG_TM, cnt[e] - r);
-      at += cnt[e];
-    }
-    for (; tiles < max_tiles; ++tiles) tile_e[tiles] = -1, tile_r0[tiles] = 0, tile_rows[tiles] = 0;
+  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
+    const int e = sel[p];
+    if (e < experts) atomicAdd(&cnt[e], 1);  // (pairs of identity experts have no place)
   }
+  __syncthreads();
+  if (threadIdx.x < NS_WAVE) {  // first places and first tiles: a scan over 64 experts at a time
+    int rows_before = 0, tiles_before = 0;
+    for (int e0 = 0; e0 < experts; e0 += NS_WAVE) {
+      const int e = e0 + threadIdx.x, c = e < experts ? cnt[e] : 0, t = (c + cap - 1) / cap;
+      int rows = c, tiles = t;
+#pragma unroll
+      for (int o = 1; o < NS_WAVE; o <<= 1) {
+        const int r = __shfl_up(rows, o, NS_WAVE), u = __shfl_up(tiles, o, NS_WAVE);
+        if ((int)threadIdx.x >= o) rows += r, tiles += u;
+      }
+      if (e < experts) cur[e] = rows_before + rows - c, tiles_of[e] = tiles_before + tiles - t;
+      rows_before += __shfl(rows, NS_WAVE - 1, NS_WAVE), tiles_before += __shfl(tiles, NS_WAVE - 1, NS_WAVE);
+    }
+    if (threadIdx.x == 0) used = tiles_before;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    const int c = cnt[e], t = (c + cap - 1) / cap, blocks = (c + 15) / 16;
+    for (int i = 0, at = 0; i < t; ++i) {
+      const int rows = min(c - at, 16 * (blocks / t + (i < blocks % t ? 1 : 0)));
+      tile_e[tiles_of[e] + i] = e, tile_r0[tiles_of[e] + i] = cur[e] + at, tile_rows[tiles_of[e] + i] = rows;
+      at += rows;
+    }
+  }
+  for (int i = used + threadIdx.x; i < max_tiles; i += blockDim.x) tile_e[i] = -1, tile_r0[i] = 0, tile_rows[i] = 0;
   __syncthreads();
   // (which pair of an expert gets which of its places depends on timing; a pair's result does not depend on its place)
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = sel[p];
-    if (e < experts) perm[off[e] + atomicAdd(&cur[e], 1)] = p;
+    if (e < experts) perm[atomicAdd(&cur[e], 1)] = p;
   }
 }
 
+// Steps of few rows an expert (decoding): the work is reading the chosen experts' matrices once.  A workgroup takes a tile of up to
+// 16 rows and 16 output channels (of gate and up both); its four waves take pieces of 128 along K in turn, weights and rows going straight
+// from memory into the operands of v_mfma_f32_16x16x32_bf16 (a wave's four loads of a matrix are 256 contiguous bytes of 16 rows), the
+// next piece on its way beside the current one's products, and the waves' sums meet in LDS in a fixed order.
+// Bound by the matrices' bytes: 8 tokens, 32 pairs over 32 experts of 1,024 in a width of 2,048, sorting included: 93 -> 58 us (4.0 TB/s
+// of the chosen experts' matrices); the tiled kernel below, 160 workgroups of 128 channels there, left the GPU half idle.
 template <bool FIRST, bool DUAL>
-__global__ __launch_bounds__(256) void moe_group_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
+__global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
+                                                         const bf16_t* __restrict__ B1, const int* __restrict__ perm,
+                                                         const int* __restrict__ tile_e, const int* __restrict__ tile_r0,
+                                                         const int* __restrict__ tile_rows, bf16_t* __restrict__ act_out, float* __restrict__ out,
+                                                         const float* __restrict__ wt, int N, int K, int top, float limit, float alpha, float shift,
+                                                         int act_kind) {
+  constexpr int MATS = DUAL ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) float part[4][MATS][16][20];  // [wave][matrix][row][channel]
+  const int tile = blockIdx.y, e = tile_e[tile];
+  if (e < 0) return;
+  const int r0 = tile_r0[tile], rows = tile_rows[tile], n0 = blockIdx.x * 16;
+  const int tid = threadIdx.x, lane = tid % NS_WAVE, wave = tid / NS_WAVE, r = lane % 16, g = lane / 16;
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const size_t wrow = ((size_t)e * N + min(n0 + r, N - 1)) * K + 8 * g;
+  const int xslot = r0 + min(r, rows - 1);
+  const bf16_t* xrow = A + (size_t)(FIRST ? perm[xslot] / top : xslot) * a_stride + 8 * g;
+  bf16x8 w[2][MATS][4], x[2][4];
+  auto fetch = [&](int buf, int k0) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = k0 + 32 * s;
+      const bool ok = k + 8 * g < K;
+      w[buf][0][s] = ok ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(B0 + wrow + k)) : zero;
+      if (DUAL) w[buf][MATS - 1][s] = ok ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(B1 + wrow + k)) : zero;
+      x[buf][s] = ok ? *reinterpret_cast<const bf16x8*>(xrow + k) : zero;
+    }
+  };
+  f32x4 acc[MATS];
+#pragma unroll
+  for (int i = 0; i < MATS; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < MATS; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[buf][i][s], x[buf][s], acc[i], 0, 0, 0);
+  };
+  // (a piece beyond K is zeros and adds nothing)
+  fetch(0, 128 * wave);
+  for (int k0 = 128 * wave; k0 < K; k0 += 2 * 512) {
+    fetch(1, k0 + 512);
+    multiply(0);
+    fetch(0, k0 + 1024);
+    multiply(1);
+  }
+#pragma unroll
+  for (int i = 0; i < MATS; ++i) *reinterpret_cast<f32x4*>(&part[wave][i][r][4 * g]) = acc[i];
+  __syncthreads();
+  const int row = tid / 16, c = tid % 16, col = n0 + c;
+  if (row >= rows || col >= N) return;
+  float v[MATS];
+#pragma unroll
+  for (int i = 0; i < MATS; ++i) v[i] = (part[0][i][row][c] + part[1][i][row][c]) + (part[2][i][row][c] + part[3][i][row][c]);
+  const int slot = r0 + row;
+  if (DUAL)
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu(round_to<bf16_t>(v[0]), round_to<bf16_t>(v[MATS - 1]), limit, alpha, shift));
+  else if (FIRST)
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of(round_to<bf16_t>(v[0]), act_kind));
+  else
+    out[(size_t)perm[slot] * N + col] = wt[perm[slot]] * v[0];
+}
+
+template <bool FIRST, bool DUAL>
+__global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
                                                         const bf16_t* __restrict__ B1, const int* __restrict__ perm,
                                                         const int* __restrict__ tile_e, const int* __restrict__ tile_r0,
                                                         const int* __restrict__ tile_rows, bf16_t* __restrict__ act_out, float* __restrict__ out,
@@ -458,7 +552,10 @@ __global__ __launch_bounds__(256) void moe_group_kernel(const bf16_t* __restrict
       if (DUAL) acc1[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-  const int a_at = (MG_TM / 2 * wm + r) * MG_LD + 8 * g, b_at = (MG_TN / 2 * wn + r) * MG_LD + 8 * g;
+  // the tile's blocks of 16 rows go to the two waves of a column in turn, so that a tile that is not full keeps both busy; a block
+  // without rows costs no product
+  const int my_blocks = ((rows + 15) / 16 - wm + 1) / 2;
+  const int a_at = (16 * wm + r) * MG_LD + 8 * g, b_at = (MG_TN / 2 * wn + r) * MG_LD + 8 * g;
   fetch(0);
   for (int k0 = 0; k0 < K; k0 += MG_KC) {
     stage();
@@ -468,19 +565,21 @@ __global__ __launch_bounds__(256) void moe_group_kernel(const bf16_t* __restrict
     for (int ks = 0; ks < MG_KC; ks += 32) {
       bf16x8 af[MG_RI], bf0[MG_CJ], bf1[MG_CJ];
 #pragma unroll
-      for (int i = 0; i < MG_RI; ++i) af[i] = *reinterpret_cast<const bf16x8*>(As + a_at + 16 * i * MG_LD + ks);
+      for (int i = 0; i < MG_RI; ++i) af[i] = *reinterpret_cast<const bf16x8*>(As + a_at + 32 * i * MG_LD + ks);  // (blocks without rows too)
 #pragma unroll
       for (int j = 0; j < MG_CJ; ++j) {
         bf0[j] = *reinterpret_cast<const bf16x8*>(Bs + b_at + 16 * j * MG_LD + ks);
         if (DUAL) bf1[j] = *reinterpret_cast<const bf16x8*>(Bs + MG_TN * MG_LD + b_at + 16 * j * MG_LD + ks);
       }
 #pragma unroll
-      for (int i = 0; i < MG_RI; ++i)
+      for (int i = 0; i < MG_RI; ++i) {
+        if (i >= my_blocks) break;
 #pragma unroll
         for (int j = 0; j < MG_CJ; ++j) {
           acc0[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf0[j], acc0[i][j], 0, 0, 0);
           if (DUAL) acc1[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf1[j], acc1[i][j], 0, 0, 0);
         }
+      }
     }
     __syncthreads();
   }
@@ -489,7 +588,7 @@ __global__ __launch_bounds__(256) void moe_group_kernel(const bf16_t* __restrict
   for (int i = 0; i < MG_RI; ++i)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int row = MG_TM / 2 * wm + 16 * i + 4 * g + q;
+      const int row = 16 * (2 * i + wm) + 4 * g + q;
       if (row >= rows) continue;
       const int slot = r0 + row;
       const int pair = FIRST ? 0 : perm[slot];
@@ -508,8 +607,46 @@ __global__ __launch_bounds__(256) void moe_group_kernel(const bf16_t* __restrict
     }
 }
 
+// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees four rows on average, else 128 (the
+// tiled one).  32 experts of 1,024 in a width of 2,048, four a token, sorting included: 8 tokens 58 us streamed and 84 tiled, 24 tokens 92 and 94, 40 tokens
+// 99 and 94 (an expert with more than 16 rows is read twice).
+static int moe_tile_cap(long long pairs, int experts) { return pairs <= 4LL * experts ? 16 : MG_TM; }
+
 // tiles that any choice of experts can need
-extern "C" int ns_moe_group_tiles(int pairs, int experts) { return (pairs + MG_TM - 1) / MG_TM + experts; }
+extern "C" int ns_moe_group_tiles(int pairs, int experts) {
+  const int cap = moe_tile_cap(pairs, experts);
+  return (pairs + cap - 1) / cap + experts;
+}
+
+struct MoeLaunch {
+  const bf16_t *h, *wg, *wu, *wd;
+  bf16_t* act;
+  float* out;
+  const int *perm, *tile_e, *tile_r0, *tile_rows;
+  const float* wt;
+  int h_stride, W, ff, top, tiles, act_kind;
+  float limit, alpha, shift;
+  hipStream_t stream;
+
+  template <bool DUAL>
+  void first(int cap) const {
+    const bf16_t *b0 = DUAL ? wg : wu, *b1 = DUAL ? wu : nullptr;
+    if (cap == 16)
+      moe_stream_kernel<true, DUAL><<<dim3((ff + 15) / 16, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr,
+                                                                                    nullptr, ff, W, top, limit, alpha, shift, act_kind);
+    else
+      moe_group_kernel<true, DUAL><<<dim3((ff + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act,
+                                                                                              nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
+  }
+  void second(int cap) const {
+    if (cap == 16)
+      moe_stream_kernel<false, false><<<dim3((W + 15) / 16, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt,
+                                                                                     W, ff, top, limit, alpha, shift, act_kind);
+    else
+      moe_group_kernel<false, false><<<dim3((W + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr,
+                                                                                              out, wt, W, ff, top, limit, alpha, shift, act_kind);
+  }
+};
 
 // ``ints``: scratch of pairs + 3 * ns_moe_group_tiles(pairs, experts) 32-bit words; ``act``: bfloat16 [pairs][ff]
 extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg, const void* wu, const void* wd, const int* sel, const float* wt,
@@ -526,17 +663,16 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
   int* tile_e = ints + pairs;
   int* tile_r0 = tile_e + tiles;
   int* tile_rows = tile_r0 + tiles;
-  moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, perm, tile_e, tile_r0, tile_rows, tiles);
+  const int cap = moe_tile_cap(pairs, experts);
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
-  dim3 g1((ff + MG_TN - 1) / MG_TN, tiles), g2((W + MG_TN - 1) / MG_TN, tiles);
+  moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
+  const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,
+                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, stream};
   if (wg)
-    moe_group_kernel<true, true><<<g1, 256, 0, stream>>>((const bf16_t*)h, h_stride, (const bf16_t*)wg, (const bf16_t*)wu, perm, tile_e, tile_r0,
-                                                          tile_rows, (bf16_t*)act, nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
+    l.first<true>(cap);
   else
-    moe_group_kernel<true, false><<<g1, 256, 0, stream>>>((const bf16_t*)h, h_stride, (const bf16_t*)wu, nullptr, perm, tile_e, tile_r0, tile_rows,
-                                                           (bf16_t*)act, nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
-  moe_group_kernel<false, false><<<g2, 256, 0, stream>>>((const bf16_t*)act, ff, (const bf16_t*)wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr,
-                                                          out, wt, W, ff, top, limit, alpha, shift, act_kind);
+    l.first<false>(cap);
+  l.second(cap);
   return ns_launch_status();
 }
 

@@ -1094,3 +1094,43 @@ def test_attention_f32_keeps_infinities_to_the_rows_that_see_them():
     one = torch.tensor([(0, 0, 0, 1, n, 0, 0, 0)], dtype=torch.int32, device=DEV)
     out = ops.attention_f32(q[:1], torch.zeros(1, heads * hd, device=DEV), k, v, one, table, heads, kvh, hd, 0.2, rows=True, range_keys=64)
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("routing", ["spread", "one expert", "identity"])
+@pytest.mark.parametrize("n,experts,top,width,ff,gated", [(8, 8, 4, 64, 24, True), (16, 32, 4, 136, 40, False), (33, 32, 4, 72, 136, True), (40, 5, 2, 264, 16, True),
+                                                          (130, 3, 1, 64, 264, False), (517, 70, 3, 128, 72, True)])
+def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
+    """The sorted experts' products, streamed and tiled: tiles of 1 to 16 and to 128 rows, experts with more rows than a tile and with
+    none, pairs without an expert, sizes that end inside a tile and inside a piece of K."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n + experts)
+    rnd = lambda *shape: torch.randn(*shape, generator=g)
+    h = rnd(n, width).bfloat16()
+    gate, up, down = ((rnd(experts, *s) * s[1] ** -0.5).bfloat16() for s in ((ff, width), (ff, width), (width, ff)))
+    sel = torch.stack([torch.randperm(experts + 1, generator=g)[:top] for _ in range(n)]).to(torch.int32)
+    if routing == "one expert":
+        sel[:, 0] = experts - 1
+    if routing != "identity":
+        sel = sel % experts  # (the same expert twice in a token is two pairs)
+    wt = torch.rand(n, top, generator=g)
+    take = lambda shape, dtype: torch.full(shape, 7, dtype=dtype, device=DEV) if dtype == torch.int32 else torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+    dev = lambda t: t.to(DEV) if t is not None else None
+    out = ops.moe_experts(dev(h), dev(gate) if gated else None, dev(up), dev(down), dev(sel), dev(wt), 7.0 if gated else 0.0, 1.702 if gated else 0.0, take,
+                          1.0 if gated else 0.0, *(() if gated else ("relu2",))).cpu()
+    for t in range(n):
+        for k in range(top):
+            e = int(sel[t, k])
+            if e >= experts:
+                continue
+            x = h[t].double()
+            u = (up[e].double() @ x).float().bfloat16().double()
+            if gated:
+                a = (gate[e].double() @ x).float().bfloat16().double().clamp(max=7.0)
+                act = a * torch.sigmoid(1.702 * a) * (u.clamp(-7.0, 7.0) + 1.0)
+            else:
+                act = u.clamp(min=0.0) ** 2
+            act = act.float().bfloat16().double()
+            want = float(wt[t, k]) * (down[e].double() @ act)
+            # an inner channel's sum may round to the next bfloat16 (2^-8 of it at most), and so may the activation made of it
+            bound = float(wt[t, k]) * 2.0 ** -6 * (down[e].double().abs() @ act.abs()) + 1e-5
+            assert ((out[t, k].double() - want).abs() <= bound).all(), (t, k, e)

@@ -767,7 +767,7 @@ def mfma_attention_takes(dtype, head_dim: int, page_size: int) -> bool:
     return dtype == torch.bfloat16 and head_dim % 16 == 0 and 16 <= head_dim <= 256 and page_size >= 4 and page_size & (page_size - 1) == 0
 
 
-TILE_INTS = 8  # ints per attention tile descriptor: request, first token, first row, tokens, keys, 0, 0, 0
+TILE_INTS = 8  # ints per attention tile descriptor (``parts.attention.TilePlan``); the kernels but ``latent_prompt`` read the first six
 
 
 def attention_mfma(q, out, k_cache, v_cache, tiles, block_table, heads: int, kv_heads: int, head_dim: int, scale: float,
@@ -1754,6 +1754,51 @@ def headwise_product(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.T
                                          ctypes.c_long(channel_gate.stride(0) if channel_gate is not None else 0), _ptr(out),
                                          ctypes.c_long(out.stride(0)), c_int(out_head), c_int(n), c_int(H), c_int(N), c_int(K), _stream()),
            "headwise_product")
+    return out
+
+
+def latent_prompt_block(dtype, heads: int, dim: int, rot: int, value: int, latent: int) -> int:
+    """Elements of scratch that a block of 64 keys takes in ``latent_prompt`` for all heads; 0 where it does not take the sizes."""
+    if dtype != torch.bfloat16 or latent % 32:
+        return 0
+    fn = build.core().ns_latent_prompt_block
+    fn.restype = ctypes.c_long
+    return int(fn(c_int(heads), c_int(dim), c_int(rot), c_int(value)))
+
+
+def latent_prompt(q: torch.Tensor, latents: torch.Tensor, uk: torch.Tensor, uv: torch.Tensor, scratch: torch.Tensor, tiles: torch.Tensor, block_table,
+                  inv_freq: torch.Tensor, factor: float, heads: int, dim: int, rot: int, value: int, latent: int, portions: int, blocks: int, scale: float,
+                  out: torch.Tensor, window: int = 0, interleaved: bool = False, gate: torch.Tensor | None = None,
+                  channel_gate: torch.Tensor | None = None, sink_logits: torch.Tensor | None = None) -> torch.Tensor:
+    """Attention of the prompt portions in ``tiles`` (int32 [n_tiles, 8], up to ``portions`` of them) over keys and values that are made
+    from the latents in ``latents`` [pages, 1, page, latent + rot]: k_h = [uk_h c | r], v_h = uv_h c (``uk`` [heads * dim, latent], ``uv``
+    [heads * value, latent]).  q [rows, heads * (dim + rot)] is not rotated yet.  out [rows, heads * value], times the gates as in
+    ``headwise_product``; rows of no portion are left alone.  ``blocks``: blocks of 64 keys, an even number, that no portion exceeds;
+    ``scratch``: portions * blocks * ``latent_prompt_block`` elements."""
+    _gpu(q, latents, uk, uv, scratch, tiles, block_table, out)
+    n, page = q.shape[0], latents.shape[2] if latents.dim() == 4 else 0
+    _i32(tiles, "tiles"), _i32(block_table, "block_table"), _f32(inv_freq, "inv_freq")
+    block = latent_prompt_block(q.dtype, heads, dim, rot, value, latent)
+    if (not block or page < 1 or page & (page - 1) or q.dim() != 2 or q.shape[1] != heads * (dim + rot) or q.stride(1) != 1 or q.stride(0) % 8
+            or any(t.dtype != q.dtype for t in (latents, uk, uv, scratch, out)) or any(not t.is_contiguous() for t in (latents, uk, uv, scratch, out))
+            or latents.shape[1:] != (1, page, latent + rot) or uk.numel() != heads * dim * latent or uv.numel() != heads * value * latent
+            or out.shape != (n, heads * value) or inv_freq.numel() < rot // 2 or tiles.dim() != 2 or tiles.shape[1] != TILE_INTS
+            or any(t.data_ptr() % 16 for t in (q, latents, uk, uv, scratch)) or out.data_ptr() % 8):
+        raise KernelRefused(f"latent_prompt does not take {heads} heads of {dim} + {rot} and {value} channels over latents of {latent} in {q.dtype}")
+    if blocks < 2 or blocks % 2 or not 1 <= portions <= tiles.shape[0] or scratch.numel() < portions * blocks * block:
+        raise KernelRefused("latent_prompt: blocks is an even number, every portion has a tile, and scratch holds portions * blocks blocks")
+    _check_channel_gate(channel_gate, q, n, heads * value, "latent_prompt")
+    for name, t in (("gate", gate), ("sink_logits", sink_logits)):
+        if t is not None and _f32(t, name).numel() != (n * heads if name == "gate" else heads):
+            raise KernelRefused(f"latent_prompt: {name} is float32, one number a head")
+    # few workgroups: 64 tokens each instead of 128
+    cols = 2 if tiles.shape[0] * heads // 4 >= 2 * compute_units(q.device) else 1
+    _check(build.core().ns_latent_prompt(_ptr(out), _ptr(q), c_int(q.stride(0)), _ptr(latents), _ptr(uk), _ptr(uv), _ptr(scratch), _ptr(tiles),
+                                         _ptr(block_table), c_int(block_table.stride(0)), _ptr(inv_freq), _ptr(gate), _ptr(channel_gate),
+                                         c_int(channel_gate.stride(0) if channel_gate is not None else 0), _ptr(sink_logits), c_int(tiles.shape[0]),
+                                         c_int(portions), c_int(blocks), c_int(heads), c_int(dim), c_int(rot), c_int(value), c_int(latent), c_int(page),
+                                         c_int(window), c_float(scale), c_int(cols), c_int(1 if interleaved else 0), c_float(factor), _stream()),
+           "latent_prompt")
     return out
 
 

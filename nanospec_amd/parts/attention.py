@@ -35,9 +35,10 @@ class TilePlan:
     """The batch as the matrix-core attention kernel walks it (a batch plan, see ``engine.context``): the requests that
     bring more than one token cut into tiles of ``TOKENS`` tokens, then the requests that bring exactly one, a tile each.
     A tile is ``ops.TILE_INTS`` ints: request, first token of the tile among the request's tokens of this step, row of the
-    request's first token, tokens of the request in this step, keys after this step, and for one-token tiles the keys that
+    request's first token, tokens of the request in this step, keys after this step, for one-token tiles the keys that
     all of them read in this step over all layers (by which the kernel chooses its loads: what cannot stay cached until
-    the next step is read past the caches).  shape = (portion tiles, one-token tiles); a region of a fixed shape may hold
+    the next step is read past the caches); for portion tiles the number of their portion in the seventh int, and in the eighth,
+    whichever tile it stands in, as the p-th one of them the number of portion p's first tile (-1 behind the last portion).  shape = (portion tiles, one-token tiles); a region of a fixed shape may hold
     more portion tiles than the batch needs: the rest bring no tokens and the kernel skips them."""
 
     key = "attention.tiles"
@@ -57,9 +58,13 @@ class TilePlan:
         tc, td = shape
         lens, indptr, kv, n = facts.lens, facts.indptr, facts.kv, facts.covered
         if tc:
-            rows = [(b, t0, indptr[b], lens[b], kv[b], 0, 0, 0) for b in range(n) if lens[b] != 1 for t0 in range(0, lens[b], self.TOKENS)]
-            rows += [(facts.n_reqs - 1, 0, 0, 0, 0, 0, 0, 0)] * (tc - len(rows))  # tiles without tokens
-            out[: ops.TILE_INTS * tc] = np.asarray(rows, dtype=np.int32).reshape(-1)
+            many = [b for b in range(n) if lens[b] != 1]
+            rows = [(b, t0, indptr[b], lens[b], kv[b], 0, p, -1) for p, b in enumerate(many) for t0 in range(0, lens[b], self.TOKENS)]
+            rows += [(facts.n_reqs - 1, 0, 0, 0, 0, 0, 0, -1)] * (tc - len(rows))  # tiles without tokens
+            tiles = np.asarray(rows, dtype=np.int32)
+            first = np.cumsum([0] + [-(-int(lens[b]) // self.TOKENS) for b in many])[:-1]
+            tiles[: len(many), 7] = first
+            out[: ops.TILE_INTS * tc] = tiles.reshape(-1)
         if td:
             req = np.nonzero(lens[:n] == 1)[0].astype(np.int32)
             d = np.zeros((td, ops.TILE_INTS), dtype=np.int32)
@@ -140,15 +145,16 @@ WIDE_RANGE_KEYS = 64  # the fewest keys that a range of a row's keys is worth a 
 
 
 def wide_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_dim: int, v_dim: int, scale: float, window: int = 0,
-                   slope_exp: float = 0.0, sink_logits=None):
+                   slope_exp: float = 0.0, sink_logits=None, portions: bool = True):
     """Launch ``ops.attention_wide`` (keys and values of two sizes on the matrix cores) over the tile lists of the batch:
     prompt portions as sets of 16 tokens of one head, decode rows with up to 16 heads of a group in one wave's columns and
-    the keys cut into ranges until the launch fills the GPU (an item of that kernel is one wave)."""
+    the keys cut into ranges until the launch fills the GPU (an item of that kernel is one wave).  ``portions`` = False: the
+    single tokens only."""
     units = ops.compute_units(ctx.token_ids.device)
     group = heads // kv_heads
     chunk_tiles, decode_tiles = TilePlan.views(ctx)
     take = ctx.arena.take
-    if chunk_tiles.shape[0]:
+    if chunk_tiles.shape[0] and portions:
         qt = TilePlan.TOKENS // 16
         waves = chunk_tiles.shape[0] * qt * heads
         longest = min(ctx.max_chunk_kv, window + TilePlan.TOKENS) if window else ctx.max_chunk_kv

@@ -22,9 +22,17 @@ import torch
 
 from ..kernels import ops
 from . import registry
-from .attention import TILES, wide_attention
+from .attention import TILES, TilePlan, wide_attention
 from .linear import LinearWeight
 from .needs import PagedNeed
+
+
+# Prompt portions run over keys and values made from the latents (``csrc/latent_prompt.hip``) where they bring this many tokens
+# together, and this many each on average: making a key costs what about seventy tokens save on it (a latent of 512, heads of
+# 64 + 32 and 64 channels; twice as many tokens in a portion that starts a prompt, whose keys half of its tokens see).
+EXPAND_TOKENS, EXPAND_TOKENS_EACH = 128, 64
+EXPAND_KEYS_PER_TOKEN = 16  # keys, at most, that a portion's tokens may find for each of them
+EXPAND_SCRATCH = 1 << 30  # bytes of scratch for them, at most
 
 
 class LatentAttention:
@@ -96,6 +104,9 @@ class LatentAttention:
                         and (s.q_rank > 0 or self.first.n % 8 == 0))
         self._mfma_o = ops.headwise_takes(dtype, E, C, C, E)
         uk, uv = to(n["uk"]), to(n["uv"])
+        # prompt portions read both as the checkpoint has them
+        self._block = ops.latent_prompt_block(dtype, s.heads, D, R, E, C) if self._mfma_q and self._mfma_o else 0
+        self.uk_rows = uk if self._block else None
         self.uk = uk.view(s.heads, D, C).transpose(1, 2).contiguous() if self._mfma_q else uk  # [heads, latent, dim] | [heads * dim, latent]
         self.uv = uv.view(s.heads, E, C) if self._mfma_o else uv.view(s.heads, E, C).transpose(1, 2).contiguous()  # [heads, value, latent] | [heads, latent, value]
         self.wo = LinearWeight(to(n["o"]), keep_plain=plain)
@@ -135,24 +146,57 @@ class LatentAttention:
             ops.latent_prep(proj[:, self.q_cols :], None, self.dkv_norm, pos.inv_freq, self._factor, ctx.positions, ctx.token_req, table, cache.k,
                             cache.v, 0, C, R, 0, s.norm_eps, None, None, interleaved=self._interleaved)
             q = proj[:, : self.q_cols]
-        q_lat = take((n, H * (C + R)), x.dtype)
-        if self._mfma_q:
-            ops.headwise_product(q, D + R, self.uk, q_lat, C + R)
-        ops.latent_q_absorb(q, None if self._mfma_q else self.uk, pos.inv_freq, self._factor, ctx.positions, H, D, R, C, out=q_lat,
-                            interleaved=self._interleaved)
-        o_lat = take((n, H * C), x.dtype)
-        if ops.wide_attention_takes(x.dtype, C + R, C, cache.k.shape[2]):
-            wide_attention(ctx, q_lat, o_lat, cache, table, H, 1, C + R, C, s.softmax_scale, window=s.window, sink_logits=self.sink_logits)
-        else:
-            ops.attention_generic(q_lat, o_lat, cache.k, cache.v, ctx.token_req, ctx.positions, table, H, 1, C + R, s.softmax_scale,
-                                  window=s.window, v_dim=C, sink_logits=self.sink_logits)
         att = take((n, H * E), x.dtype)
         channel_gate = proj[:, self.gate_at : self.gate_at + H * E] if s.out_gate else None
+        count, blocks = self._expands(ctx, n, cache)
+        singles = TilePlan.views(ctx)[1].shape[0]
+        if not count:
+            self._rows(ctx, q, cache, table, gate, channel_gate, att, True)
+        elif singles:
+            # (the single tokens of a captured step are its first rows; elsewhere they may stand anywhere, and what is formed for the
+            # portions' rows on the way is written over)
+            m = singles if ctx.captured else n
+            first = lambda t: t[:m] if t is not None else None
+            self._rows(ctx, q[:m], cache, table, first(gate), first(channel_gate), att[:m], False)
+        if count:
+            scratch = take((count * blocks * self._block,), x.dtype)
+            ops.latent_prompt(q, cache.k, self.uk_rows, self.uv, scratch, TilePlan.views(ctx)[0], table, pos.inv_freq, self._factor, H, D, R, E, C, count,
+                              blocks, s.softmax_scale, att, window=s.window, interleaved=self._interleaved, gate=gate, channel_gate=channel_gate,
+                              sink_logits=self.sink_logits)
+        return self.wo(att, out=out if out is not None else take((n, s.hidden), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)
+
+
+    def _expands(self, ctx, n: int, cache) -> tuple[int, int]:
+        """Whether the step's prompt portions run over keys and values made from the latents: (portions, blocks of 64 keys of the longest, an
+        even number), or (0, 0)."""
+        chunk_tiles, decode_tiles = TilePlan.views(ctx)
+        singles, page, keys = decode_tiles.shape[0], cache.k.shape[2], ctx.max_chunk_kv
+        count = min(ctx.n_reqs - singles, chunk_tiles.shape[0])  # (a captured step counts the request that owns its padding too)
+        tokens, blocks = n - singles, -(-keys // 128) * 2
+        if (not self._block or not count or page & (page - 1) or tokens < EXPAND_TOKENS or (not ctx.captured and tokens < EXPAND_TOKENS_EACH * count)
+                or keys > EXPAND_KEYS_PER_TOKEN * tokens or 2 * count * blocks * self._block > EXPAND_SCRATCH):
+            return 0, 0
+        return count, blocks
+
+    def _rows(self, ctx, q, cache, table, gate, channel_gate, att, portions: bool) -> None:
+        """Single tokens (and ``portions`` too) over the latents themselves: absorbed queries, one wide key/value head."""
+        s, take = self.spec, ctx.arena.take
+        n = q.shape[0]
+        H, D, R, E, C = s.heads, s.head_dim, s.rot_dim, s.value_dim, s.kv_rank
+        positions, token_req, inv_freq = ctx.positions[:n], ctx.token_req[:n], self.position.inv_freq
+        q_lat, o_lat = take((n, H * (C + R)), q.dtype), take((n, H * C), q.dtype)
+        if self._mfma_q:
+            ops.headwise_product(q, D + R, self.uk, q_lat, C + R)
+        ops.latent_q_absorb(q, None if self._mfma_q else self.uk, inv_freq, self._factor, positions, H, D, R, C, out=q_lat, interleaved=self._interleaved)
+        if ops.wide_attention_takes(q.dtype, C + R, C, cache.k.shape[2]):
+            wide_attention(ctx, q_lat, o_lat, cache, table, H, 1, C + R, C, s.softmax_scale, window=s.window, sink_logits=self.sink_logits, portions=portions)
+        else:
+            ops.attention_generic(q_lat, o_lat, cache.k, cache.v, token_req, positions, table, H, 1, C + R, s.softmax_scale, window=s.window, v_dim=C,
+                                  sink_logits=self.sink_logits)
         if self._mfma_o:
             ops.headwise_product(o_lat, C, self.uv, att, E, gate=gate, channel_gate=channel_gate)
         else:
             ops.latent_out(o_lat, self.uv, gate, H, C, E, out=att, channel_gate=channel_gate)
-        return self.wo(att, out=out if out is not None else take((n, s.hidden), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)
 
 
 registry.register("mixer", "latent_attention", LatentAttention)

@@ -1134,3 +1134,89 @@ def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
             # an inner channel's sum may round to the next bfloat16 (2^-8 of it at most), and so may the activation made of it
             bound = float(wt[t, k]) * 2.0 ** -6 * (down[e].double().abs() @ act.abs()) + 1e-5
             assert ((out[t, k].double() - want).abs() <= bound).all(), (t, k, e)
+
+
+@pytest.mark.parametrize("gates", [False, True])
+@pytest.mark.parametrize("starts,lens,window", [([0], [200], 0), ([0, 70, 0], [1, 129, 40], 0), ([300, 0, 1000], [64, 33, 140], 100), ([0, 5], [577, 2], 64)])
+@pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 96, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])
+def test_latent_prompt(heads, dim, rot, value, latent, page, starts, lens, window, gates):
+    """Prompt portions over keys and values made from latents, against the same in 64 bits: tiles that are not full, portions that end
+    inside a block of keys, blocks that a window cuts, pages that it has let go, a single token among the portions, both pairings."""
+    from nanospec_amd.parts.attention import TilePlan
+    from nanospec_amd.engine.context import BatchFacts
+    import numpy as np
+
+    ops = _ops()
+    g = torch.Generator().manual_seed(heads + sum(lens))
+    rnd = lambda *shape: torch.randn(*shape, generator=g).bfloat16()
+    total = [s + l for s, l in zip(starts, lens)]
+    pages = sum(-(-t // page) for t in total) + 3
+    table = scattered_tables(total, page, pages, seed=6)
+    if window:
+        for b, s in enumerate(starts):
+            table[b, : max(0, s - window + 1) // page] = -1
+    n, C = sum(lens), latent
+    cache = torch.full((pages, 1, page, C + rot), float("nan")).bfloat16()
+    lat = [rnd(t, C + rot) for t in total]
+    for b, t in enumerate(total):
+        for p in range(t):
+            if table[b, p // page] >= 0:
+                cache[table[b, p // page], 0, p % page] = lat[b][p]
+    q, uk, uv = rnd(n, heads * (dim + rot)), (rnd(heads * dim, C).float() * C ** -0.5).bfloat16(), (rnd(heads * value, C).float() * C ** -0.5).bfloat16()
+    inv = 10000.0 ** (-torch.arange(0, rot, 2).float() / rot)
+    sink = torch.randn(heads, generator=g) if gates else None
+    gate = torch.rand(n, heads, generator=g) if gates else None
+    zgate = rnd(n, heads * value + 8)[:, : heads * value] if gates else None
+    indptr = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    i32 = lambda x: np.asarray(x, dtype=np.int32)
+    plan = TilePlan()
+    tc, td = plan.shape(lens)
+    region = np.zeros(plan.ints((tc + 1, td)), dtype=np.int32)  # one tile more than the batch needs
+    plan.fill(region, (tc + 1, td), BatchFacts(n, len(lens), i32(lens), i32(starts), indptr, i32(total), len(lens), 1))
+    tiles = torch.from_numpy(region[: 8 * (tc + 1)].reshape(-1, 8)).to(DEV)
+    blocks = -(-max(total) // 128) * 2
+    portions = min(tc + 1, len(lens) + 1)
+    scale, dev = (dim + rot) ** -0.5, lambda t: t.to(DEV) if t is not None else None
+    for interleaved in (False, True):
+        out = torch.full((n, heads * value), 7.0, dtype=torch.bfloat16, device=DEV)
+        scratch = torch.full((portions * blocks * ops.latent_prompt_block(torch.bfloat16, heads, dim, rot, value, C),), float("nan"), dtype=torch.bfloat16, device=DEV)
+        zg = dev(zgate)
+        ops.latent_prompt(dev(q), dev(cache), dev(uk), dev(uv), scratch, tiles, table.to(DEV), dev(inv), 1.0, heads, dim, rot, value, C, portions, blocks, scale, out,
+                          window=window, interleaved=interleaved, gate=dev(gate), channel_gate=zg, sink_logits=dev(sink))
+        out = out.cpu()
+        turn = lambda x, pos: _turned(x, pos, inv.double(), interleaved)
+        for b, (s, l, t) in enumerate(zip(starts, lens, total)):
+            r0 = int(indptr[b])
+            if l == 1:
+                assert bool((out[r0] == 7).all())
+                continue
+            c = lat[b][:, :C].double()
+            k_rot = lat[b][:, C:].double()
+            pos = torch.arange(s, t)
+            seen = (torch.arange(t)[None] <= pos[:, None]) & ((torch.arange(t)[None] > pos[:, None] - window) if window else torch.ones(l, t, dtype=torch.bool))
+            for h in range(heads):
+                qh = q[r0 : r0 + l, h * (dim + rot) : (h + 1) * (dim + rot)].double()
+                kh = torch.cat([(c @ uk[h * dim : (h + 1) * dim].double().T).bfloat16().double(), k_rot], 1)
+                vh = (c @ uv[h * value : (h + 1) * value].double().T).bfloat16().double()
+                qt = torch.cat([qh[:, :dim], turn(qh[:, dim:], pos).bfloat16().double()], 1)
+                sc = (qt @ kh.T * scale).masked_fill(~seen, float("-inf"))
+                if sink is not None:
+                    sc = torch.cat([sc, sink[h].double().expand(l, 1)], 1)
+                pr = torch.softmax(sc, 1)[:, :t]
+                want = pr @ vh
+                mag = pr @ vh.abs()
+                if gates:
+                    f = gate[r0 : r0 + l, h, None].double() * torch.sigmoid(zgate[r0 : r0 + l, h * value : (h + 1) * value].double())
+                    want, mag = want * f, mag * f
+                got = out[r0 : r0 + l, h * value : (h + 1) * value].double()
+                # weights and result rounded to bfloat16 (2^-9 each), keys and values whose sums another order rounds to the other side (2^-8)
+                assert ((got - want).abs() <= 2.0 ** -6 * mag + 2.0 ** -8 * want.abs() + 1e-6).all(), (b, h, interleaved)
+
+
+def _turned(x, pos, inv, interleaved):
+    half = len(inv)
+    ang = (pos[:, None].float() * inv.float()[None]).double()
+    c, s = ang.cos(), ang.sin()
+    a, b = (x[:, 0::2], x[:, 1::2]) if interleaved else (x[:, :half], x[:, half:])
+    u, v = a * c - b * s, b * c + a * s
+    return torch.stack([u, v], -1).flatten(-2) if interleaved else torch.cat([u, v], -1)

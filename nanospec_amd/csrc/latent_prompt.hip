@@ -8,14 +8,15 @@
 //   latent_expand_kernel: k_h(j) = [Uk_h c(j) | r(j)] and v_h(j) = Uv_h c(j) for the keys that a portion sees, from the cache's pages
 //     into scratch laid out as the attention reads it: [portion][block of 64 keys][head]{ keys [64][D + R] | values [E][64] }, a
 //     channel's keys in the order in which the lanes hold weights (within 32 keys, key 16 t + 4 g + i at place 8 g + 4 t + i).  A wave takes 32
-//     keys of a head through both matrices; a fragment of the latents serves both as either operand.  Bound by its reads of the
-//     matrices and latents from L2: 2,048 keys, 32 heads, latent 512: FIGURE_EXPAND.
-//   latent_prompt_kernel: a workgroup is 64 COLS tokens of a head, a wave 16 COLS; a block of 64 keys and values is contiguous in the
+//     keys of a head through both matrices; a fragment of the latents serves both as either operand.  Bound by the matrices' and
+//     latents' way from L2 (each wave reading the matrices itself: 42 us for 2,048 keys, 32 heads, latent 512; through LDS: 20 us).
+//   latent_prompt_kernel: a workgroup is 64 tokens of a head, a wave 16; a block of 64 keys and values is contiguous in the
 //     scratch and goes through LDS, two buffers, the next one on its way in registers.  S^T = K Q^T and O^T = V^T P^T on
 //     v_mfma_f32_16x16x32_bf16, so a token's scores, maximum and sums are its own lanes'.  Queries are rotated as they are read; the
 //     sink's term, the gate per head and the gate per channel are applied to the 32-bit result before it is rounded.  LDS rows are 32
 //     bytes longer than their data (no bank conflicts).  Bound by the matrix and the vector unit in turn (the soft-max of a block takes
-//     about as long as its products).  2,048 tokens, 32 heads of 64 + 32: FIGURE_PROMPT.
+//     about as long as its products) and the longest tile's chain of blocks, hence 64 tokens and not 128.  2,048 tokens, 32 heads of
+//     64 + 32, both kernels: 69 to 80 us (128 tokens: 25 us more); the wide form took 585 us and 127 us around it.
 #include "common.h"
 #include "rope.h"
 
@@ -23,7 +24,8 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 #define LP_KEYS 64
-#define LP_TILE 32  // tokens of a tile of the batch's tile list
+#define LP_TOKENS 64       // tokens of a workgroup: two tiles of the batch's tile list
+#define LX_ROW (64 + 16)   // bfloat16 values between the rows of a matrix's piece in LDS
 
 struct LatentPromptParams {
   const bf16_t* latents;  // K pages [page][token][C + R] of the cache: normed latent, rotated part
@@ -62,8 +64,6 @@ __global__ __launch_bounds__(256) void latent_expand_kernel(LatentPromptParams p
     const int key = min(max(key0 + 32 * wave + 16 * t + r, lo), kv - 1);  // (keys outside are masked where they are read)
     lat[t] = p.latents + (((size_t)table[key >> p.page_shift] << p.page_shift) + (key & mask)) * CR + 8 * g;
   }
-  const bf16_t* wk = p.uk + ((size_t)h * D + r) * p.C + 8 * g;
-  const bf16_t* wv = p.uv + ((size_t)h * E + r) * p.C + 8 * g;
   f32x4 ak[2][JK], av[2][JV];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -72,21 +72,60 @@ __global__ __launch_bounds__(256) void latent_expand_kernel(LatentPromptParams p
 #pragma unroll
     for (int j = 0; j < JV; ++j) av[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-#pragma unroll 2
-  for (int c = 0; c < p.C; c += 32) {
-    bf16x8 x[2], k[JK], v[JV];
+  // the matrices' rows go through LDS in pieces of 64 latent channels, which all four waves read (rows 32 bytes apart from their data:
+  // no bank conflicts), the latents straight into operands; the next piece is on its way beside the current one's products
+  __shared__ __attribute__((aligned(16))) bf16_t ws[2][(D + E) * LX_ROW];
+  constexpr int PER = (D + E) * 8 / 256;
+  bf16x8 rows[PER], x[2][2][2];
+  auto fetch = [&](int c) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) x[t] = *reinterpret_cast<const bf16x8*>(lat[t] + c);
+    for (int i = 0; i < PER; ++i) {
+      const int row = (i * 256 + (int)threadIdx.x) / 8, at = c + threadIdx.x % 8 * 8;
+      rows[i] = *reinterpret_cast<const bf16x8*>((row < D ? p.uk + ((size_t)h * D + row) * p.C : p.uv + ((size_t)h * E + row - D) * p.C) + at);
+    }
+  };
+  auto fetch_latents = [&](int buf, int c) {
 #pragma unroll
-    for (int j = 0; j < JK; ++j) k[j] = *reinterpret_cast<const bf16x8*>(wk + (size_t)16 * j * p.C + c);
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int j = 0; j < JV; ++j) v[j] = *reinterpret_cast<const bf16x8*>(wv + (size_t)16 * j * p.C + c);
+      for (int t = 0; t < 2; ++t) x[buf][s][t] = *reinterpret_cast<const bf16x8*>(lat[t] + c + 32 * s);
+  };
+  auto park = [&](int buf) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int i = 0; i < PER; ++i) *reinterpret_cast<bf16x8*>(&ws[buf][(i * 256 + threadIdx.x) / 8 * LX_ROW + threadIdx.x % 8 * 8]) = rows[i];
+  };
+  auto multiply = [&](int buf) {
 #pragma unroll
-      for (int j = 0; j < JK; ++j) ak[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j], x[t], ak[t][j], 0, 0, 0);  // [channel][key]
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 k[JK], v[JV];
 #pragma unroll
-      for (int j = 0; j < JV; ++j) av[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[t], v[j], av[t][j], 0, 0, 0);  // [key][channel]
+      for (int j = 0; j < JK; ++j) k[j] = *reinterpret_cast<const bf16x8*>(&ws[buf][(16 * j + r) * LX_ROW + 32 * s + 8 * g]);
+#pragma unroll
+      for (int j = 0; j < JV; ++j) v[j] = *reinterpret_cast<const bf16x8*>(&ws[buf][(D + 16 * j + r) * LX_ROW + 32 * s + 8 * g]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int j = 0; j < JK; ++j) ak[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j], x[buf][s][t], ak[t][j], 0, 0, 0);  // [channel][key]
+#pragma unroll
+        for (int j = 0; j < JV; ++j) av[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[buf][s][t], v[j], av[t][j], 0, 0, 0);  // [key][channel]
+      }
+    }
+  };
+  fetch(0);
+  fetch_latents(0, 0);
+  park(0);
+  for (int c = 0; c < p.C; c += 2 * 64) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (c + 64 * u >= p.C) break;
+      __syncthreads();
+      const bool more = c + 64 * (u + 1) < p.C;
+      if (more) {
+        fetch(c + 64 * (u + 1));
+        fetch_latents(u ^ 1, c + 64 * (u + 1));
+      }
+      multiply(u);
+      if (more) park(u ^ 1);
     }
   }
   const int block = (key0 + 32 * wave) / LP_KEYS, in_block = 32 * (wave & 1);
@@ -104,33 +143,30 @@ __global__ __launch_bounds__(256) void latent_expand_kernel(LatentPromptParams p
   }
 }
 
-template <int D, int R, int E, int COLS>
+template <int D, int R, int E>
 __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p) {
-  constexpr int KD = D + R, KS = KD / 32, VT = E / 16, KROW = KD + 16, VROW = LP_KEYS + 16, TOKENS = 64 * COLS;
+  constexpr int KD = D + R, KS = KD / 32, VT = E / 16, KROW = KD + 16, VROW = LP_KEYS + 16;
   constexpr int BLOCK = LP_KEYS * (KD + E), BUF = LP_KEYS * KROW + E * VROW, PER = BLOCK / 8 / 256;
   static_assert(BLOCK % (8 * 256) == 0 && KD % 32 == 0 && R % 32 == 0 && E % 16 == 0, "pieces of 16 bytes, 256 threads");
   __shared__ __attribute__((aligned(16))) bf16_t lds[2 * BUF];
   const int h = blockIdx.x % p.H, tile = p.n_tiles - 1 - (int)blockIdx.x / p.H;  // the tiles behind have the most keys and start first
   const int* info = p.tiles + 8 * tile;
   const int t0 = info[1], n = info[3], kv = info[4];
-  if (t0 >= n || t0 % TOKENS) return;  // (the tiles of 32 tokens in between belong to the workgroup of the one in front)
+  if (t0 >= n || t0 % LP_TOKENS) return;  // (the tiles of 32 tokens in between belong to the workgroup of the one in front)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
-  const int base = kv - n + t0, n_tok = min(TOKENS, n - t0), hi = base + n_tok - 1;
+  const int base = kv - n + t0, n_tok = min(LP_TOKENS, n - t0), hi = base + n_tok - 1;
   auto first_key = [&](int pos) { return p.window > 0 ? max(0, pos - p.window + 1) : 0; };
-  const int w0 = 16 * COLS * wave;  // the wave's first token of the tile
+  const int w0 = 16 * wave;  // the wave's first token of the tile
   const bool works = w0 < n_tok;
-  const int wave_lo = first_key(base + w0), wave_hi = base + min(w0 + 16 * COLS, n_tok) - 1;
+  const int wave_lo = first_key(base + w0), wave_hi = base + min(w0 + 16, n_tok) - 1;
   const int full_lo = first_key(wave_hi), full_hi = base + w0;  // keys that every token of the wave sees
-  int pos[COLS], lo[COLS];
-  size_t row[COLS];
-  bf16x8 q[COLS][KS];
+  const int tok = min(w0 + c, n_tok - 1), pos = base + tok, lo = first_key(pos);
+  const size_t row = (size_t)info[2] + t0 + tok;
+  bf16x8 q[KS];
+  {
+    const bf16_t* qr = p.q + row * p.q_stride + (size_t)h * KD;
 #pragma unroll
-  for (int u = 0; u < COLS; ++u) {
-    const int tok = min(w0 + 16 * u + c, n_tok - 1);
-    pos[u] = base + tok, lo[u] = first_key(pos[u]), row[u] = (size_t)info[2] + t0 + tok;
-    const bf16_t* qr = p.q + row[u] * p.q_stride + (size_t)h * KD;
-#pragma unroll
-    for (int i = 0; i < D / 32; ++i) q[u][i] = *reinterpret_cast<const bf16x8*>(qr + 32 * i + 8 * g);
+    for (int i = 0; i < D / 32; ++i) q[i] = *reinterpret_cast<const bf16x8*>(qr + 32 * i + 8 * g);
     // the rotated part: both channels of a pair are read, this lane's eight kept
 #pragma unroll
     for (int i = 0; i < R / 32; ++i) {
@@ -142,9 +178,9 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
         const bool second = p.form.interleaved ? e & 1 : d0 >= R / 2;
         const float mine = to_f(own[e]), partner = p.form.interleaved ? to_f(own[e ^ 1]) : to_f(far[e]);
         float cs, sn, a, b;
-        rope_cos_sin(p.form, pos[u], p.inv_freq[pair], cs, sn);
+        rope_cos_sin(p.form, pos, p.inv_freq[pair], cs, sn);
         rope_turn(second ? partner : mine, second ? mine : partner, cs, sn, a, b);
-        q[u][D / 32 + i][e] = from_f<bf16_t>(second ? b : a);
+        q[D / 32 + i][e] = from_f<bf16_t>(second ? b : a);
       }
     }
   }
@@ -163,14 +199,10 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
       *reinterpret_cast<bf16x8*>(&lds[buf * BUF + at]) = reg[i];
     }
   };
-  f32x4 o[COLS][VT];
-  float m[COLS], l[COLS];
+  f32x4 o[VT];
+  float m = -INFINITY, l = 0.f;  // l: this lane's keys
 #pragma unroll
-  for (int u = 0; u < COLS; ++u) {
-    m[u] = -INFINITY, l[u] = 0.f;  // l: this lane's keys
-#pragma unroll
-    for (int t = 0; t < VT; ++t) o[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int t = 0; t < VT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   fetch(b0);
   park(0);
   for (int b = b0; b < b1; ++b) {
@@ -180,95 +212,77 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
     if (works && k0 <= wave_hi && k0 + LP_KEYS > wave_lo) {
       const bf16_t* ks = lds + buf * BUF + c * KROW + 8 * g;
       const bf16_t* vs = lds + buf * BUF + LP_KEYS * KROW + c * VROW + 8 * g;
-      f32x4 s[COLS][4];
+      f32x4 s[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         bf16x8 k[KS];
 #pragma unroll
         for (int i = 0; i < KS; ++i) k[i] = *reinterpret_cast<const bf16x8*>(ks + 16 * t * KROW + 32 * i);
+        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < COLS; ++u) {
-          s[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < KS; ++i) s[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[i], q[u][i], s[u][t], 0, 0, 0);
-        }
+        for (int i = 0; i < KS; ++i) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[i], q[i], s[t], 0, 0, 0);
       }
       const bool full = k0 >= full_lo && k0 + LP_KEYS - 1 <= full_hi;
-      bf16x8 w[COLS][2];
+      bf16x8 w[2];
+      float top = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < COLS; ++u) {
-        float top = -INFINITY;
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = k0 + 16 * t + 4 * g + i;
-            if (!full && (key < lo[u] || key > pos[u])) s[u][t][i] = -INFINITY;
-            top = fmaxf(top, s[u][t][i]);
-          }
-        top = fmaxf(top, __shfl_xor(top, 16, 64));
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
-        const float m_new = fmaxf(m[u], top), ref = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f((m[u] - ref) * p.scale_log2), shift = -ref * p.scale_log2;
-        const bool moved = __any(m_new != m[u]);
-        m[u] = m_new;
-        float sum = 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float e = __builtin_amdgcn_exp2f(fmaf(s[u][t][i], p.scale_log2, shift));
-            sum += e;
-            w[u][t / 2][4 * (t % 2) + i] = (bf16_t)e;
-          }
-        if (moved) {
-          l[u] *= alpha;
-#pragma unroll
-          for (int t = 0; t < VT; ++t) o[u][t] *= alpha;
+        for (int i = 0; i < 4; ++i) {
+          const int key = k0 + 16 * t + 4 * g + i;
+          if (!full && (key < lo || key > pos)) s[t][i] = -INFINITY;
+          top = fmaxf(top, s[t][i]);
         }
-        l[u] += sum;
+      top = fmaxf(top, __shfl_xor(top, 16, 64));
+      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      const float m_new = fmaxf(m, top), ref = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f((m - ref) * p.scale_log2), shift = -ref * p.scale_log2;
+      const bool moved = __any(m_new != m);
+      m = m_new;
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[t][i], p.scale_log2, shift));
+          sum += e;
+          w[t / 2][4 * (t % 2) + i] = (bf16_t)e;
+        }
+      if (moved) {
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) o[t] *= alpha;
       }
+      l += sum;
 #pragma unroll
-      for (int t = 0; t < VT; ++t) {
-        bf16x8 v[2];
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) v[i] = *reinterpret_cast<const bf16x8*>(vs + 16 * t * VROW + 32 * i);
-#pragma unroll
-        for (int u = 0; u < COLS; ++u)
-#pragma unroll
-          for (int i = 0; i < 2; ++i) o[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], w[u][i], o[u][t], 0, 0, 0);
-      }
+        for (int i = 0; i < 2; ++i)
+          o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(vs + 16 * t * VROW + 32 * i), w[i], o[t], 0, 0, 0);
     }
     if (b + 1 < b1) park(buf ^ 1);
   }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (w0 + c >= n_tok) return;
+  if (p.sink_logits) l += exp2f(p.sink_logits[h] * 1.4426950408889634f - m * p.scale_log2);
+  const float f = (p.gate ? p.gate[row * p.H + h] : 1.f) / l;
 #pragma unroll
-  for (int u = 0; u < COLS; ++u) {
-    if (w0 + 16 * u + c >= n_tok) continue;
-    float sum = l[u];
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    if (p.sink_logits) sum += exp2f(p.sink_logits[h] * 1.4426950408889634f - m[u] * p.scale_log2);
-    const float f = (p.gate ? p.gate[row[u] * p.H + h] : 1.f) / sum;
+  for (int t = 0; t < VT; ++t) {
+    f32x4 v = o[t] * f;
+    if (p.zgate) {
+      const bf16x4 z = *reinterpret_cast<const bf16x4*>(p.zgate + row * p.z_stride + (size_t)h * E + 16 * t + 4 * g);
 #pragma unroll
-    for (int t = 0; t < VT; ++t) {
-      f32x4 v = o[u][t] * f;
-      if (p.zgate) {
-        const bf16x4 z = *reinterpret_cast<const bf16x4*>(p.zgate + row[u] * p.z_stride + (size_t)h * E + 16 * t + 4 * g);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] /= 1.f + expf(-to_f(z[i]));
-      }
-      *reinterpret_cast<bf16x4*>(p.out + (row[u] * p.H + h) * E + 16 * t + 4 * g) = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      for (int i = 0; i < 4; ++i) v[i] /= 1.f + expf(-to_f(z[i]));
     }
+    *reinterpret_cast<bf16x4*>(p.out + (row * p.H + h) * E + 16 * t + 4 * g) = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
   }
 }
 
 template <int D, int R, int E>
-static void launch_latent_prompt(const LatentPromptParams& p, int portions, int cols, hipStream_t stream) {
+static void launch_latent_prompt(const LatentPromptParams& p, int portions, hipStream_t stream) {
   latent_expand_kernel<D, R, E><<<dim3((p.blocks + 1) / 2, p.H, portions), 256, 0, stream>>>(p);
-  if (cols == 2)
-    latent_prompt_kernel<D, R, E, 2><<<p.n_tiles * p.H, 256, 0, stream>>>(p);
-  else
-    latent_prompt_kernel<D, R, E, 1><<<p.n_tiles * p.H, 256, 0, stream>>>(p);
+  latent_prompt_kernel<D, R, E><<<p.n_tiles * p.H, 256, 0, stream>>>(p);
 }
 
 // Elements of scratch a block of 64 keys takes for all heads; 0: the sizes are not taken.
@@ -277,15 +291,14 @@ extern "C" long ns_latent_prompt_block(int H, int D, int R, int E) {
 }
 
 // ``scratch``: portions * blocks * ns_latent_prompt_block elements; ``blocks`` (even): blocks of 64 keys that the longest portion's keys take at most.
-// ``cols`` (1 or 2): a workgroup takes 64 ``cols`` tokens.
 extern "C" int ns_latent_prompt(void* out, const void* q, int q_stride, const void* latents, const void* uk, const void* uv, void* scratch,
                                 const int* tiles, const int* block_table, int table_stride, const float* inv_freq, const float* gate, const void* zgate,
                                 int z_stride, const float* sink_logits, int n_tiles, int portions, int blocks, int H, int D, int R, int E, int C,
-                                int page_size, int window, float scale, int cols, int interleaved, float factor, hipStream_t stream) {
+                                int page_size, int window, float scale, int interleaved, float factor, hipStream_t stream) {
   if (n_tiles <= 0 || portions <= 0 || portions > 65535 || blocks <= 0 || blocks % 2 || H <= 0 || H > 65535 || C <= 0 || window < 0 || !(scale > 0.f) ||
-      cols < 1 || cols > 2 || (long)n_tiles * H > 0x7fffffffL)
+      (long)n_tiles * H > 0x7fffffffL)
     return NS_ERR_BAD_ARG;
-  if (!ns_latent_prompt_block(H, D, R, E) || C % 32 || page_size < 1 || page_size & (page_size - 1) || q_stride % 8 || (zgate && z_stride % 4) ||
+  if (!ns_latent_prompt_block(H, D, R, E) || C % 64 || page_size < 1 || page_size & (page_size - 1) || q_stride % 8 || (zgate && z_stride % 4) ||
       (((uintptr_t)out | (uintptr_t)zgate) & 7) || (((uintptr_t)q | (uintptr_t)latents | (uintptr_t)uk | (uintptr_t)uv | (uintptr_t)scratch) & 15))
     return NS_ERR_UNSUPPORTED;
   int shift = 0;
@@ -294,8 +307,8 @@ extern "C" int ns_latent_prompt(void* out, const void* q, int q_stride, const vo
                              block_table, inv_freq, gate, (const bf16_t*)zgate, sink_logits, q_stride, z_stride, table_stride, n_tiles, H, C, shift, blocks,
                              window, scale * 1.4426950408889634f, RopeForm{R, interleaved, factor}};
   if (D == 64)
-    launch_latent_prompt<64, 32, 64>(p, portions, cols, stream);
+    launch_latent_prompt<64, 32, 64>(p, portions, stream);
   else
-    launch_latent_prompt<128, 64, 128>(p, portions, cols, stream);
+    launch_latent_prompt<128, 64, 128>(p, portions, stream);
   return ns_launch_status();
 }

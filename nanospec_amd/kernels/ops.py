@@ -1759,7 +1759,7 @@ def headwise_product(x: torch.Tensor, x_head: int, w: torch.Tensor, out: torch.T
 
 def latent_prompt_block(dtype, heads: int, dim: int, rot: int, value: int, latent: int) -> int:
     """Elements of scratch that a block of 64 keys takes in ``latent_prompt`` for all heads; 0 where it does not take the sizes."""
-    if dtype != torch.bfloat16 or latent % 32:
+    if dtype != torch.bfloat16 or latent % 64:
         return 0
     fn = build.core().ns_latent_prompt_block
     fn.restype = ctypes.c_long
@@ -1791,13 +1791,11 @@ def latent_prompt(q: torch.Tensor, latents: torch.Tensor, uk: torch.Tensor, uv: 
     for name, t in (("gate", gate), ("sink_logits", sink_logits)):
         if t is not None and _f32(t, name).numel() != (n * heads if name == "gate" else heads):
             raise KernelRefused(f"latent_prompt: {name} is float32, one number a head")
-    # few workgroups: 64 tokens each instead of 128
-    cols = 2 if tiles.shape[0] * heads // 4 >= 2 * compute_units(q.device) else 1
     _check(build.core().ns_latent_prompt(_ptr(out), _ptr(q), c_int(q.stride(0)), _ptr(latents), _ptr(uk), _ptr(uv), _ptr(scratch), _ptr(tiles),
                                          _ptr(block_table), c_int(block_table.stride(0)), _ptr(inv_freq), _ptr(gate), _ptr(channel_gate),
                                          c_int(channel_gate.stride(0) if channel_gate is not None else 0), _ptr(sink_logits), c_int(tiles.shape[0]),
                                          c_int(portions), c_int(blocks), c_int(heads), c_int(dim), c_int(rot), c_int(value), c_int(latent), c_int(page),
-                                         c_int(window), c_float(scale), c_int(cols), c_int(1 if interleaved else 0), c_float(factor), _stream()),
+                                         c_int(window), c_float(scale), c_int(1 if interleaved else 0), c_float(factor), _stream()),
            "latent_prompt")
     return out
 

@@ -1138,7 +1138,7 @@ def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
 
 @pytest.mark.parametrize("gates", [False, True])
 @pytest.mark.parametrize("starts,lens,window", [([0], [200], 0), ([0, 70, 0], [1, 129, 40], 0), ([300, 0, 1000], [64, 33, 140], 100), ([0, 5], [577, 2], 64)])
-@pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 96, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])
+@pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 192, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])
 def test_latent_prompt(heads, dim, rot, value, latent, page, starts, lens, window, gates):
     """Prompt portions over keys and values made from latents, against the same in 64 bits: tiles that are not full, portions that end
     inside a block of keys, blocks that a window cuts, pages that it has let go, a single token among the portions, both pairings."""

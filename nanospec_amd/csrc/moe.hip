@@ -408,7 +408,7 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 // choice can need (pairs / 128 + experts), and a tile without rows returns.
 // Bound by the matrices' bytes up to some hundred tokens (300: 104 us of which the 403 MB take 82 at a large copy's rate), by what
 // a compute unit takes in from L2 beyond.  32 experts of 1,024, width 2,048, four a token, sorting included: 1,024 tokens 212 -> 146 us,
-// 2,048 tokens 311 -> 238 us (even tiles, blocks without rows skipped, LDS rows without bank conflicts, the sort's scan).
+// 2,048 tokens 311 -> 237 us (even tiles, blocks without rows skipped, LDS rows without bank conflicts, the sort's scan).
 //   first:  rows gathered from h by the sorted pairs; gate (if there is one: DUAL) and up matrices in the same pass; act [pairs
 //           sorted][ff] in bfloat16
 //   second: act times the down matrix; out [tokens][top][W] in 32-bit, each row back at its pair and times its weight
@@ -540,7 +540,11 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
     out[(size_t)perm[slot] * N + col] = wt[perm[slot]] * v[0];
 }
 
-template <bool FIRST, bool DUAL>
+// ONCE: most experts have one tile, so a matrix is read once: past the caches, and starting at a piece of K of its own for every expert and
+// block of channels, because workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (300
+// tokens: 105 -> 96 us with the sort).  Where experts have several tiles the matrices come from L2 the second time (2,048 tokens, 1,536
+// channels: 275 -> 237 us without the non-temporal loads).
+template <bool FIRST, bool DUAL, bool ONCE>
 __global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
                                                         const bf16_t* __restrict__ B1, const int* __restrict__ perm,
                                                         const int* __restrict__ tile_e, const int* __restrict__ tile_r0,
@@ -574,14 +578,15 @@ __global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restr
     brow1[i] = (DUAL && col < N) ? B1 + ((size_t)e * N + col) * K : nullptr;
   }
   bf16x8 pa[MG_FA], pb0[MG_FB], pb1[MG_FB];
+  auto read = [](const bf16_t* w) { return ONCE ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(w)) : *reinterpret_cast<const bf16x8*>(w); };
   auto fetch = [&](int k0) {
     const bool ok = k0 + kp < K;
 #pragma unroll
     for (int i = 0; i < MG_FA; ++i) pa[i] = (ok && arow[i]) ? *reinterpret_cast<const bf16x8*>(arow[i] + k0 + kp) : zero;
 #pragma unroll
     for (int i = 0; i < MG_FB; ++i) {
-      pb0[i] = (ok && brow0[i]) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(brow0[i] + k0 + kp)) : zero;
-      if (DUAL) pb1[i] = (ok && brow1[i]) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(brow1[i] + k0 + kp)) : zero;
+      pb0[i] = (ok && brow0[i]) ? read(brow0[i] + k0 + kp) : zero;
+      if (DUAL) pb1[i] = (ok && brow1[i]) ? read(brow1[i] + k0 + kp) : zero;
     }
   };
   auto stage = [&]() {
@@ -608,11 +613,13 @@ __global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restr
   // without rows costs no product
   const int my_blocks = ((rows + 15) / 16 - wm + 1) / 2;
   const int a_at = (16 * wm + r) * MG_LD + 8 * g, b_at = (MG_TN / 2 * wn + r) * MG_LD + 8 * g;
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += MG_KC) {
+  const int steps = (K + MG_KC - 1) / MG_KC, turn = ONCE ? (blockIdx.x * 5 + e * 3) % steps : 0;
+  auto piece = [&](int i) { return (i + turn >= steps ? i + turn - steps : i + turn) * MG_KC; };
+  fetch(piece(0));
+  for (int i = 0; i < steps; ++i) {
     stage();
     __syncthreads();
-    if (k0 + MG_KC < K) fetch(k0 + MG_KC);
+    if (i + 1 < steps) fetch(piece(i + 1));
 #pragma unroll
     for (int ks = 0; ks < MG_KC; ks += 32) {
       bf16x8 af[MG_RI], bf0[MG_CJ], bf1[MG_CJ];
@@ -678,6 +685,7 @@ struct MoeLaunch {
   const float* wt;
   int h_stride, W, ff, top, tiles, act_kind;
   float limit, alpha, shift;
+  bool once;  // see moe_group_kernel
   hipStream_t stream;
 
   template <bool DUAL>
@@ -687,16 +695,16 @@ struct MoeLaunch {
       moe_stream_kernel<true, DUAL><<<dim3((ff + 15) / 16, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr,
                                                                                     nullptr, ff, W, top, limit, alpha, shift, act_kind);
     else
-      moe_group_kernel<true, DUAL><<<dim3((ff + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act,
-                                                                                              nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
+      (once ? moe_group_kernel<true, DUAL, true> : moe_group_kernel<true, DUAL, false>)<<<dim3((ff + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(
+          h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
   }
   void second(int cap) const {
     if (cap == 16)
       moe_stream_kernel<false, false><<<dim3((W + 15) / 16, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt,
                                                                                      W, ff, top, limit, alpha, shift, act_kind);
     else
-      moe_group_kernel<false, false><<<dim3((W + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr,
-                                                                                              out, wt, W, ff, top, limit, alpha, shift, act_kind);
+      (once ? moe_group_kernel<false, false, true> : moe_group_kernel<false, false, false>)<<<dim3((W + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(
+          act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt, W, ff, top, limit, alpha, shift, act_kind);
   }
 };
 
@@ -719,7 +727,7 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
   moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
   const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,
-                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, stream};
+                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, pairs <= MG_TM * 3LL / 4 * experts, stream};
   if (wg)
     l.first<true>(cap);
   else

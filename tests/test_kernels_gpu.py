@@ -1136,6 +1136,49 @@ def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
             assert ((out[t, k].double() - want).abs() <= bound).all(), (t, k, e)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,rows,width", [(9, 31, 16), (16, 32, 48), (17, 33, 80), (33, 65, 2048), (40, 7, 20)])
+def test_moe_router_of_many_tokens(n, rows, width, dtype):
+    """Logits where a tile of 16 tokens or of 32 rows ends, pieces of K that four waves cannot share evenly, a width of no whole pieces."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n)
+    h, router, bias = (torch.randn(*s, generator=g) for s in ((n, width + 4), (rows, width), (rows,)))
+    h = h.to(dtype)[:, :width]
+    z, sel, wt = torch.full((n, rows), float("nan"), device=DEV), torch.zeros(n, 2, dtype=torch.int32, device=DEV), torch.zeros(n, 2, device=DEV)
+    wide = torch.zeros(n, width + 4, dtype=dtype, device=DEV)
+    wide[:, :width] = h.to(DEV)
+    ops.moe_route(wide[:, :width], router.to(DEV), bias.to(DEV), 2, sel, wt, logits=z)
+    want = h.double() @ router.double().T + bias.double()
+    # a 32-bit sum of `width` products and a bias: at most width + 1 roundings of 2^-24 of the sum of the magnitudes
+    bound = (width + 1) * 2.0 ** -24 * (h.double().abs() @ router.double().abs().T + bias.double().abs())
+    assert ((z.cpu().double() - want).abs() <= bound).all()
+    assert torch.equal(sel.cpu().long(), z.cpu().topk(2).indices)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,top,width", [(1, 1, 4), (3, 4, 1020), (5, 2, 1028), (2, 3, 2050)])
+def test_moe_combine(n, top, width, dtype):
+    """The experts' parts added up: rows that end inside a workgroup's 1,024 columns, the input in a part's place, a gated base or none."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(width)
+    parts, base, gate, h, wt = (torch.randn(*s, generator=g) for s in ((n, top, width), (n, width), (n, 3), (n, width), (n, top)))
+    base, h = base.to(dtype), h.to(dtype)
+    sel = torch.randint(0, 6, (n, top), generator=g, dtype=torch.int32)
+    d = lambda t: t.to(DEV)
+    for with_base, with_gate, identity in ((True, False, False), (True, True, True), (False, False, True)):
+        out = torch.full((n, width), float("nan"), dtype=dtype, device=DEV)
+        ops.moe_combine(d(parts), d(base) if with_base else None, out, d(gate)[:, 1] if with_gate else None, (d(sel), d(wt), d(h), 4) if identity else None)
+        terms = parts.double()
+        if identity:
+            terms = torch.where((sel >= 4)[:, :, None], wt.double()[:, :, None] * h.double()[:, None], terms)
+        if with_base:
+            b = base.double() * (torch.sigmoid(gate[:, 1:2].double()) if with_gate else 1.0)
+            terms = torch.cat([terms, b[:, None]], 1)
+        # a rounding of 2^-24 of the magnitudes for every term and a few for the sigmoid, then one to the output's type
+        bound = terms.abs().sum(1) * ((top + 6) * 2.0 ** -24 + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0))
+        assert ((out.cpu().double() - terms.sum(1)).abs() <= bound).all(), (with_base, with_gate, identity)
+
+
 @pytest.mark.parametrize("gates", [False, True])
 @pytest.mark.parametrize("starts,lens,window", [([0], [200], 0), ([0, 70, 0], [1, 129, 40], 0), ([300, 0, 1000], [64, 33, 140], 100), ([0, 5], [577, 2], 64)])
 @pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 192, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])

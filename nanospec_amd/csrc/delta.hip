@@ -234,13 +234,13 @@ template <bool VEC, int RG, int ROWS>
 __global__ __launch_bounds__(256) void delta_scan_kernel(float* __restrict__ o, const float* __restrict__ qkv,
                                                          const float* __restrict__ g, const float* __restrict__ beta,
                                                          float* __restrict__ state, size_t slot_stride, const int* __restrict__ qo_indptr,
-                                                         const int* __restrict__ state_slots, DeltaShape p) {
+                                                         const int* __restrict__ state_slots, DeltaShape p, int below) {
   __shared__ __attribute__((aligned(16))) float stage[2][ND_STAGE_FLOATS];
   // (the request is the slowest index of the launch: workgroups are dealt to the eight XCDs in turn, and with the request
   // as the fastest index all workgroups of the one long request among eight would land on one XCD)
   const int b = blockIdx.z, h = blockIdx.y;
   const int r0 = qo_indptr[b], r1 = qo_indptr[b + 1];
-  if (r1 <= r0) return;
+  if (r1 <= r0 || r1 - r0 >= below) return;
   const int D = p.D, E = p.E;
   constexpr int PITCH = ROWS + 4;  // floats between two row groups' channels in LDS
   constexpr int DL = RG * PITCH, COLS = 256 / RG;
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(float* __restrict__ o, 
 }
 
 extern "C" int ns_delta_scan(float* o, const float* qkv, int C, const float* g, const float* beta, float* state, size_t slot_stride,
-                             const int* qo_indptr, const int* state_slots, int n_reqs, int H, int G, int D, int E, hipStream_t stream) {
+                             const int* qo_indptr, const int* state_slots, int n_reqs, int H, int G, int D, int E, int below, hipStream_t stream) {
   if (n_reqs <= 0 || H <= 0 || G <= 0 || H % G || D <= 0 || D > ND_ROWS * NS_WAVE || E <= 0 || H > 65535) return NS_ERR_BAD_ARG;
   DeltaShape p;
   p.C = C, p.H = H, p.G = G, p.D = D, p.E = E;
@@ -426,8 +426,8 @@ extern "C" int ns_delta_scan(float* o, const float* qkv, int C, const float* g, 
   if (n_reqs > 65535) return NS_ERR_BAD_ARG;
   const dim3 grid(zb, H, n_reqs);
 #define ND_LAUNCH2(R, W)                                                                                                               \
-  if (p.vec4) delta_scan_kernel<true, R, W><<<grid, 256, 0, stream>>>(o, qkv, g, beta, state, slot_stride, qo_indptr, state_slots, p); \
-  else delta_scan_kernel<false, R, W><<<grid, 256, 0, stream>>>(o, qkv, g, beta, state, slot_stride, qo_indptr, state_slots, p)
+  if (p.vec4) delta_scan_kernel<true, R, W><<<grid, 256, 0, stream>>>(o, qkv, g, beta, state, slot_stride, qo_indptr, state_slots, p, below); \
+  else delta_scan_kernel<false, R, W><<<grid, 256, 0, stream>>>(o, qkv, g, beta, state, slot_stride, qo_indptr, state_slots, p, below)
 #define ND_LAUNCH(R)                    \
   case R:                               \
     if (rows == 8) { ND_LAUNCH2(R, 8); } \
@@ -445,6 +445,363 @@ extern "C" int ns_delta_scan(float* o, const float* qkv, int C, const float* g, 
 #undef ND_LAUNCH2
 #undef ND_LAUNCH
   return ns_launch_status();
+}
+
+// ------------------------------------------------------------------------------------------------
+// The same recurrence for prompt portions, sixteen tokens at a time.  With G_i the product of the decays of the chunk's tokens up to
+// i (by key channel) and S the state before the chunk, the tokens of a chunk are one small triangular system:
+//   A_ij = sum_d k_i k_j prod_{j < t <= i} g_t  (j < i);   P_ij = the same with q_i (j <= i);   T = (1 + diag(beta) A)^-1 diag(beta)
+//   U = T (V - (K G) S);   O = (Q G) S + P U;   S <- G_15 S + (K prod_{t > i} g_t)^T U
+// All products of decays are formed by multiplication, so that they are at most one and a decay of zero is no special case.
+//
+// The token form above is a chain of some 340 ns a token, whatever the GPU could do beside it.  Here what does not depend on the state (A, P, T
+// and the scaled keys and queries) is made for all chunks at once by ``delta_chunk_kernel``, as the matrix instruction's operands in the order
+// of its lanes, and ``delta_pass_kernel`` goes from chunk to chunk: four waves hold 16 columns of S in the layout in which the instruction
+// leaves its result and takes its second operand alike (v_mfma_f32_16x16x4_f32, 32-bit products and sums), so S never leaves the
+// registers; their shares of (K G) S and (Q G) S + P U meet in LDS, one barrier a chunk; a fifth wave adds up and writes the output.
+// Bound by the chain of a chunk (29 matrix instructions of 32 cycles, two of them waiting for LDS).  16 heads of 128 by 128, 2,048 tokens:
+// 672 us token by token, 43 + 114 us so; 512 tokens 174 -> 46 us.  The workgroups of a head lie on one XCD, whose L2 then serves the
+// records to all its columns.  Sums over channels, products of decays and T are formed in 64 bits, which costs 18 us of the 43:
+// relative error (2-norm, against 64 bits throughout) of the output 8.8e-8 token by token and 6.5e-8 so with decays around 0.5,
+// 2.0e-7 and 1.6e-7 with decays around 0.99, of the state 5.1e-8 and 5.1e-8, 1.9e-7 and 1.5e-7.
+// A sum of a product with a zero beside an infinity would carry a token's infinity to the tokens before it; where a chunk's values are
+// not finite its sums leave out what they may not see.
+//
+// A request's chunks have numbers of their own without a plan: its first is floor(first row / 16) + its place in the batch.
+// ------------------------------------------------------------------------------------------------
+#define DC_T 16  // tokens of a chunk
+// Row m of a chunk's matrices is this token: the four rows that a lane holds of a result are what it gives to the four instructions of the next
+// product, and each instruction adds four neighbouring tokens, the oldest first, so that the newest, which no decay has
+// made smaller yet, are added last, as in the token form.
+__device__ __forceinline__ int chunk_token(int m) { return 4 * (m % 4) + m / 4; }
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct DeltaChunks {
+  const float *qkv, *g, *beta;
+  float *o, *state, *scratch;  // scratch: a record for every chunk and head: K G | Q G | K rest (16 D each) | T | P (256 each) | G_15 (D)
+  const int *qo_indptr, *state_slots;
+  size_t slot_stride;
+  int C, H, G, E, n_reqs, from, min_tokens;  // the records begin at chunk `from`
+};
+
+template <int D>
+__device__ __forceinline__ size_t chunk_record(const DeltaChunks& p, int chunk, int h) {
+  return ((size_t)(chunk - p.from) * p.H + h) * (3 * DC_T * D + 2 * DC_T * DC_T + D);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaChunks p) {
+  constexpr int LD = D + 4, CH = D / 16;  // channels of a thread in the sums over channels
+  constexpr int TASKS = (2 * D + 255) / 256;
+  __shared__ __attribute__((aligned(16))) float kqg[3][DC_T][LD];
+  __shared__ double a_s[DC_T][DC_T + 1];
+  __shared__ float p_s[DC_T][DC_T + 1], t_s[DC_T][DC_T + 1], beta_s[DC_T];
+  const int chunk = p.from + blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
+  // the last request whose first chunk is not behind this one
+  int lo = 0, hi = p.n_reqs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (p.qo_indptr[mid] / DC_T + mid <= chunk) lo = mid; else hi = mid - 1;
+  }
+  const int r0 = p.qo_indptr[lo], r1 = p.qo_indptr[lo + 1], row0 = r0 + (chunk - r0 / DC_T - lo) * DC_T;
+  if (row0 >= r1 || r1 - r0 < p.min_tokens) return;
+  const int n = min(DC_T, r1 - row0), kh = h / (p.H / p.G);
+  // tokens beyond the request's last: no key, no query, a decay of one, a write strength of zero
+  for (int e = tid; e < 3 * DC_T * (D / 4); e += 256) {
+    const int which = e / (DC_T * (D / 4)), i = e / (D / 4) % DC_T, d = 4 * (e % (D / 4));
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (which == 2) v = f32x4{1.f, 1.f, 1.f, 1.f};
+    if (i < n) {
+      const size_t r = row0 + i;
+      v = *reinterpret_cast<const f32x4*>(which == 0   ? p.qkv + r * p.C + (size_t)p.G * D + (size_t)kh * D + d
+                                          : which == 1 ? p.qkv + r * p.C + (size_t)kh * D + d
+                                                       : p.g + (r * p.H + h) * D + d);
+    }
+    *reinterpret_cast<f32x4*>(&kqg[which][i][d]) = v;
+  }
+  if (tid < DC_T) beta_s[tid] = tid < n ? p.beta[(size_t)(row0 + tid) * p.H + h] : 0.f;
+  __syncthreads();
+  {  // A and P: a thread has one token j and every 16th piece of four channels
+    const int j = tid / 16, seg = tid % 16;
+    double w[CH], v[2 * DC_T];
+#pragma unroll
+    for (int u = 0; u < CH; u += 4) {
+      const f32x4 k = *reinterpret_cast<const f32x4*>(&kqg[0][j][4 * seg + 16 * u]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w[u + c] = k[c];
+    }
+#pragma unroll
+    for (int i = 0; i < DC_T; ++i) {
+      double ka = 0., qa = 0.;
+#pragma unroll
+      for (int u = 0; u < CH; u += 4) {
+        const f32x4 k = *reinterpret_cast<const f32x4*>(&kqg[0][i][4 * seg + 16 * u]), q = *reinterpret_cast<const f32x4*>(&kqg[1][i][4 * seg + 16 * u]);
+        const f32x4 g = *reinterpret_cast<const f32x4*>(&kqg[2][i][4 * seg + 16 * u]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          w[u + c] = i > j ? w[u + c] * g[c] : w[u + c];
+          ka = fma((double)k[c], w[u + c], ka);
+          qa = fma((double)q[c], w[u + c], qa);
+        }
+      }
+      v[i] = ka, v[DC_T + i] = qa;
+    }
+    // 32 sums over 16 lanes: in four steps every lane gives away half of what it has; lane seg ends up with sums 2 seg and 2 seg + 1
+#pragma unroll
+    for (int o = 8; o; o >>= 1)
+#pragma unroll
+      for (int x = 0; x < 2 * o; ++x) {
+        const bool up = seg & o;
+        const double keep = up ? v[x + 2 * o] : v[x], give = up ? v[x] : v[x + 2 * o];
+        v[x] = keep + __shfl_xor(give, o, NS_WAVE);
+      }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int i = (2 * seg + x) % DC_T;
+      if (seg < 8) a_s[i][j] = i > j ? v[x] : 0.;
+      else p_s[i][j] = i >= j ? (float)v[x] : 0.f;
+    }
+  }
+  // products of decays along the tokens: a thread a channel, forwards for K G and Q G, backwards for the keys' way to the chunk's end
+  float* rec = p.scratch + chunk_record<D>(p, chunk, h);
+  float first[TASKS][DC_T], second[TASKS][DC_T];
+#pragma unroll
+  for (int x = 0; x < TASKS; ++x) {
+    const int task = tid + 256 * x, d = task % D;
+    if (task < D) {
+      double all = 1.;
+#pragma unroll
+      for (int i = 0; i < DC_T; ++i) {
+        all *= kqg[2][i][d];
+        first[x][i] = (float)(kqg[0][i][d] * all), second[x][i] = (float)(kqg[1][i][d] * all);
+      }
+      rec[3 * DC_T * D + 2 * DC_T * DC_T + d] = (float)all;
+    } else if (task < 2 * D) {
+      double rest = 1.;
+#pragma unroll
+      for (int i = DC_T - 1; i >= 0; --i) {
+        first[x][i] = (float)(kqg[0][i][d] * rest);
+        rest *= kqg[2][i][d];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < TASKS; ++x) {
+    const int task = tid + 256 * x, d = task % D;
+    if (task < D) {
+#pragma unroll
+      for (int i = 0; i < DC_T; ++i) kqg[0][i][d] = first[x][i], kqg[1][i][d] = second[x][i];
+    } else if (task < 2 * D) {
+#pragma unroll
+      for (int i = 0; i < DC_T; ++i) kqg[2][i][d] = first[x][i];
+    }
+  }
+  if (tid < DC_T) {  // T, a column a lane
+    double x[DC_T];
+#pragma unroll
+    for (int i = 0; i < DC_T; ++i) {
+      double s = 0.;
+#pragma unroll
+      for (int j = 0; j < i; ++j) s = fma(a_s[i][j], x[j], s);
+      x[i] = i < tid ? 0. : (i == tid ? 1. : -beta_s[i] * s);
+    }
+#pragma unroll
+    for (int i = 0; i < DC_T; ++i) t_s[i][tid] = (float)(x[i] * beta_s[tid]);
+  }
+  __syncthreads();
+  for (int e = tid; e < 3 * DC_T * (D / 4); e += 256) {
+    const int which = e / (DC_T * (D / 4)), at = e % (DC_T * (D / 4)), tile = at / NS_WAVE, r = at % 16, gq = at % NS_WAVE / 16;
+    f32x4 v;
+    if (which < 2) {  // row: token, four channels of the tile
+      v = *reinterpret_cast<const f32x4*>(&kqg[which][chunk_token(r)][16 * tile + 4 * gq]);
+    } else {  // row: channel of the tile, four tokens
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = kqg[2][chunk_token(4 * gq + i)][16 * tile + r];
+    }
+    *reinterpret_cast<f32x4*>(rec + 4 * (size_t)e) = v;
+  }
+  if (tid < 2 * NS_WAVE) {
+    const int r = tid % 16, gq = tid % NS_WAVE / 16;
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (tid < NS_WAVE ? t_s : p_s)[chunk_token(r)][chunk_token(4 * gq + i)];
+    *reinterpret_cast<f32x4*>(rec + 3 * DC_T * D + 4 * tid) = v;
+  }
+}
+
+__device__ __forceinline__ bool not_finite(const f32x4 v) { return !(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY); }
+
+// sum_j m[row][j] x[j] by the lane that holds rows 4 g .. + 3 of column c of x, without the tokens behind the row's
+__device__ __forceinline__ f32x4 lower_product(const float* __restrict__ m, const f32x4 x, int lane) {
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int j = 0; j < DC_T; ++j) {
+    const float pick = (j & 2) ? ((j & 1) ? x[3] : x[2]) : ((j & 1) ? x[1] : x[0]);
+    const float xj = __shfl(pick, j / 4 * 16 + lane % 16, NS_WAVE);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * (lane / 16) + i;
+      const bool seen = chunk_token(j) <= chunk_token(row);
+      r[i] = fmaf(m[(j / 4 * 16 + row) * 4 + j % 4], seen ? xj : 0.f, r[i]);  // (m is finite where a token is not seen: zero)
+    }
+  }
+  return r;
+}
+
+template <int D>
+__global__ __launch_bounds__(5 * NS_WAVE) void delta_pass_kernel(const DeltaChunks p, int to) {
+  constexpr int TILES = D / 64;  // tiles of 16 key channels a wave holds
+  __shared__ f32x4 part[2][2][4][NS_WAVE];
+  const int b = blockIdx.z, h = blockIdx.x, lane = threadIdx.x & 63, c = lane & 15, gq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r0 = p.qo_indptr[b], r1 = p.qo_indptr[b + 1], first = r0 / DC_T + b;
+  if (r1 - r0 < p.min_tokens) return;
+  const int begin = max(first, p.from), end = min(first + (r1 - r0 + DC_T - 1) / DC_T, to);
+  if (begin >= end) return;
+  // the token of a lane's row i of a chunk is 4 i + gq; the last one that the request has
+  auto last_of = [&](int chunk) { return min(DC_T, r1 - r0 - (chunk - first) * DC_T) - 1; };
+  struct Operands {
+    f32x4 k[TILES], q[TILES], rest[TILES], all[TILES], t, v;
+    float p;
+  };
+  auto joined = [&](int which, int buf) {
+    return (part[buf][which][0][lane] + part[buf][which][1][lane]) + (part[buf][which][2][lane] + part[buf][which][3][lane]);
+  };
+  // the operands of the two chunks ahead are on their way while one is worked through; (Q G) S + P U of a chunk is made behind the
+  // barrier, (Q G) S while (K G) S comes back from LDS, and so meets the fifth wave a barrier later
+  auto every = [&](auto&& fetch, auto&& work) {
+    Operands o0, o1, o2;
+    fetch(o0, begin), fetch(o1, begin + 1);
+    int chunk = begin;
+    for (; chunk + 2 < end; chunk += 3) {
+      fetch(o2, chunk + 2);
+      work(o0, chunk);
+      fetch(o0, chunk + 3);
+      work(o1, chunk + 1);
+      fetch(o1, chunk + 4);
+      work(o2, chunk + 2);
+    }
+    if (chunk < end) work(o0, chunk);
+    if (chunk + 1 < end) work(o1, chunk + 1);
+  };
+  if (wave < 4) {
+    float* S = p.state + (size_t)p.state_slots[b] * p.slot_stride + ((size_t)h * D + wave * TILES * 16 + 4 * gq) * p.E + blockIdx.y * 16 + c;
+    const float* v_src = p.qkv + (size_t)2 * p.G * D + (size_t)h * p.E + blockIdx.y * 16;
+    unsigned v_at[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v_at[i] = (4 * i + gq) * p.C + c;
+    f32x4 s[TILES];
+#pragma unroll
+    for (int x = 0; x < TILES; ++x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[x][i] = S[(size_t)(x * 16 + i) * p.E];
+    every(
+        [&](Operands& o, int chunk) {
+          chunk = min(chunk, end - 1);
+          const float* rec = p.scratch + chunk_record<D>(p, chunk, h);
+#pragma unroll
+          for (int x = 0; x < TILES; ++x) {
+            const int tile = wave * TILES + x;
+            o.k[x] = *reinterpret_cast<const f32x4*>(rec + tile * 256 + 4 * lane);
+            o.q[x] = *reinterpret_cast<const f32x4*>(rec + DC_T * D + tile * 256 + 4 * lane);
+            o.rest[x] = *reinterpret_cast<const f32x4*>(rec + 2 * DC_T * D + tile * 256 + 4 * lane);
+            o.all[x] = *reinterpret_cast<const f32x4*>(rec + 3 * DC_T * D + 2 * DC_T * DC_T + tile * 16 + 4 * gq);
+          }
+          o.t = *reinterpret_cast<const f32x4*>(rec + 3 * DC_T * D + 4 * lane);
+          o.p = rec[3 * DC_T * D + DC_T * DC_T + 4 * lane + wave];  // what this wave gives of P U: four tokens
+          const float* from = v_src + (size_t)(r0 + (chunk - first) * DC_T) * p.C;
+          const unsigned last = last_of(chunk) * p.C + c;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o.v[i] = from[min(v_at[i], last)];
+        },
+        [&](const Operands& o, int chunk) {
+          f32x4 ak[TILES], aq[TILES];
+#pragma unroll
+          for (int x = 0; x < TILES; ++x) ak[x] = aq[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < TILES; ++x) ak[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[x][i], s[x][i], ak[x], 0, 0, 0);
+#pragma unroll
+          for (int x = 1; x < TILES; ++x) ak[0] += ak[x];
+          part[chunk & 1][0][wave][lane] = ak[0];
+          __syncthreads();
+          f32x4 w = o.v - joined(0, chunk & 1), u = {0.f, 0.f, 0.f, 0.f};
+          const int last = last_of(chunk);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[i] = 4 * i + gq <= last ? w[i] : 0.f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < TILES; ++x) aq[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[x][i], s[x][i], aq[x], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], w[i], u, 0, 0, 0);
+#pragma unroll
+          for (int x = 1; x < TILES; ++x) aq[0] += aq[x];
+          if (__any(not_finite(w) || not_finite(u))) {
+            const float* t = p.scratch + chunk_record<D>(p, chunk, h) + 3 * DC_T * D;
+            u = lower_product(t, w, lane);
+            if (wave == 0) aq[0] += lower_product(t + DC_T * DC_T, u, lane);
+          } else {
+            aq[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p, wave < 2 ? (wave == 0 ? u[0] : u[1]) : (wave == 2 ? u[2] : u[3]), aq[0], 0, 0, 0);
+          }
+          part[chunk & 1][1][wave][lane] = aq[0];
+#pragma unroll
+          for (int x = 0; x < TILES; ++x) s[x] *= o.all[x];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < TILES; ++x) s[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.rest[x][i], u[i], s[x], 0, 0, 0);
+        });
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < TILES; ++x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[(size_t)(x * 16 + i) * p.E] = s[x][i];
+  } else {
+    float* to_o = p.o + (size_t)h * p.E + blockIdx.y * 16;
+    const int o_stride = p.H * p.E;
+    for (int chunk = begin; chunk <= end; ++chunk) {
+      __syncthreads();
+      if (chunk == begin) continue;
+      const f32x4 out = joined(1, (chunk - 1) & 1);
+      float* row = to_o + (size_t)(r0 + (chunk - 1 - first) * DC_T) * o_stride;
+      const int last = last_of(chunk - 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (4 * i + gq <= last) row[(4 * i + gq) * o_stride + c] = out[i];
+    }
+  }
+}
+
+template <int D>
+static int delta_chunks(DeltaChunks p, int n_tokens, size_t scratch_floats, hipStream_t stream) {
+  const int chunks = n_tokens / DC_T + p.n_reqs;
+  const size_t per = (size_t)p.H * (3 * DC_T * D + 2 * DC_T * DC_T + D);
+  const size_t fit = scratch_floats / per;  // chunks whose records fit; a longer batch goes in several passes, the state in its slots between them
+  if (fit < 1) return NS_ERR_BAD_ARG;
+  for (int from = 0; from < chunks;) {
+    const int left = chunks - from < 65535 ? chunks - from : 65535, now = fit < (size_t)left ? (int)fit : left;
+    p.from = from;
+    delta_chunk_kernel<D><<<dim3(p.H, now), 256, 0, stream>>>(p);
+    delta_pass_kernel<D><<<dim3(p.H, p.E / 16, p.n_reqs), 5 * NS_WAVE, 0, stream>>>(p, from + now);
+    from += now;
+  }
+  return ns_launch_status();
+}
+
+// Requests of at least ``min_tokens`` tokens; the others are ``ns_delta_scan``'s (with ``below`` the same number).
+extern "C" int ns_delta_chunks(float* o, const float* qkv, int C, const float* g, const float* beta, float* state, size_t slot_stride, const int* qo_indptr,
+                               const int* state_slots, int n_tokens, int n_reqs, int H, int G, int D, int E, int min_tokens, float* scratch,
+                               size_t scratch_floats, hipStream_t stream) {
+  if (n_tokens <= 0 || n_reqs <= 0 || n_reqs > 65535 || H <= 0 || H > 65535 || G <= 0 || H % G || E <= 0 || E % 16 || C % 4 || min_tokens < 1 ||
+      (uintptr_t)qkv % 16 || (uintptr_t)g % 16 || (uintptr_t)scratch % 16)
+    return NS_ERR_BAD_ARG;
+  const DeltaChunks p{qkv, g, beta, o, state, scratch, qo_indptr, state_slots, slot_stride, C, H, G, E, n_reqs, 0, min_tokens};
+  if (D == 64) return delta_chunks<64>(p, n_tokens, scratch_floats, stream);
+  if (D == 128) return delta_chunks<128>(p, n_tokens, scratch_floats, stream);
+  return NS_ERR_UNSUPPORTED;
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -1859,6 +1859,13 @@ def activation(x: torch.Tensor, kind: str, out: torch.Tensor | None = None) -> t
 
 MAX_CONV_TAPS = 16
 DELTA_MAX_KEY_DIM = 1024
+# Prompt portions of the delta rule chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
+# the tokens from which on a request is worth the two launches (16 heads of 128: 16 tokens 11 us token by token, 32 tokens 16.5 and 15.5,
+# 64 tokens 26.6 and 18.4) and the scratch in bytes that the chunks' records may take (27 KiB a chunk and head at 128 channels, a
+# prompt of 2,048 tokens of 16 heads in one piece; what does not fit goes in several passes, 8,192 tokens of 32 heads 2,750 -> 970 us).
+DELTA_CHUNK_KEY_DIMS = (64, 128)
+DELTA_CHUNK_MIN = 32
+DELTA_CHUNK_SCRATCH = 64 << 20
 
 
 def _state_args(state: torch.Tensor, what: str):
@@ -1914,10 +1921,11 @@ def delta_prep(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, dt_bias: tor
 
 
 def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, qo_indptr, state_slots, heads: int,
-               kv_heads: int, key_dim: int, value_dim: int, out: torch.Tensor) -> torch.Tensor:
+               kv_heads: int, key_dim: int, value_dim: int, out: torch.Tensor, take=None) -> torch.Tensor:
     """The gated delta rule over every request's tokens of this step, from and into ``state[slot, : heads * key_dim *
     value_dim]`` (S [heads, key_dim, value_dim] per request): S = g_t * S (by key channel); u = beta_t (v_t - S^T k_t);
-    S = S + k_t u^T; o_t = S^T q_t.  ``qkv`` as ``delta_prep`` leaves it; ``out`` float32 [tokens, heads * value_dim]."""
+    S = S + k_t u^T; o_t = S^T q_t.  ``qkv`` as ``delta_prep`` leaves it; ``out`` float32 [tokens, heads * value_dim].
+    ``take(shape, dtype)`` gives scratch: with it, requests of at least DELTA_CHUNK_MIN tokens go chunk by chunk where the sizes allow it."""
     _f32(qkv, "qkv"), _f32(g, "g"), _f32(beta, "beta"), _f32(out, "out")
     _i32(qo_indptr, "qo_indptr"), _i32(state_slots, "state_slots")
     n, reqs = qkv.shape[0], state_slots.numel()
@@ -1927,8 +1935,20 @@ def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: to
             or state.shape[1] < heads * key_dim * value_dim):
         raise KernelRefused("delta_scan: operands do not fit heads, key size and value size")
     sp, stride = _state_args(state, "delta_scan")
+    below = 0x7FFFFFFF
+    # some request has that many tokens only if the others leave them; in a captured step the counts are all that is known
+    if (take is not None and n - reqs + 1 >= DELTA_CHUNK_MIN and key_dim in DELTA_CHUNK_KEY_DIMS and value_dim % 16 == 0 and C % 4 == 0
+            and not (qkv.data_ptr() | g.data_ptr()) % 16):
+        below = DELTA_CHUNK_MIN
+        record = heads * (49 * key_dim + 512)
+        scratch = take((min((n // 16 + reqs) * record, max(record, DELTA_CHUNK_SCRATCH // 4)),), torch.float32)
+        _check(build.core().ns_delta_chunks(_ptr(out), _ptr(qkv), c_int(C), _ptr(g), _ptr(beta), sp, stride, _ptr(qo_indptr), _ptr(state_slots),
+                                            c_int(n), c_int(reqs), c_int(heads), c_int(kv_heads), c_int(key_dim), c_int(value_dim), c_int(below),
+                                            _ptr(scratch), c_size_t(scratch.numel()), _stream()), "delta_chunks")
+        if reqs == 1:
+            return out
     _check(build.core().ns_delta_scan(_ptr(out), _ptr(qkv), c_int(C), _ptr(g), _ptr(beta), sp, stride, _ptr(qo_indptr), _ptr(state_slots),
-                                      c_int(reqs), c_int(heads), c_int(kv_heads), c_int(key_dim), c_int(value_dim), _stream()), "delta_scan")
+                                      c_int(reqs), c_int(heads), c_int(kv_heads), c_int(key_dim), c_int(value_dim), c_int(below), _stream()), "delta_scan")
     return out
 
 

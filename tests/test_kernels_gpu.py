@@ -1179,6 +1179,69 @@ def test_moe_combine(n, top, width, dtype):
         assert ((out.cpu().double() - terms.sum(1)).abs() <= bound).all(), (with_base, with_gate, identity)
 
 
+@pytest.mark.parametrize("scratch", [0, 64 << 20], ids=["piecewise", "whole"])
+@pytest.mark.parametrize("H,G,D,E,lens", [(2, 1, 64, 16, [32]), (2, 2, 128, 48, [33, 1, 0, 47, 31, 100]), (8, 4, 64, 32, [5, 64, 49]), (3, 3, 128, 16, [1, 257])])
+def test_delta_rule_by_chunks(monkeypatch, H, G, D, E, lens, scratch):
+    """Prompt portions sixteen tokens at a time against the recurrence in 64 bits: last chunks of one and of fifteen tokens, requests that
+    are too short for it among them, decays of zero and of one, the records of all chunks at once and of one at a time."""
+    ops = _ops()
+    monkeypatch.setattr(ops, "DELTA_CHUNK_SCRATCH", scratch)
+    gen = torch.Generator().manual_seed(D + len(lens))
+    n, B, C = sum(lens), len(lens), 2 * G * D + H * E
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    q, k, v = unit(rnd(n, G, D)) * D ** -0.5, unit(rnd(n, G, D)), rnd(n, H, E)
+    g, beta, S0 = torch.rand(n, H, D, generator=gen) ** 0.2, torch.rand(n, H, generator=gen), rnd(B + 1, H * D * E) * 0.2
+    g[:, :, 0], g[:, :, 1], g[7::16, :, 2] = 0.0, 1.0, 0.0
+    state = S0.clone().to(DEV)
+    slots = torch.arange(B, 0, -1, dtype=torch.int32)
+    indptr = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
+    qkv = torch.cat([q.flatten(1), k.flatten(1), v.flatten(1)], 1).to(DEV)
+    out = torch.full((n, H * E), float("nan"), device=DEV)
+    take = lambda shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+    ops.delta_scan(qkv, g.flatten(1).to(DEV).contiguous(), beta.to(DEV), state, indptr.to(DEV), slots.to(DEV), H, G, D, E, out=out, take=take)
+    wide = lambda t: t.double().repeat_interleave(H // G, 0)
+    got, after = out.cpu().double().view(n, H, E), state.cpu().double()
+    for b in range(B):
+        S, top = S0[slots[b]].double().view(H, D, E), 1.0
+        for t in range(int(indptr[b]), int(indptr[b + 1])):
+            S = S * g[t].double()[:, :, None]
+            u = beta[t].double()[:, None] * (v[t].double() - (wide(k[t])[:, :, None] * S).sum(1))
+            S = S + wide(k[t])[:, :, None] * u[:, None]
+            top = max(top, float(S.norm(dim=1).max()), float(v[t].norm(dim=1).max()))
+            want = (wide(q[t])[:, :, None] * S).sum(1)
+            # a step rounds sums of D + 16 terms and hands its error on undamped at most: 2^-24 of the largest column a term and a step
+            steps = t - int(indptr[b]) + 1
+            assert ((got[t] - want).abs().max() <= (D + 16 + steps) * 2.0 ** -24 * top * D ** -0.5 * 4), (b, t)
+        torch.testing.assert_close(after[slots[b]], S.flatten(), rtol=0, atol=(D + 16 + lens[b]) * 2.0 ** -24 * top)
+    assert torch.equal(after[0], S0[0].double())
+
+
+def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens():
+    """An infinity or NaN at one token reaches neither the tokens before it nor other requests, as token by token."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(3)
+    D, E, n, C = 64, 16, 80, 2 * 64 + 16
+    qkv, g, beta = torch.randn(n, C, generator=gen) * 0.1, torch.rand(n, D, generator=gen) ** 0.2, torch.rand(n, 1, generator=gen)
+    indptr, slots = torch.tensor([0, 40, 80], dtype=torch.int32, device=DEV), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=DEV)
+
+    def run(x, gg):
+        out = torch.empty(n, E, device=DEV)
+        return ops.delta_scan(x.to(DEV), gg.to(DEV), beta.to(DEV), torch.zeros(2, D * E, device=DEV), indptr, slots, 1, 1, D, E, out=out, take=take).cpu()
+
+    clean = run(qkv, g)
+    assert torch.isfinite(clean).all()
+    for bad in (float("inf"), float("nan")):
+        for column in (3, D + 3, 2 * D + 3):  # of q, k and v
+            x = qkv.clone()
+            x[21, column] = bad
+            out = run(x, g)
+            others = torch.arange(n) != 21 if column < D else (torch.arange(n) < 21) | (torch.arange(n) >= 40)
+            torch.testing.assert_close(out[others], clean[others], rtol=1e-5, atol=1e-6)
+            assert not torch.isfinite(out[21]).all()
+
+
 @pytest.mark.parametrize("gates", [False, True])
 @pytest.mark.parametrize("starts,lens,window", [([0], [200], 0), ([0, 70, 0], [1, 129, 40], 0), ([300, 0, 1000], [64, 33, 140], 100), ([0, 5], [577, 2], 64)])
 @pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 192, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])

@@ -9,7 +9,7 @@
 // parts of the two dot products by lane exchange, and nothing waits at a barrier.  Everything here is 32-bit.
 //
 // A request's slot holds S [H][D][E] and behind it the last K - 1 inputs of the convolution [K - 1][C] (oldest first).
-#include "common.h"
+#include "chunk16.h"
 
 #define ND_MAX_TAPS 16
 #define ND_ROWS 16  // key channels of a column that one thread owns
@@ -466,16 +466,7 @@ extern "C" int ns_delta_scan(float* o, const float* qkv, int C, const float* g, 
 // 2.0e-7 and 1.6e-7 with decays around 0.99, of the state 5.1e-8 and 5.1e-8, 1.9e-7 and 1.5e-7.
 // A sum of a product with a zero beside an infinity would carry a token's infinity to the tokens before it; where a chunk's values are
 // not finite its sums leave out what they may not see.
-//
-// A request's chunks have numbers of their own without a plan: its first is floor(first row / 16) + its place in the batch.
 // ------------------------------------------------------------------------------------------------
-#define DC_T 16  // tokens of a chunk
-// Row m of a chunk's matrices is this token: the four rows that a lane holds of a result are what it gives to the four instructions of the next
-// product, and each instruction adds four neighbouring tokens, the oldest first, so that the newest, which no decay has
-// made smaller yet, are added last, as in the token form.
-__device__ __forceinline__ int chunk_token(int m) { return 4 * (m % 4) + m / 4; }
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 struct DeltaChunks {
   const float *qkv, *g, *beta;
   float *o, *state, *scratch;  // scratch: a record for every chunk and head: K G | Q G | K rest (16 D each) | T | P (256 each) | G_15 (D)
@@ -497,12 +488,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaChunks p) {
   __shared__ double a_s[DC_T][DC_T + 1];
   __shared__ float p_s[DC_T][DC_T + 1], t_s[DC_T][DC_T + 1], beta_s[DC_T];
   const int chunk = p.from + blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
-  // the last request whose first chunk is not behind this one
-  int lo = 0, hi = p.n_reqs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (p.qo_indptr[mid] / DC_T + mid <= chunk) lo = mid; else hi = mid - 1;
-  }
+  const int lo = chunk_request(p.qo_indptr, p.n_reqs, chunk);
   const int r0 = p.qo_indptr[lo], r1 = p.qo_indptr[lo + 1], row0 = r0 + (chunk - r0 / DC_T - lo) * DC_T;
   if (row0 >= r1 || r1 - r0 < p.min_tokens) return;
   const int n = min(DC_T, r1 - row0), kh = h / (p.H / p.G);
@@ -628,25 +614,6 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaChunks p) {
     for (int i = 0; i < 4; ++i) v[i] = (tid < NS_WAVE ? t_s : p_s)[chunk_token(r)][chunk_token(4 * gq + i)];
     *reinterpret_cast<f32x4*>(rec + 3 * DC_T * D + 4 * tid) = v;
   }
-}
-
-__device__ __forceinline__ bool not_finite(const f32x4 v) { return !(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY); }
-
-// sum_j m[row][j] x[j] by the lane that holds rows 4 g .. + 3 of column c of x, without the tokens behind the row's
-__device__ __forceinline__ f32x4 lower_product(const float* __restrict__ m, const f32x4 x, int lane) {
-  f32x4 r = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int j = 0; j < DC_T; ++j) {
-    const float pick = (j & 2) ? ((j & 1) ? x[3] : x[2]) : ((j & 1) ? x[1] : x[0]);
-    const float xj = __shfl(pick, j / 4 * 16 + lane % 16, NS_WAVE);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 4 * (lane / 16) + i;
-      const bool seen = chunk_token(j) <= chunk_token(row);
-      r[i] = fmaf(m[(j / 4 * 16 + row) * 4 + j % 4], seen ? xj : 0.f, r[i]);  // (m is finite where a token is not seen: zero)
-    }
-  }
-  return r;
 }
 
 template <int D>

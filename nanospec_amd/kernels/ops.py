@@ -1195,14 +1195,23 @@ def memory_state_floats(heads: int, key_dim: int, value_dim: int) -> int:
     return heads * value_dim * key_dim + heads * memory_blocks(key_dim, value_dim) * (key_dim + 1)
 
 
+# Prompt portions of the matrix memory chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
+# the tokens from which on a request is worth the three launches (8 heads of 128 by 256: 32 tokens 16 us token by token and 18 so, 64 tokens
+# 27 and 19), and the scratch in bytes that the chunks' records may take (17 KiB a chunk and head at 128 channels; what does not fit goes in several passes).
+MEMORY_CHUNK_KEY_DIMS = (64, 128)
+MEMORY_CHUNK_MIN = 48
+MEMORY_CHUNK_SCRATCH = 64 << 20
+
+
 def memory_scan(proj: torch.Tensor, offsets: tuple[int, int, int, int, int], gate_bias_i: torch.Tensor | None, gate_bias_f: torch.Tensor | None,
                 state: torch.Tensor, qo_indptr, state_slots, heads: int, key_dim: int, value_dim: int, cap: float, q_scale: float,
-                out: torch.Tensor, den: torch.Tensor, den_eps: float = 1e-6) -> torch.Tensor:
+                out: torch.Tensor, den: torch.Tensor, den_eps: float = 1e-6, take=None) -> torch.Tensor:
     """The matrix memory's recurrence over every request's tokens of the step, in order (``csrc/memory.hip``).  A row of
     ``proj`` holds q and k [heads * key_dim], v [heads * value_dim] and the two gate inputs [heads] at the column
     ``offsets`` (q, k, v, input gate, forget gate); ``state`` float32 [slots, >= memory_state_floats].  ``out`` float32
     [tokens, heads * value_dim] receives S^T q and ``den`` float32 [tokens, heads] the denominators max(|n . q|, exp(-m)) +
-    den_eps: the read-out is out / den (``gated_rms`` divides as it reads)."""
+    den_eps: the read-out is out / den (``gated_rms`` divides as it reads).  ``take(shape, dtype)`` gives scratch: with it, requests of at least
+    MEMORY_CHUNK_MIN tokens go chunk by chunk where the sizes allow it."""
     _gpu(proj, state, qo_indptr, state_slots, out, den, gate_bias_i, gate_bias_f)
     _f32(out, "out"), _f32(den, "den"), _i32(qo_indptr, "qo_indptr"), _i32(state_slots, "state_slots")
     n = proj.shape[0]
@@ -1220,10 +1229,22 @@ def memory_scan(proj: torch.Tensor, offsets: tuple[int, int, int, int, int], gat
     reqs = qo_indptr.numel() - 1
     if state_slots.numel() < reqs:
         raise KernelRefused("memory_scan: one state slot per request")
-    _check(build.core().ns_memory_scan(_ptr(proj), c_int(proj.stride(0)), c_int(q_off), c_int(k_off), c_int(v_off), c_int(i_off), c_int(f_off),
-                                       _ptr(gate_bias_i), _ptr(gate_bias_f), _ptr(state), ctypes.c_longlong(state.stride(0)), _ptr(qo_indptr),
-                                       _ptr(state_slots), _ptr(out), _ptr(den), c_int(reqs), c_int(heads), c_int(key_dim), c_int(value_dim), c_float(cap),
-                                       c_float(q_scale), c_float(den_eps), c_int(_dtype_code(proj)), _stream()), "memory_scan")
+    row = (_ptr(proj), c_int(proj.stride(0)), c_int(q_off), c_int(k_off), c_int(v_off), c_int(i_off), c_int(f_off), _ptr(gate_bias_i), _ptr(gate_bias_f),
+           _ptr(state), ctypes.c_longlong(state.stride(0)), _ptr(qo_indptr), _ptr(state_slots), _ptr(out), _ptr(den))
+    sizes = (c_int(reqs), c_int(heads), c_int(key_dim), c_int(value_dim), c_float(cap), c_float(q_scale), c_float(den_eps))
+    below = 0x7FFFFFFF
+    # some request has that many tokens only if the others leave them; in a captured step the counts are all that is known
+    if (take is not None and n - reqs + 1 >= MEMORY_CHUNK_MIN and key_dim in MEMORY_CHUNK_KEY_DIMS and value_dim % 16 == 0
+            and not (proj.stride(0) % 8 or q_off % 8 or k_off % 8 or proj.data_ptr() % (8 * proj.element_size()))):
+        below = MEMORY_CHUNK_MIN
+        record = heads * (32 * key_dim + 276)
+        gates = take((4 * n * heads + reqs * heads,), torch.float32)
+        scratch = take((min((n // 16 + reqs) * record, max(record, MEMORY_CHUNK_SCRATCH // 4)),), torch.float32)
+        _check(build.core().ns_memory_chunks(*row, c_int(n), *sizes, c_int(below), _ptr(gates), _ptr(scratch), c_size_t(scratch.numel()),
+                                             c_int(_dtype_code(proj)), _stream()), "memory_chunks")
+        if reqs == 1:
+            return out
+    _check(build.core().ns_memory_scan(*row, *sizes, c_int(below), c_int(_dtype_code(proj)), _stream()), "memory_scan")
     return out
 
 

@@ -1242,6 +1242,91 @@ def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens():
             assert not torch.isfinite(out[21]).all()
 
 
+def test_matrix_memory_by_chunks_keeps_infinities_to_later_tokens():
+    """An infinity or NaN at one token, in any of its inputs, reaches neither the tokens before it nor other requests."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(4)
+    D, E, n = 64, 16, 120
+    proj = torch.randn(n, 152, generator=gen)
+    at = (0, D, 2 * D, 2 * D + E, 2 * D + E + 1)
+    indptr, slots = torch.tensor([0, 60, 120], dtype=torch.int32, device=DEV), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=DEV)
+
+    def run(x):
+        out, den = torch.empty(n, E, device=DEV), torch.empty(n, 1, device=DEV)
+        state = torch.zeros(2, ops.memory_state_floats(1, D, E), device=DEV)
+        ops.memory_scan(x.to(DEV), at, None, None, state, indptr, slots, 1, D, E, 15.0, D ** -0.5, out, den, take=take)
+        return torch.cat([out, den], 1).cpu()
+
+    clean = run(proj)
+    assert torch.isfinite(clean).all()
+    for bad in (float("inf"), float("nan")):
+        for column in (3, at[1] + 3, at[2] + 3) + ((at[3], at[4]) if bad != bad else ()):  # (the gates' logs are capped: an infinity is the cap)
+            x = proj.clone()
+            x[21, column] = bad
+            out = run(x)
+            others = torch.arange(n) != 21 if column < D else (torch.arange(n) < 21) | (torch.arange(n) >= 60)
+            torch.testing.assert_close(out[others], clean[others], rtol=1e-5, atol=1e-6)
+            assert not torch.isfinite(out[21]).all()
+
+
+@pytest.mark.parametrize("scratch", [0, 64 << 20], ids=["piecewise", "whole"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D,E,lens", [(2, 64, 16, [48]), (1, 128, 48, [49, 1, 0, 63, 47, 130]), (3, 128, 32, [5, 1100])])
+def test_matrix_memory_by_chunks(monkeypatch, H, D, E, lens, dtype, scratch):
+    """Prompt portions sixteen tokens at a time against the recurrence in 64 bits: last chunks of one and of fifteen tokens, requests that are
+    too short for it among them, more tokens than the gates' kernel takes at once, the records of all chunks at once and of one at a time."""
+    ops = _ops()
+    monkeypatch.setattr(ops, "MEMORY_CHUNK_SCRATCH", scratch)
+    gen = torch.Generator().manual_seed(D + len(lens))
+    n, B = sum(lens), len(lens)
+    at = (0, H * D, 2 * H * D, 2 * H * D + H * E, 2 * H * D + H * E + H)
+    proj = torch.randn(n, -(-(at[4] + H) // 8) * 8, generator=gen).to(dtype)
+    bias_i, bias_f = torch.randn(H, generator=gen), torch.randn(H, generator=gen) * 3
+    words = ops.memory_state_floats(H, D, E)
+    S0 = torch.zeros(B + 1, words)
+    S0[:, : H * E * D] = torch.randn(B + 1, H * E * D, generator=gen) * 0.2
+    state, slots = S0.clone().to(DEV), torch.arange(B, 0, -1, dtype=torch.int32)
+    indptr = torch.tensor([0, *lens]).cumsum(0).to(torch.int32)
+    out, den = torch.full((n, H * E), float("nan"), device=DEV), torch.full((n, H), float("nan"), device=DEV)
+    take = lambda shape, dt: torch.full(shape, float("nan"), dtype=dt, device=DEV)
+    run = lambda a, b, st, **kw: ops.memory_scan(proj[a:b].to(DEV), at, bias_i.to(DEV), bias_f.to(DEV), st, *kw.pop("who"), H, D, E, 15.0, D ** -0.5, out[a:b],
+                                                 den[a:b], **kw)
+    run(0, n, state, who=(indptr.to(DEV), slots.to(DEV)), take=take)
+    got, gden = out.cpu().double().view(n, H, E), den.cpu().double()
+    x = proj.double()
+    gi = 15 * torch.tanh((x[:, at[3] : at[3] + H] + bias_i.double()) / 15)
+    gf = torch.nn.functional.logsigmoid(15 * torch.tanh((x[:, at[4] : at[4] + H] + bias_f.double()) / 15))
+    for b in range(B):
+        S, N, m = S0[slots[b], : H * E * D].double().view(H, E, D), torch.zeros(H, D).double(), torch.zeros(H).double()
+        size, nsize = S.abs(), N.abs()  # the same with magnitudes: what roundings are relative to
+        for t in range(int(indptr[b]), int(indptr[b + 1])):
+            q, k, v = x[t, : H * D].view(H, D) * D ** -0.5, x[t, at[1] : at[1] + H * D].view(H, D), x[t, at[2] : at[2] + H * E].view(H, E)
+            new = torch.maximum(gf[t] + m, gi[t])
+            a, c, m = torch.exp(gf[t] + m - new)[:, None], torch.exp(gi[t] - new)[:, None], new
+            S, size = a[:, :, None] * S + (c * v)[:, :, None] * k[:, None], a[:, :, None] * size + (c * v).abs()[:, :, None] * k.abs()[:, None]
+            N, nsize = a * N + c * k, a * nsize + c * k.abs()
+            # sums of D terms, at most two roundings a token that the state has passed, exponents of up to 30 and their logs' roundings
+            bound = (D + 128 + 2 * (t - int(indptr[b]))) * 2.0 ** -24
+            assert ((got[t] - (S * q[:, None]).sum(2)).abs() <= bound * (size * q.abs()[:, None]).sum(2) + 1e-30).all(), (b, t)
+            want = torch.maximum((N * q).sum(1).abs(), torch.exp(-m)) + 1e-6
+            assert ((gden[t] - want).abs() <= bound * ((nsize * q.abs()).sum(1) + want)).all(), (b, t)
+    # a token more, on what the chunks left in the slots: the token form finds S, n and every copy of m
+    kept, live = state.clone(), [b for b in range(B) if lens[b]]
+    rows = torch.tensor([int(indptr[b + 1]) - 1 for b in live])
+    more = proj[rows].contiguous().to(DEV)
+    o1, d1 = torch.empty(len(live), H * E, device=DEV), torch.empty(len(live), H, device=DEV)
+    who = (torch.arange(len(live) + 1, dtype=torch.int32, device=DEV), slots[live].to(DEV))
+    ops.memory_scan(more, at, bias_i.to(DEV), bias_f.to(DEV), kept, *who, H, D, E, 15.0, D ** -0.5, o1, d1)
+    plain, o2, d2 = S0.clone().to(DEV), torch.empty_like(o1), torch.empty_like(d1)
+    run(0, n, plain, who=(indptr.to(DEV), slots.to(DEV)))
+    ops.memory_scan(more, at, bias_i.to(DEV), bias_f.to(DEV), plain, *who, H, D, E, 15.0, D ** -0.5, o2, d2)
+    # (both forms differ from 64 bits by less than the bound above, whose factor is at most 2 (D + 128 + 2 n) 2^-24 of the magnitudes)
+    scale = 2 * (D + 128 + 2 * n) * 2.0 ** -24
+    assert (o1 - o2).abs().max() <= scale * D * o2.abs().max() and (d1 - d2).abs().max() <= scale * D * d2.abs().max()
+    assert torch.equal(state[0].cpu(), S0[0])
+
+
 @pytest.mark.parametrize("gates", [False, True])
 @pytest.mark.parametrize("starts,lens,window", [([0], [200], 0), ([0, 70, 0], [1, 129, 40], 0), ([300, 0, 1000], [64, 33, 140], 100), ([0, 5], [577, 2], 64)])
 @pytest.mark.parametrize("heads,dim,rot,value,latent,page", [(3, 64, 32, 64, 192, 16), (2, 128, 64, 128, 64, 8), (8, 64, 32, 64, 512, 64)])

@@ -1,5 +1,6 @@
 // Soft-max attention over the paged cache for any head size and either storage type, one query row
-// and one head per workgroup.  It is the attention of the true 32-bit path.  Keys are walked in
+// and one head per workgroup.  It takes what the matrix cores' kernels do not: head or value sizes that are no multiples of
+// theirs, odd pages, and in 32-bit the options that attn_f32.hip has not.  Keys are walked in
 // fixed chunks of 256 counted from key 0, so a row's result does not depend on how the tokens were
 // cut into steps or on what else is in the batch.
 //

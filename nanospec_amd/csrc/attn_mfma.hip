@@ -51,7 +51,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 // A tile descriptor, filled on the host: {request, first token of the tile among the request's tokens of this step
 // (tiles of one request follow each other every 16 qt / hp tokens),
 // row of the request's first token in the batch, tokens of the request in this step, keys after this step,
-// for decode tiles the keys that all decode rows of the step read together over all layers, 0, 0}.
+// for decode tiles the keys that all decode rows of the step read together over all layers, and two ints for
+// the latent form's portions (csrc/latent_prompt.hip)}.
 struct AttnParams {
   bf16_t* out;        // [tokens, heads, HD]
   float* part_o;      // [n_tiles * (16 / hp) * heads, splits, HD]   (splits > 1)

@@ -777,7 +777,7 @@ def attention_mfma(q, out, k_cache, v_cache, tiles, block_table, heads: int, kv_
                    sink_logits: torch.Tensor | None = None) -> torch.Tensor:
     """bfloat16 attention on the matrix cores for the tiles described in ``tiles`` (int32 [n_tiles, 8]: request, first
     token of the tile among the request's tokens of this step, row of the request's first token in ``q``, tokens of the
-    request in this step, keys after this step, three zeros).  ``hp`` heads of a group times 16/hp tokens make a tile;
+    request in this step, keys after this step, three that these kernels do not read for portions).  ``hp`` heads of a group times 16/hp tokens make a tile;
     with ``qt`` = 2 (only with hp = 1) a tile is 32 tokens.  ``splits`` > 1 cuts the keys of every tile
     into that many ranges (at most 64) and needs ``workspace`` = (part_o, part_ml) float32 tensors.  With ``coop`` the four
     waves of a workgroup share each tile and range (for decode, where a wave's chain of loads is what takes the time); with

@@ -185,7 +185,8 @@ def wide_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_di
 
 def f32_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_dim: int, scale: float, window: int = 0, chunk: int = 0,
                   **options) -> torch.Tensor:
-    """32-bit attention of the batch's portion tiles and single tokens on the matrix cores (sizes: ``ops.f32_attention_takes``).
+    """32-bit attention of the batch's portion tiles and single tokens on the matrix cores (sizes: ``ops.f32_attention_takes``; a block that
+    hands on no batch plans has no tiles, and its 32-bit layers run ``ops.attention_generic``, which needs none).
     A single token's keys go in ranges of ``F32_RANGE_KEYS`` from key 0 whatever else is in the batch, so its result does not
     depend on it; a portion's are cut only where its tiles leave the GPU idle."""
     chunk_tiles, decode_tiles = TilePlan.views(ctx)
@@ -400,7 +401,7 @@ class Attention:
                 ops.attention_mfma(qkv, att, cache.k, cache.v, plan.tiles, table, s.heads, s.kv_heads, s.head_dim,
                                    s.softmax_scale, window=s.window, hp=plan.hp, splits=plan.splits, workspace=plan.workspace,
                                    qt=plan.qt, coop=plan.coop)
-        elif ops.f32_attention_takes(x.dtype, s.head_dim, s.head_dim, page):
+        elif TilePlan.key in ctx.plans and ops.f32_attention_takes(x.dtype, s.head_dim, s.head_dim, page):
             f32_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.softmax_scale, window=s.window)
         else:
             ops.attention_generic(qkv, att, cache.k, cache.v, ctx.token_req, ctx.positions, table, s.heads, s.kv_heads,
@@ -467,7 +468,7 @@ class Attention:
             # bfloat16, values of another size than the keys or a bias by distance: the two-size matrix-core kernel
             wide_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.v_dim, s.softmax_scale, window=s.window,
                            slope_exp=s.slope_exp, sink_logits=self.sink_logits)
-        elif ops.f32_attention_takes(x.dtype, s.head_dim, s.v_dim, cache.k.shape[2]) and qkv.stride(0) % 4 == 0:
+        elif TilePlan.key in ctx.plans and ops.f32_attention_takes(x.dtype, s.head_dim, s.v_dim, cache.k.shape[2]) and qkv.stride(0) % 4 == 0:
             f32_attention(ctx, qkv, att, cache, table, s.heads, s.kv_heads, s.head_dim, s.softmax_scale, window=s.window, chunk=s.chunk,
                           cap=s.score_cap, sink=s.sink, slope_exp=s.slope_exp, sink_logits=self.sink_logits)
         else:

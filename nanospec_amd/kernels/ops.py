@@ -1197,9 +1197,9 @@ def memory_state_floats(heads: int, key_dim: int, value_dim: int) -> int:
 
 # Prompt portions of the matrix memory chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
 # the tokens from which on a request is worth the three launches (8 heads of 128 by 256: 32 tokens 16 us token by token and 18 so, 64 tokens
-# 27 and 19), and the scratch in bytes that the chunks' records may take (17 KiB a chunk and head at 128 channels; what does not fit goes in several passes).
+# 27 and 19, 40 requests of 48 tokens 145 and 99; what the delta rule loses with few small heads holds here too), and the scratch in bytes that the chunks' records may take (17 KiB a chunk and head at 128 channels; what does not fit goes in several passes).
 MEMORY_CHUNK_KEY_DIMS = (64, 128)
-MEMORY_CHUNK_MIN = 48
+MEMORY_CHUNK_MIN = 64
 MEMORY_CHUNK_SCRATCH = 64 << 20
 
 
@@ -1882,10 +1882,10 @@ MAX_CONV_TAPS = 16
 DELTA_MAX_KEY_DIM = 1024
 # Prompt portions of the delta rule chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
 # the tokens from which on a request is worth the two launches (16 heads of 128: 16 tokens 11 us token by token, 32 tokens 16.5 and 15.5,
-# 64 tokens 26.6 and 18.4) and the scratch in bytes that the chunks' records may take (27 KiB a chunk and head at 128 channels, a
+# 64 tokens 26.6 and 18.4; 64 requests of 32 tokens and 4 heads of 64: 15 and 27, of 16 heads of 128: 204 and 175) and the scratch in bytes that the chunks' records may take (27 KiB a chunk and head at 128 channels, a
 # prompt of 2,048 tokens of 16 heads in one piece; what does not fit goes in several passes, 8,192 tokens of 32 heads 2,750 -> 970 us).
 DELTA_CHUNK_KEY_DIMS = (64, 128)
-DELTA_CHUNK_MIN = 32
+DELTA_CHUNK_MIN = 64
 DELTA_CHUNK_SCRATCH = 64 << 20
 
 

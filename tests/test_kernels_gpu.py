@@ -1186,6 +1186,7 @@ def test_delta_rule_by_chunks(monkeypatch, H, G, D, E, lens, scratch):
     are too short for it among them, decays of zero and of one, the records of all chunks at once and of one at a time."""
     ops = _ops()
     monkeypatch.setattr(ops, "DELTA_CHUNK_SCRATCH", scratch)
+    monkeypatch.setattr(ops, "DELTA_CHUNK_MIN", 32)
     gen = torch.Generator().manual_seed(D + len(lens))
     n, B, C = sum(lens), len(lens), 2 * G * D + H * E
     rnd = lambda *shape: torch.randn(*shape, generator=gen)
@@ -1217,9 +1218,10 @@ def test_delta_rule_by_chunks(monkeypatch, H, G, D, E, lens, scratch):
     assert torch.equal(after[0], S0[0].double())
 
 
-def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens():
+def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
     """An infinity or NaN at one token reaches neither the tokens before it nor other requests, as token by token."""
     ops = _ops()
+    monkeypatch.setattr(ops, "DELTA_CHUNK_MIN", 32)
     gen = torch.Generator().manual_seed(3)
     D, E, n, C = 64, 16, 80, 2 * 64 + 16
     qkv, g, beta = torch.randn(n, C, generator=gen) * 0.1, torch.rand(n, D, generator=gen) ** 0.2, torch.rand(n, 1, generator=gen)
@@ -1242,9 +1244,10 @@ def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens():
             assert not torch.isfinite(out[21]).all()
 
 
-def test_matrix_memory_by_chunks_keeps_infinities_to_later_tokens():
+def test_matrix_memory_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
     """An infinity or NaN at one token, in any of its inputs, reaches neither the tokens before it nor other requests."""
     ops = _ops()
+    monkeypatch.setattr(ops, "MEMORY_CHUNK_MIN", 48)
     gen = torch.Generator().manual_seed(4)
     D, E, n = 64, 16, 120
     proj = torch.randn(n, 152, generator=gen)
@@ -1278,6 +1281,7 @@ def test_matrix_memory_by_chunks(monkeypatch, H, D, E, lens, dtype, scratch):
     too short for it among them, more tokens than the gates' kernel takes at once, the records of all chunks at once and of one at a time."""
     ops = _ops()
     monkeypatch.setattr(ops, "MEMORY_CHUNK_SCRATCH", scratch)
+    monkeypatch.setattr(ops, "MEMORY_CHUNK_MIN", 48)
     gen = torch.Generator().manual_seed(D + len(lens))
     n, B = sum(lens), len(lens)
     at = (0, H * D, 2 * H * D, 2 * H * D + H * E, 2 * H * D + H * E + H)

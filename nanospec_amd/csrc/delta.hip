@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const DeltaChunks p) {
       x[i] = i < tid ? 0. : (i == tid ? 1. : -beta_s[i] * s);
     }
 #pragma unroll
-    for (int i = 0; i < DC_T; ++i) t_s[i][tid] = (float)(x[i] * beta_s[tid]);
+    for (int i = 0; i < DC_T; ++i) t_s[i][tid] = i < tid ? 0.f : (float)(x[i] * beta_s[tid]);  // (beta may be no number: 0 beta is none either)
   }
   __syncthreads();
   for (int e = tid; e < 3 * DC_T * (D / 4); e += 256) {

@@ -1219,7 +1219,8 @@ def test_delta_rule_by_chunks(monkeypatch, H, G, D, E, lens, scratch):
 
 
 def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
-    """An infinity or NaN at one token reaches neither the tokens before it nor other requests, as token by token."""
+    """An infinity or NaN at one token, in any of its inputs or in all of them, reaches neither the tokens before it nor other requests, as
+    token by token."""
     ops = _ops()
     monkeypatch.setattr(ops, "DELTA_CHUNK_MIN", 32)
     gen = torch.Generator().manual_seed(3)
@@ -1228,9 +1229,9 @@ def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
     indptr, slots = torch.tensor([0, 40, 80], dtype=torch.int32, device=DEV), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
     take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=DEV)
 
-    def run(x, gg):
+    def run(x, gg, bb=beta):
         out = torch.empty(n, E, device=DEV)
-        return ops.delta_scan(x.to(DEV), gg.to(DEV), beta.to(DEV), torch.zeros(2, D * E, device=DEV), indptr, slots, 1, 1, D, E, out=out, take=take).cpu()
+        return ops.delta_scan(x.to(DEV), gg.to(DEV), bb.to(DEV), torch.zeros(2, D * E, device=DEV), indptr, slots, 1, 1, D, E, out=out, take=take).cpu()
 
     clean = run(qkv, g)
     assert torch.isfinite(clean).all()
@@ -1240,6 +1241,18 @@ def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
             x[21, column] = bad
             out = run(x, g)
             others = torch.arange(n) != 21 if column < D else (torch.arange(n) < 21) | (torch.arange(n) >= 40)
+            torch.testing.assert_close(out[others], clean[others], rtol=1e-5, atol=1e-6)
+            assert not torch.isfinite(out[21]).all()
+        others = (torch.arange(n) < 21) | (torch.arange(n) >= 40)
+        for what in ("beta", "g", "all"):  # (a token whose row of the stream is not finite has no number anywhere)
+            x, gg, bb = qkv.clone(), g.clone(), beta.clone()
+            if what in ("beta", "all"):
+                bb[21] = bad
+            if what in ("g", "all"):
+                gg[21, 3 if what == "g" else slice(None)] = bad
+            if what == "all":
+                x[21] = bad
+            out = run(x, gg, bb)
             torch.testing.assert_close(out[others], clean[others], rtol=1e-5, atol=1e-6)
             assert not torch.isfinite(out[21]).all()
 

@@ -59,14 +59,20 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const T* __restrict__ h
 }
 
 // The same logits for many tokens, on the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: 32-bit products and sums): a workgroup takes 16
-// tokens and up to 32 rows of the router, its four waves every fourth piece of 16 columns, and adds the waves' sums in a fixed order; a
+// tokens and up to 32 rows of the router, its eight waves every eighth piece of 16 columns, and adds the waves' sums in a fixed order; a
 // token's logits do not depend on the tokens beside it.  Lane l holds columns 4 (l / 16) .. + 3 of row (token) l % 16 of an operand, one
-// load for four instructions, 64 columns on their way.  The kernel above is bound by its reads of the tokens (every four experts read them
-// anew) and by the exchange that adds 64 lanes' sums: 2,048 tokens, 33 rows of 2,048: 38 -> 14 us.  W a multiple of 16.
+// load for four instructions, four pieces on their way.  The kernel above is bound by its reads of the tokens (every four experts read them
+// anew) and by the exchange that adds 64 lanes' sums; this one by the latency of a wave's rounds.  33 rows of 2,048, with the choice behind:
+// 2,048 tokens 37.5 -> 19.9 us, 508 tokens 18.7 -> 18.5 (four waves 22.7 and 21.7).
+// The logits decide which experts run, so no 32-bit chain is longer than 8 columns (two instructions), and the chains are added in 64 bits.
+// Relative error (2-norm, against 64 bits) at 2,048 columns 5.9e-8, of the kernel above 1.2e-7, with one chain a wave 4.0e-7; it is below
+// the other's down to 64 columns, from where on the launch takes this kernel.  W a multiple of 16.
+#define MOE_LOGIT_WAVES 8
 template <typename T>
-__global__ __launch_bounds__(256) void moe_logits_many_kernel(const T* __restrict__ h, int h_stride, const float* __restrict__ wr,
+__global__ __launch_bounds__(NS_WAVE * MOE_LOGIT_WAVES) void moe_logits_many_kernel(const T* __restrict__ h, int h_stride, const float* __restrict__ wr,
                                                               const float* __restrict__ br, float* __restrict__ z, int n, int W, int experts) {
-  __shared__ __attribute__((aligned(16))) float part[4][2][16][20];  // [wave][16 rows of the router][token][row]
+  constexpr int STEP = 16 * MOE_LOGIT_WAVES;  // columns from one piece of a wave to the next
+  __shared__ double part[MOE_LOGIT_WAVES][2][16][17];  // [wave][16 rows of the router][token][row]
   const int lane = threadIdx.x % NS_WAVE, wave = threadIdx.x / NS_WAVE, r = lane % 16, g = lane / 16;
   const int t0 = blockIdx.x * 16, e0 = blockIdx.y * 32;
   const T* x = h + (size_t)min(t0 + r, n - 1) * h_stride + 4 * g;
@@ -74,33 +80,44 @@ __global__ __launch_bounds__(256) void moe_logits_many_kernel(const T* __restric
 #pragma unroll
   for (int i = 0; i < 2; ++i) w[i] = wr + (size_t)min(e0 + 16 * i + r, experts - 1) * W + 4 * g;
   typedef T t4 __attribute__((ext_vector_type(4)));
-  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  for (int c = 16 * wave; c < W; c += 4 * 64) {
+  double sum[2][4] = {};
+  for (int c = 16 * wave; c < W; c += 4 * STEP) {
     t4 xv[4];
     f32x4 wv[4][2];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {  // (a piece beyond the row is read at its start and not used)
-      const int at = c + 64 * s < W ? c + 64 * s : 0;
+      const int at = c + STEP * s < W ? c + STEP * s : 0;
       xv[s] = *reinterpret_cast<const t4*>(x + at);
 #pragma unroll
       for (int i = 0; i < 2; ++i) wv[s][i] = *reinterpret_cast<const f32x4*>(w[i] + at);
     }
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (c + 64 * s < W)
+    for (int s = 0; s < 4; ++s) {
+      if (c + STEP * s >= W) break;
+      f32x4 acc[2][2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
-          for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s][i][k], to_f((T)xv[s][k]), acc[i], 0, 0, 0);
+        for (int i = 0; i < 2; ++i)
+          acc[k / 2][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s][i][k], to_f((T)xv[s][k]), k % 2 ? acc[k / 2][i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum[i][k] += (double)acc[0][i][k] + (double)acc[1][i][k];
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4*>(&part[wave][i][r][4 * g]) = acc[i];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[wave][i][r][4 * g + k] = sum[i][k];
   __syncthreads();
-  for (int i = threadIdx.x; i < 512; i += 256) {
+  for (int i = threadIdx.x; i < 512; i += NS_WAVE * MOE_LOGIT_WAVES) {
     const int t = i / 32, e = i % 32;
-    if (t0 + t < n && e0 + e < experts)
-      z[(size_t)(t0 + t) * experts + e0 + e] = ((part[0][e / 16][t][e % 16] + part[1][e / 16][t][e % 16]) + (part[2][e / 16][t][e % 16] + part[3][e / 16][t][e % 16])) +
-                                               (br ? br[e0 + e] : 0.f);
+    if (t0 + t >= n || e0 + e >= experts) continue;
+    double v = br ? (double)br[e0 + e] : 0.;
+#pragma unroll
+    for (int j = 0; j < MOE_LOGIT_WAVES; ++j) v += part[j][e / 16][t][e % 16];
+    z[(size_t)(t0 + t) * experts + e0 + e] = (float)v;
   }
 }
 
@@ -267,12 +284,12 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
       moe_logits_few_kernel<float><<<rows, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
     else
       moe_logits_few_kernel<bf16_t><<<rows, 256, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows, vec);
-  } else if (vec && W % 16 == 0) {
+  } else if (vec && W % 16 == 0 && W >= 64) {
     const dim3 many((n + 15) / 16, (rows + 31) / 32);
     if (dtype == NS_DTYPE_F32)
-      moe_logits_many_kernel<float><<<many, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows);
+      moe_logits_many_kernel<float><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows);
     else
-      moe_logits_many_kernel<bf16_t><<<many, 256, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows);
+      moe_logits_many_kernel<bf16_t><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows);
   } else if (dtype == NS_DTYPE_F32)
     moe_logits_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
   else

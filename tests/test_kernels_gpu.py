@@ -1156,6 +1156,25 @@ def test_moe_router_of_many_tokens(n, rows, width, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,rows,width", [(64, 33, 2048), (300, 16, 4096), (40, 64, 512), (500, 64, 64)])
+def test_moe_router_of_many_tokens_is_as_exact_as_the_plain_kernel(n, rows, width, dtype):
+    """The logits decide which experts run: on the matrix instruction they are no further from 64 bits (2-norm over thousands of
+    logits) than the plain kernel's, which takes the same rows where they lie off their 16-byte places."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(width)
+    h, router = torch.randn(n, width, generator=g).to(dtype), torch.randn(rows, width, generator=g) * 0.02
+    want = h.double() @ router.double().T
+    err = []
+    for off in (0, 1):
+        wide = torch.zeros(n, width + 4, dtype=dtype, device=DEV)
+        wide[:, off : off + width] = h.to(DEV)
+        z, sel, wt = torch.full((n, rows), float("nan"), device=DEV), torch.zeros(n, 2, dtype=torch.int32, device=DEV), torch.zeros(n, 2, device=DEV)
+        ops.moe_route(wide[:, off : off + width], router.to(DEV), None, 2, sel, wt, logits=z)
+        err.append(float((z.cpu().double() - want).norm() / want.norm()))
+    assert err[0] <= err[1], err
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,top,width", [(1, 1, 4), (3, 4, 1020), (5, 2, 1028), (2, 3, 2050)])
 def test_moe_combine(n, top, width, dtype):
     """The experts' parts added up: rows that end inside a workgroup's 1,024 columns, the input in a part's place, a gated base or none."""

@@ -15,10 +15,14 @@
 //     v_mfma_f32_16x16x32_bf16, so a token's scores, maximum and sums are its own lanes'.  Queries are rotated as they are read; the
 //     sink's term, the gate per head and the gate per channel are applied to the 32-bit result before it is rounded.  LDS rows are 32
 //     bytes longer than their data (no bank conflicts).  Bound by the matrix and the vector unit in turn (the soft-max of a block takes
-//     about as long as its products) and the longest tile's chain of blocks, hence 64 tokens and not 128.  2,048 tokens, 32 heads of
-//     64 + 32, both kernels: 69 to 80 us (128 tokens: 25 us more); the wide form took 585 us and 127 us around it.
+//     about as long as its products) and the longest tile's chain of blocks, hence 64 tokens and not 128.  What is not finite
+//     reaches the tokens that see it and no others; blocks at a tile's edges have code of their own for that, and the others then do
+//     without a mask.  2,048 tokens, 32 heads of 64 + 32, both kernels: 75 us (128 tokens a workgroup: 25 us more); the wide form takes
+//     545 us and 120 us around it.
 #include "common.h"
 #include "rope.h"
+
+#include <type_traits>
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(256) void latent_expand_kernel(LatentPromptParams p
 }
 
 template <int D, int R, int E>
-__global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p) {
+__global__ __launch_bounds__(256, D == 64 ? 3 : 1) void latent_prompt_kernel(LatentPromptParams p) {
   constexpr int KD = D + R, KS = KD / 32, VT = E / 16, KROW = KD + 16, VROW = LP_KEYS + 16;
   constexpr int BLOCK = LP_KEYS * (KD + E), BUF = LP_KEYS * KROW + E * VROW, PER = BLOCK / 8 / 256;
   static_assert(BLOCK % (8 * 256) == 0 && KD % 32 == 0 && R % 32 == 0 && E % 16 == 0, "pieces of 16 bytes, 256 threads");
@@ -159,7 +163,6 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
   const int w0 = 16 * wave;  // the wave's first token of the tile
   const bool works = w0 < n_tok;
   const int wave_lo = first_key(base + w0), wave_hi = base + min(w0 + 16, n_tok) - 1;
-  const int full_lo = first_key(wave_hi), full_hi = base + w0;  // keys that every token of the wave sees
   const int tok = min(w0 + c, n_tok - 1), pos = base + tok, lo = first_key(pos);
   const size_t row = (size_t)info[2] + t0 + tok;
   bf16x8 q[KS];
@@ -203,6 +206,85 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
   float m = -INFINITY, l = 0.f;  // l: this lane's keys
 #pragma unroll
   for (int t = 0; t < VT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a block's part of a wave's 16 tokens; EDGE: some token of the workgroup does not see all of its keys
+  auto work = [&](auto edge, int k0, int buf) {
+    constexpr bool EDGE = decltype(edge)::value;
+    const bf16_t* ks = lds + buf * BUF + c * KROW + 8 * g;
+    const bf16_t* vs = lds + buf * BUF + LP_KEYS * KROW + c * VROW + 8 * g;
+    f32x4 s[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      bf16x8 k[KS];
+#pragma unroll
+      for (int i = 0; i < KS; ++i) k[i] = *reinterpret_cast<const bf16x8*>(ks + 16 * t * KROW + 32 * i);
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < KS; ++i) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[i], q[i], s[t], 0, 0, 0);
+    }
+    bf16x8 w[2];
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = k0 + 16 * t + 4 * g + i;
+        if (EDGE && (key < lo || key > pos)) s[t][i] = -INFINITY;
+        top = fmaxf(top, s[t][i]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float m_new = fmaxf(m, top), ref = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f((m - ref) * p.scale_log2), shift = -ref * p.scale_log2;
+    const bool moved = __any(m_new != m);
+    m = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[t][i], p.scale_log2, shift));
+        sum += e;
+        w[t / 2][4 * (t % 2) + i] = (bf16_t)e;
+      }
+    if (moved) {
+      l *= alpha;
+#pragma unroll
+      for (int t = 0; t < VT; ++t) o[t] *= alpha;
+    }
+    l += sum;
+    unsigned odd = 0;
+    if (EDGE) {  // an infinite value or one that is no number among those that some token does not see: all bits of its exponent are set
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const uint4 v = *reinterpret_cast<const uint4*>(vs + 16 * t * VROW + 32 * i);
+          const unsigned pairs[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) odd |= (pairs[e] & 0x7f807f80u) + 0x00800080u;
+        }
+    }
+    if (!EDGE || !__any(odd & 0x80008000u)) {
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(vs + 16 * t * VROW + 32 * i), w[i], o[t], 0, 0, 0);
+    } else {  // a weight of zero would make it that token's too, so each token adds the keys it sees only
+      const bf16_t* at = lds + buf * BUF + LP_KEYS * KROW + 4 * g * VROW;
+#pragma unroll
+      for (int x = 0; x < 16; ++x)  // the weight that lanes 16 gg + c hold in place x % 8 of w[x / 8] is of key 32 (x / 8) + 16 (x % 8 / 4) + 4 gg + x % 4
+        for (int gg = 0; gg < 4; ++gg) {
+          const int key = k0 + 32 * (x / 8) + 16 * (x % 8 / 4) + 4 * gg + x % 4;
+          const float weight = __shfl(to_f(w[x / 8][x % 8]), 16 * gg + c, 64);
+          if (key < lo || key > pos) continue;
+#pragma unroll
+          for (int t = 0; t < VT; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[t][j] = fmaf(weight, to_f(at[(16 * t + j) * VROW + 32 * (x / 8) + 8 * gg + x % 8]), o[t][j]);
+        }
+    }
+  };
   fetch(b0);
   park(0);
   for (int b = b0; b < b1; ++b) {
@@ -210,55 +292,10 @@ __global__ __launch_bounds__(256) void latent_prompt_kernel(LatentPromptParams p
     __syncthreads();
     if (b + 1 < b1) fetch(b + 1);
     if (works && k0 <= wave_hi && k0 + LP_KEYS > wave_lo) {
-      const bf16_t* ks = lds + buf * BUF + c * KROW + 8 * g;
-      const bf16_t* vs = lds + buf * BUF + LP_KEYS * KROW + c * VROW + 8 * g;
-      f32x4 s[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        bf16x8 k[KS];
-#pragma unroll
-        for (int i = 0; i < KS; ++i) k[i] = *reinterpret_cast<const bf16x8*>(ks + 16 * t * KROW + 32 * i);
-        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < KS; ++i) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[i], q[i], s[t], 0, 0, 0);
-      }
-      const bool full = k0 >= full_lo && k0 + LP_KEYS - 1 <= full_hi;
-      bf16x8 w[2];
-      float top = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = k0 + 16 * t + 4 * g + i;
-          if (!full && (key < lo || key > pos)) s[t][i] = -INFINITY;
-          top = fmaxf(top, s[t][i]);
-        }
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
-      const float m_new = fmaxf(m, top), ref = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f((m - ref) * p.scale_log2), shift = -ref * p.scale_log2;
-      const bool moved = __any(m_new != m);
-      m = m_new;
-      float sum = 0.f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float e = __builtin_amdgcn_exp2f(fmaf(s[t][i], p.scale_log2, shift));
-          sum += e;
-          w[t / 2][4 * (t % 2) + i] = (bf16_t)e;
-        }
-      if (moved) {
-        l *= alpha;
-#pragma unroll
-        for (int t = 0; t < VT; ++t) o[t] *= alpha;
-      }
-      l += sum;
-#pragma unroll
-      for (int t = 0; t < VT; ++t)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(vs + 16 * t * VROW + 32 * i), w[i], o[t], 0, 0, 0);
+      if (k0 >= first_key(hi) && k0 + LP_KEYS - 1 <= base)
+        work(std::false_type{}, k0, buf);
+      else
+        work(std::true_type{}, k0, buf);
     }
     if (b + 1 < b1) park(buf ^ 1);
   }

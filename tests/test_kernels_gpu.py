@@ -1440,6 +1440,48 @@ def test_latent_prompt(heads, dim, rot, value, latent, page, starts, lens, windo
                 assert ((got - want).abs() <= 2.0 ** -6 * mag + 2.0 ** -8 * want.abs() + 1e-6).all(), (b, h, interleaved)
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("window", [0, 70])
+def test_latent_prompt_keeps_infinities_to_the_rows_that_see_them(window, bad):
+    """A latent that is infinite or no number belongs to the tokens that see its position; the others' results are what they would be
+    without it, also where they share a block of keys with it."""
+    from nanospec_amd.parts.attention import TilePlan
+    from nanospec_amd.engine.context import BatchFacts
+    import numpy as np
+
+    ops = _ops()
+    heads, dim, rot, value, C, page, start, n, at = 2, 64, 32, 64, 64, 16, 20, 150, 90
+    g = torch.Generator().manual_seed(8)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).bfloat16().to(DEV)
+    total = start + n
+    pages = -(-total // page)
+    cache, q = rnd(pages, 1, page, C + rot), rnd(n, heads * (dim + rot))
+    uk, uv = rnd(heads * dim, C) * C ** -0.5, rnd(heads * value, C) * C ** -0.5
+    inv = (10000.0 ** (-torch.arange(0, rot, 2).float() / rot)).to(DEV)
+    i32 = lambda x: np.asarray(x, dtype=np.int32)
+    plan = TilePlan()
+    shape = plan.shape([n])
+    region = np.zeros(plan.ints(shape), dtype=np.int32)
+    plan.fill(region, shape, BatchFacts(n, 1, i32([n]), i32([start]), i32([0, n]), i32([total]), 1, 1))
+    tiles, table = torch.from_numpy(region.reshape(-1, 8)).to(DEV), torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
+    blocks = -(-total // 128) * 2
+
+    def run():
+        scratch = torch.zeros(blocks * ops.latent_prompt_block(torch.bfloat16, heads, dim, rot, value, C), dtype=torch.bfloat16, device=DEV)
+        out = torch.zeros(n, heads * value, dtype=torch.bfloat16, device=DEV)
+        return ops.latent_prompt(q, cache, uk, uv, scratch, tiles, table, inv, 1.0, heads, dim, rot, value, C, 1, blocks, 0.1, out, window=window).float()
+
+    clean = run()
+    assert torch.isfinite(clean).all()
+    cache[at // page, 0, at % page, 5] = bad
+    out = run()
+    pos = torch.arange(start, total, device=DEV)
+    sees = (pos >= at) & (pos - at < window if window else torch.ones_like(pos, dtype=torch.bool))
+    # (the sums run in another order: the result may round to the next bfloat16)
+    torch.testing.assert_close(out[~sees], clean[~sees], rtol=2.0 ** -7, atol=2.0 ** -12)
+    assert not torch.isfinite(out[sees]).all(dim=1).any()
+
+
 def _turned(x, pos, inv, interleaved):
     half = len(inv)
     ang = (pos[:, None].float() * inv.float()[None]).double()

@@ -15,15 +15,22 @@
 //   attn_f32_rows_kernel: single tokens.  All heads of a group are a wave's columns, keys and values go from the cache straight into
 //     operand registers, four waves take a range's tiles of 16 keys in turn; ranges are added by attn_f32_join_kernel.  Bound
 //     by the cache's bytes and the latency of a wave's loads.  5 rows at 900 keys, 32 heads of 64 over 8: 201 -> 16 us with the joining.
-// A row's result depends on its own keys only, not on the tile or the rows beside it: blocks and the ranges of single tokens
-// start at fixed keys, and one without a key that a token sees changes nothing of it.  (As a single token, or where a portion's
-// keys are cut into ranges because its tiles are few, the sums are ordered differently.)
+// A row's result depends on its own keys only, whatever stands beside it in the batch and however many workgroups share the work: keys go in
+// ranges that lie at fixed places (256 keys of a portion, 128 of a single token, counted from key 0), every range is summed from nothing
+// and the ranges are added in order by the same operations, in the registers of a workgroup that walks all of them or by
+// attn_f32_join_kernel.  A row with more than 16 (64) of them has ranges of twice as many keys, four times, ...: a portion's tile and a single
+// token choose by their own keys.  A block or range without a key that a token sees changes nothing of it.  (As a single token and as one
+// of a portion a token's sums are ordered differently, and so they are for the tokens of a tile across 4,096, 8,192, ... keys when another cut
+// of the prompt moves the tile.)
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define AF_KEYS 64
 #define AF_TOKENS 32
 #define AF_ROWS_TILES 4  // waves of a workgroup of the kernel for single tokens
+#define AF_RANGE 4       // blocks of a range of a portion's keys
+#define AF_RANGES 16     // the most ranges of a portion's keys
+#define AF_ROWS_RANGES 64  // and of a single token's
 
 struct AttnF32Params {
   float* out;        // [rows][heads * HD]
@@ -36,6 +43,7 @@ struct AttnF32Params {
   const int* block_table;
   const float* sink_logit;
   int q_stride, table_stride, heads, kv_heads, page_shift, splits, range_tiles, window, chunk, sink, n_tiles;  // range_tiles: of 16 keys (single tokens)
+  int rows;
   float scale, cap, slope_exp;
 };
 
@@ -55,6 +63,33 @@ __device__ __forceinline__ f32x4 finish_scores(const AttnF32Params& p, f32x4 s, 
     s[i] = key0 + i >= lo && key0 + i <= pos ? v : -INFINITY;
   }
   return s;
+}
+
+// The ranges of blocks (of tiles of 16 keys for a single token) lo .. hi: ``length`` of them each, or twice as many, four times, ... until there
+// are no more than ``most`` ranges; first: the one that holds lo, counted from key 0.
+struct KeyRanges {
+  unsigned length, first;
+};
+__device__ __forceinline__ KeyRanges key_ranges(unsigned lo, unsigned hi, unsigned length, unsigned most) {
+  unsigned first = lo / length;
+  for (; hi >= (first + most) * length; length *= 2) first /= 2;
+  return {length, first};
+}
+
+// How a portion's tile is cut.  (The workspace may have room for fewer ranges than AF_RANGES; it then has room for all that a tile needs.)
+__device__ __forceinline__ KeyRanges portion_ranges(const AttnF32Params& p, int tile_lo, int hi) {
+  return key_ranges(tile_lo / AF_KEYS, hi / AF_KEYS, AF_RANGE, p.splits > 1 ? p.splits : AF_RANGES);
+}
+__device__ __forceinline__ unsigned range_count(const KeyRanges& r, int hi) { return (hi / AF_KEYS >> (31 - __clz(r.length))) - r.first + 1; }
+
+// What a range with maximum m does to the sums of the ranges before it, whose maximum is top: sum = sum * old + range * now, the product
+// with ``old`` rounded first.  The same operations wherever it is done.
+struct RangeWeights {
+  float old, now;
+};
+__device__ __forceinline__ RangeWeights range_weights(float top, float m) {
+  const float both = fmaxf(top, m), ref = both == -INFINITY ? 0.f : both;
+  return {top == -INFINITY ? 0.f : expf(top - ref), m == -INFINITY ? 0.f : expf(m - ref)};
 }
 
 __device__ __forceinline__ float over_groups_max(float v) {
@@ -100,9 +135,10 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnF32Params p) {
 #pragma unroll
   for (int c = 0; c < C; ++c) q[c] = *reinterpret_cast<const f32x4*>(p.q + row * p.q_stride + head * HD + 16 * c + 4 * g) * p.scale;
 
-  const int blocks_lo = tile_lo / AF_KEYS, blocks = hi / AF_KEYS + 1 - blocks_lo;
-  const int share = (blocks + p.splits - 1) / p.splits;
-  const int b0 = blocks_lo + (int)blockIdx.y * share, b1 = min(blocks_lo + blocks, b0 + share);
+  // this workgroup's ranges, a like share for each of the launch's workgroups in y
+  const KeyRanges ranges = portion_ranges(p, tile_lo, hi);
+  const int count = range_count(ranges, hi), share = gridDim.y == 1 ? count : (count + gridDim.y - 1) / gridDim.y, range0 = ranges.first + blockIdx.y * share;
+  const int b0 = max(tile_lo / AF_KEYS, range0 * (int)ranges.length), b1 = min(hi / AF_KEYS + 1, (range0 + share) * (int)ranges.length);
 
   // a block of 64 keys: keys in pieces of four channels, values in pieces of four keys, PER of each a thread.  Keys outside of what the tile
   // sees are read as the nearest one it does (their pages may be gone) and their values taken as zero.
@@ -147,16 +183,44 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnF32Params p) {
     if (lane == 0) odd_values[buf][wave] = any;
   };
 
-  float m = -INFINITY, l = 0.f;  // l: this lane's keys of every block
-  f32x4 acc[C];
+  float m = -INFINITY, l = 0.f;  // of the range so far; l: this lane's keys of every block
+  float top = -INFINITY, sum = 0.f;  // of the ranges before
+  f32x4 acc[C], all[C];
 #pragma unroll
-  for (int c = 0; c < C; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < C; ++c) acc[c] = all[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (b0 < b1) {
     pages(b0);
     fetch(b0);
     pages(b0 + 1);
     park(b0, 0);
   }
+  const bool mine = works && 16 * (wave & 1) + col < n_tok;
+  size_t at = (((size_t)tile * AF_TOKENS + tok) * p.heads + head) * p.splits + blockIdx.y * share;  // place of the range in the workspace
+  auto end_range = [&]() {
+    l = over_groups_sum(l);
+    if (p.splits > 1) {
+      if (mine) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) *reinterpret_cast<f32x4*>(p.part_o + at * HD + 16 * c + 4 * g) = acc[c];
+        if (g == 0) p.part_ml[2 * at] = m, p.part_ml[2 * at + 1] = l;
+      }
+      ++at;
+    } else if (count == 1) {  // (what the sums below come to)
+      top = m, sum = l;
+#pragma unroll
+      for (int c = 0; c < C; ++c) all[c] = acc[c];
+    } else {
+      const RangeWeights w = range_weights(top, m);
+      top = fmaxf(top, m), sum = fmaf(l, w.now, sum * w.old);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) all[c][i] = fmaf(acc[c][i], w.now, all[c][i] * w.old);
+    }
+    m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
   for (int b = b0; b < b1; ++b) {
     const int buf = (b - b0) & 1;
     __syncthreads();
@@ -184,23 +248,23 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnF32Params p) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) s[t] = finish_scores(p, s[t], k0 + 16 * t + 4 * g, lo, pos, slope);
       }
-      float top = s[0][0];
+      float highest = s[0][0];
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) top = fmaxf(top, s[t][i]);
-      const float m_new = fmaxf(m, over_groups_max(top));
+        for (int i = 0; i < 4; ++i) highest = fmaxf(highest, s[t][i]);
+      const float m_new = fmaxf(m, over_groups_max(highest));
       const float ref = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = m == -INFINITY ? 0.f : expf(m - ref);
-      float sum = 0.f;
+      float weights = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           s[t][i] = expf(s[t][i] - ref);
-          sum += s[t][i];
+          weights += s[t][i];
         }
-      l = l * alpha + sum;
+      l = l * alpha + weights;
       m = m_new;
 #pragma unroll
       for (int c = 0; c < C; ++c) acc[c] *= alpha;
@@ -237,19 +301,12 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnF32Params p) {
       }
     }
     if (b + 1 < b1) park(b + 1, buf ^ 1);
+    if (b + 1 == b1 || !((b + 1) & (ranges.length - 1))) end_range();  // (a power of two)
   }
-  if (!works || 16 * (wave & 1) + col >= n_tok) return;
-  l = over_groups_sum(l);
-  if (p.splits > 1) {
-    const size_t at = (((size_t)tile * AF_TOKENS + tok) * p.heads + head) * p.splits + blockIdx.y;
+  if (!mine || p.splits > 1) return;
+  sum += sink_term(p, head, top);
 #pragma unroll
-    for (int c = 0; c < C; ++c) *reinterpret_cast<f32x4*>(p.part_o + at * HD + 16 * c + 4 * g) = acc[c];
-    if (g == 0) p.part_ml[2 * at] = m, p.part_ml[2 * at + 1] = l;
-    return;
-  }
-  l += sink_term(p, head, m);
-#pragma unroll
-  for (int c = 0; c < C; ++c) *reinterpret_cast<f32x4*>(p.out + (row * p.heads + head) * HD + 16 * c + 4 * g) = acc[c] / l;
+  for (int c = 0; c < C; ++c) *reinterpret_cast<f32x4*>(p.out + (row * p.heads + head) * HD + 16 * c + 4 * g) = all[c] / sum;
 }
 
 template <int HD>
@@ -271,9 +328,9 @@ __global__ __launch_bounds__(256) void attn_f32_rows_kernel(AttnF32Params p) {
 #pragma unroll
   for (int c = 0; c < C; ++c) q[c] = *reinterpret_cast<const f32x4*>(p.q + row * p.q_stride + head * HD + 16 * c + 4 * g) * p.scale;
 
-  // ranges of keys start at multiples of their length; the first one launched is the one with the first key that the token sees
-  const int range = lo / (16 * p.range_tiles) + blockIdx.y;
-  const int first = range * p.range_tiles + wave, end = min(pos / 16 + 1, (range + 1) * p.range_tiles);
+  const KeyRanges ranges = key_ranges(lo / 16, pos / 16, p.range_tiles, AF_ROWS_RANGES);
+  const int range = ranges.first + blockIdx.y;
+  const int first = range * (int)ranges.length + wave, end = min(pos / 16 + 1, (range + 1) * (int)ranges.length);
   const int mask = (1 << p.page_shift) - 1;
   int kid, vid;
   f32x4 k[2][C], v[2][C];
@@ -369,7 +426,8 @@ __global__ __launch_bounds__(256) void attn_f32_rows_kernel(AttnF32Params p) {
   }
 }
 
-// Adds the ranges of a (tile, token of the tile, head): a wave each, at most 64 ranges.
+// Adds the ranges of a (tile, token of the tile, head): a wave each.  A portion's in their order, as the kernel above does; a single token's, at
+// most 64, by their common maximum.
 __global__ __launch_bounds__(256) void attn_f32_join_kernel(AttnF32Params p, int tokens, int hd) {
   const int lane = threadIdx.x & 63;
   const size_t column = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -377,10 +435,39 @@ __global__ __launch_bounds__(256) void attn_f32_join_kernel(AttnF32Params p, int
   const int head = column % p.heads, tok = column / p.heads % tokens, tile = column / p.heads / tokens;
   const int* info = p.tiles + 8 * tile;
   if (info[1] + tok >= info[3]) return;  // the tile holds fewer tokens
+  const size_t row = (size_t)info[2] + info[1] + tok;
+  if (!p.rows) {
+    const int base = info[4] - info[3] + info[1];
+    const KeyRanges ranges = portion_ranges(p, first_key(p, base), base + min(AF_TOKENS, info[3] - info[1]) - 1);
+    // lane s: range s, the maximum of the ranges before it and its weights
+    const int count = range_count(ranges, base + min(AF_TOKENS, info[3] - info[1]) - 1);
+    const bool has = lane < count;
+    const float m = has ? p.part_ml[2 * (column * p.splits + lane)] : -INFINITY, l = has ? p.part_ml[2 * (column * p.splits + lane) + 1] : 0.f;
+    float top = m;
+    for (int d = 1; d < AF_ROWS_RANGES; d *= 2) {
+      const float before = __shfl_up(top, d, 64);
+      if (lane >= d) top = fmaxf(before, top);
+    }
+    const float before = __shfl_up(top, 1, 64);
+    const RangeWeights w = range_weights(lane ? before : -INFINITY, m);
+    float sum = 0.f, o[2] = {0.f, 0.f};  // (a head is at most 128 channels)
+#pragma unroll 4
+    for (int s = 0; s < count; ++s) {
+      const float old = __shfl(w.old, s, 64), now = __shfl(w.now, s, 64);
+      sum = fmaf(__shfl(l, s, 64), now, sum * old);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (64 * i + lane < hd) o[i] = fmaf(p.part_o[(column * p.splits + s) * hd + 64 * i + lane], now, o[i] * old);
+    }
+    sum += sink_term(p, head, __shfl(top, 63, 64));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (64 * i + lane < hd) p.out[(row * p.heads + head) * hd + 64 * i + lane] = o[i] / sum;
+    return;
+  }
   const float m = lane < p.splits ? p.part_ml[2 * (column * p.splits + lane)] : -INFINITY;
   const float top = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - top);
   const float l = wave_sum(lane < p.splits ? f * p.part_ml[2 * (column * p.splits + lane) + 1] : 0.f) + sink_term(p, head, top);
-  const size_t row = (size_t)info[2] + info[1] + tok;
   for (int d0 = 0; d0 < hd; d0 += 64) {  // (every lane takes part in the exchange, whatever the head size)
     const int d = d0 + lane;
     float o = 0.f;
@@ -393,27 +480,29 @@ __global__ __launch_bounds__(256) void attn_f32_join_kernel(AttnF32Params p, int
 }
 
 template <int HD>
-static void launch_attn_f32(const AttnF32Params& p, int rows, hipStream_t stream) {
+static void launch_attn_f32(const AttnF32Params& p, int groups, hipStream_t stream) {
   const int group = p.heads / p.kv_heads;
-  if (rows)
+  if (p.rows)
     attn_f32_rows_kernel<HD><<<dim3(p.n_tiles * p.kv_heads * ((group + 15) / 16), p.splits), 256, 0, stream>>>(p);
   else
-    attn_f32_kernel<HD><<<dim3(p.n_tiles * p.kv_heads * ((group + 1) / 2), p.splits), 256, 0, stream>>>(p);
+    attn_f32_kernel<HD><<<dim3(p.n_tiles * p.kv_heads * ((group + 1) / 2), groups), 256, 0, stream>>>(p);
   if (p.splits > 1) {
-    const int tokens = rows ? 1 : AF_TOKENS;
+    const int tokens = p.rows ? 1 : AF_TOKENS;
     attn_f32_join_kernel<<<((size_t)p.n_tiles * tokens * p.heads + 3) / 4, 256, 0, stream>>>(p, tokens, HD);
   }
 }
 
-// ``rows`` != 0: the tiles are single tokens, whose keys go in ``splits`` ranges of 16 ``range_tiles`` keys, counted from the range of the first
-// key that the token sees (the caller launches as many as the longest row needs); 0: up to 32 tokens each, keys in ``splits`` equal ranges.  Workspace, when splits > 1 (at most 64): part_o holds n_tiles *
-// (rows ? 1 : 32) * heads * splits * hd floats and part_ml twice as many as there are ranges.
+// ``rows`` != 0: the tiles are single tokens, whose keys go in ranges of 16 ``range_tiles`` keys (or twice as many, ... so that there are at most 64);
+// the caller launches ``splits`` workgroups, as many as the row with the most ranges has, one each.  0: up to 32 tokens each, whose keys
+// go in at most 16 ranges of 256 keys or more; ``splits`` = 1: each tile's ranges by one workgroup, or the number of ranges that the workspace
+// has room for (fewer than 16 only if no tile has more), dealt to ``groups`` workgroups.  Workspace, when splits > 1 (at most 64): part_o holds
+// n_tiles * (rows ? 1 : 32) * heads * splits * hd floats and part_ml twice as many as there are ranges.
 extern "C" int ns_attn_f32(float* out, float* part_o, float* part_ml, const float* q, int q_stride, const float* k_cache, const float* v_cache,
                            const int* tiles, const int* block_table, int table_stride, int n_tiles, int heads, int kv_heads, int hd,
-                           int page_size, int rows, int splits, int range_tiles, float scale, int window, int chunk, float cap, int sink,
+                           int page_size, int rows, int splits, int groups, int range_tiles, float scale, int window, int chunk, float cap, int sink,
                            const float* sink_logit, float slope_exp, hipStream_t stream) {
   if (n_tiles <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || window < 0 || chunk < 0 || cap < 0.f || slope_exp < 0.f ||
-      splits < 1 || splits > 64 || range_tiles < 1 || (splits > 1 && (!part_o || !part_ml)))
+      splits < 1 || splits > AF_ROWS_RANGES || groups < 1 || groups > splits || range_tiles < 1 || (splits > 1 && (!part_o || !part_ml)))
     return NS_ERR_BAD_ARG;
   if (hd % 16 || hd < 16 || hd > 128 || page_size < 4 || page_size & (page_size - 1) || q_stride % 4 ||
       (((uintptr_t)out | (uintptr_t)part_o | (uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15))
@@ -422,16 +511,16 @@ extern "C" int ns_attn_f32(float* out, float* part_o, float* part_ml, const floa
   int shift = 0;
   while (1 << shift < page_size) ++shift;
   const AttnF32Params p{out, part_o, part_ml, q, k_cache, v_cache, tiles, block_table, sink_logit, q_stride, table_stride, heads, kv_heads,
-                        shift, splits, range_tiles, window, chunk, sink, n_tiles, scale, cap, slope_exp};
+                        shift, splits, range_tiles, window, chunk, sink, n_tiles, rows, scale, cap, slope_exp};
   switch (hd) {
-    case 16: launch_attn_f32<16>(p, rows, stream); break;
-    case 32: launch_attn_f32<32>(p, rows, stream); break;
-    case 48: launch_attn_f32<48>(p, rows, stream); break;
-    case 64: launch_attn_f32<64>(p, rows, stream); break;
-    case 80: launch_attn_f32<80>(p, rows, stream); break;
-    case 96: launch_attn_f32<96>(p, rows, stream); break;
-    case 112: launch_attn_f32<112>(p, rows, stream); break;
-    default: launch_attn_f32<128>(p, rows, stream); break;
+    case 16: launch_attn_f32<16>(p, groups, stream); break;
+    case 32: launch_attn_f32<32>(p, groups, stream); break;
+    case 48: launch_attn_f32<48>(p, groups, stream); break;
+    case 64: launch_attn_f32<64>(p, groups, stream); break;
+    case 80: launch_attn_f32<80>(p, groups, stream); break;
+    case 96: launch_attn_f32<96>(p, groups, stream); break;
+    case 112: launch_attn_f32<112>(p, groups, stream); break;
+    default: launch_attn_f32<128>(p, groups, stream); break;
   }
   return ns_launch_status();
 }

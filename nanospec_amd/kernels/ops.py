@@ -697,6 +697,7 @@ def attention_generic(q, out, k_cache, v_cache, token_req, positions, block_tabl
 
 
 F32_ATTENTION_MAX_RANGES = 64
+F32_ATTENTION_PORTION_KEYS, F32_ATTENTION_PORTION_RANGES = 256, 16  # a range of a portion's keys at least, and as many ranges at most
 
 
 def f32_attention_takes(dtype, head_dim: int, v_dim: int, page_size: int) -> bool:
@@ -705,12 +706,15 @@ def f32_attention_takes(dtype, head_dim: int, v_dim: int, page_size: int) -> boo
 
 def attention_f32(q, out, k_cache, v_cache, tiles, block_table, heads: int, kv_heads: int, head_dim: int, scale: float, rows: bool,
                   splits: int = 1, range_keys: int = 0, workspace: tuple[torch.Tensor, torch.Tensor] | None = None, window: int = 0, chunk: int = 0,
-                  cap: float = 0.0, sink: bool = False, slope_exp: float = 0.0, sink_logits: torch.Tensor | None = None) -> torch.Tensor:
+                  cap: float = 0.0, sink: bool = False, slope_exp: float = 0.0, sink_logits: torch.Tensor | None = None,
+                  groups: int | None = None) -> torch.Tensor:
     """32-bit attention on the matrix cores for the tiles described in ``tiles`` (as for ``attention_mfma``): single tokens
-    (``rows``) whose keys go in ``splits`` ranges of ``range_keys`` (a multiple of 16; the ranges start at multiples of it, and the first is
-    the one with the first key that the token sees, so ``splits`` of them have to reach the last key), or up to 32 tokens of a
-    request whose keys are cut into ``splits`` equal ranges.  ``splits`` > 1 needs ``workspace`` = (part_o, part_ml) float32 tensors.  The other
-    arguments: as for ``attention_generic``."""
+    (``rows``) whose keys go in ranges of ``range_keys`` (a multiple of 16; the ranges start at multiples of it, and a token with more than
+    F32_ATTENTION_MAX_RANGES of them has ranges of twice as many keys, ...), of which ``splits`` have to be as many as any token has, or up
+    to 32 tokens of a request whose keys go in ranges of F32_ATTENTION_PORTION_KEYS from key 0 (or twice as many, ...: at most
+    F32_ATTENTION_PORTION_RANGES): with ``splits`` = 1 by one workgroup for a tile, or with room in the workspace for ``splits`` ranges by ``groups``
+    workgroups (``splits`` if None), with the same result if that is F32_ATTENTION_PORTION_RANGES or as many as any tile has.
+    ``splits`` > 1 needs ``workspace`` = (part_o, part_ml) float32 tensors.  The other arguments: as for ``attention_generic``."""
     page = _check_attn(q, out, k_cache, v_cache, heads, kv_heads, head_dim)
     if sink_logits is not None and _f32(sink_logits, "sink_logits").numel() != heads:
         raise KernelRefused(f"attention_f32: sink_logits holds one float32 value for each of the {heads} heads")
@@ -733,7 +737,7 @@ def attention_f32(q, out, k_cache, v_cache, tiles, block_table, heads: int, kv_h
             raise KernelRefused("attention_f32: workspace too small")
     _check(build.core().ns_attn_f32(_ptr(out), _ptr(po), _ptr(pm), _ptr(q), c_int(q.stride(0)), _ptr(k_cache), _ptr(v_cache), _ptr(tiles),
                                     _ptr(block_table), c_int(block_table.stride(0)), c_int(tiles.shape[0]), c_int(heads), c_int(kv_heads),
-                                    c_int(head_dim), c_int(page), c_int(1 if rows else 0), c_int(splits), c_int(range_keys // 16 if rows else 1),
+                                    c_int(head_dim), c_int(page), c_int(1 if rows else 0), c_int(splits), c_int(groups or splits), c_int(range_keys // 16 if rows else 1),
                                     c_float(scale), c_int(window), c_int(chunk), c_float(cap), c_int(1 if sink else 0), _ptr(sink_logits),
                                     c_float(slope_exp), _stream()), "attention_f32")
     return out

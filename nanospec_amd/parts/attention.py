@@ -26,7 +26,6 @@ PORTION_SINGLE_SET_BLOCKS = 128  # 32-key blocks of the longest row from which a
 DECODE_WAVES_PER_UNIT = 4  # decode rows' keys are cut into ranges until about this many waves per compute unit are at work
 LONG_ROW_KEYS = 8192  # rows that may reach this many keys get up to 32 ranges instead of 16
 F32_RANGE_KEYS = 128  # keys of a range of a single token's row in 32-bit: two tiles of 16 for each wave of its workgroup
-F32_PORTION_RANGE_BLOCKS = 4  # the fewest 64-key blocks that a range of a portion's keys is worth a workgroup of its own in 32-bit
 QKV_JOIN_MAX_RANGES = 4  # 17 to 128 rows: the kernel that joins the ranges of the q/k/v product, rotates and writes the cache reads
 #                          every range, so more of them cost it what they gain the product
 
@@ -187,30 +186,31 @@ def f32_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_dim
                   **options) -> torch.Tensor:
     """32-bit attention of the batch's portion tiles and single tokens on the matrix cores (sizes: ``ops.f32_attention_takes``; a block that
     hands on no batch plans has no tiles, and its 32-bit layers run ``ops.attention_generic``, which needs none).
-    A single token's keys go in ranges of ``F32_RANGE_KEYS`` from key 0 whatever else is in the batch, so its result does not
-    depend on it; a portion's are cut only where its tiles leave the GPU idle."""
+    A token's result does not depend on what else is in the batch: its keys go in ranges at fixed places (single tokens: of ``F32_RANGE_KEYS``,
+    portions: of ``ops.F32_ATTENTION_PORTION_KEYS``; longer ones only where it has very many keys itself), which are added in the
+    same way whether one workgroup walks them or, where a portion's tiles leave the GPU idle, several."""
     chunk_tiles, decode_tiles = TilePlan.views(ctx)
     units = ops.compute_units(ctx.token_ids.device)
     span = min(n for n in (window, chunk, 1 << 30) if n)
     group, take = heads // kv_heads, ctx.arena.take
 
-    def launch(tiles, rows: bool, splits: int, range_keys: int = 0) -> None:
+    def launch(tiles, rows: bool, splits: int, **cut) -> None:
         cols = tiles.shape[0] * (1 if rows else TilePlan.TOKENS) * heads
         ws = (take((cols * splits * head_dim,), torch.float32), take((cols * splits * 2,), torch.float32)) if splits > 1 else None
-        ops.attention_f32(q, out, cache.k, cache.v, tiles, table, heads, kv_heads, head_dim, scale, rows=rows, splits=splits, range_keys=range_keys,
-                          workspace=ws, window=window, chunk=chunk, **options)
+        ops.attention_f32(q, out, cache.k, cache.v, tiles, table, heads, kv_heads, head_dim, scale, rows=rows, splits=splits, workspace=ws,
+                          window=window, chunk=chunk, **cut, **options)
 
     if chunk_tiles.shape[0]:
         wgs = chunk_tiles.shape[0] * kv_heads * -(-group // 2)
-        blocks = -(-min(ctx.max_chunk_kv, span + TilePlan.TOKENS) // 64)
-        launch(chunk_tiles, False, max(1, min(16, 2 * units // wgs, blocks // F32_PORTION_RANGE_BLOCKS)))
-    if decode_tiles.shape[0]:
         # (a span of keys may begin anywhere in its first range)
+        seen, edge = (ctx.max_chunk_kv, 0) if ctx.max_chunk_kv <= span + TilePlan.TOKENS else (span + TilePlan.TOKENS, 1)
+        ranges = min(ops.F32_ATTENTION_PORTION_RANGES, -(-seen // ops.F32_ATTENTION_PORTION_KEYS) + edge)
+        # (a second workgroup is worth the joining from two whole ranges on)
+        groups = max(1, min(2 * units // wgs, ranges)) if seen >= 2 * ops.F32_ATTENTION_PORTION_KEYS else 1
+        launch(chunk_tiles, False, ranges if groups > 1 else 1, groups=groups)
+    if decode_tiles.shape[0]:
         longest, edge = (ctx.max_kv_len, 0) if ctx.max_kv_len <= span else (span, 1)
-        range_keys = F32_RANGE_KEYS
-        while -(-longest // range_keys) + edge > ops.F32_ATTENTION_MAX_RANGES:
-            range_keys *= 2
-        launch(decode_tiles, True, -(-longest // range_keys) + edge, range_keys)
+        launch(decode_tiles, True, min(ops.F32_ATTENTION_MAX_RANGES, -(-longest // F32_RANGE_KEYS) + edge), range_keys=F32_RANGE_KEYS)
     return out
 
 

@@ -1068,6 +1068,53 @@ def test_attention_f32(case, option, heads, kvh, hd, page):
     assert rows.numel() and bool((alone[: first[b] + lens[b] - 1] == 7).all())
 
 
+@pytest.mark.parametrize("window", [0, 300])
+@pytest.mark.parametrize("heads,kvh,hd", [(8, 2, 64), (4, 4, 128)])
+def test_attention_f32_does_not_depend_on_the_batch(heads, kvh, hd, window):
+    """32-bit attention of a portion and of a single token, alone and beside others that change the launch (more tiles, longer rows, a
+    table of many more keys): the same bits.  The last portion has so many keys that its ranges grow."""
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from nanospec_amd.engine.context import BatchFacts
+    from nanospec_amd.parts.attention import TilePlan, f32_attention
+
+    torch.manual_seed(hd + window)
+    page, kept = 16, {"portion": (3000, 40), "single": (700, 1), "long": (9900, 70), "far": (8600, 1)}
+    q = {name: torch.randn(l, heads * hd, device=DEV) for name, (_, l) in kept.items()}
+    pages = {name: -(-(s + l) // page) for name, (s, l) in kept.items()}
+    k, v = torch.randn(1400, kvh, page, hd, device=DEV), torch.randn(1400, kvh, hd, page, device=DEV)
+    first_page = dict(zip(kept, np.cumsum([0, *pages.values()])))
+
+    def run(names, others, capacity=None):
+        reqs = [(*kept[n], first_page[n], q[n]) for n in names] + [(s, l, 0, torch.randn(l, heads * hd, device=DEV)) for s, l in others]
+        lens, starts = [r[1] for r in reqs], [r[0] for r in reqs]
+        total = [s + l for s, l in zip(starts, lens)]
+        i32 = lambda x: np.asarray(x, dtype=np.int32)
+        plan, indptr = TilePlan(), np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+        shape = plan.shape(lens)
+        region = np.zeros(plan.ints(shape), dtype=np.int32)
+        plan.fill(region, shape, BatchFacts(sum(lens), len(lens), i32(lens), i32(starts), indptr, i32(total), len(lens), 1))
+        table = torch.zeros(len(reqs), -(-max(total) // page), dtype=torch.int32)
+        for b, r in enumerate(reqs):
+            m = -(-total[b] // page)
+            table[b, :m] = torch.arange(r[2], r[2] + m) % 1400
+        dev = torch.from_numpy(region).to(DEV)
+        ctx = SimpleNamespace(plans={TilePlan.key: (dev, shape)}, arena=SimpleNamespace(take=lambda sh, dt: torch.full(sh, float("nan"), dtype=dt, device=DEV)),
+                              token_ids=dev, max_kv_len=capacity or max(total), max_chunk_kv=capacity or max([t for t, l in zip(total, lens) if l > 1], default=0))
+        x = torch.cat([r[3] for r in reqs])
+        out = f32_attention(ctx, x, torch.empty_like(x), SimpleNamespace(k=k, v=v), table.to(DEV), heads, kvh, hd, hd ** -0.5, window=window)
+        assert torch.isfinite(out).all()
+        return {n: out[indptr[i] : indptr[i + 1]] for i, n in enumerate(names)}
+
+    alone = {n: run([n], [])[n] for n in kept}
+    for others, capacity in (([], None), ([(0, 900)], None), ([(20, 1), (12000, 1)], None), ([(5000, 33), (0, 2000), (300, 1)], None), ([(7, 3)], 32768)):
+        got = run(list(kept), others, capacity)
+        for n in kept:
+            assert torch.equal(got[n], alone[n]), (n, others, capacity)
+
+
 def test_attention_f32_keeps_infinities_to_the_rows_that_see_them():
     """A value that is infinite or no number belongs to the tokens at its position and behind; the others' results are what they
     would be without it.  The same for keys, and for what earlier owners left in a page behind the last key."""

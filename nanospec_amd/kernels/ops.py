@@ -1201,21 +1201,38 @@ def memory_state_floats(heads: int, key_dim: int, value_dim: int) -> int:
 
 # Prompt portions of the matrix memory chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
 # the tokens from which on a request is worth the three launches (8 heads of 128 by 256: 32 tokens 16 us token by token and 18 so, 64 tokens
-# 27 and 19, 40 requests of 48 tokens 145 and 99; what the delta rule loses with few small heads holds here too), and the scratch in bytes that the chunks' records may take (17 KiB a chunk and head at 128 channels; what does not fit goes in several passes).
+# 27 and 19), and the scratch in bytes that the chunks' records may take (17 KiB a chunk and head at 128 channels; what does not fit goes in several passes).
 MEMORY_CHUNK_KEY_DIMS = (64, 128)
 MEMORY_CHUNK_MIN = 64
 MEMORY_CHUNK_SCRATCH = 64 << 20
 
 
+def _longest_and_portions(n: int, reqs: int, longest: int | None, portions: int | None, floor: int) -> tuple[int, int]:
+    """What is not known of a step's requests, from its counts: some request has so many tokens only if the others leave them."""
+    return n - reqs + 1 if longest is None else min(longest, n), min(reqs if portions is None else portions, reqs, n // max(floor, 1))
+
+
+def memory_chunk_min(portions: int, heads: int, key_dim: int) -> int:
+    """Tokens from which on a request of the step goes chunk by chunk.  Many requests keep the GPU busy token by token too; with keys of 64
+    channels that is ahead for short ones (us token by token and by chunks): 32 requests of 64 tokens, 16 heads of 64 by 64: 53 and 55, of
+    96 tokens 74 and 69; 128 requests of 64 tokens 168 and 186, of 96: 231 and 231, of 128: 301 and 298.  8 heads of 128 by 256, 128
+    requests of 64 tokens: 483 and 352."""
+    if key_dim == 64 and portions * heads >= 512:
+        return max(MEMORY_CHUNK_MIN, 128 if portions * heads >= 2048 else 96)
+    return MEMORY_CHUNK_MIN
+
+
 def memory_scan(proj: torch.Tensor, offsets: tuple[int, int, int, int, int], gate_bias_i: torch.Tensor | None, gate_bias_f: torch.Tensor | None,
                 state: torch.Tensor, qo_indptr, state_slots, heads: int, key_dim: int, value_dim: int, cap: float, q_scale: float,
-                out: torch.Tensor, den: torch.Tensor, den_eps: float = 1e-6, take=None) -> torch.Tensor:
+                out: torch.Tensor, den: torch.Tensor, den_eps: float = 1e-6, take=None, longest: int | None = None,
+                portions: int | None = None) -> torch.Tensor:
     """The matrix memory's recurrence over every request's tokens of the step, in order (``csrc/memory.hip``).  A row of
     ``proj`` holds q and k [heads * key_dim], v [heads * value_dim] and the two gate inputs [heads] at the column
     ``offsets`` (q, k, v, input gate, forget gate); ``state`` float32 [slots, >= memory_state_floats].  ``out`` float32
     [tokens, heads * value_dim] receives S^T q and ``den`` float32 [tokens, heads] the denominators max(|n . q|, exp(-m)) +
     den_eps: the read-out is out / den (``gated_rms`` divides as it reads).  ``take(shape, dtype)`` gives scratch: with it, requests of at least
-    MEMORY_CHUNK_MIN tokens go chunk by chunk where the sizes allow it."""
+    ``memory_chunk_min`` tokens go chunk by chunk where the sizes allow it.  ``longest``: the most tokens that a request brings, ``portions``: the
+    most requests that bring more than one (None: not known)."""
     _gpu(proj, state, qo_indptr, state_slots, out, den, gate_bias_i, gate_bias_f)
     _f32(out, "out"), _f32(den, "den"), _i32(qo_indptr, "qo_indptr"), _i32(state_slots, "state_slots")
     n = proj.shape[0]
@@ -1237,10 +1254,10 @@ def memory_scan(proj: torch.Tensor, offsets: tuple[int, int, int, int, int], gat
            _ptr(state), ctypes.c_longlong(state.stride(0)), _ptr(qo_indptr), _ptr(state_slots), _ptr(out), _ptr(den))
     sizes = (c_int(reqs), c_int(heads), c_int(key_dim), c_int(value_dim), c_float(cap), c_float(q_scale), c_float(den_eps))
     below = 0x7FFFFFFF
-    # some request has that many tokens only if the others leave them; in a captured step the counts are all that is known
-    if (take is not None and n - reqs + 1 >= MEMORY_CHUNK_MIN and key_dim in MEMORY_CHUNK_KEY_DIMS and value_dim % 16 == 0
+    longest, portions = _longest_and_portions(n, reqs, longest, portions, MEMORY_CHUNK_MIN)
+    if (take is not None and longest >= memory_chunk_min(portions, heads, key_dim) and key_dim in MEMORY_CHUNK_KEY_DIMS and value_dim % 16 == 0
             and not (proj.stride(0) % 8 or q_off % 8 or k_off % 8 or proj.data_ptr() % (8 * proj.element_size()))):
-        below = MEMORY_CHUNK_MIN
+        below = memory_chunk_min(portions, heads, key_dim)
         record = heads * (32 * key_dim + 276)
         gates = take((4 * n * heads + reqs * heads,), torch.float32)
         scratch = take((min((n // 16 + reqs) * record, max(record, MEMORY_CHUNK_SCRATCH // 4)),), torch.float32)
@@ -1886,11 +1903,26 @@ MAX_CONV_TAPS = 16
 DELTA_MAX_KEY_DIM = 1024
 # Prompt portions of the delta rule chunk by chunk: the key sizes that have kernels (four waves hold D / 64 tiles of 16 channels each),
 # the tokens from which on a request is worth the two launches (16 heads of 128: 16 tokens 11 us token by token, 32 tokens 16.5 and 15.5,
-# 64 tokens 26.6 and 18.4; 64 requests of 32 tokens and 4 heads of 64: 15 and 27, of 16 heads of 128: 204 and 175) and the scratch in bytes that the chunks' records may take (27 KiB a chunk and head at 128 channels, a
+# 64 tokens 26.6 and 18.4) and the scratch in bytes that the chunks' records may take (27 KiB a chunk and head at 128 channels, a
 # prompt of 2,048 tokens of 16 heads in one piece; what does not fit goes in several passes, 8,192 tokens of 32 heads 2,750 -> 970 us).
 DELTA_CHUNK_KEY_DIMS = (64, 128)
 DELTA_CHUNK_MIN = 64
 DELTA_CHUNK_SCRATCH = 64 << 20
+
+
+def delta_chunk_min(portions: int, heads: int, key_dim: int, value_dim: int) -> int:
+    """Tokens from which on a request of the step goes chunk by chunk (more than any has: none does).  Many requests keep the GPU busy
+    token by token too, and the chunks' 64-bit sums then cost more than the shorter chain gives (us token by token and by chunks): keys of 64
+    channels, 4 heads of 64 values, 32 requests of 64 tokens 22 and 25, of 96 tokens 31 and 30, 64 requests of 64 tokens 25 and 39, of
+    256 tokens 78 and 93; 8 heads of 128 values, 8 requests of 64 tokens 23 and 20, 16 requests 26 and 32, 64 requests of 256 tokens 236
+    and 266.  Keys of 128 channels: 128 requests of 64 tokens, 16 heads 626 and 614, 32 heads 1,223 and 1,293, of 128 tokens 2,217 and
+    2,195."""
+    chains = portions * heads
+    if key_dim == 64 and (chains >= 256 or chains * value_dim >= 16384):
+        return 0x7FFFFFFF
+    if key_dim == 64 and chains >= 128:
+        return max(DELTA_CHUNK_MIN, 96)
+    return max(DELTA_CHUNK_MIN, 128) if chains >= 4096 else DELTA_CHUNK_MIN
 
 
 def _state_args(state: torch.Tensor, what: str):
@@ -1946,11 +1978,13 @@ def delta_prep(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, dt_bias: tor
 
 
 def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, qo_indptr, state_slots, heads: int,
-               kv_heads: int, key_dim: int, value_dim: int, out: torch.Tensor, take=None) -> torch.Tensor:
+               kv_heads: int, key_dim: int, value_dim: int, out: torch.Tensor, take=None, longest: int | None = None,
+               portions: int | None = None) -> torch.Tensor:
     """The gated delta rule over every request's tokens of this step, from and into ``state[slot, : heads * key_dim *
     value_dim]`` (S [heads, key_dim, value_dim] per request): S = g_t * S (by key channel); u = beta_t (v_t - S^T k_t);
     S = S + k_t u^T; o_t = S^T q_t.  ``qkv`` as ``delta_prep`` leaves it; ``out`` float32 [tokens, heads * value_dim].
-    ``take(shape, dtype)`` gives scratch: with it, requests of at least DELTA_CHUNK_MIN tokens go chunk by chunk where the sizes allow it."""
+    ``take(shape, dtype)`` gives scratch: with it, requests of at least ``delta_chunk_min`` tokens go chunk by chunk where the sizes allow it.
+    ``longest``: the most tokens that a request brings, ``portions``: the most requests that bring more than one (None: not known)."""
     _f32(qkv, "qkv"), _f32(g, "g"), _f32(beta, "beta"), _f32(out, "out")
     _i32(qo_indptr, "qo_indptr"), _i32(state_slots, "state_slots")
     n, reqs = qkv.shape[0], state_slots.numel()
@@ -1961,10 +1995,10 @@ def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: to
         raise KernelRefused("delta_scan: operands do not fit heads, key size and value size")
     sp, stride = _state_args(state, "delta_scan")
     below = 0x7FFFFFFF
-    # some request has that many tokens only if the others leave them; in a captured step the counts are all that is known
-    if (take is not None and n - reqs + 1 >= DELTA_CHUNK_MIN and key_dim in DELTA_CHUNK_KEY_DIMS and value_dim % 16 == 0 and C % 4 == 0
+    longest, portions = _longest_and_portions(n, reqs, longest, portions, DELTA_CHUNK_MIN)
+    if (take is not None and longest >= delta_chunk_min(portions, heads, key_dim, value_dim) and key_dim in DELTA_CHUNK_KEY_DIMS and value_dim % 16 == 0 and C % 4 == 0
             and not (qkv.data_ptr() | g.data_ptr()) % 16):
-        below = DELTA_CHUNK_MIN
+        below = delta_chunk_min(portions, heads, key_dim, value_dim)
         record = heads * (49 * key_dim + 512)
         scratch = take((min((n // 16 + reqs) * record, max(record, DELTA_CHUNK_SCRATCH // 4)),), torch.float32)
         _check(build.core().ns_delta_chunks(_ptr(out), _ptr(qkv), c_int(C), _ptr(g), _ptr(beta), sp, stride, _ptr(qo_indptr), _ptr(state_slots),

@@ -1323,6 +1323,37 @@ def test_delta_rule_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
             assert not torch.isfinite(out[21]).all()
 
 
+@pytest.mark.parametrize("D,lens,longest,chunks", [(64, [63, 63], 63, False), (64, [63, 64], 64, True), (128, [40, 40], 40, False), (64, [64] * 128, 64, False),
+                                                  (128, [64] * 16, 64, True), (64, [40, 90], None, True)])
+def test_recurrences_by_chunks_where_a_request_is_long_enough(D, lens, longest, chunks):
+    """Chunks are launched where a request has the tokens that they are worth, told by the step's longest request; many requests with
+    small heads stay token by token."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(D)
+    H, E, n, B = 2, 16, sum(lens), len(lens)
+    indptr, slots = torch.tensor([0, *lens]).cumsum(0).to(torch.int32).to(DEV), torch.arange(B, dtype=torch.int32, device=DEV)
+    taken = []
+
+    def take(shape, dtype):
+        taken.append(shape)
+        return torch.empty(shape, dtype=dtype, device=DEV)
+
+    def scans(**kw):
+        qkv, g, beta = torch.randn(n, 2 * H * D + H * E, generator=gen) * 0.1, torch.rand(n, H * D, generator=gen), torch.rand(n, H, generator=gen)
+        ops.delta_scan(qkv.to(DEV), g.to(DEV), beta.to(DEV), torch.zeros(B, H * D * E, device=DEV), indptr, slots, H, H, D, E,
+                       out=torch.empty(n, H * E, device=DEV), take=take, **kw)
+        yield bool(taken)
+        taken.clear()
+        at = (0, H * D, 2 * H * D, 2 * H * D + H * E, 2 * H * D + H * E + H)
+        proj = torch.randn(n, -(-(at[4] + H) // 8) * 8, generator=gen).to(DEV)
+        ops.memory_scan(proj, at, None, None, torch.zeros(B, ops.memory_state_floats(H, D, E), device=DEV), indptr, slots, H, D, E, 15.0, D ** -0.5,
+                        torch.empty(n, H * E, device=DEV), torch.empty(n, H, device=DEV), take=take, **kw)
+        yield bool(taken)
+
+    delta, memory = scans(longest=longest, portions=None if longest is None else B)
+    assert delta == chunks and memory == (chunks or B == 128)  # (the memory's chunks are ahead at 128 requests of two heads)
+
+
 def test_matrix_memory_by_chunks_keeps_infinities_to_later_tokens(monkeypatch):
     """An infinity or NaN at one token, in any of its inputs, reaches neither the tokens before it nor other requests."""
     ops = _ops()

@@ -33,6 +33,14 @@ from .needs import PagedNeed
 EXPAND_TOKENS, EXPAND_TOKENS_EACH = 128, 64
 EXPAND_KEYS_PER_TOKEN = 16  # keys, at most, that a portion's tokens may find for each of them
 EXPAND_SCRATCH = 1 << 30  # bytes of scratch for them, at most
+# How far the wide form is behind goes by its products a (query, key) pair and head over this one's, (2 C + R) / (D + R + E): 6.6 at those
+# sizes, 3.4 at heads of 128 + 64 and 128, 1.8 at 64 + 32 and 64 over a latent of 128.  Below EXPAND_CLEAR, tiles too few for the GPU (one
+# workgroup each walks all keys, where the wide form cuts them) and many keys are slower: 512 tokens at 7,000 keys, 8 heads over 128: 120 us,
+# wide 111; 128 tokens at 1,900: 41 and 38; at 512 keys 21 and 33.
+EXPAND_CLEAR, EXPAND_FULL, EXPAND_KEYS_FEW = 3.0, 256, 5
+# Beside single tokens an eager step forms the wide form's queries and outputs for every row all the same, and only the attention itself
+# counts: 4 portions of 64 tokens, 16 heads of 128 + 64 over 512: 29 us, wide 21; 128 tokens, 8 heads over 128: 13.3 and 12.7, 300 tokens 16.5 and 20.
+EXPAND_BESIDE = 400  # tokens each, times the factor
 
 
 class LatentAttention:
@@ -165,16 +173,22 @@ class LatentAttention:
                               sink_logits=self.sink_logits)
         return self.wo(att, out=out if out is not None else take((n, s.hidden), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)
 
-
     def _expands(self, ctx, n: int, cache) -> tuple[int, int]:
         """Whether the step's prompt portions run over keys and values made from the latents: (portions, blocks of 64 keys of the longest, an
         even number), or (0, 0)."""
+        s = self.spec
         chunk_tiles, decode_tiles = TilePlan.views(ctx)
         singles, page, keys = decode_tiles.shape[0], cache.k.shape[2], ctx.max_chunk_kv
         count = min(ctx.n_reqs - singles, chunk_tiles.shape[0])  # (a captured step counts the request that owns its padding too)
         tokens, blocks = n - singles, -(-keys // 128) * 2
-        if (not self._block or not count or page & (page - 1) or tokens < EXPAND_TOKENS or (not ctx.captured and tokens < EXPAND_TOKENS_EACH * count)
-                or keys > EXPAND_KEYS_PER_TOKEN * tokens or 2 * count * blocks * self._block > EXPAND_SCRATCH):
+        if not self._block or not count or page & (page - 1) or tokens < EXPAND_TOKENS or 2 * count * blocks * self._block > EXPAND_SCRATCH:
+            return 0, 0
+        each = tokens if ctx.captured else tokens / count
+        factor = (2 * s.kv_rank + s.rot_dim) / (s.head_dim + s.rot_dim + s.value_dim)
+        few = factor < EXPAND_CLEAR and -(-tokens // 64) * s.heads < EXPAND_FULL
+        if each < EXPAND_TOKENS_EACH or keys > (EXPAND_KEYS_FEW if few else EXPAND_KEYS_PER_TOKEN) * tokens:
+            return 0, 0
+        if singles and (each * factor < EXPAND_BESIDE or (s.window and factor < 1.5)):
             return 0, 0
         return count, blocks
 

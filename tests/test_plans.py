@@ -49,3 +49,38 @@ def test_many_rows_in_blocks():
     assert nt == 4 and ksplit == 1  # 32 groups of row tiles times 16 blocks of rows fill the GPU without cutting K
     ksplit, nt = ops.rows_plan(4096, 14336, 130, gated=False, units=UNITS)
     assert nt == 4 and ksplit >= 2
+
+
+def expands(lens, kv, sizes, window=0, captured=False):
+    """What ``LatentAttention._expands`` says of a step of these requests: (portions, blocks of 64 keys)."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from nanospec_amd.parts.attention import TILES, TilePlan
+    from nanospec_amd.parts.latent import LatentAttention
+
+    H, D, R, E, C = sizes
+    shape = TILES.shape(lens)
+    part = object.__new__(LatentAttention)
+    part.spec, part._block = SimpleNamespace(heads=H, head_dim=D, rot_dim=R, value_dim=E, kv_rank=C, window=window), H * 64 * (D + R + E)
+    ctx = SimpleNamespace(plans={TilePlan.key: (torch.zeros(TILES.ints(shape), dtype=torch.int32), shape)}, n_reqs=len(lens), captured=captured,
+                          max_chunk_kv=max(k for k, n in zip(kv, lens) if n > 1) if any(n > 1 for n in lens) else 0)
+    return part._expands(ctx, sum(lens), SimpleNamespace(k=torch.zeros(1, 1, 16, C + R)))
+
+
+def test_where_latent_portions_have_keys_and_values_made():
+    """By the portions' tokens, the keys they find, how far the wide form is behind at these sizes, and whether it has to be formed for
+    single tokens all the same."""
+    wide, middle, near = (32, 64, 32, 64, 512), (16, 128, 64, 128, 512), (8, 64, 32, 64, 128)
+    assert expands([127], [127], wide) == (0, 0) and expands([128], [128], wide) == (1, 2) and expands([128], [2028], wide) == (1, 32)
+    assert expands([128], [2049], wide) == (0, 0)
+    assert expands([60] * 4, [60] * 4, wide) == (0, 0) and expands([64] * 4, [64] * 4, wide) == (4, 2)
+    # a latent of 128: few tiles and many keys stay with the wide form, which cuts the keys
+    assert expands([512], [7512], near) == (0, 0) and expands([128], [640], near) == (1, 10) and expands([2048], [10048], near) == (1, 158)
+    # beside single tokens
+    assert expands([64, 64, 64, 64, 1], [64, 64, 64, 64, 9], wide) == (4, 2)
+    assert expands([64, 64, 64, 64], [64] * 4, middle) == (4, 2) and expands([64, 64, 64, 64, 1], [64, 64, 64, 64, 9], middle) == (0, 0)
+    assert expands([128, 1], [128, 9], near) == (0, 0) and expands([300, 1], [300, 9], near) == (1, 6)
+    # a captured step knows its tokens and the keys that its tables can name
+    assert expands([512, 1], [1024, 9], wide, captured=True) == (1, 16)

@@ -37,8 +37,9 @@ class TilePlan:
     request's first token, tokens of the request in this step, keys after this step, for one-token tiles the keys that
     all of them read in this step over all layers (by which the kernel chooses its loads: what cannot stay cached until
     the next step is read past the caches); for portion tiles the number of their portion in the seventh int, and in the eighth,
-    whichever tile it stands in, as the p-th one of them the number of portion p's first tile (-1 behind the last portion).  shape = (portion tiles, one-token tiles); a region of a fixed shape may hold
-    more portion tiles than the batch needs: the rest bring no tokens and the kernel skips them."""
+    whichever tile it stands in, as the p-th one of them the number of portion p's first tile (-1 behind the last portion that brings
+    tokens).  shape = (portion tiles, one-token tiles); a region of a fixed shape may hold more portion tiles than the batch needs: the
+    rest bring no tokens and the kernel skips them."""
 
     key = "attention.tiles"
     TOKENS = 32
@@ -57,7 +58,7 @@ class TilePlan:
         tc, td = shape
         lens, indptr, kv, n = facts.lens, facts.indptr, facts.kv, facts.covered
         if tc:
-            many = [b for b in range(n) if lens[b] != 1]
+            many = [b for b in range(n) if lens[b] > 1]  # (a captured step's unused portions bring none)
             rows = [(b, t0, indptr[b], lens[b], kv[b], 0, p, -1) for p, b in enumerate(many) for t0 in range(0, lens[b], self.TOKENS)]
             rows += [(facts.n_reqs - 1, 0, 0, 0, 0, 0, 0, -1)] * (tc - len(rows))  # tiles without tokens
             tiles = np.asarray(rows, dtype=np.int32)

@@ -84,3 +84,31 @@ def test_where_latent_portions_have_keys_and_values_made():
     assert expands([128, 1], [128, 9], near) == (0, 0) and expands([300, 1], [300, 9], near) == (1, 6)
     # a captured step knows its tokens and the keys that its tables can name
     assert expands([512, 1], [1024, 9], wide, captured=True) == (1, 16)
+
+
+@pytest.mark.parametrize("lens,unused,spare", [([40, 1, 2, 65], 0, 0), ([40, 1], 3, 4), ([1, 1, 33], 1, 1), ([1], 4, 3)])
+def test_tiles_number_the_portions_that_bring_tokens(lens, unused, spare):
+    """The tile list of a batch whose fixed shape has room for more portions and more tiles: a portion's tiles carry its number, the p-th
+    tile's last int is portion p's first tile, and nothing is said of portions without tokens."""
+    import numpy as np
+
+    from nanospec_amd.engine.context import BatchFacts
+    from nanospec_amd.parts.attention import TILES
+
+    all_lens = lens + [0] * unused + [7]  # (the last request is the stand-in that owns the padding)
+    i32 = lambda x: np.asarray(x, dtype=np.int32)
+    shape = TILES.shape(lens)
+    shape = (shape[0] + spare, shape[1])
+    starts = [10 * b for b in range(len(lens))] + [0] * (unused + 1)
+    indptr = i32(np.concatenate(([0], np.cumsum(all_lens))))
+    out = np.full(TILES.ints(shape), -5, dtype=np.int32)
+    TILES.fill(out, shape, BatchFacts(sum(all_lens), len(all_lens), i32(all_lens), i32(starts), indptr, i32(starts) + i32(all_lens), len(all_lens) - 1, 1))
+    tiles = out[: 8 * shape[0]].reshape(-1, 8)
+    many = [b for b, n in enumerate(lens) if n > 1]
+    at = 0
+    for p, b in enumerate(many):
+        assert tiles[p, 7] == at
+        for t0 in range(0, lens[b], 32):
+            assert tuple(tiles[at, :7]) == (b, t0, indptr[b], lens[b], starts[b] + lens[b], 0, p)
+            at += 1
+    assert (tiles[at:, 1:7] == 0).all() and (tiles[len(many) :, 7] == -1).all()

@@ -71,6 +71,52 @@ def replay(model, steps, where, ref, dtype, max_tokens, page, graphs=True, loose
     return rep
 
 
+def counted(monkeypatch, owner, name):
+    """-> a list that grows by one with every call of ``owner.name``."""
+    calls, real = [], getattr(owner, name)
+
+    def call(*args, **kw):
+        calls.append(1)
+        return real(*args, **kw)
+
+    monkeypatch.setattr(owner, name, call)
+    return calls
+
+
+def in_long_portions(model, seqs, ref, check, page, graphs, calls):
+    """Prompts in portions that are long enough for the kernels of many tokens, beside decoded tokens and beside each other, first ones and
+    later ones, with decoding and short portions in between, by captured steps (whose shapes are filled in different ways) or by eager
+    ones (single tokens anywhere among the portions).  ``seqs``: a short sequence "s" and long ones "l" (at least 400 tokens) and "m" (at
+    least 260).  ``check(logits, plain rows, what)`` compares; ``calls`` (see ``counted``) grows where the kernels are meant to run."""
+    from nanospec_amd.engine.replay import Replayer
+
+    steps = [  # (request, sequence, from, to), and whether the kernels are meant to run where the step is not captured
+        ([("d", "s", 0, 20)], False),
+        ([("a", "l", 0, 250), ("d", "s", 20, 21)], True),
+        ([("d", "s", 21, 22), ("a", "l", 250, 251)], False),
+        ([("b", "m", 0, 240), ("d", "s", 22, 23), ("a", "l", 251, 252), ("c", "l", 0, 256)], True),
+        ([("b", "m", 240, 243), ("d", "s", 23, 24), ("c", "l", 256, 257)], False),
+        ([("b", "m", 243, 244), ("a", "l", 252, 390), ("c", "l", 257, 397)], None),
+        ([("a", "l", 390, 391), ("b", "m", 244, 245), ("c", "l", 397, 400)], False),
+        ([("e", "l", 0, 400)], True),
+        ([("d", "s", 24, 25), ("a", "l", 391, 392), ("b", "m", 245, 260)], False),
+        ([("f", "l", 0, 230), ("d", "s", 25, 26), ("g", "m", 0, 260), ("a", "l", 392, 393)], True),
+        ([("f", "l", 230, 231), ("d", "s", 26, 27)], False),
+    ]
+    rep = Replayer(model, 4096, page_size=page, use_graphs=graphs)
+    for i, (step, runs) in enumerate(steps * 2):  # (the second time all captured steps are there)
+        before, turn = len(calls), i // len(steps)
+        entries = [{"id": f"{rid}{turn}", "tokens": seqs[name][a:b], "want": sorted({0, b - a - 1})} for rid, name, a, b in step]
+        out = rep.step(entries, [f"{rid}{turn}" for rid, name, a, b in step if b == len(seqs[name])])
+        assert rep.runner.last_used_graph == graphs
+        if runs is not None and not graphs:
+            assert (len(calls) > before) == runs, (i, step)
+        rows = [ref[name][p] for rid, name, a, b in step for p in sorted({a, b - 1})]
+        check(out, torch.stack(rows), (i, step))
+    assert calls
+    rep.manager.check()
+
+
 def batch(lens, slots):
     """Device arrays of a step's batch for hand-made requests: (token_req, qo_indptr, state_slots)."""
     req = torch.tensor([b for b, n in enumerate(lens) for _ in range(n)], dtype=torch.int32, device=DEV)

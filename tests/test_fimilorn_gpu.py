@@ -13,7 +13,7 @@ import torch
 
 import plain_fimilorn as pf
 import traces
-from harness import batch, close, paged, replay, step_context
+from harness import batch, close, counted, in_long_portions, paged, replay, step_context
 from tiny import random_tokens
 
 pytestmark = pytest.mark.gpu
@@ -65,6 +65,7 @@ def layer(mixer, mlp):
 # B: one head everywhere, one expert of one, a group of one expert each, no loop, a window of 5, the whole head rotated, no
 #    rotation at all in the retention layer, a decay of 1.
 # C: sizes the matrix-core kernels take in bfloat16, keys and values of one size, all layers run twice, all experts chosen.
+# D: latent layers whose long prompt portions have keys and values of their own made (with a window and without).
 CONFIGS = {
     "A": dict(cfg={"architecture": "Fimilorn", "vocab": 300, "width": 90, "norm": {"eps": 1e-5}, "loop": {"start": 1, "stop": 3, "times": 3},
                    "layers": [layer(attn(6, 2, 20, 14, 12, 0.3, base=5000.0), dense(50, 0.7)),
@@ -83,6 +84,10 @@ CONFIGS = {
                               layer(latent(4, 32, 32, 64, 96, 0.15, 40), dense(256, 1.0)),
                               layer(reten(4, 32, 64, 32, (0.9, 0.95, 0.99, 0.999)), moe(16, 3, 32, groups=(4, 2), shared=64))]},
               seed=5, page=16, lengths=(5, 31, 64, 100, 260)),
+    "D": dict(cfg={"architecture": "Fimilorn", "vocab": 200, "width": 128, "norm": {"eps": 1e-5},
+                   "layers": [layer(latent(4, 64, 32, 64, 128, 0.12, 100), dense(128, 1.0)),
+                              layer(latent(8, 64, 32, 64, 128, 0.1, None), moe(8, 2, 64, shared=64))]},
+              seed=6, page=16, lengths=(3, 27, 130, 260, 400)),
 }
 # what random weights of the usual law leave so small that soft-maxes are flat, gates constant, clips idle and sinks weightless
 SHARPEN = {"q.norm": 2.0, "k.norm": 2.0, "mix.sink": 10.0, "router": 10.0, "correction": 4.0, ".gate": 4.0, ".up": 4.0, "mix.g": 8.0,
@@ -230,6 +235,20 @@ def test_one_position_however_it_is_reached(folders, name, dtype):
     tol = 2e-5 if dtype == torch.float32 else 0.05
     for g in got[1:]:
         assert (g - got[0]).abs().max() <= tol * got[0].abs().max()
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["eager", "captured"])
+def test_long_portions_of_latent_layers(folders, monkeypatch, graphs):
+    """Portions over keys and values made from the latents, beside single tokens over the latents themselves, and one after the other for
+    the same request."""
+    from nanospec_amd.kernels import ops
+
+    dtype, loose = torch.bfloat16, []
+    model, have, ref = engine_model(folders["D"], "D", dtype), sequences("D"), plain_logits(folders["D"], "D", dtype)
+    names = {"s": "r1", "m": "r3", "l": "r4"}
+    in_long_portions(model, {k: have[r] for k, r in names.items()}, {k: ref[r] for k, r in names.items()},
+                     lambda got, want, what: close(got, want, dtype, what, loose), CONFIGS["D"]["page"], graphs, counted(monkeypatch, ops, "latent_prompt"))
+    assert len(loose) <= 8, loose  # (of 82 rows, each counted twice: a token may take another expert)
 
 
 def test_long_decoding_keeps_the_state(folders):

@@ -12,6 +12,7 @@ import torch
 
 import plain_vuzelix as pv
 import traces
+from harness import counted, in_long_portions
 from tiny import random_tokens
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +40,7 @@ def attn_layer(heads, kv_heads, dim, vdim, scale, ff, softcap=None, chunk=None, 
 # Q: one plain stream (no hyper-connection tensors), multiplier and scales of 1, one head, one tap, chunks of 8 tokens (an
 #    edge every half page), no caps.
 # R: a single hyper-connected stream, two streams' worth of nothing else special: many small heads, five taps, all keys seen.
+# S: delta layers whose long prompt portions go chunk by chunk, with keys of 64 and of 128 channels.
 CONFIGS = {
     "P": dict(cfg={"architecture": "Vuzelix", "vocab": 300, "width": 96, "embedding": {"scale": 2.0}, "norm": {"eps": 1e-5},
                    "residual_mult": 0.5, "streams": 3, "logit_softcap": 10.0,
@@ -59,6 +61,12 @@ CONFIGS = {
                               attn_layer(8, 8, 16, 32, 0.25, 128),
                               attn_layer(8, 8, 16, 32, 0.5, 64, kv_from=1)]},
               ranks=(16, 4), seed=5, page=4, lengths=(5, 31, 64, 100)),
+    "S": dict(cfg={"architecture": "Vuzelix", "vocab": 200, "width": 128, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-5},
+                   "residual_mult": 0.7, "streams": 2,
+                   "layers": [delta_layer(2, 1, 64, 16, 4, 128),
+                              attn_layer(4, 2, 32, 32, 0.2, 128),
+                              delta_layer(2, 2, 128, 32, 3, None)]},
+              ranks=(16, 8), seed=6, page=16, lengths=(5, 27, 100, 260, 400)),
 }
 
 
@@ -210,6 +218,19 @@ def test_one_position_however_it_is_reached(folders, dtype):
     tol = 2e-5 if dtype == torch.float32 else 0.05
     for g in got[1:]:
         assert (g - got[0]).abs().max() <= tol * got[0].abs().max()
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["eager", "captured"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_long_portions_of_delta_layers(folders, monkeypatch, dtype, graphs):
+    """Portions that go chunk by chunk, beside single tokens and short portions that go token by token, and one after the other for the
+    same request's state."""
+    from nanospec_amd.kernels import build
+
+    model, have, ref = engine_model(folders["S"], "S", dtype), sequences("S"), plain_logits(folders["S"], "S", dtype)
+    names = {"s": "r1", "m": "r3", "l": "r4"}
+    in_long_portions(model, {k: have[r] for k, r in names.items()}, {k: ref[r] for k, r in names.items()},
+                     lambda got, want, what: close(got.float().cpu(), want, dtype, what), CONFIGS["S"]["page"], graphs, counted(monkeypatch, build.core(), "ns_delta_chunks"))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])

@@ -12,7 +12,7 @@ import torch
 
 import plain_zipedra as pz
 import traces
-from harness import batch, close, paged, replay, step_context
+from harness import batch, close, counted, in_long_portions, paged, replay, step_context
 from tiny import random_tokens
 
 pytestmark = pytest.mark.gpu
@@ -48,6 +48,7 @@ def layer(mixer, mlp):
 # B: one head everywhere, one expert of one, no loop and no token input (both sublayers' outputs wait for the next layer's
 #    read), no logit scale, one rotated pair, a head that never forgets.
 # C: sizes the matrix-core kernels take in bfloat16, all layers run twice, all experts chosen in one of them.
+# D: latent layers whose long prompt portions have keys and values of their own made (both sets of sizes).
 CONFIGS = {
     "A": dict(cfg={"architecture": "Zipedra", "vocab": 300, "width": 90, "norm": {"eps": 1e-5}, "logit_scale": 0.5, "token_side": {"dim": 7},
                    "loop": {"start": 1, "stop": 3, "times": 3},
@@ -67,6 +68,10 @@ CONFIGS = {
                               layer(lightning(4, 32, 48, (0.9, 0.95, 0.99, 0.999)), dense(256)),
                               layer(lightning(2, 64, 32, (0.8, 0.97)), moe(16, 3, 32, shared=64))]},
               seed=5, page=16, lengths=(5, 31, 64, 100, 260)),
+    "D": dict(cfg={"architecture": "Zipedra", "vocab": 200, "width": 128, "norm": {"eps": 1e-5}, "logit_scale": 2.0,
+                   "layers": [layer(latent(4, 64, 32, 64, 128, 0.15, base=1e6), moe(8, 2, 64, shared=96)),
+                              layer(latent(2, 128, 64, 128, 128, 0.1), dense(256))]},
+              seed=6, page=16, lengths=(3, 27, 130, 260, 400)),
 }
 # what random weights of the usual law leave so small that soft-maxes are flat, gates constant and SiLUs linear (the first
 # tail of a name that fits)
@@ -265,6 +270,20 @@ def test_long_portions_beside_decoded_tokens_through_captured_steps(folders, dty
             close(out, torch.stack([ref["r3"][at], ref["r4"][a], ref["r4"][b - 1]]), dtype, (trial, a, b), loose)
             at, rows = at + 1, rows + 3
     assert len(loose) <= max(2, rows // 10), loose
+
+
+@pytest.mark.parametrize("graphs", [False, True], ids=["eager", "captured"])
+def test_long_portions_of_latent_layers(folders, monkeypatch, graphs):
+    """Portions over keys and values made from the latents, beside single tokens over the latents themselves, and one after the other for
+    the same request."""
+    from nanospec_amd.kernels import ops
+
+    dtype, loose = torch.bfloat16, []
+    model, have, ref = engine_model(folders["D"], "D", dtype), sequences("D"), plain_logits(folders["D"], "D", dtype)
+    names = {"s": "r1", "m": "r3", "l": "r4"}
+    in_long_portions(model, {k: have[r] for k, r in names.items()}, {k: ref[r] for k, r in names.items()},
+                     lambda got, want, what: close(got, want, dtype, what, loose), CONFIGS["D"]["page"], graphs, counted(monkeypatch, ops, "latent_prompt"))
+    assert len(loose) <= 8, loose  # (of 82 rows, each counted twice: a token may take another expert)
 
 
 def test_long_decoding_keeps_the_state(folders):

@@ -507,7 +507,7 @@ extern "C" int ns_attn_f32(float* out, float* part_o, float* part_ml, const floa
   if (hd % 16 || hd < 16 || hd > 128 || page_size < 4 || page_size & (page_size - 1) || q_stride % 4 ||
       (((uintptr_t)out | (uintptr_t)part_o | (uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15))
     return NS_ERR_UNSUPPORTED;
-  if ((long)n_tiles * kv_heads * heads * AF_TOKENS > 0x7fffffffL) return NS_ERR_BAD_ARG;
+  if ((long)n_tiles * heads * AF_TOKENS > 0x7fffffffL) return NS_ERR_BAD_ARG;
   int shift = 0;
   while (1 << shift < page_size) ++shift;
   const AttnF32Params p{out, part_o, part_ml, q, k_cache, v_cache, tiles, block_table, sink_logit, q_stride, table_stride, heads, kv_heads,

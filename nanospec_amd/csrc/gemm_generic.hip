@@ -150,6 +150,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 4) void gemm_rows_f32_kernel(float
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define G32_K 64
 #define G32_LD (G32_K + 8)
+#define G32_MAX_BLOCKS 0xffffffL  // workgroups of 256 threads that one dimension of a launch holds
 
 // ENDS: the loop is asked for its end at every stage, not every 2 DEPTH of them; same sums.
 template <int TM, int TN, int DEPTH, bool ENDS>
@@ -246,7 +247,7 @@ template <int TM, int TN, int DEPTH>
 static int launch_gemm_f32(float* out, const float* x, const float* w, int M, int N, int K, int x_stride, int out_stride, hipStream_t stream) {
   const int m_tiles = (M + TM - 1) / TM, n_tiles = (N + TN - 1) / TN;
   const long blocks = (long)m_tiles * ((n_tiles + 7) / 8 * 8);
-  if (blocks > 0x7fffffffL) return NS_ERR_BAD_ARG;
+  if (blocks > G32_MAX_BLOCKS) return NS_ERR_BAD_ARG;
   // Asking at every stage costs a long K up to 15% (777 rows, N 2,048, K 8,192: 273 -> 325 us) and saves a short one the stages of zeros behind
   // its last (2,048 rows, N 2,048, K 64: 45 -> 18 us): it pays where they are more than a fifth of the others.
   const int stages = (K + G32_K - 1) / G32_K, zeros = (2 * DEPTH - stages % (2 * DEPTH)) % (2 * DEPTH);
@@ -261,7 +262,10 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
   if (M <= 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N) return NS_ERR_BAD_ARG;
   dim3 grid((N + GT_N - 1) / GT_N, (M + GT_M - 1) / GT_M);
   if (grid.y > 65535) return NS_ERR_BAD_ARG;
-  if (dtype == NS_DTYPE_F32 && K % 4 == 0 && x_stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
+  // (more tiles of 32 x 32, in groups of eight, or of eight rows of w than one dimension of a launch holds: the plain kernel, which has two)
+  const long tiles = (long)((M + 31) / 32) * (((long)N + 255) / 256 * 8);
+  if (dtype == NS_DTYPE_F32 && K % 4 == 0 && x_stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && tiles <= G32_MAX_BLOCKS &&
+      N < (1 << 26)) {
     float* o = (float*)out;
     const float *xf = (const float*)x, *wf = (const float*)w;
     if (M <= ROWS_M) {

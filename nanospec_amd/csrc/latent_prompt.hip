@@ -9,7 +9,8 @@
 //     into scratch laid out as the attention reads it: [portion][block of 64 keys][head]{ keys [64][D + R] | values [E][64] }, a
 //     channel's keys in the order in which the lanes hold weights (within 32 keys, key 16 t + 4 g + i at place 8 g + 4 t + i).  A wave takes 32
 //     keys of a head through both matrices; a fragment of the latents serves both as either operand.  Bound by the matrices' and
-//     latents' way from L2 (each wave reading the matrices itself: 42 us for 2,048 keys, 32 heads, latent 512; through LDS: 20 us).
+//     latents' way from L2 (each wave reading the matrices itself: 42 us for 2,048 keys, 32 heads, latent 512; through LDS: 20 us, and 29
+//     in a prompt, where the matrices come from memory).
 //   latent_prompt_kernel: a workgroup is 64 tokens of a head, a wave 16; a block of 64 keys and values is contiguous in the
 //     scratch and goes through LDS, two buffers, the next one on its way in registers.  S^T = K Q^T and O^T = V^T P^T on
 //     v_mfma_f32_16x16x32_bf16, so a token's scores, maximum and sums are its own lanes'.  Queries are rotated as they are read; the

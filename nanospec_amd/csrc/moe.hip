@@ -422,7 +422,7 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 // and 128 output channels and multiplies on the matrix cores (v_mfma_f32_16x16x32_bf16): its four waves own 64 x 64 each
 // (every second block of 16 rows), operands come through LDS in pieces of 64 along K, the next piece is fetched into registers
 // while the current one is multiplied.  The host never learns which experts were chosen: the launch has as many tiles as any
-// choice can need (pairs / 128 + experts), and a tile without rows returns.
+// choice can need (pairs / 128 or 16 + experts), and a tile without rows returns.
 // Bound by the matrices' bytes up to some hundred tokens (300: 104 us of which the 403 MB take 82 at a large copy's rate), by what
 // a compute unit takes in from L2 beyond.  32 experts of 1,024, width 2,048, four a token, sorting included: 1,024 tokens 212 -> 146 us,
 // 2,048 tokens 311 -> 237 us (even tiles, blocks without rows skipped, LDS rows without bank conflicts, the sort's scan).

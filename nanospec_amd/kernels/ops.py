@@ -261,7 +261,7 @@ def _check_linear(x, w, out, out_f32):
 
 
 def linear_generic(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, out_f32: bool = False) -> torch.Tensor:
-    """x @ w.T with the plain tiled kernel: any sizes, float32 or bfloat16, 32-bit accumulation in a fixed order."""
+    """x @ w.T by the kernels of ``csrc/gemm_generic.hip``: any sizes, float32 or bfloat16, 32-bit accumulation in a fixed order."""
     out = _check_linear(x, w, out, out_f32)
     m, k = x.shape
     _check(build.core().ns_gemm_generic(_ptr(out), _ptr(x), _ptr(w), c_int(m), c_int(w.shape[0]), c_int(k), c_int(x.stride(0)),

@@ -1,7 +1,8 @@
 """x @ W^T for the parts: ``LinearWeight`` holds a weight matrix and chooses the kernel by precision and row count.
 
-float32: always the plain tiled kernel with 32-bit fused multiply-adds in a fixed order (the true 32-bit path; no
-matrix-core mode of reduced precision is ever used).
+float32: always ``csrc/gemm_generic.hip``, 32-bit products and sums in a fixed order (the true 32-bit path; no matrix-core
+mode of reduced precision is ever used): up to 8 rows stream the weights, more run the 32-bit matrix instruction, odd sizes the
+plain tiled kernel.
 
 bfloat16: decode and short portions (up to ``STREAM_ROWS`` rows) run the hand-written matrix-core kernel that streams
 the weights once; it reads them in a layout re-laid at load time (``kernels.ops.TiledWeight``) in which every load

@@ -18,9 +18,9 @@
 // A row's result depends on its own keys only, whatever stands beside it in the batch and however many workgroups share the work: keys go in
 // ranges that lie at fixed places (256 keys of a portion, 128 of a single token, counted from key 0), every range is summed from nothing
 // and the ranges are added in order by the same operations, in the registers of a workgroup that walks all of them or by
-// attn_f32_join_kernel.  A row with more than 16 (64) of them has ranges of twice as many keys, four times, ...: a portion's tile and a single
+// attn_f32_join_kernel.  A row with more than 32 (64) of them has ranges of twice as many keys, four times, ...: a portion's tile and a single
 // token choose by their own keys.  A block or range without a key that a token sees changes nothing of it.  (As a single token and as one
-// of a portion a token's sums are ordered differently, and so they are for the tokens of a tile across 4,096, 8,192, ... keys when another cut
+// of a portion a token's sums are ordered differently, and so they are for the tokens of a tile across 8,192, 16,384, ... keys when another cut
 // of the prompt moves the tile.)
 #include "common.h"
 
@@ -29,7 +29,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define AF_TOKENS 32
 #define AF_ROWS_TILES 4  // waves of a workgroup of the kernel for single tokens
 #define AF_RANGE 4       // blocks of a range of a portion's keys
-#define AF_RANGES 16     // the most ranges of a portion's keys
+#define AF_RANGES 32     // the most ranges of a portion's keys
 #define AF_ROWS_RANGES 64  // and of a single token's
 
 struct AttnF32Params {
@@ -451,13 +451,21 @@ __global__ __launch_bounds__(256) void attn_f32_join_kernel(AttnF32Params p, int
     const float before = __shfl_up(top, 1, 64);
     const RangeWeights w = range_weights(lane ? before : -INFINITY, m);
     float sum = 0.f, o[2] = {0.f, 0.f};  // (a head is at most 128 channels)
-#pragma unroll 4
-    for (int s = 0; s < count; ++s) {
-      const float old = __shfl(w.old, s, 64), now = __shfl(w.now, s, 64);
-      sum = fmaf(__shfl(l, s, 64), now, sum * old);
+    for (int s0 = 0; s0 < count; s0 += 8) {  // eight ranges' loads at a time
+      float part[8][2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        if (64 * i + lane < hd) o[i] = fmaf(p.part_o[(column * p.splits + s) * hd + 64 * i + lane], now, o[i] * old);
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          part[s][i] = s0 + s < count && 64 * i + lane < hd ? p.part_o[(column * p.splits + s0 + s) * hd + 64 * i + lane] : 0.f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        if (s0 + s >= count) break;
+        const float old = __shfl(w.old, s0 + s, 64), now = __shfl(w.now, s0 + s, 64);
+        sum = fmaf(__shfl(l, s0 + s, 64), now, sum * old);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) o[i] = fmaf(part[s][i], now, o[i] * old);
+      }
     }
     sum += sink_term(p, head, __shfl(top, 63, 64));
 #pragma unroll
@@ -494,8 +502,8 @@ static void launch_attn_f32(const AttnF32Params& p, int groups, hipStream_t stre
 
 // ``rows`` != 0: the tiles are single tokens, whose keys go in ranges of 16 ``range_tiles`` keys (or twice as many, ... so that there are at most 64);
 // the caller launches ``splits`` workgroups, as many as the row with the most ranges has, one each.  0: up to 32 tokens each, whose keys
-// go in at most 16 ranges of 256 keys or more; ``splits`` = 1: each tile's ranges by one workgroup, or the number of ranges that the workspace
-// has room for (fewer than 16 only if no tile has more), dealt to ``groups`` workgroups.  Workspace, when splits > 1 (at most 64): part_o holds
+// go in at most 32 ranges of 256 keys or more; ``splits`` = 1: each tile's ranges by one workgroup, or the number of ranges that the workspace
+// has room for (fewer than 32 only if no tile has more), dealt to ``groups`` workgroups.  Workspace, when splits > 1 (at most 64): part_o holds
 // n_tiles * (rows ? 1 : 32) * heads * splits * hd floats and part_ml twice as many as there are ranges.
 extern "C" int ns_attn_f32(float* out, float* part_o, float* part_ml, const float* q, int q_stride, const float* k_cache, const float* v_cache,
                            const int* tiles, const int* block_table, int table_stride, int n_tiles, int heads, int kv_heads, int hd,

@@ -697,7 +697,7 @@ def attention_generic(q, out, k_cache, v_cache, token_req, positions, block_tabl
 
 
 F32_ATTENTION_MAX_RANGES = 64
-F32_ATTENTION_PORTION_KEYS, F32_ATTENTION_PORTION_RANGES = 256, 16  # a range of a portion's keys at least, and as many ranges at most
+F32_ATTENTION_PORTION_KEYS, F32_ATTENTION_PORTION_RANGES = 256, 32  # a range of a portion's keys at least, and as many ranges at most
 
 
 def f32_attention_takes(dtype, head_dim: int, v_dim: int, page_size: int) -> bool:

@@ -206,8 +206,11 @@ def f32_attention(ctx, q, out, cache, table, heads: int, kv_heads: int, head_dim
         # (a span of keys may begin anywhere in its first range)
         seen, edge = (ctx.max_chunk_kv, 0) if ctx.max_chunk_kv <= span + TilePlan.TOKENS else (span + TilePlan.TOKENS, 1)
         ranges = min(ops.F32_ATTENTION_PORTION_RANGES, -(-seen // ops.F32_ATTENTION_PORTION_KEYS) + edge)
-        # (a second workgroup is worth the joining from two whole ranges on)
-        groups = max(1, min(2 * units // wgs, ranges)) if seen >= 2 * ops.F32_ATTENTION_PORTION_KEYS else 1
+        # two workgroups fit a compute unit, of heads of more than 64 channels one: of those, more than the units hold are worth it only to
+        # even out a few ranges (777 tokens, 8 heads of 128: four workgroups a tile 41 us, two 64; 20 tokens at 8,000 keys, 32 heads: 83 us
+        # for 32, 68 for 16); a second one is worth the joining from two whole ranges on
+        most = 2 * units // wgs if head_dim <= 64 else max(units // wgs, min(4, 2 * units // wgs))
+        groups = max(1, min(most, ranges)) if seen >= 2 * ops.F32_ATTENTION_PORTION_KEYS else 1
         launch(chunk_tiles, False, ranges if groups > 1 else 1, groups=groups)
     if decode_tiles.shape[0]:
         longest, edge = (ctx.max_kv_len, 0) if ctx.max_kv_len <= span else (span, 1)

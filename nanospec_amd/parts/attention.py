@@ -10,6 +10,7 @@ all heads of a group with the keys cut into ranges that are joined afterwards.
 
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
 
 import numpy as np
@@ -58,13 +59,17 @@ class TilePlan:
         tc, td = shape
         lens, indptr, kv, n = facts.lens, facts.indptr, facts.kv, facts.covered
         if tc:
-            many = [b for b in range(n) if lens[b] > 1]  # (a captured step's unused portions bring none)
-            rows = [(b, t0, indptr[b], lens[b], kv[b], 0, p, -1) for p, b in enumerate(many) for t0 in range(0, lens[b], self.TOKENS)]
-            rows += [(facts.n_reqs - 1, 0, 0, 0, 0, 0, 0, -1)] * (tc - len(rows))  # tiles without tokens
-            tiles = np.asarray(rows, dtype=np.int32)
-            first = np.cumsum([0] + [-(-int(lens[b]) // self.TOKENS) for b in many])[:-1]
-            tiles[: len(many), 7] = first
-            out[: ops.TILE_INTS * tc] = tiles.reshape(-1)
+            # plain integers in one flat list (2,048 tokens: 56 us with numpy's integers and a tuple a tile, 19 us so)
+            tiles, first = [], []
+            for b, (length, row, keys) in enumerate(zip(lens[:n].tolist(), indptr.tolist(), kv.tolist())):
+                if length > 1:  # (a captured step's unused portions bring none)
+                    p = len(first)
+                    first.append(len(tiles) // ops.TILE_INTS)
+                    for t0 in range(0, length, self.TOKENS):
+                        tiles += (b, t0, row, length, keys, 0, p, -1)
+            tiles += (facts.n_reqs - 1, 0, 0, 0, 0, 0, 0, -1) * (tc - len(tiles) // ops.TILE_INTS)  # tiles without tokens
+            tiles[7 : 7 + ops.TILE_INTS * len(first) : ops.TILE_INTS] = first
+            out[: ops.TILE_INTS * tc] = array("i", tiles)
         if td:
             req = np.nonzero(lens[:n] == 1)[0].astype(np.int32)
             d = np.zeros((td, ops.TILE_INTS), dtype=np.int32)

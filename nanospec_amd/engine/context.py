@@ -100,7 +100,8 @@ class StepContext:
         self.max_chunk_kv = max_kv_len if max_chunk_kv is None else max_chunk_kv
         # every request of the step brings one token (padding requests of a captured step likewise)
         self.single_tokens = single_tokens
-        # the most tokens that a request of the step brings, and the most requests that bring more than one (None: not known)
+        # the most tokens that a request of the step brings (a captured step: that it is laid out for, it may be some more), and the most requests
+        # that bring more than one (None: not known)
         self.longest, self.portions = longest, portions
         # blocks may let the products around an RMS norm do the norm's work (see parts.block.PreNormBlock.forward)
         self.link_norms = link_norms

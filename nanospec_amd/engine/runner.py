@@ -86,8 +86,16 @@ class _StepGraph:
     def context(self, runner, arena) -> StepContext:
         return StepContext(self.layout, self.dev_buf, arena, link_norms=runner.link_norms, max_position=0,
                            max_kv_len=self.width * runner.page_size, captured=True, pad_slot=runner.manager.get(PAD_REQUEST).slot,
-                           model_state=getattr(runner.storage, "model_state", None), single_tokens=not self.chunk, longest=self.chunk or 1,
-                           portions=self.portions)
+                           model_state=getattr(runner.storage, "model_state", None), single_tokens=not self.chunk,
+                           longest=self.longest(self.chunk), portions=self.portions)
+
+    @staticmethod
+    def longest(chunk: int) -> int:
+        """The tokens of a portion that a captured step of ``chunk`` portion tokens is laid out for.  It takes portions of up to
+        ``MIXED_TOKEN_STEP`` - 1 fewer too, and kernels for long portions that only its very fullest fillings use cost the others more
+        than they save those: two launches a delta layer that find nothing in a prompt of 40 tokens (16 heads of 128: 2.4 us a layer, a step of
+        431 us 436), where 64 tokens would take 18 us instead of 27.  So those fillings do not count: the last fifth of what a shape takes."""
+        return max(1, chunk - MIXED_TOKEN_STEP // 5)
 
 
 class ModelRunner:

@@ -112,3 +112,20 @@ def test_tiles_number_the_portions_that_bring_tokens(lens, unused, spare):
             assert tuple(tiles[at, :7]) == (b, t0, indptr[b], lens[b], starts[b] + lens[b], 0, p)
             at += 1
     assert (tiles[at:, 1:7] == 0).all() and (tiles[len(many) :, 7] == -1).all()
+
+
+def test_captured_steps_laid_out_for_long_portions():
+    """Kernels for portions of 64 tokens and more are in a captured step unless hardly any portion that it takes is so long."""
+    from nanospec_amd.engine.runner import MIXED_MAX_TOKENS, ModelRunner, _StepGraph
+
+    runner = object.__new__(ModelRunner)
+    for rows in (0, 1, 8, 48):
+        for n in range(2, MIXED_MAX_TOKENS + 1):
+            shape = runner._graph_shape([1] * rows + [n], 1)
+            longest = _StepGraph.longest(shape[1])
+            assert shape[1] - 12 <= longest <= shape[1]
+            if shape[1] <= 64:  # a prompt of 40 tokens, alone
+                assert longest < 64
+            if n >= 77:
+                assert longest >= 64
+    assert _StepGraph.longest(0) == 1

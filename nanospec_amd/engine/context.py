@@ -119,6 +119,10 @@ class StepContext:
         self.token_ids, self.positions, self.token_req = view("token_ids"), view("positions"), view("token_req")
         self.qo_indptr, self.kv_lens, self.state_slots = view("qo_indptr"), view("kv_lens"), view("state_slots")
         self.want_rows = view("want_rows")
+        # (qo_indptr, state_slots) of the requests whose tokens are one behind the other for a recurrence: without the stand-in of a captured step, whose
+        # padding behind the portions, up to 63 tokens that nobody reads, would be the longest chain of a step of short portions
+        behind = captured and not single_tokens
+        self.spans = (self.qo_indptr[:-1], self.state_slots[:-1]) if behind else (self.qo_indptr, self.state_slots)
         # what the parts' batch plans wrote, by key: (device view of the plan's region, its shape for this batch)
         self.plans = {key: (view(key), shape) for key, (_, shape) in layout.plans.items()}
         self.block_tables = [dev_buf[o : o + layout.B * layout.P].view(layout.B, layout.P) for o in layout.table_off]

@@ -116,7 +116,8 @@ class ChannelDelta:
                                   out=take((n, self.channels), torch.float32), single=getattr(ctx, "single_tokens", False))
         g, beta = take((n, H * D), torch.float32), take((n, H), torch.float32)
         ops.delta_prep(qkv, thin, proj[:, self.b_at :], self.dt_bias, self.a_log, H, G, D, g, beta)
-        o = ops.delta_scan(qkv, g, beta, state, ctx.qo_indptr, ctx.state_slots, H, G, D, E, out=take((n, H * E), torch.float32), take=take,
+        indptr, slots = getattr(ctx, "spans", (ctx.qo_indptr, ctx.state_slots))
+        o = ops.delta_scan(qkv, g, beta, state, indptr, slots, H, G, D, E, out=take((n, H * E), torch.float32), take=take,
                            longest=getattr(ctx, "longest", None), portions=getattr(ctx, "portions", None))
         gated = ops.gated_rms(o, thin[:, H * D :], self.norm, s.norm_eps, H, out=take((n, H * E), x.dtype))
         return self.w_out(gated, out=out if out is not None else take((n, s.hidden), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)

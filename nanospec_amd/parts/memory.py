@@ -90,8 +90,9 @@ class MatrixMemory:
         n, take = x.shape[0], ctx.arena.take
         proj = self.w_in(x, out=take((n, self.w_in.n), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)
         den = take((n, s.heads), torch.float32)  # the read-out's denominators; the gated norm divides as it reads a head
-        o = ops.memory_scan(proj, (0, self.k_at, self.v_at, self.i_at, self.f_at), self.bias_i, self.bias_f, cache.state, ctx.qo_indptr,
-                            ctx.state_slots, s.heads, s.key_dim, s.value_dim, s.gate_cap, s.key_dim ** -0.5, den_eps=s.den_eps,
+        indptr, slots = getattr(ctx, "spans", (ctx.qo_indptr, ctx.state_slots))
+        o = ops.memory_scan(proj, (0, self.k_at, self.v_at, self.i_at, self.f_at), self.bias_i, self.bias_f, cache.state, indptr,
+                            slots, s.heads, s.key_dim, s.value_dim, s.gate_cap, s.key_dim ** -0.5, den_eps=s.den_eps,
                             out=take((n, self.vw), torch.float32), den=den, take=take, longest=getattr(ctx, "longest", None),
                             portions=getattr(ctx, "portions", None))
         gated = ops.gated_rms(o, proj[:, self.g_at : self.g_at + self.vw], self.norm, s.norm_eps, s.heads, out=take((n, self.vw), x.dtype),

@@ -129,3 +129,17 @@ def test_captured_steps_laid_out_for_long_portions():
             if n >= 77:
                 assert longest >= 64
     assert _StepGraph.longest(0) == 1
+
+
+def test_recurrences_leave_out_the_padding_behind_portions():
+    """A captured step's stand-in request owns the tokens behind the portions; padding rows of one token are rows like others."""
+    import torch
+
+    from nanospec_amd.engine.context import BatchLayout, StepContext
+
+    layout = BatchLayout(70, 5, 2, 1, 4)
+    make = lambda **kw: StepContext(layout, torch.arange(layout.total, dtype=torch.int32), None, 0, 64, **kw)
+    for kw, left_out in ((dict(captured=True), 1), (dict(captured=True, single_tokens=True), 0), (dict(), 0)):
+        ctx = make(**kw)
+        indptr, slots = ctx.spans
+        assert torch.equal(indptr, ctx.qo_indptr[: 6 - left_out]) and torch.equal(slots, ctx.state_slots[: 5 - left_out])

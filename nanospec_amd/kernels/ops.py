@@ -1255,9 +1255,10 @@ def memory_scan(proj: torch.Tensor, offsets: tuple[int, int, int, int, int], gat
     sizes = (c_int(reqs), c_int(heads), c_int(key_dim), c_int(value_dim), c_float(cap), c_float(q_scale), c_float(den_eps))
     below = 0x7FFFFFFF
     longest, portions = _longest_and_portions(n, reqs, longest, portions, MEMORY_CHUNK_MIN)
-    if (take is not None and longest >= memory_chunk_min(portions, heads, key_dim) and key_dim in MEMORY_CHUNK_KEY_DIMS and value_dim % 16 == 0
+    least = memory_chunk_min(portions, heads, key_dim)
+    if (take is not None and longest >= least and key_dim in MEMORY_CHUNK_KEY_DIMS and value_dim % 16 == 0
             and not (proj.stride(0) % 8 or q_off % 8 or k_off % 8 or proj.data_ptr() % (8 * proj.element_size()))):
-        below = memory_chunk_min(portions, heads, key_dim)
+        below = least
         record = heads * (32 * key_dim + 276)
         gates = take((4 * n * heads + reqs * heads,), torch.float32)
         scratch = take((min((n // 16 + reqs) * record, max(record, MEMORY_CHUNK_SCRATCH // 4)),), torch.float32)
@@ -1910,19 +1911,25 @@ DELTA_CHUNK_MIN = 64
 DELTA_CHUNK_SCRATCH = 64 << 20
 
 
-def delta_chunk_min(portions: int, heads: int, key_dim: int, value_dim: int) -> int:
+def delta_chunk_min(portions: int, heads: int, key_dim: int, value_dim: int, singles: int = 0) -> int:
     """Tokens from which on a request of the step goes chunk by chunk (more than any has: none does).  Many requests keep the GPU busy
     token by token too, and the chunks' 64-bit sums then cost more than the shorter chain gives (us token by token and by chunks): keys of 64
     channels, 4 heads of 64 values, 32 requests of 64 tokens 22 and 25, of 96 tokens 31 and 30, 64 requests of 64 tokens 25 and 39, of
     256 tokens 78 and 93; 8 heads of 128 values, 8 requests of 64 tokens 23 and 20, 16 requests 26 and 32, 64 requests of 256 tokens 236
     and 266.  Keys of 128 channels: 128 requests of 64 tokens, 16 heads 626 and 614, 32 heads 1,223 and 1,293, of 128 tokens 2,217 and
-    2,195."""
+    2,195.
+    ``singles``: requests of one token beside them.  Reading and writing their states takes the GPU as long as a short portion's chain, which then runs
+    beside it, where chunks come before it: 16 heads of 128, 64 of them beside 64 tokens 95 and 99, 80 tokens 99 and 100, 96 tokens 105 and 101
+    (a whole captured step with 70 tokens 759 and 768); 16 of them beside 80 tokens 48 and 44; 32 heads, 64 of them beside 160 tokens 200 and 201,
+    192 tokens 214 and 203.  Keys and values of 64, 16 heads, 64 of them beside 64 tokens 34 and 33."""
     chains = portions * heads
     if key_dim == 64 and (chains >= 256 or chains * value_dim >= 16384):
         return 0x7FFFFFFF
     if key_dim == 64 and chains >= 128:
         return max(DELTA_CHUNK_MIN, 96)
-    return max(DELTA_CHUNK_MIN, 128) if chains >= 4096 else DELTA_CHUNK_MIN
+    states = singles * heads * key_dim * value_dim  # floats
+    beside = 192 if states >= 1 << 25 else 96 if states >= 1 << 23 else 0
+    return max(DELTA_CHUNK_MIN, beside, 128 if chains >= 4096 else 0)
 
 
 def _state_args(state: torch.Tensor, what: str):
@@ -1996,9 +2003,10 @@ def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: to
     sp, stride = _state_args(state, "delta_scan")
     below = 0x7FFFFFFF
     longest, portions = _longest_and_portions(n, reqs, longest, portions, DELTA_CHUNK_MIN)
-    if (take is not None and longest >= delta_chunk_min(portions, heads, key_dim, value_dim) and key_dim in DELTA_CHUNK_KEY_DIMS and value_dim % 16 == 0 and C % 4 == 0
+    least = delta_chunk_min(portions, heads, key_dim, value_dim, reqs - portions)
+    if (take is not None and longest >= least and key_dim in DELTA_CHUNK_KEY_DIMS and value_dim % 16 == 0 and C % 4 == 0
             and not (qkv.data_ptr() | g.data_ptr()) % 16):
-        below = delta_chunk_min(portions, heads, key_dim, value_dim)
+        below = least
         record = heads * (49 * key_dim + 512)
         scratch = take((min((n // 16 + reqs) * record, max(record, DELTA_CHUNK_SCRATCH // 4)),), torch.float32)
         _check(build.core().ns_delta_chunks(_ptr(out), _ptr(qkv), c_int(C), _ptr(g), _ptr(beta), sp, stride, _ptr(qo_indptr), _ptr(state_slots),

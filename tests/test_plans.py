@@ -143,3 +143,12 @@ def test_recurrences_leave_out_the_padding_behind_portions():
         ctx = make(**kw)
         indptr, slots = ctx.spans
         assert torch.equal(indptr, ctx.qo_indptr[: 6 - left_out]) and torch.equal(slots, ctx.state_slots[: 5 - left_out])
+
+
+def test_chunks_of_the_delta_rule_beside_single_tokens():
+    """Single tokens whose states take as long as a short portion's chain keep that portion token by token."""
+    least = lambda portions, heads, dim, singles: ops.delta_chunk_min(portions, heads, dim, dim, singles)
+    assert [least(1, 16, 128, n) for n in (0, 16, 31, 32, 64, 127, 128)] == [64, 64, 64, 96, 96, 96, 192]
+    assert [least(1, 32, 128, n) for n in (8, 16, 32, 64)] == [64, 96, 96, 192]
+    assert [least(1, 16, 64, n) for n in (0, 64, 127, 128)] == [64, 64, 64, 96]
+    assert least(4, 16, 64, 64) == 64 and least(8, 16, 64, 0) == 96 and least(16, 16, 64, 0) == 0x7FFFFFFF

@@ -683,14 +683,21 @@ __global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restr
     }
 }
 
-// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees four rows on average, else 128 (the
-// tiled one).  32 experts of 1,024 in a width of 2,048, four a token, sorting included: 8 tokens 58 us streamed and 84 tiled, 24 tokens 92 and 94, 40 tokens
-// 99 and 94 (an expert with more than 16 rows is read twice).
-static int moe_tile_cap(long long pairs, int experts) { return pairs <= 4LL * experts ? 16 : MG_TM; }
+// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees few rows on average, else 128 (the tiled one).
+// Streaming is ahead up to two rows an expert, and up to four where the tiled kernel has too few workgroups for the GPU, or just enough with one matrix
+// each to keep its loads going.  us streamed and tiled, sorting included, width 2,048, 32 experts, four a token, 32 tokens: 512 channels with gates 55
+// and 73, 1,024 64 and 75 without gates and 97 and 86 with them, 1,536 96 and 89, 135 and 107; 16 experts of 1,408, two a token, 70 and 88; 64 of
+// 1,024, 64 tokens, 175 and 146; 256 of 512, eight a token, 128 tokens, 318 and 267 (one expert that all tokens choose: 331 and 278).
+// (One step of 20 decoding requests with experts of 1,536, beside the other layers: 1,164 and 1,062 us.)
+static int moe_tile_cap(long long pairs, int experts, int ff, int gated) {
+  const long long groups = (long long)experts * ((ff + MG_TN - 1) / MG_TN);
+  const bool fills = groups >= 256 && groups * (gated ? 2 : 1) > 256;  // compute units
+  return pairs <= (fills ? 2LL : 4LL) * experts ? 16 : MG_TM;
+}
 
 // tiles that any choice of experts can need
-extern "C" int ns_moe_group_tiles(int pairs, int experts) {
-  const int cap = moe_tile_cap(pairs, experts);
+extern "C" int ns_moe_group_tiles(int pairs, int experts, int ff, int gated) {
+  const int cap = moe_tile_cap(pairs, experts, ff, gated);
   return (pairs + cap - 1) / cap + experts;
 }
 
@@ -725,7 +732,7 @@ struct MoeLaunch {
   }
 };
 
-// ``ints``: scratch of pairs + 3 * ns_moe_group_tiles(pairs, experts) 32-bit words; ``act``: bfloat16 [pairs][ff]
+// ``ints``: scratch of pairs + 3 * ns_moe_group_tiles(...) 32-bit words; ``act``: bfloat16 [pairs][ff]
 extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg, const void* wu, const void* wd, const int* sel, const float* wt,
                                     int* ints, void* act, float* out, int n, int W, int ff, int top, int experts, float limit, float alpha, float shift,
                                     int act_kind, hipStream_t stream) {
@@ -735,12 +742,12 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
     return NS_ERR_UNSUPPORTED;
   const long long pairs = (long long)n * top;
   if (pairs > (1 << 24)) return NS_ERR_UNSUPPORTED;
-  const int tiles = ns_moe_group_tiles((int)pairs, experts);
+  const int tiles = ns_moe_group_tiles((int)pairs, experts, ff, wg != nullptr);
   int* perm = ints;
   int* tile_e = ints + pairs;
   int* tile_r0 = tile_e + tiles;
   int* tile_rows = tile_r0 + tiles;
-  const int cap = moe_tile_cap(pairs, experts);
+  const int cap = moe_tile_cap(pairs, experts, ff, wg != nullptr);
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
   moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
   const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,

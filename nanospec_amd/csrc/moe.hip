@@ -12,6 +12,7 @@
 // The last outputs of a router may be identity experts, which have no matrices: what such a pair adds is its weight times the
 // input row, formed where the pairs are added up (``moe_combine``); the experts' kernels leave these pairs out.
 #include "common.h"
+#include "tile_bf16.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 #define MOE_MAX_EXPERTS 1024
@@ -418,29 +419,16 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 
 // ------------------------------------------------------------------------------------------------ many rows
 // Steps of many rows (bfloat16): the (token, chosen expert) pairs are sorted by expert on the device, and every expert's
-// pairs are cut into even tiles of at most 128 rows (16 where the experts see few; ``moe_tile_cap``).  A workgroup takes one tile
-// and 128 output channels and multiplies on the matrix cores (v_mfma_f32_16x16x32_bf16): its four waves own 64 x 64 each
-// (every second block of 16 rows), operands come through LDS in pieces of 64 along K, the next piece is fetched into registers
-// while the current one is multiplied.  The host never learns which experts were chosen: the launch has as many tiles as any
-// choice can need (pairs / 128 or 16 + experts), and a tile without rows returns.
-// Bound by the matrices' bytes up to some hundred tokens (300: 104 us of which the 403 MB take 82 at a large copy's rate), by what
-// a compute unit takes in from L2 beyond.  32 experts of 1,024, width 2,048, four a token, sorting included: 1,024 tokens 212 -> 146 us,
-// 2,048 tokens 311 -> 237 us (even tiles, blocks without rows skipped, LDS rows without bank conflicts, the sort's scan).
+// pairs are cut into even tiles of at most 128 rows (16 where the experts see few; ``moe_tile_cap``), which are multiplied on the matrix
+// cores (v_mfma_f32_16x16x32_bf16).  The host never learns which experts were chosen: the launch has as many tiles as any
+// choice can need (pairs / cap + experts), and workgroups beyond the tiles in use return.
 //   first:  rows gathered from h by the sorted pairs; gate (if there is one: DUAL) and up matrices in the same pass; act [pairs
 //           sorted][ff] in bfloat16
 //   second: act times the down matrix; out [tokens][top][W] in 32-bit, each row back at its pair and times its weight
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 
-#define MG_TM 128
-#define MG_TN 128
-#define MG_KC 64
-// bfloat16 values between two rows of a staged tile: 32 bytes more than its data, so that the lanes 0-7 and 16-23 that a 16-byte read serves together
-// touch all banks once (with 16 bytes more the eighth row's second piece meets the first row's first)
-#define MG_LD (MG_KC + 16)
-#define MG_RI (MG_TM / 32)  // 16-row blocks of a wave's 64 x 64 (the four waves are 2 x 2)
-#define MG_CJ (MG_TN / 32)
-#define MG_FA (MG_TM / 32)  // pieces of 8 values that a thread fetches of a staged tile of MG_TM rows (256 threads, 8 pieces a row)
-#define MG_FB (MG_TN / 32)
+#define MG_ROWS 128                                 // rows of a tile at most
+typedef TileBf16<MG_ROWS, 256, 2, 4, 3> MoeTile;        // by 256 rows of the matrices: one workgroup of eight waves a compute unit
+typedef TileBf16<MG_ROWS, 128, 2, 2, 2, true> MoeFewTile;  // by 128: two workgroups of four waves
 
 // Pairs sorted by expert and every expert's pairs cut into the fewest tiles of at most ``cap`` rows, as even as whole blocks of
 // 16 rows allow (an expert with a few rows more than ``cap`` makes two tiles of about half, not a full one and a sliver).  The counts
@@ -480,7 +468,8 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
       at += rows;
     }
   }
-  for (int i = used + threadIdx.x; i < max_tiles; i += blockDim.x) tile_e[i] = -1, tile_r0[i] = 0, tile_rows[i] = 0;
+  // (max_tiles is at least one more than any choice uses: behind the last tile stands how many there are)
+  for (int i = used + threadIdx.x; i < max_tiles; i += blockDim.x) tile_e[i] = -1, tile_r0[i] = used, tile_rows[i] = 0;
   __syncthreads();
   // (which pair of an expert gets which of its places depends on timing; a pair's result does not depend on its place)
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
@@ -557,130 +546,74 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
     out[(size_t)perm[slot] * N + col] = wt[perm[slot]] * v[0];
 }
 
-// ONCE: most experts have one tile, so a matrix is read once: past the caches, and starting at a piece of K of its own for every expert and
-// block of channels, because workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (300
-// tokens: 105 -> 96 us with the sort).  Where experts have several tiles the matrices come from L2 the second time (2,048 tokens, 1,536
-// channels: 275 -> 237 us without the non-temporal loads).
-template <bool FIRST, bool DUAL, bool ONCE>
-__global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
-                                                        const bf16_t* __restrict__ B1, const int* __restrict__ perm,
-                                                        const int* __restrict__ tile_e, const int* __restrict__ tile_r0,
-                                                        const int* __restrict__ tile_rows, bf16_t* __restrict__ act_out, float* __restrict__ out,
-                                                        const float* __restrict__ wt, int N, int K, int top, float limit, float alpha, float shift,
-                                                        int act_kind) {
-  __shared__ __attribute__((aligned(16))) bf16_t As[MG_TM * MG_LD];
-  __shared__ __attribute__((aligned(16))) bf16_t Bs[(DUAL ? 2 : 1) * MG_TN * MG_LD];
-  const int tile = blockIdx.y, e = tile_e[tile];
-  if (e < 0) return;
-  const int r0 = tile_r0[tile], rows = tile_rows[tile], n0 = blockIdx.x * MG_TN;
-  const int tid = threadIdx.x, lane = tid % NS_WAVE, wave = tid / NS_WAVE, r = lane % 16, g = lane / 16;
-  const int wm = wave / 2, wn = wave % 2;
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+// Many rows an expert.  A workgroup takes a tile of the sorted rows and BN rows of the matrices (with gates BN / 2 channels of
+// both: half of a wave's 64 are of the gate and the other half the same channels of the up matrix) through LDS (tile_bf16.h).
+// Bound by the matrices' bytes up to some hundred tokens, beyond by what L2 gives the compute units (14.7 TB/s with the products
+// taken out, where the products alone would take two thirds of the time) and by how evenly the experts' tiles deal.  32 experts of 1,024 with
+// gates, width 2,048, four a token chosen evenly, sorting included, against the kernel before (128 x 128, operands through registers, two
+// barriers a piece): 100 tokens 94 -> 80 us, 508 112 -> 90, 1,024 153 -> 136, 1,531 182 -> 142, 2,048 241 -> 200; 1,536 channels
+// without gates, 2,048 tokens 244 -> 197.
+// Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the tiles in use, neighbours first, so that an expert's
+// matrices and rows come into one L2 (2,048 tokens: 216 -> 200 us).  Every expert and block of channels begins at a stage of K of its own:
+// workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (508 tokens: 111 -> 90 us).
+template <class T, bool FIRST, bool DUAL>
+__global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void moe_tile_kernel(
+    const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0, const bf16_t* __restrict__ B1, const int* __restrict__ perm,
+    const int* __restrict__ tile_e, const int* __restrict__ tile_r0, const int* __restrict__ tile_rows, int tiles, bf16_t* __restrict__ act_out,
+    float* __restrict__ out, const float* __restrict__ wt, int N, int K, int top, float limit, float alpha, float shift, int act_kind) {
+  constexpr int CH = DUAL ? T::BN / 2 : T::BN;          // output channels of a workgroup
+  constexpr int WCH = CH / T::WC;                       // and of a wave
+  constexpr int NJ = DUAL ? T::NJ / 2 : T::NJ;          // its blocks of 16
+  __shared__ __attribute__((aligned(16))) bf16_t moe_tiles[T::ST * T::STAGE];
+  const int blocks_n = (N + CH - 1) / CH;
+  const long long used = (long long)tile_r0[tiles - 1] * blocks_n, share = (used + 7) / 8;
+  const long long item = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= share || item >= used) return;
+  const int tile = (int)(item / blocks_n), n0 = (int)(item % blocks_n) * CH;
+  const int e = tile_e[tile], r0 = tile_r0[tile], rows = tile_rows[tile];
 
-  // the pieces (8 values along K) of each staged tile that this thread fetches: rows tid / 8 + 32 i, piece tid % 8
-  const int kp = (tid % 8) * 8;
-  const bf16_t* arow[MG_FA];
-  const bf16_t* brow0[MG_FB];
-  const bf16_t* brow1[MG_FB];
+  T t;
+  t.init(moe_tiles, K, (int)(item % blocks_n) * 7 + e * 11);
 #pragma unroll
-  for (int i = 0; i < MG_FA; ++i) {
-    const int row = tid / 8 + 32 * i;
+  for (int p = 0; p < T::PER; ++p) {
+    const int row = t.row_of(p);
+    if (p < T::PA) {
+      const int slot = r0 + min(row, rows - 1);
+      t.src[p] = A + (size_t)(FIRST ? perm[slot] / top : slot) * a_stride + t.piece();
+    } else {
+      const int in = row % (16 * T::NJ), col = DUAL ? n0 + row / (16 * T::NJ) * WCH + in % WCH : n0 + row;
+      t.src[p] = (DUAL && in >= WCH ? B1 : B0) + ((size_t)e * N + min(col, N - 1)) * K + t.piece();
+    }
+  }
+  t.start();
+  t.run(((rows + 15) / 16 - t.wm + T::WR - 1) / T::WR);
+
+  const int r = t.lane % 16, g = t.lane / 16;
+#pragma unroll
+  for (int i = 0; i < T::MI; ++i) {
+    const int row = 16 * (T::WR * i + t.wm) + r;
+    if (row >= rows) continue;
     const int slot = r0 + row;
-    arow[i] = row < rows ? A + (size_t)(FIRST ? perm[slot] / top : slot) * a_stride : nullptr;
-  }
+    const int pair = FIRST ? 0 : perm[slot];
+    const float share_of = FIRST ? 0.f : wt[pair];
 #pragma unroll
-  for (int i = 0; i < MG_FB; ++i) {
-    const int col = n0 + tid / 8 + 32 * i;
-    brow0[i] = col < N ? B0 + ((size_t)e * N + col) * K : nullptr;
-    brow1[i] = (DUAL && col < N) ? B1 + ((size_t)e * N + col) * K : nullptr;
-  }
-  bf16x8 pa[MG_FA], pb0[MG_FB], pb1[MG_FB];
-  auto read = [](const bf16_t* w) { return ONCE ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(w)) : *reinterpret_cast<const bf16x8*>(w); };
-  auto fetch = [&](int k0) {
-    const bool ok = k0 + kp < K;
+    for (int j = 0; j < NJ; ++j) {
+      const int col = n0 + t.wn * WCH + 16 * j + 4 * g;
+      if (col >= N) continue;  // (N is a multiple of 8: four columns are all inside or all outside)
+      if (FIRST) {
+        typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 o;
 #pragma unroll
-    for (int i = 0; i < MG_FA; ++i) pa[i] = (ok && arow[i]) ? *reinterpret_cast<const bf16x8*>(arow[i] + k0 + kp) : zero;
-#pragma unroll
-    for (int i = 0; i < MG_FB; ++i) {
-      pb0[i] = (ok && brow0[i]) ? read(brow0[i] + k0 + kp) : zero;
-      if (DUAL) pb1[i] = (ok && brow1[i]) ? read(brow1[i] + k0 + kp) : zero;
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int i = 0; i < MG_FA; ++i) *reinterpret_cast<bf16x8*>(As + (tid / 8 + 32 * i) * MG_LD + kp) = pa[i];
-#pragma unroll
-    for (int i = 0; i < MG_FB; ++i) {
-      const int at = (tid / 8 + 32 * i) * MG_LD + kp;
-      *reinterpret_cast<bf16x8*>(Bs + at) = pb0[i];
-      if (DUAL) *reinterpret_cast<bf16x8*>(Bs + MG_TN * MG_LD + at) = pb1[i];
-    }
-  };
-
-  f32x4 acc0[MG_RI][MG_CJ], acc1[DUAL ? MG_RI : 1][DUAL ? MG_CJ : 1];
-#pragma unroll
-  for (int i = 0; i < MG_RI; ++i)
-#pragma unroll
-    for (int j = 0; j < MG_CJ; ++j) {
-      acc0[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (DUAL) acc1[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-
-  // the tile's blocks of 16 rows go to the two waves of a column in turn, so that a tile that is not full keeps both busy; a block
-  // without rows costs no product
-  const int my_blocks = ((rows + 15) / 16 - wm + 1) / 2;
-  const int a_at = (16 * wm + r) * MG_LD + 8 * g, b_at = (MG_TN / 2 * wn + r) * MG_LD + 8 * g;
-  const int steps = (K + MG_KC - 1) / MG_KC, turn = ONCE ? (blockIdx.x * 5 + e * 3) % steps : 0;
-  auto piece = [&](int i) { return (i + turn >= steps ? i + turn - steps : i + turn) * MG_KC; };
-  fetch(piece(0));
-  for (int i = 0; i < steps; ++i) {
-    stage();
-    __syncthreads();
-    if (i + 1 < steps) fetch(piece(i + 1));
-#pragma unroll
-    for (int ks = 0; ks < MG_KC; ks += 32) {
-      bf16x8 af[MG_RI], bf0[MG_CJ], bf1[MG_CJ];
-#pragma unroll
-      for (int i = 0; i < MG_RI; ++i) af[i] = *reinterpret_cast<const bf16x8*>(As + a_at + 32 * i * MG_LD + ks);  // (blocks without rows too)
-#pragma unroll
-      for (int j = 0; j < MG_CJ; ++j) {
-        bf0[j] = *reinterpret_cast<const bf16x8*>(Bs + b_at + 16 * j * MG_LD + ks);
-        if (DUAL) bf1[j] = *reinterpret_cast<const bf16x8*>(Bs + MG_TN * MG_LD + b_at + 16 * j * MG_LD + ks);
-      }
-#pragma unroll
-      for (int i = 0; i < MG_RI; ++i) {
-        if (i >= my_blocks) break;
-#pragma unroll
-        for (int j = 0; j < MG_CJ; ++j) {
-          acc0[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf0[j], acc0[i][j], 0, 0, 0);
-          if (DUAL) acc1[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf1[j], acc1[i][j], 0, 0, 0);
+        for (int q = 0; q < 4; ++q) {
+          const float z = round_to<bf16_t>(t.acc[i][j][q]);
+          o[q] = from_f<bf16_t>(DUAL ? clipped_glu(z, round_to<bf16_t>(t.acc[i][T::NJ / 2 + j][q]), limit, alpha, shift) : activation_of(z, act_kind));
         }
+        *reinterpret_cast<bf16x4*>(act_out + (size_t)slot * N + col) = o;
+      } else {
+        *reinterpret_cast<f32x4*>(out + (size_t)pair * N + col) = share_of * t.acc[i][j];
       }
     }
-    __syncthreads();
   }
-  // element q of a lane's sums is row 4 g + q of the 16 x 16 block, column r
-#pragma unroll
-  for (int i = 0; i < MG_RI; ++i)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 16 * (2 * i + wm) + 4 * g + q;
-      if (row >= rows) continue;
-      const int slot = r0 + row;
-      const int pair = FIRST ? 0 : perm[slot];
-      const float share = FIRST ? 0.f : wt[pair];
-#pragma unroll
-      for (int j = 0; j < MG_CJ; ++j) {
-        const int col = n0 + MG_TN / 2 * wn + 16 * j + r;
-        if (col >= N) continue;
-        if (DUAL)
-          act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu(round_to<bf16_t>(acc0[i][j][q]), round_to<bf16_t>(acc1[i][j][q]), limit, alpha, shift));
-        else if (FIRST)
-          act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of(round_to<bf16_t>(acc0[i][j][q]), act_kind));
-        else
-          out[(size_t)pair * N + col] = share * acc0[i][j][q];
-      }
-    }
 }
 
 // Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees few rows on average, else 128 (the tiled one).
@@ -690,10 +623,15 @@ __global__ __launch_bounds__(256, 2) void moe_group_kernel(const bf16_t* __restr
 // 1,024, 64 tokens, 175 and 146; 256 of 512, eight a token, 128 tokens, 318 and 267 (one expert that all tokens choose: 331 and 278).
 // (One step of 20 decoding requests with experts of 1,536, beside the other layers: 1,164 and 1,062 us.)
 static int moe_tile_cap(long long pairs, int experts, int ff, int gated) {
-  const long long groups = (long long)experts * ((ff + MG_TN - 1) / MG_TN);
+  const long long groups = (long long)experts * ((ff + 127) / 128);
   const bool fills = groups >= 256 && groups * (gated ? 2 : 1) > 256;  // compute units
-  return pairs <= (fills ? 2LL : 4LL) * experts ? 16 : MG_TM;
+  return pairs <= (fills ? 2LL : 4LL) * experts ? 16 : MG_ROWS;
 }
+
+// Which tiles: up to 96 rows an expert on average most experts have one tile, a matrix is read once (past the caches) and the launch is short of
+// workgroups, so the smaller ones (a step of 508 tokens whose experts see 18 to 390 rows, beside other work: 1,454 us with these and 1,479 to
+// 1,496 with the others); beyond, the larger ones, which read less (2,048 tokens: 196 us and 206).
+static bool moe_few_rows(long long pairs, int experts) { return pairs <= 96LL * experts; }
 
 // tiles that any choice of experts can need
 extern "C" int ns_moe_group_tiles(int pairs, int experts, int ff, int gated) {
@@ -709,26 +647,35 @@ struct MoeLaunch {
   const float* wt;
   int h_stride, W, ff, top, tiles, act_kind;
   float limit, alpha, shift;
-  bool once;  // see moe_group_kernel
+  bool few_rows;
   hipStream_t stream;
 
+  template <class T, bool FIRST, bool DUAL>
+  void tiled(const bf16_t* a, int a_stride, const bf16_t* b0, const bf16_t* b1, int n, int k) const {
+    constexpr int CH = DUAL ? T::BN / 2 : T::BN;
+    const long long blocks = ((long long)tiles * ((n + CH - 1) / CH) + 7) / 8 * 8;
+    moe_tile_kernel<T, FIRST, DUAL><<<(unsigned)blocks, T::THREADS, 0, stream>>>(a, a_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, tiles, act, out, wt,
+                                                                                 n, k, top, limit, alpha, shift, act_kind);
+  }
   template <bool DUAL>
   void first(int cap) const {
     const bf16_t *b0 = DUAL ? wg : wu, *b1 = DUAL ? wu : nullptr;
     if (cap == 16)
       moe_stream_kernel<true, DUAL><<<dim3((ff + 15) / 16, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr,
                                                                                     nullptr, ff, W, top, limit, alpha, shift, act_kind);
+    else if (few_rows)
+      tiled<MoeFewTile, true, DUAL>(h, h_stride, b0, b1, ff, W);
     else
-      (once ? moe_group_kernel<true, DUAL, true> : moe_group_kernel<true, DUAL, false>)<<<dim3((ff + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(
-          h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr, nullptr, ff, W, top, limit, alpha, shift, act_kind);
+      tiled<MoeTile, true, DUAL>(h, h_stride, b0, b1, ff, W);
   }
   void second(int cap) const {
     if (cap == 16)
       moe_stream_kernel<false, false><<<dim3((W + 15) / 16, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt,
                                                                                      W, ff, top, limit, alpha, shift, act_kind);
+    else if (few_rows)
+      tiled<MoeFewTile, false, false>(act, ff, wd, nullptr, W, ff);
     else
-      (once ? moe_group_kernel<false, false, true> : moe_group_kernel<false, false, false>)<<<dim3((W + MG_TN - 1) / MG_TN, tiles), 256, 0, stream>>>(
-          act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt, W, ff, top, limit, alpha, shift, act_kind);
+      tiled<MoeTile, false, false>(act, ff, wd, nullptr, W, ff);
   }
 };
 
@@ -751,7 +698,7 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
   moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
   const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,
-                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, pairs <= MG_TM * 3LL / 4 * experts, stream};
+                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, moe_few_rows(pairs, experts), stream};
   if (wg)
     l.first<true>(cap);
   else

@@ -1146,9 +1146,10 @@ def test_attention_f32_keeps_infinities_to_the_rows_that_see_them():
 @pytest.mark.parametrize("routing", ["spread", "one expert", "identity"])
 @pytest.mark.parametrize("n,experts,top,width,ff,gated", [(8, 8, 4, 64, 24, True), (16, 32, 4, 136, 40, False), (33, 32, 4, 72, 136, True), (40, 5, 2, 264, 16, True),
                                                           (130, 3, 1, 64, 264, False), (517, 70, 3, 128, 72, True), (64, 256, 8, 64, 16, True), (65, 256, 8, 64, 16, True),
-                                                          (80, 256, 8, 64, 136, False), (80, 256, 8, 64, 16, False)])
+                                                          (80, 256, 8, 64, 136, False), (80, 256, 8, 64, 16, False), (400, 6, 2, 136, 136, True),
+                                                          (450, 3, 1, 72, 264, False), (150, 4, 2, 520, 264, True)])
 def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
-    """The sorted experts' products, streamed and tiled: tiles of 1 to 16 and to 128 rows, experts with more rows than a tile and with
+    """The sorted experts' products, streamed and tiled: tiles of 1 to 16 and to 128 rows in both forms, experts with more rows than a tile and with
     none, pairs without an expert, sizes that end inside a tile and inside a piece of K."""
     ops = _ops()
     g = torch.Generator().manual_seed(n + experts)

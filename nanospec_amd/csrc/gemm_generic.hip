@@ -8,6 +8,7 @@
 // result as one of few rows and as one of many differ by rounding.
 // (reference: the nn.Linear calls of model/llama.py:175,184,195,286)
 #include "common.h"
+#include "lds_loads.h"
 
 #define GT_M 64
 #define GT_N 64
@@ -137,68 +138,94 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 4) void gemm_rows_f32_kernel(float
 
 // Many rows in 32-bit on the matrix cores (v_mfma_f32_16x16x4_f32, 32-bit products and sums: 157 TFLOP/s at the boost clock,
 // the vector unit's own rate, but 2,048 operations an instruction and far fewer operand reads).  Bound by the matrix unit for many
-// rows, by the latency of a workgroup's loads for few.  Against the tiled kernel above: 777 rows, N 16,384 K 2,048: 903 -> 512 us
-// (102 TFLOP/s), N 2,048 K 8,192: 1,049 -> 283 us (92); 64 rows: 320 -> 51 and 1,201 -> 41 us; 9 rows: 263 -> 30 and 978 -> 33 us.
-// Relative error (2-norm, against 64 bits) 4.1e-7 instead of 8.1e-7 at K 2,048, 8.1e-7 instead of 1.6e-6 at K 8,192: four chains for one.
+// rows (the library's best is 131 TFLOP/s at 4,096 cubed), by the latency of a workgroup's loads for few.
 // A workgroup of four waves owns TM rows of x and TN rows of w.  A stage is 64 k of both in LDS; wave i multiplies the k
 // 16 i .. 16 i + 15 of every stage for the whole tile (so that a fragment from LDS serves as many instructions as the tile has
 // rows or columns of 16) and the four waves' sums are added in a fixed order at the end: an output is the same four chains
 // over k whatever the tile, so a row's result depends neither on the rows beside it nor on how many there are.  The operand
 // lane l of an instruction holds row l % 16 and k = 4 (l / 16) + i in the i-th of four instructions: one 16-byte LDS read each.
-// LDS rows are 64 + 8 floats long: lanes 0-7 and 16-23, which a 16-byte read serves together, then touch all 64 banks once.
-// Loads run DEPTH stages ahead in registers.  K and the row strides multiples of 4, 16-byte aligned operands.
+// The loads write into LDS themselves (16 bytes a lane, the 64 lanes of an instruction side by side: 4 rows of 64 k), ST stages on their way or in
+// use.  The fragments of the next stage are read under the products of this one, behind the barrier at which the next
+// stage has come and every wave has read all of this one, whose place is given to a new stage there.
+// A row's sixteen pieces of 16 bytes lie in an order of their own, piece p of row r at place p ^ (2 (r % 8)): lanes 0-7 and 16-23, which a
+// 16-byte LDS read serves together, then touch all 64 banks once.
+// Against the kernel before, whose loads went through registers (the same sums, bit by bit): 777 rows, N 16,384, K 2,048: 558 -> 430 us (121
+// TFLOP/s), N 2,048, K 8,192: 276 -> 231 (113), N 3,072, K 2,048: 117 -> 86; 300 rows, N 2,048, K 8,192: 125 -> 101; 16 rows 34 -> 25, 64 rows, N 2,048, K 2,048:
+// 12.4 -> 10.0.  A third of that is addresses: with a 64-bit sum a load in the vector unit the first of these takes 481 us.
+// Relative error (2-norm, against 64 bits) 4.1e-7 at K 2,048, 8.1e-7 at K 8,192, half of the tiled kernel's above: four chains for one.
+// K and the row strides multiples of 4, 16-byte aligned operands.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define G32_K 64
-#define G32_LD (G32_K + 8)
-#define G32_MAX_BLOCKS 0xffffffL  // workgroups of 256 threads that one dimension of a launch holds
+#define G32_MAX_BLOCKS 0xffffffL    // workgroups of 256 threads that one dimension of a launch holds
+#define G32_MAX_STRIDE (1 << 24)    // 64 rows of fewer floats than this are addressed by 32 bits
 
-// ENDS: the loop is asked for its end at every stage, not every 2 DEPTH of them; same sums.
-template <int TM, int TN, int DEPTH, bool ENDS>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ out, const float* __restrict__ x,
-                                                                 const float* __restrict__ w, int M, int N, int K, int x_stride,
-                                                                 int out_stride, int m_tiles, int n_tiles) {
-  constexpr int ROWS = TM + TN, PER = ROWS / 16;  // 16-byte pieces of a stage per thread: a row's 16 pieces by 16 neighbouring threads
-  constexpr int MI = TM / 16, NI = TN / 16;
-  constexpr int STAGE = ROWS * G32_LD, JOIN = 4 * TM * (TN + 4);
-  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE > JOIN ? 2 * STAGE : JOIN];
+template <int TM, int TN, int ST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f32_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, int M, int N,
+                                                            int K, int x_stride, int out_stride, int m_tiles, int n_tiles) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  constexpr int ROWS = TM + TN, PER = ROWS / 16, MI = TM / 16, NI = TN / 16, STAGE = ROWS * G32_K, JOIN = 4 * TM * (TN + 4);
+  __shared__ __attribute__((aligned(16))) float lds[ST * STAGE > JOIN ? ST * STAGE : JOIN];
   // workgroups are dealt to the eight XCDs in launch order: an XCD takes every eighth tile of w and runs all tiles of x against
   // it one after the other, so that w is read into one L2 only
   const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
   const int nt = (turn / m_tiles) * 8 + xcd, mt = turn % m_tiles;
   if (nt >= n_tiles) return;
   const int m0 = mt * TM, n0 = nt * TN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int piece = tid & 15;  // k of this thread's pieces: 4 piece .. 4 piece + 3 of the stage
-  const float* src[PER];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int piece = 4 * (r ^ (2 * ((wave * 4 + g) & 7)));  // k of a stage that this lane fetches of each of its rows
+  // bytes from the tile's first row of x or w to this lane's piece of each row it fetches (32 bits: the launch sees to it); along K the scalar
+  // unit counts, so a load costs the vector unit nothing
+  unsigned from[PER];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
-    const int r = p * 16 + (tid >> 4);
-    src[p] = (r < TM ? x + (size_t)min(m0 + r, M - 1) * x_stride : w + (size_t)min(n0 + r - TM, N - 1) * K) + 4 * piece;
+    const int row = (p * 4 + wave) * 4 + g;
+    from[p] = 4u * ((p * 16 < TM ? (unsigned)min(row, M - 1 - m0) * x_stride : (unsigned)min(row - TM, N - 1 - n0) * K) + piece);
   }
-  f32x4 reg[DEPTH][PER];
+  const float *x0 = x + (size_t)m0 * x_stride, *w0 = w + (size_t)n0 * K;
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)x0, 0, 0xffffffff, 0x00020000);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)w0, 0, 0xffffffff, 0x00020000);
   const int stages = (K + G32_K - 1) / G32_K;
-  auto fetch = [&](f32x4* to, int stage) {
-    const int k = stage * G32_K + 4 * piece;
+  auto issue = [&](int buf, int stage) {
+    const int k = stage * G32_K;
+    if (k + G32_K <= K) {
 #pragma unroll
-    for (int p = 0; p < PER; ++p) to[p] = k < K ? *reinterpret_cast<const f32x4*>(src[p] + stage * G32_K) : f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  auto park = [&](const f32x4* from, int buf) {
+      for (int p = 0; p < PER; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(p * 16 < TM ? xr : wr, (lds_ptr)(lds + buf * STAGE + (p * 4 + wave) * 4 * G32_K), 16, from[p], 4 * k, 0, 0);
+    } else {
 #pragma unroll
-    for (int p = 0; p < PER; ++p) *reinterpret_cast<f32x4*>(&lds[buf * STAGE + (p * 16 + (tid >> 4)) * G32_LD + 4 * piece]) = from[p];
+      for (int p = 0; p < PER; ++p) {
+        const float* at = k + piece < K ? (p * 16 < TM ? x0 : w0) + from[p] / 4 + k : reinterpret_cast<const float*>(&tile_zeros);
+        __builtin_amdgcn_global_load_lds(at, (lds_ptr)(lds + buf * STAGE + (p * 4 + wave) * 4 * G32_K), 16, 0, 0);
+      }
+    }
   };
   f32x4 acc[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int frag = (lane & 15) * G32_LD + 16 * wave + 4 * (lane >> 4);
-  auto multiply = [&](int buf) {
+  const int frag = r * G32_K + 4 * ((4 * wave + g) ^ (2 * (r & 7)));
+  auto read = [&](int buf, f32x4* a, f32x4* b) {
     const float* base = &lds[buf * STAGE + frag];
-    f32x4 a[NI], b[MI];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) b[i] = *reinterpret_cast<const f32x4*>(base + i * 16 * G32_LD);
+    for (int j = 0; j < NI; ++j) a[j] = *reinterpret_cast<const f32x4*>(base + (TM + j * 16) * G32_K);
 #pragma unroll
-    for (int j = 0; j < NI; ++j) a[j] = *reinterpret_cast<const f32x4*>(base + (TM + j * 16) * G32_LD);
+    for (int i = 0; i < MI; ++i) b[i] = *reinterpret_cast<const f32x4*>(base + i * 16 * G32_K);
+  };
+  int buf = 0;
+  // stage s + 1 has come and stage s has been read by all: on with the next, under the products of s
+  auto step = [&](int s, const f32x4* a, const f32x4* b, f32x4* a_next, f32x4* b_next) {
+    if (s + ST <= stages)
+      TILE_WAIT_LOADS((ST - 2) * PER);
+    else
+      TILE_WAIT_LOADS(0);
+    TILE_WAIT_LDS();
+    TILE_BARRIER();
+    if (s + ST < stages) issue(buf, s + ST);
+    buf = buf + 1 == ST ? 0 : buf + 1;
+    read(buf, a_next, b_next);  // (behind the last stage: what happens to lie there, not used)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -207,26 +234,28 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ out, 
         for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][e], b[i][e], acc[i][j], 0, 0, 0);
   };
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) fetch(reg[d], d);  // (a stage beyond K is zeros)
-  park(reg[0], 0);
-  for (int s0 = 0; s0 < stages; s0 += 2 * DEPTH) {
-#pragma unroll
-    for (int u = 0; u < 2 * DEPTH; ++u) {  // (stages beyond K, at most 2 DEPTH - 1, add zeros, unless ENDS)
-      const int s = s0 + u;
-      if (ENDS && s >= stages) break;
-      __syncthreads();
-      fetch(reg[u % DEPTH], s + DEPTH);
-      multiply(u & 1);
-      park(reg[(u + 1) % DEPTH], (u + 1) & 1);
-    }
+  for (int s = 0; s < ST; ++s)
+    if (s < stages) issue(s, s);
+  if (ST <= stages)
+    TILE_WAIT_LOADS((ST - 1) * PER);
+  else
+    TILE_WAIT_LOADS(0);
+  TILE_BARRIER();
+  f32x4 a0[NI], b0[MI], a1[NI], b1[MI];
+  read(0, a0, b0);
+  int s = 0;
+  for (; s + 1 < stages; s += 2) {
+    step(s, a0, b0, a1, b1);
+    step(s + 1, a1, b1, a0, b0);
   }
-  __syncthreads();
+  if (s < stages) step(s, a0, b0, a1, b1);
   // the waves' sums: [wave][row of x][row of w], rows 16 bytes apart from a multiple of the banks
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j)
-      *reinterpret_cast<f32x4*>(&lds[(wave * TM + i * 16 + (lane & 15)) * (TN + 4) + j * 16 + 4 * (lane >> 4)]) = acc[i][j];
+      *reinterpret_cast<f32x4*>(&lds[(wave * TM + i * 16 + r) * (TN + 4) + j * 16 + 4 * g]) = acc[i][j];
   __syncthreads();
   for (int e = tid; e < TM * TN / 4; e += 256) {
     const int m = e / (TN / 4), n = 4 * (e % (TN / 4));
@@ -241,18 +270,15 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ out, 
         if (n0 + n + c < N) o[c] = sum[c];
     }
   }
+#endif
 }
 
-template <int TM, int TN, int DEPTH>
+template <int TM, int TN, int ST>
 static int launch_gemm_f32(float* out, const float* x, const float* w, int M, int N, int K, int x_stride, int out_stride, hipStream_t stream) {
   const int m_tiles = (M + TM - 1) / TM, n_tiles = (N + TN - 1) / TN;
   const long blocks = (long)m_tiles * ((n_tiles + 7) / 8 * 8);
   if (blocks > G32_MAX_BLOCKS) return NS_ERR_BAD_ARG;
-  // Asking at every stage costs a long K up to 15% (777 rows, N 2,048, K 8,192: 273 -> 325 us) and saves a short one the stages of zeros behind
-  // its last (2,048 rows, N 2,048, K 64: 45 -> 18 us): it pays where they are more than a fifth of the others.
-  const int stages = (K + G32_K - 1) / G32_K, zeros = (2 * DEPTH - stages % (2 * DEPTH)) % (2 * DEPTH);
-  (5 * zeros > stages ? gemm_f32_kernel<TM, TN, DEPTH, true> : gemm_f32_kernel<TM, TN, DEPTH, false>)<<<(unsigned)blocks, 256, 0, stream>>>(
-      out, x, w, M, N, K, x_stride, out_stride, m_tiles, n_tiles);
+  gemm_f32_kernel<TM, TN, ST><<<(unsigned)blocks, 256, 0, stream>>>(out, x, w, M, N, K, x_stride, out_stride, m_tiles, n_tiles);
   return ns_launch_status();
 }
 
@@ -262,10 +288,11 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
   if (M <= 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N) return NS_ERR_BAD_ARG;
   dim3 grid((N + GT_N - 1) / GT_N, (M + GT_M - 1) / GT_M);
   if (grid.y > 65535) return NS_ERR_BAD_ARG;
-  // (more tiles of 32 x 32, in groups of eight, or of eight rows of w than one dimension of a launch holds: the plain kernel, which has two)
+  // (more tiles of 32 x 32, in groups of eight, or of eight rows of w than one dimension of a launch holds: the plain kernel, which has two;
+  // and where 32 bits do not address a tile's rows)
   const long tiles = (long)((M + 31) / 32) * (((long)N + 255) / 256 * 8);
   if (dtype == NS_DTYPE_F32 && K % 4 == 0 && x_stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && tiles <= G32_MAX_BLOCKS &&
-      N < (1 << 26)) {
+      N < (1 << 26) && x_stride < G32_MAX_STRIDE) {
     float* o = (float*)out;
     const float *xf = (const float*)x, *wf = (const float*)w;
     if (M <= ROWS_M) {
@@ -280,12 +307,13 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
         gemm_rows_f32_kernel<8><<<blocks, 64 * ROWS_WAVES, 0, stream>>>(o, xf, wf, M, N, K, x_stride, out_stride);
       return ns_launch_status();
     }
-    // Tiles of 32 x 32 where they fill the GPU and are not half empty, of 16 x 16 otherwise (777 rows, N 16,384, K 2,048: 512
-    // against 740 us; 16 rows there 41 against 30; 64 rows, N 2,048, K 8,192: 73 against 41).  Larger tiles deal less evenly and
-    // leave fewer workgroups to hide each other's loads (64 x 64: 583 us in the first of these, 350 against 283 at N 2,048, K 8,192).
-    if (M <= 16 || (long)((M + 31) / 32) * ((N + 31) / 32) < 256)
-      return launch_gemm_f32<16, 16, 8>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
-    return launch_gemm_f32<32, 32, 4>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+    // Tiles of 32 x 64 where there are four for every compute unit (777 rows, N 16,384, K 2,048: 430 against 442 us, 2,048 rows 1,066 against
+    // 1,171), of 32 x 32 where they fill the GPU and are not half empty (777 rows, N 2,048, K 8,192: 231 against 253; 100 rows 50 against 57
+    // with 16 x 16), of 16 x 16 otherwise (64 rows, N 2,048, K 8,192: 36 against 50).  64 x 64 deals less evenly (443 us in the first of these).
+    const long m32 = (M + 31) / 32;
+    if (M <= 16 || m32 * ((N + 31) / 32) < 256) return launch_gemm_f32<16, 16, 8>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+    if (m32 * ((N + 63) / 64) >= 1024) return launch_gemm_f32<32, 64, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+    return launch_gemm_f32<32, 32, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
   }
   if (dtype == NS_DTYPE_F32)
     gemm_generic_kernel<float, float><<<grid, 256, 0, stream>>>((float*)out, (const float*)x, (const float*)w, M, N, K, x_stride, out_stride);

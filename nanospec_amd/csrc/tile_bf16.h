@@ -8,25 +8,13 @@
 // The order.  A stage is two halves of 32 k.  While the products of one half run, the fragments of the next are read; the wait for the
 // next stage and the barrier stand between the halves, where every wave has work of its own in the matrix unit and the last
 // reads of a stage are done, so the stage's place is given to a new one right behind the barrier.
-// The waits are counted by hand (`s_waitcnt vmcnt(n)` before a plain `s_barrier`): __syncthreads() would wait for the stages that
-// are still wanted in flight.  No other vector load may be issued between start() and the end of run().
+// The waits are counted by hand (lds_loads.h).  No other vector load may be issued between start() and the end of run().
 #pragma once
-#include "common.h"
+#include "lds_loads.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 
 #define TILE_K 64
-#define TILE_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
-#define TILE_WAIT_LDS() __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4))
-#define TILE_BARRIER()             \
-  do {                             \
-    asm volatile("" ::: "memory"); \
-    __builtin_amdgcn_s_barrier();  \
-    asm volatile("" ::: "memory"); \
-  } while (0)
-
-static __device__ const int4 tile_zeros = {0, 0, 0, 0};  // what stands for a piece beyond K
-
 // WR x WC waves; wave (wm, wn) owns the blocks of 16 rows wm, wm + WR, .. of x (so that a tile whose last blocks are empty keeps all waves
 // equally busy) and 16 NJ neighbouring rows of w.  acc[i][j]: lane l holds for row 16 (WR i + wm) + l % 16 of x the sums with rows 16 NJ wn + 16 j +
 // 4 (l / 16) .. + 3 of w.

@@ -31,8 +31,8 @@ struct TileBf16 {
 
   typedef float f32x4 __attribute__((__vector_size__(4 * sizeof(float))));
   bf16_t* lds;
-  int lane, wave, wm, wn, K, stages, turn;
-  const bf16_t* src[PER];  // this lane's piece of each row it fetches, at k = 0
+  int lane, wave, wm, wn, K, stages, turn, next;
+  const bf16_t* src[PER];  // this lane's piece of each row it fetches: at k = 0, from start() on at the next stage to fetch
   f32x4 acc[MI][NJ];
 
   // the row of x (p < PA) or w that load p of this lane fetches
@@ -52,30 +52,43 @@ struct TileBf16 {
       for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  __device__ __forceinline__ void issue(int buf, int stage) {
+  __device__ __forceinline__ void issue(int buf) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef __attribute__((address_space(3))) void* lds_ptr;
     bf16_t* to = lds + buf * STAGE + wave * 8 * TILE_K;
-    const int k = (stage + turn < stages ? stage + turn : stage + turn - stages) * TILE_K;
-    const bool whole = k + TILE_K <= K;
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-      const bf16_t* from = src[p] + k;
-      if (!whole && k + piece() >= K) from = reinterpret_cast<const bf16_t*>(&tile_zeros);
+    const int k = next;  // of the stage that is issued: they come in order
+    auto load = [&](int p, const bf16_t* from) {
       const lds_ptr at = (lds_ptr)(to + (p < PA ? p * WAVES * 8 * TILE_K : (BM + (p - PA) * WAVES * 8) * TILE_K));
       if (W_ONCE && p >= PA)
         __builtin_amdgcn_global_load_lds(from, at, 16, 0, 2);  // (non-temporal)
       else
         __builtin_amdgcn_global_load_lds(from, at, 16, 0, 0);
+    };
+    if (k + TILE_K <= K) {  // (no selection where none is needed, and one sum a load: the vector unit is short of time here)
+#pragma unroll
+      for (int p = 0; p < PER; ++p) load(p, src[p]), src[p] += TILE_K;
+      next += TILE_K;
+      if (next == K) {
+        next = 0;
+#pragma unroll
+        for (int p = 0; p < PER; ++p) src[p] -= K;
+      }
+    } else {
+      const bool in = k + piece() < K;
+#pragma unroll
+      for (int p = 0; p < PER; ++p) load(p, in ? src[p] : reinterpret_cast<const bf16_t*>(&tile_zeros)), src[p] -= k;
+      next = 0;
     }
 #endif
   }
 
-  // the first stages on their way
   __device__ __forceinline__ void start() {
+    next = turn * TILE_K;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) src[p] += next;
 #pragma unroll
     for (int s = 0; s < ST; ++s)
-      if (s < stages) issue(s, s);
+      if (s < stages) issue(s);
   }
 
   template <int BLOCKS>
@@ -129,7 +142,7 @@ struct TileBf16 {
         TILE_WAIT_LOADS(0);
       TILE_WAIT_LDS();  // this wave has read all of stage s
       TILE_BARRIER();
-      if (s + ST < stages) issue(buf, s + ST);
+      if (s + ST < stages) issue(buf);
       buf = buf + 1 == ST ? 0 : buf + 1;
       __builtin_amdgcn_sched_barrier(0);
       frags<BLOCKS>(buf, 0, a0, b0);  // (behind the last stage: what happens to lie there, not used)

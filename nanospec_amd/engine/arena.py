@@ -8,8 +8,6 @@ buffers back for the next layer.
 
 from __future__ import annotations
 
-import math
-
 import torch
 
 _ALIGN = 256
@@ -20,46 +18,53 @@ class Arena:
     def __init__(self, device, nbytes: int = 0, fixed: bool = False) -> None:
         self.device, self.fixed = device, fixed
         self._chunks: list[torch.Tensor] = []
+        self._sizes: list[int] = []  # bytes of each chunk
         self._typed: dict = {}  # (chunk, dtype) -> the chunk seen as that type
         self._cur, self._off = -1, 0
         self.high_water = 0  # the most bytes that were in use at once since the arena was made (tails of chunks that a buffer
         #                      did not fit into count as used: one chunk of this size holds the same sequence of buffers)
         if nbytes:
-            self._chunks.append(torch.empty(nbytes, dtype=torch.uint8, device=device))
+            self._add(nbytes)
             self._cur = 0
 
+    def _add(self, nbytes: int) -> None:
+        self._chunks.append(torch.empty(nbytes, dtype=torch.uint8, device=self.device))
+        self._sizes.append(nbytes)
+
     def take(self, shape, dtype) -> torch.Tensor:
-        shape = tuple(int(s) for s in shape)
         esize = _ESIZE.get(dtype) or _ESIZE.setdefault(dtype, torch.empty(0, dtype=dtype).element_size())
-        count = math.prod(shape)
-        nbytes = max(1, count) * esize
-        need = -(-nbytes // _ALIGN) * _ALIGN
-        while self._cur < 0 or self._off + need > self._chunks[self._cur].numel():
+        # (a step of a small model asks a hundred times, kernel by kernel, and is bound by the host there: one view a buffer, no
+        # tensor asked for its size)
+        count, strides = 1, []
+        for s in reversed(shape):
+            strides.append(count)
+            count *= int(s)
+        strides.reverse()
+        need = -(-max(1, count) * esize // _ALIGN) * _ALIGN
+        while self._cur < 0 or self._off + need > self._sizes[self._cur]:
             if self._cur + 1 < len(self._chunks):
                 self._cur, self._off = self._cur + 1, 0
                 continue
             if self.fixed:
-                raise RuntimeError(f"a fixed arena of {sum(c.numel() for c in self._chunks)} bytes is exhausted")
-            size = max(need, 2 * sum(c.numel() for c in self._chunks), 1 << 20)
-            self._chunks.append(torch.empty(size, dtype=torch.uint8, device=self.device))
+                raise RuntimeError(f"a fixed arena of {sum(self._sizes)} bytes is exhausted")
+            self._add(max(need, 2 * sum(self._sizes), 1 << 20))
             self._cur, self._off = len(self._chunks) - 1, 0
-        # a view of the chunk in the wanted type is kept, so a buffer costs one slice and one reshape (offsets are
-        # multiples of 256 bytes, hence of every element size)
+        # a view of the chunk in the wanted type is kept, so a buffer costs one view (offsets are multiples of 256 bytes,
+        # hence of every element size)
         typed = self._typed.get((self._cur, dtype))
         if typed is None:
             chunk = self._chunks[self._cur]
-            typed = self._typed[self._cur, dtype] = chunk[: chunk.numel() // esize * esize].view(dtype)
-        first = self._off // esize
-        out = typed[first : first + count].view(shape)
+            typed = self._typed[self._cur, dtype] = chunk[: self._sizes[self._cur] // esize * esize].view(dtype)
+        out = typed.as_strided(tuple(shape), tuple(strides), self._off // esize)
         self._off += need
-        used = self._off + sum(c.numel() for c in self._chunks[: self._cur])
+        used = self._off + (sum(self._sizes[: self._cur]) if self._cur else 0)
         if used > self.high_water:
             self.high_water = used
         return out
 
     @property
     def capacity(self) -> int:
-        return sum(c.numel() for c in self._chunks)
+        return sum(self._sizes)
 
     def mark(self) -> tuple[int, int]:
         return self._cur, self._off
@@ -70,7 +75,8 @@ class Arena:
     def reset(self) -> None:
         """Start of a step.  Several chunks mean the arena grew during the last step: merge them."""
         if len(self._chunks) > 1 and not self.fixed:
-            total = sum(c.numel() for c in self._chunks)
-            self._chunks = [torch.empty(total, dtype=torch.uint8, device=self.device)]
+            total = sum(self._sizes)
+            self._chunks, self._sizes = [], []
             self._typed.clear()
+            self._add(total)
         self._cur, self._off = (0, 0) if self._chunks else (-1, 0)

@@ -1223,6 +1223,32 @@ def test_moe_router_of_many_tokens_is_as_exact_as_the_plain_kernel(n, rows, widt
     assert err[0] <= err[1], err
 
 
+@pytest.mark.parametrize("experts,groups,keep,best", [(1, 1, 1, 1), (31, 1, 1, 2), (63, 9, 4, 2), (64, 1, 1, 1), (64, 32, 7, 2), (64, 64, 9, 2), (65, 13, 3, 1), (130, 5, 2, 2)])
+@pytest.mark.parametrize("n", [1, 6])
+def test_moe_choice_among_a_wave_of_experts_and_more(experts, groups, keep, best, n):
+    """The choice by lanes (up to 64 experts) and by turns: many equal scores, scores that are no numbers, the smallest and largest groups."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(experts + groups + n)
+    # a router of unit vectors: the logits are the input's columns, whole numbers (no two different pairs of their scores add up alike)
+    h = torch.randint(0, 4, (n, experts), generator=g).float()
+    per = experts // groups
+    top = min(4, keep * per)
+    corr = torch.zeros(experts)
+    corr[experts // 2] = float("nan")  # counts as the lowest score
+    sel, wt = torch.zeros(n, top, dtype=torch.int32, device=DEV), torch.zeros(n, top, device=DEV)
+    ops.moe_route(h.to(DEV), torch.eye(experts, device=DEV), None, top, sel, wt, score="sigmoid", correction=corr.to(DEV), groups=groups, keep=keep,
+                  group_best=best)
+    s = torch.sigmoid(h)
+    by = (s + corr).nan_to_num(nan=float("-inf"))
+    for t in range(n):
+        row = by[t].tolist()
+        tops = [sorted(row[i * per : (i + 1) * per], reverse=True)[: min(best, per)] for i in range(groups)]
+        order = sorted(range(groups), key=lambda i: (-sum(tops[i]), i))[:keep]
+        want = sorted((e for e in range(experts) if e // per in order), key=lambda e: (-row[e], e))[:top]
+        assert sel[t].tolist() == want
+        torch.testing.assert_close(wt[t].cpu(), s[t, want], rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,top,width", [(1, 1, 4), (3, 4, 1020), (5, 2, 1028), (2, 3, 2050)])
 def test_moe_combine(n, top, width, dtype):

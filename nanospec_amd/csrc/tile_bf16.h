@@ -82,6 +82,7 @@ struct TileBf16 {
 #endif
   }
 
+  // the rows' addresses to the stage to begin with, and the first stages on their way
   __device__ __forceinline__ void start() {
     next = turn * TILE_K;
 #pragma unroll

@@ -14,7 +14,7 @@
 
 The experts' matrices are stacked at load time ([experts, ff, W] and [experts, W, ff]).  Steps of few rows run one
 workgroup per (token, chosen expert), which streams that expert's matrices; steps of many rows sort the (token, expert)
-pairs by expert on the device and run the experts as grouped products of 16-row tiles (``csrc/moe.hip``).  Nothing
+pairs by expert on the device and run the experts as grouped products in tiles of up to 16 or 128 rows (``csrc/moe.hip``).  Nothing
 depends on the host knowing which experts were chosen, so a step can be captured.
 """
 

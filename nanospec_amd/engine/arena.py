@@ -78,5 +78,6 @@ class Arena:
             total = sum(self._sizes)
             self._chunks, self._sizes = [], []
             self._typed.clear()
+            self._cur, self._off = -1, 0  # (one chunk of that size may not be had where the several were: the next buffers then start anew)
             self._add(total)
         self._cur, self._off = (0, 0) if self._chunks else (-1, 0)

@@ -33,3 +33,23 @@ def test_a_fixed_arena_ends():
     a.take((256,), torch.float32)
     with pytest.raises(RuntimeError, match="exhausted"):
         a.take((1,), torch.float32)
+
+
+def test_a_merge_that_finds_no_memory_leaves_an_arena_that_works(monkeypatch):
+    a = Arena("cpu")
+    a.take((1 << 18,), torch.float32)
+    a.take((1 << 20,), torch.float32)  # (a second chunk)
+    empty = torch.empty
+
+    def none(*args, **kwargs):
+        raise torch.OutOfMemoryError("none left")
+
+    monkeypatch.setattr(torch, "empty", none)
+    with pytest.raises(torch.OutOfMemoryError):
+        a.reset()
+    with pytest.raises(torch.OutOfMemoryError):  # (still none: the allocation's own error, not one of the arena's books)
+        a.take((4,), torch.float32)
+    monkeypatch.setattr(torch, "empty", empty)
+    assert a.take((4,), torch.float32).fill_(1).sum() == 4 and a.capacity >= 16
+    a.reset()
+    assert a.take((4,), torch.float32).storage_offset() == 0

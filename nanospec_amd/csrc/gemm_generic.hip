@@ -9,6 +9,7 @@
 // (reference: the nn.Linear calls of model/llama.py:175,184,195,286)
 #include "common.h"
 #include "lds_loads.h"
+#include <type_traits>
 
 #define GT_M 64
 #define GT_N 64
@@ -159,7 +160,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define G32_MAX_BLOCKS 0xffffffL    // workgroups of 256 threads that one dimension of a launch holds
 #define G32_MAX_STRIDE (1 << 24)    // 64 rows of fewer floats than this are addressed by 32 bits
 
-template <int TM, int TN, int ST>
+// FAR: rows further apart than 32 bits address from a tile's first: every load by a 64-bit address from the vector unit (9 rows 2^24 floats apart
+// are 600 MB: such calls are rare, and the plain kernel would add up in one chain instead of four, at twice the error).
+template <int TM, int TN, int ST, bool FAR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f32_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, int M, int N,
                                                             int K, int x_stride, int out_stride, int m_tiles, int n_tiles) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -177,11 +180,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int piece = 4 * (r ^ (2 * ((wave * 4 + g) & 7)));  // k of a stage that this lane fetches of each of its rows
   // bytes from the tile's first row of x or w to this lane's piece of each row it fetches (32 bits: the launch sees to it); along K the scalar
   // unit counts, so a load costs the vector unit nothing
-  unsigned from[PER];
+  typedef typename std::conditional<FAR, size_t, unsigned>::type offset;
+  offset from[PER];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     const int row = (p * 4 + wave) * 4 + g;
-    from[p] = 4u * ((p * 16 < TM ? (unsigned)min(row, M - 1 - m0) * x_stride : (unsigned)min(row - TM, N - 1 - n0) * K) + piece);
+    from[p] = (offset)4 * ((p * 16 < TM ? (offset)min(row, M - 1 - m0) * x_stride : (offset)min(row - TM, N - 1 - n0) * K) + piece);
   }
   const float *x0 = x + (size_t)m0 * x_stride, *w0 = w + (size_t)n0 * K;
   const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)x0, 0, 0xffffffff, 0x00020000);
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int stages = (K + G32_K - 1) / G32_K;
   auto issue = [&](int buf, int stage) {
     const int k = stage * G32_K;
-    if (k + G32_K <= K) {
+    if (!FAR && k + G32_K <= K) {
 #pragma unroll
       for (int p = 0; p < PER; ++p)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(p * 16 < TM ? xr : wr, (lds_ptr)(lds + buf * STAGE + (p * 4 + wave) * 4 * G32_K), 16, from[p], 4 * k, 0, 0);
@@ -273,12 +277,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #endif
 }
 
-template <int TM, int TN, int ST>
+template <int TM, int TN, int ST, bool FAR = false>
 static int launch_gemm_f32(float* out, const float* x, const float* w, int M, int N, int K, int x_stride, int out_stride, hipStream_t stream) {
   const int m_tiles = (M + TM - 1) / TM, n_tiles = (N + TN - 1) / TN;
   const long blocks = (long)m_tiles * ((n_tiles + 7) / 8 * 8);
   if (blocks > G32_MAX_BLOCKS) return NS_ERR_BAD_ARG;
-  gemm_f32_kernel<TM, TN, ST><<<(unsigned)blocks, 256, 0, stream>>>(out, x, w, M, N, K, x_stride, out_stride, m_tiles, n_tiles);
+  gemm_f32_kernel<TM, TN, ST, FAR><<<(unsigned)blocks, 256, 0, stream>>>(out, x, w, M, N, K, x_stride, out_stride, m_tiles, n_tiles);
   return ns_launch_status();
 }
 
@@ -288,11 +292,10 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
   if (M <= 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N) return NS_ERR_BAD_ARG;
   dim3 grid((N + GT_N - 1) / GT_N, (M + GT_M - 1) / GT_M);
   if (grid.y > 65535) return NS_ERR_BAD_ARG;
-  // (more tiles of 32 x 32, in groups of eight, or of eight rows of w than one dimension of a launch holds: the plain kernel, which has two;
-  // and where 32 bits do not address a tile's rows)
+  // (more tiles of 32 x 32, in groups of eight, or of eight rows of w than one dimension of a launch holds: the plain kernel, which has two)
   const long tiles = (long)((M + 31) / 32) * (((long)N + 255) / 256 * 8);
   if (dtype == NS_DTYPE_F32 && K % 4 == 0 && x_stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && tiles <= G32_MAX_BLOCKS &&
-      N < (1 << 26) && x_stride < G32_MAX_STRIDE) {
+      N < (1 << 26)) {
     float* o = (float*)out;
     const float *xf = (const float*)x, *wf = (const float*)w;
     if (M <= ROWS_M) {
@@ -311,6 +314,7 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
     // 1,171), of 32 x 32 where they fill the GPU and are not half empty (777 rows, N 2,048, K 8,192: 231 against 253; 100 rows 50 against 57
     // with 16 x 16), of 16 x 16 otherwise (64 rows, N 2,048, K 8,192: 36 against 50).  64 x 64 deals less evenly (443 us in the first of these).
     const long m32 = (M + 31) / 32;
+    if (x_stride >= G32_MAX_STRIDE) return launch_gemm_f32<32, 32, 3, true>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
     if (M <= 16 || m32 * ((N + 31) / 32) < 256) return launch_gemm_f32<16, 16, 8>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
     if (m32 * ((N + 63) / 64) >= 1024) return launch_gemm_f32<32, 64, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
     return launch_gemm_f32<32, 32, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);

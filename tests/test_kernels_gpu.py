@@ -103,6 +103,19 @@ def test_linear_f32_forms(m, n, k):
     assert torch.equal(ops.linear_generic(x[:rows], w), out[:rows, :n])
 
 
+@pytest.mark.parametrize("m", [1, 8, 9, 33])
+@pytest.mark.parametrize("stride", [(1 << 24) - 4, 1 << 24])
+@pytest.mark.parametrize("n,k", [(130, 68), (4130, 324)])
+def test_linear_f32_of_rows_far_apart(m, stride, n, k):
+    """Rows that 32 bits address from a tile's first and rows that they do not: the same sums, bit by bit, as of rows side by side."""
+    ops = _ops()
+    torch.manual_seed(m + n)
+    x, w = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
+    far = torch.empty((m - 1) * stride + k, device=DEV).as_strided((m, k), (stride, 1))
+    far.copy_(x)
+    assert torch.equal(ops.linear_generic(far, w), ops.linear_generic(x, w))
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("n,k", [(48, 64), (130, 200), (1000, 4096), (257, 1064), (16, 8), (4096, 14336)])
 def test_linear_tiled(m, n, k):

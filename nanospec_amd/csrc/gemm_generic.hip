@@ -315,7 +315,15 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
     // with 16 x 16), of 16 x 16 otherwise (64 rows, N 2,048, K 8,192: 36 against 50).  64 x 64 deals less evenly (443 us in the first of these).
     const long m32 = (M + 31) / 32;
     if (x_stride >= G32_MAX_STRIDE) return launch_gemm_f32<32, 32, 3, true>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
-    if (M <= 16 || m32 * ((N + 31) / 32) < 256) return launch_gemm_f32<16, 16, 8>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+    if (M <= 16 || m32 * ((N + 31) / 32) < 256) {
+      // Eight stages of a 16 x 16 tile take 64 KB of LDS, two workgroups a compute unit.  Where an XCD has more of them than that, three stages
+      // and up to six workgroups hide the loads better: 96 rows, N 2,048, K 2,048 (768 tiles): 14.8 -> 12.2 us, K 8,192: 47.9 -> 34.4; 2,048 rows, N 64
+      // (on four XCDs), K 64: 4.3 -> 3.7; 1,024 rows, N 132, K 4,096: 36.3 -> 25.9.  Up to 16 rows and a long K the weight's bytes bound it,
+      // and eight stages bring them faster (16 rows, N 128,256, K 512: 51 us and 41 with three, K 768: 91 and 88, K 2,048: 196 and 206; N 28,672, K 6,144: 135 and 149).
+      const long slots = (long)((M + 15) / 16) * (((long)N + 127) / 128 * 8);
+      if (slots > 512 && (M > 16 || K <= 960)) return launch_gemm_f32<16, 16, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+      return launch_gemm_f32<16, 16, 8>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
+    }
     if (m32 * ((N + 63) / 64) >= 1024) return launch_gemm_f32<32, 64, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
     return launch_gemm_f32<32, 32, 3>(o, xf, wf, M, N, K, x_stride, out_stride, stream);
   }

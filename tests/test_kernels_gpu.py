@@ -86,10 +86,11 @@ def test_linear_generic(dtype, m, n, k):
 
 
 @pytest.mark.parametrize("m", [1, 2, 3, 8, 9, 16, 17, 33, 515])
-@pytest.mark.parametrize("n,k", [(1, 4), (7, 2052), (33, 60), (130, 64), (700, 516), (4100, 576), (4130, 100), (65, 2500)])
+@pytest.mark.parametrize("n,k", [(1, 4), (7, 2052), (33, 60), (130, 64), (700, 516), (4100, 576), (4130, 100), (65, 2500),
+                                 (250, 516), (8210, 252)])
 def test_linear_f32_forms(m, n, k):
     """32-bit products of few and of many rows at the edges of their tiles (8 rows or columns, 16, 32, 64), of a stage of 64 k and of
-    the stages that are in flight; rows of x and of the result with a stride of their own."""
+    the stages that are in flight (three or eight, before and after a place in LDS is used again); rows of x and of the result with a stride of their own."""
     ops = _ops()
     torch.manual_seed(m + n + k)
     wide = torch.randn(m, k + 12, device=DEV)

@@ -489,6 +489,20 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 #define MG_ROWS 128                                 // rows of a tile at most
 typedef TileBf16<MG_ROWS, 256, 2, 4, 3> MoeTile;        // by 256 rows of the matrices: one workgroup of eight waves a compute unit
 typedef TileBf16<MG_ROWS, 128, 2, 2, 2, true> MoeFewTile;  // by 128: two workgroups of four waves
+#define MG_GROUP 4                                  // blocks of channels that an expert's tiles take together
+
+// What a tile is, in three words, from which a workgroup works out any tile of the same expert without another trip to memory: ``tile_e`` the expert
+// and which of its tiles this is (-1: no tile), ``tile_r0`` the expert's first sorted row, ``tile_rows`` the expert's rows.
+#define MG_E_BITS 10
+static_assert(MOE_MAX_EXPERTS <= 1 << MG_E_BITS, "2^24 pairs in tiles of 16: an expert has 2^20 tiles at most");
+__device__ __forceinline__ int tile_expert(int word) { return word & ((1 << MG_E_BITS) - 1); }
+
+// rows before tile ``i`` of ``t`` even tiles of ``c`` rows (whole blocks of 16; c itself for i = t)
+__device__ __forceinline__ int rows_before_tile(int c, int t, int i) {
+  if (t == 1) return i ? c : 0;
+  const int blocks = (c + 15) / 16;
+  return min(c, 16 * (i * (blocks / t) + min(i, blocks % t)));
+}
 
 // Pairs sorted by expert and every expert's pairs cut into the fewest tiles of at most ``cap`` rows, as even as whole blocks of
 // 16 rows allow (an expert with a few rows more than ``cap`` makes two tiles of about half, not a full one and a sliver).  The counts
@@ -521,12 +535,9 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   }
   __syncthreads();
   for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-    const int c = cnt[e], t = (c + cap - 1) / cap, blocks = (c + 15) / 16;
-    for (int i = 0, at = 0; i < t; ++i) {
-      const int rows = min(c - at, 16 * (blocks / t + (i < blocks % t ? 1 : 0)));
-      tile_e[tiles_of[e] + i] = e, tile_r0[tiles_of[e] + i] = cur[e] + at, tile_rows[tiles_of[e] + i] = rows;
-      at += rows;
-    }
+    const int c = cnt[e], t = (c + cap - 1) / cap;
+    for (int i = 0; i < t; ++i)
+      tile_e[tiles_of[e] + i] = e | i << MG_E_BITS, tile_r0[tiles_of[e] + i] = cur[e], tile_rows[tiles_of[e] + i] = c;
   }
   // (max_tiles is at least one more than any choice uses: behind the last tile stands how many there are)
   for (int i = used + threadIdx.x; i < max_tiles; i += blockDim.x) tile_e[i] = -1, tile_r0[i] = used, tile_rows[i] = 0;
@@ -553,9 +564,10 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
                                                          int act_kind) {
   constexpr int MATS = DUAL ? 2 : 1;
   __shared__ __attribute__((aligned(16))) float part[4][MATS][16][20];  // [wave][matrix][row][channel]
-  const int tile = blockIdx.y, e = tile_e[tile];
-  if (e < 0) return;
-  const int r0 = tile_r0[tile], rows = tile_rows[tile], n0 = blockIdx.x * 16;
+  const int tile = blockIdx.y, word = tile_e[tile];
+  if (word < 0) return;
+  const int e = tile_expert(word), row0 = 16 * (word >> MG_E_BITS);  // (tiles of 16 rows: every one but an expert's last is full)
+  const int r0 = tile_r0[tile] + row0, rows = min(16, tile_rows[tile] - row0), n0 = blockIdx.x * 16;
   const int tid = threadIdx.x, lane = tid % NS_WAVE, wave = tid / NS_WAVE, r = lane % 16, g = lane / 16;
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const size_t wrow = ((size_t)e * N + min(n0 + r, N - 1)) * K + 8 * g;
@@ -613,8 +625,13 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
 // gates, width 2,048, four a token chosen evenly, sorting included, against the kernel before (128 x 128, operands through registers, two
 // barriers a piece): 100 tokens 94 -> 80 us, 508 112 -> 90, 1,024 153 -> 136, 1,531 182 -> 142, 2,048 241 -> 200; 1,536 channels
 // without gates, 2,048 tokens 244 -> 197.
-// Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the tiles in use, neighbours first, so that an expert's
-// matrices and rows come into one L2 (2,048 tokens: 216 -> 200 us).  Every expert and block of channels begins at a stage of K of its own:
+// Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the work in use, neighbours first, so that an expert's
+// matrices and rows come into one L2 (2,048 tokens: 216 -> 200 us).  Where an expert has several tiles, all of them take four blocks of
+// channels before the next four: all blocks of one tile first bring matrices larger than an L2 from beyond it once a tile.  8 experts, two a token,
+// width 4,096, with gates, chosen unevenly, all blocks of a tile first and as it is: 14,336 channels 2,000 tokens 2,264 and 1,689 us, 512 tokens 822 and 689, 4,096
+// channels 2,000 tokens 638 and 515.  (One block at a time is level there and behind with small matrices: 8 of 2,048, width 2,048, without
+// gates, 2,000 tokens 146 and with four 140.)
+// Every expert and block of channels begins at a stage of K of its own:
 // workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (508 tokens: 111 -> 90 us).
 template <class T, bool FIRST, bool DUAL>
 __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void moe_tile_kernel(
@@ -629,11 +646,20 @@ __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   const long long used = (long long)tile_r0[tiles - 1] * blocks_n, share = (used + 7) / 8;
   const long long item = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= share || item >= used) return;
-  const int tile = (int)(item / blocks_n), n0 = (int)(item % blocks_n) * CH;
-  const int e = tile_e[tile], r0 = tile_r0[tile], rows = tile_rows[tile];
+  // the expert that this item falls to and its first tile; then four blocks at a time, tile by tile
+  const int some = (int)(item / blocks_n), word = tile_e[some], c = tile_rows[some], e = tile_expert(word), of_e = (c + MG_ROWS - 1) / MG_ROWS;
+  const long long at = item - (long long)(some - (word >> MG_E_BITS)) * blocks_n;
+  int nth = 0, block = (int)at;
+  if (of_e > 1) {
+    const int group = (int)(at / (MG_GROUP * of_e)), in_group = (int)(at % (MG_GROUP * of_e));
+    const int wide = min(MG_GROUP, blocks_n - MG_GROUP * group);
+    nth = in_group / wide, block = MG_GROUP * group + in_group % wide;
+  }
+  const int row0 = rows_before_tile(c, of_e, nth), rows = rows_before_tile(c, of_e, nth + 1) - row0;
+  const int n0 = block * CH, r0 = tile_r0[some] + row0;
 
   T t;
-  t.init(moe_tiles, K, (int)(item % blocks_n) * 7 + e * 11);
+  t.init(moe_tiles, K, block * 7 + e * 11);
 #pragma unroll
   for (int p = 0; p < T::PER; ++p) {
     const int row = t.row_of(p);

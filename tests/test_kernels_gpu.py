@@ -1161,10 +1161,13 @@ def test_attention_f32_keeps_infinities_to_the_rows_that_see_them():
 @pytest.mark.parametrize("n,experts,top,width,ff,gated", [(8, 8, 4, 64, 24, True), (16, 32, 4, 136, 40, False), (33, 32, 4, 72, 136, True), (40, 5, 2, 264, 16, True),
                                                           (130, 3, 1, 64, 264, False), (517, 70, 3, 128, 72, True), (64, 256, 8, 64, 16, True), (65, 256, 8, 64, 16, True),
                                                           (80, 256, 8, 64, 136, False), (80, 256, 8, 64, 16, False), (400, 6, 2, 136, 136, True),
-                                                          (450, 3, 1, 72, 264, False), (150, 4, 2, 520, 264, True)])
+                                                          (450, 3, 1, 72, 264, False), (150, 4, 2, 520, 264, True), (400, 6, 2, 328, 264, True),
+                                                          (400, 3, 2, 1320, 648, True), (450, 3, 1, 648, 1320, False), (300, 7, 2, 712, 328, True),
+                                                          (300, 7, 2, 328, 712, False)])
 def test_moe_expert_groups(routing, n, experts, top, width, ff, gated):
     """The sorted experts' products, streamed and tiled: tiles of 1 to 16 and to 128 rows in both forms, experts with more rows than a tile and with
-    none, pairs without an expert, sizes that end inside a tile and inside a piece of K."""
+    none, several tiles of an expert over more blocks of channels than they take together, pairs without an expert, sizes that end inside
+    a tile and inside a piece of K, before and after a place in LDS is used again."""
     ops = _ops()
     g = torch.Generator().manual_seed(n + experts)
     rnd = lambda *shape: torch.randn(*shape, generator=g)

@@ -644,8 +644,8 @@ __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   __shared__ __attribute__((aligned(16))) bf16_t moe_tiles[T::ST * T::STAGE];
   const int blocks_n = (N + CH - 1) / CH;
   const long long used = (long long)tile_r0[tiles - 1] * blocks_n, share = (used + 7) / 8;
-  const long long item = (blockIdx.x & 7) * share + (blockIdx.x >> 3);
-  if ((blockIdx.x >> 3) >= share || item >= used) return;
+  const long long turn = (long long)blockIdx.y * (gridDim.x >> 3) + (blockIdx.x >> 3), item = (blockIdx.x & 7) * share + turn;
+  if (turn >= share || item >= used) return;
   // the expert that this item falls to and its first tile; then four blocks at a time, tile by tile
   const int some = (int)(item / blocks_n), word = tile_e[some], c = tile_rows[some], e = tile_expert(word), of_e = (c + MG_ROWS - 1) / MG_ROWS;
   const long long at = item - (long long)(some - (word >> MG_E_BITS)) * blocks_n;
@@ -725,6 +725,18 @@ extern "C" int ns_moe_group_tiles(int pairs, int experts, int ff, int gated) {
   return (pairs + cap - 1) / cap + experts;
 }
 
+// The launch for so many items of a tile and a block of channels: the XCDs' eight workgroups of a turn side by side, and the turns in two dimensions,
+// because one holds fewer than 2^32 threads.
+static dim3 moe_tile_grid(long long items) {
+  const long long turns = (items + 7) / 8, row = turns < 65536 ? turns : 65536;
+  return dim3((unsigned)(8 * row), (unsigned)((turns + row - 1) / row));
+}
+
+extern "C" void ns_moe_tile_grid(long long items, unsigned* xy) {
+  const dim3 grid = moe_tile_grid(items);
+  xy[0] = grid.x, xy[1] = grid.y;
+}
+
 struct MoeLaunch {
   const bf16_t *h, *wg, *wu, *wd;
   bf16_t* act;
@@ -739,9 +751,9 @@ struct MoeLaunch {
   template <class T, bool FIRST, bool DUAL>
   void tiled(const bf16_t* a, int a_stride, const bf16_t* b0, const bf16_t* b1, int n, int k) const {
     constexpr int CH = DUAL ? T::BN / 2 : T::BN;
-    const long long blocks = ((long long)tiles * ((n + CH - 1) / CH) + 7) / 8 * 8;
-    moe_tile_kernel<T, FIRST, DUAL><<<(unsigned)blocks, T::THREADS, 0, stream>>>(a, a_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, tiles, act, out, wt,
-                                                                                 n, k, top, limit, alpha, shift, act_kind);
+    const dim3 grid = moe_tile_grid((long long)tiles * ((n + CH - 1) / CH));
+    moe_tile_kernel<T, FIRST, DUAL><<<grid, T::THREADS, 0, stream>>>(a, a_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, tiles, act, out, wt, n, k, top,
+                                                                     limit, alpha, shift, act_kind);
   }
   template <bool DUAL>
   void first(int cap) const {

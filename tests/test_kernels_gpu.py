@@ -1266,6 +1266,26 @@ def test_moe_choice_among_a_wave_of_experts_and_more(experts, groups, keep, best
         torch.testing.assert_close(wt[t].cpu(), s[t, want], rtol=1e-6, atol=0)
 
 
+def test_moe_tiles_of_more_blocks_than_a_row_of_the_launch():
+    """One expert of more channels than 8 x 65,536 workgroups of 64 take: the launch's second dimension."""
+    ops = _ops()
+    ff, width, n = (1 << 25) + 4104, 8, 3
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rnd = lambda *shape: torch.randint(-2, 3, shape, generator=g, device=DEV, dtype=torch.int8).bfloat16()
+    h, gate, up, down = rnd(n, width), rnd(1, ff, width), rnd(1, ff, width), torch.zeros(1, width, ff, dtype=torch.bfloat16, device=DEV)
+    sel, wt = torch.zeros(n, 1, dtype=torch.int32, device=DEV), torch.ones(n, 1, device=DEV)
+    act = torch.full((n, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ints, out = torch.zeros(64, dtype=torch.int32, device=DEV), torch.full((n, 1, width), float("nan"), device=DEV)
+    ops.moe_expert_groups(h, gate, up, down, sel, wt, float("inf"), 1.0, ints, act, out, shift=0.0)
+    assert bool((out == 0).all())
+    perm = ints[:n].long()  # (the places that the pairs got)
+    for i in range(n):
+        x = h[perm[i]].float()
+        for at in range(0, ff, 1 << 20):
+            a, b = gate[0, at : at + (1 << 20)].float() @ x, up[0, at : at + (1 << 20)].float() @ x  # whole numbers, exact
+            torch.testing.assert_close(act[i, at : at + (1 << 20)].float(), a * torch.sigmoid(a) * b, rtol=2.0 ** -7, atol=1e-6)  # (one rounding to bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,top,width", [(1, 1, 4), (3, 4, 1020), (5, 2, 1028), (2, 3, 2050)])
 def test_moe_combine(n, top, width, dtype):

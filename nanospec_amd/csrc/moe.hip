@@ -696,7 +696,11 @@ __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         }
         *reinterpret_cast<bf16x4*>(act_out + (size_t)slot * N + col) = o;
       } else {
-        *reinterpret_cast<f32x4*>(out + (size_t)pair * N + col) = share_of * t.acc[i][j];
+        typedef float f32x4_anywhere __attribute__((ext_vector_type(4), aligned(4)));  // (``out`` is a float's address and no more)
+        f32x4_anywhere o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = share_of * t.acc[i][j][q];
+        *reinterpret_cast<f32x4_anywhere*>(out + (size_t)pair * N + col) = o;
       }
     }
   }

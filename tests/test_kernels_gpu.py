@@ -1266,6 +1266,25 @@ def test_moe_choice_among_a_wave_of_experts_and_more(experts, groups, keep, best
         torch.testing.assert_close(wt[t].cpu(), s[t, want], rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("n,experts,ff", [(24, 8, 264), (200, 8, 264), (700, 4, 136)])
+def test_moe_results_at_any_address(n, experts, ff):
+    """A result that begins a float behind a 16-byte boundary: streamed, in the smaller tiles and in the larger ones."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    width, top = 136, 1
+    h, gate, up, down = rnd(n, width), rnd(experts, ff, width), rnd(experts, ff, width), rnd(experts, width, ff)
+    sel, wt = torch.randint(0, experts, (n, top), generator=g, device=DEV, dtype=torch.int32), torch.rand(n, top, generator=g, device=DEV)
+    got = []
+    for first in (0, 1):
+        out = torch.full((first + n * top * width + 3,), 7.0, device=DEV)
+        ints, act = torch.zeros(8 * (n + experts), dtype=torch.int32, device=DEV), torch.zeros(n * top, ff, dtype=torch.bfloat16, device=DEV)
+        ops.moe_expert_groups(h, gate, up, down, sel, wt, 7.0, 1.702, ints, act, out[first : first + n * top * width].view(n, top, width))
+        assert bool((out[:first] == 7).all()) and bool((out[first + n * top * width :] == 7).all())
+        got.append(out[first : first + n * top * width])
+    assert torch.equal(*got)
+
+
 def test_moe_tiles_of_more_blocks_than_a_row_of_the_launch():
     """One expert of more channels than 8 x 65,536 workgroups of 64 take: the launch's second dimension."""
     ops = _ops()

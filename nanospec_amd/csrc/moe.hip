@@ -223,7 +223,8 @@ __global__ __launch_bounds__(64) void moe_choose_kernel(const float* __restrict_
         if (v > a) b = a, a = v;
         else if (v > b) b = v;
       }
-      gs[g] = per > 1 && group_best > 1 ? a + b : a;
+      const float v = per > 1 && group_best > 1 ? a + b : a;
+      gs[g] = v == v ? v : -INFINITY;  // (what is no number, an expert's score or a group's, counts as the lowest: it would stop the exchange below)
       gkept[g] = 0;
     }
     __syncthreads();

@@ -1305,6 +1305,40 @@ def test_moe_tiles_of_more_blocks_than_a_row_of_the_launch():
             torch.testing.assert_close(act[i, at : at + (1 << 20)].float(), a * torch.sigmoid(a) * b, rtol=2.0 ** -7, atol=1e-6)  # (one rounding to bfloat16)
 
 
+@pytest.mark.parametrize("score", ["softmax", "sigmoid", "softmax_all"])
+@pytest.mark.parametrize("infinite", ["lowest", "both"])
+@pytest.mark.parametrize("experts,groups,keep,best,top", [(8, 1, 1, 1, 3), (8, 4, 2, 2, 3), (64, 32, 7, 2, 8), (64, 1, 1, 2, 12), (66, 1, 1, 1, 4), (130, 65, 9, 2, 8), (130, 5, 2, 2, 6)])
+def test_moe_choice_among_scores_that_are_not_finite(score, infinite, experts, groups, keep, best, top):
+    """Both forms of the choice, every score: infinite logits, corrections that are infinite or no number, groups whose two best add up to no number
+    (they count as the lowest, like experts' scores that are none)."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(experts + groups)
+    n, per, inf = 6, experts // groups, float("inf")
+    h = torch.randint(0, 4, (n, experts), generator=g).float()  # the logits: the router is of unit vectors
+    bias, corr = torch.zeros(experts), torch.zeros(experts)
+    bias[1::5] = -inf
+    if infinite == "both" and score != "softmax_all":  # (an infinite logit leaves no number among a soft-max's scores)
+        bias[2::7] = inf
+    corr[experts // 2] = float("nan")
+    if infinite == "both":
+        corr[0], corr[1], corr[experts - 1] = inf, -inf, -inf
+    corr = None if score == "softmax" else corr
+    sel, wt = torch.zeros(n, top, dtype=torch.int32, device=DEV), torch.zeros(n, top, device=DEV)
+    ops.moe_route(h.to(DEV), torch.eye(experts, device=DEV), bias.to(DEV), top, sel, wt, score=score, correction=None if corr is None else corr.to(DEV),
+                  groups=groups, keep=keep, group_best=best)
+    lowest = lambda v: v if v == v else -inf
+    for t in range(n):
+        z = h[t] + bias
+        w = {"softmax": z, "sigmoid": torch.sigmoid(z), "softmax_all": torch.softmax(z, 0)}[score]
+        row = [lowest(v) for v in (w if corr is None else w + corr).tolist()]
+        tops = [sorted(row[i * per : (i + 1) * per], reverse=True)[: min(best, per)] for i in range(groups)]
+        order = sorted(range(groups), key=lambda i: (-lowest(sum(tops[i])), i))[:keep]
+        want = sorted((e for e in range(experts) if e // per in order), key=lambda e: (-row[e], e))[:top]
+        assert sel[t].tolist() == want
+        chosen = torch.softmax(z[want], 0) if score == "softmax" else w[want] / (w[want].sum() if score == "softmax_all" else 1.0)
+        torch.testing.assert_close(wt[t].cpu(), chosen, rtol=1e-5, atol=0, equal_nan=True)  # (exponentials of 32 bits and a sum of up to 12)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,top,width", [(1, 1, 4), (3, 4, 1020), (5, 2, 1028), (2, 3, 2050)])
 def test_moe_combine(n, top, width, dtype):

@@ -324,6 +324,19 @@ __global__ __launch_bounds__(256) void moe_choose_lanes_kernel(const float* __re
   }
 }
 
+// Which of the two (the results are the same), by what each takes, in steps of a walk over the experts (35 ns a token's chain, 110 ns of 8,192 tokens):
+// by lanes one walk, three where experts are chosen in groups; by turns 20 an expert to choose, 10 a group to keep and 2.5 an expert of a
+// group; with the GPU full of tokens 27 and 18, and the turns' workgroups of one wave cost 28 to 32 more.  us by turns and by lanes, with the
+// logits, 64 tokens: 64 experts, one chosen 15.6 and 17.1, 8 chosen 20.5 and 17.3; 32 experts, one chosen 15.6 and 15.9, two 0.4 less by lanes;
+// 64 in 8 groups of which 4 are kept, two chosen 2.4 more by lanes, 8 chosen 1.6 less; 64 in 2 groups, one kept, 8 chosen 24.4 and 22.6; 32 in 8,
+// 4 kept, 4 chosen 2.4 less.  8,192 tokens: 64 in 8 groups, 4 kept, 4 chosen 5.3 less by lanes, one chosen 3.8 more.
+static bool moe_choose_by_lanes(int n, int experts, int top, int groups, int keep) {
+  if (experts > NS_WAVE) return false;
+  const bool full = n >= 4096;
+  if (groups == 1) return experts - (full ? 28 : 4) <= (full ? 27 : 20) * top;
+  return 3 * experts - (full ? 52 : 20) <= (full ? 27 : 20) * top + (full ? 18 : 10) * keep + 5 * (experts / groups) / 2;
+}
+
 // ``z``: float32 [n][experts + extra]; ``extra``: rows of ``wr`` (and ``br``) below the experts'
 extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const float* br, float* z, int* sel, float* wt, int n, int W, int experts,
                             int extra, int top, int score, const float* correction, int groups, int keep, int group_best, float scale, int dtype,
@@ -353,7 +366,7 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
     moe_logits_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
   else
     moe_logits_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows, vec);
-  if (experts <= NS_WAVE)
+  if (moe_choose_by_lanes(n, experts, top, groups, keep))
     moe_choose_lanes_kernel<<<(n + 3) / 4, 256, 0, stream>>>(z, rows, sel, wt, n, experts, top, score, correction, groups, keep, group_best, scale);
   else
     moe_choose_kernel<<<n, 64, 0, stream>>>(z, rows, sel, wt, n, experts, top, score, correction, groups, keep, group_best, scale);

@@ -29,6 +29,7 @@
 // 32x32 matrix instruction with keys and values loaded straight into LDS).  Compiled with -DNS_PREFILL16 the second
 // serves those head sizes too: that is for measurements of one against the other.
 #include "common.h"
+#include "lds_loads.h"
 #include <type_traits>
 
 #if !defined(NS_HEAD_DIM) || !defined(NS_PAGE_SIZE)

@@ -61,9 +61,6 @@ __device__ __forceinline__ float max_with_other_half(float x) {  // over lanes l
   return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
 }
 
-// Wait until at most `n` of this wave's loads are still on their way (and for nothing else).
-#define NS_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
-
 template <int SETS>
 __global__ __launch_bounds__(SETS * 256) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill32_kernel(AttnParams a) {
   if constexpr (DMA_OK) {
@@ -270,12 +267,12 @@ __global__ __launch_bounds__(SETS * 256) __attribute__((amdgpu_waves_per_eu(2)))
     // (loads land in the order they were asked for: the first scores wait for the keys of block 0 only, the first round for the
     // values of block 0 and the keys of block 1; a range of fewer than three blocks waits for all it asked for)
     if (kb1 - kb0 > 2)
-      NS_WAIT_LOADS(4 * IPW);
+      TILE_WAIT_LOADS(4 * IPW);
     else
-      NS_WAIT_LOADS(0);
+      TILE_WAIT_LOADS(0);
     __builtin_amdgcn_s_barrier();
     if (head_ok && kb0 < kb1) scores(0);
-    if (kb1 - kb0 > 2) NS_WAIT_LOADS(2 * IPW);
+    if (kb1 - kb0 > 2) TILE_WAIT_LOADS(2 * IPW);
     __builtin_amdgcn_s_barrier();  // (the scores' LDS reads are done: a matrix instruction has taken each of them)
 
     // What round `it` asks for: the keys of block it + 3 over those of block it, whose scores are formed, and the values
@@ -322,11 +319,11 @@ __global__ __launch_bounds__(SETS * 256) __attribute__((amdgpu_waves_per_eu(2)))
     // on their way), and all waves have read what this round reads.
     auto round_end = [&](int asked) {
       if (asked == 2 * IPW)
-        NS_WAIT_LOADS(2 * IPW);
+        TILE_WAIT_LOADS(2 * IPW);
       else if (asked == IPW)
-        NS_WAIT_LOADS(IPW);
+        TILE_WAIT_LOADS(IPW);
       else
-        NS_WAIT_LOADS(0);
+        TILE_WAIT_LOADS(0);
       __builtin_amdgcn_s_barrier();
     };
     // One round of the general form.  Both sets pass every barrier; the second may have no block in the last round.
@@ -515,7 +512,7 @@ __global__ __launch_bounds__(SETS * 256) __attribute__((amdgpu_waves_per_eu(2)))
       if (GUARDED) {
         round_end(asked);
       } else {
-        NS_WAIT_LOADS(2 * IPW);
+        TILE_WAIT_LOADS(2 * IPW);
         __builtin_amdgcn_s_barrier();
       }
     };

@@ -152,7 +152,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 4) void gemm_rows_f32_kernel(float
 // 16-byte LDS read serves together, then touch all 64 banks once.
 // Against the kernel before, whose loads went through registers (the same sums, bit by bit): 777 rows, N 16,384, K 2,048: 558 -> 430 us (121
 // TFLOP/s), N 2,048, K 8,192: 276 -> 231 (113), N 3,072, K 2,048: 117 -> 86; 300 rows, N 2,048, K 8,192: 125 -> 101; 16 rows 34 -> 25, 64 rows, N 2,048, K 2,048:
-// 12.4 -> 10.0.  A third of that is addresses: with a 64-bit sum a load in the vector unit the first of these takes 481 us.
+// 12.4 -> 10.0; a short K, 2,048 rows, N 2,048, K 64: 18.7 -> 16.5.  A third of that is addresses: with a 64-bit sum a load in the vector unit the first of these takes 481 us.
 // Relative error (2-norm, against 64 bits) 4.1e-7 at K 2,048, 8.1e-7 at K 8,192, half of the tiled kernel's above: four chains for one.
 // K and the row strides multiples of 4, 16-byte aligned operands.
 typedef float f32x4 __attribute__((ext_vector_type(4)));

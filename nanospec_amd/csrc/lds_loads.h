@@ -13,4 +13,4 @@
     asm volatile("" ::: "memory"); \
   } while (0)
 
-static __device__ const int4 tile_zeros = {0, 0, 0, 0};  // what stands for a piece beyond K
+[[maybe_unused]] static __device__ const int4 tile_zeros = {0, 0, 0, 0};  // what stands for a piece beyond K

@@ -568,7 +568,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
 // from memory into the operands of v_mfma_f32_16x16x32_bf16 (a wave's four loads of a matrix are 256 contiguous bytes of 16 rows), the
 // next piece on its way beside the current one's products, and the waves' sums meet in LDS in a fixed order.
 // Bound by the matrices' bytes: 8 tokens, 32 pairs over 32 experts of 1,024 in a width of 2,048, sorting included: 93 -> 58 us (4.0 TB/s
-// of the chosen experts' matrices); the tiled kernel below, 160 workgroups of 128 channels there, left the GPU half idle.
+// of the chosen experts' matrices), against a tiled kernel of 160 workgroups (``moe_tile_cap`` has the present ones).
 template <bool FIRST, bool DUAL>
 __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0,
                                                          const bf16_t* __restrict__ B1, const int* __restrict__ perm,
@@ -638,7 +638,8 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
 // taken out, where the products alone would take two thirds of the time) and by how evenly the experts' tiles deal.  32 experts of 1,024 with
 // gates, width 2,048, four a token chosen evenly, sorting included, against the kernel before (128 x 128, operands through registers, two
 // barriers a piece): 100 tokens 94 -> 80 us, 508 112 -> 90, 1,024 153 -> 136, 1,531 182 -> 142, 2,048 241 -> 200; 1,536 channels
-// without gates, 2,048 tokens 244 -> 197.
+// without gates, 2,048 tokens 244 -> 197.  Chosen as models' routers choose: 508 tokens (8 to 293 rows an expert) 117 and 116, nothing gained; 1,531 (153 to
+// 255 rows) 178 -> 137; 2,048 without gates, 1,536 channels (156 to 387 rows) 238 -> 186.
 // Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the work in use, neighbours first, so that an expert's
 // matrices and rows come into one L2 (2,048 tokens: 216 -> 200 us).  Where an expert has several tiles, all of them take four blocks of
 // channels before the next four: all blocks of one tile first bring matrices larger than an L2 from beyond it once a tile.  8 experts, two a token,
@@ -720,21 +721,26 @@ __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   }
 }
 
-// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees few rows on average, else 128 (the tiled one).
-// Streaming is ahead up to two rows an expert, and up to four where the tiled kernel has too few workgroups for the GPU, or just enough with one matrix
-// each to keep its loads going.  us streamed and tiled, sorting included, width 2,048, 32 experts, four a token, 32 tokens: 512 channels with gates 55
-// and 73, 1,024 64 and 75 without gates and 97 and 86 with them, 1,536 96 and 89, 135 and 107; 16 experts of 1,408, two a token, 70 and 88; 64 of
-// 1,024, 64 tokens, 175 and 146; 256 of 512, eight a token, 128 tokens, 318 and 267 (one expert that all tokens choose: 331 and 278).
-// (One step of 20 decoding requests with experts of 1,536, beside the other layers: 1,164 and 1,062 us.)
+// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees few rows on average, else 128 (the tiled ones):
+// up to two rows an expert, and up to four where workgroups of 128 channels were too few for the GPU.  The line was drawn with a tiled kernel that was up
+// to a third slower; as things are the tiles are ahead from some two rows on where experts have gates and are many, and the streamed
+// kernel keeps what is below and what is small.  us streamed and in the smaller tiles, sorting included, width 2,048, unevenly chosen, with gates and
+// without: 32 experts, four a token, 16 tokens (2 rows an expert): 512 channels 45 and 47, 32 and 46, 1,024 76 and 61, 49 and 59, 1,536 107 and 102, 77 and 73; 32
+// tokens (4 rows): 55 and 48, 37 and 47; 92 and 65, 63 and 63; 133 and 107, 91 and 75; 16 experts of 1,408, two a token, 32 tokens 70 and 62, 49 and 58;
+// 8 of 1,024, two a token, 16 tokens 28 and 50, 23 and 49; 64 of 1,024, four a token, 32 tokens 126 and 116, 95 and 85; 256 of 512, eight a token, 64 tokens 240 and
+// 219, 175 and 159.
 static int moe_tile_cap(long long pairs, int experts, int ff, int gated) {
   const long long groups = (long long)experts * ((ff + 127) / 128);
   const bool fills = groups >= 256 && groups * (gated ? 2 : 1) > 256;  // compute units
   return pairs <= (fills ? 2LL : 4LL) * experts ? 16 : MG_ROWS;
 }
 
-// Which tiles: up to 96 rows an expert on average most experts have one tile, a matrix is read once (past the caches) and the launch is short of
-// workgroups, so the smaller ones (a step of 508 tokens whose experts see 18 to 390 rows, beside other work: 1,454 us with these and 1,479 to
-// 1,496 with the others); beyond, the larger ones, which read less (2,048 tokens: 196 us and 206).
+// Which tiles: up to 96 rows an expert on average the smaller ones, whose loads of the matrices go past the caches (most experts have one
+// tile); beyond, the larger ones, which read less.  Neither is far ahead of the other near the line, and it moves with more than rows: us smaller
+// and larger, with gates, 32 experts of 1,024, width 2,048, four a token: 64 rows an expert chosen evenly 80 and 88, unevenly (2 to 218 rows) 120 and 124, as a
+// model's router chose (8 to 293) 117 and 122, and in its step beside other work 1,454 and 1,479 to 1,496; 128 rows 140 and 129, 142 and 132.  8 experts,
+// width 4,096, two a token, 4,096 channels: 64 rows 154 and 163, unevenly 195 and 196, 100 rows 167 and 175, 228 and 209; 14,336 channels, 64 rows 562 and 559,
+// 626 and 602.  Few small experts fill the GPU with neither: 8 of 1,024, one a token, 100 rows each 58 and 60.
 static bool moe_few_rows(long long pairs, int experts) { return pairs <= 96LL * experts; }
 
 // tiles that any choice of experts can need

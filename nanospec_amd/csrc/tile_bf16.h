@@ -18,7 +18,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 // WR x WC waves; wave (wm, wn) owns the blocks of 16 rows wm, wm + WR, .. of x (so that a tile whose last blocks are empty keeps all waves
 // equally busy) and 16 NJ neighbouring rows of w.  acc[i][j]: lane l holds for row 16 (WR i + wm) + l % 16 of x the sums with rows 16 NJ wn + 16 j +
 // 4 (l / 16) .. + 3 of w.
-// W_ONCE: the rows of w are read by few workgroups: past the caches.
+// W_ONCE: most rows of w are read by one workgroup: past the caches.
 template <int BM_, int BN_, int WR_, int WC_, int ST_, bool W_ONCE = false>
 struct TileBf16 {
   static constexpr int BM = BM_, BN = BN_, WR = WR_, WC = WC_, ST = ST_;

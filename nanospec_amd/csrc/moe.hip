@@ -578,10 +578,10 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
                                                          int act_kind) {
   constexpr int MATS = DUAL ? 2 : 1;
   __shared__ __attribute__((aligned(16))) float part[4][MATS][16][20];  // [wave][matrix][row][channel]
-  const int tile = blockIdx.y, word = tile_e[tile];
+  const int tile = blockIdx.y, word = tile_e[tile], e_row0 = tile_r0[tile], e_rows = tile_rows[tile];  // (r0 and rows in one trip to memory)
   if (word < 0) return;
   const int e = tile_expert(word), row0 = 16 * (word >> MG_E_BITS);  // (tiles of 16 rows: every one but an expert's last is full)
-  const int r0 = tile_r0[tile] + row0, rows = min(16, tile_rows[tile] - row0), n0 = blockIdx.x * 16;
+  const int r0 = e_row0 + row0, rows = min(16, e_rows - row0), n0 = blockIdx.x * 16;
   const int tid = threadIdx.x, lane = tid % NS_WAVE, wave = tid / NS_WAVE, r = lane % 16, g = lane / 16;
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const size_t wrow = ((size_t)e * N + min(n0 + r, N - 1)) * K + 8 * g;

@@ -164,7 +164,7 @@ static bool launch_rmsnorm_vec(void* out, void* resid, const void* x, const void
 // For dim a multiple of 4 and at most 4 * MAXC * threads.
 template <typename T, int MAXC>
 __global__ void rmsnorm_partial_kernel(T* __restrict__ out, T* resid, const float* __restrict__ partial, size_t plane, int ksplit,
-                                       const T* __restrict__ w, const int* __restrict__ rows, int dim, float eps, int write_resid) {
+                                       const T* __restrict__ w, const int* __restrict__ rows, int dim, float eps, int write_resid, int once) {
   typedef T vec4_t __attribute__((ext_vector_type(4)));
   __shared__ float scratch[16];
   const int i = blockIdx.x;
@@ -197,8 +197,8 @@ __global__ void rmsnorm_partial_kernel(T* __restrict__ out, T* resid, const floa
       if (rr) rv = *reinterpret_cast<const vec4_t*>(rr + idx * 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float v = round_to<T>(xs[e]);
-        if (rr) v = round_to<T>(to_f(rv[e]) + v);
+        float v = once ? xs[e] : round_to<T>(xs[e]);
+        if (rr || once) v = round_to<T>((rr ? to_f(rv[e]) : 0.f) + v);
         val[c][e] = v;
         ss += v * v;
       }
@@ -224,9 +224,10 @@ __global__ void rmsnorm_partial_kernel(T* __restrict__ out, T* resid, const floa
   }
 }
 
-// partial: float32 [ksplit][plane / dim rows][dim].
+// partial: float32 [ksplit][plane / dim rows][dim].  once: resid and the ranges are added in 32-bit and rounded once; otherwise the ranges' sum is rounded
+// as a product's result would be, and then the sum with resid.
 extern "C" int ns_rmsnorm_partial(void* out, void* resid, const void* partial, size_t plane, int ksplit, const void* w,
-                                  const int* rows, int n_rows, int dim, float eps, int write_resid, int dtype,
+                                  const int* rows, int n_rows, int dim, float eps, int write_resid, int once, int dtype,
                                   hipStream_t stream) {
   if (n_rows <= 0 || dim <= 0 || (dim & 3) || ksplit < 1 || !partial || (plane & 3) || ((uintptr_t)partial & 15) ||
       (((uintptr_t)out | (uintptr_t)resid | (uintptr_t)w) & 7))
@@ -238,11 +239,11 @@ extern "C" int ns_rmsnorm_partial(void* out, void* resid, const void* partial, s
   const int chunks = (n4 + threads - 1) / threads;
   if (chunks > 4) return NS_ERR_UNSUPPORTED;
   if (chunks <= 1)
-    rmsnorm_partial_kernel<bf16_t, 1><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid);
+    rmsnorm_partial_kernel<bf16_t, 1><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid, once);
   else if (chunks == 2)
-    rmsnorm_partial_kernel<bf16_t, 2><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid);
+    rmsnorm_partial_kernel<bf16_t, 2><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid, once);
   else
-    rmsnorm_partial_kernel<bf16_t, 4><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid);
+    rmsnorm_partial_kernel<bf16_t, 4><<<n_rows, threads, 0, stream>>>((bf16_t*)out, (bf16_t*)resid, (const float*)partial, plane, ksplit, (const bf16_t*)w, rows, dim, eps, write_resid, once);
   return ns_launch_status();
 }
 

@@ -8,6 +8,7 @@ elsewhere instead.  Tensors are torch tensors on the GPU; only their addresses c
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_float, c_int, c_size_t, c_uint32, c_void_p
 
 import torch
@@ -106,10 +107,11 @@ def logit_transform(logits: torch.Tensor, scale: float = 1.0, softcap: float = 0
 
 class PartialSums:
     """A product whose K was cut into ranges that have not been added up yet (``linear_wide(..., defer=True)``):
-    ``ws`` holds float32 [ksplit, rows, n].  ``rmsnorm`` adds them while it reads them; ``reduce_partial`` makes the tensor."""
+    ``ws`` holds float32 [ksplit, rows, n].  ``rmsnorm`` adds them while it reads them; ``reduce_partial`` makes the tensor.
+    ``once``: the reader adds them to the residual stream in 32-bit and rounds that sum alone, not the product before it."""
 
-    def __init__(self, ws: torch.Tensor, ksplit: int, rows: int, n: int, dtype: torch.dtype) -> None:
-        self.ws, self.ksplit, self.rows, self.n, self.dtype = ws, ksplit, rows, n, dtype
+    def __init__(self, ws: torch.Tensor, ksplit: int, rows: int, n: int, dtype: torch.dtype, once: bool = False) -> None:
+        self.ws, self.ksplit, self.rows, self.n, self.dtype, self.once = ws, ksplit, rows, n, dtype, once
         self.shape = (rows, n)
 
 
@@ -146,7 +148,7 @@ def rmsnorm(weight: torch.Tensor, eps: float, resid: torch.Tensor | None = None,
                 raise KernelRefused("rmsnorm: out has the wrong shape")
             _check(build.core().ns_rmsnorm_partial(_ptr(out), _ptr(resid), _ptr(p.ws), c_size_t(p.rows * dim), c_int(p.ksplit), _ptr(weight),
                                                    _ptr(rows), c_int(n), c_int(dim), c_float(eps), c_int(1 if write_resid else 0),
-                                                   c_int(_dtype_code(weight)), _stream()), "rmsnorm")
+                                                   c_int(1 if p.once else 0), c_int(_dtype_code(weight)), _stream()), "rmsnorm")
             return out
     src = resid if resid is not None else x
     if src is None:
@@ -573,6 +575,90 @@ def linear_rows(x: torch.Tensor, w: TiledWeight, w2: TiledWeight | None = None, 
                                           c_int(1 if out_f32 else 0), c_int(ksplit), c_int(nt), c_int(0), _stream()),
            "linear_rows")
     return out
+
+
+MANY_TILES = ((64, 64), (128, 64), (128, 128), (256, 128))  # rows of x by rows of w, as ``linear_many`` numbers them
+MANY_K_MULTIPLE, MANY_K_MIN, MANY_K_MAX = 128, 512, 1 << 22  # (the smallest tile takes 384, the others 256)
+MANY_MIN_ROWS = WIDE_TALL_ROWS + 1  # fewer are the streaming kernels'
+
+
+MANY_SPLIT_FORM = 2
+
+
+def many_ranges(m: int, n: int, units: int) -> int:
+    """The most ranges of K that ``many_plan`` cuts a product of m rows and n columns into (1: none)."""
+    tiles = -(-m // MANY_TILES[MANY_SPLIT_FORM][0]) * -(-n // MANY_TILES[MANY_SPLIT_FORM][1])
+    return 4 if 4 * tiles <= units else 2 if 2 * tiles <= units else 1
+
+
+@functools.lru_cache(maxsize=1 << 14)
+def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split: bool = False) -> tuple[int, int] | None:
+    """(form, ranges of K) for ``linear_many``, or None where the platform's library is the faster one (``n``: all rows of w, of gate and up
+    both).  ``may_split``: whoever reads the result can add up ranges of K.
+
+    One workgroup a compute unit takes a tile as long whatever the others do, so the smallest tile is taken whose count still fits the units
+    once, and a product is the library's from there on: it has larger tiles, which read less.  Both sides in us, alone and a call beside
+    two others, the library first, weights that no cache holds:
+    K up to 2,048: 160 rows of 2,048 11.9 / 5.6 and (64 x 64) 10.5 / 5.1; 512 13.2 / 8.1 and 11.5 / 8.3; 512 of 3,072 15.8 / 10.4 and (128 x 64) 15.8 / 10.0; 508 of 4,096 18.1 / 13.0
+    and 16.0 / 12.9; 1,024 of 4,096 25.6 / 19.3 and (128 x 128) 22.5 / 18.6; with two copies of x's and w's rows in the caches 2,048 of 4,096 34.5 / 34.2 and (256 x
+    128) 32.8 / 31.8; more than that: 1,024 of 6,144 29.5 / 25.0 and 31.4 / 25.7, 2,048 of 8,192 52.8 / 52.5 and 67.4 / 64.8.
+    A longer K shows the units that have no tile: K 4,096, 256 of 2,048 (128 tiles) 14.8 / 11.2 and 16.0 / 10.7, 1,024 of 3,072 (192) 37.1 / 29.3 and 37.7 / 25.7; K 8,192,
+    768 of 4,096 (192) 63 / 62 and 71 / 64, 1,024 of 4,096 (256) 76 / 77 and 69 / 61.
+    Rows of a tile beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 / 27.2 and 34.0 / 31.9, 512 37.8 / 35.8 and 35.8 / 34.0.
+    Gate and up in one product save a kernel besides: 160 of 16,384 30.0 / 19.5 and 23.5 / 17.8, 512 44.4 / 39.1 and 37.7 / 33.6, 1,024 (two tiles a unit) 70.7 / 64.6 and 67.9 / 65.8.
+    Ranges of K fill the units where the tiles do not, and cost the reader their sums (with the norm that reads them): 512 of 2,048, K 8,192, four 39.1 / 33.8 and
+    31.2 / 22.6; 256 of 4,096, K 14,336, four 67 / 61 and 51 / 40; 800 of 2,048, K 8,192, two 51 / 51 and 42 / 33; 512 of 2,048, K 2,048, two 16.2 / 9.0 and 17.1 / 10.2 (one 14.7 / 8.6)."""
+    if m < MANY_MIN_ROWS or n % (8 if gated else 4) or k % MANY_K_MULTIPLE or not MANY_K_MIN <= k < MANY_K_MAX:
+        return None
+    count = [-(-m // bm) * -(-n // bn) for bm, bn in MANY_TILES]
+    if may_split and k >= 4096:
+        for ranges in (4, 2):
+            if ranges <= many_ranges(m, n, units) and k % (MANY_K_MULTIPLE * ranges) == 0:
+                return MANY_SPLIT_FORM, ranges
+    for form, (bm, bn) in enumerate(MANY_TILES):
+        if count[form] <= units and not (gated and form < 2):
+            filled = count[form] / units  # the share of the units that have a tile
+            used = m * n / (count[form] * bm * bn)  # and of the tiles that is not beyond the last row or column
+            if filled < (0.0 if k <= 2048 and form < 3 else 0.625 if k <= 4096 and form == 2 else 0.75 if k <= 4096 and form < 2 else 0.85):
+                return None
+            return (form, 1) if used >= (0.6 if gated or form < 2 else 0.7 if form == 2 else 0.85) else None
+    return None
+
+
+def many_takes(x: torch.Tensor, k: int) -> bool:
+    """Whether ``linear_many`` takes rows like these: bfloat16, whole 16-byte pieces, an inner size in whole pairs of stages."""
+    return (x.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.stride(0) < MANY_K_MAX and x.data_ptr() % 16 == 0)
+
+
+def many_writes(out: torch.Tensor) -> bool:
+    """Whether ``linear_many`` can write a result there: whole pieces of four values."""
+    return out.dim() == 2 and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
+
+
+def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, w2: torch.Tensor | None = None, act: str | None = None,
+                add: bool = False, ranges: int = 1):
+    """bfloat16 x @ w.T for many rows, w in plain rows, tiles of ``MANY_TILES[form]`` (``many_plan`` chooses): into ``out``; with ``act`` that
+    activation of it; with ``w2`` silu(x @ w.T) * (x @ w2.T); with ``add`` added to ``out`` in 32-bit, rounded once.  With ``ranges`` > 1 (none of
+    these) ``out`` is float32 scratch of ranges * rows * w.shape[0] and a ``PartialSums`` over it comes back, whose reader rounds once."""
+    _gpu(x, w, w2, out)
+    m, (n, k) = x.shape[0], w.shape
+    if x.dim() != 2 or x.shape[1] != k or not many_takes(x, k) or w.dtype != x.dtype or not w.is_contiguous():
+        raise KernelRefused(f"linear_many takes bfloat16 x [rows, K] and w [N, K] with K a multiple of {MANY_K_MULTIPLE}; got {tuple(x.shape)}, {tuple(w.shape)}")
+    if w2 is not None and (w2.shape != w.shape or w2.dtype != w.dtype or not w2.is_contiguous()):
+        raise KernelRefused("linear_many: w2 must match w")
+    if (act is not None) + (w2 is not None) + bool(add) + (ranges > 1) > 1 or (act is not None and act not in ACTIVATIONS):
+        raise KernelRefused("linear_many: one thing at most follows the product")
+    if ranges > 1:
+        if out.dtype != torch.float32 or out.numel() < ranges * m * n or not out.is_contiguous():
+            raise KernelRefused("linear_many: scratch too small")
+    elif out.shape != (m, n) or out.dtype != x.dtype or out.stride(1) != 1:
+        raise KernelRefused("linear_many: out has the wrong shape or dtype")
+    epi = 4 if ranges > 1 else 3 if add else 2 if w2 is not None else 1 if act is not None else 0
+    _check(build.core().ns_gemm_many_bf16(_ptr(out), _ptr(x), _ptr(w), _ptr(w2), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
+                                          c_int(n if ranges > 1 else out.stride(0)), c_int(epi), c_int(0 if act is None else ACTIVATIONS[act]),
+                                          c_int(ranges), c_int(form), _stream()), "linear_many")
+    return PartialSums(out, ranges, m, n, x.dtype, once=True) if ranges > 1 else out
 
 
 def qkv_rope_row_order(heads: int, kv_heads: int, head_dim: int, rotary_dim: int, interleaved: bool = False) -> torch.Tensor:

@@ -65,8 +65,8 @@ class PreNormBlock:
         """``delta``: what the block before left to be added: a tensor (None at the start), a ``PartialSums``, a
         ``PreNormed``, in which case ``resid`` is already whole and the first norm's input comes ready for a product that
         ``links_norms``, or an ``Added`` (``resid`` is whole, nothing else comes with it).  ``next_norm``: the norm that will read this block's result (the next block's first one), if it
-        ``links_products``; ``next_sums`` (float32 [tokens, ceil(width / 16)]) and ``next_carry`` (float32, 16 * tokens *
-        width, or None): buffers that live as long as the step.
+        ``links_products``; ``next_sums`` (float32 [tokens, ceil(width / 16)]) and ``next_carry`` (float32, room for the
+        ranges of a product, or None): buffers that live as long as the step.
         -> None, with the block's not yet added output in ``delta_out``; or that output in one of the forms of
         ``IntoResidual`` (a tensor is then ``delta_out``)."""
         n = resid.shape[0]

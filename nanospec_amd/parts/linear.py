@@ -10,7 +10,8 @@ of a wave is one contiguous kilobyte.  17 to 64 rows run a second hand-written k
 through LDS, K cut into ranges) where it is ahead of the library, and so do products of up to 128 rows that end in the
 residual stream (at 65 to 128 rows the library takes two to three times as long for them).  More rows go to the platform's GEMM library on the
 plain layout, as the reference's nn.Linear does (model/llama.py:168-171).  32-bit results (logits) always come from the
-hand-written kernels, in slices of 64 rows, so that no logit is rounded to bfloat16.  Both layouts are kept in memory unless
+hand-written kernels, in slices of 64 rows, so that no logit is rounded to bfloat16.  Of the products of more rows those
+whose tiles come to about one a compute unit run a third hand-written kernel on the plain layout (``ops.many_plan`` says which).  Both layouts are kept in memory unless
 ``keep_plain=False``.
 """
 
@@ -32,6 +33,8 @@ GATED_WIDE_ROWS = 80  # up to here gate and up with the activation go through th
 WIDE_HEAD_ROWS = 12  # above this many rows a wide 32-bit product (the head) is faster through the 17-to-64-row kernel
 WIDE_MAX_N = 4096  # 17 to 64 rows: the hand-written kernel is ahead of the library for outputs up to this width (and for
 #                    32-bit results, which the library does not give); wider products go to the library
+SPLIT_MIN_K = 8192  # from this inner size on ranges of K are worth a kernel that adds them up, where no norm does it (512 rows of 2,048, K 8,192: 35 / 35
+#                     us in the library, alone and beside two others, 32 / 24 in four ranges with that kernel; K 4,096 20 / 15 and 21 / 16)
 LIBRARY_MAX_K = 14336  # the longest inner size over which the library's product has run here, kernel by kernel and inside
 #                        captured steps, with every replay checked.  ``library_product`` refuses a longer one: such a product is cut
 #                        into slices of its inner size in steps that are launched kernel by kernel, and runs through the
@@ -46,13 +49,36 @@ UNTILE_MIN_ROWS = 768  # where only the re-laid copy is kept: from this many row
 #                        kernel by kernel only: the scratch is as large as the matrix, and every captured step keeps its own.
 
 
-def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None = None, into: torch.Tensor | None = None) -> torch.Tensor:
-    """The one door to the platform's GEMM library: x @ w_t (``w_t`` [in, out], usually the transposed view of a matrix
-    in plain rows).  ``into``: the product is added to this tensor in place, summed in 32-bit and rounded once; a 32-bit
-    ``into`` beside bfloat16 operands keeps the sum in 32-bit.  An inner size beyond ``LIBRARY_MAX_K`` is refused: the
-    library chooses other kernels for it, none of which has run here."""
-    if x.shape[1] > LIBRARY_MAX_K:
-        raise ops.KernelRefused(f"a library product over an inner size of {x.shape[1]} (more than {LIBRARY_MAX_K}) must be cut into slices")
+def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None = None, into: torch.Tensor | None = None,
+                    plain: torch.Tensor | None = None, take=None, split: bool = False, gated: torch.Tensor | None = None):
+    """The one door to products of many rows with a matrix in plain rows: x @ w_t (``w_t`` [in, out], usually the transposed view of a
+    matrix in plain rows).  ``into``: the product is added to this tensor in place, summed in 32-bit and rounded once; a 32-bit
+    ``into`` beside bfloat16 operands keeps the sum in 32-bit.  ``gated`` (with ``plain`` and ``take``): of a product with stacked gate and up matrices
+    silu(gate) * up goes there.
+    It goes to the platform's GEMM library, or with ``plain`` (``w_t`` untransposed) to ``ops.linear_many`` where that is the faster one (``ops.many_plan``).  ``take`` (shape,
+    dtype) gives scratch for ranges of K; with ``split`` (and ``into``) the ranges may come back as a ``PartialSums``, not yet added.
+    An inner size beyond ``LIBRARY_MAX_K`` is refused: the library chooses other kernels for it, none of which has run here."""
+    m, k = x.shape
+    if k > LIBRARY_MAX_K:
+        raise ops.KernelRefused(f"a library product over an inner size of {k} (more than {LIBRARY_MAX_K}) must be cut into slices")
+    if gated is not None:
+        inter = w_t.shape[1] // 2
+        plan = ops.many_plan(m, 2 * inter, k, ops.compute_units(x.device), gated=True)
+        if plan is not None and ops.many_takes(x, k) and ops.many_writes(gated):
+            return ops.linear_many(x, plain[:inter], gated, plan[0], w2=plain[inter:])
+        return ops.silu_mul(torch.matmul(x, w_t, out=take((m, 2 * inter), x.dtype)), out=gated)
+    if plain is not None:
+        n, to = w_t.shape[1], into if into is not None else out
+        may_split = take is not None and (split if into is not None else k >= SPLIT_MIN_K)
+        plan = ops.many_plan(m, n, k, ops.compute_units(x.device), may_split=may_split)
+        if plan is not None and ops.many_takes(x, k) and (to is None or ops.many_writes(to)):
+            form, ranges = plan
+            if ranges > 1:
+                parts = ops.linear_many(x, plain, take((ranges * m * n,), torch.float32), form, ranges=ranges)
+                return parts if into is not None else ops.reduce_partial(parts, out=out)
+            if to is None:
+                to = torch.empty((m, n), dtype=x.dtype, device=x.device)
+            return ops.linear_many(x, plain, to, form, add=into is not None)
     if into is not None:
         if into.dtype == torch.float32 and x.dtype != torch.float32:
             return torch.addmm(into, x, w_t, out_dtype=torch.float32, out=into)
@@ -66,12 +92,12 @@ class IntoResidual:
       * ``kernels.ops.PreNormed``: ``resid += output`` has been done in place and the norm needs no kernel of its own
         (at most 16 rows: the product's epilogue did the sum and the norm's statistics);
       * ``kernels.ops.PartialSums``: the ranges of a product whose K was cut, which the norm kernel adds up as it reads
-        them (17 to 128 rows);
-      * ``kernels.ops.Added``: ``resid += output`` has been done in place by the product itself (more rows, through
-        the library), the norm still has its kernel;
+        them (17 to 128 rows, and more where their tiles alone leave most of the GPU idle);
+      * ``kernels.ops.Added``: ``resid += output`` has been done in place by the product itself (more rows),
+        the norm still has its kernel;
       * a tensor: the output, still to be added by the norm kernel.
     ``next_weight``, ``eps``: that norm's weight and epsilon.  ``x_next`` (like resid), ``ssq`` (float32 [rows,
-    ceil(width / 16)]) and ``carry`` (float32, 16 * rows * width): where the results go if they must outlive the block's
+    ceil(width / 16)]) and ``carry`` (float32, room for the ranges: 16 * rows * width for up to 128 rows, ``ops.many_ranges`` for more): where the results go if they must outlive the block's
     scratch (``outlives``); otherwise scratch is taken."""
 
     def __init__(self, resid: torch.Tensor, next_weight: torch.Tensor, eps: float, x_next: torch.Tensor | None = None,
@@ -143,9 +169,15 @@ class LinearWeight:
                     return ops.Added()
                 # (a captured step: the hand-written kernels below)
             else:
-                plain_t = self._plain_t if have_plain else ops.untile(self.tiled, take((self.n, self.k), self.dtype)).t()
-                library_product(x, plain_t, into=r)
-                return ops.Added()
+                if not have_plain:
+                    library_product(x, ops.untile(self.tiled, take((self.n, self.k), self.dtype)).t(), into=r)
+                    return ops.Added()
+                # (ranges of K, where the product is cut, lie where the norm still finds them)
+                room = (lambda shape, dtype: link.carry) if link.carry is not None else take
+                split = (not link.outlives if link.carry is None
+                         else link.carry.numel() >= ops.many_ranges(m, self.n, ops.compute_units(x.device)) * m * self.n)
+                done = library_product(x, self._plain_t, into=r, plain=self.plain, take=room, split=split)
+                return done if isinstance(done, ops.PartialSums) else ops.Added()
         out = link.x_next if link.x_next is not None else take((m, self.n), x.dtype)
         return self(x, out=out, arena=arena, plain_copy=plain_copy)
 
@@ -186,7 +218,8 @@ class LinearWeight:
         if self.plain is not None and (not out_f32 or self.tiled is None) and (self.k <= LIBRARY_MAX_K or self.tiled is None):
             if out_f32:
                 return ops.linear_generic(x, self.plain, out=out, out_f32=True)
-            return library_product(x, self._plain_t, out=out)
+            scratch = arena.take if arena is not None else (lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device))
+            return library_product(x, self._plain_t, out=out, plain=self.plain, take=scratch)
         if out is None:
             out = torch.empty((m, self.n), dtype=torch.float32 if out_f32 else x.dtype, device=x.device)
         if self.plain is None and m >= UNTILE_MIN_ROWS and not out_f32 and plain_copy and self.k <= PLAIN_SLICE_K:  # only the tiled layout is kept, many rows: a plain copy for this one product
@@ -281,9 +314,6 @@ class GatedWeights:
                 e = min(m, s + step)
                 ops.linear_wide(x[s:e], self.tiled[0], w2=self.tiled[1], out=out[s:e], ksplit=1, nt=1)
             return out
-        gu = ctx.arena.take((m, 2 * self.inter), x.dtype)
         if self.dtype == torch.float32 or self.k % 8:
-            ops.linear_generic(x, self.stacked, out=gu)
-        else:
-            library_product(x, self._stacked_t, out=gu)
-        return ops.silu_mul(gu, out=out)
+            return ops.silu_mul(ops.linear_generic(x, self.stacked, out=ctx.arena.take((m, 2 * self.inter), x.dtype)), out=out)
+        return library_product(x, self._stacked_t, gated=out, plain=self.stacked, take=ctx.arena.take)

@@ -217,7 +217,10 @@ class DecoderModel:
         order = self.spec.run_order
         # buffers for what one block hands to the next (see PreNormBlock.forward)
         sums = ctx.arena.take((n, -(-self.spec.hidden // 16)), torch.float32)
-        carry = ctx.arena.take((16 * n * self.spec.hidden,), torch.float32) if 16 < n <= ops.WIDE_TALL_ROWS and self.dtype == torch.bfloat16 else None
+        ranges = 0  # that a product's K may be cut into on its way into the stream
+        if self.dtype == torch.bfloat16 and n > 16:
+            ranges = 16 if n <= ops.WIDE_TALL_ROWS else ops.many_ranges(n, self.spec.hidden, ops.compute_units(resid.device))
+        carry = ctx.arena.take((ranges * n * self.spec.hidden,), torch.float32) if ranges > 1 else None
         for i, call in enumerate(order):
             layer = self.layers[call.layer]
             if getattr(layer, "links_blocks", False) and i + 1 < len(order):

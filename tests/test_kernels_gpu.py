@@ -182,6 +182,52 @@ def test_linear_wide(m, n, k):
         assert ulps_of_row_max(act.cpu(), ref * torch.sigmoid(ref) * u).max() <= 1.0
 
 
+@pytest.mark.parametrize("form", range(4))
+@pytest.mark.parametrize("m,n,k", [(1, 4, 384), (129, 68, 384), (257, 132, 512), (300, 640, 2048), (1100, 260, 640)])
+def test_linear_many(form, m, n, k):
+    """Products of many rows from plain matrices: every tile at sizes off its edges (and more tiles than an XCD's patch), the shortest
+    inner sizes, strided rows and results, everything that may follow the product, ranges of K."""
+    ops = _ops()
+    torch.manual_seed(m + n + k)
+    x = torch.randn(m + 3, k + 8, dtype=torch.bfloat16, device=DEV)[:m, :k]
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV)
+    w2 = torch.randn(n, k, dtype=torch.bfloat16, device=DEV)
+    ref, u = x.cpu().float() @ w.cpu().float().T, x.cpu().float() @ w2.cpu().float().T
+    wide = torch.full((m + 1, n + 4), 7.0, dtype=torch.bfloat16, device=DEV)  # nothing beside the result is written
+    out = wide[:m, :n]
+    assert ulps_of_row_max(ops.linear_many(x, w, out, form).cpu(), ref).max() <= 1.0
+    assert bool((wide[m] == 7).all()) and bool((wide[:, n:] == 7).all())
+    plain = out.clone()
+    for act in ops.ACTIVATIONS:
+        torch.testing.assert_close(ops.linear_many(x, w, out, form, act=act), ops.activation(plain.clone(), act), rtol=2**-7, atol=0)
+    resid = torch.randn(m, n, dtype=torch.bfloat16, device=DEV) * 30
+    out.copy_(resid)
+    assert ulps_of_row_max(ops.linear_many(x, w, out, form, add=True).cpu(), resid.cpu().float() + ref).max() <= 1.0
+    if n % 8 == 0 or form < 2:
+        assert ulps_of_row_max(ops.linear_many(x, w, out, form, w2=w2).cpu(), ref * torch.sigmoid(ref) * u).max() <= 1.5
+    weight = (1 + 0.1 * torch.randn(n, device=DEV)).bfloat16()
+    for ranges in (2, 4):
+        if k % (128 * ranges) or k // ranges < (384 if form == 0 else 256):
+            continue
+        parts = ops.linear_many(x, w, torch.empty(ranges * m * n, device=DEV), form, ranges=ranges)
+        torch.testing.assert_close(parts.ws.view(ranges, m, n).double().sum(0).cpu(), x.cpu().double() @ w.cpu().double().T, rtol=1e-5, atol=1e-5 * math.sqrt(k))
+        assert ulps_of_row_max(ops.reduce_partial(parts).cpu(), ref).max() <= 1.0
+        # the norm that reads them: the stream and the ranges are added in 32-bit and rounded once
+        r = resid.clone()
+        y = ops.rmsnorm(weight, 1e-5, resid=r, x=parts, write_resid=True)
+        assert ulps_of_row_max(r.cpu(), resid.cpu().float() + ref).max() <= 0.51
+        torch.testing.assert_close(y.cpu(), pl.rms_norm(r.cpu(), weight.cpu(), 1e-5), **_tol(torch.bfloat16))
+
+
+def test_linear_many_refuses():
+    ops = _ops()
+    x, w, out = (torch.zeros(200, k, dtype=torch.bfloat16, device=DEV) for k in (512, 512, 200))
+    for bad in (dict(x=x[:, :128], w=w[:, :128].contiguous()), dict(x=x[:, 4:260], w=w[:, :256].contiguous()), dict(out=out[:, :198], w=w[:198].contiguous()),
+                dict(ranges=3), dict(add=True, act="silu"), dict(form=7), dict(x=x.float())):
+        with pytest.raises(ops.KernelRefused):
+            ops.linear_many(**{**dict(x=x, w=w, out=out, form=2), **bad})
+
+
 @pytest.mark.parametrize("m", [17, 33, 48, 64, 5])
 @pytest.mark.parametrize("n,k", [(48, 64), (130, 200), (1000, 4096), (257, 1064), (1440, 512)])
 def test_linear_wide_dealt_to_the_compute_units(m, n, k):

@@ -51,6 +51,25 @@ def test_many_rows_in_blocks():
     assert nt == 4 and ksplit >= 2
 
 
+def test_many_rows_take_the_smallest_tile_that_fits_the_units_once():
+    plan = lambda *a, **k: ops.many_plan(*a, UNITS, **k)
+    assert plan(512, 2048, 2048) == (0, 1) and plan(512, 3072, 2048) == (1, 1) and plan(2048, 2048, 8192) == (2, 1) and plan(2048, 4096, 14336) == (3, 1)
+    assert plan(2048, 6144, 2048) is None and plan(1024, 6144, 2048) is None  # more tiles than units
+    assert plan(384, 16384, 2048) is None and plan(512, 16384, 2048) == (3, 1)  # a quarter of the tiles' rows beyond the last
+    assert plan(768, 4096, 2048) == (2, 1) and plan(768, 4096, 8192) is None   # a quarter of the units without a tile, and a long K
+    assert plan(512, 16384, 2048, gated=True) == (3, 1) and plan(160, 16384, 2048, gated=True) == (2, 1) and plan(2048, 28672, 4096, gated=True) is None
+    # ranges of K only for readers that add them up, no more of them than fill the units, each of whole pairs of stages
+    assert plan(512, 2048, 8192, may_split=True) == (2, 4) and plan(800, 2048, 8192, may_split=True) == (2, 2) and plan(512, 2048, 2048, may_split=True) == (0, 1)
+    assert plan(512, 2048, 4096 + 256, may_split=True) == (2, 2)
+    for m, n, k in ((128, 2048, 2048), (512, 2048, 2048 + 64), (512, 2050, 2048), (512, 2048, 128)):
+        assert plan(m, n, k) is None
+    for m in (129, 300, 512, 1000, 1531, 2048):
+        for n in (68, 2048, 4096, 16384):
+            form_ranges = plan(m, n, 4096, may_split=True)
+            if form_ranges is not None and form_ranges[1] > 1:
+                assert form_ranges[0] == ops.MANY_SPLIT_FORM and form_ranges[1] <= ops.many_ranges(m, n, UNITS)
+
+
 def expands(lens, kv, sizes, window=0, captured=False):
     """What ``LatentAttention._expands`` says of a step of these requests: (portions, blocks of 64 keys)."""
     from types import SimpleNamespace

@@ -1006,8 +1006,7 @@ __global__ void gelu_gather_mul_kernel(T* __restrict__ out, const T* __restrict_
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
     const size_t t = i / dim, j = i % dim;
     const float z = to_f(g[t * g_stride + j]);
-    const float gl = 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-    out[i] = from_f<T>(round_to<T>(gl) * to_f(table[(size_t)ids[t] * dim + j]));
+    out[i] = from_f<T>(round_to<T>(gelu_tanh(z)) * to_f(table[(size_t)ids[t] * dim + j]));
   }
 }
 

@@ -35,6 +35,9 @@ WIDE_MAX_N = 4096  # 17 to 64 rows: the hand-written kernel is ahead of the libr
 #                    32-bit results, which the library does not give); wider products go to the library
 SPLIT_MIN_K = 8192  # from this inner size on ranges of K are worth a kernel that adds them up, where no norm does it (512 rows of 2,048, K 8,192: 35 / 35
 #                     us in the library, alone and beside two others, 32 / 24 in four ranges with that kernel; K 4,096 20 / 15 and 21 / 16)
+ACT_FORMS = 3  # the tiles of ``ops.linear_many`` (the first of them) that apply an activation in the product's epilogue: 512 rows of 8,192, K 2,048, in tiles of 128 x 128 30.5 /
+#                22.4 us with a kernel behind it and 31.1 / 19.8 in the epilogue, alone and beside two others; the largest tile's epilogue, a workgroup a
+#                unit with nothing beside it, costs more than that kernel
 LIBRARY_MAX_K = 14336  # the longest inner size over which the library's product has run here, kernel by kernel and inside
 #                        captured steps, with every replay checked.  ``library_product`` refuses a longer one: such a product is cut
 #                        into slices of its inner size in steps that are launched kernel by kernel, and runs through the
@@ -50,11 +53,12 @@ UNTILE_MIN_ROWS = 768  # where only the re-laid copy is kept: from this many row
 
 
 def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None = None, into: torch.Tensor | None = None,
-                    plain: torch.Tensor | None = None, take=None, split: bool = False, gated: torch.Tensor | None = None):
+                    plain: torch.Tensor | None = None, take=None, split: bool = False, gated: torch.Tensor | None = None,
+                    act: str | None = None):
     """The one door to products of many rows with a matrix in plain rows: x @ w_t (``w_t`` [in, out], usually the transposed view of a
     matrix in plain rows).  ``into``: the product is added to this tensor in place, summed in 32-bit and rounded once; a 32-bit
     ``into`` beside bfloat16 operands keeps the sum in 32-bit.  ``gated`` (with ``plain`` and ``take``): of a product with stacked gate and up matrices
-    silu(gate) * up goes there.
+    silu(gate) * up goes there.  ``act``: an activation (``ops.ACTIVATIONS``) of the product (not with ``into``).
     It goes to the platform's GEMM library, or with ``plain`` (``w_t`` untransposed) to ``ops.linear_many`` where that is the faster one (``ops.many_plan``).  ``take`` (shape,
     dtype) gives scratch for ranges of K; with ``split`` (and ``into``) the ranges may come back as a ``PartialSums``, not yet added.
     An inner size beyond ``LIBRARY_MAX_K`` is refused: the library chooses other kernels for it, none of which has run here."""
@@ -73,17 +77,24 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
         plan = ops.many_plan(m, n, k, ops.compute_units(x.device), may_split=may_split)
         if plan is not None and ops.many_takes(x, k) and (to is None or ops.many_writes(to)):
             form, ranges = plan
-            if ranges > 1:
-                parts = ops.linear_many(x, plain, take((ranges * m * n,), torch.float32), form, ranges=ranges)
-                return parts if into is not None else ops.reduce_partial(parts, out=out)
             if to is None:
                 to = torch.empty((m, n), dtype=x.dtype, device=x.device)
-            return ops.linear_many(x, plain, to, form, add=into is not None)
+            if ranges > 1:
+                parts = ops.linear_many(x, plain, take((ranges * m * n,), torch.float32), form, ranges=ranges)
+                if into is not None:
+                    return parts
+                ops.reduce_partial(parts, out=to)
+            elif act is not None and form < ACT_FORMS:
+                return ops.linear_many(x, plain, to, form, act=act)
+            else:
+                ops.linear_many(x, plain, to, form, add=into is not None)
+            return to if act is None else ops.activation(to, act)
     if into is not None:
         if into.dtype == torch.float32 and x.dtype != torch.float32:
             return torch.addmm(into, x, w_t, out_dtype=torch.float32, out=into)
         return into.addmm_(x, w_t)
-    return torch.matmul(x, w_t) if out is None else torch.matmul(x, w_t, out=out)
+    y = torch.matmul(x, w_t) if out is None else torch.matmul(x, w_t, out=out)
+    return y if act is None else ops.activation(y, act)
 
 
 class IntoResidual:
@@ -186,12 +197,16 @@ class LinearWeight:
         """``arena``: where the workspace of the 17-to-64-row kernel comes from (``ctx.arena``); without it it is allocated.
         ``x`` may be a ``PreNormed`` where ``links_norms`` holds.  ``plain_copy``: where only the re-laid copy is kept, many
         rows may go to the library through a plain copy of the matrix in scratch (see ``UNTILE_MIN_ROWS``).  ``act``: an
-        activation (``ops.ACTIVATIONS``) on the result: in the streaming kernel's epilogue for few rows, a kernel of its own
-        otherwise; the values are the same either way."""
+        activation (``ops.ACTIVATIONS``) on the result: in the product's epilogue for few rows and for many where it is the
+        faster one, a kernel of its own otherwise; the values are the same either way."""
         if act is not None:
             if (not out_f32 and self.tiled is not None and not isinstance(x, ops.PreNormed) and x.shape[0] <= STREAM_ROWS
                     and x.dtype == self.dtype and ops.tiled_takes(x[:1], self.k)):
                 return ops.linear_tiled(x, self.tiled, out=out, act=act)
+            if (not out_f32 and self.plain is not None and x.dtype == self.dtype and x.shape[0] >= ops.MANY_MIN_ROWS and self.k <= LIBRARY_MAX_K
+                    and ops.many_takes(x, self.k)):
+                scratch = arena.take if arena is not None else (lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device))
+                return library_product(x, self._plain_t, out=out, plain=self.plain, take=scratch, act=act)
             return ops.activation(self(x, out=out, out_f32=out_f32, arena=arena, plain_copy=plain_copy), act)
         if isinstance(x, ops.PreNormed):
             if not self.links_norms(x.shape[0]):

@@ -12,7 +12,7 @@
 // The last outputs of a router may be identity experts, which have no matrices: what such a pair adds is its weight times the
 // input row, formed where the pairs are added up (``moe_combine``); the experts' kernels leave these pairs out.
 #include "common.h"
-#include "tile_bf16.h"
+#include "tile_quarters.h"
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 #define MOE_MAX_EXPERTS 1024
@@ -373,10 +373,11 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
   return ns_launch_status();
 }
 
+template <typename T>
 __device__ __forceinline__ float clipped_glu(float g, float u, float limit, float alpha, float shift) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.f + expf(-alpha * g)) * (u + shift);
+  return times_sigmoid<T>(g, alpha * g) * (u + shift);
 }
 
 // ------------------------------------------------------------------------------------------------ few rows
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(256) void moe_rows_up_kernel(const T* __restrict__ 
     const float g = wg ? row_dot(wg + row, moe_lds, W, lane, vec) : 0.f, u = row_dot(wu + row, moe_lds, W, lane, vec);
     if (lane == 0)
       act[((size_t)t * top + k) * ff + f] =
-          round_to<T>(wg ? clipped_glu(round_to<T>(g), round_to<T>(u), limit, alpha, shift) : activation_of(round_to<T>(u), act_kind));
+          round_to<T>(wg ? clipped_glu<T>(round_to<T>(g), round_to<T>(u), limit, alpha, shift) : activation_of<T>(round_to<T>(u), act_kind));
   }
 }
 
@@ -501,8 +502,17 @@ extern "C" int ns_moe_expert_rows(const void* h, int h_stride, const void* wg, c
 //   second: act times the down matrix; out [tokens][top][W] in 32-bit, each row back at its pair and times its weight
 
 #define MG_ROWS 128                                 // rows of a tile at most
-typedef TileBf16<MG_ROWS, 256, 2, 4, 3> MoeTile;        // by 256 rows of the matrices: one workgroup of eight waves a compute unit
-typedef TileBf16<MG_ROWS, 128, 2, 2, 2, true> MoeFewTile;  // by 128: two workgroups of four waves
+// By 256 rows of the matrices: one workgroup a compute unit; and by 128: two, with more stages on their way where half of the rows are enough (the matrices come
+// from memory then: 8 experts of 4,096, two a token, with gates, 8 tokens three stages instead of two 83 -> 77 us).
+// TURN: the stage of K that a workgroup begins with, block by block of channels (see moe_tile_kernel).
+struct MoeTile {
+  static constexpr int BN = 256, HALF_STAGES = 2, TURN = 0;
+  static constexpr bool W_ONCE = false;
+};
+struct MoeFewTile {
+  static constexpr int BN = 128, HALF_STAGES = 3, TURN = 7;
+  static constexpr bool W_ONCE = true;
+};
 #define MG_GROUP 4                                  // blocks of channels that an expert's tiles take together
 
 // What a tile is, in three words, from which a workgroup works out any tile of the same expert without another trip to memory: ``tile_e`` the expert
@@ -625,44 +635,110 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
   for (int i = 0; i < MATS; ++i) v[i] = (part[0][i][row][c] + part[1][i][row][c]) + (part[2][i][row][c] + part[3][i][row][c]);
   const int slot = r0 + row;
   if (DUAL)
-    act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu(round_to<bf16_t>(v[0]), round_to<bf16_t>(v[MATS - 1]), limit, alpha, shift));
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu<bf16_t>(round_to<bf16_t>(v[0]), round_to<bf16_t>(v[MATS - 1]), limit, alpha, shift));
   else if (FIRST)
-    act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of(round_to<bf16_t>(v[0]), act_kind));
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of<bf16_t>(round_to<bf16_t>(v[0]), act_kind));
   else
     out[(size_t)perm[slot] * N + col] = wt[perm[slot]] * v[0];
 }
 
 // Many rows an expert.  A workgroup takes a tile of the sorted rows and BN rows of the matrices (with gates BN / 2 channels of
-// both: half of a wave's 64 are of the gate and the other half the same channels of the up matrix) through LDS (tile_bf16.h).
-// Bound by the matrices' bytes up to some hundred tokens, beyond by what L2 gives the compute units (14.7 TB/s with the products
-// taken out, where the products alone would take two thirds of the time) and by how evenly the experts' tiles deal.  32 experts of 1,024 with
-// gates, width 2,048, four a token chosen evenly, sorting included, against the kernel before (128 x 128, operands through registers, two
-// barriers a piece): 100 tokens 94 -> 80 us, 508 112 -> 90, 1,024 153 -> 136, 1,531 182 -> 142, 2,048 241 -> 200; 1,536 channels
-// without gates, 2,048 tokens 244 -> 197.  Chosen as models' routers choose: 508 tokens (8 to 293 rows an expert) 117 and 116, nothing gained; 1,531 (153 to
-// 255 rows) 178 -> 137; 2,048 without gates, 1,536 channels (156 to 387 rows) 238 -> 186.
+// both, the lower half of the tile's rows of w from the gate and the upper the same channels of the up matrix) through LDS (tile_quarters.h); up to 64 rows in
+// half a tile.  Bound by the matrices' bytes up to some hundred tokens, beyond by the way from L2 to LDS and by how unevenly the experts' tiles deal.  us a call, sorting
+// included, before (tiles by eight waves a whole stage ahead, every tile whole) and now, width 2,048, four of 32 a token, chosen unevenly (as a model's router does): 1,024
+// channels with gates, 508 tokens 119 and 98, 1,531 149 and 146, 2,048 198 and 195; evenly 77 and 75, 147 and 141, 162 and 150; 1,536 without gates,
+// 2,048 tokens 196 and 200, evenly 174 and 181 (one and a half tiles a compute unit: a tile's end, with nothing beside it, counts); six of 64 of 1,408 without gates, 300 tokens 155 and
+// 138; two of 8 of 14,336 with gates, width 4,096, 2,000 tokens 1,719 and 1,653, evenly 1,502 and 1,330.
 // Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the work in use, neighbours first, so that an expert's
-// matrices and rows come into one L2 (2,048 tokens: 216 -> 200 us).  Where an expert has several tiles, all of them take four blocks of
-// channels before the next four: all blocks of one tile first bring matrices larger than an L2 from beyond it once a tile.  8 experts, two a token,
-// width 4,096, with gates, chosen unevenly, all blocks of a tile first and as it is: 14,336 channels 2,000 tokens 2,264 and 1,689 us, 512 tokens 822 and 689, 4,096
-// channels 2,000 tokens 638 and 515.  (One block at a time is level there and behind with small matrices: 8 of 2,048, width 2,048, without
-// gates, 2,000 tokens 146 and with four 140.)
-// Every expert and block of channels begins at a stage of K of its own:
-// workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (508 tokens: 111 -> 90 us).
-template <class T, bool FIRST, bool DUAL>
-__global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void moe_tile_kernel(
-    const bf16_t* __restrict__ A, int a_stride, const bf16_t* __restrict__ B0, const bf16_t* __restrict__ B1, const int* __restrict__ perm,
-    const int* __restrict__ tile_e, const int* __restrict__ tile_r0, const int* __restrict__ tile_rows, int tiles, bf16_t* __restrict__ act_out,
-    float* __restrict__ out, const float* __restrict__ wt, int N, int K, int top, float limit, float alpha, float shift, int act_kind) {
-  constexpr int CH = DUAL ? T::BN / 2 : T::BN;          // output channels of a workgroup
-  constexpr int WCH = CH / T::WC;                       // and of a wave
-  constexpr int NJ = DUAL ? T::NJ / 2 : T::NJ;          // its blocks of 16
-  __shared__ __attribute__((aligned(16))) bf16_t moe_tiles[T::ST * T::STAGE];
-  const int blocks_n = (N + CH - 1) / CH;
-  const long long used = (long long)tile_r0[tiles - 1] * blocks_n, share = (used + 7) / 8;
+// matrices and rows come into one L2.  Where an expert has several tiles, all of them take four blocks of
+// channels before the next four: all blocks of one tile first bring matrices larger than an L2 from beyond it once a tile (8 experts, two a token,
+// width 4,096, 14,336 channels with gates, 2,000 tokens, with the tiles before: 2,264 and 1,689).
+// Every expert begins at a stage of K of its own, and in the smaller tiles every block of channels too:
+// workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (begun alike: 2 to 10% slower; in the larger tiles by blocks too: 1 to 4%).
+struct MoeTileParams {
+  const bf16_t *A, *B0, *B1;
+  const int *perm, *tile_e, *tile_r0, *tile_rows;
+  bf16_t* act_out;
+  float* out;
+  const float* wt;
+  int a_stride, tiles, N, K, top, act_kind;
+  float limit, alpha, shift;
+};
+
+// ``rows`` sorted rows from ``r0`` on times expert e's rows of the matrices from channel n0 on
+template <class T, bool FIRST, bool DUAL, bool ANY>
+__device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds, int e, int r0, int rows, int n0, int turn) {
+  constexpr int HALF = T::BN / 2, NJ = DUAL ? T::NH : T::NJ;
+  T t;
+  t.init(lds, p.K, turn);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const bf16_t* w = (DUAL && h ? p.B1 : p.B0) + ((size_t)e * p.N + n0) * p.K;
+    const bf16_t* x = FIRST ? p.A : p.A + (size_t)r0 * p.a_stride;
+    t.x_from(h, x), t.w_from(h, w);
+#pragma unroll
+    for (int q = 0; q < T::LA; ++q) {
+      const int row = min(h * (T::BM / 2) + t.row_of(q), rows - 1), at = FIRST ? p.perm[r0 + row] / p.top : row;
+      if (ANY)
+        t.x_row(h, q, x + (size_t)at * p.a_stride);
+      else
+        t.xo[h][q] = 2 * (at * p.a_stride + t.piece());
+    }
+#pragma unroll
+    for (int q = 0; q < T::LB; ++q) {
+      const int row = min((DUAL ? 0 : h * HALF) + t.row_of(q), p.N - 1 - n0);
+      if (ANY)
+        t.w_row(h, q, w + (size_t)row * p.K);
+      else
+        t.wo[h][q] = 2 * (row * p.K + t.piece());
+    }
+  }
+  t.run();
+
+  const int r = t.lane % 16, g = t.lane / 16;
+#pragma unroll
+  for (int i = 0; i < T::MI; ++i) {
+    const int row = 16 * (2 * i + t.wm) + r;
+    if (row >= rows) continue;
+    const int slot = r0 + row;
+    const int pair = FIRST ? 0 : p.perm[slot];
+    const float share_of = FIRST ? 0.f : p.wt[pair];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int col = n0 + 16 * (2 * j + t.wn) + 4 * g;
+      if (col >= p.N) continue;  // (N is a multiple of 8: four columns are all inside or all outside)
+      if (FIRST) {
+        typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float z = round_to<bf16_t>(t.acc[i][j][q]);
+          o[q] = from_f<bf16_t>(DUAL ? clipped_glu<bf16_t>(z, round_to<bf16_t>(t.acc[i][T::NH + j][q]), p.limit, p.alpha, p.shift) : activation_of<bf16_t>(z, p.act_kind));
+        }
+        *reinterpret_cast<bf16x4*>(p.act_out + (size_t)slot * p.N + col) = o;
+      } else {
+        typedef float f32x4_anywhere __attribute__((ext_vector_type(4), aligned(4)));  // (``out`` is a float's address and no more)
+        f32x4_anywhere o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = share_of * t.acc[i][j][q];
+        *reinterpret_cast<f32x4_anywhere*>(p.out + (size_t)pair * p.N + col) = o;
+      }
+    }
+  }
+}
+
+template <class S, bool FIRST, bool DUAL, bool ANY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void moe_tile_kernel(const MoeTileParams p) {
+  constexpr int CH = DUAL ? S::BN / 2 : S::BN;  // output channels of a workgroup
+  typedef QuarterTile<MG_ROWS, S::BN, 2, S::W_ONCE, ANY> Whole;
+  typedef QuarterTile<MG_ROWS / 2, S::BN, S::HALF_STAGES, S::W_ONCE, ANY> Half;
+  __shared__ __attribute__((aligned(16))) bf16_t moe_tiles[Whole::VALUES > Half::VALUES ? Whole::VALUES : Half::VALUES];
+  const int blocks_n = (p.N + CH - 1) / CH;
+  const long long used = (long long)p.tile_r0[p.tiles - 1] * blocks_n, share = (used + 7) / 8;
   const long long turn = (long long)blockIdx.y * (gridDim.x >> 3) + (blockIdx.x >> 3), item = (blockIdx.x & 7) * share + turn;
   if (turn >= share || item >= used) return;
   // the expert that this item falls to and its first tile; then four blocks at a time, tile by tile
-  const int some = (int)(item / blocks_n), word = tile_e[some], c = tile_rows[some], e = tile_expert(word), of_e = (c + MG_ROWS - 1) / MG_ROWS;
+  const int some = (int)(item / blocks_n), word = p.tile_e[some], c = p.tile_rows[some], e = tile_expert(word), of_e = (c + MG_ROWS - 1) / MG_ROWS;
   const long long at = item - (long long)(some - (word >> MG_E_BITS)) * blocks_n;
   int nth = 0, block = (int)at;
   if (of_e > 1) {
@@ -671,83 +747,37 @@ __global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     nth = in_group / wide, block = MG_GROUP * group + in_group % wide;
   }
   const int row0 = rows_before_tile(c, of_e, nth), rows = rows_before_tile(c, of_e, nth + 1) - row0;
-  const int n0 = block * CH, r0 = tile_r0[some] + row0;
-
-  T t;
-  t.init(moe_tiles, K, block * 7 + e * 11);
-#pragma unroll
-  for (int p = 0; p < T::PER; ++p) {
-    const int row = t.row_of(p);
-    if (p < T::PA) {
-      const int slot = r0 + min(row, rows - 1);
-      t.src[p] = A + (size_t)(FIRST ? perm[slot] / top : slot) * a_stride + t.piece();
-    } else {
-      const int in = row % (16 * T::NJ), col = DUAL ? n0 + row / (16 * T::NJ) * WCH + in % WCH : n0 + row;
-      t.src[p] = (DUAL && in >= WCH ? B1 : B0) + ((size_t)e * N + min(col, N - 1)) * K + t.piece();
-    }
-  }
-  t.start();
-  t.run(((rows + 15) / 16 - t.wm + T::WR - 1) / T::WR);
-
-  const int r = t.lane % 16, g = t.lane / 16;
-#pragma unroll
-  for (int i = 0; i < T::MI; ++i) {
-    const int row = 16 * (T::WR * i + t.wm) + r;
-    if (row >= rows) continue;
-    const int slot = r0 + row;
-    const int pair = FIRST ? 0 : perm[slot];
-    const float share_of = FIRST ? 0.f : wt[pair];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int col = n0 + t.wn * WCH + 16 * j + 4 * g;
-      if (col >= N) continue;  // (N is a multiple of 8: four columns are all inside or all outside)
-      if (FIRST) {
-        typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
-        bf16x4 o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float z = round_to<bf16_t>(t.acc[i][j][q]);
-          o[q] = from_f<bf16_t>(DUAL ? clipped_glu(z, round_to<bf16_t>(t.acc[i][T::NJ / 2 + j][q]), limit, alpha, shift) : activation_of(z, act_kind));
-        }
-        *reinterpret_cast<bf16x4*>(act_out + (size_t)slot * N + col) = o;
-      } else {
-        typedef float f32x4_anywhere __attribute__((ext_vector_type(4), aligned(4)));  // (``out`` is a float's address and no more)
-        f32x4_anywhere o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = share_of * t.acc[i][j][q];
-        *reinterpret_cast<f32x4_anywhere*>(out + (size_t)pair * N + col) = o;
-      }
-    }
-  }
+  const int n0 = block * CH, r0 = p.tile_r0[some] + row0;
+  if (rows <= MG_ROWS / 2)
+    moe_one_tile<Half, FIRST, DUAL, ANY>(p, moe_tiles, e, r0, rows, n0, block * S::TURN + e * 11);
+  else
+    moe_one_tile<Whole, FIRST, DUAL, ANY>(p, moe_tiles, e, r0, rows, n0, block * S::TURN + e * 11);
 }
 
-// Rows that a tile holds at most: 16 (the kernel that streams matrices) while an expert sees few rows on average, else 128 (the tiled ones):
-// up to two rows an expert, and up to four where workgroups of 128 channels were too few for the GPU.  The line was drawn with a tiled kernel that was up
-// to a third slower; as things are the tiles are ahead from some two rows on where experts have gates and are many, and the streamed
-// kernel keeps what is below and what is small.  us streamed and in the smaller tiles, sorting included, width 2,048, unevenly chosen, with gates and
-// without: 32 experts, four a token, 16 tokens (2 rows an expert): 512 channels 45 and 47, 32 and 46, 1,024 76 and 61, 49 and 59, 1,536 107 and 102, 77 and 73; 32
-// tokens (4 rows): 55 and 48, 37 and 47; 92 and 65, 63 and 63; 133 and 107, 91 and 75; 16 experts of 1,408, two a token, 32 tokens 70 and 62, 49 and 58;
-// 8 of 1,024, two a token, 16 tokens 28 and 50, 23 and 49; 64 of 1,024, four a token, 32 tokens 126 and 116, 95 and 85; 256 of 512, eight a token, 64 tokens 240 and
-// 219, 175 and 159.
-static int moe_tile_cap(long long pairs, int experts, int ff, int gated) {
-  const long long groups = (long long)experts * ((ff + 127) / 128);
-  const bool fills = groups >= 256 && groups * (gated ? 2 : 1) > 256;  // compute units
-  return pairs <= (fills ? 2LL : 4LL) * experts ? 16 : MG_ROWS;
+// Rows that a tile holds at most: 16 (the kernel that streams matrices) for the smallest steps, else 128 (the tiled ones).  The tiled kernels take some 28 us
+// however little there is to do (two kernels, each the chain of a tile's stages), the streamed one as long as the chosen experts' matrices take at some 4 TB/s,
+// and longer where an expert has more than 16 rows.  So tiles from 2^27 bytes of matrices on, if there are workgroups enough for them (experts
+// times blocks of 128 of the width) or the rows are several an expert, and from four rows an expert on in any case.  us streamed and in tiles, sorting included,
+// width 2,048, unevenly chosen, with gates and without: 32 experts of 1,024, four a token, 2 tokens 30 and 29, 22 and 30; 4 44 and 36, 33 and 34; 8 66 and 61, 42 and 40; 16
+// 81 and 65, 62 and 48; 16 of 1,408, two a token, 2 27 and 33, 21 and 30; 4 37 and 35, 28 and 35; 8 55 and 51, 36 and 36; 8 of 4,096, two a token, 2 43 and 48, 39 and 47; 4 60 and
+// 67, 50 and 53; 8 88 and 77, 60 and 55; 16 83 and 78, 70 and 58; 8 of 1,024, one a token, 32 tokens 31 and 32, 25 and 30, 64 36 and 31, 33 and 30; 256 of 512, eight a
+// token, 2 36 and 30, 29 and 29; 32 218 and 187, 145 and 125.
+static int moe_tile_cap(long long pairs, int experts, int W, int ff, int gated) {
+  const long long chosen = pairs < experts ? pairs : experts, bytes = chosen * ff * W * (gated ? 6 : 4);
+  const bool enough = chosen * ((W + 127) / 128) >= 192 || pairs >= 2LL * experts;
+  return pairs > 4LL * experts || (bytes >= 1LL << 27 && enough) ? MG_ROWS : 16;
 }
+static int moe_tiles(long long pairs, int experts, int cap) { return (int)((pairs + cap - 1) / cap) + experts; }
 
 // Which tiles: up to 96 rows an expert on average the smaller ones, whose loads of the matrices go past the caches (most experts have one
 // tile); beyond, the larger ones, which read less.  Neither is far ahead of the other near the line, and it moves with more than rows: us smaller
-// and larger, with gates, 32 experts of 1,024, width 2,048, four a token: 64 rows an expert chosen evenly 80 and 88, unevenly (2 to 218 rows) 120 and 124, as a
-// model's router chose (8 to 293) 117 and 122, and in its step beside other work 1,454 and 1,479 to 1,496; 128 rows 140 and 129, 142 and 132.  8 experts,
-// width 4,096, two a token, 4,096 channels: 64 rows 154 and 163, unevenly 195 and 196, 100 rows 167 and 175, 228 and 209; 14,336 channels, 64 rows 562 and 559,
-// 626 and 602.  Few small experts fill the GPU with neither: 8 of 1,024, one a token, 100 rows each 58 and 60.
+// and larger, evenly and unevenly chosen: with gates, 32 experts of 1,024, width 2,048, four a token: 64 rows an expert 79 and 91, 102 and 121, 128 rows 98 and 105, 142 and
+// 135, 192 rows 153 and 140, 158 and 144; 1,536 channels without gates 128 rows 112 and 121, 157 and 165, 256 rows 174 and 181, 217 and 199; 8 experts, width 4,096, two a
+// token: 4,096 channels 96 rows 153 and 182, 162 and 181, 128 rows 164 and 185, 243 and 222; 14,336 channels 64 rows 479 and 584, 501 and 600 (most unevenly 654 and 617).
 static bool moe_few_rows(long long pairs, int experts) { return pairs <= 96LL * experts; }
 
-// tiles that any choice of experts can need
-extern "C" int ns_moe_group_tiles(int pairs, int experts, int ff, int gated) {
-  const int cap = moe_tile_cap(pairs, experts, ff, gated);
-  return (pairs + cap - 1) / cap + experts;
-}
+// tiles that any choice of experts can need, whichever kernel takes them
+extern "C" int ns_moe_group_tiles(int pairs, int experts) { return moe_tiles(pairs, experts, 16); }
 
 // The launch for so many items of a tile and a block of channels: the XCDs' eight workgroups of a turn side by side, and the turns in two dimensions,
 // because one holds fewer than 2^32 threads.
@@ -770,14 +800,25 @@ struct MoeLaunch {
   int h_stride, W, ff, top, tiles, act_kind;
   float limit, alpha, shift;
   bool few_rows;
+  long long rows;  // of h
   hipStream_t stream;
 
-  template <class T, bool FIRST, bool DUAL>
+  template <class S, bool FIRST, bool DUAL, bool ANY>
+  void launch(const MoeTileParams& p) const {
+    constexpr int CH = DUAL ? S::BN / 2 : S::BN;
+    moe_tile_kernel<S, FIRST, DUAL, ANY><<<moe_tile_grid((long long)tiles * ((p.N + CH - 1) / CH)), 256, 0, stream>>>(p);
+  }
+  template <bool FIRST, bool DUAL>
   void tiled(const bf16_t* a, int a_stride, const bf16_t* b0, const bf16_t* b1, int n, int k) const {
-    constexpr int CH = DUAL ? T::BN / 2 : T::BN;
-    const dim3 grid = moe_tile_grid((long long)tiles * ((n + CH - 1) / CH));
-    moe_tile_kernel<T, FIRST, DUAL><<<grid, T::THREADS, 0, stream>>>(a, a_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, tiles, act, out, wt, n, k, top,
-                                                                     limit, alpha, shift, act_kind);
+    const MoeTileParams p{a, b0, b1, perm, tile_e, tile_r0, tile_rows, act, out, wt, a_stride, tiles, n, k, top, act_kind, limit, alpha, shift};
+    // whole pairs of stages, and all rows within 31 bits of bytes of their first; other sizes are no model's
+    const bool plain = k % QUARTER_K_MULTIPLE == 0 && k >= 4 * QUARTER_K && k < 1 << 22 && a_stride < 1 << 22 && (!FIRST || rows * a_stride < 1LL << 30);
+    if (!plain)
+      launch<MoeFewTile, FIRST, DUAL, true>(p);
+    else if (few_rows)
+      launch<MoeFewTile, FIRST, DUAL, false>(p);
+    else
+      launch<MoeTile, FIRST, DUAL, false>(p);
   }
   template <bool DUAL>
   void first(int cap) const {
@@ -785,19 +826,15 @@ struct MoeLaunch {
     if (cap == 16)
       moe_stream_kernel<true, DUAL><<<dim3((ff + 15) / 16, tiles), 256, 0, stream>>>(h, h_stride, b0, b1, perm, tile_e, tile_r0, tile_rows, act, nullptr,
                                                                                     nullptr, ff, W, top, limit, alpha, shift, act_kind);
-    else if (few_rows)
-      tiled<MoeFewTile, true, DUAL>(h, h_stride, b0, b1, ff, W);
     else
-      tiled<MoeTile, true, DUAL>(h, h_stride, b0, b1, ff, W);
+      tiled<true, DUAL>(h, h_stride, b0, b1, ff, W);
   }
   void second(int cap) const {
     if (cap == 16)
       moe_stream_kernel<false, false><<<dim3((W + 15) / 16, tiles), 256, 0, stream>>>(act, ff, wd, nullptr, perm, tile_e, tile_r0, tile_rows, nullptr, out, wt,
                                                                                      W, ff, top, limit, alpha, shift, act_kind);
-    else if (few_rows)
-      tiled<MoeFewTile, false, false>(act, ff, wd, nullptr, W, ff);
     else
-      tiled<MoeTile, false, false>(act, ff, wd, nullptr, W, ff);
+      tiled<false, false>(act, ff, wd, nullptr, W, ff);
   }
 };
 
@@ -811,16 +848,15 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
     return NS_ERR_UNSUPPORTED;
   const long long pairs = (long long)n * top;
   if (pairs > (1 << 24)) return NS_ERR_UNSUPPORTED;
-  const int tiles = ns_moe_group_tiles((int)pairs, experts, ff, wg != nullptr);
+  const int cap = moe_tile_cap(pairs, experts, W, ff, wg != nullptr), tiles = moe_tiles(pairs, experts, cap);
   int* perm = ints;
   int* tile_e = ints + pairs;
   int* tile_r0 = tile_e + tiles;
   int* tile_rows = tile_r0 + tiles;
-  const int cap = moe_tile_cap(pairs, experts, ff, wg != nullptr);
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
   moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
   const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,
-                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, moe_few_rows(pairs, experts), stream};
+                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, moe_few_rows(pairs, experts), n, stream};
   if (wg)
     l.first<true>(cap);
   else
@@ -834,12 +870,38 @@ template <typename T>
 __global__ void clipped_glu_kernel(T* __restrict__ out, const T* __restrict__ gu, int gu_stride, int ff, size_t count, float limit, float alpha, float shift) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
     const size_t t = i / ff, f = i % ff;
-    out[i] = from_f<T>(clipped_glu(to_f(gu[t * gu_stride + f]), to_f(gu[t * gu_stride + ff + f]), limit, alpha, shift));
+    out[i] = from_f<T>(clipped_glu<T>(to_f(gu[t * gu_stride + f]), to_f(gu[t * gu_stride + ff + f]), limit, alpha, shift));
+  }
+}
+
+// The same in pieces of 16 bytes, a workgroup 256 of them of a row (nothing is divided).  Bound by the bytes: 2,048 rows of 4,096, bfloat16, 19.4 -> 9.8 us.
+template <typename T>
+__global__ __launch_bounds__(256) void clipped_glu_vec_kernel(T* __restrict__ out, const T* __restrict__ gu, int gu_stride, int n, int ff, float limit, float alpha,
+                                                             float shift) {
+  constexpr int V = 16 / sizeof(T);
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+  const int f = (blockIdx.x * 256 + threadIdx.x) * V;
+  if (f >= ff) return;
+  for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) {
+    const vec_t g = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + f), u = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + ff + f);
+    vec_t o;
+#pragma unroll
+    for (int i = 0; i < V; ++i) o[i] = from_f<T>(clipped_glu<T>(to_f((T)g[i]), to_f((T)u[i]), limit, alpha, shift));
+    *reinterpret_cast<vec_t*>(out + t * ff + f) = o;
   }
 }
 
 extern "C" int ns_clipped_glu(void* out, const void* gu, int gu_stride, int n, int ff, float limit, float alpha, float shift, int dtype, hipStream_t stream) {
   if (n <= 0 || ff <= 0) return NS_ERR_BAD_ARG;
+  const int v = dtype == NS_DTYPE_F32 ? 4 : 8;
+  if ((dtype == NS_DTYPE_F32 || dtype == NS_DTYPE_BF16) && ff % v == 0 && gu_stride % v == 0 && !(((uintptr_t)out | (uintptr_t)gu) & 15)) {
+    const dim3 grid((ff / v + 255) / 256, n < 65535 ? n : 65535);
+    if (dtype == NS_DTYPE_F32)
+      clipped_glu_vec_kernel<float><<<grid, 256, 0, stream>>>((float*)out, (const float*)gu, gu_stride, n, ff, limit, alpha, shift);
+    else
+      clipped_glu_vec_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)gu, gu_stride, n, ff, limit, alpha, shift);
+    return ns_launch_status();
+  }
   const size_t count = (size_t)n * ff;
   size_t blocks = (count + 255) / 256;
   if (blocks > 65535) blocks = 65535;

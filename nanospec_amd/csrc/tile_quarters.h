@@ -26,7 +26,8 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 // Wave (wm, wn) of 2 x 2 owns the blocks of 16 rows wm, wm + 2, .. of x and wn, wn + 2, .. of w.  acc[i][j]: lane l holds for row 16 (2 i + wm) + l % 16 of x
 // the sums with rows 16 (2 j + wn) + 4 (l / 16) .. + 3 of w.
 // W_ONCE: most rows of w are read by one workgroup: past the caches.
-template <int BM_, int BN_, int ST_ = 2, bool W_ONCE = false>
+// ANY: any K that is a multiple of 8 (stages beyond it are zeros), and rows anywhere: an address of 64 bits and a choice for every load.
+template <int BM_, int BN_, int ST_ = 2, bool W_ONCE = false, bool ANY = false>
 struct QuarterTile {
   static constexpr int BM = BM_, BN = BN_, ST = ST_, WAVES = 4;
   static constexpr int MI = BM / 32, NJ = BN / 32, MH = MI / 2, NH = NJ / 2;
@@ -41,8 +42,10 @@ struct QuarterTile {
   typedef float f32x4 __attribute__((__vector_size__(4 * sizeof(float))));
   bf16_t* lds;
   int lane, wave, wm, wn, stages, at;  // at: the stage of K that is loaded next
+  int K;
   int xo[2][LA], wo[2][LB];            // bytes from the halves' first rows to this lane's piece of each row it fetches, at k = 0
   __amdgpu_buffer_rsrc_t xr[2], wr[2];
+  const bf16_t *xp[2][LA], *wp[2][LB];  // (ANY: the same as addresses)
   f32x4 acc[MI][NJ];
 
   // the row of its half that load q of this lane fetches
@@ -51,8 +54,8 @@ struct QuarterTile {
   __device__ __forceinline__ int piece() const { return 8 * ((lane % 8) ^ (lane / 8)); }
 
   // ``turn``: the stage of K to begin with (any number; the sums run over K from there and round)
-  __device__ __forceinline__ void init(bf16_t* lds_, int K, int turn = 0) {
-    lds = lds_, stages = K / QUARTER_K, at = turn % stages;
+  __device__ __forceinline__ void init(bf16_t* lds_, int K_, int turn = 0) {
+    lds = lds_, K = K_, stages = ANY ? max(BEHIND, (K + 2 * QUARTER_K - 1) / (2 * QUARTER_K) * 2) : K / QUARTER_K, at = turn % stages;
     lane = threadIdx.x % NS_WAVE;
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NS_WAVE % WAVES);
     wm = wave / 2, wn = wave % 2;
@@ -64,6 +67,10 @@ struct QuarterTile {
   // where the low (0) or high (1) half's offsets count from
   __device__ __forceinline__ void x_from(int half, const bf16_t* p) { xr[half] = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0xffffffff, 0x00020000); }
   __device__ __forceinline__ void w_from(int half, const bf16_t* p) { wr[half] = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0xffffffff, 0x00020000); }
+
+  // ANY: this lane's piece of the row that its load q fetches
+  __device__ __forceinline__ void x_row(int half, int q, const bf16_t* p) { xp[half][q] = p + piece(); }
+  __device__ __forceinline__ void w_row(int half, int q, const bf16_t* p) { wp[half][q] = p + piece(); }
 
   static constexpr bool of_x(int u) { return u == X_LOW || u == X_HIGH; }
   static constexpr int place(int u) { return u == X_LOW ? 0 : u == W_LOW ? UA : u == W_HIGH ? UA + UB : UA + 2 * UB; }
@@ -81,7 +88,11 @@ struct QuarterTile {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     const lds_ptr to = (lds_ptr)(lds + slot + place(U) + (q * WAVES + wave) * 8 * QUARTER_K);
     constexpr int half = U == X_HIGH || U == W_HIGH;
-    if constexpr (of_x(U))
+    if constexpr (ANY) {
+      const bf16_t* from = (of_x(U) ? xp[half][q] : wp[half][q]) + k * QUARTER_K;
+      if (k * QUARTER_K + piece() >= K) from = reinterpret_cast<const bf16_t*>(&tile_zeros);
+      __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+    } else if constexpr (of_x(U))
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr[half], to, 16, xo[half][q], k * (QUARTER_K * 2), 0, 0);
     else if constexpr (W_ONCE)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr[half], to, 16, wo[half][q], k * (QUARTER_K * 2), 0, 2);  // (non-temporal)

@@ -1684,7 +1684,7 @@ def moe_expert_groups(h: torch.Tensor, gate: torch.Tensor | None, up: torch.Tens
     experts, ff = up.shape[0], up.shape[1]
     top = sel.shape[1]
     kind = _expert_form(gate, up, activation, "moe_expert_groups")
-    tiles = int(build.core().ns_moe_group_tiles(c_int(n * top), c_int(experts), c_int(ff), c_int(gate is not None)))
+    tiles = int(build.core().ns_moe_group_tiles(c_int(n * top), c_int(experts)))
     if (not moe_groups_take(h, ff) or h.stride(1) != 1 or up.shape != (experts, ff, W) or down.shape != (experts, W, ff)
             or sel.shape != (n, top) or weights.shape != (n, top) or out.shape != (n, top, W) or act.shape != (n * top, ff) or act.dtype != h.dtype
             or not act.is_contiguous() or ints.numel() < n * top + 3 * tiles or any(t.dtype != h.dtype or not t.is_contiguous() for t in (gate, up, down) if t is not None)):
@@ -1705,7 +1705,7 @@ def moe_experts(h: torch.Tensor, gate: torch.Tensor | None, up: torch.Tensor, do
     top = sel.shape[1]
     out = take((n, top, W), torch.float32)
     if n * top >= max(experts, 16) and moe_groups_take(h, ff):
-        tiles = int(build.core().ns_moe_group_tiles(c_int(n * top), c_int(experts), c_int(ff), c_int(gate is not None)))
+        tiles = int(build.core().ns_moe_group_tiles(c_int(n * top), c_int(experts)))
         return moe_expert_groups(h, gate, up, down, sel, weights, limit, alpha, take((n * top + 3 * tiles,), torch.int32),
                                  take((n * top, ff), h.dtype), out, shift=shift, activation=activation)
     return moe_expert_rows(h, gate, up, down, sel, weights, limit, alpha, take((n, top, ff), torch.float32), out, shift=shift,

@@ -273,13 +273,20 @@ __global__ __launch_bounds__(64) void moe_choose_kernel(const float* __restrict_
 // bit.  Logits and choice, width 2,048, four chosen of 32: 8 tokens in groups 14.1 -> 11.8 us, 2,048 tokens 18.8 -> 16.5; of 36 in groups, 508 tokens 20.7 -> 19.3.
 __device__ __forceinline__ float lane_read(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
 
-__global__ __launch_bounds__(256) void moe_choose_lanes_kernel(const float* __restrict__ z, int z_stride, int* __restrict__ sel, float* __restrict__ wt,
-                                                               int n, int experts, int top, int score, const float* __restrict__ correction, int groups,
-                                                               int keep, int group_best, float scale) {
-  const int t = blockIdx.x * 4 + threadIdx.x / NS_WAVE, lane = threadIdx.x % NS_WAVE;
-  if (t >= n) return;
+struct MoeChoice {
+  int experts, top, score;
+  const float* correction;
+  int groups, keep, group_best;
+  float scale;
+};
+
+// a wave's choice for token t, whose logits its lanes hold (``w``)
+__device__ __forceinline__ void moe_choose_lanes(float w, size_t t, int* __restrict__ sel, float* __restrict__ wt, const MoeChoice& p) {
+  const int lane = threadIdx.x % NS_WAVE, experts = p.experts, top = p.top, score = p.score, groups = p.groups, keep = p.keep, group_best = p.group_best;
+  const float* __restrict__ correction = p.correction;
+  const float scale = p.scale;
   const bool mine = lane < experts;
-  float w = mine ? z[(size_t)t * z_stride + lane] : -INFINITY;  // what the weights are made from: the logits, or the scores
+  w = mine ? w : -INFINITY;  // what the weights are made from: the logits, or the scores
   if (score == MOE_SOFTMAX) {
     const float zmax = wave_max(fmaxf(-INFINITY, w));
     const float e = expf(w - zmax);
@@ -324,6 +331,61 @@ __global__ __launch_bounds__(256) void moe_choose_lanes_kernel(const float* __re
   }
 }
 
+__global__ __launch_bounds__(256) void moe_choose_lanes_kernel(const float* __restrict__ z, int z_stride, int* __restrict__ sel, float* __restrict__ wt,
+                                                               int n, const MoeChoice p) {
+  const int t = blockIdx.x * 4 + threadIdx.x / NS_WAVE, lane = threadIdx.x % NS_WAVE;
+  if (t >= n) return;
+  moe_choose_lanes(lane < p.experts ? z[(size_t)t * z_stride + lane] : 0.f, t, sel, wt, p);
+}
+
+// Logits and choice of a step of few tokens in one launch: a workgroup a token, its four teams of four waves every fourth row of the router, four rows at a time; the
+// first wave chooses by lanes.  Every workgroup reads the whole router (from L2 but for the first), so it has to be small; what is saved is a launch and a trip of the
+// logits through memory in a chain of dependent kernels.  A logit's sum is ordered as in moe_logits_few_kernel, whose results these are bit by bit.
+// us in two launches and in one: 8 tokens, width 2,048, four of 32 8.5 and 7.0, in 8 groups of which 4 are kept 11.2 and 9.7; 2 tokens, 4,096, two of 16 6.9 and 5.7; a larger router
+// is more than a compute unit reads in that time: 8 of 4,096, 32 experts 10.4 and 10.5; 36 of 2,048 11.1 and 11.5 (a third round); 64 of 2,048 10.1 and 12.8.
+#define MOE_ROUTE_FEW_ROWS 32
+#define MOE_ROUTE_FEW_BYTES (256 << 10)
+template <typename T>
+__global__ __launch_bounds__(1024) void moe_route_few_kernel(const T* __restrict__ h, int h_stride, const float* __restrict__ wr, const float* __restrict__ br,
+                                                             float* __restrict__ z, int* __restrict__ sel, float* __restrict__ wt, int W, int rows,
+                                                             const MoeChoice p) {
+  constexpr int TEAMS = 4, AT_ONCE = 4;
+  __shared__ float part[4][MOE_ROUTE_FEW_ROWS], zs[MOE_ROUTE_FEW_ROWS];
+  const size_t t = blockIdx.x;
+  const int team = threadIdx.x / 256, tid = threadIdx.x % 256, lane = threadIdx.x % NS_WAVE, wave = tid / NS_WAVE;
+  const T* x = h + t * h_stride;
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  for (int e0 = team; e0 < rows; e0 += TEAMS * AT_ONCE) {
+    float acc[AT_ONCE];
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k) acc[k] = 0.f;
+    for (int c = tid * 4; c < W; c += 256 * 4) {
+      const t4 xc = *reinterpret_cast<const t4*>(x + c);
+      float4 wc[AT_ONCE];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) wc[k] = *reinterpret_cast<const float4*>(wr + (size_t)min(e0 + TEAMS * k, rows - 1) * W + c);
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        acc[k] = fmaf(to_f((T)xc[0]), wc[k].x, acc[k]), acc[k] = fmaf(to_f((T)xc[1]), wc[k].y, acc[k]);
+        acc[k] = fmaf(to_f((T)xc[2]), wc[k].z, acc[k]), acc[k] = fmaf(to_f((T)xc[3]), wc[k].w, acc[k]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k) {
+      const float v = wave_sum(acc[k]);
+      if (lane == 0 && e0 + TEAMS * k < rows) part[wave][e0 + TEAMS * k] = v;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < rows) {
+    const int e = threadIdx.x;
+    const float v = ((part[0][e] + part[1][e]) + (part[2][e] + part[3][e])) + (br ? br[e] : 0.f);
+    zs[e] = v, z[t * rows + e] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < NS_WAVE) moe_choose_lanes(lane < rows ? zs[lane] : 0.f, t, sel, wt, p);
+}
+
 // Which of the two (the results are the same), by what each takes, in steps of a walk over the experts (35 ns a token's chain, 110 ns of 8,192 tokens):
 // by lanes one walk, three where experts are chosen in groups; by turns 20 an expert to choose, 10 a group to keep and 2.5 an expert of a
 // group; with the GPU full of tokens 27 and 18, and the turns' workgroups of one wave cost 28 to 32 more.  us by turns and by lanes, with the
@@ -351,6 +413,15 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
   const size_t elem = dtype == NS_DTYPE_F32 ? 4 : 2;
   const int vec = W % 4 == 0 && h_stride % 4 == 0 && (uintptr_t)wr % 16 == 0 && (uintptr_t)h % (4 * elem) == 0;
   if (dtype != NS_DTYPE_F32 && dtype != NS_DTYPE_BF16) return NS_ERR_UNSUPPORTED;
+  const bool by_lanes = moe_choose_by_lanes(n, experts, top, groups, keep);
+  const MoeChoice choice{experts, top, score, correction, groups, keep, group_best, scale};
+  if (n <= ROUTE_TOK && vec && by_lanes && rows <= MOE_ROUTE_FEW_ROWS && (size_t)rows * W * sizeof(float) <= MOE_ROUTE_FEW_BYTES) {
+    if (dtype == NS_DTYPE_F32)
+      moe_route_few_kernel<float><<<n, 1024, 0, stream>>>((const float*)h, h_stride, wr, br, z, sel, wt, W, rows, choice);
+    else
+      moe_route_few_kernel<bf16_t><<<n, 1024, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, sel, wt, W, rows, choice);
+    return ns_launch_status();
+  }
   if (n <= ROUTE_TOK) {  // few tokens: a workgroup an expert
     if (dtype == NS_DTYPE_F32)
       moe_logits_few_kernel<float><<<rows, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
@@ -366,8 +437,8 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
     moe_logits_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
   else
     moe_logits_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows, vec);
-  if (moe_choose_by_lanes(n, experts, top, groups, keep))
-    moe_choose_lanes_kernel<<<(n + 3) / 4, 256, 0, stream>>>(z, rows, sel, wt, n, experts, top, score, correction, groups, keep, group_best, scale);
+  if (by_lanes)
+    moe_choose_lanes_kernel<<<(n + 3) / 4, 256, 0, stream>>>(z, rows, sel, wt, n, choice);
   else
     moe_choose_kernel<<<n, 64, 0, stream>>>(z, rows, sel, wt, n, experts, top, score, correction, groups, keep, group_best, scale);
   return ns_launch_status();

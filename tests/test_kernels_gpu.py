@@ -1731,3 +1731,69 @@ def _turned(x, pos, inv, interleaved):
     a, b = (x[:, 0::2], x[:, 1::2]) if interleaved else (x[:, :half], x[:, half:])
     u, v = a * c - b * s, b * c + a * s
     return torch.stack([u, v], -1).flatten(-2) if interleaved else torch.cat([u, v], -1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("experts,extra,top,groups,keep,width", [(32, 0, 4, 1, 1, 2048), (32, 0, 4, 8, 4, 2048), (31, 1, 3, 1, 1, 260), (8, 0, 8, 2, 2, 8192), (5, 0, 1, 1, 1, 4), (28, 4, 4, 4, 2, 1032)])
+def test_moe_route_of_few_tokens_in_one_launch(dtype, experts, extra, top, groups, keep, width):
+    """A small router's logits and choice for up to 8 tokens are one kernel, a workgroup a token: the same bits as in two launches
+    (which a row at an odd stride still takes), however many tokens the step holds."""
+    ops = _ops()
+    torch.manual_seed(experts + width)
+    h = torch.randn(8, width, device=DEV).to(dtype)
+    odd = torch.empty(8, width + 1, dtype=dtype, device=DEV)[:, :width].copy_(h)
+    router = torch.randn(experts + extra, width, device=DEV) * 0.1
+    bias = torch.randn(experts + extra, device=DEV) if not extra else None
+
+    def route(x, n):
+        sel, wt = torch.full((n, top), -1, dtype=torch.int32, device=DEV), torch.zeros(n, top, device=DEV)
+        z = torch.zeros(n, experts + extra, device=DEV)
+        ops.moe_route(x[:n], router, bias, top, sel, wt, logits=z, groups=groups, keep=keep, extra=extra)
+        return sel, wt, z
+
+    got = route(h, 8)
+    want = h.double() @ router.double().T + (0 if bias is None else bias.double())
+    torch.testing.assert_close(got[2].double(), want, rtol=1e-5, atol=1e-5 * math.sqrt(width))
+    for n in (1, 3, 8):
+        for a, b in zip(route(h, n), got):
+            assert torch.equal(a, b[:n])
+    two = route(odd, 8)
+    torch.testing.assert_close(two[2], got[2], rtol=1e-5, atol=1e-5 * math.sqrt(width))
+    clear = (two[0] == got[0]).all(1)  # (a row without pieces of 16 bytes is added up in another order: a tie may fall the other way)
+    assert int(clear.sum()) >= 7
+    torch.testing.assert_close(two[1][clear], got[1][clear], rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("n,width,ff,experts,top", [(1, 256, 256, 2, 2), (65, 256, 264, 2, 1), (129, 384, 520, 3, 2), (300, 264, 136, 5, 2), (40, 2048, 1024, 16, 2), (64, 1024, 2048, 8, 2)])
+def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, gated):
+    """Experts' tiles: halves and whole ones (64 and 65 rows an expert, 128 and 129), inner sizes in whole pairs of stages and not, the
+    smaller and the larger tiles, an expert without rows."""
+    ops = _ops()
+    torch.manual_seed(n + ff)
+    h = torch.randn(n, width, dtype=torch.bfloat16, device=DEV)
+    mk = lambda a, b: (torch.randn(experts, a, b, device=DEV) * b**-0.5).bfloat16()
+    wg, wu, wd = mk(ff, width) if gated else None, mk(ff, width), mk(width, ff)
+    sel = torch.rand(n, experts, device=DEV).mul_(torch.arange(experts, device=DEV) != experts - 1).topk(top, -1).indices.int() if experts > top else \
+        torch.arange(top, device=DEV).int().repeat(n, 1)
+    wt = torch.rand(n, top, device=DEV)
+    tiles = int(ops.build.core().ns_moe_group_tiles(n * top, experts))
+    ints = torch.full((n * top + 3 * tiles + 64,), 77, dtype=torch.int32, device=DEV)
+    out = torch.full((n, top, width), float("nan"), device=DEV)
+    ops.moe_expert_groups(h, wg, wu, wd, sel.contiguous(), wt, 7.0, 1.702, ints[: n * top + 3 * tiles], torch.empty(n * top, ff, dtype=torch.bfloat16, device=DEV), out, shift=1.0,
+                          activation=None if gated else "silu")
+    assert bool((ints[-64:] == 77).all())
+    x = h.double().cpu()
+    for t in range(0, n, max(1, n // 16)):
+        for k in range(top):
+            e = int(sel[t, k])
+            u = (wu[e].double().cpu() @ x[t]).bfloat16().double()
+            if gated:
+                g = (wg[e].double().cpu() @ x[t]).bfloat16().double().clamp(max=7.0)
+                a = g * torch.sigmoid(1.702 * g) * (u.clamp(-7.0, 7.0) + 1.0)
+            else:
+                a = u * torch.sigmoid(u)
+            y = float(wt[t, k]) * (wd[e].double().cpu() @ a.bfloat16().double())
+            # the roundings of act to 8 bits, where a sum in another order falls to the other side: some of ff of them
+            err = float((out[t, k].double().cpu() - y).norm() / y.norm())
+            assert err < 2**-8, (t, k, err)

@@ -1797,3 +1797,43 @@ def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, g
             # the roundings of act to 8 bits, where a sum in another order falls to the other side: some of ff of them
             err = float((out[t, k].double().cpu() - y).norm() / y.norm())
             assert err < 2**-8, (t, k, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,width", [(1, 8), (3, 2056), (70, 4096), (5, 36), (4, 77)])
+def test_scaled_sum_and_clipped_glu_in_pieces_and_alone(dtype, n, width):
+    """Rows in whole pieces of 16 bytes and rows that are not, results at the edges of a workgroup, what is no number where it was in a sum."""
+    ops = _ops()
+    torch.manual_seed(n + width)
+    a, b = (torch.randn(n, width, device=DEV).mul_(3).to(dtype) for _ in range(2))
+    u, v = (torch.randn(width, device=DEV).to(dtype) for _ in range(2))
+    a[0, 0], b[0, width - 1], a[n - 1, width - 1] = float("nan"), float("inf"), float("-inf")
+    eps = 2**-8 if dtype == torch.bfloat16 else 2**-22
+    for bias, bias_b in ((None, None), (u, None), (u, v)):
+        ref = 0.75 * (a.double() + (0 if bias is None else bias.double())) - 1.5 * (b.double() + (0 if bias_b is None else bias_b.double()))
+        got = ops.scaled_sum(a, b, 0.75, -1.5, torch.empty_like(a), bias=bias, bias_b=bias_b)
+        torch.testing.assert_close(got.double(), ref, rtol=eps, atol=1e-5, equal_nan=True)
+    a, b = a.nan_to_num(1.0, -30.0, 30.0), b.nan_to_num(1.0, 30.0, -30.0)
+    g, up = a.double().clamp(max=7.0), b.double().clamp(-7.0, 7.0)
+    got = ops.clipped_glu(torch.cat([a, b], 1), 7.0, 1.702, torch.empty_like(a), shift=1.0)
+    torch.testing.assert_close(got.double(), g * torch.sigmoid(1.702 * g) * (up + 1.0), rtol=2 * eps, atol=1e-6)
+
+
+def test_silu_and_gelu_at_the_ends_of_their_range():
+    """bfloat16 results by the vector unit's own exponential and reciprocal: every bfloat16 value against 64 bits, within half an ulp of the
+    result (2^-8 of it at most, 8 bits) and a hair of its 32-bit value, and exact at the ends."""
+    ops = _ops()
+    z = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    z = z[torch.isfinite(z)]
+    z = torch.cat([z, torch.zeros(-len(z) % 64, dtype=torch.bfloat16)]).view(-1, 64).contiguous()
+    d = z.double()
+    u = 0.7978845608028654 * (d + 0.044715 * d**3)
+    refs = {"silu": torch.where(d < -700, torch.zeros_like(d), d / (1 + torch.exp(-d.clamp(min=-700)))),
+            "gelu_tanh": torch.where(u < -350, torch.zeros_like(d), d / (1 + torch.exp(-2 * u.clamp(min=-350))))}
+    for kind, ref in refs.items():
+        got = ops.activation(z.to(DEV).clone(), kind).cpu().double()
+        # (2^-110: below it a result may be zero where the divisor or the power is out of range)
+        assert bool(((got - ref).abs() <= ref.abs() * (2**-8 + 2**-19) + 2.0**-110).all()), kind
+        ends = torch.tensor([[float("inf"), float("nan")] * 32], dtype=torch.bfloat16, device=DEV)
+        out = ops.activation(ends, kind)
+        assert bool(torch.isinf(out[0, 0])) and float(out[0, 0]) > 0 and bool(torch.isnan(out[0, 1])), kind

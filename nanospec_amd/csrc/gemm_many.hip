@@ -85,7 +85,7 @@ __global__ __launch_bounds__(T::WAVES * NS_WAVE) __attribute__((amdgpu_waves_per
           o[e] = from_f<bf16_t>(to_f((bf16_t)o[e]) + z);
         else if (EPI == MANY_GATED) {
           const float gate = round_to<bf16_t>(z), up = round_to<bf16_t>(t.acc[i][T::NH + j][e]);
-          o[e] = from_f<bf16_t>(silu_as<bf16_t>(gate) * up);
+          o[e] = from_f<bf16_t>(gate / (1.f + expf(-gate)) * up);
         } else
           o[e] = from_f<bf16_t>(z);
       }

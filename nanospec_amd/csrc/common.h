@@ -23,21 +23,6 @@ template <typename T> __device__ __forceinline__ float round_to(float v) { retur
 // The activations a kernel may be asked for by number: 0 the tanh form of GELU, 0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715
 // z^3))); 1 SiLU, z sigmoid(z); 2 the square of the ReLU.
 #define NS_ACTIVATIONS 3
-// v / (1 + exp(-z)).  For a result that is stored as bfloat16 in some 15 instructions, where expf and a division take 25 (a wave's instruction takes four
-// cycles, and in the epilogue of a product nothing else is there to do): 2^t by the vector unit with what t = -z log2(e) rounds away added, its reciprocal, and
-// the quotient once put right.  In the 2-norm 4.0e-8 from 64 bits either way (v = z normal: 4.02e-8 and 3.99e-8, hence not in 32 bits).  2,048 x 28,672 bfloat16 values, gate and up:
-// 28.4 -> 27.1 us; 32 gated experts of 1,024, 2,048 tokens chosen evenly, 154 -> 152.6.
-// Beyond z = 100 the divisor is 1 and an infinite v stays; below -87 the divisor stays that of -87, whose reciprocal is a number still, and below -104 the quotient is 0.
-template <typename T>
-__device__ __forceinline__ float times_sigmoid(float v, float z) {
-  if constexpr (sizeof(T) == 4) return v / (1.f + expf(-z));
-  constexpr float LOG2E = 1.44269504f, REST = 1.92596299e-8f, LN2 = 0.693147181f;  // log2(e) in two parts
-  const float a = fminf(fmaxf(-z, -100.f), 87.f), t = a * LOG2E, off = fmaf(a, REST, fmaf(a, LOG2E, -t));
-  const float e = __builtin_amdgcn_exp2f(t), d = 1.f + fmaf(e, off * LN2, e), r = __builtin_amdgcn_rcpf(d);
-  const float n = z < -104.f ? 0.f * v : v, q = n * r;
-  return z > 100.f ? v : fmaf(fmaf(-d, q, n), r, q);
-}
-template <typename T> __device__ __forceinline__ float silu_as(float z) { return times_sigmoid<T>(z, z); }
 // The tanh form of GELU as what it takes away: with e = exp(-2 |u|) <= 1, z e / (1 + e) for z <= 0, and z minus that above.  What is taken away is small where z is
 // large, so the vector unit's own 2^x and 1 / x (an ulp each) are nearer than 0.5 z (1 + tanhf(u)), whose sum rounds at 1: against 64 bits in
 // the 2-norm, z normal with a deviation of 0.3, 1.2, 4: 4.12e-8, 2.76e-8, 1.60e-8 and before 4.10e-8, 3.68e-8, 2.15e-8 (largest 2.4e-7 and 4.3e-7).
@@ -47,11 +32,10 @@ __device__ __forceinline__ float gelu_tanh(float z) {
   const float e = __builtin_amdgcn_exp2f(-fabsf(z * fmaf(A * 0.044715f, z * z, A))), share = e * __builtin_amdgcn_rcpf(1.f + e);
   return z <= 0.f ? z * share : e > 0.f ? fmaf(-share, z, z) : z;
 }
-// (T: what the result is stored as)
-template <typename T>
+__device__ __forceinline__ float silu_of(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float activation_of(float z, int act) {
   if (act == 0) return gelu_tanh(z);
-  if (act == 1) return silu_as<T>(z);
+  if (act == 1) return silu_of(z);
   const float r = fmaxf(z, 0.f);
   return r * r;
 }

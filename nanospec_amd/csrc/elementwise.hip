@@ -524,7 +524,7 @@ __global__ void silu_mul_kernel(T* __restrict__ out, const T* __restrict__ gu, i
     const size_t n = e / inter;
     const int i = (int)(e - n * inter);
     const float g = to_f(gu[n * 2 * inter + i]), u = to_f(gu[n * 2 * inter + inter + i]);
-    out[e] = from_f<T>(silu_as<T>(g) * u);
+    out[e] = from_f<T>(silu_of(g) * u);
   }
 }
 
@@ -542,7 +542,7 @@ __global__ void silu_mul_vec_kernel(T* __restrict__ out, const T* __restrict__ g
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       const float gf = to_f(g[k]);
-      y[k] = from_f<T>(silu_as<T>(gf) * to_f(u[k]));
+      y[k] = from_f<T>(silu_of(gf) * to_f(u[k]));
     }
     reinterpret_cast<vec_t*>(out + n * inter)[i] = y;
   }
@@ -574,7 +574,7 @@ __global__ void silu_mul_bias_kernel(T* __restrict__ out, const T* __restrict__ 
     const size_t n = e / inter;
     const int i = (int)(e - n * inter);
     const float g = to_f(gu[n * 2 * inter + i]) + to_f(bias[i]), u = to_f(gu[n * 2 * inter + inter + i]) + to_f(bias[inter + i]);
-    out[e] = from_f<T>(silu_as<T>(g) * u);
+    out[e] = from_f<T>(silu_of(g) * u);
   }
 }
 
@@ -592,7 +592,7 @@ __global__ void silu_mul_bias_vec_kernel(T* __restrict__ out, const T* __restric
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       const float gf = to_f(g[k]) + to_f(bg[k]);
-      y[k] = from_f<T>(silu_as<T>(gf) * (to_f(u[k]) + to_f(bu[k])));
+      y[k] = from_f<T>(silu_of(gf) * (to_f(u[k]) + to_f(bu[k])));
     }
     reinterpret_cast<vec_t*>(out + n * inter)[i] = y;
   }

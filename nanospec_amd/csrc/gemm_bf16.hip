@@ -288,7 +288,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_tiled_kernel(OutT* __restrict
     }
     if (EPI == EPI_ACT) {
       const float z = (float)(bf16_t)s;
-      s = activation_of<OutT>(z, nl.act);
+      s = activation_of(z, nl.act);
     }
     out[(size_t)m * out_stride + n] = (OutT)s;
   }

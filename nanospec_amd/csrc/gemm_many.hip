@@ -80,7 +80,7 @@ __global__ __launch_bounds__(T::WAVES * NS_WAVE) __attribute__((amdgpu_waves_per
         const float z = t.acc[i][j][e];
         // (what stands between the product and an activation is rounded as a store would round it)
         if (EPI == MANY_ACT)
-          o[e] = from_f<bf16_t>(activation_of<bf16_t>(round_to<bf16_t>(z), p.act));
+          o[e] = from_f<bf16_t>(activation_of(round_to<bf16_t>(z), p.act));
         else if (EPI == MANY_ADD)
           o[e] = from_f<bf16_t>(to_f((bf16_t)o[e]) + z);
         else if (EPI == MANY_GATED) {

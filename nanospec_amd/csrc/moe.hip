@@ -444,11 +444,10 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
   return ns_launch_status();
 }
 
-template <typename T>
 __device__ __forceinline__ float clipped_glu(float g, float u, float limit, float alpha, float shift) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return times_sigmoid<T>(g, alpha * g) * (u + shift);
+  return g / (1.f + expf(-alpha * g)) * (u + shift);
 }
 
 // ------------------------------------------------------------------------------------------------ few rows
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(256) void moe_rows_up_kernel(const T* __restrict__ 
     const float g = wg ? row_dot(wg + row, moe_lds, W, lane, vec) : 0.f, u = row_dot(wu + row, moe_lds, W, lane, vec);
     if (lane == 0)
       act[((size_t)t * top + k) * ff + f] =
-          round_to<T>(wg ? clipped_glu<T>(round_to<T>(g), round_to<T>(u), limit, alpha, shift) : activation_of<T>(round_to<T>(u), act_kind));
+          round_to<T>(wg ? clipped_glu(round_to<T>(g), round_to<T>(u), limit, alpha, shift) : activation_of(round_to<T>(u), act_kind));
   }
 }
 
@@ -706,9 +705,9 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
   for (int i = 0; i < MATS; ++i) v[i] = (part[0][i][row][c] + part[1][i][row][c]) + (part[2][i][row][c] + part[3][i][row][c]);
   const int slot = r0 + row;
   if (DUAL)
-    act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu<bf16_t>(round_to<bf16_t>(v[0]), round_to<bf16_t>(v[MATS - 1]), limit, alpha, shift));
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(clipped_glu(round_to<bf16_t>(v[0]), round_to<bf16_t>(v[MATS - 1]), limit, alpha, shift));
   else if (FIRST)
-    act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of<bf16_t>(round_to<bf16_t>(v[0]), act_kind));
+    act_out[(size_t)slot * N + col] = from_f<bf16_t>(activation_of(round_to<bf16_t>(v[0]), act_kind));
   else
     out[(size_t)perm[slot] * N + col] = wt[perm[slot]] * v[0];
 }
@@ -784,7 +783,7 @@ __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const float z = round_to<bf16_t>(t.acc[i][j][q]);
-          o[q] = from_f<bf16_t>(DUAL ? clipped_glu<bf16_t>(z, round_to<bf16_t>(t.acc[i][T::NH + j][q]), p.limit, p.alpha, p.shift) : activation_of<bf16_t>(z, p.act_kind));
+          o[q] = from_f<bf16_t>(DUAL ? clipped_glu(z, round_to<bf16_t>(t.acc[i][T::NH + j][q]), p.limit, p.alpha, p.shift) : activation_of(z, p.act_kind));
         }
         *reinterpret_cast<bf16x4*>(p.act_out + (size_t)slot * p.N + col) = o;
       } else {
@@ -941,7 +940,7 @@ template <typename T>
 __global__ void clipped_glu_kernel(T* __restrict__ out, const T* __restrict__ gu, int gu_stride, int ff, size_t count, float limit, float alpha, float shift) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
     const size_t t = i / ff, f = i % ff;
-    out[i] = from_f<T>(clipped_glu<T>(to_f(gu[t * gu_stride + f]), to_f(gu[t * gu_stride + ff + f]), limit, alpha, shift));
+    out[i] = from_f<T>(clipped_glu(to_f(gu[t * gu_stride + f]), to_f(gu[t * gu_stride + ff + f]), limit, alpha, shift));
   }
 }
 
@@ -957,7 +956,7 @@ __global__ __launch_bounds__(256) void clipped_glu_vec_kernel(T* __restrict__ ou
     const vec_t g = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + f), u = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + ff + f);
     vec_t o;
 #pragma unroll
-    for (int i = 0; i < V; ++i) o[i] = from_f<T>(clipped_glu<T>(to_f((T)g[i]), to_f((T)u[i]), limit, alpha, shift));
+    for (int i = 0; i < V; ++i) o[i] = from_f<T>(clipped_glu(to_f((T)g[i]), to_f((T)u[i]), limit, alpha, shift));
     *reinterpret_cast<vec_t*>(out + t * ff + f) = o;
   }
 }

@@ -405,7 +405,7 @@ extern "C" int ns_stream_step(float* x, const float* mix, const float* gain, con
 template <typename T>
 __global__ void activation_kernel(T* __restrict__ out, const T* __restrict__ x, size_t count, int act) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
-    out[i] = from_f<T>(activation_of<T>(to_f(x[i]), act));
+    out[i] = from_f<T>(activation_of(to_f(x[i]), act));
   }
 }
 
@@ -420,7 +420,7 @@ __global__ void activation_vec_kernel(T* __restrict__ out, const T* __restrict__
     const vec_t a = xv[i];
     vec_t r;
 #pragma unroll
-    for (int e = 0; e < V; ++e) r[e] = from_f<T>(activation_of<T>(to_f(a[e]), act));
+    for (int e = 0; e < V; ++e) r[e] = from_f<T>(activation_of(to_f(a[e]), act));
     ov[i] = r;
   }
 }

@@ -1819,21 +1819,47 @@ def test_scaled_sum_and_clipped_glu_in_pieces_and_alone(dtype, n, width):
     torch.testing.assert_close(got.double(), g * torch.sigmoid(1.702 * g) * (up + 1.0), rtol=2 * eps, atol=1e-6)
 
 
-def test_silu_and_gelu_at_the_ends_of_their_range():
-    """bfloat16 results by the vector unit's own exponential and reciprocal: every bfloat16 value against 64 bits, within half an ulp of the
-    result (2^-8 of it at most, 8 bits) and a hair of its 32-bit value, and exact at the ends."""
-    ops = _ops()
+def _finite_bf16():
     z = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     z = z[torch.isfinite(z)]
-    z = torch.cat([z, torch.zeros(-len(z) % 64, dtype=torch.bfloat16)]).view(-1, 64).contiguous()
+    return torch.cat([z, torch.zeros(-len(z) % 64, dtype=torch.bfloat16)]).view(-1, 64).contiguous()
+
+
+def _within_half_a_step(got, ref, floor):
+    """bfloat16 results within half a step of 64 bits (2^-8 of the value: 8 bits) and a hair of the 32-bit value; results below ``floor`` no larger than
+    the true one and of its sign."""
+    near = (got - ref).abs() <= ref.abs() * (2**-8 + 2**-19) + 2.0**-134  # (half of the smallest bfloat16)
+    return bool((near | ((ref.abs() < floor) & (got.abs() <= ref.abs()) & (got * ref >= 0))).all())
+
+
+def test_silu_at_the_ends_of_its_range():
+    """Every finite bfloat16 value against 64 bits, in each kernel that divides by 1 + exp(-z) with nothing else behind it: down to where the
+    divisor is out of range (z = -88.7, a result of 2^-121), and zero from there on, not something that grows."""
+    ops = _ops()
+    z = _finite_bf16()
+    d = z.double()
+    ref = torch.where(d < -700, torch.zeros_like(d), d / (1 + torch.exp(-d.clamp(min=-700))))
+    g, one, zero = z.to(DEV), torch.ones_like(z, device=DEV), torch.zeros_like(z, device=DEV)
+    bias = torch.zeros(128, dtype=torch.bfloat16, device=DEV)
+    for name, got in (("activation", ops.activation(g.clone(), "silu")), ("silu_mul", ops.silu_mul(torch.cat([g, one], 1))),
+                      ("silu_mul_bias", ops.silu_mul_bias(torch.cat([g, one], 1), bias)),
+                      ("clipped_glu", ops.clipped_glu(torch.cat([g, zero], 1), float("inf"), 1.0, torch.empty_like(g), shift=1.0))):
+        got = got.cpu().double()
+        assert _within_half_a_step(got, ref, 2.0**-121), name
+        assert bool((got[d < -89] == 0).all()), name
+    ends = torch.tensor([[float("inf"), float("nan")] * 32], dtype=torch.bfloat16, device=DEV)
+    out = ops.activation(ends, "silu")
+    assert bool(torch.isinf(out[0, 0])) and float(out[0, 0]) > 0 and bool(torch.isnan(out[0, 1]))
+
+
+def test_gelu_at_the_ends_of_its_range():
+    """Every finite bfloat16 value against 64 bits: down to where the exponential is out of range (a result of some 2^-123), and exact at the ends."""
+    ops = _ops()
+    z = _finite_bf16()
     d = z.double()
     u = 0.7978845608028654 * (d + 0.044715 * d**3)
-    refs = {"silu": torch.where(d < -700, torch.zeros_like(d), d / (1 + torch.exp(-d.clamp(min=-700)))),
-            "gelu_tanh": torch.where(u < -350, torch.zeros_like(d), d / (1 + torch.exp(-2 * u.clamp(min=-350))))}
-    for kind, ref in refs.items():
-        got = ops.activation(z.to(DEV).clone(), kind).cpu().double()
-        # (2^-110: below it a result may be zero where the divisor or the power is out of range)
-        assert bool(((got - ref).abs() <= ref.abs() * (2**-8 + 2**-19) + 2.0**-110).all()), kind
-        ends = torch.tensor([[float("inf"), float("nan")] * 32], dtype=torch.bfloat16, device=DEV)
-        out = ops.activation(ends, kind)
-        assert bool(torch.isinf(out[0, 0])) and float(out[0, 0]) > 0 and bool(torch.isnan(out[0, 1])), kind
+    ref = torch.where(u < -350, torch.zeros_like(d), d / (1 + torch.exp(-2 * u.clamp(min=-350))))
+    assert _within_half_a_step(ops.activation(z.to(DEV).clone(), "gelu_tanh").cpu().double(), ref, 2.0**-121)
+    ends = torch.tensor([[float("inf"), float("nan")] * 32], dtype=torch.bfloat16, device=DEV)
+    out = ops.activation(ends, "gelu_tanh")
+    assert bool(torch.isinf(out[0, 0])) and float(out[0, 0]) > 0 and bool(torch.isnan(out[0, 1]))

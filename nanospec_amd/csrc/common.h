@@ -35,12 +35,14 @@ __device__ __forceinline__ float gelu_tanh(float z) {
   return z <= 0.f ? z * share : e > 0.f ? fmaf(-share, z, z) : z;
 }
 __device__ __forceinline__ float silu_of(float z) { return z / (1.f + expf(-z)); }
-__device__ __forceinline__ float activation_of(float z, int act) {
-  if (act == 0) return gelu_tanh(z);
-  if (act == 1) return silu_of(z);
+template <int ACT>
+__device__ __forceinline__ float activation_as(float z) {
+  if constexpr (ACT == 0) return gelu_tanh(z);
+  if constexpr (ACT == 1) return silu_of(z);
   const float r = fmaxf(z, 0.f);
   return r * r;
 }
+__device__ __forceinline__ float activation_of(float z, int act) { return act == 0 ? activation_as<0>(z) : act == 1 ? activation_as<1>(z) : activation_as<2>(z); }
 
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 

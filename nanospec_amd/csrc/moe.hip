@@ -717,7 +717,7 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
 // half a tile.  Bound by the matrices' bytes up to some hundred tokens, beyond by the way from L2 to LDS and by how unevenly the experts' tiles deal.  us a call, sorting
 // included, before (tiles by eight waves a whole stage ahead, every tile whole) and now, width 2,048, four of 32 a token, chosen unevenly (as a model's router does): 1,024
 // channels with gates, 508 tokens 119 and 98, 1,531 149 and 146, 2,048 198 and 195; evenly 77 and 75, 147 and 141, 162 and 150; 1,536 without gates,
-// 2,048 tokens 196 and 200, evenly 174 and 181 (one and a half tiles a compute unit: a tile's end, with nothing beside it, counts); six of 64 of 1,408 without gates, 300 tokens 155 and
+// 2,048 tokens 193 and 185, evenly 174 and 162; six of 64 of 1,408 without gates, 300 tokens 155 and
 // 138; two of 8 of 14,336 with gates, width 4,096, 2,000 tokens 1,719 and 1,653, evenly 1,502 and 1,330.
 // Workgroups go to the eight XCDs in launch order: each XCD takes an eighth of the work in use, neighbours first, so that an expert's
 // matrices and rows come into one L2.  Where an expert has several tiles, all of them take four blocks of
@@ -735,10 +735,48 @@ struct MoeTileParams {
   float limit, alpha, shift;
 };
 
+// What follows a tile's products.  The activation (ACT; of experts without gates) is chosen once for the tile: with a choice for every value a wave, alone on its
+// SIMD, waits for each value's chain of instructions (the first product of 32 experts of 1,536, width 2,048, 2,048 tokens, four a token evenly: 109 us with the
+// choice inside, 87 as it is; the square of the ReLU, the whole call 183 and 162, chosen unevenly 201 and 185, 1,024 tokens 121 and 109).
+template <class T, bool FIRST, bool DUAL, int ACT>
+__device__ __forceinline__ void moe_tile_results(const MoeTileParams& p, const T& t, int r0, int rows, int n0) {
+  constexpr int NJ = DUAL ? T::NH : T::NJ;
+  const int r = t.lane % 16, g = t.lane / 16;
+#pragma unroll
+  for (int i = 0; i < T::MI; ++i) {
+    const int row = 16 * (2 * i + t.wm) + r;
+    if (row >= rows) continue;
+    const int slot = r0 + row;
+    const int pair = FIRST ? 0 : p.perm[slot];
+    const float share_of = FIRST ? 0.f : p.wt[pair];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int col = n0 + 16 * (2 * j + t.wn) + 4 * g;
+      if (col >= p.N) continue;  // (N is a multiple of 8: four columns are all inside or all outside)
+      if (FIRST) {
+        typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float z = round_to<bf16_t>(t.acc[i][j][q]);
+          o[q] = from_f<bf16_t>(DUAL ? clipped_glu(z, round_to<bf16_t>(t.acc[i][T::NH + j][q]), p.limit, p.alpha, p.shift) : activation_as<ACT>(z));
+        }
+        *reinterpret_cast<bf16x4*>(p.act_out + (size_t)slot * p.N + col) = o;
+      } else {
+        typedef float f32x4_anywhere __attribute__((ext_vector_type(4), aligned(4)));  // (``out`` is a float's address and no more)
+        f32x4_anywhere o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = share_of * t.acc[i][j][q];
+        *reinterpret_cast<f32x4_anywhere*>(p.out + (size_t)pair * p.N + col) = o;
+      }
+    }
+  }
+}
+
 // ``rows`` sorted rows from ``r0`` on times expert e's rows of the matrices from channel n0 on
 template <class T, bool FIRST, bool DUAL, bool ANY>
 __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds, int e, int r0, int rows, int n0, int turn) {
-  constexpr int HALF = T::BN / 2, NJ = DUAL ? T::NH : T::NJ;
+  constexpr int HALF = T::BN / 2;
   T t;
   t.init(lds, p.K, turn);
 #pragma unroll
@@ -765,36 +803,12 @@ __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds
   }
   t.run();
 
-  const int r = t.lane % 16, g = t.lane / 16;
-#pragma unroll
-  for (int i = 0; i < T::MI; ++i) {
-    const int row = 16 * (2 * i + t.wm) + r;
-    if (row >= rows) continue;
-    const int slot = r0 + row;
-    const int pair = FIRST ? 0 : p.perm[slot];
-    const float share_of = FIRST ? 0.f : p.wt[pair];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int col = n0 + 16 * (2 * j + t.wn) + 4 * g;
-      if (col >= p.N) continue;  // (N is a multiple of 8: four columns are all inside or all outside)
-      if (FIRST) {
-        typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
-        bf16x4 o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float z = round_to<bf16_t>(t.acc[i][j][q]);
-          o[q] = from_f<bf16_t>(DUAL ? clipped_glu(z, round_to<bf16_t>(t.acc[i][T::NH + j][q]), p.limit, p.alpha, p.shift) : activation_of(z, p.act_kind));
-        }
-        *reinterpret_cast<bf16x4*>(p.act_out + (size_t)slot * p.N + col) = o;
-      } else {
-        typedef float f32x4_anywhere __attribute__((ext_vector_type(4), aligned(4)));  // (``out`` is a float's address and no more)
-        f32x4_anywhere o;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = share_of * t.acc[i][j][q];
-        *reinterpret_cast<f32x4_anywhere*>(p.out + (size_t)pair * p.N + col) = o;
-      }
-    }
-  }
+  if (!FIRST || DUAL || p.act_kind == 2)
+    moe_tile_results<T, FIRST, DUAL, 2>(p, t, r0, rows, n0);
+  else if (p.act_kind == 1)
+    moe_tile_results<T, FIRST, DUAL, 1>(p, t, r0, rows, n0);
+  else
+    moe_tile_results<T, FIRST, DUAL, 0>(p, t, r0, rows, n0);
 }
 
 template <class S, bool FIRST, bool DUAL, bool ANY>

@@ -1764,6 +1764,52 @@ def test_moe_route_of_few_tokens_in_one_launch(dtype, experts, extra, top, group
     torch.testing.assert_close(two[1][clear], got[1][clear], rtol=1e-4, atol=1e-6)
 
 
+def _check_experts(out, h, gate, up, down, sel, wt, limit, alpha, shift, activation):
+    """``out`` [tokens, top, width] against 64 bits.  An inner channel's sum may round to the next bfloat16 (2^-8 of it at most), and so may the
+    activation made of it."""
+    x = h.double()
+    for e in range(up.shape[0]):
+        t, k = (sel == e).nonzero(as_tuple=True)
+        if not len(t):
+            continue
+        u = (x[t] @ up[e].double().T).bfloat16().double()
+        if gate is not None:
+            a = (x[t] @ gate[e].double().T).bfloat16().double().clamp(max=limit)
+            act = a * torch.sigmoid(alpha * a) * (u.clamp(-limit, limit) + shift)
+        else:
+            act = {"relu2": lambda v: v.clamp(min=0) ** 2, "silu": lambda v: v * torch.sigmoid(v),
+                   "gelu_tanh": lambda v: v * torch.sigmoid(2 * 0.7978845608028654 * (v + 0.044715 * v**3))}[activation](u)
+        act = act.bfloat16().double()
+        share = wt[t, k].double()[:, None]
+        want, bound = share * (act @ down[e].double().T), share * 2.0**-6 * (act.abs() @ down[e].double().abs().T) + 1e-5
+        assert bool(((out[t, k].double() - want).abs() <= bound).all()), e
+
+
+def _experts_call(n, width, ff, experts, sel, gated, activation, seed):
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    h = rnd(n, width).bfloat16()
+    gate, up, down = ((rnd(experts, *s) * s[1] ** -0.5).bfloat16() for s in ((ff, width), (ff, width), (width, ff)))
+    gate = gate if gated else None
+    top = sel.shape[1]
+    sel, wt = sel.to(DEV).int().contiguous(), torch.rand(n, top, generator=g, device=DEV)
+    tiles = int(ops.build.core().ns_moe_group_tiles(n * top, experts))
+    ints = torch.full((n * top + 3 * tiles + 64,), 77, dtype=torch.int32, device=DEV)
+    act, out = torch.full((n * top, ff), float("nan"), dtype=torch.bfloat16, device=DEV), torch.full((n, top, width), float("nan"), device=DEV)
+    ops.moe_expert_groups(h, gate, up, down, sel, wt, 7.0, 1.702, ints[: n * top + 3 * tiles], act, out, shift=1.0, activation=activation)
+    assert bool((ints[-64:] == 77).all())
+    _check_experts(out, h, gate, up, down, sel, wt, 7.0, 1.702, 1.0, activation)
+
+
+@pytest.mark.parametrize("activation", ["relu2", "silu", "gelu_tanh"])
+@pytest.mark.parametrize("n,width,ff,experts", [(400, 256, 384, 3), (40, 256, 384, 3), (9, 256, 384, 3), (400, 264, 136, 3)])
+def test_experts_without_gates_apply_each_activation(n, width, ff, experts, activation):
+    """In the larger tiles, the smaller ones, streamed, and where the inner size is in no whole pairs of stages."""
+    sel = torch.randint(0, experts, (n, 1), generator=torch.Generator().manual_seed(n))
+    _experts_call(n, width, ff, experts, sel, False, activation, n)
+
+
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("n,width,ff,experts,top", [(1, 256, 256, 2, 2), (65, 256, 264, 2, 1), (129, 384, 520, 3, 2), (300, 264, 136, 5, 2), (40, 2048, 1024, 16, 2), (64, 1024, 2048, 8, 2)])
 def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, gated):

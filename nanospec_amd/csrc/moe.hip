@@ -725,6 +725,9 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16_t* __restric
 // width 4,096, 14,336 channels with gates, 2,000 tokens, with the tiles before: 2,264 and 1,689).
 // Every expert begins at a stage of K of its own, and in the smaller tiles every block of channels too:
 // workgroups that all read the same columns of rows 4 KiB apart keep a few memory channels busy (begun alike: 2 to 10% slower; in the larger tiles by blocks too: 1 to 4%).
+// Inner sizes of an odd number of stages (2,880, 704) have a form of their own: with 64-bit addresses and a choice for every load, as sizes of no whole stages have them, and read
+// through the caches, width and channels 2,880, with gates, took (evenly and unevenly) 64 tokens 284 and 192 us and take 260 and 178, 300 300 and 306 and 281 and 289, 512 319
+// and 345 and 300 and 332, 1,024 377 and 424 and 358 and 411, 2,048 545 and 642 and 513 and 580.
 struct MoeTileParams {
   const bf16_t *A, *B0, *B1;
   const int *perm, *tile_e, *tile_r0, *tile_rows;
@@ -774,7 +777,7 @@ __device__ __forceinline__ void moe_tile_results(const MoeTileParams& p, const T
 }
 
 // ``rows`` sorted rows from ``r0`` on times expert e's rows of the matrices from channel n0 on
-template <class T, bool FIRST, bool DUAL, bool ANY>
+template <class T, bool FIRST, bool DUAL>
 __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds, int e, int r0, int rows, int n0, int turn) {
   constexpr int HALF = T::BN / 2;
   T t;
@@ -787,7 +790,7 @@ __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds
 #pragma unroll
     for (int q = 0; q < T::LA; ++q) {
       const int row = min(h * (T::BM / 2) + t.row_of(q), rows - 1), at = FIRST ? p.perm[r0 + row] / p.top : row;
-      if (ANY)
+      if (T::ANY)
         t.x_row(h, q, x + (size_t)at * p.a_stride);
       else
         t.xo[h][q] = 2 * (at * p.a_stride + t.piece());
@@ -795,7 +798,7 @@ __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds
 #pragma unroll
     for (int q = 0; q < T::LB; ++q) {
       const int row = min((DUAL ? 0 : h * HALF) + t.row_of(q), p.N - 1 - n0);
-      if (ANY)
+      if (T::ANY)
         t.w_row(h, q, w + (size_t)row * p.K);
       else
         t.wo[h][q] = 2 * (row * p.K + t.piece());
@@ -811,11 +814,19 @@ __device__ __forceinline__ void moe_one_tile(const MoeTileParams& p, bf16_t* lds
     moe_tile_results<T, FIRST, DUAL, 0>(p, t, r0, rows, n0);
 }
 
-template <class S, bool FIRST, bool DUAL, bool ANY>
+template <class S, bool FIRST, bool DUAL, QuarterInner INNER, bool W_ONCE>
+__device__ __forceinline__ void moe_half_or_whole(const MoeTileParams& p, bf16_t* lds, int e, int r0, int rows, int n0, int turn) {
+  if (rows <= MG_ROWS / 2)
+    moe_one_tile<QuarterTile<MG_ROWS / 2, S::BN, S::HALF_STAGES, W_ONCE, INNER>, FIRST, DUAL>(p, lds, e, r0, rows, n0, turn);
+  else
+    moe_one_tile<QuarterTile<MG_ROWS, S::BN, 2, W_ONCE, INNER>, FIRST, DUAL>(p, lds, e, r0, rows, n0, turn);
+}
+
+template <class S, bool FIRST, bool DUAL, QuarterInner INNER>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void moe_tile_kernel(const MoeTileParams p) {
   constexpr int CH = DUAL ? S::BN / 2 : S::BN;  // output channels of a workgroup
-  typedef QuarterTile<MG_ROWS, S::BN, 2, S::W_ONCE, ANY> Whole;
-  typedef QuarterTile<MG_ROWS / 2, S::BN, S::HALF_STAGES, S::W_ONCE, ANY> Half;
+  typedef QuarterTile<MG_ROWS, S::BN, 2> Whole;
+  typedef QuarterTile<MG_ROWS / 2, S::BN, S::HALF_STAGES> Half;
   __shared__ __attribute__((aligned(16))) bf16_t moe_tiles[Whole::VALUES > Half::VALUES ? Whole::VALUES : Half::VALUES];
   const int blocks_n = (p.N + CH - 1) / CH;
   const long long used = (long long)p.tile_r0[p.tiles - 1] * blocks_n, share = (used + 7) / 8;
@@ -832,10 +843,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void m
   }
   const int row0 = rows_before_tile(c, of_e, nth), rows = rows_before_tile(c, of_e, nth + 1) - row0;
   const int n0 = block * CH, r0 = p.tile_r0[some] + row0;
-  if (rows <= MG_ROWS / 2)
-    moe_one_tile<Half, FIRST, DUAL, ANY>(p, moe_tiles, e, r0, rows, n0, block * S::TURN + e * 11);
+  // Past the caches only what is read once.  (Inner sizes of an odd number of stages, experts of several tiles, with and without the hint: width and channels 2,880, with
+  // gates, 512 tokens of four experts, unevenly, 375 and 332 us; experts of one tile, evenly, 307 and 328, 64 tokens 250 and 285.)
+  const int first_stage = block * S::TURN + e * 11;
+  if (S::W_ONCE && INNER == QUARTER_ODD && of_e > 1)
+    moe_half_or_whole<S, FIRST, DUAL, INNER, false>(p, moe_tiles, e, r0, rows, n0, first_stage);
   else
-    moe_one_tile<Whole, FIRST, DUAL, ANY>(p, moe_tiles, e, r0, rows, n0, block * S::TURN + e * 11);
+    moe_half_or_whole<S, FIRST, DUAL, INNER, S::W_ONCE>(p, moe_tiles, e, r0, rows, n0, first_stage);
 }
 
 // Rows that a tile holds at most: 16 (the kernel that streams matrices) for the smallest steps, else 128 (the tiled ones).  The tiled kernels take some 28 us
@@ -858,7 +872,13 @@ static int moe_tiles(long long pairs, int experts, int cap) { return (int)((pair
 // and larger, evenly and unevenly chosen: with gates, 32 experts of 1,024, width 2,048, four a token: 64 rows an expert 79 and 91, 102 and 121, 128 rows 98 and 105, 142 and
 // 135, 192 rows 153 and 140, 158 and 144; 1,536 channels without gates 128 rows 112 and 121, 157 and 165, 256 rows 174 and 181, 217 and 199; 8 experts, width 4,096, two a
 // token: 4,096 channels 96 rows 153 and 182, 162 and 181, 128 rows 164 and 185, 243 and 222; 14,336 channels 64 rows 479 and 584, 501 and 600 (most unevenly 654 and 617).
-static bool moe_few_rows(long long pairs, int experts) { return pairs <= 96LL * experts; }
+// Inner sizes of an odd number of stages, whose smaller tiles read the matrices past the caches only where an expert has one tile (see moe_tile_kernel): up to 128. 128 and 192
+// rows, with gates, width 2,880, 2,880 channels: 358 and 343, 411 and 424; 499 and 480, 502 and 512; 1,440 channels 208 and 227, 246 and 262; width 2,048, 704 channels, 125
+// rows 75 and 81, 114 and 120.  Of no whole stages: the smaller ones at any number, on whose address and choice a load there is less to wait: 2,056 channels,
+// width 1,448, 256 rows 309 and 316, 329 and 338; 1,440 of 1,440 204 and 205, 219 and 228, without gates 512 rows 257 and 244, 274 and 290.
+static bool moe_few_rows(long long pairs, int experts, QuarterInner inner) {
+  return inner == QUARTER_ANY || pairs <= (inner == QUARTER_ODD ? 128LL : 96LL) * experts;
+}
 
 // tiles that any choice of experts can need, whichever kernel takes them
 extern "C" int ns_moe_group_tiles(int pairs, int experts) { return moe_tiles(pairs, experts, 16); }
@@ -883,26 +903,33 @@ struct MoeLaunch {
   const float* wt;
   int h_stride, W, ff, top, tiles, act_kind;
   float limit, alpha, shift;
-  bool few_rows;
-  long long rows;  // of h
+  long long pairs, rows;  // (rows of h)
+  int experts;
   hipStream_t stream;
 
-  template <class S, bool FIRST, bool DUAL, bool ANY>
+  template <class S, bool FIRST, bool DUAL, QuarterInner INNER>
   void launch(const MoeTileParams& p) const {
     constexpr int CH = DUAL ? S::BN / 2 : S::BN;
-    moe_tile_kernel<S, FIRST, DUAL, ANY><<<moe_tile_grid((long long)tiles * ((p.N + CH - 1) / CH)), 256, 0, stream>>>(p);
+    moe_tile_kernel<S, FIRST, DUAL, INNER><<<moe_tile_grid((long long)tiles * ((p.N + CH - 1) / CH)), 256, 0, stream>>>(p);
+  }
+  template <bool FIRST, bool DUAL, QuarterInner INNER>
+  void sized(const MoeTileParams& p) const {
+    if (moe_few_rows(pairs, experts, INNER))
+      launch<MoeFewTile, FIRST, DUAL, INNER>(p);
+    else if constexpr (INNER != QUARTER_ANY)
+      launch<MoeTile, FIRST, DUAL, INNER>(p);
   }
   template <bool FIRST, bool DUAL>
   void tiled(const bf16_t* a, int a_stride, const bf16_t* b0, const bf16_t* b1, int n, int k) const {
     const MoeTileParams p{a, b0, b1, perm, tile_e, tile_r0, tile_rows, act, out, wt, a_stride, tiles, n, k, top, act_kind, limit, alpha, shift};
-    // whole pairs of stages, and all rows within 31 bits of bytes of their first; other sizes are no model's
-    const bool plain = k % QUARTER_K_MULTIPLE == 0 && k >= 4 * QUARTER_K && k < 1 << 22 && a_stride < 1 << 22 && (!FIRST || rows * a_stride < 1LL << 30);
+    // whole stages, and all rows within 31 bits of bytes of their first
+    const bool plain = k % QUARTER_K == 0 && k >= (k / QUARTER_K % 2 ? 5 : 4) * QUARTER_K && k < 1 << 22 && a_stride < 1 << 22 && (!FIRST || rows * a_stride < 1LL << 30);
     if (!plain)
-      launch<MoeFewTile, FIRST, DUAL, true>(p);
-    else if (few_rows)
-      launch<MoeFewTile, FIRST, DUAL, false>(p);
+      sized<FIRST, DUAL, QUARTER_ANY>(p);
+    else if (k % QUARTER_K_MULTIPLE)
+      sized<FIRST, DUAL, QUARTER_ODD>(p);
     else
-      launch<MoeTile, FIRST, DUAL, false>(p);
+      sized<FIRST, DUAL, QUARTER_PAIRS>(p);
   }
   template <bool DUAL>
   void first(int cap) const {
@@ -940,7 +967,7 @@ extern "C" int ns_moe_expert_groups(const void* h, int h_stride, const void* wg,
   if (tiles > 65535) return NS_ERR_UNSUPPORTED;
   moe_sort_kernel<<<1, 1024, 0, stream>>>(sel, (int)pairs, experts, cap, perm, tile_e, tile_r0, tile_rows, tiles);
   const MoeLaunch l{(const bf16_t*)h, (const bf16_t*)wg, (const bf16_t*)wu, (const bf16_t*)wd, (bf16_t*)act, out, perm, tile_e, tile_r0,
-                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, moe_few_rows(pairs, experts), n, stream};
+                    tile_rows, wt, h_stride, W, ff, top, tiles, act_kind, limit, alpha, shift, pairs, n, experts, stream};
   if (wg)
     l.first<true>(cap);
   else

@@ -23,19 +23,23 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 #define QUARTER_K 64           // values of K a stage
 #define QUARTER_K_MULTIPLE 128  // what K must be a multiple of (an even number of stages)
 
+// What K may be.  PAIRS: an even number of stages.  ODD: an odd one; the first is multiplied ahead of the loop of pairs.  ANY: any multiple of 8 (stages beyond
+// K are zeros), and rows anywhere: an address of 64 bits and a choice for every load.
+enum QuarterInner { QUARTER_PAIRS, QUARTER_ODD, QUARTER_ANY };
+
 // Wave (wm, wn) of 2 x 2 owns the blocks of 16 rows wm, wm + 2, .. of x and wn, wn + 2, .. of w.  acc[i][j]: lane l holds for row 16 (2 i + wm) + l % 16 of x
 // the sums with rows 16 (2 j + wn) + 4 (l / 16) .. + 3 of w.
 // W_ONCE: most rows of w are read by one workgroup: past the caches.
-// ANY: any K that is a multiple of 8 (stages beyond it are zeros), and rows anywhere: an address of 64 bits and a choice for every load.
-template <int BM_, int BN_, int ST_ = 2, bool W_ONCE = false, bool ANY = false>
+template <int BM_, int BN_, int ST_ = 2, bool W_ONCE = false, QuarterInner INNER = QUARTER_PAIRS>
 struct QuarterTile {
+  static constexpr bool ANY = INNER == QUARTER_ANY;
   static constexpr int BM = BM_, BN = BN_, ST = ST_, WAVES = 4;
   static constexpr int MI = BM / 32, NJ = BN / 32, MH = MI / 2, NH = NJ / 2;
   static constexpr int UA = BM / 2 * QUARTER_K, UB = BN / 2 * QUARTER_K;   // values of a unit of x and of w
   static constexpr int STAGE = 2 * (UA + UB), VALUES = ST * STAGE;         // values of a stage, and of LDS
   static constexpr int LA = BM / 2 / 8 / WAVES, LB = BN / 2 / 8 / WAVES;   // loads of a wave for a unit
   static_assert(MH * 64 == BM && NH * 64 == BN && LA * 64 == BM && LB * 64 == BN, "whole blocks and whole loads");
-  static constexpr int BEHIND = ST + 1 + (ST + 1) % 2;                     // stages behind the loop, an even number; K has at least as many
+  static constexpr int BEHIND = ST + 1 + (ST + 1) % 2;                     // stages behind the loop, an even number; K has at least as many (ODD: one more)
   static_assert(ST >= 2 && VALUES * 2 <= 160 * 1024 && 2 * ST * (LA + LB) < 64, "stages");
   enum { X_LOW, W_LOW, W_HIGH, X_HIGH };  // the units, in the order in which they are wanted
 
@@ -91,6 +95,7 @@ struct QuarterTile {
     if constexpr (ANY) {
       const bf16_t* from = (of_x(U) ? xp[half][q] : wp[half][q]) + k * QUARTER_K;
       if (k * QUARTER_K + piece() >= K) from = reinterpret_cast<const bf16_t*>(&tile_zeros);
+      // (through the caches: rows of no whole 128 bytes share lines with their neighbours.  64 tokens, 32 experts of 2,056, width 1,448, past them 153 us, so 133)
       __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
     } else if constexpr (of_x(U))
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr[half], to, 16, xo[half][q], k * (QUARTER_K * 2), 0, 0);
@@ -167,6 +172,15 @@ struct QuarterTile {
     if constexpr (LEFT > 0) last_stages<LEFT - 1>(slot, low, high, b1, b0);
   }
 
+  // ``count`` stages, an even number
+  __device__ __forceinline__ void all_but_odd(int count, int& slot, bf16x8* low, bf16x8* high, bf16x8* b0, bf16x8* b1) {
+    for (int s = 0; s + 2 + BEHIND <= count; s += 2) {
+      stage<ST + 1>(slot, low, high, b0, b1);
+      stage<ST + 1>(slot, low, high, b1, b0);
+    }
+    last_stages<BEHIND - 1>(slot, low, high, b0, b1);
+  }
+
   __device__ __forceinline__ void run() {
     bf16x8 low[2 * MH], high[2 * MH], b0[2 * NH], b1[2 * NH];
 #pragma unroll
@@ -184,10 +198,10 @@ struct QuarterTile {
     TILE_BARRIER();
     load_unit<X_LOW>(0, at);
     int slot = 0;
-    for (int s = 0; s + 2 + BEHIND <= stages; s += 2) {
+    if constexpr (INNER == QUARTER_ODD) {
       stage<ST + 1>(slot, low, high, b0, b1);
-      stage<ST + 1>(slot, low, high, b1, b0);
-    }
-    last_stages<BEHIND - 1>(slot, low, high, b0, b1);
+      all_but_odd(stages - 1, slot, low, high, b1, b0);
+    } else
+      all_but_odd(stages, slot, low, high, b0, b1);
   }
 };

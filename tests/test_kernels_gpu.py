@@ -1811,6 +1811,15 @@ def test_experts_without_gates_apply_each_activation(n, width, ff, experts, acti
 
 
 @pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("width,ff", [(320, 576), (704, 320), (448, 2880), (264, 1448), (192, 72)])
+@pytest.mark.parametrize("n", [40, 250, 400])
+def test_experts_of_an_odd_number_of_stages_and_of_no_whole_ones(n, width, ff, gated):
+    """Inner sizes of an odd number of stages of 64 (five at least) and of no whole stages, each in halves and wholes of the smaller tiles and in the larger
+    ones (13, 83 and 133 rows an expert)."""
+    _experts_call(n, width, ff, 3, torch.randint(0, 3, (n, 1), generator=torch.Generator().manual_seed(n)), gated, None if gated else "silu", n)
+
+
+@pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("n,width,ff,experts,top", [(1, 256, 256, 2, 2), (65, 256, 264, 2, 1), (129, 384, 520, 3, 2), (300, 264, 136, 5, 2), (40, 2048, 1024, 16, 2), (64, 1024, 2048, 8, 2)])
 def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, gated):
     """Experts' tiles: halves and whole ones (64 and 65 rows an expert, 128 and 129), inner sizes in whole pairs of stages and not, the

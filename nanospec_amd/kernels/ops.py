@@ -597,31 +597,43 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
     both).  ``may_split``: whoever reads the result can add up ranges of K.
 
     One workgroup a compute unit takes a tile as long whatever the others do, so the smallest tile is taken whose count still fits the units
-    once, and a product is the library's from there on: it has larger tiles, which read less.  Both sides in us, alone and a call beside
-    two others, the library first, weights that no cache holds:
-    K up to 2,048: 160 rows of 2,048 11.9 / 5.6 and (64 x 64) 10.5 / 5.1; 512 13.2 / 8.1 and 11.5 / 8.3; 512 of 3,072 15.8 / 10.4 and (128 x 64) 15.8 / 10.0; 508 of 4,096 18.1 / 13.0
-    and 16.0 / 12.9; 1,024 of 4,096 25.6 / 19.3 and (128 x 128) 22.5 / 18.6; with two copies of x's and w's rows in the caches 2,048 of 4,096 34.5 / 34.2 and (256 x
-    128) 32.8 / 31.8; more than that: 1,024 of 6,144 29.5 / 25.0 and 31.4 / 25.7, 2,048 of 8,192 52.8 / 52.5 and 67.4 / 64.8.
-    A longer K shows the units that have no tile: K 4,096, 256 of 2,048 (128 tiles) 14.8 / 11.2 and 16.0 / 10.7, 1,024 of 3,072 (192) 37.1 / 29.3 and 37.7 / 25.7; K 8,192,
-    768 of 4,096 (192) 63 / 62 and 71 / 64, 1,024 of 4,096 (256) 76 / 77 and 69 / 61.
-    Rows of a tile beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 / 27.2 and 34.0 / 31.9, 512 37.8 / 35.8 and 35.8 / 34.0.
-    Gate and up in one product save a kernel besides: 160 of 16,384 30.0 / 19.5 and 23.5 / 17.8, 512 44.4 / 39.1 and 37.7 / 33.6, 1,024 (two tiles a unit) 70.7 / 64.6 and 67.9 / 65.8.
-    Ranges of K fill the units where the tiles do not, and cost the reader their sums (with the norm that reads them): 512 of 2,048, K 8,192, four 39.1 / 33.8 and
-    31.2 / 22.6; 256 of 4,096, K 14,336, four 67 / 61 and 51 / 40; 800 of 2,048, K 8,192, two 51 / 51 and 42 / 33; 512 of 2,048, K 2,048, two 16.2 / 9.0 and 17.1 / 10.2 (one 14.7 / 8.6)."""
+    once, and a product is the library's from there on: it has larger tiles, which read less.  It is the library's too where too many units
+    have no tile, which shows the more the longer K is, or where too much of the tiles lies beyond the last row or column.  Measured over 129 to
+    2,048 rows and 16 to 28,672 columns, a call behind another, weights that no cache holds: this kernel's time over the library's, median (largest), by the share of the
+    units that have a tile:
+      64 x 64: K 1,024 from an eighth on 0.80 (1.04); 2,048 three eighths 1.02 (1.07), half 0.96 (1.07), all 0.93 (0.98); 4,096 half 1.19 (1.24), five eighths 0.94 (0.99); 6,144 all
+      1.06 (1.08);
+      128 x 64: K 2,048 half 1.05 (1.08), three quarters 0.99 (1.06); 4,096 three quarters 1.06 (1.12), all 0.96 (1.01);
+      128 x 128: K 1,024 half 0.93 (1.05); 2,048 half 1.03 (1.13), five eighths 0.87 (0.95); 4,096 five eighths 1.02 (1.05), three quarters 1.01 (1.14), all 0.96 (1.05);
+      256 x 128: three quarters 0.99 to 1.08 (1.15), all 0.91 to 1.00 (1.15);
+      gate and up with the gate behind them, 128 x 128: K 1,024 an eighth 0.94 (0.97); 2,048 three eighths 1.00 (1.14), half 0.97 (1.06); 4,096 half 1.04 (1.17), five
+      eighths 0.95 (1.00), all 0.87; 6,144 three quarters 1.04 (1.18), all 0.97 (1.00).
+    Rows beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 us in the library and 34.0, 512 37.8 and 35.8; gated, K 6,144, 384 92 and 98.
+    Ranges of K fill the units where the tiles do not, and cost the reader their sums.  The same, with the norm that reads them (and, from K 8,192 on, with a kernel that adds them):
+      four: K 4,096 half 1.04 (1.08), five eighths 0.88; 6,144 three eighths 0.97 (1.00), half 0.88 (0.97); 8,192 three eighths 0.94 and 1.02 (1.09), half 0.85 and 0.90 (1.02);
+      10,240 a quarter 0.99 (1.15) and 1.07 (1.23), three eighths 0.89 and 0.94;
+      two: K 4,096 five eighths 0.94 (0.98), three quarters 0.99 (1.05), all 0.94; 5,120 0.97 (1.05), 1.05 (1.08), 0.91; 8,192 half 1.13 and 1.19 (1.31), five eighths 0.92 and 0.99 (1.03), all
+      0.88 and 0.97."""
     if m < MANY_MIN_ROWS or n % (8 if gated else 4) or k % MANY_K_MULTIPLE or not MANY_K_MIN <= k < MANY_K_MAX:
         return None
     count = [-(-m // bm) * -(-n // bn) for bm, bn in MANY_TILES]
     if may_split and k >= 4096:
         for ranges in (4, 2):
-            if ranges <= many_ranges(m, n, units) and k % (MANY_K_MULTIPLE * ranges) == 0:
+            need = (0.625 if k < 5120 else 0.5 if k <= 8192 else 0.375) if ranges == 4 else (0.875 if k < 6144 else 0.625)
+            if ranges <= many_ranges(m, n, units) and k % (MANY_K_MULTIPLE * ranges) == 0 and ranges * count[MANY_SPLIT_FORM] >= need * units:
                 return MANY_SPLIT_FORM, ranges
     for form, (bm, bn) in enumerate(MANY_TILES):
         if count[form] <= units and not (gated and form < 2):
             filled = count[form] / units  # the share of the units that have a tile
             used = m * n / (count[form] * bm * bn)  # and of the tiles that is not beyond the last row or column
-            if filled < (0.0 if k <= 2048 and form < 3 else 0.625 if k <= 4096 and form == 2 else 0.75 if k <= 4096 and form < 2 else 0.85):
-                return None
-            return (form, 1) if used >= (0.6 if gated or form < 2 else 0.7 if form == 2 else 0.85) else None
+            if form == 3:
+                need = 0.85
+            elif gated:
+                need = 0.0 if k <= 1024 else 0.5 if k <= 2048 else 0.625 if k <= 4608 else 0.875
+            else:
+                need = 0.0 if k <= 1024 else (0.5, 0.75, 0.625)[form] if k <= 2048 else (0.625 if k <= 4608 else 2.0, 0.875, 0.875)[form]
+            whole = 0.85 if form == 3 and (not gated or k > 4608) else 0.7 if form == 2 and not gated else 0.6
+            return (form, 1) if filled >= need and used >= whole else None
     return None
 
 

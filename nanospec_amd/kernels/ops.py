@@ -637,15 +637,17 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
     return None
 
 
-def many_takes(x: torch.Tensor, k: int) -> bool:
-    """Whether ``linear_many`` takes rows like these: bfloat16, whole 16-byte pieces, an inner size in whole pairs of stages."""
-    return (x.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.stride(0) < MANY_K_MAX and x.data_ptr() % 16 == 0)
+def many_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_many`` takes these operands: bfloat16, whole 16-byte pieces, rows of x one behind the other, w in plain rows, an inner size in
+    whole pairs of stages."""
+    k = w.shape[1]
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and k <= x.stride(0) < MANY_K_MAX and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
-def many_writes(out: torch.Tensor) -> bool:
-    """Whether ``linear_many`` can write a result there: whole pieces of four values."""
-    return out.dim() == 2 and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
+def many_writes(out: torch.Tensor, m: int, n: int) -> bool:
+    """Whether ``linear_many`` can write a result of m rows and n columns there: whole pieces of four values."""
+    return out.shape == (m, n) and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
 
 
 def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, w2: torch.Tensor | None = None, act: str | None = None,
@@ -655,7 +657,7 @@ def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, 
     these) ``out`` is float32 scratch of ranges * rows * w.shape[0] and a ``PartialSums`` over it comes back, whose reader rounds once."""
     _gpu(x, w, w2, out)
     m, (n, k) = x.shape[0], w.shape
-    if x.dim() != 2 or x.shape[1] != k or not many_takes(x, k) or w.dtype != x.dtype or not w.is_contiguous():
+    if x.dim() != 2 or x.shape[1] != k or not many_takes(x, w):
         raise KernelRefused(f"linear_many takes bfloat16 x [rows, K] and w [N, K] with K a multiple of {MANY_K_MULTIPLE}; got {tuple(x.shape)}, {tuple(w.shape)}")
     if w2 is not None and (w2.shape != w.shape or w2.dtype != w.dtype or not w2.is_contiguous()):
         raise KernelRefused("linear_many: w2 must match w")

@@ -68,14 +68,14 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
     if gated is not None:
         inter = w_t.shape[1] // 2
         plan = ops.many_plan(m, 2 * inter, k, ops.compute_units(x.device), gated=True)
-        if plan is not None and ops.many_takes(x, k) and ops.many_writes(gated):
+        if plan is not None and ops.many_takes(x, plain) and ops.many_writes(gated, m, inter):
             return ops.linear_many(x, plain[:inter], gated, plan[0], w2=plain[inter:])
         return ops.silu_mul(torch.matmul(x, w_t, out=take((m, 2 * inter), x.dtype)), out=gated)
     if plain is not None:
         n, to = w_t.shape[1], into if into is not None else out
         may_split = take is not None and (split if into is not None else k >= SPLIT_MIN_K)
         plan = ops.many_plan(m, n, k, ops.compute_units(x.device), may_split=may_split)
-        if plan is not None and ops.many_takes(x, k) and (to is None or ops.many_writes(to)):
+        if plan is not None and ops.many_takes(x, plain) and (to is None or ops.many_writes(to, m, n)):
             form, ranges = plan
             if to is None:
                 to = torch.empty((m, n), dtype=x.dtype, device=x.device)
@@ -204,7 +204,7 @@ class LinearWeight:
                     and x.dtype == self.dtype and ops.tiled_takes(x[:1], self.k)):
                 return ops.linear_tiled(x, self.tiled, out=out, act=act)
             if (not out_f32 and self.plain is not None and x.dtype == self.dtype and x.shape[0] >= ops.MANY_MIN_ROWS and self.k <= LIBRARY_MAX_K
-                    and ops.many_takes(x, self.k)):
+                    and ops.many_takes(x, self.plain)):
                 scratch = arena.take if arena is not None else (lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device))
                 return library_product(x, self._plain_t, out=out, plain=self.plain, take=scratch, act=act)
             return ops.activation(self(x, out=out, out_f32=out_f32, arena=arena, plain_copy=plain_copy), act)

@@ -1,6 +1,7 @@
 """How products of few rows are dealt to the compute units (``ops.wide_plan``, ``ops.wide_waves``, ``ops.rows_plan``):
 plain arithmetic on sizes, so it runs without a GPU when the number of compute units is given."""
 import pytest
+import torch
 
 from nanospec_amd.kernels import ops
 
@@ -179,3 +180,39 @@ def test_chunks_of_the_delta_rule_beside_single_tokens():
     assert [least(1, 32, 128, n) for n in (8, 16, 32, 64)] == [64, 96, 96, 192]
     assert [least(1, 16, 64, n) for n in (0, 64, 127, 128)] == [64, 64, 64, 96]
     assert least(4, 16, 64, 64) == 64 and least(8, 16, 64, 0) == 96 and least(16, 16, 64, 0) == 0x7FFFFFFF
+
+
+def _operands(form, device="cpu", m=160, n=256, k=512):
+    """bfloat16 x [m, k] and w [n, k] of small whole numbers, in whole pieces and rows behind one another but for what ``form`` names."""
+    base = torch.arange((n + m) * (k + 16), device=device).remainder(13).sub(6).bfloat16()
+    x, w = base[: m * k].view(m, k), base[m * k : (m + n) * k].view(n, k)
+    return {"whole": (x, w), "x of one row": (x[:1].expand(m, k), w), "x overlapping": (base.as_strided((m, k), (k // 2, 1)), w),
+            "w in wider rows": (x, base.as_strided((n, k), (k + 8, 1))), "w by columns": (x, base[: n * k].view(k, n).t()),
+            "w off its pieces": (x, base[4 : 4 + n * k].view(n, k)), "x off its pieces": (base[4 : 4 + m * k].view(m, k), w)}[form]
+
+
+FORMS = ("x of one row", "x overlapping", "w in wider rows", "w by columns", "w off its pieces", "x off its pieces")
+
+
+def test_what_the_product_of_many_rows_takes():
+    """Rows that overlap or repeat and matrices that do not lie in plain rows of whole pieces are not the own kernel's."""
+    assert ops.many_takes(*_operands("whole"))
+    for form in FORMS:
+        assert not ops.many_takes(*_operands(form)), form
+    out = torch.zeros(160, 264, dtype=torch.bfloat16)
+    assert ops.many_writes(out, 160, 264) and ops.many_writes(out[:, :256], 160, 256)
+    assert not ops.many_writes(out, 160, 256) and not ops.many_writes(out[:, 1:257], 160, 256) and not ops.many_writes(out[:, :256].t(), 256, 160)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("form", ("whole",) + FORMS)
+def test_operands_of_any_layout_have_their_product(form, act):
+    """At a size that the own kernel is chosen for, whichever takes them.  Every sum is a whole number of at most 36 * 512, so the result is rounded once."""
+    from nanospec_amd.parts.linear import LinearWeight
+
+    x, w = _operands(form, "cuda")
+    assert ops.many_plan(*x.shape[:1], *w.shape, UNITS) is not None
+    want = (x.cpu().double() @ w.cpu().double().T).bfloat16().cuda()
+    got = LinearWeight(w, tiled=False)(x, act=act)
+    assert torch.equal(got, want if act is None else ops.activation(want, act))

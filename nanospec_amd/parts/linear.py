@@ -67,15 +67,15 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
         raise ops.KernelRefused(f"a library product over an inner size of {k} (more than {LIBRARY_MAX_K}) must be cut into slices")
     if gated is not None:
         inter = w_t.shape[1] // 2
-        plan = ops.many_plan(m, 2 * inter, k, ops.compute_units(x.device), gated=True)
-        if plan is not None and ops.many_takes(x, plain) and ops.many_writes(gated, m, inter):
+        plan = ops.many_plan(m, 2 * inter, k, ops.compute_units(x.device), gated=True) if ops.many_takes(x, plain) else None
+        if plan is not None and ops.many_writes(gated, m, inter):
             return ops.linear_many(x, plain[:inter], gated, plan[0], w2=plain[inter:])
         return ops.silu_mul(torch.matmul(x, w_t, out=take((m, 2 * inter), x.dtype)), out=gated)
     if plain is not None:
         n, to = w_t.shape[1], into if into is not None else out
         may_split = take is not None and (split if into is not None else k >= SPLIT_MIN_K)
-        plan = ops.many_plan(m, n, k, ops.compute_units(x.device), may_split=may_split)
-        if plan is not None and ops.many_takes(x, plain) and (to is None or ops.many_writes(to, m, n)):
+        plan = ops.many_plan(m, n, k, ops.compute_units(x.device), may_split=may_split) if ops.many_takes(x, plain) else None
+        if plan is not None and (to is None or ops.many_writes(to, m, n)):
             form, ranges = plan
             if to is None:
                 to = torch.empty((m, n), dtype=x.dtype, device=x.device)

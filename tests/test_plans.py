@@ -196,9 +196,13 @@ FORMS = ("x of one row", "x overlapping", "w in wider rows", "w by columns", "w 
 
 def test_what_the_product_of_many_rows_takes():
     """Rows that overlap or repeat and matrices that do not lie in plain rows of whole pieces are not the own kernel's."""
-    assert ops.many_takes(*_operands("whole"))
-    for form in FORMS:
-        assert not ops.many_takes(*_operands(form)), form
+    from unittest import mock
+
+    with mock.patch.object(torch.Tensor, "is_cuda", True):
+        assert ops.many_takes(*_operands("whole"))
+        for form in FORMS:
+            assert not ops.many_takes(*_operands(form)), form
+    assert not ops.many_takes(*_operands("whole"))
     out = torch.zeros(160, 264, dtype=torch.bfloat16)
     assert ops.many_writes(out, 160, 264) and ops.many_writes(out[:, :256], 160, 256)
     assert not ops.many_writes(out, 160, 256) and not ops.many_writes(out[:, 1:257], 160, 256) and not ops.many_writes(out[:, :256].t(), 256, 160)
@@ -216,3 +220,11 @@ def test_operands_of_any_layout_have_their_product(form, act):
     want = (x.cpu().double() @ w.cpu().double().T).bfloat16().cuda()
     got = LinearWeight(w, tiled=False)(x, act=act)
     assert torch.equal(got, want if act is None else ops.activation(want, act))
+
+
+def test_a_product_of_many_rows_on_the_cpu():
+    """A matrix kept in plain rows alone needs none of the kernels: its product is the library's wherever it lies."""
+    from nanospec_amd.parts.linear import LinearWeight
+
+    x, w = _operands("whole")
+    assert torch.equal(LinearWeight(w, tiled=False)(x), (x.double() @ w.double().T).bfloat16())

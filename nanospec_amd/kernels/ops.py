@@ -639,9 +639,9 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
 
 def many_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``linear_many`` takes these operands: bfloat16 on the GPU, whole 16-byte pieces, rows of x one behind the other, w in plain rows, an inner
-    size in whole pairs of stages."""
+    size in whole pairs of stages, and no gradient asked for."""
     k = w.shape[1]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1
+    return (x.is_cuda and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1
             and x.stride(0) % 8 == 0 and k <= x.stride(0) < MANY_K_MAX and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 

@@ -228,3 +228,18 @@ def test_a_product_of_many_rows_on_the_cpu():
 
     x, w = _operands("whole")
     assert torch.equal(LinearWeight(w, tiled=False)(x), (x.double() @ w.double().T).bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("of", ["x", "w"])
+def test_a_product_of_many_rows_has_its_gradient(of):
+    """Whole numbers: the gradients of the results' sum are column sums, exact in 32-bit and rounded once (by at most half a step, 2^-9)."""
+    from nanospec_amd.parts.linear import LinearWeight
+
+    x, w = (t.clone() for t in _operands("whole", "cuda"))
+    (x if of == "x" else w).requires_grad_()
+    LinearWeight(w, tiled=False)(x).sum().backward()
+    got, want = (x.grad, w.detach().double().sum(0).expand_as(x)) if of == "x" else (w.grad, x.detach().double().sum(0).expand_as(w))
+    torch.testing.assert_close(got.double(), want, rtol=2**-8, atol=0)
+    with torch.no_grad():
+        assert ops.many_takes(x, w)

@@ -94,27 +94,39 @@ __global__ __launch_bounds__(T::WAVES * NS_WAVE) __attribute__((amdgpu_waves_per
   }
 }
 
-template <class T>
-static int launch_many(ManyParams p, int epi, hipStream_t stream) {
-  const int ch = epi == MANY_GATED ? T::BN / 2 : T::BN;
-  p.m_tiles = (p.M + T::BM - 1) / T::BM, p.n_tiles = (p.N + ch - 1) / ch;
-  if (p.K / p.ranges < T::BEHIND * QUARTER_K) return NS_ERR_UNSUPPORTED;
-  const long long items = (long long)p.m_tiles * p.n_tiles * p.ranges;
-  if (items > (1 << 22)) return NS_ERR_UNSUPPORTED;
-  const unsigned blocks = (unsigned)((items + 7) / 8 * 8);
-  switch (epi) {
-    case MANY_PLAIN: gemm_many_kernel<T, MANY_PLAIN><<<blocks, T::WAVES * NS_WAVE, 0, stream>>>(p); break;
-    case MANY_ACT: gemm_many_kernel<T, MANY_ACT><<<blocks, T::WAVES * NS_WAVE, 0, stream>>>(p); break;
-    case MANY_GATED: gemm_many_kernel<T, MANY_GATED><<<blocks, T::WAVES * NS_WAVE, 0, stream>>>(p); break;
-    case MANY_ADD: gemm_many_kernel<T, MANY_ADD><<<blocks, T::WAVES * NS_WAVE, 0, stream>>>(p); break;
-    default: gemm_many_kernel<T, MANY_RANGES><<<blocks, T::WAVES * NS_WAVE, 0, stream>>>(p);
+// What may follow a product in tiles of T, other pairs are not built: the gate stands behind tiles of 128 columns (half as many channels), ranges of K behind the tile
+// that they are for, an activation behind all but the largest tile, whose end costs more than a kernel of its own.
+template <class T, int EPI>
+static int launch_many(ManyParams p, hipStream_t stream) {
+  constexpr bool LARGEST = T::BM == 256, SMALL = T::BN == 64;
+  if constexpr ((EPI == MANY_GATED && SMALL) || (EPI == MANY_RANGES && (SMALL || LARGEST)) || (EPI == MANY_ACT && LARGEST))
+    return NS_ERR_UNSUPPORTED;
+  else {
+    const int ch = EPI == MANY_GATED ? T::BN / 2 : T::BN;
+    p.m_tiles = (p.M + T::BM - 1) / T::BM, p.n_tiles = (p.N + ch - 1) / ch;
+    if (p.K / p.ranges < T::BEHIND * QUARTER_K) return NS_ERR_UNSUPPORTED;
+    const long long items = (long long)p.m_tiles * p.n_tiles * p.ranges;
+    if (items > (1 << 22)) return NS_ERR_UNSUPPORTED;
+    gemm_many_kernel<T, EPI><<<(unsigned)((items + 7) / 8 * 8), T::WAVES * NS_WAVE, 0, stream>>>(p);
+    return ns_launch_status();
   }
-  return ns_launch_status();
+}
+
+template <class T>
+static int launch_many(const ManyParams& p, int epi, hipStream_t stream) {
+  switch (epi) {
+    case MANY_PLAIN: return launch_many<T, MANY_PLAIN>(p, stream);
+    case MANY_ACT: return launch_many<T, MANY_ACT>(p, stream);
+    case MANY_GATED: return launch_many<T, MANY_GATED>(p, stream);
+    case MANY_ADD: return launch_many<T, MANY_ADD>(p, stream);
+    default: return launch_many<T, MANY_RANGES>(p, stream);
+  }
 }
 
 // ``form``: the tile, rows of x by rows of w: 0 64 x 64, 1 128 x 64, 2 128 x 128, 3 256 x 128.
 // ``epi``: 0 out = x w^T; 1 an activation of it (``act`` as common.h numbers them); 2 silu(x w^T) * (x w2^T); 3 out += x w^T (summed in 32-bit,
 // rounded once); 4 out: float32 [ranges][M][N], the sums over each of ``ranges`` equal ranges of K (one range in the other four).
+// Not every tile with every ``epi``: 1 with forms 0 to 2, 2 with 2 and 3, 4 with 2 (NS_ERR_UNSUPPORTED otherwise).
 // K: a multiple of 128 a range and at least 256 (form 0: 384); x_stride a multiple of 8, N and out_stride of 4; x, w, w2 on 16 bytes, out on 8 (on 16 with ranges).
 extern "C" int ns_gemm_many_bf16(void* out, const void* x, const void* w, const void* w2, int M, int N, int K, int x_stride, int out_stride, int epi,
                                  int act, int ranges, int form, hipStream_t stream) {

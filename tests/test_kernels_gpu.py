@@ -186,7 +186,7 @@ def test_linear_wide(m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 4, 384), (129, 68, 384), (257, 132, 512), (300, 640, 2048), (1100, 260, 640)])
 def test_linear_many(form, m, n, k):
     """Products of many rows from plain matrices: every tile at sizes off its edges (and more tiles than an XCD's patch), the shortest
-    inner sizes, strided rows and results, everything that may follow the product, ranges of K."""
+    inner sizes, strided rows and results, everything that may follow the product in that tile, and the others refused; an activation has the values that its own kernel has."""
     ops = _ops()
     torch.manual_seed(m + n + k)
     x = torch.randn(m + 3, k + 8, dtype=torch.bfloat16, device=DEV)[:m, :k]
@@ -199,17 +199,29 @@ def test_linear_many(form, m, n, k):
     assert bool((wide[m] == 7).all()) and bool((wide[:, n:] == 7).all())
     plain = out.clone()
     for act in ops.ACTIVATIONS:
-        torch.testing.assert_close(ops.linear_many(x, w, out, form, act=act), ops.activation(plain.clone(), act), rtol=2**-7, atol=0)
+        if form < 3:
+            assert torch.equal(ops.linear_many(x, w, out, form, act=act), ops.activation(plain.clone(), act)), act
+        else:
+            with pytest.raises(ops.KernelRefused):
+                ops.linear_many(x, w, out, form, act=act)
     resid = torch.randn(m, n, dtype=torch.bfloat16, device=DEV) * 30
     out.copy_(resid)
     assert ulps_of_row_max(ops.linear_many(x, w, out, form, add=True).cpu(), resid.cpu().float() + ref).max() <= 1.0
-    if n % 8 == 0 or form < 2:
+    if form >= 2:
         assert ulps_of_row_max(ops.linear_many(x, w, out, form, w2=w2).cpu(), ref * torch.sigmoid(ref) * u).max() <= 1.5
+    else:
+        with pytest.raises(ops.KernelRefused):
+            ops.linear_many(x, w, out, form, w2=w2)
     weight = (1 + 0.1 * torch.randn(n, device=DEV)).bfloat16()
     for ranges in (2, 4):
-        if k % (128 * ranges) or k // ranges < (384 if form == 0 else 256):
+        if k % (128 * ranges) or k // ranges < 256:
             continue
-        parts = ops.linear_many(x, w, torch.empty(ranges * m * n, device=DEV), form, ranges=ranges)
+        scratch = torch.empty(ranges * m * n, device=DEV)
+        if form != 2:
+            with pytest.raises(ops.KernelRefused):
+                ops.linear_many(x, w, scratch, form, ranges=ranges)
+            continue
+        parts = ops.linear_many(x, w, scratch, form, ranges=ranges)
         torch.testing.assert_close(parts.ws.view(ranges, m, n).double().sum(0).cpu(), x.cpu().double() @ w.cpu().double().T, rtol=1e-5, atol=1e-5 * math.sqrt(k))
         assert ulps_of_row_max(ops.reduce_partial(parts).cpu(), ref).max() <= 1.0
         # the norm that reads them: the stream and the ranges are added in 32-bit and rounded once

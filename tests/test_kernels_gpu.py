@@ -1324,9 +1324,9 @@ def test_moe_choice_among_a_wave_of_experts_and_more(experts, groups, keep, best
         torch.testing.assert_close(wt[t].cpu(), s[t, want], rtol=1e-6, atol=0)
 
 
-@pytest.mark.parametrize("n,experts,ff", [(24, 8, 264), (200, 8, 264), (700, 4, 136)])
+@pytest.mark.parametrize("n,experts,ff", [(24, 8, 264), (200, 8, 264), (700, 4, 136), (700, 4, 384)])
 def test_moe_results_at_any_address(n, experts, ff):
-    """A result that begins a float behind a 16-byte boundary: streamed, in the smaller tiles and in the larger ones."""
+    """A result that begins a float behind a 16-byte boundary: streamed, in the smaller tiles (700 rows of 136 channels, no whole stages, among them) and in the larger ones."""
     ops = _ops()
     g = torch.Generator(device=DEV).manual_seed(n)
     rnd = lambda *shape: torch.randn(*shape, generator=g, device=DEV).bfloat16()
@@ -1749,31 +1749,25 @@ def _turned(x, pos, inv, interleaved):
 @pytest.mark.parametrize("experts,extra,top,groups,keep,width", [(32, 0, 4, 1, 1, 2048), (32, 0, 4, 8, 4, 2048), (31, 1, 3, 1, 1, 260), (8, 0, 8, 2, 2, 8192), (5, 0, 1, 1, 1, 4), (28, 4, 4, 4, 2, 1032)])
 def test_moe_route_of_few_tokens_in_one_launch(dtype, experts, extra, top, groups, keep, width):
     """A small router's logits and choice for up to 8 tokens are one kernel, a workgroup a token: the same bits as in two launches
-    (which a row at an odd stride still takes), however many tokens the step holds."""
+    (which a router of 33 rows takes, here the same one with rows that belong to no expert below it), however many tokens the step holds."""
     ops = _ops()
     torch.manual_seed(experts + width)
     h = torch.randn(8, width, device=DEV).to(dtype)
-    odd = torch.empty(8, width + 1, dtype=dtype, device=DEV)[:, :width].copy_(h)
-    router = torch.randn(experts + extra, width, device=DEV) * 0.1
-    bias = torch.randn(experts + extra, device=DEV) if not extra else None
+    router = torch.randn(33, width, device=DEV) * 0.1
+    bias = torch.randn(33, device=DEV) if not extra else None
 
-    def route(x, n):
+    def route(n, rows=experts + extra):
         sel, wt = torch.full((n, top), -1, dtype=torch.int32, device=DEV), torch.zeros(n, top, device=DEV)
-        z = torch.zeros(n, experts + extra, device=DEV)
-        ops.moe_route(x[:n], router, bias, top, sel, wt, logits=z, groups=groups, keep=keep, extra=extra)
-        return sel, wt, z
+        z = torch.zeros(n, rows, device=DEV)
+        ops.moe_route(h[:n], router[:rows], None if bias is None else bias[:rows], top, sel, wt, logits=z, groups=groups, keep=keep, extra=rows - experts)
+        return sel, wt, z[:, : experts + extra]
 
-    got = route(h, 8)
-    want = h.double() @ router.double().T + (0 if bias is None else bias.double())
+    got = route(8)
+    want = h.double() @ router[: experts + extra].double().T + (0 if bias is None else bias[: experts + extra].double())
     torch.testing.assert_close(got[2].double(), want, rtol=1e-5, atol=1e-5 * math.sqrt(width))
     for n in (1, 3, 8):
-        for a, b in zip(route(h, n), got):
-            assert torch.equal(a, b[:n])
-    two = route(odd, 8)
-    torch.testing.assert_close(two[2], got[2], rtol=1e-5, atol=1e-5 * math.sqrt(width))
-    clear = (two[0] == got[0]).all(1)  # (a row without pieces of 16 bytes is added up in another order: a tie may fall the other way)
-    assert int(clear.sum()) >= 7
-    torch.testing.assert_close(two[1][clear], got[1][clear], rtol=1e-4, atol=1e-6)
+        for a, b, c in zip(route(n), got, route(n, 33)):
+            assert torch.equal(a, b[:n]) and torch.equal(a, c)
 
 
 def _check_experts(out, h, gate, up, down, sel, wt, limit, alpha, shift, activation):
@@ -1832,10 +1826,19 @@ def test_experts_of_an_odd_number_of_stages_and_of_no_whole_ones(n, width, ff, g
 
 
 @pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("width,ff", [(384, 640), (256, 328), (512, 256)])
+@pytest.mark.parametrize("rows", [(64, 65, 128, 129, 300, 0), (64, 65, 128, 129, 300, 0, 0, 0), (1, 0, 126, 257)], ids=["larger", "smaller", "few"])
+def test_experts_of_so_many_rows(rows, width, ff, gated):
+    """Exactly so many rows an expert: a half tile and a row more, a whole one and a row more, several tiles.  114 an expert on average take the larger tiles, 86 and 96 the
+    smaller ones, inner sizes in whole pairs of stages (but for down's with 328 channels), blocks of channels whole and cut."""
+    sel = torch.cat([torch.full((r,), e) for e, r in enumerate(rows)])[torch.randperm(sum(rows), generator=torch.Generator().manual_seed(ff))]
+    _experts_call(sum(rows), width, ff, len(rows), sel[:, None], gated, None if gated else "silu", ff)
+
+
+@pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("n,width,ff,experts,top", [(1, 256, 256, 2, 2), (65, 256, 264, 2, 1), (129, 384, 520, 3, 2), (300, 264, 136, 5, 2), (40, 2048, 1024, 16, 2), (64, 1024, 2048, 8, 2)])
 def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, gated):
-    """Experts' tiles: halves and whole ones (64 and 65 rows an expert, 128 and 129), inner sizes in whole pairs of stages and not, the
-    smaller and the larger tiles, an expert without rows."""
+    """Experts' tiles, streamed and smaller, at inner sizes in whole pairs of stages and not, with several experts a token, an expert without rows."""
     ops = _ops()
     torch.manual_seed(n + ff)
     h = torch.randn(n, width, dtype=torch.bfloat16, device=DEV)

@@ -598,16 +598,19 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
 
     One workgroup a compute unit takes a tile as long whatever the others do, so the smallest tile is taken whose count still fits the units
     once, and a product is the library's from there on: it has larger tiles, which read less.  It is the library's too where too many units
-    have no tile, which shows the more the longer K is, or where too much of the tiles lies beyond the last row or column.  Measured over 129 to
-    2,048 rows and 16 to 28,672 columns, a call behind another, weights that no cache holds: this kernel's time over the library's, median (largest), by the share of the
-    units that have a tile:
-      64 x 64: K 1,024 from an eighth on 0.80 (1.04); 2,048 three eighths 1.02 (1.07), half 0.96 (1.07), all 0.93 (0.98); 4,096 half 1.19 (1.24), five eighths 0.94 (0.99); 6,144 all
-      1.06 (1.08);
-      128 x 64: K 2,048 half 1.05 (1.08), three quarters 0.99 (1.06); 4,096 three quarters 1.06 (1.12), all 0.96 (1.01);
-      128 x 128: K 1,024 half 0.93 (1.05); 2,048 half 1.03 (1.13), five eighths 0.87 (0.95); 4,096 five eighths 1.02 (1.05), three quarters 1.01 (1.14), all 0.96 (1.05);
-      256 x 128: three quarters 0.99 to 1.08 (1.15), all 0.91 to 1.00 (1.15);
-      gate and up with the gate behind them, 128 x 128: K 1,024 an eighth 0.94 (0.97); 2,048 three eighths 1.00 (1.14), half 0.97 (1.06); 4,096 half 1.04 (1.17), five
-      eighths 0.95 (1.00), all 0.87; 6,144 three quarters 1.04 (1.18), all 0.97 (1.00).
+    have no tile, which shows the more the longer K is, or where too much of the tiles lies beyond the last row or column.  This kernel's time over the library's, weights that
+    no cache holds, 129 to 2,048 rows, by the share of the units that have a tile: a call behind another, median (largest) / beside two others of its kind, where what one leaves idle the others use:
+      64 x 64: K to 2,048 a quarter 1.11 (1.14) / 1.05 (1.09), three eighths 1.06 (1.11) / 1.00 (1.12), half 0.96 (1.08) / 0.96 (1.05); to 4,608 half 1.00 (1.27) / 0.91 (0.98), five
+      eighths 0.96 (1.03) / 0.92 (1.00);
+      128 x 64: K to 2,048 half 0.96 (1.04) / 0.98 (1.01); to 4,608 five eighths 1.05 (1.14) / 1.02 (1.05), three quarters 1.00 (1.07) / 0.95 (1.04);
+      128 x 128: K to 2,048 half 0.87 (1.12) / 0.86 (1.01); to 4,096 half 0.96 (1.15) / 0.83 (0.99), five eighths 1.03 (1.19) / 0.87 (0.92), three quarters 0.89 (1.07) / 0.86 (0.93); 4,608 five eighths
+      1.02 (1.21) / 0.90 (0.99), three quarters 0.92 (1.02) / 0.88 (0.94);
+      gate and up with the gate behind them, 128 x 128: K to 2,048 a quarter 0.88 (1.01) / 0.90 (0.94); to 4,608 three eighths 1.14 (1.25) / 0.86 (0.96), half 0.96 (1.04) / 0.80 (0.93), five
+      eighths 0.88 (0.96) / 0.80 (0.87).
+    A call behind another alone: 64 x 64, K 1,024 from an eighth on 0.80 (1.04), 6,144 all 1.06 (1.08); 256 x 128 three quarters 0.99 to 1.08 (1.15), all 0.91 to 1.00 (1.15); gated, K 6,144 three quarters
+    1.04 (1.18), all 0.97 (1.00).  Where both are level this kernel is taken: its launch costs the host 11 us, the library's 20, and steps of many tokens that run kernel by kernel
+    are bound by that (three prompts of 1,531 tokens of the 4-layer design with memory, four products each of 256 columns, K 2,048, three eighths, and of 2,048, K 4,096, three quarters: the step's
+    1,960 us are 2,030 with both in the library).
     Rows beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 us in the library and 34.0, 512 37.8 and 35.8; gated, K 6,144, 384 92 and 98.
     Ranges of K fill the units where the tiles do not, and cost the reader their sums.  The same, with the norm that reads them (and, from K 8,192 on, with a kernel that adds them):
       four: K 4,096 half 1.04 (1.08), five eighths 0.88; 6,144 three eighths 0.97 (1.00), half 0.88 (0.97); 8,192 three eighths 0.94 and 1.02 (1.09), half 0.85 and 0.90 (1.02);
@@ -629,9 +632,9 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
             if form == 3:
                 need = 0.85
             elif gated:
-                need = 0.0 if k <= 1024 else 0.5 if k <= 2048 else 0.625 if k <= 4608 else 0.875
+                need = 0.0 if k <= 1024 else 0.25 if k <= 2048 else 0.625 if k <= 4608 else 0.875
             else:
-                need = 0.0 if k <= 1024 else (0.5, 0.75, 0.625)[form] if k <= 2048 else (0.625 if k <= 4608 else 2.0, 0.875, 0.875)[form]
+                need = 0.0 if k <= 1024 else (0.375, 0.5, 0.5)[form] if k <= 2048 else (0.625, 0.75, 0.625 if k <= 4096 else 0.75)[form] if k <= 4608 else (2.0, 0.875, 0.875)[form]
             whole = 0.85 if form == 3 and (not gated or k > 4608) else 0.7 if form == 2 and not gated else 0.6
             return (form, 1) if filled >= need and used >= whole else None
     return None

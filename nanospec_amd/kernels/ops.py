@@ -643,9 +643,10 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
 def many_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``linear_many`` takes these operands: bfloat16 on the GPU, whole 16-byte pieces, rows of x one behind the other, w in plain rows, an inner
     size in whole pairs of stages, and no gradient asked for."""
-    k = w.shape[1]
-    return (x.is_cuda and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % MANY_K_MULTIPLE == 0 and 0 < k < MANY_K_MAX and x.stride(1) == 1
-            and x.stride(0) % 8 == 0 and k <= x.stride(0) < MANY_K_MAX and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+    k, row = w.shape[1], x.stride(0)
+    return (k % MANY_K_MULTIPLE == 0 and row % 8 == 0 and 0 < k <= row < MANY_K_MAX and x.stride(1) == 1 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.is_cuda and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous()
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
 def many_writes(out: torch.Tensor, m: int, n: int) -> bool:
@@ -660,7 +661,8 @@ def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, 
     these) ``out`` is float32 scratch of ranges * rows * w.shape[0] and a ``PartialSums`` over it comes back, whose reader rounds once."""
     _gpu(x, w, w2, out)
     m, (n, k) = x.shape[0], w.shape
-    if x.dim() != 2 or x.shape[1] != k or not many_takes(x, w):
+    # (what else ``many_takes`` asks of addresses, strides and K the launch checks itself)
+    if x.dim() != 2 or x.shape[1] != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.stride(1) != 1 or not w.is_contiguous():
         raise KernelRefused(f"linear_many takes bfloat16 x [rows, K] and w [N, K] with K a multiple of {MANY_K_MULTIPLE}; got {tuple(x.shape)}, {tuple(w.shape)}")
     if w2 is not None and (w2.shape != w.shape or w2.dtype != w.dtype or not w2.is_contiguous()):
         raise KernelRefused("linear_many: w2 must match w")

@@ -985,15 +985,30 @@ __global__ void clipped_glu_kernel(T* __restrict__ out, const T* __restrict__ gu
   }
 }
 
-// The same in pieces of 16 bytes, a workgroup 256 of them of a row (nothing is divided).  Bound by the bytes: 2,048 rows of 4,096, bfloat16, 19.4 -> 9.8 us.
+// A workgroup of 256 for rows of so many pieces of 16 bytes: x along a row, y rows.  As many along a row as leave the fewest beyond its end, half a KiB of it at least where
+// it has that: with 256 along every row most of the threads of a narrow one have nothing to do (65,536 rows of 64 bfloat16 values, sum of two
+// and clipped gate: 256 along 29.9 and 30.8 us, value by value 6.2 and 10.1, as it is 3.5 and 5.9; 2,048 of 2,560 6.4 and 9.6, 8.7 and 12.7, 4.2 and 7.2).
+static dim3 piece_block(int pieces) {
+  const auto padded = [pieces](int x) { return (pieces + x - 1) / x * x; };
+  int x = 256;
+  while (x > 32 && padded(x / 2) < padded(x)) x /= 2;
+  while (x >= 2 * pieces) x /= 2;
+  return dim3(x, 256 / x);
+}
+static dim3 piece_grid(int pieces, int rows, dim3 block) {
+  const unsigned y = (rows + block.y - 1) / block.y;
+  return dim3((pieces + block.x - 1) / block.x, y < 65535 ? y : 65535);
+}
+
+// The same in pieces of 16 bytes (nothing is divided).  Bound by the bytes: 2,048 rows of 4,096, bfloat16, 19.4 -> 9.8 us.
 template <typename T>
 __global__ __launch_bounds__(256) void clipped_glu_vec_kernel(T* __restrict__ out, const T* __restrict__ gu, int gu_stride, int n, int ff, float limit, float alpha,
                                                              float shift) {
   constexpr int V = 16 / sizeof(T);
   typedef T vec_t __attribute__((ext_vector_type(V)));
-  const int f = (blockIdx.x * 256 + threadIdx.x) * V;
+  const int f = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (f >= ff) return;
-  for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) {
+  for (size_t t = blockIdx.y * blockDim.y + threadIdx.y; t < (size_t)n; t += gridDim.y * blockDim.y) {
     const vec_t g = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + f), u = *reinterpret_cast<const vec_t*>(gu + t * gu_stride + ff + f);
     vec_t o;
 #pragma unroll
@@ -1006,11 +1021,11 @@ extern "C" int ns_clipped_glu(void* out, const void* gu, int gu_stride, int n, i
   if (n <= 0 || ff <= 0) return NS_ERR_BAD_ARG;
   const int v = dtype == NS_DTYPE_F32 ? 4 : 8;
   if ((dtype == NS_DTYPE_F32 || dtype == NS_DTYPE_BF16) && ff % v == 0 && gu_stride % v == 0 && !(((uintptr_t)out | (uintptr_t)gu) & 15)) {
-    const dim3 grid((ff / v + 255) / 256, n < 65535 ? n : 65535);
+    const dim3 block = piece_block(ff / v), grid = piece_grid(ff / v, n, block);
     if (dtype == NS_DTYPE_F32)
-      clipped_glu_vec_kernel<float><<<grid, 256, 0, stream>>>((float*)out, (const float*)gu, gu_stride, n, ff, limit, alpha, shift);
+      clipped_glu_vec_kernel<float><<<grid, block, 0, stream>>>((float*)out, (const float*)gu, gu_stride, n, ff, limit, alpha, shift);
     else
-      clipped_glu_vec_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)gu, gu_stride, n, ff, limit, alpha, shift);
+      clipped_glu_vec_kernel<bf16_t><<<grid, block, 0, stream>>>((bf16_t*)out, (const bf16_t*)gu, gu_stride, n, ff, limit, alpha, shift);
     return ns_launch_status();
   }
   const size_t count = (size_t)n * ff;
@@ -1122,18 +1137,18 @@ __global__ void scaled_sum_kernel(T* __restrict__ out, const T* __restrict__ a, 
   }
 }
 
-// The same in pieces of 16 bytes, a workgroup 256 of them of a row (nothing is divided).  Bound by the bytes: 1,531 rows of 2,048, bfloat16, 5.4 -> 3.5 us, 2,048 of 4,096 15.8 -> 9.0.
+// The same in pieces of 16 bytes (nothing is divided).  Bound by the bytes: 1,531 rows of 2,048, bfloat16, 5.4 -> 3.5 us, 2,048 of 4,096 15.8 -> 9.0.
 template <typename T>
 __global__ __launch_bounds__(256) void scaled_sum_vec_kernel(T* __restrict__ out, const T* __restrict__ a, const T* __restrict__ b, const T* __restrict__ bias,
                                                             const T* __restrict__ bias_b, float sa, float sb, int n, int W) {
   constexpr int V = 16 / sizeof(T);
   typedef T vec_t __attribute__((ext_vector_type(V)));
-  const int c = (blockIdx.x * 256 + threadIdx.x) * V;
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (c >= W) return;
   vec_t ba = {}, bb = {};
   if (bias) ba = *reinterpret_cast<const vec_t*>(bias + c);
   if (bias_b) bb = *reinterpret_cast<const vec_t*>(bias_b + c);
-  for (size_t t = blockIdx.y; t < (size_t)n; t += gridDim.y) {
+  for (size_t t = blockIdx.y * blockDim.y + threadIdx.y; t < (size_t)n; t += gridDim.y * blockDim.y) {
     const vec_t av = *reinterpret_cast<const vec_t*>(a + t * W + c), bv = *reinterpret_cast<const vec_t*>(b + t * W + c);
     vec_t o;
 #pragma unroll
@@ -1148,11 +1163,11 @@ extern "C" int ns_scaled_sum(void* out, const void* a, const void* b, const void
   const int v = dtype == NS_DTYPE_F32 ? 4 : 8;
   if ((dtype == NS_DTYPE_F32 || dtype == NS_DTYPE_BF16) && W % v == 0 &&
       !(((uintptr_t)out | (uintptr_t)a | (uintptr_t)b | (uintptr_t)bias | (uintptr_t)bias_b) & 15)) {
-    const dim3 grid((W / v + 255) / 256, n < 65535 ? n : 65535);
+    const dim3 block = piece_block(W / v), grid = piece_grid(W / v, n, block);
     if (dtype == NS_DTYPE_F32)
-      scaled_sum_vec_kernel<float><<<grid, 256, 0, stream>>>((float*)out, (const float*)a, (const float*)b, (const float*)bias, (const float*)bias_b, sa, sb, n, W);
+      scaled_sum_vec_kernel<float><<<grid, block, 0, stream>>>((float*)out, (const float*)a, (const float*)b, (const float*)bias, (const float*)bias_b, sa, sb, n, W);
     else
-      scaled_sum_vec_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)bias, (const bf16_t*)bias_b, sa, sb, n, W);
+      scaled_sum_vec_kernel<bf16_t><<<grid, block, 0, stream>>>((bf16_t*)out, (const bf16_t*)a, (const bf16_t*)b, (const bf16_t*)bias, (const bf16_t*)bias_b, sa, sb, n, W);
     return ns_launch_status();
   }
   const size_t count = (size_t)n * W;

@@ -1870,7 +1870,7 @@ def test_expert_groups_at_the_edges_of_their_tiles(n, width, ff, experts, top, g
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n,width", [(1, 8), (3, 2056), (70, 4096), (5, 36), (4, 77)])
+@pytest.mark.parametrize("n,width", [(1, 8), (3, 2056), (70, 4096), (5, 36), (4, 77), (1000, 8), (300, 64), (70, 2560), (66000, 72)])
 def test_scaled_sum_and_clipped_glu_in_pieces_and_alone(dtype, n, width):
     """Rows in whole pieces of 16 bytes and rows that are not, results at the edges of a workgroup, what is no number where it was in a sum."""
     ops = _ops()

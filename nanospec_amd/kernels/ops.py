@@ -607,35 +607,37 @@ def many_plan(m: int, n: int, k: int, units: int, gated: bool = False, may_split
       1.02 (1.21) / 0.90 (0.99), three quarters 0.92 (1.02) / 0.88 (0.94);
       gate and up with the gate behind them, 128 x 128: K to 2,048 a quarter 0.88 (1.01) / 0.90 (0.94); to 4,608 three eighths 1.14 (1.25) / 0.86 (0.96), half 0.96 (1.04) / 0.80 (0.93), five
       eighths 0.88 (0.96) / 0.80 (0.87).
-    A call behind another alone: 64 x 64, K 1,024 from an eighth on 0.80 (1.04), 6,144 all 1.06 (1.08); 256 x 128 three quarters 0.99 to 1.08 (1.15), all 0.91 to 1.00 (1.15); gated, K 6,144 three quarters
-    1.04 (1.18), all 0.97 (1.00).  Where both are level this kernel is taken: its launch costs the host 11 us, the library's 20, and steps of many tokens that run kernel by kernel
+      K of 5,120 to 14,336: 64 x 64 half 1.01 (1.22) / 0.95 (1.12), seven eighths 1.02 (1.12) / 0.93 (1.11); 128 x 64 three quarters 1.01 (1.09) / 1.03 (1.25), seven eighths 0.97 (1.04) / 0.99 (1.17); 128 x 128 three
+      quarters 1.03 (1.09) / 0.95 (1.17), seven eighths 0.92 (1.05) / 0.89 (1.05); gated half 1.02 (1.09) / 0.85 (0.99), five eighths 0.93 (1.22) / 0.94 (1.16), seven eighths 0.87 (0.99) / 0.89 (1.23);
+      256 x 128: half 1.14 (1.22) / 0.81 (1.16), three quarters 0.91 (1.15) / 0.96 (1.23), seven eighths 0.89 (0.99) / 0.96 (1.05).
+    K of 1,024 alone: 64 x 64 from an eighth on 0.80 (1.04).  Where both are level this kernel is taken: its launch costs the host 11 us, the library's 20, and steps of many tokens that run kernel by kernel
     are bound by that (three prompts of 1,531 tokens of the 4-layer design with memory, four products each of 256 columns, K 2,048, three eighths, and of 2,048, K 4,096, three quarters: the step's
     1,960 us are 2,030 with both in the library).
-    Rows beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 us in the library and 34.0, 512 37.8 and 35.8; gated, K 6,144, 384 92 and 98.
-    Ranges of K fill the units where the tiles do not, and cost the reader their sums.  The same, with the norm that reads them (and, from K 8,192 on, with a kernel that adds them):
-      four: K 4,096 half 1.04 (1.08), five eighths 0.88; 6,144 three eighths 0.97 (1.00), half 0.88 (0.97); 8,192 three eighths 0.94 and 1.02 (1.09), half 0.85 and 0.90 (1.02);
-      10,240 a quarter 0.99 (1.15) and 1.07 (1.23), three eighths 0.89 and 0.94;
-      two: K 4,096 five eighths 0.94 (0.98), three quarters 0.99 (1.05), all 0.94; 5,120 0.97 (1.05), 1.05 (1.08), 0.91; 8,192 half 1.13 and 1.19 (1.31), five eighths 0.92 and 0.99 (1.03), all
-      0.88 and 0.97."""
+    Rows beyond the last cost as much as others: 384 of 16,384 in tiles of 256 31.7 us in the library and 34.0, 512 37.8 and 35.8; gated, where a kernel is saved, 161 of 28,256, K 8,192, 129 and 123.
+    Ranges of K fill the units where the tiles do not, and cost the reader their sums.  The same, over the faster of the library and whole tiles, with the norm that reads them (from K 8,192 on with a kernel that adds them: the
+    same lines):
+      four: K to 4,608 a quarter 0.94 (1.10) / 0.99 (1.57), three eighths 0.97 (1.05) / 0.94 (0.98), half 0.95 (1.07) / 0.89 (0.99); to 8,192 a quarter 1.00 (1.16) / 0.96 (1.37), three eighths 0.90 (1.02) / 0.83
+      (0.94); beyond a quarter 0.99 (1.05) / 0.91 (0.98), three eighths 0.80 (0.90) / 0.70 (0.88);
+      two: K to 4,608 half 1.04 (1.14) / 1.02 (1.36), five eighths 0.97 (0.98) / 0.97 (1.04); 5,120 half 0.98 (1.05) / 1.02 (1.33); to 8,192 half 0.98 (1.11) / 0.77 (1.12), beyond 1.00 (1.05) / 0.71 (1.00)."""
     if m < MANY_MIN_ROWS or n % (8 if gated else 4) or k % MANY_K_MULTIPLE or not MANY_K_MIN <= k < MANY_K_MAX:
         return None
     count = [-(-m // bm) * -(-n // bn) for bm, bn in MANY_TILES]
     if may_split and k >= 4096:
         for ranges in (4, 2):
-            need = (0.625 if k < 5120 else 0.5 if k <= 8192 else 0.375) if ranges == 4 else (0.875 if k < 6144 else 0.625)
+            need = (0.375 if k <= 8192 else 0.25) if ranges == 4 else (0.625 if k < 6144 else 0.5)
             if ranges <= many_ranges(m, n, units) and k % (MANY_K_MULTIPLE * ranges) == 0 and ranges * count[MANY_SPLIT_FORM] >= need * units:
                 return MANY_SPLIT_FORM, ranges
     for form, (bm, bn) in enumerate(MANY_TILES):
         if count[form] <= units and not (gated and form < 2):
             filled = count[form] / units  # the share of the units that have a tile
             used = m * n / (count[form] * bm * bn)  # and of the tiles that is not beyond the last row or column
-            if form == 3:
+            if form == 3 or k > 4608:
                 need = 0.85
             elif gated:
-                need = 0.0 if k <= 1024 else 0.25 if k <= 2048 else 0.625 if k <= 4608 else 0.875
+                need = 0.0 if k <= 1024 else 0.25 if k <= 2048 else 0.625
             else:
-                need = 0.0 if k <= 1024 else (0.375, 0.5, 0.5)[form] if k <= 2048 else (0.625, 0.75, 0.625 if k <= 4096 else 0.75)[form] if k <= 4608 else (2.0, 0.875, 0.875)[form]
-            whole = 0.85 if form == 3 and (not gated or k > 4608) else 0.7 if form == 2 and not gated else 0.6
+                need = 0.0 if k <= 1024 else (0.375, 0.5, 0.5)[form] if k <= 2048 else (0.625, 0.75, 0.625 if k <= 4096 else 0.75)[form]
+            whole = 0.6 if gated or form < 2 else 0.7 if form == 2 else 0.85
             return (form, 1) if filled >= need and used >= whole else None
     return None
 

@@ -64,13 +64,13 @@ def test_many_rows_take_the_smallest_tile_that_fits_the_units_once():
     assert plan(800, 2048, 4096 + 256, may_split=True) == (2, 2)  # (512 rows, half of the units: 30.5 us, in whole tiles 26.4 and 27.5 in the library)
     # and only where they fill enough of them
     assert plan(129, 16, 8192, may_split=True) is None and plan(129, 68, 4096, may_split=True) is None and plan(256, 1024, 8192, may_split=True) is None
-    assert plan(200, 2048, 4096, may_split=True) is None and plan(200, 2048, 8192, may_split=True) == (2, 4) and plan(512, 2048, 4352, may_split=True) == (0, 1)
-    assert plan(384, 4096, 4096, may_split=True) == (1, 1) and plan(384, 4096, 8192, may_split=True) == (2, 2)
+    assert plan(200, 1024, 4096, may_split=True) is None and plan(200, 2048, 4096, may_split=True) == (2, 4) and plan(200, 2048, 8192, may_split=True) == (2, 4) and plan(512, 2048, 4352, may_split=True) == (0, 1)
+    assert plan(384, 4096, 4096, may_split=True) == (2, 2) and plan(200, 4480, 4096, may_split=True) is None and plan(384, 4096, 8192, may_split=True) == (2, 2)
     # too few tiles for the units: the more the longer K is
     assert plan(200, 64, 1024) == (0, 1) and plan(200, 64, 2048) is None and plan(1024, 512, 2048) == (0, 1) and plan(1024, 512, 4096) is None
-    assert plan(2048, 512, 4096) == (0, 1) and plan(2048, 512, 6144) is None and plan(512, 2560, 4096) is None and plan(384, 8192, 4608) == (2, 1) and plan(384, 8192, 5120) is None
+    assert plan(2048, 512, 4096) == (0, 1) and plan(2048, 512, 6144) == (0, 1) and plan(1600, 512, 6144) is None and plan(512, 2560, 4096) is None and plan(384, 8192, 4608) == (2, 1) and plan(384, 8192, 5120) is None
     assert plan(1531, 256, 2048) == (0, 1) and plan(1531, 2048, 4096) == (2, 1)  # (level alone, ahead beside other work and on the host)
-    assert plan(160, 1024, 2048, gated=True) is None and plan(256, 4096, 1024, gated=True) == (2, 1) and plan(384, 16384, 8192, gated=True) is None
+    assert plan(160, 1024, 2048, gated=True) is None and plan(256, 4096, 1024, gated=True) == (2, 1) and plan(384, 16384, 8192, gated=True) == (3, 1)
     for m, n, k in ((128, 2048, 2048), (512, 2048, 2048 + 64), (512, 2050, 2048), (512, 2048, 128)):
         assert plan(m, n, k) is None
     for m in (129, 300, 512, 1000, 1531, 2048):

@@ -271,6 +271,64 @@ def linear_generic(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = 
     return out
 
 
+# ``linear_split``: rows of x a tile (by 128 rows of w) and what a row of each takes over one of the largest (2,048 rows of 16,384 x 2,048)
+SPLIT_TILES = ((128, 1.0), (112, 1.035), (96, 1.03), (64, 1.2))
+SPLIT_COLUMNS = 128
+SPLIT_K_MULTIPLE = 32
+SPLIT_MIN_ROWS = 48
+SPLIT_MIN_K = 1024
+SPLIT_MIN_WORK = 3e9  # rows times columns times K
+SPLIT_CHUNK_ROWS = 4096  # more are taken in portions, so that the parts of x take no more than 24 KB for each of its columns
+
+
+@functools.lru_cache(maxsize=1 << 14)
+def split_plan(m: int, n: int, k: int, units: int) -> tuple[int, int] | None:
+    """(rows of a tile, ranges of K) for ``linear_split``, or None where ``linear_generic`` is the faster one or the sizes are not taken.
+
+    Ranges fill the units where the tiles do not: 777 rows, N 2,048, K 8,192 one, two, four 388 / 198, 201 / 135, 171 / 133 us (alone / beside two others), N 3,072, K 2,048 one,
+    two, four 110 / 59, 89 / 53, 77 / 56.  Below ``SPLIT_MIN_WORK`` products the splitting of x and the sum of the ranges cost alone what the product gains: its time over
+    linear_generic's, 48 to 2,048 rows, median (largest), alone / beside: 1 to 2e9 1.18 (1.33) / 0.95 (1.07), 2 to 3e9 0.96 (1.25) / 0.78 (0.95), 3 to 6e9 0.96 (1.21) / 0.67 (0.78),
+    from 6e9 on 0.71 (1.11) / 0.61 (0.80)."""
+    if m < SPLIT_MIN_ROWS or k < SPLIT_MIN_K or k % SPLIT_K_MULTIPLE or k >= 1 << 21 or m * n * k < SPLIT_MIN_WORK:
+        return None
+    m, columns = min(m, SPLIT_CHUNK_ROWS), -(-n // SPLIT_COLUMNS)
+    tiles = lambda rows: -(-m // rows) * columns
+    if tiles(64) < 0.375 * units:
+        return None
+    rows = min((t for t in SPLIT_TILES if 4 * tiles(t[0]) >= units), key=lambda t: -(-m // t[0]) * t[0] * t[1])[0]
+    enough = (1.5 if k >= 4096 else 1) * units
+    return rows, 1 if tiles(rows) >= enough else 2 if 2 * tiles(rows) >= enough else 4
+
+
+def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_split`` takes these operands: float32, whole 16-byte pieces, w in plain rows."""
+    return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1
+            and x.stride(0) >= x.shape[1] and x.stride(0) % 4 == 0 and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None) -> torch.Tensor:
+    """float32 x @ w.T for many rows on the bfloat16 matrix cores, each operand as the sum of three bfloat16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
+    with ``ranges`` ranges of K (``split_plan`` chooses).  ``take`` (shape, dtype): scratch, 6 K bytes a row of x and with ranges 4 N a row and range."""
+    out = _check_linear(x, w, out, False)
+    if not split_takes(x, w):
+        raise KernelRefused("linear_split takes float32 x [rows, K] in rows of whole 16-byte pieces and w [N, K], both on 16 bytes")
+    m, (n, k) = x.shape[0], w.shape
+    if take is None:
+        take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device)
+    lib, most = build.core(), min(m, SPLIT_CHUNK_ROWS)
+    parts = take((-(-most // 16) * 16 * 3 * k,), torch.bfloat16)
+    sums = take((ranges * most * n,), torch.float32) if ranges > 1 else None
+    for s in range(0, m, SPLIT_CHUNK_ROWS):
+        piece, to = (x, out) if m == most else (x[s : s + SPLIT_CHUNK_ROWS], out[s : s + SPLIT_CHUNK_ROWS])
+        h = c_int(piece.shape[0])
+        _check(lib.ns_split_rows(_ptr(parts), _ptr(piece), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
+        _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(piece), _ptr(w), h, c_int(n), c_int(k), c_int(x.stride(0)),
+                                 c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
+        if sums is not None:
+            reduce_partial(PartialSums(sums, ranges, piece.shape[0], n, torch.float32), out=to)
+    return out
+
+
 SKINNY_MAX_ROWS = 64
 WIDE_TALL_ROWS = 128  # ``linear_wide`` with one matrix and one row tile per wave takes this many rows
 

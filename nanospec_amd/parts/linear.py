@@ -1,8 +1,8 @@
 """x @ W^T for the parts: ``LinearWeight`` holds a weight matrix and chooses the kernel by precision and row count.
 
-float32: always ``csrc/gemm_generic.hip``, 32-bit products and sums in a fixed order (the true 32-bit path; no matrix-core
-mode of reduced precision is ever used): up to 8 rows stream the weights, more run the 32-bit matrix instruction, odd sizes the
-plain tiled kernel.
+float32: ``csrc/gemm_generic.hip``, 32-bit products and sums in a fixed order: up to 8 rows stream the weights, more run the 32-bit matrix
+instruction, odd sizes the plain tiled kernel; and ``csrc/gemm_split.hip`` for many rows, whose operands are sums of three bfloat16 values
+and whose results are nearer to 64 bits than those.  (The true 32-bit path: no mode of reduced precision is ever used.)
 
 bfloat16: decode and short portions (up to ``STREAM_ROWS`` rows) run the hand-written matrix-core kernel that streams
 the weights once; it reads them in a layout re-laid at load time (``kernels.ops.TiledWeight``) in which every load
@@ -95,6 +95,18 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
         return into.addmm_(x, w_t)
     y = torch.matmul(x, w_t) if out is None else torch.matmul(x, w_t, out=out)
     return y if act is None else ops.activation(y, act)
+
+
+def product_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, arena) -> torch.Tensor:
+    """x @ w^T in 32-bit: many rows of a wide enough matrix on the bfloat16 matrix cores, no less exact (``ops.linear_split``; its scratch comes from ``arena``, without one it is
+    not taken), the others on the 32-bit ones."""
+    plan = ops.split_plan(x.shape[0], w.shape[0], w.shape[1], ops.compute_units(x.device)) if arena is not None and x.is_cuda else None
+    if plan is None or not ops.split_takes(x, w):
+        return ops.linear_generic(x, w, out=out)
+    mark = arena.mark()
+    out = ops.linear_split(x, w, *plan, out=out, take=arena.take)
+    arena.release(mark)
+    return out
 
 
 class IntoResidual:
@@ -214,7 +226,9 @@ class LinearWeight:
             return ops.linear_tiled(x, self.tiled, out=out, out_f32=out_f32)
         if x.dtype != self.dtype:
             raise ops.KernelRefused(f"linear: input is {x.dtype}, the weight {self.dtype}")
-        if self.dtype == torch.float32 or self.k % 8 or not ops.tiled_takes(x[:1], self.k):
+        if self.dtype == torch.float32:
+            return product_f32(x, self.plain, out, arena)
+        if self.k % 8 or not ops.tiled_takes(x[:1], self.k):
             return ops.linear_generic(x, self.plain, out=out, out_f32=out_f32)
         m = x.shape[0]
         if self.tiled is not None and WIDE_HEAD_ROWS < m <= STREAM_ROWS and out_f32 and self.n >= 8192:
@@ -302,6 +316,8 @@ class GatedWeights:
             gu = ctx.arena.take((m, 2 * self.inter), x.dtype)
             if self._stacked_linear is not None:
                 self._stacked_linear(x, out=gu, arena=ctx.arena, plain_copy=not ctx.captured)
+            elif self.dtype == torch.float32:
+                product_f32(x, self.stacked, gu, ctx.arena)
             else:
                 ops.linear_generic(x, self.stacked, out=gu)
             return ops.silu_mul_bias(gu, self.bias_stacked, out=out)
@@ -330,5 +346,7 @@ class GatedWeights:
                 ops.linear_wide(x[s:e], self.tiled[0], w2=self.tiled[1], out=out[s:e], ksplit=1, nt=1)
             return out
         if self.dtype == torch.float32 or self.k % 8:
-            return ops.silu_mul(ops.linear_generic(x, self.stacked, out=ctx.arena.take((m, 2 * self.inter), x.dtype)), out=out)
+            gu = ctx.arena.take((m, 2 * self.inter), x.dtype)
+            product = product_f32(x, self.stacked, gu, ctx.arena) if self.dtype == torch.float32 else ops.linear_generic(x, self.stacked, out=gu)
+            return ops.silu_mul(product, out=out)
         return library_product(x, self._stacked_t, gated=out, plain=self.stacked, take=ctx.arena.take)

@@ -117,6 +117,63 @@ def test_linear_f32_of_rows_far_apart(m, stride, n, k):
     assert torch.equal(ops.linear_generic(far, w), ops.linear_generic(x, w))
 
 
+@pytest.mark.parametrize("rows", [64, 96, 112, 128])
+@pytest.mark.parametrize("m,n,k,ranges", [(1, 1, 32, 1), (15, 130, 64, 2), (17, 131, 96, 3), (113, 257, 160, 1), (129, 64, 1056, 4), (300, 2060, 1024, 2)])
+def test_linear_split(rows, m, n, k, ranges):
+    """32-bit products through three bfloat16 parts of each operand at the edges of the tiles (16 rows and the tile's, 16 and 128 columns), of a stage of 32 k and of
+    uneven ranges; rows of x and of the result with a stride of their own."""
+    ops = _ops()
+    torch.manual_seed(m + n + k)
+    wide = torch.randn(m, k + 12, device=DEV)
+    x, w, out = wide[:, 4 : 4 + k], torch.randn(n, k, device=DEV), torch.full((m, n + 3), 7.0, device=DEV)
+    ref = x.cpu().double() @ w.cpu().double().T
+    # a stage's sum is rounded 24 times (six instructions, four blocks of 8 k each) and leaves out 2^-24; then a stage or range is added at a time
+    bound = (25 + k / 32 + ranges) * 2.0**-24 * (x.cpu().double().abs() @ w.cpu().double().abs().T)
+    ops.linear_split(x, w, rows, ranges, out=out[:, :n])
+    assert ((out[:, :n].cpu().double() - ref).abs() <= bound).all()
+    assert bool((out[:, n:] == 7).all())
+    if m * n > 1000:  # nearer to 64 bits than the 32-bit instruction
+        far = lambda y: float((y.cpu().double() - ref).norm())
+        assert far(out[:, :n]) <= far(ops.linear_generic(x, w))
+
+
+@pytest.mark.parametrize("ranges", [1, 2])
+def test_linear_split_beyond_the_parts(ranges):
+    """Infinities, no numbers, the largest floats (whose first part would round up to infinity) and floats whose lower parts bfloat16 does not hold."""
+    ops = _ops()
+    torch.manual_seed(3)
+    x, w = torch.randn(70, 128, device=DEV), torch.randn(140, 128, device=DEV)
+    x[3, 5], x[4, 6], x[5, 7], x[6] = math.inf, -math.inf, math.nan, 0.0
+    x[7], w[11, 3], w[12, 100] = 0.0, 0.0, math.inf
+    x[8, 9] = x[9, 9] = 3.4028234e38  # (times a normal number: a large float, or infinity)
+    x[10:20] *= 2.0**-120
+    x[7, 1] = 2.0**-126 * 1.2345678
+    out = ops.linear_split(x, w, 64, ranges).cpu()
+    a, b = x.cpu().double(), w.cpu().double()
+    ref = a @ b.T
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    over = ref.abs() > 3.4028235e38 * (1 + 2.0**-24)
+    assert bool((out[over] == torch.sign(ref[over]).float() * math.inf).all())
+    fine = torch.isfinite(ref) & (ref.abs() < 3.4e38)
+    bound = 2.0**-17 * (a.abs().clamp(max=3.5e38) @ b.abs().clamp(max=3.5e38).T) + 128 * 2.0**-149  # one chain of 128, floored by the smallest float
+    assert bool(((out.double() - ref).abs()[fine] <= bound[fine]).all())
+
+
+def test_split_plan():
+    """What goes to the split kernel: whole stages, enough tiles; every plan is one that the launch takes."""
+    from nanospec_amd.kernels import ops
+
+    for m in (1, 47, 48, 65, 112, 128, 130, 777, 2048, 5000):
+        for n in (1, 512, 2048, 3072, 16384, 128256):
+            for k in (32, 1000, 1024, 1056, 2048, 8192):
+                plan = ops.split_plan(m, n, k, 256)
+                if plan is not None:
+                    rows, ranges = plan
+                    assert m >= 48 and m * n * k >= 3e9 and k % 32 == 0 and rows in (64, 96, 112, 128) and 1 <= ranges <= k // 32
+    assert ops.split_plan(777, 16384, 2048, 256) == (112, 1) and ops.split_plan(512, 2048, 8192, 256) == (128, 4)
+    assert ops.split_plan(47, 128256, 2048, 256) is None and ops.split_plan(256, 512, 2048, 256) is None
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("n,k", [(48, 64), (130, 200), (1000, 4096), (257, 1064), (16, 8), (4096, 14336)])
 def test_linear_tiled(m, n, k):

@@ -11,6 +11,8 @@
 #include "lds_loads.h"
 #include <type_traits>
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 #define GT_M 64
 #define GT_N 64
 #define GT_K 16
@@ -59,82 +61,93 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(OutT* __restrict__ ou
   }
 }
 
-// Few rows (decode) in 32-bit: the work is reading w once.  A workgroup of eight waves owns ROWS_N rows of w and deals their
-// K to its 512 lanes in units of four (16-byte loads, a wave's load a contiguous KiB of a row); every lane sums its own k in
-// order for each of up to ROWS_M rows of x, the 64 partial sums of an output are added by a fixed butterfly that halves the
-// values a lane holds at each step, and the eight waves' sums in LDS.  An output's value depends on its own row of x and of w
-// only.  For K and the row strides multiples of 4 and 16-byte aligned operands.
-// Bound by the loads: the waves of a workgroup share its rows of w, so each piece of x is read once for eight rows (once for
-// four by a wave alone, over the whole of K, was bound by x coming from L2), and N = 2,048 still fills 256 compute units;
-// two workgroups a unit, hence at most 128 registers (132 and one workgroup: 308 us in the last line).  Five rows:
-//   N 2,048 K 2,048: 20 -> 8 us; N 2,048 K 8,192: 64 -> 19 us (3.5 TB/s); N 16,384 K 2,048: 38 -> 30 us (4.5 TB/s); N 128,256: 207 us
-//   either way (5.1 TB/s)
+// Few rows (decode) in 32-bit: the work is reading w once.  A workgroup of WAVES waves owns eight rows of w and deals their
+// K to its lanes in units of four (16-byte loads, a wave's load a contiguous KiB of a row); every lane sums its own k in
+// order for each of MT rows of x, the 64 partial sums of an output are added in a fixed order by the vector unit (what lanes exchange for a sum of two of a wave's
+// halves or quarters at a time, then of neighbours), and the waves' sums in LDS.  An output's value depends on its own row of x and of w only.
+// For K and the row strides multiples of 4 and 16-byte aligned operands.
+// Bound by the loads of w, read past the caches; what stands beside them are x, which comes from L2 (all of it once a workgroup) and the products, so a number of rows has
+// a kernel of its own, and the addresses, which the scalar unit holds but for the lane's (in vector registers they would not leave room for 8 rows).  us, alone and a call beside two
+// others, with sums through LDS's crossbar and 1, 2, 4 or 8 rows of x, and now: five rows, N 16,384, K 2,048 32.5 / 27.0 and 24.9 / 20.8 (5.4 TB/s, 6.5); N 2,048, K 8,192 19.0 /
+// 13.6 and 16.0 / 12.8; N 2,048, K 2,048 8.7 / 6.2 and 7.2 / 5.4; N 128,256, K 2,048 212 / 215 and 158 / 158 (6.7 TB/s); eight rows 215 / 218 and 173 / 176, one row 170 / 165 and 156 / 152.
 #define ROWS_M 8
 #define ROWS_N 8
-#define ROWS_WAVES 8
 
-// Sums of VALS (a power of two up to 64) values over the 64 lanes; lane l ends up with value l / (64 / VALS).
-template <int VALS, int O = 32>
-__device__ __forceinline__ float sum_over_lanes(float* v, int lane) {
-  if constexpr (VALS > 1) {
-    const bool upper = lane & O;
+// Lanes 0-31 (of every pair of rows of 16 lanes the lower one) get the sum of ``a`` over both halves (rows), the others that of ``b``.
+__device__ __forceinline__ float sum_halves(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float sum_rows(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <int MT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 4) void gemm_rows_f32_kernel(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, int N, int K,
+                                                                      int x_stride, int out_stride) {
+  __shared__ float part[WAVES][ROWS_N * MT];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n0 = blockIdx.x * ROWS_N;
+  float acc[ROWS_N][MT];
 #pragma unroll
-    for (int i = 0; i < VALS / 2; ++i) {
-      const float give = upper ? v[i] : v[VALS / 2 + i], keep = upper ? v[VALS / 2 + i] : v[i];
-      v[i] = keep + __shfl_xor(give, O, 64);
+  for (int j = 0; j < ROWS_N; ++j)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[j][m] = 0.f;
+  const char *wr[ROWS_N], *xr[MT];
+#pragma unroll
+  for (int j = 0; j < ROWS_N; ++j) wr[j] = reinterpret_cast<const char*>(w + (size_t)min(n0 + j, N - 1) * K);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xr[m] = reinterpret_cast<const char*>(x + (size_t)m * x_stride);
+  for (unsigned i = threadIdx.x; i < (unsigned)K / 4; i += 64 * WAVES) {
+    const unsigned at = 16 * i;  // (32 bits, so that a row's address stays in the scalar unit)
+    f32x4 wv[ROWS_N];
+#pragma unroll
+    for (int j = 0; j < ROWS_N; ++j) wv[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(wr[j] + at));
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const f32x4 xv = *reinterpret_cast<const f32x4*>(xr[m] + at);
+#pragma unroll
+      for (int j = 0; j < ROWS_N; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][m] = fmaf(xv[e], wv[j][e], acc[j][m]);
     }
-    return sum_over_lanes<VALS / 2, O / 2>(v, lane);
-  } else {
-    float r = v[0];
+  }
+  // lanes 8 j .. 8 j + 7 end up with row j of w
 #pragma unroll
-    for (int o = O; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
-    return r;
+  for (int m = 0; m < MT; ++m) {
+    float half[4], row[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) half[j] = sum_halves(acc[j][m], acc[j + 4][m]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) row[j] = sum_rows(half[j], half[j + 2]);
+    const bool upper = lane & 8;
+    const float keep = upper ? row[1] : row[0], give = upper ? row[0] : row[1];
+    const float sum = group_sum<8>(keep + dpp_read<0x128>(give));  // row_ror 8
+    if (lane % 8 == 0) part[wave][lane / 8 * MT + m] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x < ROWS_N * MT) {
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES; ++i) v += part[i][threadIdx.x];
+    const int n = n0 + threadIdx.x / MT, m = threadIdx.x % MT;
+    if (n < N) out[(size_t)m * out_stride + n] = v;
   }
 }
 
-template <int MT>  // rows of x that are summed for (a power of two; M of them count)
-__global__ __launch_bounds__(64 * ROWS_WAVES, 4) void gemm_rows_f32_kernel(float* __restrict__ out, const float* __restrict__ x,
-                                                                        const float* __restrict__ w, int M, int N, int K, int x_stride,
-                                                                        int out_stride) {
-  constexpr int VALS = ROWS_N * MT;
-  __shared__ float part[ROWS_WAVES][VALS];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n0 = blockIdx.x * ROWS_N;
-  float acc[VALS];
-#pragma unroll
-  for (int i = 0; i < VALS; ++i) acc[i] = 0.f;
-  const float4* wr[ROWS_N];
-#pragma unroll
-  for (int j = 0; j < ROWS_N; ++j) wr[j] = reinterpret_cast<const float4*>(w + (size_t)min(n0 + j, N - 1) * K);
-  const int k4 = K / 4;
-  for (int i = threadIdx.x; i < k4; i += 64 * ROWS_WAVES) {
-    float4 wv[ROWS_N];
-#pragma unroll
-    for (int j = 0; j < ROWS_N; ++j) wv[j] = wr[j][i];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const float4 xv = reinterpret_cast<const float4*>(x + (size_t)min(m, M - 1) * x_stride)[i];
-#pragma unroll
-      for (int j = 0; j < ROWS_N; ++j) {
-        float a = acc[j * MT + m];
-        a = fmaf(xv.x, wv[j].x, a);
-        a = fmaf(xv.y, wv[j].y, a);
-        a = fmaf(xv.z, wv[j].z, a);
-        a = fmaf(xv.w, wv[j].w, a);
-        acc[j * MT + m] = a;
-      }
-    }
-  }
-  const float r = sum_over_lanes<VALS>(acc, lane);
-  if (lane % (64 / VALS) == 0) part[wave][lane / (64 / VALS)] = r;
-  __syncthreads();
-  if (threadIdx.x < VALS) {
-    float v = 0.f;
-#pragma unroll
-    for (int i = 0; i < ROWS_WAVES; ++i) v += part[i][threadIdx.x];
-    const int n = n0 + threadIdx.x / MT, m = threadIdx.x % MT;
-    if (n < N && m < M) out[(size_t)m * out_stride + n] = v;
-  }
+template <int MT = 1>
+static int launch_rows_f32(float* out, const float* x, const float* w, int M, int N, int K, int x_stride, int out_stride, hipStream_t stream) {
+  if constexpr (MT < ROWS_M)
+    if (M > MT) return launch_rows_f32<MT + 1>(out, x, w, M, N, K, x_stride, out_stride, stream);
+  const int blocks = (N + ROWS_N - 1) / ROWS_N;
+  // Four waves where a row is then no more than two loads a lane (the sums of a longer chain are further from 64 bits: K 8,192 1.3e-7 instead of 1.15e-7) and there are two
+  // workgroups for every compute unit: five rows, N 128,256, K 2,048 158 us, with eight waves 169; N 32,000, K 1,024 25 and 32; N 3,072, K 2,048 9.1 and 9.2; N 512 5.2 and 4.4.
+  // (The sums depend on this choice, so it is the same for any number of rows.)
+  if (K <= 2048 && N >= 4096)
+    gemm_rows_f32_kernel<MT, 4><<<blocks, 256, 0, stream>>>(out, x, w, N, K, x_stride, out_stride);
+  else
+    gemm_rows_f32_kernel<MT, 8><<<blocks, 512, 0, stream>>>(out, x, w, N, K, x_stride, out_stride);
+  return ns_launch_status();
 }
 
 // Many rows in 32-bit on the matrix cores (v_mfma_f32_16x16x4_f32, 32-bit products and sums: 157 TFLOP/s at the boost clock,
@@ -155,7 +168,6 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 4) void gemm_rows_f32_kernel(float
 // 12.4 -> 10.0; a short K, 2,048 rows, N 2,048, K 64: 18.7 -> 16.5.  A third of that is addresses: with a 64-bit sum a load in the vector unit the first of these takes 481 us.
 // Relative error (2-norm, against 64 bits) 4.1e-7 at K 2,048, 8.1e-7 at K 8,192, half of the tiled kernel's above: four chains for one.
 // K and the row strides multiples of 4, 16-byte aligned operands.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define G32_K 64
 #define G32_MAX_BLOCKS 0xffffffL    // workgroups of 256 threads that one dimension of a launch holds
 #define G32_MAX_STRIDE (1 << 24)    // 64 rows of fewer floats than this are addressed by 32 bits
@@ -298,18 +310,7 @@ extern "C" int ns_gemm_generic(void* out, const void* x, const void* w, int M, i
       N < (1 << 26)) {
     float* o = (float*)out;
     const float *xf = (const float*)x, *wf = (const float*)w;
-    if (M <= ROWS_M) {
-      const int blocks = (N + ROWS_N - 1) / ROWS_N;
-      if (M == 1)
-        gemm_rows_f32_kernel<1><<<blocks, 64 * ROWS_WAVES, 0, stream>>>(o, xf, wf, M, N, K, x_stride, out_stride);
-      else if (M == 2)
-        gemm_rows_f32_kernel<2><<<blocks, 64 * ROWS_WAVES, 0, stream>>>(o, xf, wf, M, N, K, x_stride, out_stride);
-      else if (M <= 4)
-        gemm_rows_f32_kernel<4><<<blocks, 64 * ROWS_WAVES, 0, stream>>>(o, xf, wf, M, N, K, x_stride, out_stride);
-      else
-        gemm_rows_f32_kernel<8><<<blocks, 64 * ROWS_WAVES, 0, stream>>>(o, xf, wf, M, N, K, x_stride, out_stride);
-      return ns_launch_status();
-    }
+    if (M <= ROWS_M && K < 1 << 30) return launch_rows_f32(o, xf, wf, M, N, K, x_stride, out_stride, stream);
     // Tiles of 32 x 64 where there are four for every compute unit (777 rows, N 16,384, K 2,048: 430 against 442 us, 2,048 rows 1,066 against
     // 1,171), of 32 x 32 where they fill the GPU and are not half empty (777 rows, N 2,048, K 8,192: 231 against 253; 100 rows 50 against 57
     // with 16 x 16), of 16 x 16 otherwise (64 rows, N 2,048, K 8,192: 36 against 50).  64 x 64 deals less evenly (443 us in the first of these).

@@ -109,6 +109,259 @@ extern "C" int ns_attn_generic(void* out, const void* q, int q_stride, const voi
 }
 
 // ------------------------------------------------------------------------------------------------
+// What stands between an attention layer's projections and its scores, in pieces of 8 bytes: biases, the RMS norm of a head or of a whole projection, the rotation, keys and values
+// into their pages.  The three entry points below take these kernels where sizes and addresses allow (``kv_rows_take``) and the plain ones, an element a lane, elsewhere.
+// A workgroup is a token.  L neighbouring lanes take a head's channels, two pieces of H each (``unit_of``): with the half-split pairing a piece and its partners, else one
+// after the other.  The cosines and sines of a token are made once for all its heads (with them in every head a third of the time).  Of the tokens of a request that stand side by
+// side in a run of whole 16 bytes of a value page the first writes the values of all, 16 bytes a store; an element a store they are 2 bytes in every line of 32.
+// Bound by launches and the row's way from memory and back, us before (plain) and now, bfloat16, 2,048 tokens, 32 heads of 64 over 8: norm a head 26.8 / 21.8 -> 18.2 / 11.8 (alone / beside
+// two others), with weights, biases and rotation, 1,531 tokens, 29.8 / 24.0 -> 17.1 / 10.9; norm of the projection with rotation, 512 tokens, 15.4 / 8.5 -> 10.5 / 5.6, 8 tokens 6.9 / 4.1 -> 4.7 / 3.2.
+// ------------------------------------------------------------------------------------------------
+template <typename T>
+struct KvRows {
+  T* qkv;
+  const T *bias, *qw, *kw;  // (each may be null)
+  const int *positions, *token_req, *block_table;
+  const float* inv_freq;
+  T *k_cache, *v_cache;
+  int stride, table_stride, n_tokens, heads, kv_heads, hd, vd, page_size, lanes, shares;  // kv_heads 0: no keys and values of its own
+  float eps;
+  RopeForm form;
+  int norm_q, norm_k, v_is_k;
+  const T *lambda, *v_other;  // values <- (1 - lambda) values + lambda v_other
+  T* v_keep;
+  int v_other_stride, v_keep_stride;
+};
+
+template <typename T>
+struct KvPiece {
+  static constexpr int H = 8 / sizeof(T);
+  typedef T type __attribute__((ext_vector_type(H)));
+};
+
+// the first channels of a lane's two pieces
+template <typename T>
+__device__ __forceinline__ void unit_of(const KvRows<T>& p, int l, int& d1, int& d2) {
+  constexpr int H = KvPiece<T>::H;
+  const int turned = p.form.interleaved ? 0 : p.form.rot / 2 / H;  // lanes whose pieces are partners
+  d1 = l < turned ? l * H : 2 * l * H;
+  d2 = d1 + (l < turned ? p.form.rot / 2 : H);
+}
+
+template <typename T>
+__device__ __forceinline__ void load_piece(const T* row, const T* bias, float* v) {
+  constexpr int H = KvPiece<T>::H;
+  const auto r = *reinterpret_cast<const typename KvPiece<T>::type*>(row);
+#pragma unroll
+  for (int e = 0; e < H; ++e) v[e] = to_f((T)r[e]);
+  if (bias) {
+    const auto b = *reinterpret_cast<const typename KvPiece<T>::type*>(bias);
+#pragma unroll
+    for (int e = 0; e < H; ++e) v[e] += to_f((T)b[e]);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void store_piece(T* to, const float* v) {
+  typename KvPiece<T>::type o;
+#pragma unroll
+  for (int e = 0; e < KvPiece<T>::H; ++e) o[e] = from_f<T>(v[e]);
+  *reinterpret_cast<typename KvPiece<T>::type*>(to) = o;
+}
+
+// A unit's channels times ``f`` (if its part is normed) and the weights, rotated, and to where they belong.  ``w``: the head's weights or null.
+template <typename T>
+__device__ __forceinline__ void finish_unit(const KvRows<T>& p, T* row, int h, int d1, int d2, float* a, float* b, float f, bool normed, const T* w, const float* cs, int page,
+                                            int slot) {
+  constexpr int H = KvPiece<T>::H;
+  if (normed) {
+#pragma unroll
+    for (int e = 0; e < H; ++e) a[e] *= f, b[e] *= f;
+  }
+  if (w) {
+    float wa[H], wb[H];
+    load_piece<T>(w + d1, nullptr, wa), load_piece<T>(w + d2, nullptr, wb);
+#pragma unroll
+    for (int e = 0; e < H; ++e) a[e] *= wa[e], b[e] *= wb[e];
+  }
+  const int half = p.form.rot / 2;
+  if (p.form.interleaved) {
+#pragma unroll
+    for (int e = 0; e < H; e += 2) {
+      if (d1 + e < p.form.rot) rope_turn(a[e], a[e + 1], cs[(d1 + e) / 2], cs[half + (d1 + e) / 2], a[e], a[e + 1]);
+      if (d2 + e < p.form.rot) rope_turn(b[e], b[e + 1], cs[(d2 + e) / 2], cs[half + (d2 + e) / 2], b[e], b[e + 1]);
+    }
+  } else if (d1 < half) {
+#pragma unroll
+    for (int e = 0; e < H; ++e) rope_turn(a[e], b[e], cs[d1 + e], cs[half + d1 + e], a[e], b[e]);
+  }
+  T* to = h < p.heads ? row + (size_t)h * p.hd : p.k_cache + (((size_t)page * p.kv_heads + (h - p.heads)) * p.page_size + slot) * p.hd;
+  store_piece(to + d1, a), store_piece(to + d2, b);
+}
+
+// The values of a token, or of a run of tokens by its first.
+template <typename T>
+__device__ __forceinline__ void write_values(const KvRows<T>& p, int t) {
+  constexpr int H = KvPiece<T>::H, V = 2 * H;
+  typedef T run_t __attribute__((ext_vector_type(V)));
+  const int lane = threadIdx.x % NS_WAVE, req = p.token_req[t], pos = p.positions[t], slot = pos % p.page_size, nq = p.heads * p.hd;
+  const int page = p.block_table[(size_t)req * p.table_stride + pos / p.page_size];
+  int count = 1;
+  if (p.page_size % V == 0) {  // lane i asks whether token t - 1 + i goes on with this one's run (one after the other that is a trip to memory each)
+    const int other = min(max(t - 1 + lane, 0), p.n_tokens - 1), place = pos - 1 + lane;
+    const bool goes_on = lane <= V && other == t - 1 + lane && p.token_req[other] == req && p.positions[other] == place && place / V == pos / V;
+    const unsigned long long with = __ballot(goes_on);
+    if (with & 1) return;
+    count = __ffsll((long long)~(with >> 1)) - 1;
+  }
+  const int at = p.v_is_k ? nq : nq + p.kv_heads * p.hd;  // of the values in a row
+  const float lam = p.lambda && p.v_other ? to_f(p.lambda[0]) : 0.f;
+  // (neighbouring lanes have neighbouring channels, whose runs in a page are neighbours: four channels a lane, whose stores lie 128 bytes apart, 19.9 / 13.1 us in the first line above)
+  for (int c = threadIdx.x; c < p.kv_heads * p.vd; c += blockDim.x) {
+    T* to = p.v_cache + ((size_t)page * p.kv_heads * p.vd + c) * p.page_size + slot;  // (a page's heads and their channels lie one behind the other)
+    const T *from = p.qkv + (size_t)t * p.stride + at + c, *from_other = p.v_other ? p.v_other + (size_t)t * p.v_other_stride + c : nullptr;
+    const float bias = p.bias ? to_f(p.bias[at + c]) : 0.f;
+    auto value = [&](int i, T v, T other) {  // of token t + i, from its own and the other layer's
+      float z = to_f(v) + bias;
+      if (from_other) z = (1.f - lam) * z + lam * to_f(other);
+      v = from_f<T>(z);
+      if (p.v_keep) p.v_keep[(size_t)(t + i) * p.v_keep_stride + c] = v;
+      return v;
+    };
+    if (count == V) {  // (all loads ahead of the first use)
+      run_t v, other = {};
+#pragma unroll
+      for (int i = 0; i < V; ++i) v[i] = from[(size_t)i * p.stride];
+      if (from_other) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) other[i] = from_other[(size_t)i * p.v_other_stride];
+      }
+#pragma unroll
+      for (int i = 0; i < V; ++i) v[i] = value(i, v[i], other[i]);
+      *reinterpret_cast<run_t*>(to) = v;
+    } else {
+      for (int i = 0; i < count; ++i) to[i] = value(i, from[(size_t)i * p.stride], from_other ? from_other[(size_t)i * p.v_other_stride] : from_f<T>(0.f));
+    }
+  }
+}
+
+// Few tokens: ``shares`` workgroups for a token's heads and one more for its values (8 tokens 6.7 -> 3.8 us, 64 tokens of 40 heads of 128 6.4 -> 5.5); many: one for all of it.
+template <typename T>
+__device__ __forceinline__ bool only_values(const KvRows<T>& p) { return (int)blockIdx.y == p.shares; }
+template <typename T>
+__device__ __forceinline__ bool values_too(const KvRows<T>& p) { return p.kv_heads && gridDim.y == 1; }
+
+// A norm over every head.
+template <typename T>
+__global__ __launch_bounds__(512) void head_rows_kernel(const KvRows<T> p) {
+  constexpr int H = KvPiece<T>::H;
+  extern __shared__ float cs[];  // cos[rot / 2] | sin[rot / 2]
+  const int t = blockIdx.x;
+  if (only_values(p)) return write_values(p, t);
+  const int pos = p.positions[t], half = p.form.rot / 2;
+  T* row = p.qkv + (size_t)t * p.stride;
+  const int page = p.kv_heads ? p.block_table[(size_t)p.token_req[t] * p.table_stride + pos / p.page_size] : 0, slot = pos % p.page_size;
+  if (half) {
+    for (int j = threadIdx.x; j < half; j += blockDim.x) rope_cos_sin(p.form, pos, p.inv_freq[j], cs[j], cs[half + j]);
+    __syncthreads();
+  }
+  // (a head's lanes stand in one wave and go round together)
+  for (int u = blockIdx.y * blockDim.x + threadIdx.x; u < (p.heads + p.kv_heads) * p.lanes; u += p.shares * blockDim.x) {
+    const int h = u / p.lanes;
+    const bool is_q = h < p.heads, normed = is_q ? p.norm_q : p.norm_k;
+    int d1, d2;
+    unit_of(p, u % p.lanes, d1, d2);
+    float a[H], b[H];
+    load_piece<T>(row + (size_t)h * p.hd + d1, p.bias ? p.bias + (size_t)h * p.hd + d1 : nullptr, a);
+    load_piece<T>(row + (size_t)h * p.hd + d2, p.bias ? p.bias + (size_t)h * p.hd + d2 : nullptr, b);
+    float ss = 0.f;
+    if (normed) {
+#pragma unroll
+      for (int e = 0; e < H; ++e) ss = fmaf(a[e], a[e], ss);
+#pragma unroll
+      for (int e = 0; e < H; ++e) ss = fmaf(b[e], b[e], ss);
+      for (int o = 1; o < p.lanes; o <<= 1) ss += __shfl_xor(ss, o, NS_WAVE);
+    }
+    finish_unit(p, row, h, d1, d2, a, b, 1.f / sqrtf(ss / (float)p.hd + p.eps), normed, is_q ? p.qw : p.kw, cs, page, slot);
+  }
+  if (values_too(p)) write_values(p, t);
+}
+
+// A norm over all heads of q and one over all of k; a thread keeps up to UNITS units between the sums and what follows them.
+#define WHOLE_UNITS 2
+template <typename T>
+__global__ __launch_bounds__(1024) void whole_rows_kernel(const KvRows<T> p) {
+  constexpr int H = KvPiece<T>::H;
+  extern __shared__ float cs[];  // cos[rot / 2] | sin[rot / 2]
+  __shared__ float sums[2][16];
+  const int t = blockIdx.x;
+  if (only_values(p)) return write_values(p, t);
+  const int pos = p.positions[t], half = p.form.rot / 2, units = (p.heads + p.kv_heads) * p.lanes;
+  T* row = p.qkv + (size_t)t * p.stride;
+  const int page = p.block_table[(size_t)p.token_req[t] * p.table_stride + pos / p.page_size], slot = pos % p.page_size;
+  float a[WHOLE_UNITS][H], b[WHOLE_UNITS][H], sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int i = 0; i < WHOLE_UNITS; ++i) {
+    const int u = threadIdx.x + i * blockDim.x, h = u / p.lanes;
+    if (u >= units) continue;
+    int d1, d2;
+    unit_of(p, u % p.lanes, d1, d2);
+    load_piece<T>(row + (size_t)h * p.hd + d1, p.bias ? p.bias + (size_t)h * p.hd + d1 : nullptr, a[i]);
+    load_piece<T>(row + (size_t)h * p.hd + d2, p.bias ? p.bias + (size_t)h * p.hd + d2 : nullptr, b[i]);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < H; ++e) ss = fmaf(a[i][e], a[i][e], ss);
+#pragma unroll
+    for (int e = 0; e < H; ++e) ss = fmaf(b[i][e], b[i][e], ss);
+    (h < p.heads ? sq : sk) += ss;
+  }
+  for (int j = threadIdx.x; j < half; j += blockDim.x) rope_cos_sin(p.form, pos, p.inv_freq[j], cs[j], cs[half + j]);
+  sq = wave_sum(sq), sk = wave_sum(sk);
+  if (threadIdx.x % NS_WAVE == 0) sums[0][threadIdx.x / NS_WAVE] = sq, sums[1][threadIdx.x / NS_WAVE] = sk;
+  __syncthreads();
+  sq = sk = 0.f;
+  for (int i = 0; i < (int)blockDim.x / NS_WAVE; ++i) sq += sums[0][i], sk += sums[1][i];
+  const float fq = 1.f / sqrtf(sq / (float)(p.heads * p.hd) + p.eps), fk = 1.f / sqrtf(sk / (float)(p.kv_heads * p.hd) + p.eps);
+#pragma unroll
+  for (int i = 0; i < WHOLE_UNITS; ++i) {
+    const int u = threadIdx.x + i * blockDim.x, h = u / p.lanes;
+    if (u >= units) continue;
+    const bool is_q = h < p.heads;
+    int d1, d2;
+    unit_of(p, u % p.lanes, d1, d2);
+    const T* w = is_q ? p.qw : p.kw;
+    finish_unit(p, row, h, d1, d2, a[i], b[i], is_q ? fq : fk, is_q ? p.norm_q : p.norm_k, w ? w + (size_t)(is_q ? h : h - p.heads) * p.hd : nullptr, cs, page, slot);
+  }
+  if (values_too(p)) write_values(p, t);
+}
+
+// Whether the kernels above take these sizes and addresses; sets ``lanes``.
+template <typename T>
+static bool kv_rows_take(KvRows<T>& p) {
+  constexpr int H = KvPiece<T>::H;
+  const int rot = p.form.rot;
+  if (p.hd % (2 * H) || p.vd % H || p.stride % H || (p.v_other && p.v_other_stride % H) || (p.v_keep && p.v_keep_stride % H)) return false;
+  p.lanes = p.hd / (2 * H);
+  if (p.lanes > NS_WAVE || (p.lanes & (p.lanes - 1))) return false;
+  if (rot && !p.form.interleaved && (rot / 2 % H || (p.hd - rot) % (2 * H))) return false;
+  if (((uintptr_t)p.qkv | (uintptr_t)p.bias | (uintptr_t)p.qw | (uintptr_t)p.kw | (uintptr_t)p.k_cache | (uintptr_t)p.v_other | (uintptr_t)p.v_keep) & 7) return false;
+  return p.kv_heads == 0 || ((uintptr_t)p.v_cache & 15) == 0;
+}
+
+#define FEW_TOKENS 256
+template <typename T>
+static dim3 kv_rows_grid(const KvRows<T>& p) { return dim3(p.n_tokens, p.shares + (p.kv_heads && p.n_tokens < FEW_TOKENS)); }
+
+template <typename T>
+static void launch_head_rows(KvRows<T> p, hipStream_t stream) {
+  const int units = (p.heads + p.kv_heads) * p.lanes;
+  p.shares = p.n_tokens < FEW_TOKENS ? (units + 255) / 256 : 1;
+  const int rounds = p.shares > 1 ? p.shares : (units + 511) / 512;  // (as even as whole waves allow)
+  int threads = ((units + rounds - 1) / rounds + NS_WAVE - 1) / NS_WAVE * NS_WAVE;
+  if (threads < 256 && p.kv_heads * p.vd > threads) threads = p.kv_heads * p.vd < 256 ? (p.kv_heads * p.vd + NS_WAVE - 1) / NS_WAVE * NS_WAVE : 256;
+  head_rows_kernel<T><<<kv_rows_grid(p), threads, p.form.rot * sizeof(float), stream>>>(p);
+}
+
+// ------------------------------------------------------------------------------------------------
 // What an attention layer without rotation does between its projections and its scores: the queries and keys of every
 // head are divided by their root mean square over the head (``eps`` >= 0; a negative eps leaves them as they are), the
 // queries in place; keys and values go into the pages of their positions.  A row of ``qkv`` is q [heads][hd], then, if
@@ -156,6 +409,17 @@ extern "C" int ns_unit_kv_write(void* qkv, int stride, const int* positions, con
                                 void* k_cache, void* v_cache, int n_tokens, int heads, int kv_heads, int hd, int vd, int page_size,
                                 float eps, int own_kv, int dtype, hipStream_t stream) {
   if (n_tokens <= 0 || heads <= 0 || kv_heads <= 0 || hd <= 0 || vd <= 0 || page_size <= 0) return NS_ERR_BAD_ARG;
+  auto in_pieces = [&](auto* rows, auto* k, auto* v) {
+    KvRows<typename std::remove_pointer<decltype(rows)>::type> p{};
+    p.qkv = rows, p.k_cache = k, p.v_cache = v, p.positions = positions, p.token_req = token_req, p.block_table = block_table;
+    p.stride = stride, p.table_stride = table_stride, p.n_tokens = n_tokens, p.heads = heads, p.kv_heads = own_kv ? kv_heads : 0, p.hd = hd, p.vd = vd, p.page_size = page_size;
+    p.eps = eps, p.norm_q = p.norm_k = eps >= 0.f;
+    if (!kv_rows_take(p)) return false;
+    if (own_kv || eps >= 0.f) launch_head_rows(p, stream);
+    return true;
+  };
+  if (dtype == NS_DTYPE_F32 ? in_pieces((float*)qkv, (float*)k_cache, (float*)v_cache) : dtype == NS_DTYPE_BF16 && in_pieces((bf16_t*)qkv, (bf16_t*)k_cache, (bf16_t*)v_cache))
+    return ns_launch_status();
   const int vec_blocks = (heads + (own_kv ? kv_heads : 0) + 3) / 4, copy_blocks = own_kv ? (kv_heads * vd + 1023) / 1024 : 0;
   if (vec_blocks + copy_blocks > 65535) return NS_ERR_BAD_ARG;
   const dim3 grid(n_tokens, vec_blocks + copy_blocks);
@@ -267,6 +531,23 @@ extern "C" int ns_whole_norm_kv_write(void* qkv, int stride, const void* bias, c
   if (n_tokens <= 0 || heads <= 0 || kv_heads <= 0 || hd <= 0 || vd <= 0 || page_size <= 0) return NS_ERR_BAD_ARG;
   if (rot < 0 || rot > hd || rot % 2 || (rot > 0 && !inv_freq)) return NS_ERR_BAD_ARG;
   const RopeForm form{rot, interleaved, factor};
+  auto in_pieces = [&](auto* rows) {
+    typedef typename std::remove_pointer<decltype(rows)>::type T;
+    KvRows<T> p{};
+    p.qkv = rows, p.bias = (const T*)bias, p.qw = (const T*)qw, p.kw = (const T*)kw, p.positions = positions, p.token_req = token_req, p.block_table = block_table;
+    p.inv_freq = inv_freq, p.k_cache = (T*)k_cache, p.v_cache = (T*)v_cache, p.stride = stride, p.table_stride = table_stride, p.n_tokens = n_tokens;
+    p.heads = heads, p.kv_heads = kv_heads, p.hd = hd, p.vd = vd, p.page_size = page_size, p.eps = eps, p.form = form, p.norm_q = qw != nullptr, p.norm_k = kw != nullptr;
+    p.lambda = (const T*)lambda, p.v_other = (const T*)v_other, p.v_keep = (T*)v_keep, p.v_other_stride = v_other_stride, p.v_keep_stride = v_keep_stride;
+    if (!kv_rows_take(p)) return false;
+    const int units = (heads + kv_heads) * p.lanes, each = (units + WHOLE_UNITS - 1) / WHOLE_UNITS;
+    if (each > 1024) return false;
+    // few tokens: a unit a thread, if there are threads
+    const int wanted = n_tokens <= 64 && units <= 1024 ? units : each;
+    p.shares = 1;
+    whole_rows_kernel<T><<<kv_rows_grid(p), (wanted + NS_WAVE - 1) / NS_WAVE * NS_WAVE, rot * sizeof(float), stream>>>(p);
+    return true;
+  };
+  if (dtype == NS_DTYPE_F32 ? in_pieces((float*)qkv) : dtype == NS_DTYPE_BF16 && in_pieces((bf16_t*)qkv)) return ns_launch_status();
   const int threads = n_tokens <= 64 && heads * hd > 1024 ? 1024 : 256;  // few tokens: more threads for each
   if (dtype == NS_DTYPE_F32)
     whole_norm_kv_write_kernel<float><<<n_tokens, threads, 0, stream>>>((float*)qkv, stride, (const float*)bias, (const float*)qw, (const float*)kw,
@@ -356,6 +637,18 @@ extern "C" int ns_head_norm_rope_kv_write(void* qkv, int stride, const void* bia
   if (v_is_k && vd != hd) return NS_ERR_BAD_ARG;
   if (rot > 0 && !inv_freq) return NS_ERR_BAD_ARG;
   const RopeForm form{rot, interleaved, factor};
+  auto in_pieces = [&](auto* rows) {
+    typedef typename std::remove_pointer<decltype(rows)>::type T;
+    KvRows<T> p{};
+    p.qkv = rows, p.bias = (const T*)bias, p.qw = (const T*)qw, p.kw = (const T*)kw, p.positions = positions, p.token_req = token_req, p.block_table = block_table;
+    p.inv_freq = inv_freq, p.k_cache = (T*)k_cache, p.v_cache = (T*)v_cache, p.stride = stride, p.table_stride = table_stride, p.n_tokens = n_tokens;
+    p.heads = heads, p.kv_heads = kv_heads, p.hd = hd, p.vd = vd, p.page_size = page_size, p.eps = eps, p.form = form, p.norm_q = qw != nullptr, p.norm_k = kw != nullptr;
+    p.v_is_k = v_is_k;
+    if (!kv_rows_take(p)) return false;
+    launch_head_rows(p, stream);
+    return true;
+  };
+  if (dtype == NS_DTYPE_F32 ? in_pieces((float*)qkv) : dtype == NS_DTYPE_BF16 && in_pieces((bf16_t*)qkv)) return ns_launch_status();
   // few tokens: a wave a head at once, over several workgroups a token
   const int shares = n_tokens >= 256 ? 1 : (heads + kv_heads + 3) / 4;
   if (n_tokens > 65535 * 32768 || shares > 65535) return NS_ERR_BAD_ARG;

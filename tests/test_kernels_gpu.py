@@ -159,6 +159,70 @@ def test_linear_split_beyond_the_parts(ranges):
     assert bool(((out.double() - ref).abs()[fine] <= bound[fine]).all())
 
 
+# (positions, requests) of a batch: runs that fill 16-byte runs of a page, begin and end inside one, stand out of order, repeat a place of the pad page
+KV_ORDERS = (([0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18], [0] * 19), ([5, 6, 7, 8, 9, 3, 4, 5], [0] * 5 + [1] * 3),
+             ([9, 8, 31, 30, 16, 17, 19, 20], [0, 0, 1, 1, 1, 1, 1, 1]), ([0, 0, 0, 12], [0, 0, 0, 1]), ([7], [1]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("order", range(len(KV_ORDERS)))
+@pytest.mark.parametrize("kind,H,G,D,E,page,rot,interleaved", [
+    ("unit", 5, 2, 64, 64, 16, 0, False), ("unit", 3, 1, 16, 40, 4, 0, False), ("unit", 4, 4, 512, 8, 32, 0, False), ("borrow", 6, 2, 32, 32, 16, 0, False),
+    ("bare", 2, 2, 128, 64, 8, 0, False), ("head", 6, 2, 64, 64, 16, 64, False), ("head", 3, 3, 128, 64, 8, 64, False), ("head", 2, 1, 64, 24, 32, 30, True),
+    ("head", 5, 1, 16, 16, 6, 16, True), ("same", 4, 2, 32, 32, 16, 16, False), ("whole", 32, 8, 64, 64, 16, 64, False), ("whole", 3, 1, 64, 128, 16, 32, True),
+    ("mixed", 5, 2, 32, 64, 4, 0, False), ("whole", 70, 20, 128, 64, 16, 128, False)])
+def test_keys_and_values_in_pieces(dtype, order, kind, H, G, D, E, page, rot, interleaved):
+    """Norm, rotation and write of keys and values in pieces of 8 bytes against the plain kernels, which take the same rows an odd number of values apart."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(H * D + order)
+    pos, req = (torch.tensor(a, dtype=torch.int32, device=DEV) for a in KV_ORDERS[order])
+    n, own, same = len(pos), kind != "borrow", kind == "same"
+    width = H * D + (G * (D + (0 if same else E)) if own else 0)
+    make = lambda *shape: (2.0 * torch.randn(*shape, generator=g)).to(dtype).to(DEV)
+    rows, bias, other = make(n, width), make(width), make(n, G * E)
+    per = 1 if kind in ("head", "same") else H
+    qw, kw = make(per * D), make((1 if per == 1 else G) * D)
+    inv = torch.rand(max(1, rot // 2), generator=g).to(DEV)
+    pages = 1 + 33 // page
+    table = torch.randperm(2 * pages, generator=g).to(torch.int32).view(2, pages).to(DEV)
+    mix = torch.full((1,), 0.375, dtype=dtype, device=DEV)
+    got = []
+    for extra in (0, 3):  # (rows of whole pieces; three columns more)
+        wide = torch.full((n, width + 8 * (extra > 0) + extra), 5.0, dtype=dtype, device=DEV)
+        wide[:, :width] = rows
+        kc, vc = torch.zeros(2 * pages, G, page, D, dtype=dtype, device=DEV), torch.zeros(2 * pages, G, E, page, dtype=dtype, device=DEV)
+        keep = torch.zeros(n, G * E, dtype=dtype, device=DEV)
+        x = wide[:, : wide.shape[1] - extra] if extra else wide
+        if kind in ("unit", "borrow", "bare"):
+            ops.unit_kv_write(x, pos, req, table, kc, vc, H, G, D, E, None if kind == "bare" else 1e-3, own_kv=own)
+        elif kind in ("head", "same"):
+            ops.head_norm_rope_kv_write(x, pos, req, table, inv[: rot // 2], kc, vc, H, G, D, E, 1e-3, rot, bias=bias, q_weight=qw, k_weight=None if E == 24 else kw,
+                                        value_is_key=same, interleaved=interleaved, factor=1.25)
+        else:
+            mixed = dict(mix=mix, v_other=other, v_keep=keep) if kind == "mixed" else {}
+            ops.whole_norm_kv_write(x, pos, req, table, kc, vc, H, G, D, E, 1e-3, bias=bias, q_weight=qw, k_weight=None if E == 128 else kw, inv_freq=inv, rotary_dim=rot,
+                                    interleaved=interleaved, **mixed)
+        got.append((wide[:, :width], kc, vc, keep))
+    # the sums of squares are in another order, and a channel is then a product of three: a few units of 2^-24 before it is rounded
+    tol = dict(rtol=2.0**-19, atol=2.0**-18) if dtype == torch.float32 else dict(rtol=2.0**-7, atol=2.0**-8)
+    last = {(int(r), int(p)): i for i, (r, p) in enumerate(zip(req, pos))}  # (a place that several tokens write keeps any of them)
+    once = [i for (r, p), i in last.items() if sum(int(a) == r and int(b) == p for a, b in zip(req, pos)) == 1]
+    # values are the same bit by bit; of two mixed values (1 - m) a + m b one product is rounded ahead of the sum, which one the compiler chooses: 2^-24 of it
+    # (at most 0.625 times a number below 16), and a bfloat16 result may then round the other way
+    alike = torch.equal if kind != "mixed" else lambda a, b: torch.allclose(a, b, rtol=0 if dtype == torch.float32 else 2.0**-7, atol=2.0**-20)
+    assert torch.allclose(got[0][0], got[1][0], **tol) and alike(got[0][3], got[1][3])
+    for i in once:
+        at = int(table[req[i], pos[i] // page]), int(pos[i]) % page
+        assert torch.allclose(got[0][1][at[0], :, at[1]], got[1][1][at[0], :, at[1]], **tol)
+        assert alike(got[0][2][at[0], :, :, at[1]], got[1][2][at[0], :, :, at[1]])
+    if order != 3 and own:
+        written = sorted((int(table[r, p // page]), p % page) for r, p in last)
+        blank = torch.ones(2 * pages, page, dtype=torch.bool)
+        for a, b in written:
+            blank[a, b] = False
+        assert bool((got[0][1].cpu().transpose(1, 2)[blank] == 0).all()) and bool((got[0][2].cpu().permute(0, 3, 1, 2)[blank] == 0).all())
+
+
 def test_split_plan():
     """What goes to the split kernel: whole stages, enough tiles; every plan is one that the launch takes."""
     from nanospec_amd.kernels import ops

@@ -10,6 +10,7 @@
 //
 // A request's slot holds S [H][D][E] and behind it the last K - 1 inputs of the convolution [K - 1][C] (oldest first).
 #include "chunk16.h"
+#include <type_traits>
 
 #define ND_MAX_TAPS 16
 #define ND_ROWS 16  // key channels of a column that one thread owns
@@ -45,57 +46,107 @@ __global__ void conv_silu_kernel(float* __restrict__ out, T* __restrict__ copy, 
 }
 
 // The same for four neighbouring channels a thread, with 16-byte accesses to taps, carried inputs and results, for the
-// usual numbers of taps (so that the taps are registers) and channels that are a multiple of four.
-template <typename T, int K>
-__global__ void conv_silu_vec_kernel(float* __restrict__ out, T* __restrict__ copy, const T* __restrict__ x, int x_stride,
+// usual numbers of taps (so that the taps are registers) and channels that are a multiple of four.  A thread takes STRIP tokens one after the other: taps are
+// 64 bytes a thread and an input is read by K tokens, for 8 bytes of new input and 16 of result.  UNITS: the first ``vectors`` runs of 4 LANES channels then become unit
+// vectors, as delta_prep_kernel makes them, while their sums of squares are at hand (C a multiple of 4 LANES): as a kernel of its own that reads and writes them again.
+// Bound by the results' bytes: 2,048 tokens of 6,144 channels, 4 taps, bfloat16, a token a thread 35.0 / 27.2 us (alone / beside two
+// others) and the unit vectors and decays behind it 38.3 / 31.8, both in a row 69.1 / 57.4; so 30.6 / 19.8 and (decays alone) 18.7 / 14.3, 46.3 / 31.5.  Strips of four or two: level.
+template <int LANES>
+__device__ __forceinline__ float unit_scale(const float* y, bool first_half) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss = fmaf(y[e], y[e], ss);
+  return (first_half ? 1.f / sqrtf(4.f * LANES) : 1.f) / sqrtf(group_sum<LANES>(ss) + 1e-6f);
+}
+
+struct ConvUnits {
+  int vectors, lanes;  // (lanes: of a vector, a power of two)
+};
+
+template <typename T, int K, int STRIP>
+__global__ __launch_bounds__(256) void conv_silu_vec_kernel(float* __restrict__ out, T* __restrict__ copy, const T* __restrict__ x, int x_stride,
                                      const float* __restrict__ taps, const float* __restrict__ bias, float* __restrict__ state, size_t slot_stride, size_t conv_off, const int* __restrict__ token_req,
-                                     const int* __restrict__ qo_indptr, const int* __restrict__ state_slots, int C, int carry) {
+                                     const int* __restrict__ qo_indptr, const int* __restrict__ state_slots, int n, int C, int carry, ConvUnits units) {
   typedef T vec_t __attribute__((ext_vector_type(4)));
-  const int r = blockIdx.x, c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  const int r0 = blockIdx.x * STRIP, c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
   if (c >= C) return;
-  const int b = token_req[r];
-  const int i = r - qo_indptr[b];
-  float* carried = state + (size_t)state_slots[b] * slot_stride + conv_off;
+  // (all loads of the strip's inputs ahead of the first use; beyond the last token the last)
+  vec_t in[STRIP];
+#pragma unroll
+  for (int s = 0; s < STRIP; ++s) in[s] = *reinterpret_cast<const vec_t*>(x + (size_t)min(r0 + s, n - 1) * x_stride + c);
   float tp[4 * K];  // taps of channel c + e / K, tap e % K
 #pragma unroll
   for (int e = 0; e < K; ++e) {
     const float4 t = reinterpret_cast<const float4*>(taps + (size_t)c * K)[e];
     tp[4 * e] = t.x, tp[4 * e + 1] = t.y, tp[4 * e + 2] = t.z, tp[4 * e + 3] = t.w;
   }
-  float y[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias) {
-    const float4 bv = *reinterpret_cast<const float4*>(bias + c);
-    y[0] = bv.x, y[1] = bv.y, y[2] = bv.z, y[3] = bv.w;
-  }
+  float4 bv = {0.f, 0.f, 0.f, 0.f};
+  if (bias) bv = *reinterpret_cast<const float4*>(bias + c);
+  float before[K - 1][4];  // the inputs before the token, oldest first
+  int req = -1;
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const int t = i - (K - 1) + j;
-    float v[4];
-    if (t >= 0) {
-      const vec_t xv = *reinterpret_cast<const vec_t*>(x + (size_t)(r - (K - 1) + j) * x_stride + c);
+  for (int s = 0; s < STRIP; ++s) {
+    const int r = r0 + s;
+    if (r >= n) break;
+    const int b = token_req[r];
+    float* carried = state + (size_t)state_slots[b] * slot_stride + conv_off;
+    if (b != req) {  // (the strip's first token, or a request's; the same for the whole workgroup)
+      const int i = r - qo_indptr[b];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = to_f(xv[e]);
-    } else {
-      const float4 cv = *reinterpret_cast<const float4*>(carried + (size_t)(K - 1 + t) * C + c);
-      v[0] = cv.x, v[1] = cv.y, v[2] = cv.z, v[3] = cv.w;
+      for (int j = 0; j < K - 1; ++j) {
+        const int t = i - (K - 1) + j;
+        if (t >= 0) {
+          const vec_t xv = *reinterpret_cast<const vec_t*>(x + (size_t)(r - (K - 1) + j) * x_stride + c);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) before[j][e] = to_f((T)xv[e]);
+        } else {
+          const float4 cv = *reinterpret_cast<const float4*>(carried + (size_t)(K - 1 + t) * C + c);
+          before[j][0] = cv.x, before[j][1] = cv.y, before[j][2] = cv.z, before[j][3] = cv.w;
+        }
+      }
+      req = b;
+    }
+    float y[4] = {bv.x, bv.y, bv.z, bv.w}, now[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      now[e] = to_f((T)in[s][e]);
+#pragma unroll
+      for (int j = 0; j < K - 1; ++j) y[e] = fmaf(tp[e * K + j], before[j][e], y[e]);
+      y[e] = fmaf(tp[e * K + K - 1], now[e], y[e]);
+    }
+    if (carry && qo_indptr[b + 1] - qo_indptr[b] == 1) {
+#pragma unroll
+      for (int j = 0; j + 1 < K; ++j) {
+        const float* v = j + 2 < K ? before[j + 1 < K - 1 ? j + 1 : 0] : now;
+        *reinterpret_cast<float4*>(carried + (size_t)j * C + c) = make_float4(v[0], v[1], v[2], v[3]);
+      }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = fmaf(tp[e * K + j], v[e], y[e]);
-  }
-  if (carry && qo_indptr[b + 1] - qo_indptr[b] == 1) {
-#pragma unroll
     for (int j = 0; j + 2 < K; ++j)
-      *reinterpret_cast<float4*>(carried + (size_t)j * C + c) = *reinterpret_cast<const float4*>(carried + (size_t)(j + 1) * C + c);
-    const vec_t xv = *reinterpret_cast<const vec_t*>(x + (size_t)r * x_stride + c);
-    *reinterpret_cast<float4*>(carried + (size_t)(K - 2) * C + c) = make_float4(to_f(xv[0]), to_f(xv[1]), to_f(xv[2]), to_f(xv[3]));
-  }
-  float4 res;
-  res.x = y[0] / (1.f + expf(-y[0])), res.y = y[1] / (1.f + expf(-y[1]));
-  res.z = y[2] / (1.f + expf(-y[2])), res.w = y[3] / (1.f + expf(-y[3]));
-  *reinterpret_cast<float4*>(out + (size_t)r * C + c) = res;
-  if (copy) {
-    const vec_t cv = {from_f<T>(res.x), from_f<T>(res.y), from_f<T>(res.z), from_f<T>(res.w)};
-    *reinterpret_cast<vec_t*>(copy + (size_t)r * C + c) = cv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) before[j][e] = before[j + 1][e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) before[K - 2][e] = now[e], y[e] = y[e] / (1.f + expf(-y[e]));
+    const int vector = units.vectors ? c / (4 * units.lanes) : 0;
+    if (vector < units.vectors) {
+      const bool first = vector < units.vectors / 2;
+      float f;
+      switch (units.lanes) {
+        case 2: f = unit_scale<2>(y, first); break;
+        case 4: f = unit_scale<4>(y, first); break;
+        case 8: f = unit_scale<8>(y, first); break;
+        case 16: f = unit_scale<16>(y, first); break;
+        case 32: f = unit_scale<32>(y, first); break;
+        default: f = unit_scale<64>(y, first);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] *= f;
+    }
+    *reinterpret_cast<float4*>(out + (size_t)r * C + c) = make_float4(y[0], y[1], y[2], y[3]);
+    if (copy) {
+      const vec_t cv = {from_f<T>(y[0]), from_f<T>(y[1]), from_f<T>(y[2]), from_f<T>(y[3])};
+      *reinterpret_cast<vec_t*>(copy + (size_t)r * C + c) = cv;
+    }
   }
 }
 
@@ -116,11 +167,16 @@ __global__ void conv_carry_kernel(const T* __restrict__ x, int x_stride, float* 
   }
 }
 
-// ``single``: every request brings one token (at most); one kernel then does both
+#define CONV_STRIP 8
+#define CONV_STRIP_TOKENS 512  // from so many on (fewer would leave too few workgroups)
+
+// ``single``: every request brings one token (at most); one kernel then does both.  ``unit_vectors`` (an even number, or 0): so many first runs of ``unit_size`` channels become unit
+// vectors, the first half of them times unit_size^(-1/2); unit_size a power of two from 8 to 256, and sizes and addresses as the kernel in pieces wants them (NS_ERR_UNSUPPORTED).
 extern "C" int ns_conv_silu_carry(float* out, void* copy, const void* x, int x_stride, const float* taps, const float* bias, float* state, size_t slot_stride,
                                   size_t conv_off, const int* token_req, const int* qo_indptr, const int* state_slots, int n_tokens,
-                                  int n_reqs, int C, int K, int single, int dtype, hipStream_t stream) {
-  if (n_tokens <= 0 || n_reqs <= 0 || n_reqs > 65535 || C <= 0 || K < 1 || K > ND_MAX_TAPS) return NS_ERR_BAD_ARG;
+                                  int n_reqs, int C, int K, int single, int unit_vectors, int unit_size, int dtype, hipStream_t stream) {
+  if (n_tokens <= 0 || n_reqs <= 0 || n_reqs > 65535 || C <= 0 || K < 1 || K > ND_MAX_TAPS || unit_vectors < 0 || unit_vectors % 2) return NS_ERR_BAD_ARG;
+  if (unit_vectors && (unit_size <= 0 || (long long)unit_vectors * unit_size > C)) return NS_ERR_BAD_ARG;
   if (dtype != NS_DTYPE_F32 && dtype != NS_DTYPE_BF16) return NS_ERR_UNSUPPORTED;
   const int bx = (C + 255) / 256;
   if (bx > 65535) return NS_ERR_BAD_ARG;
@@ -128,23 +184,34 @@ extern "C" int ns_conv_silu_carry(float* out, void* copy, const void* x, int x_s
   const bool vec = C % 4 == 0 && x_stride % 4 == 0 && ((uintptr_t)x % (4 * esize)) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)taps % 16) == 0 &&
                    ((uintptr_t)bias % 16) == 0 && ((uintptr_t)copy % (4 * esize)) == 0 &&
                    ((uintptr_t)state % 16) == 0 && slot_stride % 4 == 0 && conv_off % 4 == 0 && K >= 2 && K <= 4;
+  if (unit_vectors && !(vec && unit_size >= 8 && unit_size <= 256 && (unit_size & (unit_size - 1)) == 0)) return NS_ERR_UNSUPPORTED;
   if (vec) {
-    dim3 grid(n_tokens, (C / 4 + 255) / 256);
-#define ND_CONV(KK)                                                                                                                         \
-  case KK:                                                                                                                                  \
-    if (dtype == NS_DTYPE_F32)                                                                                                              \
-      conv_silu_vec_kernel<float, KK><<<grid, 256, 0, stream>>>(out, (float*)copy, (const float*)x, x_stride, taps, bias, state, slot_stride, conv_off, token_req, \
-                                                                qo_indptr, state_slots, C, single);                                        \
-    else                                                                                                                                    \
-      conv_silu_vec_kernel<bf16_t, KK><<<grid, 256, 0, stream>>>(out, (bf16_t*)copy, (const bf16_t*)x, x_stride, taps, bias, state, slot_stride, conv_off, token_req, \
-                                                                 qo_indptr, state_slots, C, single);                                       \
-    break
-    switch (K) {
-      ND_CONV(2);
-      ND_CONV(3);
-      default: ND_CONV(4);
-    }
-#undef ND_CONV
+    const ConvUnits units{unit_vectors, unit_vectors ? unit_size / 4 : 1};
+    const bool strips = n_tokens >= CONV_STRIP_TOKENS && !single;
+    const dim3 grid(strips ? (n_tokens + CONV_STRIP - 1) / CONV_STRIP : n_tokens, (C / 4 + 255) / 256);
+    auto launch = [&](auto* in, auto taps_of, auto strip) {
+      typedef typename std::remove_const<typename std::remove_pointer<decltype(in)>::type>::type T;
+      conv_silu_vec_kernel<T, decltype(taps_of)::value, decltype(strip)::value><<<grid, 256, 0, stream>>>(
+          out, (T*)copy, in, x_stride, taps, bias, state, slot_stride, conv_off, token_req, qo_indptr, state_slots, n_tokens, C, single, units);
+    };
+    auto of_taps = [&](auto* in, auto strip) {
+      if (K == 2)
+        launch(in, std::integral_constant<int, 2>(), strip);
+      else if (K == 3)
+        launch(in, std::integral_constant<int, 3>(), strip);
+      else
+        launch(in, std::integral_constant<int, 4>(), strip);
+    };
+    auto of_strip = [&](auto* in) {
+      if (strips)
+        of_taps(in, std::integral_constant<int, CONV_STRIP>());
+      else
+        of_taps(in, std::integral_constant<int, 1>());
+    };
+    if (dtype == NS_DTYPE_F32)
+      of_strip((const float*)x);
+    else
+      of_strip((const bf16_t*)x);
   } else {
     dim3 grid(n_tokens, bx);
     if (dtype == NS_DTYPE_F32)
@@ -195,10 +262,41 @@ __global__ void delta_prep_kernel(float* __restrict__ qkv, int C, float* __restr
     for (int h = threadIdx.x; h < H; h += blockDim.x) beta[(size_t)r * H + h] = 1.f / (1.f + expf(-to_f(bp[(size_t)r * b_stride + h])));
 }
 
+// The decays and write strengths alone, four decays a thread, where the unit vectors have been made already.  Sizes and strides multiples of four, whole pieces.
+template <typename T>
+__global__ __launch_bounds__(256) void delta_decay_kernel(float* __restrict__ g, float* __restrict__ beta, const T* __restrict__ a, int a_stride, const T* __restrict__ bp,
+                                                          int b_stride, const float* __restrict__ dt_bias, const float* __restrict__ a_log, int H, int D) {
+  typedef T vec_t __attribute__((ext_vector_type(4)));
+  const int r = blockIdx.x, i = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (i < H * D) {
+    const vec_t av = *reinterpret_cast<const vec_t*>(a + (size_t)r * a_stride + i);
+    const float4 dv = *reinterpret_cast<const float4*>(dt_bias + i);
+    const float rate = -expf(a_log[i / D]), dt[4] = {dv.x, dv.y, dv.z, dv.w};
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = expf(rate * softplus_f(to_f((T)av[e]) + dt[e]));
+    *reinterpret_cast<float4*>(g + (size_t)r * H * D + i) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  if (blockIdx.y == 0)
+    for (int h = threadIdx.x; h < H; h += 256) beta[(size_t)r * H + h] = 1.f / (1.f + expf(-to_f(bp[(size_t)r * b_stride + h])));
+}
+
+// ``units_made``: q and k are unit vectors already.
 extern "C" int ns_delta_prep(float* qkv, int C, float* g, float* beta, const void* a, int a_stride, const void* bp, int b_stride,
-                             const float* dt_bias, const float* a_log, int n_tokens, int H, int G, int D, int dtype, hipStream_t stream) {
+                             const float* dt_bias, const float* a_log, int n_tokens, int H, int G, int D, int units_made, int dtype, hipStream_t stream) {
   if (n_tokens <= 0 || H <= 0 || G <= 0 || H % G || D <= 0 || C < 2 * G * D) return NS_ERR_BAD_ARG;
-  const int norm_blocks = (2 * G + 3) / 4, decay_blocks = (H * D + 1023) / 1024;
+  const size_t piece = dtype == NS_DTYPE_F32 ? 16 : 8;
+  if (units_made && D % 4 == 0 && a_stride % 4 == 0 && (uintptr_t)a % piece == 0 && (((uintptr_t)g | (uintptr_t)dt_bias) & 15) == 0 &&
+      (dtype == NS_DTYPE_F32 || dtype == NS_DTYPE_BF16)) {
+    const dim3 grid(n_tokens, (H * D / 4 + 255) / 256);
+    if (grid.y > 65535) return NS_ERR_BAD_ARG;
+    if (dtype == NS_DTYPE_F32)
+      delta_decay_kernel<float><<<grid, 256, 0, stream>>>(g, beta, (const float*)a, a_stride, (const float*)bp, b_stride, dt_bias, a_log, H, D);
+    else
+      delta_decay_kernel<bf16_t><<<grid, 256, 0, stream>>>(g, beta, (const bf16_t*)a, a_stride, (const bf16_t*)bp, b_stride, dt_bias, a_log, H, D);
+    return ns_launch_status();
+  }
+  const int norm_blocks = units_made ? 0 : (2 * G + 3) / 4, decay_blocks = (H * D + 1023) / 1024;
   if (norm_blocks + decay_blocks > 65535) return NS_ERR_BAD_ARG;
   const dim3 grid(n_tokens, norm_blocks + decay_blocks);
   if (dtype == NS_DTYPE_F32)

@@ -2104,13 +2104,15 @@ def _state_args(state: torch.Tensor, what: str):
 
 
 def conv_silu_carry(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, conv_off: int, token_req, qo_indptr, state_slots,
-                    out: torch.Tensor, bias: torch.Tensor | None = None, copy: torch.Tensor | None = None, single: bool = False) -> torch.Tensor:
+                    out: torch.Tensor, bias: torch.Tensor | None = None, copy: torch.Tensor | None = None, single: bool = False,
+                    unit: tuple[int, int] | None = None) -> torch.Tensor:
     """A short causal convolution over time per channel (plus ``bias`` float32 [C]), then SiLU, across steps.  ``x`` [tokens, >= C]
     (its first C columns are convolved), ``taps`` float32 [C, K] whose last column multiplies the current token; the K - 1
     inputs before a request's first token of this step are read from ``state[slot, conv_off:]`` as [K - 1, C] (zeros for a new
     request) and replaced afterwards by the last K - 1 inputs including this step's.  ``out`` float32 [tokens, C]; ``copy``
     [tokens, C] receives the same values in the dtype of ``x``.  ``single``: the caller knows that every request brings at most
-    one token (one kernel then does what two do otherwise)."""
+    one token (one kernel then does what two do otherwise).  ``unit`` (vectors, size): the first ``vectors`` (an even number) runs of
+    ``size`` channels then become unit vectors, as ``delta_prep`` makes them of q and k (``conv_units_take`` says where)."""
     _gpu(x), _f32(taps, "taps"), _f32(out, "out")
     for name, t in (("token_req", token_req), ("qo_indptr", qo_indptr), ("state_slots", state_slots)):
         _i32(t, name)
@@ -2127,13 +2129,21 @@ def conv_silu_carry(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, co
     sp, stride = _state_args(state, "conv_silu_carry")
     _check(build.core().ns_conv_silu_carry(_ptr(out), _ptr(copy), _ptr(x), c_int(x.stride(0)), _ptr(taps), _ptr(bias), sp, stride, c_size_t(conv_off),
                                            _ptr(token_req), _ptr(qo_indptr), _ptr(state_slots), c_int(n), c_int(reqs), c_int(C), c_int(K),
-                                           c_int(1 if single else 0), c_int(_dtype_code(x)), _stream()), "conv_silu_carry")
+                                           c_int(1 if single else 0), c_int(unit[0] if unit else 0), c_int(unit[1] if unit else 0),
+                                           c_int(_dtype_code(x)), _stream()), "conv_silu_carry")
     return out
 
 
+def conv_units_take(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, conv_off: int, size: int) -> bool:
+    """Whether ``conv_silu_carry`` can make unit vectors of runs of ``size`` channels: a power of two from 8 to 256, two to four taps, whole pieces of four channels."""
+    C, K = taps.shape
+    return (2 <= K <= 4 and 8 <= size <= 256 and size & (size - 1) == 0 and C % 4 == 0 and x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0
+            and taps.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0 and state.stride(0) % 4 == 0 and conv_off % 4 == 0)
+
+
 def delta_prep(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, heads: int, kv_heads: int,
-               key_dim: int, g: torch.Tensor, beta: torch.Tensor) -> None:
-    """What the delta rule's recurrence reads, in 32-bit.  In place in ``qkv`` (float32 [tokens, C], q [kv_heads, key_dim]
+               key_dim: int, g: torch.Tensor, beta: torch.Tensor, units_made: bool = False) -> None:
+    """What the delta rule's recurrence reads, in 32-bit (``units_made``: q and k are as they are wanted already).  In place in ``qkv`` (float32 [tokens, C], q [kv_heads, key_dim]
     then k alike then v): q and k of every head become x / sqrt(sum(x^2) + 1e-6), q times key_dim^(-1/2).
     g[t, h, d] = exp(-exp(a_log[h]) * softplus(a[t, h, d] + dt_bias[h, d])); beta[t, h] = sigmoid(b[t, h]).
     ``a`` [tokens, >= heads * key_dim] and ``b`` [tokens, >= heads] may be column slices of wider tensors."""
@@ -2146,7 +2156,7 @@ def delta_prep(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, dt_bias: tor
         raise KernelRefused("delta_prep: operands do not fit heads and key size")
     _check(build.core().ns_delta_prep(_ptr(qkv), c_int(qkv.shape[1]), _ptr(g), _ptr(beta), _ptr(a), c_int(a.stride(0)), _ptr(b),
                                       c_int(b.stride(0)), _ptr(dt_bias), _ptr(a_log), c_int(n), c_int(heads), c_int(kv_heads), c_int(key_dim),
-                                      c_int(_dtype_code(a)), _stream()), "delta_prep")
+                                      c_int(1 if units_made else 0), c_int(_dtype_code(a)), _stream()), "delta_prep")
 
 
 def delta_scan(qkv: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, qo_indptr, state_slots, heads: int,

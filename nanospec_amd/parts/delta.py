@@ -112,10 +112,11 @@ class ChannelDelta:
         state = cache.state
         proj = self.w_in(x, out=take((n, self.w_in.n), x.dtype), arena=ctx.arena, plain_copy=not ctx.captured)
         thin = self.w_thin(proj[:, self.thin_at : self.b_at], out=take((n, self.w_thin.n), x.dtype), arena=ctx.arena)
+        units = ops.conv_units_take(proj, self.taps, state, self.state_floats, D)  # the convolution then leaves q and k as unit vectors
         qkv = ops.conv_silu_carry(proj, self.taps, state, self.state_floats, ctx.token_req, ctx.qo_indptr, ctx.state_slots,
-                                  out=take((n, self.channels), torch.float32), single=getattr(ctx, "single_tokens", False))
+                                  out=take((n, self.channels), torch.float32), single=getattr(ctx, "single_tokens", False), unit=(2 * G, D) if units else None)
         g, beta = take((n, H * D), torch.float32), take((n, H), torch.float32)
-        ops.delta_prep(qkv, thin, proj[:, self.b_at :], self.dt_bias, self.a_log, H, G, D, g, beta)
+        ops.delta_prep(qkv, thin, proj[:, self.b_at :], self.dt_bias, self.a_log, H, G, D, g, beta, units_made=units)
         indptr, slots = getattr(ctx, "spans", (ctx.qo_indptr, ctx.state_slots))
         o = ops.delta_scan(qkv, g, beta, state, indptr, slots, H, G, D, E, out=take((n, H * E), torch.float32), take=take,
                            longest=getattr(ctx, "longest", None), portions=getattr(ctx, "portions", None))

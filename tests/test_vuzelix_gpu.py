@@ -433,6 +433,53 @@ def test_convolution_carries_its_inputs_across_steps(K, C, pad, off):
     assert (state[:, :off] == 7.0).all() and (state[0] == torch.cat([torch.full((off,), 7.0), torch.zeros((K - 1) * C)]).to(DEV)).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("vectors,size,rest", [(2, 8, 4), (4, 128, 60), (2, 256, 8), (6, 16, 1000), (2, 32, 0)])
+def test_convolution_in_strips_with_unit_vectors(dtype, K, vectors, size, rest):
+    """Strips of eight tokens that requests begin and end inside of, a request shorter than the taps, a last strip that is not full, and a step too short for strips; unit vectors
+    made of the first channels behind it; then the decays alone."""
+    from nanospec_amd.kernels import ops
+
+    torch.manual_seed(K + size)
+    C, off = vectors * size + rest, 12
+    taps = torch.randn(C, K)
+    state = torch.zeros(6, off + (K - 1) * C, device=DEV)
+    lens, order = [1, 2, 300, 7, 211], [4, 0, 2, 5, 1]
+    xs = [(2.0 * torch.randn(2 * n, C + 4)).to(dtype) for n in lens]
+    outs, copies, done = [[] for _ in lens], [[] for _ in lens], [0] * len(lens)
+    for step in (lens, [min(5, n) for n in lens]):
+        x = torch.cat([xs[b][done[b] : done[b] + n] for b, n in enumerate(step)]).to(DEV)
+        req, indptr, slots = batch(step, order)
+        assert ops.conv_units_take(x, taps.to(DEV), state, off, size)
+        copy = torch.empty(len(x), C, dtype=dtype, device=DEV)
+        out = ops.conv_silu_carry(x, taps.to(DEV), state, off, req, indptr, slots, out=torch.empty(len(x), C, device=DEV), copy=copy, unit=(vectors, size))
+        at = 0
+        for b, n in enumerate(step):
+            outs[b].append(out[at : at + n].cpu())
+            copies[b].append(copy[at : at + n].cpu())
+            at += n
+            done[b] += n
+    for b, n in enumerate(done):
+        y = pv.causal_conv_silu(xs[b][:n, :C].double(), taps.double())
+        v = y[:, : vectors * size].view(n, vectors, size)
+        unit = v / torch.sqrt((v * v).sum(-1, keepdim=True) + 1e-6)
+        unit[:, : vectors // 2] *= size**-0.5
+        y = torch.cat([unit.flatten(1), y[:, vectors * size :]], 1)
+        torch.testing.assert_close(torch.cat(outs[b]).double(), y, rtol=1e-5, atol=1e-5)
+        assert torch.equal(torch.cat(copies[b]), torch.cat(outs[b]).to(dtype))
+    H, D, n = 3, 20, 9
+    a, bp = torch.randn(n, H * D + 4).to(dtype).to(DEV), torch.randn(n, H).to(dtype).to(DEV)
+    dt_bias, a_log = torch.randn(H * D, device=DEV), torch.log(torch.rand(H, device=DEV) * 0.5 + 0.01)
+    qkv = torch.randn(n, 2 * H * D, device=DEV)
+    made = [(torch.empty(n, H * D, device=DEV), torch.empty(n, H, device=DEV)) for _ in range(2)]
+    before = qkv.clone()
+    ops.delta_prep(qkv, a, bp, dt_bias, a_log, H, H, D, *made[0], units_made=True)
+    assert torch.equal(qkv, before)
+    ops.delta_prep(qkv, a, bp, dt_bias, a_log, H, H, D, *made[1])
+    assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
+
+
 @pytest.mark.parametrize("H,G,D,E", [(4, 2, 24, 40), (2, 2, 64, 20), (1, 1, 128, 128), (6, 3, 8, 72), (3, 1, 144, 16)])
 def test_delta_rule_across_steps(H, G, D, E):
     """Unit vectors, decays, write strengths and the recurrence against the plain loop: two requests of unequal length in

@@ -271,32 +271,35 @@ def linear_generic(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = 
     return out
 
 
-# ``linear_split``: rows of x a tile (by 128 rows of w) and what a row of each takes over one of the largest (2,048 rows of 16,384 x 2,048)
-SPLIT_TILES = ((128, 1.0), (112, 1.035), (96, 1.03), (64, 1.2))
+# ``linear_split``: rows of x a tile (by 128 rows of w) and what a row of each takes over one of the largest (2,048 rows of 28,672 x 4,096)
+SPLIT_TILES = ((128, 1.0), (112, 1.035), (96, 1.055), (64, 1.12))
 SPLIT_COLUMNS = 128
 SPLIT_K_MULTIPLE = 32
 SPLIT_MIN_ROWS = 48
 SPLIT_MIN_K = 1024
-SPLIT_MIN_WORK = 3e9  # rows times columns times K
-SPLIT_CHUNK_ROWS = 4096  # more are taken in portions, so that the parts of x take no more than 24 KB for each of its columns
+SPLIT_LONG_K = 4096  # from here on ranges of K are worth their sum until the units have one and a half tiles each
+SPLIT_MIN_WORK = 2e9  # rows times columns times K
+SPLIT_CHUNK_ROWS = 4096  # more are taken in portions, so that the parts of x take no more than 17 KB for each of its columns
 
 
 @functools.lru_cache(maxsize=1 << 14)
 def split_plan(m: int, n: int, k: int, units: int) -> tuple[int, int] | None:
     """(rows of a tile, ranges of K) for ``linear_split``, or None where ``linear_generic`` is the faster one or the sizes are not taken.
 
-    Ranges fill the units where the tiles do not: 777 rows, N 2,048, K 8,192 one, two, four 388 / 198, 201 / 135, 171 / 133 us (alone / beside two others), N 3,072, K 2,048 one,
-    two, four 110 / 59, 89 / 53, 77 / 56.  Below ``SPLIT_MIN_WORK`` products the splitting of x and the sum of the ranges cost alone what the product gains: its time over
-    linear_generic's, 48 to 2,048 rows, median (largest), alone / beside: 1 to 2e9 1.18 (1.33) / 0.95 (1.07), 2 to 3e9 0.96 (1.25) / 0.78 (0.95), 3 to 6e9 0.96 (1.21) / 0.67 (0.78),
-    from 6e9 on 0.71 (1.11) / 0.61 (0.80)."""
-    if m < SPLIT_MIN_ROWS or k < SPLIT_MIN_K or k % SPLIT_K_MULTIPLE or k >= 1 << 21 or m * n * k < SPLIT_MIN_WORK:
+    Ranges fill the units where the tiles do not, for a sum of them and the tiles' beginnings again.  us alone / beside two others: 832 rows, N 2,048, K 8,192, tiles of 128 rows
+    in one, two, four 237 / 135, 152 / 100, 122 / 102; N 3,072, K 2,048, 96 rows 66 / 35, 65 / 43, 79 / 51; N = K = 2,048, 64 rows 52 / 26, 54 / 31, 57 / 36.  Below
+    ``SPLIT_MIN_WORK`` the splitting of x and a sum of ranges cost alone what the product gains, its time over linear_generic's alone / beside: 1.1 to 1.4e9 (five sizes)
+    1.04 to 1.25 / 0.94 to 1.46, 1.7e9 0.93 / 0.73, 2 to 3e9 (four) 0.71 to 0.97 / 0.66 to 0.94, 3 to 7e9 (fourteen) 0.58 to 1.01 / 0.33 to 0.59, larger 0.40 to 0.70 / 0.31 to 0.53."""
+    if m < SPLIT_MIN_ROWS or k < SPLIT_MIN_K or k % SPLIT_K_MULTIPLE or k >= 1 << 19 or m * n * k < SPLIT_MIN_WORK:
         return None
     m, columns = min(m, SPLIT_CHUNK_ROWS), -(-n // SPLIT_COLUMNS)
     tiles = lambda rows: -(-m // rows) * columns
-    if tiles(64) < 0.375 * units:
+    long = k >= SPLIT_LONG_K
+    if tiles(64) < 0.25 * units:
         return None
-    rows = min((t for t in SPLIT_TILES if 4 * tiles(t[0]) >= units), key=lambda t: -(-m // t[0]) * t[0] * t[1])[0]
-    enough = (1.5 if k >= 4096 else 1) * units
+    enough = 1.5 * units if long else 0.75 * units
+    fits = [t for t in SPLIT_TILES if tiles(t[0]) * (4 if long else 1) >= (units if long else enough)]
+    rows = min(fits, key=lambda t: -(-m // t[0]) * t[0] * t[1])[0] if fits else SPLIT_TILES[-1][0]
     return rows, 1 if tiles(rows) >= enough else 2 if 2 * tiles(rows) >= enough else 4
 
 
@@ -306,24 +309,45 @@ def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(0) >= x.shape[1] and x.stride(0) % 4 == 0 and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None) -> torch.Tensor:
-    """float32 x @ w.T for many rows on the bfloat16 matrix cores, each operand as the sum of three bfloat16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
-    with ``ranges`` ranges of K (``split_plan`` chooses).  ``take`` (shape, dtype): scratch, 6 K bytes a row of x and with ranges 4 N a row and range."""
+class SplitWeight:
+    """A float32 matrix [N, K] as ``linear_split`` reads it: two float16 values for each of its own times a power of two a row (as many bytes again), and those powers.
+    What depends on the two beyond their range is computed from the matrix itself, which the caller keeps unchanged."""
+
+    def __init__(self, w: torch.Tensor) -> None:
+        if not split_takes(w[:1], w) or w.shape[1] % SPLIT_K_MULTIPLE:
+            raise KernelRefused("a split weight is float32 [N, K] in plain rows on 16 bytes, K a multiple of 32")
+        self.n, self.k = w.shape
+        n, k = c_int(self.n), c_int(self.k)
+        self.scales = torch.empty(self.n, dtype=torch.float32, device=w.device)
+        self.parts = torch.empty(-(-self.n // 16) * 16 * 2 * self.k, dtype=torch.float16, device=w.device)
+        lib = build.core()
+        _check(lib.ns_split_scales(_ptr(self.scales), _ptr(w), n, k, _stream()), "split_scales")
+        _check(lib.ns_split_rows(_ptr(self.parts), _ptr(w), _ptr(self.scales), n, k, k, _stream()), "split_rows")
+
+
+def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None, split: SplitWeight | None = None) -> torch.Tensor:
+    """float32 x @ w.T for many rows on the float16 matrix cores, each operand as the sum of two float16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
+    with ``ranges`` ranges of K (``split_plan`` chooses).  ``take`` (shape, dtype): scratch, 4.125 K bytes a row of x and with ranges 4 N a row and range.
+    ``split``: of w; it is made where not given."""
     out = _check_linear(x, w, out, False)
     if not split_takes(x, w):
         raise KernelRefused("linear_split takes float32 x [rows, K] in rows of whole 16-byte pieces and w [N, K], both on 16 bytes")
+    if split is None:
+        split = SplitWeight(w)
+    elif (split.n, split.k) != tuple(w.shape) or split.parts.device != x.device:
+        raise KernelRefused("linear_split: the split weight is another matrix's")
     m, (n, k) = x.shape[0], w.shape
     if take is None:
         take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device)
     lib, most = build.core(), min(m, SPLIT_CHUNK_ROWS)
-    parts = take((-(-most // 16) * 16 * 3 * k,), torch.bfloat16)
+    parts = take((-(-most // 16) * 16 * (2 * k + k // 16),), torch.float16)
     sums = take((ranges * most * n,), torch.float32) if ranges > 1 else None
     for s in range(0, m, SPLIT_CHUNK_ROWS):
         piece, to = (x, out) if m == most else (x[s : s + SPLIT_CHUNK_ROWS], out[s : s + SPLIT_CHUNK_ROWS])
         h = c_int(piece.shape[0])
-        _check(lib.ns_split_rows(_ptr(parts), _ptr(piece), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
-        _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(piece), _ptr(w), h, c_int(n), c_int(k), c_int(x.stride(0)),
-                                 c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
+        _check(lib.ns_split_rows(_ptr(parts), _ptr(piece), c_void_p(0), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
+        _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(split.parts), _ptr(piece), _ptr(w), _ptr(split.scales), h, c_int(n), c_int(k),
+                                 c_int(x.stride(0)), c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
         if sums is not None:
             reduce_partial(PartialSums(sums, ranges, piece.shape[0], n, torch.float32), out=to)
     return out

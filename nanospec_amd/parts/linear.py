@@ -1,7 +1,7 @@
 """x @ W^T for the parts: ``LinearWeight`` holds a weight matrix and chooses the kernel by precision and row count.
 
 float32: ``csrc/gemm_generic.hip``, 32-bit products and sums in a fixed order: up to 8 rows stream the weights, more run the 32-bit matrix
-instruction, odd sizes the plain tiled kernel; and ``csrc/gemm_split.hip`` for many rows, whose operands are sums of three bfloat16 values
+instruction, odd sizes the plain tiled kernel; and ``csrc/gemm_split.hip`` for many rows, whose operands are sums of two float16 values
 and whose results are nearer to 64 bits than those.  (The true 32-bit path: no mode of reduced precision is ever used.)
 
 bfloat16: decode and short portions (up to ``STREAM_ROWS`` rows) run the hand-written matrix-core kernel that streams
@@ -24,7 +24,8 @@ from ..kernels import ops
 # Which copies of a bfloat16 weight matrix a model keeps (``DecoderModel.load(..., layouts=)``; parts that say
 # ``takes_layouts`` are told at load time): the re-laid one that the streaming kernels read is always there; the plain one,
 # which the library's products for many rows read, only with "both".  With "tiled" many rows run in blocks through the
-# hand-written kernels: slower prompts, half the memory.
+# hand-written kernels: slower prompts, half the memory.  Of a float32 matrix the plain copy is always there and, with "both", one in
+# two parts that its products of many rows read (``ops.SplitWeight``).
 LAYOUTS = ("both", "tiled")
 
 
@@ -97,14 +98,22 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
     return y if act is None else ops.activation(y, act)
 
 
-def product_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, arena) -> torch.Tensor:
-    """x @ w^T in 32-bit: many rows of a wide enough matrix on the bfloat16 matrix cores, no less exact (``ops.linear_split``; its scratch comes from ``arena``, without one it is
-    not taken), the others on the 32-bit ones."""
-    plan = ops.split_plan(x.shape[0], w.shape[0], w.shape[1], ops.compute_units(x.device)) if arena is not None and x.is_cuda else None
+def split_weight(w: torch.Tensor) -> "ops.SplitWeight | None":
+    """The second copy of a float32 matrix, for ``product_f32``, or None where that has no use for it."""
+    n, k = w.shape
+    if w.dtype != torch.float32 or not w.is_cuda or not ops.SPLIT_MIN_K <= k < 1 << 19 or k % ops.SPLIT_K_MULTIPLE or n > 1 << 19 or not ops.split_takes(w[:1], w):
+        return None
+    return ops.SplitWeight(w)
+
+
+def product_f32(x: torch.Tensor, w: torch.Tensor, split: "ops.SplitWeight | None", out: torch.Tensor | None, arena) -> torch.Tensor:
+    """x @ w^T in 32-bit: many rows of a wide enough matrix on the float16 matrix cores, no less exact (``ops.linear_split``; its scratch comes from ``arena``, without one it is
+    not taken; ``split``: ``split_weight`` of w), the others on the 32-bit ones."""
+    plan = ops.split_plan(x.shape[0], w.shape[0], w.shape[1], ops.compute_units(x.device)) if arena is not None and split is not None else None
     if plan is None or not ops.split_takes(x, w):
         return ops.linear_generic(x, w, out=out)
     mark = arena.mark()
-    out = ops.linear_split(x, w, *plan, out=out, take=arena.take)
+    out = ops.linear_split(x, w, *plan, out=out, take=arena.take, split=split)
     arena.release(mark)
     return out
 
@@ -141,6 +150,7 @@ class LinearWeight:
         self.tiled = ops.TiledWeight(w) if (fast and (tiled or self.k > LIBRARY_MAX_K)) else None
         self.plain = w if (keep_plain or self.tiled is None) else None
         self._plain_t = self.plain.t() if self.plain is not None else None  # the library product's operand, made once
+        self._split = split_weight(w) if keep_plain else None
 
     def links_norms(self, rows: int) -> bool:
         """Whether a product of ``rows`` rows can take a ``PreNormed`` input and can end in the residual stream."""
@@ -227,7 +237,7 @@ class LinearWeight:
         if x.dtype != self.dtype:
             raise ops.KernelRefused(f"linear: input is {x.dtype}, the weight {self.dtype}")
         if self.dtype == torch.float32:
-            return product_f32(x, self.plain, out, arena)
+            return product_f32(x, self.plain, self._split, out, arena)
         if self.k % 8 or not ops.tiled_takes(x[:1], self.k):
             return ops.linear_generic(x, self.plain, out=out, out_f32=out_f32)
         m = x.shape[0]
@@ -284,6 +294,7 @@ class GatedWeights:
         # [2 I, K] for the two-kernel path (which biased products of more than 16 rows always take)
         self.stacked = torch.cat([gate, up]) if (keep_plain or not fast or bias is not None) else None
         self._stacked_t = self.stacked.t() if self.stacked is not None else None
+        self._split = split_weight(self.stacked) if self.stacked is not None and keep_plain else None
         # biased and bfloat16: more than 16 rows take the stacked matrix in plain rows to the library (no third copy is re-laid)
         self._stacked_linear = LinearWeight(self.stacked, keep_plain=True, tiled=False) if (bias is not None and fast) else None
 
@@ -317,7 +328,7 @@ class GatedWeights:
             if self._stacked_linear is not None:
                 self._stacked_linear(x, out=gu, arena=ctx.arena, plain_copy=not ctx.captured)
             elif self.dtype == torch.float32:
-                product_f32(x, self.stacked, gu, ctx.arena)
+                product_f32(x, self.stacked, self._split, gu, ctx.arena)
             else:
                 ops.linear_generic(x, self.stacked, out=gu)
             return ops.silu_mul_bias(gu, self.bias_stacked, out=out)
@@ -347,6 +358,6 @@ class GatedWeights:
             return out
         if self.dtype == torch.float32 or self.k % 8:
             gu = ctx.arena.take((m, 2 * self.inter), x.dtype)
-            product = product_f32(x, self.stacked, gu, ctx.arena) if self.dtype == torch.float32 else ops.linear_generic(x, self.stacked, out=gu)
+            product = product_f32(x, self.stacked, self._split, gu, ctx.arena) if self.dtype == torch.float32 else ops.linear_generic(x, self.stacked, out=gu)
             return ops.silu_mul(product, out=out)
         return library_product(x, self._stacked_t, gated=out, plain=self.stacked, take=ctx.arena.take)

@@ -102,7 +102,7 @@ class DecoderModel:
     def load(self, source, dtype: torch.dtype, device, layouts: str = "auto") -> "DecoderModel":
         """Check the source against what the model wants (one error that lists everything wrong), then read
         each tensor once.  A head that is absent is the embedding table if the configuration ties them
-        (reference: model/loader.py:62-70).  ``layouts``: "both" keeps every bfloat16 matrix in two layouts
+        (reference: model/loader.py:62-70).  ``layouts``: "both" keeps every matrix in two layouts
         (``parts.linear.LAYOUTS``), "tiled" only in the re-laid one, "auto" chooses by the memory that is free."""
         spec = self.spec
         full = self.wanted()

@@ -120,19 +120,20 @@ def test_linear_f32_of_rows_far_apart(m, stride, n, k):
 @pytest.mark.parametrize("rows", [64, 96, 112, 128])
 @pytest.mark.parametrize("m,n,k,ranges", [(1, 1, 32, 1), (15, 130, 64, 2), (17, 131, 96, 3), (113, 257, 160, 1), (129, 64, 1056, 4), (300, 2060, 1024, 2)])
 def test_linear_split(rows, m, n, k, ranges):
-    """32-bit products through three bfloat16 parts of each operand at the edges of the tiles (16 rows and the tile's, 16 and 128 columns), of a stage of 32 k and of
+    """32-bit products through two float16 parts of each operand at the edges of the tiles (16 rows and the tile's, 16 and 128 columns), of a stage of 32 k and of
     uneven ranges; rows of x and of the result with a stride of their own."""
     ops = _ops()
     torch.manual_seed(m + n + k)
     wide = torch.randn(m, k + 12, device=DEV)
     x, w, out = wide[:, 4 : 4 + k], torch.randn(n, k, device=DEV), torch.full((m, n + 3), 7.0, device=DEV)
     ref = x.cpu().double() @ w.cpu().double().T
-    # a stage's sum is rounded 24 times (six instructions, four blocks of 8 k each) and leaves out 2^-24; then a stage or range is added at a time
-    bound = (25 + k / 32 + ranges) * 2.0**-24 * (x.cpu().double().abs() @ w.cpu().double().abs().T)
+    # two parts stand for a float to 2^-23 at most and leave out 2^-22 of a product, the sum of a stage is rounded 12 times (three instructions, four blocks of 8 k
+    # each); then a stage or range is added at a time
+    bound = (2 + 2 + 4 + 12 + k / 32 + ranges) * 2.0**-24 * (x.cpu().double().abs() @ w.cpu().double().abs().T)
     ops.linear_split(x, w, rows, ranges, out=out[:, :n])
     assert ((out[:, :n].cpu().double() - ref).abs() <= bound).all()
     assert bool((out[:, n:] == 7).all())
-    if m * n > 1000:  # nearer to 64 bits than the 32-bit instruction
+    if k >= ops.SPLIT_MIN_K:  # where it is taken it is nearer to 64 bits than the 32-bit instruction (whose sums' roundings are fewer than the parts' at a few stages)
         far = lambda y: float((y.cpu().double() - ref).norm())
         assert far(out[:, :n]) <= far(ops.linear_generic(x, w))
 
@@ -223,6 +224,35 @@ def test_keys_and_values_in_pieces(dtype, order, kind, H, G, D, E, page, rot, in
         assert bool((got[0][1].cpu().transpose(1, 2)[blank] == 0).all()) and bool((got[0][2].cpu().permute(0, 3, 1, 2)[blank] == 0).all())
 
 
+@pytest.mark.parametrize("spread", [12, 24])
+def test_linear_split_of_wide_rows(spread):
+    """Values over many powers of two within a block of x and a row of w: the parts of the small ones lie below the float16 numbers of full precision, not below all of them."""
+    ops = _ops()
+    torch.manual_seed(spread)
+    small = torch.randint(-spread, 1, (2, 300, 1024)).float().exp2().to(DEV)
+    x, w = torch.randn(100, 1024, device=DEV) * small[0, :100], torch.randn(300, 1024, device=DEV) * small[1]
+    a, b = x.cpu().double(), w.cpu().double()
+    largest = a.abs().view(100, 32, 32).amax(2).repeat_interleave(32, 1)
+    # as above, and a part that is rounded to a multiple of 2^-24 where the largest value of the block or row is at least 2^14
+    bound = (2 + 2 + 4 + 12 + 32 + 1) * 2.0**-24 * (a.abs() @ b.abs().T) + 2.0**-39 * (largest @ b.abs().T + a.abs() @ b.abs().amax(1, keepdim=True).expand(300, 1024).T)
+    assert bool(((ops.linear_split(x, w, 64, 1).cpu().double() - a @ b.T).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("keep_plain", [True, False])
+def test_linear_weight_f32_of_many_rows(keep_plain):
+    """A float32 matrix through the part's own door, with its second copy and (only one copy is kept) without; both as close as 32-bit sums."""
+    from nanospec_amd.engine.arena import Arena
+    from nanospec_amd.parts.linear import LinearWeight
+
+    ops = _ops()
+    torch.manual_seed(5)
+    x, w = torch.randn(600, 2048, device=DEV), torch.randn(2064, 2048, device=DEV)
+    linear = LinearWeight(w, keep_plain=keep_plain)
+    assert ops.split_plan(600, 2064, 2048, ops.compute_units(x.device)) is not None and (linear._split is not None) == keep_plain
+    y, ref = linear(x, arena=Arena(x.device)).double(), x.double() @ w.double().T
+    assert float((y - ref).norm() / ref.norm()) <= (3e-7 if keep_plain else 6e-7)  # 1.8e-7 and 4.1e-7 measured at K 2,048
+
+
 def test_split_plan():
     """What goes to the split kernel: whole stages, enough tiles; every plan is one that the launch takes."""
     from nanospec_amd.kernels import ops
@@ -233,8 +263,8 @@ def test_split_plan():
                 plan = ops.split_plan(m, n, k, 256)
                 if plan is not None:
                     rows, ranges = plan
-                    assert m >= 48 and m * n * k >= 3e9 and k % 32 == 0 and rows in (64, 96, 112, 128) and 1 <= ranges <= k // 32
-    assert ops.split_plan(777, 16384, 2048, 256) == (112, 1) and ops.split_plan(512, 2048, 8192, 256) == (128, 4)
+                    assert m >= 48 and m * n * k >= 2e9 and k % 32 == 0 and rows in (64, 96, 112, 128) and 1 <= ranges <= k // 32
+    assert ops.split_plan(832, 16384, 2048, 256) == (128, 1) and ops.split_plan(512, 2048, 8192, 256) == (128, 4) and ops.split_plan(832, 2048, 2048, 256) == (64, 1)
     assert ops.split_plan(47, 128256, 2048, 256) is None and ops.split_plan(256, 512, 2048, 256) is None
 
 

@@ -733,6 +733,11 @@ def many_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
+def many_f32_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_many`` takes these operands with a float32 result (``MANY_SPLIT_FORM``)."""
+    return w.shape[1] >= MANY_K_MIN and w.shape[0] % 4 == 0 and many_takes(x, w)
+
+
 def many_writes(out: torch.Tensor, m: int, n: int) -> bool:
     """Whether ``linear_many`` can write a result of m rows and n columns there: whole pieces of four values."""
     return out.shape == (m, n) and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0
@@ -742,7 +747,8 @@ def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, 
                 add: bool = False, ranges: int = 1):
     """bfloat16 x @ w.T for many rows, w in plain rows, tiles of ``MANY_TILES[form]`` (``many_plan`` chooses): into ``out``; with ``act`` that
     activation of it; with ``w2`` silu(x @ w.T) * (x @ w2.T); with ``add`` added to ``out`` in 32-bit, rounded once.  With ``ranges`` > 1 (none of
-    these) ``out`` is float32 scratch of ranges * rows * w.shape[0] and a ``PartialSums`` over it comes back, whose reader rounds once."""
+    these) ``out`` is float32 scratch of ranges * rows * w.shape[0] and a ``PartialSums`` over it comes back, whose reader rounds once.  A float32 ``out``
+    (``MANY_SPLIT_FORM``, nothing behind the product) takes the sums as they are."""
     _gpu(x, w, w2, out)
     m, (n, k) = x.shape[0], w.shape
     # (what else ``many_takes`` asks of addresses, strides and K the launch checks itself)
@@ -755,9 +761,11 @@ def linear_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, form: int, 
     if ranges > 1:
         if out.dtype != torch.float32 or out.numel() < ranges * m * n or not out.is_contiguous():
             raise KernelRefused("linear_many: scratch too small")
-    elif out.shape != (m, n) or out.dtype != x.dtype or out.stride(1) != 1:
+    elif out.dtype == torch.float32 and (add or w2 is not None or act is not None or not out.is_contiguous()):
+        raise KernelRefused("linear_many: a float32 result is contiguous, and nothing follows the product")
+    elif out.shape != (m, n) or out.dtype not in (x.dtype, torch.float32) or out.stride(1) != 1:
         raise KernelRefused("linear_many: out has the wrong shape or dtype")
-    epi = 4 if ranges > 1 else 3 if add else 2 if w2 is not None else 1 if act is not None else 0
+    epi = 4 if ranges > 1 or out.dtype == torch.float32 else 3 if add else 2 if w2 is not None else 1 if act is not None else 0
     _check(build.core().ns_gemm_many_bf16(_ptr(out), _ptr(x), _ptr(w), _ptr(w2), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
                                           c_int(n if ranges > 1 else out.stride(0)), c_int(epi), c_int(0 if act is None else ACTIVATIONS[act]),
                                           c_int(ranges), c_int(form), _stream()), "linear_many")

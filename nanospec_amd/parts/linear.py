@@ -241,6 +241,10 @@ class LinearWeight:
         if self.k % 8 or not ops.tiled_takes(x[:1], self.k):
             return ops.linear_generic(x, self.plain, out=out, out_f32=out_f32)
         m = x.shape[0]
+        if out_f32 and m >= ops.MANY_MIN_ROWS and self.plain is not None and ops.many_f32_takes(x, self.plain) and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0):
+            # (2,048 columns, K 4,096, us in blocks of 128 rows from the re-laid copy and here, alone / beside two others: 130 rows 44 / 34, 32 / 22, 508 50 / 29, 32 / 20, 2,048 83 / 68,
+            # 40 / 31; 4,096 columns, K 8,192, 130 rows 58 / 38, 54 / 27, 2,048 219 / 207, 118 / 113; two or four ranges of K are level beside others at best)
+            return ops.linear_many(x, self.plain, out if out is not None else torch.empty((m, self.n), dtype=torch.float32, device=x.device), ops.MANY_SPLIT_FORM)
         if self.tiled is not None and WIDE_HEAD_ROWS < m <= STREAM_ROWS and out_f32 and self.n >= 8192:
             return ops.linear_wide(x, self.tiled, out=out, out_f32=True, ksplit=1, nt=1)
         if self.tiled is not None and m <= STREAM_ROWS:

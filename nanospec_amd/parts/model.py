@@ -138,7 +138,7 @@ class DecoderModel:
         if self.passes is not None:
             self.pass_rows = get(self.passes.name).to(device=device, dtype=dtype).contiguous()
             if self.passes.join_name:
-                self.pass_join = LinearWeight(get(self.passes.join_name).to(device=device, dtype=dtype).contiguous(), keep_plain=False)
+                self.pass_join = LinearWeight(get(self.passes.join_name).to(device=device, dtype=dtype).contiguous(), keep_plain=layouts == "both")
         if spec.streams:
             self._ones = torch.ones(spec.streams, dtype=torch.float32, device=device)
             self._eye = torch.eye(spec.streams, dtype=torch.float32, device=device)

@@ -382,6 +382,26 @@ def test_linear_many(form, m, n, k):
         torch.testing.assert_close(y.cpu(), pl.rms_norm(r.cpu(), weight.cpu(), 1e-5), **_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 4, 512), (257, 132, 640), (300, 640, 2048), (1100, 260, 4096)])
+def test_linear_many_f32(m, n, k):
+    """32-bit results of many rows: the kernel, and the part's own door to it."""
+    from nanospec_amd.parts.linear import LinearWeight
+
+    ops = _ops()
+    torch.manual_seed(m + n + k)
+    x = torch.randn(m + 3, k + 8, dtype=torch.bfloat16, device=DEV)[:m, :k]
+    w = torch.randn(n, k, dtype=torch.bfloat16, device=DEV)
+    a, b = x.cpu().double(), w.cpu().double()
+    bound = k / 8 * 2.0**-24 * (a.abs() @ b.abs().T)  # a rounding of the sum for every block of 8 k
+    wide = torch.full((m + 1, n), 7.0, device=DEV)
+    y = ops.linear_many(x, w, wide[:m], ops.MANY_SPLIT_FORM)
+    assert bool(((y.cpu().double() - a @ b.T).abs() <= bound).all()) and bool((wide[m] == 7).all())
+    assert torch.equal(LinearWeight(w)(x, out_f32=True), y)
+    for bad in (dict(act="silu"), dict(add=True), dict(out=torch.empty(m, 2 * n, device=DEV)[:, :n]), dict(form=0)):
+        with pytest.raises(ops.KernelRefused):
+            ops.linear_many(**{**dict(x=x, w=w, out=y, form=ops.MANY_SPLIT_FORM), **bad})
+
+
 def test_linear_many_refuses():
     ops = _ops()
     x, w, out = (torch.zeros(200, k, dtype=torch.bfloat16, device=DEV) for k in (512, 512, 200))

@@ -16,6 +16,7 @@ from dataclasses import dataclass
 
 import torch
 
+from ..kernels.ops import SlotTensors
 from ..parts.needs import PagedNeed, StateNeed, each_need
 from .manager import GroupSpec
 
@@ -91,9 +92,14 @@ class CacheStorage:
             t = torch.zeros((num_slots, *need.shape), dtype=need.dtype, device=device)
             self.states.append(t)
             self.model_state[name] = t
+        # (a single state is as fast through its own fill, and the CPU has no launches to save)
+        self._slots = SlotTensors(self.states) if len(self.states) > 1 and torch.device(device).type == "cuda" else None
 
     def reset_slot(self, slot: int) -> None:
         """A newly admitted request starts from zero state."""
+        if self._slots is not None:
+            self._slots.clear(slot)
+            return
         for t in self.states:
             t[slot].zero_()
 

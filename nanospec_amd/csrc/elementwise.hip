@@ -690,6 +690,23 @@ extern "C" int ns_fill_u32(void* p, uint32_t value, size_t n_words, hipStream_t 
   return ns_launch_status();
 }
 
+// One slot of every one of ``count`` tensors [slots, ...] to zeros: table holds two of 64 bits for each, its address and the bytes of a slot.  A request that is
+// admitted clears a handful of states of some hundred KB, each 4 us of the host as a launch of its own.
+__global__ __launch_bounds__(256) void clear_slots_kernel(const uint64_t* __restrict__ table, int slot) {
+  const uint64_t bytes = table[2 * blockIdx.y + 1], from = table[2 * blockIdx.y] + bytes * slot;
+  const uint64_t first = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
+  const uint64_t whole = (from & 15) ? 0 : bytes / 16;
+  for (uint64_t i = first; i < whole; i += step) reinterpret_cast<int4*>(from)[i] = int4{0, 0, 0, 0};
+  for (uint64_t i = 16 * whole + first; i < bytes; i += step) reinterpret_cast<char*>(from)[i] = 0;
+}
+// ``most``: the largest slot's bytes (how many workgroups share a tensor).
+extern "C" int ns_clear_slots(const void* table, int count, int slot, size_t most, hipStream_t stream) {
+  if (count <= 0 || count > 65535 || slot < 0 || most == 0) return NS_ERR_BAD_ARG;
+  const size_t blocks = (most + 16 * 256 * 4 - 1) / (16 * 256 * 4);
+  clear_slots_kernel<<<dim3((unsigned)(blocks < 256 ? blocks : 256), count), 256, 0, stream>>>((const uint64_t*)table, slot);
+  return ns_launch_status();
+}
+
 // dst[dst_idx[i]] = src[src_idx[i]]: token ids sampled by one step become the input ids of the next without a trip
 // to the host.
 __global__ void scatter_i32_kernel(int* __restrict__ dst, const int* __restrict__ dst_idx, const int* __restrict__ src,

@@ -236,6 +236,25 @@ def fill_u32(t: torch.Tensor, value: int = 0) -> None:
     _check(build.core().ns_fill_u32(_ptr(t), c_uint32(value), c_size_t(nbytes // 4), _stream()), "fill_u32")
 
 
+class SlotTensors:
+    """Tensors [slots, ...] that belong together, and a launch that sets one slot of them all to zero."""
+
+    def __init__(self, tensors: list[torch.Tensor]) -> None:
+        _gpu(*tensors)
+        if not tensors or any(not t.is_contiguous() or t.shape[0] != tensors[0].shape[0] for t in tensors):
+            raise KernelRefused("SlotTensors takes contiguous tensors of one number of slots")
+        self.tensors, self.slots = list(tensors), tensors[0].shape[0]
+        sizes = [t[0].numel() * t.element_size() for t in tensors]
+        self.most = max(sizes)
+        self.table = torch.tensor([v for t, n in zip(tensors, sizes) for v in (t.data_ptr(), n)], dtype=torch.int64).to(tensors[0].device)
+
+    def clear(self, slot: int) -> None:
+        if not 0 <= slot < self.slots:
+            raise KernelRefused(f"slot {slot} of {self.slots}")
+        if self.most:
+            _check(build.core().ns_clear_slots(_ptr(self.table), c_int(len(self.tensors)), c_int(slot), c_size_t(self.most), _stream()), "clear_slots")
+
+
 def scatter_i32(dst: torch.Tensor, dst_idx: torch.Tensor, src: torch.Tensor, src_idx: torch.Tensor) -> None:
     """dst[dst_idx[i]] = src[src_idx[i]] for int32 tensors on the GPU (indices are trusted: the caller built them)."""
     _gpu(dst, dst_idx, src, src_idx)

@@ -253,6 +253,22 @@ def test_linear_weight_f32_of_many_rows(keep_plain):
     assert float((y - ref).norm() / ref.norm()) <= (3e-7 if keep_plain else 6e-7)  # 1.8e-7 and 4.1e-7 measured at K 2,048
 
 
+@pytest.mark.parametrize("shapes", [[(1,)], [(3, 5), (1,), (7,)], [(16, 128, 257), (2, 2048), (1,), (13,)]])
+def test_slot_tensors(shapes):
+    """One slot of every tensor is cleared and nothing beside it: slots of single words, of odd numbers of values, of many blocks."""
+    ops = _ops()
+    kinds = (torch.float32, torch.bfloat16, torch.int32, torch.bfloat16)
+    tensors = [torch.ones((5, *shape), dtype=dtype, device=DEV) for shape, dtype in zip(shapes, kinds)]
+    slots = ops.SlotTensors(tensors)
+    for slot in (4, 0, 2):
+        slots.clear(slot)
+    for t in tensors:
+        assert [bool((t[i] == 0).all()) for i in range(5)] == [True, False, True, False, True] and bool((t[1::2] == 1).all())
+    for bad in (-1, 5):
+        with pytest.raises(ops.KernelRefused):
+            slots.clear(bad)
+
+
 def test_split_plan():
     """What goes to the split kernel: whole stages, enough tiles; every plan is one that the launch takes."""
     from nanospec_amd.kernels import ops

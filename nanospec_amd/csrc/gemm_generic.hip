@@ -1,6 +1,6 @@
 // out[M, N] = x[M, K] . w[N, K]^T  with 32-bit accumulation in a fixed order, for any M, N, K.
 //
-// The products of the true 32-bit path, and the fall-back for shapes the bfloat16 matrix-core kernels refuse.  A row's
+// The products of the true 32-bit path (of many rows where gemm_split.hip does not take them), and the fall-back for shapes the bfloat16 matrix-core kernels refuse.  A row's
 // result does not depend on which other rows share the launch.  Three kernels: a plain tiled one for any size and either
 // type, whose outputs are each one chain of fused multiply-adds over k = 0..K-1; for 32-bit operands on whole 16-byte
 // pieces one that reads w as fast as memory gives it (up to 8 rows) and one on the 32-bit matrix instructions (more rows).

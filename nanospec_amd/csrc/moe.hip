@@ -68,52 +68,56 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const T* __restrict__ h
 // The logits decide which experts run, so no 32-bit chain is longer than 8 columns (two instructions), and the chains are added in 64 bits.
 // Relative error (2-norm, against 64 bits) at 2,048 columns 5.9e-8, of the kernel above 1.2e-7, with one chain a wave 4.0e-7; it is below
 // the other's down to 64 columns, from where on the launch takes this kernel.  W a multiple of 16.
+// SETS of 16 rows of the router a workgroup: its 64-bit sums take as long as its matrix instructions, so a single set is ahead while the compute units have no more than a
+// workgroup each: with the choice behind, alone, two sets and one: 32 rows of 2,048, 508 tokens 24.2 and 20.3 us, 36 rows 23.8 and 20.6, 64 rows of 4,096 35.7 and 28.4; level or
+// behind beyond (64 rows of 4,096, 2,048 tokens 36.4 and 42.3).  The sums are the same.
 #define MOE_LOGIT_WAVES 8
-template <typename T>
+#define MOE_UNITS 256  // compute units
+template <typename T, int SETS>
 __global__ __launch_bounds__(NS_WAVE * MOE_LOGIT_WAVES) void moe_logits_many_kernel(const T* __restrict__ h, int h_stride, const float* __restrict__ wr,
                                                               const float* __restrict__ br, float* __restrict__ z, int n, int W, int experts) {
   constexpr int STEP = 16 * MOE_LOGIT_WAVES;  // columns from one piece of a wave to the next
-  __shared__ double part[MOE_LOGIT_WAVES][2][16][17];  // [wave][16 rows of the router][token][row]
+  __shared__ double part[MOE_LOGIT_WAVES][SETS][16][17];  // [wave][16 rows of the router][token][row]
   const int lane = threadIdx.x % NS_WAVE, wave = threadIdx.x / NS_WAVE, r = lane % 16, g = lane / 16;
-  const int t0 = blockIdx.x * 16, e0 = blockIdx.y * 32;
+  const int t0 = blockIdx.x * 16, e0 = blockIdx.y * 16 * SETS;
   const T* x = h + (size_t)min(t0 + r, n - 1) * h_stride + 4 * g;
-  const float* w[2];
+  const float* w[SETS];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) w[i] = wr + (size_t)min(e0 + 16 * i + r, experts - 1) * W + 4 * g;
+  for (int i = 0; i < SETS; ++i) w[i] = wr + (size_t)min(e0 + 16 * i + r, experts - 1) * W + 4 * g;
   typedef T t4 __attribute__((ext_vector_type(4)));
-  double sum[2][4] = {};
+  double sum[SETS][4] = {};
   for (int c = 16 * wave; c < W; c += 4 * STEP) {
     t4 xv[4];
-    f32x4 wv[4][2];
+    f32x4 wv[4][SETS];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {  // (a piece beyond the row is read at its start and not used)
       const int at = c + STEP * s < W ? c + STEP * s : 0;
       xv[s] = *reinterpret_cast<const t4*>(x + at);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) wv[s][i] = *reinterpret_cast<const f32x4*>(w[i] + at);
+      for (int i = 0; i < SETS; ++i) wv[s][i] = *reinterpret_cast<const f32x4*>(w[i] + at);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if (c + STEP * s >= W) break;
-      f32x4 acc[2][2];
+      f32x4 acc[2][SETS];
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < SETS; ++i)
           acc[k / 2][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s][i][k], to_f((T)xv[s][k]), k % 2 ? acc[k / 2][i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < SETS; ++i)
 #pragma unroll
         for (int k = 0; k < 4; ++k) sum[i][k] += (double)acc[0][i][k] + (double)acc[1][i][k];
     }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < SETS; ++i)
 #pragma unroll
     for (int k = 0; k < 4; ++k) part[wave][i][r][4 * g + k] = sum[i][k];
   __syncthreads();
-  for (int i = threadIdx.x; i < 512; i += NS_WAVE * MOE_LOGIT_WAVES) {
-    const int t = i / 32, e = i % 32;
+  for (int i = threadIdx.x; i < 256 * SETS; i += NS_WAVE * MOE_LOGIT_WAVES) {
+    const int t = i / (16 * SETS), e = i % (16 * SETS);
     if (t0 + t >= n || e0 + e >= experts) continue;
     double v = br ? (double)br[e0 + e] : 0.;
 #pragma unroll
@@ -428,11 +432,17 @@ extern "C" int ns_moe_route(const void* h, int h_stride, const float* wr, const 
     else
       moe_logits_few_kernel<bf16_t><<<rows, 256, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows, vec);
   } else if (vec && W % 16 == 0 && W >= 64) {
-    const dim3 many((n + 15) / 16, (rows + 31) / 32);
-    if (dtype == NS_DTYPE_F32)
-      moe_logits_many_kernel<float><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows);
-    else
-      moe_logits_many_kernel<bf16_t><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows);
+    // (sets of 16 rows of the router a workgroup: one where a compute unit then still has no more than one workgroup, MOE_UNITS of them)
+    const long one = (long)((n + 15) / 16) * ((rows + 15) / 16);
+    const bool single = one <= MOE_UNITS;
+    const dim3 many((n + 15) / 16, single ? (rows + 15) / 16 : (rows + 31) / 32);
+    if (dtype == NS_DTYPE_F32) {
+      if (single) moe_logits_many_kernel<float, 1><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows);
+      else moe_logits_many_kernel<float, 2><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows);
+    } else {
+      if (single) moe_logits_many_kernel<bf16_t, 1><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows);
+      else moe_logits_many_kernel<bf16_t, 2><<<many, NS_WAVE * MOE_LOGIT_WAVES, 0, stream>>>((const bf16_t*)h, h_stride, wr, br, z, n, W, rows);
+    }
   } else if (dtype == NS_DTYPE_F32)
     moe_logits_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, h_stride, wr, br, z, n, W, rows, vec);
   else

@@ -1466,6 +1466,23 @@ def test_moe_router_of_many_tokens(n, rows, width, dtype):
     assert torch.equal(sel.cpu().long(), z.cpu().topk(2).indices)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64])
+def test_moe_router_by_one_or_two_sets_of_rows(rows):
+    """A workgroup takes 16 rows of the router while the units have one workgroup each and 32 beyond: a token's logits are the same bits either way."""
+    ops = _ops()
+    torch.manual_seed(rows)
+    h, router = torch.randn(4100, 96, device=DEV).bfloat16(), torch.randn(rows, 96, device=DEV)
+    def logits(n):
+        z, sel, wt = torch.full((n, rows), 7.0, device=DEV), torch.empty((n, 1), dtype=torch.int32, device=DEV), torch.empty((n, 1), device=DEV)
+        ops.moe_route(h[:n], router, None, 1, sel, wt, logits=z)
+        return z
+    many = logits(4100)  # 257 workgroups and more
+    for n in (17, 800, 4096):
+        assert torch.equal(logits(n), many[:n]), n
+    ref = h.cpu().double() @ router.cpu().double().T
+    assert float((many.cpu().double() - ref).norm() / ref.norm()) <= 2.0**-22
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,rows,width", [(64, 33, 2048), (300, 16, 4096), (40, 64, 512), (500, 64, 64)])
 def test_moe_router_of_many_tokens_is_as_exact_as_the_plain_kernel(n, rows, width, dtype):

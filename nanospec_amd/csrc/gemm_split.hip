@@ -1,20 +1,26 @@
 // Products of many 32-bit rows on the float16 matrix cores, out[m][n] = sum_k x[m][k] w[n][k], in less than half of the 32-bit ones' time and nearer to 64 bits.
 // (reference: the nn.Linear calls of model/llama.py:175,184,195)
 //
-// A float times a power of two is the sum of two float16 values, a = a0 + a1, each the nearest to what is left: |a1| <= 2^-11 |a|, and 2^-23 |a| at most is lost, or 2^-25 where
-// the largest is 2^14 to 2^15: small ones keep what counts beside it.  Powers of two are chosen for each 32 k of a row of x, and for each row of w.  Of the four products of two such
-// sums three are taken, the smallest first: a1 b0, a0 b1, a0 b0; the one left out is 2^-22 of a b at most, and its sign is any.  A product of two float16 values is exact in 32 bits.
-// The matrix instruction adds up blocks of 8 k and rounds each sum to nearest, so three of them over a stage of 32 k begin at zero and the vector unit adds what they give to the
-// sums, times the power of two of x.
-// Error against 64 bits (2-norm), this in one range of K and the 32-bit instruction's four chains (gemm_generic.hip): both operands normal, K 2,048 1.8e-7 and 4.1e-7, K 8,192 3.2e-7
-// and 8.1e-7; all of one sign 1.3e-7 and 1.8e-7, 2.5e-7 and 3.5e-7; x spread over 24 powers of two 1.9e-7 and 3.9e-7, 3.3e-7 and 7.6e-7; one k of 512 10^5 times the others 1.9e-7 and
-// 4.6e-7, 3.2e-7 and 8.4e-7.  (Three bfloat16 values for a float, six products: 1.6e-7 and 3.1e-7 for normal operands, and twice the work of the matrix unit.)
+// A float times a power of two, its largest neighbour brought to 2^14 to 2^15, is a0 + 2^-11 a1 of two float16 values, each the nearest to what is left: 2^-23 |a| at most is lost.  (The second
+// at 2^11 times its size has the float16 range to itself: a value keeps its bits down to 2^-28 of the largest; at its own size down to 2^-17.)  Powers of two are chosen for each 32 k
+// of a row of x, and for each row of w.  Of the four products of two such sums three are taken, a1 b0 + a0 b1 in a sum of their own and a0 b0; the one left out is 2^-22 of a b at most, and its
+// sign is any.  A product of two float16 values is exact in 32 bits.  The matrix instruction adds up blocks of 8 k and rounds each sum to nearest, so those of a stage of 32 k begin at
+// zero and the vector unit adds what they give to the sums, times the power of two of x.
+// What the parts do not hold is counted where a block is split: values too small beside the largest, which are all that counts where that meets zeros; infinities; blocks whose products could
+// leave the range of 32 bits on their way.  A row of x or of w that has two such values, or one that is not even held to 2^-18, is given to the 32-bit instruction by a launch behind the
+// product (``split_mend_kernel``).  A single one, 10^-8 of its block's largest or less, is one in 10^8 normal values, and every product of a few million would have a row that goes that way for
+// it; two are one row of K 2,048 in 10^9.  (A row that has a value that is no number is none whatever is done with it.)
+// Error against 64 bits (2-norm), this in one range of K and the 32-bit instruction's four chains (gemm_generic.hip): both operands normal, K 2,048 1.7e-7 and 4.1e-7, K 8,192 3.0e-7
+// and 8.1e-7; all of one sign 1.3e-7 and 1.8e-7, 2.5e-7 and 3.5e-7; x spread over 16 powers of two 1.8e-7 and 4.1e-7, 3.3e-7 and 8.1e-7; one k of 512 10^5 times the others 1.9e-7 and
+// 4.6e-7, 3.3e-7 and 8.3e-7, and against zeros in w 1.7e-7 and 4.1e-7, 3.1e-7 and 8.1e-7.  Behind it only where a row is zeros but for one k of 32: 1.7e-7 and 1.1e-7, 3.0e-7 and 2.1e-7.
+// (Three bfloat16 values for a float, six products: 1.6e-7 and 3.1e-7 for normal operands, and twice the work of the matrix unit.)
 //
-// Both operands are split ahead, w once for all (as many bytes again as it has), x a call.  w split in registers on its way by every tile of x instead: 211 us for the 177 below.
+// Both operands are split ahead, w once for all (as many bytes again as it has), x a call.  w split in registers on its way by every tile of x instead: 211 us for 177 in the first size below beside two others.
 // x comes through LDS, where the four waves share it, and each wave's own columns of w straight into the registers of the matrix instruction, both two stages ahead (one: tiles that have a
 // compute unit to themselves 1.2 times as long).  us, the 32-bit instruction and this with the splitting of x and the sum of ranges of K, alone / a call beside two others:
-// 832 rows, N 16,384, K 2,048 536 / 511 and 206 / 177 (315 TFLOP/s of products of 32 bits), N 2,048, K 8,192 307 / 272 and 122 / 102, N 3,072, K 2,048 96 / 89 and 66 / 35;
-// 2,048 rows of 28,672 x 4,096 3,649 / 3,727 and 1,300 / 1,561.
+// 832 rows, N 16,384, K 2,048 536 / 511 and 217 / 175 (315 TFLOP/s of products of 32 bits), N 2,048, K 8,192 307 / 272 and 133 / 108, N 3,072, K 2,048 96 / 89 and 71 / 40;
+// 2,048 rows of 28,672 x 4,096 3,649 / 3,727 and 1,340 / 1,402.  The lower products in a sum of their own are twice the work of the vector unit: 1,273 us alone before for the last, 1,330 now, 2,048 rows of
+// 4,096 x 14,336, two tiles a compute unit, 662 and 750; taken to the sums under the products of the next block it is hidden in the smaller ones.
 // Bound by the power of the matrix unit: at the last size it works for 69% of the cycles and the clock sinks to 1.4 GHz.
 #include "common.h"
 #include "lds_loads.h"
@@ -26,9 +32,16 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 #define SPLIT_K 32       // k of a stage
 #define SPLIT_BLOCK 512  // values of a block: 16 rows of a stage
-#define SPLIT_COLUMNS 2  // blocks of 16 rows of w a wave: with four, 112 rows of x a tile and two workgroups a compute unit instead of three, 173 us for the 177 above and 49 for the 35
-#define SPLIT_DOWN 0x1p-15f  // with the scale of x: sums are kept as if a row's largest of w were 1/2 to 1, so that they are in range where x and the results are
+#define SPLIT_COLUMNS 2  // blocks of 16 rows of w a wave: with four, 112 rows of x a tile and two workgroups a compute unit instead of three, 173 us for 177 in the first size above beside two others and 49 for 35 in the third
+// Sums are kept 2^40 times what they are with a row's largest of w brought to 1/2 to 1.  With the largest of a block from 2^-64 to 2^68 that is 2^127 at most for K below 2^19, and the product
+// of the smallest values that parts hold, 2^-50 of their largest, is a normal number.
+#define SPLIT_UP 25  // (2^40 over the 2^15 of w)
+#define SPLIT_LEAST 0x1p-64f
+#define SPLIT_MOST 0x1p68f
 #define SPLIT_STAGES 3   // at hand: one that is multiplied and two on their way
+
+#define SPLIT_LOST 2  // values of a row that the parts do not hold, from which on it goes to the 32-bit instruction
+#define SPLIT_GROUP 4 // blocks of 32 k whose counts are one word, two bits for each of 16 rows
 
 union Operand {  // of the matrix instruction: eight values, made two at a time
   f16x8 v;
@@ -42,48 +55,83 @@ __device__ __forceinline__ float split_scale(float largest) {
 }
 __device__ __forceinline__ float inverse_scale(float scale) { return __builtin_bit_cast(float, (254u << 23) - __builtin_bit_cast(unsigned, scale)); }
 
-// Eight floats times a power of two into their two parts.
-__device__ __forceinline__ void split_eight(const f32x4& low, const f32x4& high, float scale, Operand* part) {
+// Eight floats times a power of two into their two parts.  How many of them are not held to 2^-23 of themselves; two for one that is not held to 2^-18 or infinite.
+__device__ __forceinline__ int split_eight(const f32x4& low, const f32x4& high, float scale, Operand* part) {
+  int lost = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const f32x4& of = e < 2 ? low : high;
-    const f32x2 v = {of[e % 2 * 2], of[e % 2 * 2 + 1]};
-    const f16x2 first = __builtin_convertvector((f32x2{v[0] * scale, v[1] * scale}), f16x2);
-    part[0].pair[e] = first;
-    part[1].pair[e] = __builtin_convertvector((f32x2{fmaf(v[0], scale, -(float)first[0]), fmaf(v[1], scale, -(float)first[1])}), f16x2);  // (exact before it is rounded)
+    const f32x2 v = {of[e % 2 * 2] * scale, of[e % 2 * 2 + 1] * scale};
+    const f16x2 first = __builtin_convertvector(v, f16x2);
+    const f32x2 left = {(v[0] - (float)first[0]) * 0x1p11f, (v[1] - (float)first[1]) * 0x1p11f};  // (exact)
+    const f16x2 second = __builtin_convertvector(left, f16x2);
+    part[0].pair[e] = first, part[1].pair[e] = second;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float raw = of[e % 2 * 2 + i], off = fabsf(left[i] - (float)second[i]), of_one = fabsf(v[i]);
+      const bool far = !(off <= 0x1p-7f * of_one) || (of_one == 0.f && raw != 0.f);
+      lost += raw != raw ? 0 : far ? 2 : off > 0x1p-12f * of_one;
+    }
   }
+  return lost;
 }
+// The same of a block of 32 k, by the four lanes that have it, no more than 2.
+__device__ __forceinline__ int lost_in(int lost) {
+  lost += __shfl_xor(lost, 16), lost += __shfl_xor(lost, 32);
+  return min(lost, 2);
+}
+__device__ __forceinline__ bool out_of_range(float largest) { return largest != 0.f && !(largest >= SPLIT_LEAST && largest <= SPLIT_MOST); }
 
 // x [M, K] as parts[block of 16 rows][block of 32 k][part][lane][8], where lane 16 g + r holds of row r the k 8 g .. 8 g + 7 of the block: an operand of the matrix
 // instruction as it lies in registers, so that any two blocks are two contiguous KB.  Rows beyond the last are zeros.
-// ``scales`` (of w): a power of two a row.  Without them (of x) one a row and block, their inverses over 2^15 behind all parts, [block of 16 rows][block of 32 k][16]
-// (below the normal numbers for the smallest of x, and exact there too).
-__global__ __launch_bounds__(256) void split_rows_kernel(_Float16* __restrict__ parts, const float* __restrict__ x, const float* __restrict__ scales, int M, int K, int x_stride) {
-  const int k_blocks = K / SPLIT_K, lane = threadIdx.x % NS_WAVE, r = lane % 16, g = lane / 16;
-  const int kb = blockIdx.x * 4 + threadIdx.x / NS_WAVE, mb = blockIdx.y, row = mb * 16 + r;
-  if (kb >= k_blocks) return;
-  f32x4 low = {0.f, 0.f, 0.f, 0.f}, high = low;
-  if (row < M) {
-    const float* at = x + (size_t)row * x_stride + kb * SPLIT_K + 8 * g;
-    low = *reinterpret_cast<const f32x4*>(at), high = *reinterpret_cast<const f32x4*>(at + 4);
-  }
-  const size_t block = (size_t)mb * k_blocks + kb;
-  float scale = 1.f;
-  if (scales) {
-    if (row < M) scale = scales[row];
-  } else {
-    float largest = 0.f;
+// ``w_scales`` (of w): a power of two a row.  Without them (of x) one a row and block, their inverses times 2^25 behind all parts, [block of 16 rows][block of 32 k][16].  lost[block of 16 rows][group
+// of 128 k]: of row r in bits 2 r and 2 r + 1 how many values the parts do not hold, 2 for more; behind them ``call``, a number of the caller's, if any does (what lies there before may be anything).
+__global__ __launch_bounds__(256) void split_rows_kernel(_Float16* __restrict__ parts, const float* __restrict__ x, const float* __restrict__ w_scales, unsigned* __restrict__ lost, unsigned call, int M,
+                                                         int K, int x_stride) {
+  __shared__ unsigned counts[SPLIT_GROUP][16];
+  const int k_blocks = K / SPLIT_K, lane = threadIdx.x % NS_WAVE, wave = threadIdx.x / NS_WAVE, r = lane % 16, g = lane / 16;
+  const int kb = blockIdx.x * SPLIT_GROUP + wave, mb = blockIdx.y, row = mb * 16 + r;
+  int count = 0;
+  if (kb < k_blocks) {
+    f32x4 low = {0.f, 0.f, 0.f, 0.f}, high = low;
+    if (row < M) {
+      const float* at = x + (size_t)row * x_stride + kb * SPLIT_K + 8 * g;
+      low = *reinterpret_cast<const f32x4*>(at), high = *reinterpret_cast<const f32x4*>(at + 4);
+    }
+    const size_t block = (size_t)mb * k_blocks + kb;
+    float scale = 1.f;
+    if (w_scales) {
+      if (row < M) scale = w_scales[row];
+    } else {
+      float largest = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) largest = fmaxf(largest, fmaxf(fabsf(low[e]), fabsf(high[e])));
-    largest = fmaxf(largest, __shfl_xor(largest, 16)), largest = fmaxf(largest, __shfl_xor(largest, 32));
-    scale = split_scale(largest);
-    if (g == 0) reinterpret_cast<float*>(parts + (size_t)gridDim.y * k_blocks * 2 * SPLIT_BLOCK)[block * 16 + r] = inverse_scale(scale) * SPLIT_DOWN;
-  }
-  Operand part[2];
-  split_eight(low, high, scale, part);
-  f16x8* to = reinterpret_cast<f16x8*>(parts + block * 2 * SPLIT_BLOCK) + lane;
+      for (int e = 0; e < 4; ++e) largest = fmaxf(largest, fmaxf(fabsf(low[e]), fabsf(high[e])));
+      largest = fmaxf(largest, __shfl_xor(largest, 16)), largest = fmaxf(largest, __shfl_xor(largest, 32));
+      scale = split_scale(largest);
+      count = out_of_range(largest) ? SPLIT_LOST : 0;
+      if (g == 0) reinterpret_cast<float*>(parts + (size_t)gridDim.y * k_blocks * 2 * SPLIT_BLOCK)[block * 16 + r] = inverse_scale(scale) * (float)(1 << SPLIT_UP);
+    }
+    Operand part[2];
+    count += split_eight(low, high, scale, part);
+    count += __shfl_xor(count, 16), count += __shfl_xor(count, 32);
+    f16x8* to = reinterpret_cast<f16x8*>(parts + block * 2 * SPLIT_BLOCK) + lane;
 #pragma unroll
-  for (int p = 0; p < 2; ++p) to[p * NS_WAVE] = part[p].v;
+    for (int p = 0; p < 2; ++p) to[p * NS_WAVE] = part[p].v;
+  }
+  if (g == 0) counts[wave][r] = count;
+  __syncthreads();
+  if (wave == 0) {
+    count = 0;
+#pragma unroll
+    for (int i = 0; i < SPLIT_GROUP; ++i) count += counts[i][r];
+    unsigned word = (unsigned)min(count, SPLIT_LOST) << 2 * r;
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2) word |= __shfl_xor(word, d);
+    if (lane == 0) {
+      lost[(size_t)mb * gridDim.x + blockIdx.x] = word;
+      if (word) lost[(size_t)gridDim.y * gridDim.x] = call;
+    }
+  }
 }
 
 // The scale of each row of w, a row a wave.
@@ -101,23 +149,35 @@ __global__ __launch_bounds__(256) void split_scales_kernel(float* __restrict__ s
   if (lane == 0) scales[n] = split_scale(largest);
 }
 
+// The blocks of 16 rows that have a row to mend: list[0] how many, then for each its number and the rows as bits, from the counts of ``lost`` [blocks][groups].  By all threads of a workgroup.
+__device__ __forceinline__ void list_lost(int* list, const unsigned* lost, int blocks, int groups) {
+  if (threadIdx.x == 0) list[0] = 0;
+  unsigned any = 0;
+  for (size_t i = threadIdx.x; i < (size_t)blocks * groups; i += blockDim.x) any |= lost[i];
+  if (!__syncthreads_or(any)) return;  // (all of the workgroup)
+  for (int b = threadIdx.x; b < blocks; b += blockDim.x) {
+    unsigned more = 0, once = 0;  // (bits 2 r: rows with two, rows with one so far)
+    for (int i = 0; i < groups; ++i) {
+      const unsigned word = lost[(size_t)b * groups + i], one = word & 0x55555555u, two = word >> 1 & 0x55555555u;
+      more |= two | (once & one), once |= one;
+    }
+    if (more) {
+      const int at = atomicAdd(list, 1);
+      int rows = 0;
+      for (int r = 0; r < 16; ++r) rows |= (int)(more >> 2 * r & 1) << r;
+      list[1 + 2 * at] = b, list[2 + 2 * at] = rows;
+    }
+  }
+  __syncthreads();
+}
+__global__ __launch_bounds__(1024) void split_list_kernel(int* __restrict__ list, const unsigned* __restrict__ lost, int blocks, int groups) { list_lost(list, lost, blocks, groups); }
+
 struct SplitParams {
   float* out;  // [M, N], or with ranges of K [ranges][M][N]
   const _Float16 *parts, *w_parts;
-  const float *x, *w, *w_scales;
-  int M, N, K, x_stride, out_stride, m_tiles, n_tiles, ranges;
+  const float* w_scales;
+  int M, N, K, out_stride, m_tiles, n_tiles, ranges;
 };
-
-// One output as one chain over k in 32 bits, until it is no number.
-__device__ __attribute__((noinline)) float split_plain(const float* a, const float* b, int k) {
-  float s = 0.f;
-  for (int i = 0; i < k && s == s; i += 4) {
-    const f32x4 u = *reinterpret_cast<const f32x4*>(a + i), v = *reinterpret_cast<const f32x4*>(b + i);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s = fmaf(u[e], v[e], s);
-  }
-  return s;
-}
 
 // Four waves, 16 MI rows of x by 128 of w.  A stage's parts of x lie in LDS and those of w in the registers of the wave whose columns they are, and the next two are on their way.
 template <int MI>
@@ -186,23 +246,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       for (int q = 0; q < 2; ++q) a[i % 2][q] = *reinterpret_cast<const f16x8*>(lds + at * STAGE + (i * 2 + q) * SPLIT_BLOCK + lane * 8);
       inverse[i % 2] = reinterpret_cast<const float*>(lds + at * STAGE + 2 * MI * SPLIT_BLOCK)[i * 16 + r];
     };
+    f32x4 low[2][NJ], sum[2][NJ];
+    float scale[2];
+    auto join = [&](int i) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(fmaf(low[i % 2][j][e], 0x1p-11f, sum[i % 2][j][e]), scale[i % 2], acc[i][j][e]);
+    };
     read_x(0);
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       if (i + 1 < MI) read_x(i + 1);  // (under the products of i)
       __builtin_amdgcn_sched_barrier(0);
-      f32x4 sum[NJ];
-      constexpr int OF_W[3] = {1, 0, 0}, OF_X[3] = {0, 1, 0};
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
+      for (int j = 0; j < NJ; ++j) low[i % 2][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[at][j][1], a[i % 2][0], zero, 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[at][j][OF_W[q]], a[i % 2][OF_X[q]], q ? sum[j] : zero, 0, 0, 0);
+      for (int j = 0; j < NJ; ++j) low[i % 2][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[at][j][0], a[i % 2][1], low[i % 2][j], 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ; ++j) sum[i % 2][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[at][j][0], a[i % 2][0], zero, 0, 0, 0);
+      scale[i % 2] = inverse[i % 2];
+      if (i > 0) join(i - 1);
+      if (i > 0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(sum[j][e], inverse[i % 2], acc[i][j][e]);
+        for (int q = 0; q < 3 * NJ; ++q) __builtin_amdgcn_sched_group_barrier(0x8, 1, 0), __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
+    join(MI - 1);
+    __builtin_amdgcn_sched_barrier(0);
   };
   load(0, from);
   load(1, min(from + 1, to - 1));
@@ -212,10 +284,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   if (kb + 1 < to) stage(1, kb + 1);
   TILE_WAIT_LOADS(0);  // (what was fetched again behind the last stage must not come into another workgroup's LDS)
 
-  // acc[i][j], lane 16 g + r: row 16 i + r of the tile, columns 16 j + 4 g .. + 3 of the wave's.  No number or an infinity, of the floats or of the sums on their way: the
-  // parts do not stand for the floats there, and the sum is taken from these.
+  // acc[i][j], lane 16 g + r: row 16 i + r of the tile, columns 16 j + 4 g .. + 3 of the wave's
   float* out = p.out + (size_t)range * p.M * p.N;
   const bool whole = p.N % 4 == 0 && p.out_stride % 4 == 0 && ((uintptr_t)out & 15) == 0;
+  int down[NJ][4];  // the power of two that sums are taken times
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) down[j][e] = 127 - SPLIT_UP - (int)(__builtin_bit_cast(unsigned, p.w_scales[min(n0 + 16 * (wave * NJ + j) + 4 * g + e, p.N - 1)]) >> 23);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int m = m0 + 16 * i + r;
@@ -224,13 +300,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     for (int j = 0; j < NJ; ++j) {
       const int n = n0 + 16 * (wave * NJ + j) + 4 * g;
       if (n >= p.N) continue;
-      f32x4 v = acc[i][j];
+      f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = ldexpf(v[e], 127 + 15 - (int)(__builtin_bit_cast(unsigned, p.w_scales[min(n + e, p.N - 1)]) >> 23));
-        if (n + e < p.N && !(fabsf(v[e]) < INFINITY))
-          v[e] = split_plain(p.x + (size_t)m * p.x_stride + from * SPLIT_K, p.w + (size_t)(n + e) * p.K + from * SPLIT_K, (to - from) * SPLIT_K);
-      }
+      for (int e = 0; e < 4; ++e) v[e] = ldexpf(acc[i][j][e], down[j][e]);
       float* at = out + (size_t)m * p.out_stride + n;
       if (whole)
         *reinterpret_cast<f32x4*>(at) = v;
@@ -253,11 +325,126 @@ static int launch_split(SplitParams p, hipStream_t stream) {
   return ns_launch_status();
 }
 
-// parts: float16, 2 K values for each of M rows rounded up to 16, and without ``scales`` (null) K / 16 more.  K a multiple of 32, x_stride of 4, both on 16 bytes.
-extern "C" int ns_split_rows(void* parts, const void* x, const void* scales, int M, int K, int x_stride, hipStream_t stream) {
+// The outputs of the rows of x and of w that the parts do not hold, by the 32-bit instruction from the floats, in gemm_f32_kernel's four chains (gemm_generic.hip): wave c adds up the k 16 c .. 16 c + 15
+// of every 64, and the four sums are added as there.  None, as good as always: then the launch is all that this costs.  A few blocks of 16 rows: a workgroup takes one against 16 rows of the other
+// operand, bound by the way of those from memory, hence 16 pieces on their way; many: four against 32, so that what comes from L2 is used more often.  One row of 832, N 16,384, K 2,048 40 us (its 134 MB of floats are read), N 2,048, K 8,192 40, N = K = 2,048 13;
+// all 832 640, 390 and 107, where the 32-bit product alone takes 427, 246 and 69.
+#define MEND_BLOCKS 256  // of 16 rows of x
+#define MEND_MANY 8      // blocks from which on they go four at a time
+#define MEND_GROUPS 512  // workgroups, two a compute unit
+struct MendParams {
+  float* out;
+  const float *x, *w;
+  const unsigned* lost;
+  const int* w_list;
+  int M, N, K, x_stride, out_stride;
+  unsigned call;
+};
+struct MendBlock {  // of 16 rows, and those of them whose outputs are written whatever the other operand's
+  int block, rows;
+};
+
+template <int MB, int NB, int AHEAD>
+__device__ __forceinline__ void mend_tile(const MendParams& p, const MendBlock* of_x, const MendBlock* of_w, f32x4* sums) {
+  const int lane = threadIdx.x % NS_WAVE, wave = threadIdx.x / NS_WAVE, r = lane % 16, g = lane / 16;
+  const int k0 = 16 * wave, pieces = (p.K - k0 + 63) / 64;  // (K a multiple of 32: pieces are whole, and waves 2 and 3 may have one less)
+  const float *a[MB], *b[NB];
+  f32x4 u[AHEAD][MB], v[AHEAD][NB], chain[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) a[i] = p.x + (size_t)min(of_x[i].block * 16 + r, p.M - 1) * p.x_stride + 4 * g;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) b[j] = p.w + (size_t)min(of_w[j].block * 16 + r, p.N - 1) * p.K + 4 * g;
+  auto load = [&](int at, int piece) {  // (behind the last piece K's last 16 once more, not used)
+    const int k = min(k0 + 64 * piece, p.K - 16);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) u[at][i] = *reinterpret_cast<const f32x4*>(a[i] + k);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) v[at][j] = *reinterpret_cast<const f32x4*>(b[j] + k);
+  };
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) chain[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < AHEAD; ++c) load(c, c);
+  for (int piece = 0; piece < pieces; piece += AHEAD) {
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) {
+      if (piece + c < pieces) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) chain[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c][j][e], u[c][i][e], chain[i][j], 0, 0, 0);
+      }
+      load(c, piece + c + AHEAD);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MB * NB; ++i) sums[(wave * MB * NB + i) * NS_WAVE + lane] = chain[i / NB][i % NB];
+  __syncthreads();
+  // row r of x, row 4 g + e of w: a wave writes one e
+#pragma unroll
+  for (int i = 0; i < MB * NB; ++i) {
+    const MendBlock x = of_x[i / NB], w = of_w[i % NB];
+    const int m = x.block * 16 + r, n = w.block * 16 + 4 * g + wave;
+    const f32x4* one = sums + i * NS_WAVE + lane;
+    const float sum = (one[0][wave] + one[MB * NB * NS_WAVE][wave]) + (one[2 * MB * NB * NS_WAVE][wave] + one[3 * MB * NB * NS_WAVE][wave]);
+    if (m < p.M && n < p.N && ((x.rows >> r | w.rows >> n % 16) & 1)) p.out[(size_t)m * p.out_stride + n] = sum;
+  }
+  __syncthreads();
+}
+
+// ``of_x``: the list is of blocks of x.
+template <bool OF_X, int LISTED, int OTHER, int AHEAD>
+__device__ __forceinline__ void mend_list(const MendParams& p, const int* list, int others, f32x4* sums) {
+  const int groups = (others + OTHER - 1) / OTHER;
+  const long items = (long)((list[0] + LISTED - 1) / LISTED) * groups;
+  for (long item = blockIdx.x; item < items; item += gridDim.x) {
+    MendBlock listed[LISTED], other[OTHER];
+#pragma unroll
+    for (int i = 0; i < LISTED; ++i) {  // (behind the last that once more)
+      const int at = min((int)(item / groups) * LISTED + i, list[0] - 1);
+      listed[i] = MendBlock{list[1 + 2 * at], list[2 + 2 * at]};
+    }
+#pragma unroll
+    for (int i = 0; i < OTHER; ++i) other[i] = MendBlock{min((int)(item % groups) * OTHER + i, others - 1), 0};
+    if constexpr (OF_X)
+      mend_tile<LISTED, OTHER, AHEAD>(p, listed, other, sums);
+    else
+      mend_tile<OTHER, LISTED, AHEAD>(p, other, listed, sums);
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void split_mend_kernel(const MendParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ int list[1 + 2 * MEND_BLOCKS];
+  __shared__ f32x4 sums[4 * 8 * NS_WAVE];
+  const int m_blocks = (p.M + 15) / 16, n_blocks = (p.N + 15) / 16, groups = (p.K / SPLIT_K + SPLIT_GROUP - 1) / SPLIT_GROUP;
+  if (p.lost[m_blocks * groups] == p.call) {
+    list_lost(list, p.lost, m_blocks, groups);
+    if (list[0] >= MEND_MANY)
+      mend_list<true, 4, 2, 4>(p, list, n_blocks, sums);
+    else
+      mend_list<true, 1, 1, 16>(p, list, n_blocks, sums);
+  }
+  if (p.w_list[0] >= MEND_MANY)
+    mend_list<false, 4, 2, 4>(p, p.w_list, m_blocks, sums);
+  else if (p.w_list[0])
+    mend_list<false, 1, 1, 16>(p, p.w_list, m_blocks, sums);
+#endif
+}
+
+static int split_groups(int K) { return (K / SPLIT_K + SPLIT_GROUP - 1) / SPLIT_GROUP; }
+
+// parts: float16, 2 K values for each of M rows rounded up to 16, and without ``w_scales`` (null) K / 16 more.  lost: a word for each 16 rows and each 128 k or what is left of them.  K a multiple of
+// 32, x_stride of 4, both on 16 bytes.  ``lost`` has one word more, for ``call``: a number that differs from one call to the next over the same scratch (in a replay it is the same, and a word that an
+// earlier replay left there only makes ns_split_mend look).
+extern "C" int ns_split_rows(void* parts, void* lost, unsigned call, const void* x, const void* w_scales, int M, int K, int x_stride, hipStream_t stream) {
   if (M <= 0 || K <= 0 || x_stride < K) return NS_ERR_BAD_ARG;
   if (K % SPLIT_K || x_stride % 4 || (((uintptr_t)x | (uintptr_t)parts) & 15) || (M + 15) / 16 > 65535) return NS_ERR_UNSUPPORTED;
-  split_rows_kernel<<<dim3((K / SPLIT_K + 3) / 4, (M + 15) / 16), 256, 0, stream>>>((_Float16*)parts, (const float*)x, (const float*)scales, M, K, x_stride);
+  split_rows_kernel<<<dim3(split_groups(K), (M + 15) / 16), NS_WAVE * SPLIT_GROUP, 0, stream>>>((_Float16*)parts, (const float*)x, (const float*)w_scales, (unsigned*)lost, call, M, K, x_stride);
   return ns_launch_status();
 }
 
@@ -269,15 +456,20 @@ extern "C" int ns_split_scales(void* scales, const void* w, int N, int K, hipStr
   return ns_launch_status();
 }
 
-// ``parts``: of ``x`` by ns_split_rows without scales; ``w_parts``: of ``w`` by ns_split_rows with ``w_scales``, those by ns_split_scales.  ``rows``: of a tile,
+// list: 1 and two words for each 16 of M rows, from what ns_split_rows counted of them.
+extern "C" int ns_split_list(void* list, const void* lost, int M, int K, hipStream_t stream) {
+  if (M <= 0 || K <= 0 || K % SPLIT_K) return NS_ERR_BAD_ARG;
+  split_list_kernel<<<1, 1024, 0, stream>>>((int*)list, (const unsigned*)lost, (M + 15) / 16, split_groups(K));
+  return ns_launch_status();
+}
+
+// ``parts``: of x by ns_split_rows without scales; ``w_parts``: of w by ns_split_rows with ``w_scales``, those by ns_split_scales.  ``rows``: of a tile,
 // 64, 96, 112 or 128.  ``ranges`` of K above 1: out is [ranges][M][N] (out_stride N), the sums of each.
-// K a multiple of 32 below 2^19 (a tile's parts within 31 bits of bytes), x_stride of 4; x, w and parts on 16 bytes.
-extern "C" int ns_gemm_split(void* out, const void* parts, const void* w_parts, const void* x, const void* w, const void* w_scales, int M, int N, int K, int x_stride,
-                             int out_stride, int rows, int ranges, hipStream_t stream) {
-  if (M <= 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N || ranges < 1 || (ranges > 1 && out_stride != N)) return NS_ERR_BAD_ARG;
-  if (K % SPLIT_K || x_stride % 4 || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)parts | (uintptr_t)w_parts) & 15) || K >= 1 << 19 || ranges > K / SPLIT_K)
-    return NS_ERR_UNSUPPORTED;
-  const SplitParams p{(float*)out, (const _Float16*)parts, (const _Float16*)w_parts, (const float*)x, (const float*)w, (const float*)w_scales, M, N, K, x_stride, out_stride, 0, 0, ranges};
+// K a multiple of 32 below 2^19 (a tile's parts within 31 bits of bytes), parts on 16 bytes.  What the parts do not hold is to be put right by ns_split_mend, behind the sum of the ranges.
+extern "C" int ns_gemm_split(void* out, const void* parts, const void* w_parts, const void* w_scales, int M, int N, int K, int out_stride, int rows, int ranges, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || out_stride < N || ranges < 1 || (ranges > 1 && out_stride != N)) return NS_ERR_BAD_ARG;
+  if (K % SPLIT_K || (((uintptr_t)parts | (uintptr_t)w_parts) & 15) || K >= 1 << 19 || ranges > K / SPLIT_K) return NS_ERR_UNSUPPORTED;
+  const SplitParams p{(float*)out, (const _Float16*)parts, (const _Float16*)w_parts, (const float*)w_scales, M, N, K, out_stride, 0, 0, ranges};
   switch (rows) {
     case 64: return launch_split<4>(p, stream);
     case 96: return launch_split<6>(p, stream);
@@ -285,4 +477,13 @@ extern "C" int ns_gemm_split(void* out, const void* parts, const void* w_parts, 
     case 128: return launch_split<8>(p, stream);
   }
   return NS_ERR_BAD_ARG;
+}
+
+// ``lost``, ``call``: of x by ns_split_rows; ``w_list``: of w by ns_split_list.  M at most 4,096; K a multiple of 32, x_stride of 4, x and w on 16 bytes.
+extern "C" int ns_split_mend(void* out, const void* x, const void* w, const void* lost, unsigned call, const void* w_list, int M, int N, int K, int x_stride, int out_stride, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N) return NS_ERR_BAD_ARG;
+  if (M > 16 * MEND_BLOCKS || K % SPLIT_K || x_stride % 4 || (((uintptr_t)x | (uintptr_t)w) & 15)) return NS_ERR_UNSUPPORTED;
+  const MendParams p{(float*)out, (const float*)x, (const float*)w, (const unsigned*)lost, (const int*)w_list, M, N, K, x_stride, out_stride, call};
+  split_mend_kernel<<<MEND_GROUPS, 256, 0, stream>>>(p);
+  return ns_launch_status();
 }

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 from ctypes import c_float, c_int, c_size_t, c_uint32, c_void_p
 
 import torch
@@ -328,9 +329,17 @@ def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.stride(0) >= x.shape[1] and x.stride(0) % 4 == 0 and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def split_lost_words(rows: int, k: int) -> int:
+    """32-bit words in which the splitting counts the values that its parts do not hold: one for 16 rows and 128 columns, and one behind them."""
+    return -(-rows // 16) * -(-k // (4 * SPLIT_K_MULTIPLE)) + 1
+
+
+_split_calls = itertools.count()  # (next() is one step of the interpreter: any number of threads may call)
+
+
 class SplitWeight:
-    """A float32 matrix [N, K] as ``linear_split`` reads it: two float16 values for each of its own times a power of two a row (as many bytes again), and those powers.
-    What depends on the two beyond their range is computed from the matrix itself, which the caller keeps unchanged."""
+    """A float32 matrix [N, K] as ``linear_split`` reads it: two float16 values for each of its own times a power of two a row (as many bytes again), those powers, and a list of the rows that the
+    two do not stand for, whose outputs are computed from the matrix itself, which the caller keeps unchanged."""
 
     def __init__(self, w: torch.Tensor) -> None:
         if not split_takes(w[:1], w) or w.shape[1] % SPLIT_K_MULTIPLE:
@@ -339,15 +348,18 @@ class SplitWeight:
         n, k = c_int(self.n), c_int(self.k)
         self.scales = torch.empty(self.n, dtype=torch.float32, device=w.device)
         self.parts = torch.empty(-(-self.n // 16) * 16 * 2 * self.k, dtype=torch.float16, device=w.device)
+        self.lost = torch.empty(1 + 2 * -(-self.n // 16), dtype=torch.int32, device=w.device)
+        counts = torch.empty(split_lost_words(self.n, self.k), dtype=torch.int32, device=w.device)
         lib = build.core()
         _check(lib.ns_split_scales(_ptr(self.scales), _ptr(w), n, k, _stream()), "split_scales")
-        _check(lib.ns_split_rows(_ptr(self.parts), _ptr(w), _ptr(self.scales), n, k, k, _stream()), "split_rows")
+        _check(lib.ns_split_rows(_ptr(self.parts), _ptr(counts), c_uint32(0), _ptr(w), _ptr(self.scales), n, k, k, _stream()), "split_rows")
+        _check(lib.ns_split_list(_ptr(self.lost), _ptr(counts), n, k, _stream()), "split_list")
 
 
 def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None, split: SplitWeight | None = None) -> torch.Tensor:
     """float32 x @ w.T for many rows on the float16 matrix cores, each operand as the sum of two float16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
-    with ``ranges`` ranges of K (``split_plan`` chooses).  ``take`` (shape, dtype): scratch, 4.125 K bytes a row of x and with ranges 4 N a row and range.
-    ``split``: of w; it is made where not given."""
+    with ``ranges`` ranges of K (``split_plan`` chooses).  The outputs of rows of either that two such values do not stand for (values that lie far apart, infinities) are those of ``linear_generic``
+    for more than 8 rows.  ``take`` (shape, dtype): scratch, 4.13 K bytes a row of x and with ranges 4 N a row and range.  ``split``: of w; it is made where not given."""
     out = _check_linear(x, w, out, False)
     if not split_takes(x, w):
         raise KernelRefused("linear_split takes float32 x [rows, K] in rows of whole 16-byte pieces and w [N, K], both on 16 bytes")
@@ -360,15 +372,17 @@ def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: 
         take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device)
     lib, most = build.core(), min(m, SPLIT_CHUNK_ROWS)
     parts = take((-(-most // 16) * 16 * (2 * k + k // 16),), torch.float16)
+    lost = take((split_lost_words(most, k),), torch.int32)
     sums = take((ranges * most * n,), torch.float32) if ranges > 1 else None
     for s in range(0, m, SPLIT_CHUNK_ROWS):
         piece, to = (x, out) if m == most else (x[s : s + SPLIT_CHUNK_ROWS], out[s : s + SPLIT_CHUNK_ROWS])
-        h = c_int(piece.shape[0])
-        _check(lib.ns_split_rows(_ptr(parts), _ptr(piece), c_void_p(0), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
-        _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(split.parts), _ptr(piece), _ptr(w), _ptr(split.scales), h, c_int(n), c_int(k),
-                                 c_int(x.stride(0)), c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
+        h, call = c_int(piece.shape[0]), c_uint32(next(_split_calls) & 0xFFFFFFFF)
+        _check(lib.ns_split_rows(_ptr(parts), _ptr(lost), call, _ptr(piece), c_void_p(0), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
+        _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(split.parts), _ptr(split.scales), h, c_int(n), c_int(k),
+                                 c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
         if sums is not None:
             reduce_partial(PartialSums(sums, ranges, piece.shape[0], n, torch.float32), out=to)
+        _check(lib.ns_split_mend(_ptr(to), _ptr(piece), _ptr(w), _ptr(lost), call, _ptr(split.lost), h, c_int(n), c_int(k), c_int(x.stride(0)), c_int(out.stride(0)), _stream()), "linear_split")
     return out
 
 

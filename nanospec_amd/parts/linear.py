@@ -1,8 +1,9 @@
 """x @ W^T for the parts: ``LinearWeight`` holds a weight matrix and chooses the kernel by precision and row count.
 
 float32: ``csrc/gemm_generic.hip``, 32-bit products and sums in a fixed order: up to 8 rows stream the weights, more run the 32-bit matrix
-instruction, odd sizes the plain tiled kernel; and ``csrc/gemm_split.hip`` for many rows, whose operands are sums of two float16 values
-and whose results are nearer to 64 bits than those.  (The true 32-bit path: no mode of reduced precision is ever used.)
+instruction, odd sizes the plain tiled kernel; and ``csrc/gemm_split.hip`` for many rows, on the float16 matrix cores: each float as the sum of two
+float16 values, which stand for it to 2^-23, a product to 2^-21, and sums nearer to 64 bits than the 32-bit instruction's unless nearly
+all of a row is zero.  Rows whose values lie too far apart for that, or are infinite, have the 32-bit instruction's results.
 
 bfloat16: decode and short portions (up to ``STREAM_ROWS`` rows) run the hand-written matrix-core kernel that streams
 the weights once; it reads them in a layout re-laid at load time (``kernels.ops.TiledWeight``) in which every load
@@ -107,8 +108,7 @@ def split_weight(w: torch.Tensor) -> "ops.SplitWeight | None":
 
 
 def product_f32(x: torch.Tensor, w: torch.Tensor, split: "ops.SplitWeight | None", out: torch.Tensor | None, arena) -> torch.Tensor:
-    """x @ w^T in 32-bit: many rows of a wide enough matrix on the float16 matrix cores, no less exact (``ops.linear_split``; its scratch comes from ``arena``, without one it is
-    not taken; ``split``: ``split_weight`` of w), the others on the 32-bit ones."""
+    """x @ w^T in 32-bit: many rows of a wide enough matrix on the float16 matrix cores (``ops.linear_split``; its scratch comes from ``arena``, without one it is not taken; ``split``: ``split_weight`` of w), the others on the 32-bit ones."""
     plan = ops.split_plan(x.shape[0], w.shape[0], w.shape[1], ops.compute_units(x.device)) if arena is not None and split is not None else None
     if plan is None or not ops.split_takes(x, w):
         return ops.linear_generic(x, w, out=out)

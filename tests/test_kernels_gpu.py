@@ -238,6 +238,32 @@ def test_linear_split_of_wide_rows(spread):
     assert bool(((ops.linear_split(x, w, 64, 1).cpu().double() - a @ b.T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("ranges", [1, 2])
+@pytest.mark.parametrize("kind", ["zero w", "small w", "zero x", "small x", "even", "sparse"])
+@pytest.mark.parametrize("factor", [1e4, 1e5, 1e6, 1e7, 1e8, 1e9, 1e10, 1e12, 1e30])
+def test_linear_split_of_values_far_apart(factor, kind, ranges):
+    """Large values that meet zeros or small ones in the other operand, so that all that counts is what is small beside them: as near to 64 bits as the 32-bit instruction."""
+    ops = _ops()
+    torch.manual_seed(17)
+    x, w = torch.randn(100, 1024, device=DEV), torch.randn(300, 1024, device=DEV)
+    if kind == "even":  # the small values all alike, one large one a block beside them
+        x[:] = 0.1
+    if kind == "sparse":  # one value a block beside the large one
+        x.view(100, 32, 32)[:, :, 6:] = 0
+        x.view(100, 32, 32)[:, :, :5] = 0
+    large, other = (w, x) if kind.endswith("x") else (x, w)
+    large[:, 3::32] *= factor
+    other[:, 3::32] *= 0 if kind in ("zero w", "zero x", "even", "sparse") else 1 / factor
+    ref = x.cpu().double() @ w.cpu().double().T
+    far = lambda y: float((y.cpu().double() - ref).norm() / ref.norm())
+    # (32 terms in all, hardly a rounding of the sums: a term is held to 2^-21, 2^-23 for either operand and 2^-22 for the product left out, and to a third of that in the mean)
+    limit = 2.0**-21 / 3 if kind == "sparse" else 0
+    y = ops.linear_split(x, w, 64, ranges)
+    assert far(y) <= max(far(ops.linear_generic(x, w)), limit)
+    if factor >= 1e12 and kind != "sparse":  # every row: the 32-bit instruction's sums
+        assert torch.equal(y, ops.linear_generic(x, w))
+
+
 @pytest.mark.parametrize("keep_plain", [True, False])
 def test_linear_weight_f32_of_many_rows(keep_plain):
     """A float32 matrix through the part's own door, with its second copy and (only one copy is kept) without; both as close as 32-bit sums."""

@@ -21,6 +21,9 @@ class Arena:
         self._sizes: list[int] = []  # bytes of each chunk
         self._typed: dict = {}  # (chunk, dtype) -> the chunk seen as that type
         self._cur, self._off = -1, 0
+        # of a captured step that ends in padding: how many rows it has, and (int32 [1] on the device) how many of them are read by anyone.  Products of so many rows
+        # may leave the others undone
+        self.read_rows: tuple[int, torch.Tensor] | None = None
         self.high_water = 0  # the most bytes that were in use at once since the arena was made (tails of chunks that a buffer
         #                      did not fit into count as used: one chunk of this size holds the same sequence of buffers)
         if nbytes:

@@ -123,6 +123,8 @@ class StepContext:
         # padding behind the portions, up to 63 tokens that nobody reads, would be the longest chain of a step of short portions
         behind = captured and not single_tokens
         self.spans = (self.qo_indptr[:-1], self.state_slots[:-1]) if behind else (self.qo_indptr, self.state_slots)
+        if arena is not None:  # (the stand-in's first row)
+            arena.read_rows = (self.n_tokens, self.qo_indptr[self.n_reqs - 1 : self.n_reqs]) if behind else None
         # what the parts' batch plans wrote, by key: (device view of the plan's region, its shape for this batch)
         self.plans = {key: (view(key), shape) for key, (_, shape) in layout.plans.items()}
         self.block_tables = [dev_buf[o : o + layout.B * layout.P].view(layout.B, layout.P) for o in layout.table_off]

@@ -352,14 +352,16 @@ class SplitWeight:
         counts = torch.empty(split_lost_words(self.n, self.k), dtype=torch.int32, device=w.device)
         lib = build.core()
         _check(lib.ns_split_scales(_ptr(self.scales), _ptr(w), n, k, _stream()), "split_scales")
-        _check(lib.ns_split_rows(_ptr(self.parts), _ptr(counts), c_uint32(0), _ptr(w), _ptr(self.scales), n, k, k, _stream()), "split_rows")
+        _check(lib.ns_split_rows(_ptr(self.parts), _ptr(counts), c_uint32(0), _ptr(w), _ptr(self.scales), c_void_p(0), c_int(0), n, k, k, _stream()), "split_rows")
         _check(lib.ns_split_list(_ptr(self.lost), _ptr(counts), n, k, _stream()), "split_list")
 
 
-def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None, split: SplitWeight | None = None) -> torch.Tensor:
+def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None, split: SplitWeight | None = None,
+                 read_rows: torch.Tensor | None = None) -> torch.Tensor:
     """float32 x @ w.T for many rows on the float16 matrix cores, each operand as the sum of two float16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
     with ``ranges`` ranges of K (``split_plan`` chooses).  The outputs of rows of either that two such values do not stand for (values that lie far apart, infinities) are those of ``linear_generic``
-    for more than 8 rows.  ``take`` (shape, dtype): scratch, 4.13 K bytes a row of x and with ranges 4 N a row and range.  ``split``: of w; it is made where not given."""
+    for more than 8 rows.  ``take`` (shape, dtype): scratch, 4.13 K bytes a row of x and with ranges 4 N a row and range.  ``split``: of w; it is made where not given.
+    ``read_rows`` (int32 [1] on the GPU): from this row on nobody reads the result, and whatever x holds there it is zeros."""
     out = _check_linear(x, w, out, False)
     if not split_takes(x, w):
         raise KernelRefused("linear_split takes float32 x [rows, K] in rows of whole 16-byte pieces and w [N, K], both on 16 bytes")
@@ -367,6 +369,8 @@ def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: 
         split = SplitWeight(w)
     elif (split.n, split.k) != tuple(w.shape) or split.parts.device != x.device:
         raise KernelRefused("linear_split: the split weight is another matrix's")
+    if read_rows is not None:
+        _gpu(read_rows), _i32(read_rows, "read_rows")
     m, (n, k) = x.shape[0], w.shape
     if take is None:
         take = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=x.device)
@@ -377,7 +381,8 @@ def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: 
     for s in range(0, m, SPLIT_CHUNK_ROWS):
         piece, to = (x, out) if m == most else (x[s : s + SPLIT_CHUNK_ROWS], out[s : s + SPLIT_CHUNK_ROWS])
         h, call = c_int(piece.shape[0]), c_uint32(next(_split_calls) & 0xFFFFFFFF)
-        _check(lib.ns_split_rows(_ptr(parts), _ptr(lost), call, _ptr(piece), c_void_p(0), h, c_int(k), c_int(x.stride(0)), _stream()), "linear_split")
+        _check(lib.ns_split_rows(_ptr(parts), _ptr(lost), call, _ptr(piece), c_void_p(0), _ptr(read_rows), c_int(s), h, c_int(k), c_int(x.stride(0)), _stream()),
+               "linear_split")
         _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(split.parts), _ptr(split.scales), h, c_int(n), c_int(k),
                                  c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
         if sums is not None:

@@ -113,7 +113,8 @@ def product_f32(x: torch.Tensor, w: torch.Tensor, split: "ops.SplitWeight | None
     if plan is None or not ops.split_takes(x, w):
         return ops.linear_generic(x, w, out=out)
     mark = arena.mark()
-    out = ops.linear_split(x, w, *plan, out=out, take=arena.take, split=split)
+    padded = arena.read_rows is not None and arena.read_rows[0] == x.shape[0]
+    out = ops.linear_split(x, w, *plan, out=out, take=arena.take, split=split, read_rows=arena.read_rows[1] if padded else None)
     arena.release(mark)
     return out
 

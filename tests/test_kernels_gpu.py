@@ -264,6 +264,31 @@ def test_linear_split_of_values_far_apart(factor, kind, ranges):
         assert torch.equal(y, ops.linear_generic(x, w))
 
 
+@pytest.mark.parametrize("read", [0, 1, 16, 77, 100])
+def test_linear_split_of_rows_that_nobody_reads(read):
+    """Padding rows are zeros whatever lies there, and none of them is left to the 32-bit instruction; the others are as they are without them, through the part's own door too."""
+    from nanospec_amd.engine.arena import Arena
+    from nanospec_amd.parts.linear import product_f32
+
+    ops = _ops()
+    torch.manual_seed(read)
+    x, w = torch.randn(100, 5120, device=DEV), torch.randn(4096, 5120, device=DEV)
+    want = ops.linear_split(x, w, 64, 1)
+    x[read:, ::3], x[read:, 1::3] = math.inf, 1e-30
+    taken, count = [], torch.tensor([read], dtype=torch.int32, device=DEV)
+    take = lambda shape, dtype: taken.append(torch.empty(shape, dtype=dtype, device=DEV)) or taken[-1]
+    y = ops.linear_split(x, w, 64, 1, take=take, read_rows=count)
+    assert torch.equal(y[:read], want[:read]) and bool((y[read:] == 0).all())
+    lost = next(t for t in taken if t.dtype == torch.int32)
+    assert not bool(lost[:-1].any())
+    arena, split = Arena(x.device), ops.SplitWeight(w)
+    assert ops.split_plan(100, 4096, 5120, ops.compute_units(x.device)) is not None
+    arena.read_rows = (100, count)
+    assert bool((product_f32(x, w, split, None, arena)[read:] == 0).all())
+    arena.read_rows = (96, count)  # (a product of other rows)
+    assert read == 100 or not bool(torch.isfinite(product_f32(x, w, split, None, arena)[read:]).all())
+
+
 @pytest.mark.parametrize("keep_plain", [True, False])
 def test_linear_weight_f32_of_many_rows(keep_plain):
     """A float32 matrix through the part's own door, with its second copy and (only one copy is kept) without; both as close as 32-bit sums."""

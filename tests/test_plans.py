@@ -174,6 +174,22 @@ def test_recurrences_leave_out_the_padding_behind_portions():
         assert torch.equal(indptr, ctx.qo_indptr[: 6 - left_out]) and torch.equal(slots, ctx.state_slots[: 5 - left_out])
 
 
+def test_products_are_told_the_rows_that_are_read():
+    """The arena of a captured step with portions knows the stand-in's first row; of any other step that uses it, nothing."""
+    import torch
+
+    from nanospec_amd.engine.arena import Arena
+    from nanospec_amd.engine.context import BatchLayout, StepContext
+
+    layout, arena = BatchLayout(70, 5, 2, 1, 4), Arena("cpu")
+    for kw in (dict(captured=True), dict(captured=True, single_tokens=True), dict()):
+        ctx = StepContext(layout, torch.arange(layout.total, dtype=torch.int32), arena, 0, 64, **kw)
+        if kw == dict(captured=True):
+            assert arena.read_rows[0] == 70 and torch.equal(arena.read_rows[1], ctx.qo_indptr[4:5])
+        else:
+            assert arena.read_rows is None
+
+
 def test_chunks_of_the_delta_rule_beside_single_tokens():
     """Single tokens whose states take as long as a short portion's chain keep that portion token by token."""
     least = lambda portions, heads, dim, singles: ops.delta_chunk_min(portions, heads, dim, dim, singles)

@@ -10,9 +10,11 @@
 // leave the range of 32 bits on their way.  A row of x or of w that has two such values, or one that is not even held to 2^-18, is given to the 32-bit instruction by a launch behind the
 // product (``split_mend_kernel``).  A single one, 10^-8 of its block's largest or less, is one in 10^8 normal values, and every product of a few million would have a row that goes that way for
 // it; two are one row of K 2,048 in 10^9.  (A row that has a value that is no number is none whatever is done with it.)
-// Error against 64 bits (2-norm), this in one range of K and the 32-bit instruction's four chains (gemm_generic.hip): both operands normal, K 2,048 1.7e-7 and 4.1e-7, K 8,192 3.0e-7
-// and 8.1e-7; all of one sign 1.3e-7 and 1.8e-7, 2.5e-7 and 3.5e-7; x spread over 16 powers of two 1.8e-7 and 4.1e-7, 3.3e-7 and 8.1e-7; one k of 512 10^5 times the others 1.9e-7 and
-// 4.6e-7, 3.3e-7 and 8.3e-7, and against zeros in w 1.7e-7 and 4.1e-7, 3.1e-7 and 8.1e-7.  Behind it only where a row is zeros but for one k of 32: 1.7e-7 and 1.1e-7, 3.0e-7 and 2.1e-7.
+// K is cut into segments, four or one by the matrix's sizes, whose sums are added in order, by one workgroup or from one each: an output is the same whatever the tile and the rows beside it.
+// Error against 64 bits (2-norm), the 32-bit instruction's four chains (gemm_generic.hip) and this in four segments and one, K 2,048, and the first two at K 8,192: both operands normal 4.1e-7, 1.3e-7,
+// 1.7e-7, 8.1e-7, 1.8e-7; all of one sign 1.8e-7, 0.5e-7, 1.3e-7, 3.5e-7, 0.7e-7; x spread over 16 powers of two 4.1e-7, 1.4e-7, 1.8e-7, 8.1e-7, 2.2e-7; one k of 512 10^5 times the others 4.6e-7,
+// 1.5e-7, 1.9e-7, 8.3e-7, 2.3e-7, and against zeros in w 4.1e-7, 1.3e-7, 1.7e-7, 8.1e-7, 2.0e-7.  Behind the 32-bit instruction only where a row is zeros but for one k of 32, 1.1e-7, 1.2e-7, 1.7e-7,
+// 2.1e-7, 1.7e-7, or but for one, none and 0.5e-7.
 // (Three bfloat16 values for a float, six products: 1.6e-7 and 3.1e-7 for normal operands, and twice the work of the matrix unit.)
 //
 // Both operands are split ahead, w once for all (as many bytes again as it has), x a call.  w split in registers on its way by every tile of x instead: 211 us for 177 in the first size below beside two others.
@@ -179,11 +181,12 @@ struct SplitParams {
   float* out;  // [M, N], or with ranges of K [ranges][M][N]
   const _Float16 *parts, *w_parts;
   const float* w_scales;
-  int M, N, K, out_stride, m_tiles, n_tiles, ranges;
+  int M, N, K, out_stride, m_tiles, n_tiles, segments, ranges;
 };
 
 // Four waves, 16 MI rows of x by 128 of w.  A stage's parts of x lie in LDS and those of w in the registers of the wave whose columns they are, and the next two are on their way.
-template <int MI>
+// SUMMED: of all segments, one after the other; else of segment blockIdx.y.
+template <int MI, bool SUMMED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_split_kernel(const SplitParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -196,8 +199,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int nt = (turn / p.m_tiles) * 8 + xcd, mt = turn % p.m_tiles;
   if (nt >= p.n_tiles) return;
   const int m0 = mt * TM, n0 = nt * TN, k_blocks = p.K / SPLIT_K;
-  const int from = __builtin_amdgcn_readfirstlane((unsigned)k_blocks * range / p.ranges);  // (fewer than 2^16 of either)
-  const int to = __builtin_amdgcn_readfirstlane((unsigned)k_blocks * (range + 1) / p.ranges);
   const int lane = threadIdx.x % NS_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / NS_WAVE), r = lane % 16, g = lane / 16;
   // blocks of rows that there are; those beyond are the last, their sums are not written
   const int high = min(MI, (p.M + 15) / 16 - mt * MI), wide = min(4 * NJ, (p.N + 15) / 16 - nt * 4 * NJ);
@@ -230,12 +231,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   };
 
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = zero;
-
+  f32x4 acc[MI][NJ], total[MI][NJ];
+  int to = 0;
   auto stage = [&](int at, int kb) {
     // this stage has come, and every wave is done with the one before it, whose place the next but one is given (behind the last stage: that once more, not used)
     TILE_WAIT_LOADS(LOADS);
@@ -279,13 +276,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     join(MI - 1);
     __builtin_amdgcn_sched_barrier(0);
   };
-  load(0, from);
-  load(1, min(from + 1, to - 1));
-  int kb = from;
-  for (; kb + 2 < to; kb += 3) stage(0, kb), stage(1, kb + 1), stage(2, kb + 2);
-  if (kb < to) stage(0, kb);
-  if (kb + 1 < to) stage(1, kb + 1);
-  TILE_WAIT_LOADS(0);  // (what was fetched again behind the last stage must not come into another workgroup's LDS)
+  for (int s = 0; s < (SUMMED ? p.segments : 1); ++s) {
+    const int segment = SUMMED ? s : range;
+    int kb = __builtin_amdgcn_readfirstlane((unsigned)k_blocks * segment / p.segments);  // (fewer than 2^16 of either)
+    to = __builtin_amdgcn_readfirstlane((unsigned)k_blocks * (segment + 1) / p.segments);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = zero;
+    if (s) TILE_BARRIER();  // (every wave is done with the segment before)
+    load(0, kb);
+    load(1, min(kb + 1, to - 1));
+    for (; kb + 2 < to; kb += 3) stage(0, kb), stage(1, kb + 1), stage(2, kb + 2);
+    if (kb < to) stage(0, kb);
+    if (kb + 1 < to) stage(1, kb + 1);
+    TILE_WAIT_LOADS(0);  // (what was fetched again behind the last stage must not come into another stage's LDS, or another workgroup's)
+    if (SUMMED) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) total[i][j] = s ? total[i][j] + acc[i][j] : acc[i][j];
+    }
+  }
 
   // acc[i][j], lane 16 g + r: row 16 i + r of the tile, columns 16 j + 4 g .. + 3 of the wave's
   float* out = p.out + (size_t)range * p.M * p.N;
@@ -305,7 +317,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       if (n >= p.N) continue;
       f32x4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = ldexpf(acc[i][j][e], down[j][e]);
+      for (int e = 0; e < 4; ++e) v[e] = ldexpf((SUMMED ? total : acc)[i][j][e], down[j][e]);
       float* at = out + (size_t)m * p.out_stride + n;
       if (whole)
         *reinterpret_cast<f32x4*>(at) = v;
@@ -324,7 +336,10 @@ static int launch_split(SplitParams p, hipStream_t stream) {
   p.m_tiles = (p.M + 16 * MI - 1) / (16 * MI), p.n_tiles = (p.N + 64 * SPLIT_COLUMNS - 1) / (64 * SPLIT_COLUMNS);
   const long blocks = (long)p.m_tiles * ((p.n_tiles + 7) / 8 * 8);
   if (blocks > (1 << 22)) return NS_ERR_UNSUPPORTED;
-  gemm_split_kernel<MI><<<dim3((unsigned)blocks, p.ranges), 256, 0, stream>>>(p);
+  if (p.ranges == 1 && p.segments > 1)
+    gemm_split_kernel<MI, true><<<(unsigned)blocks, 256, 0, stream>>>(p);
+  else
+    gemm_split_kernel<MI, false><<<dim3((unsigned)blocks, p.ranges), 256, 0, stream>>>(p);
   return ns_launch_status();
 }
 
@@ -469,12 +484,13 @@ extern "C" int ns_split_list(void* list, const void* lost, int M, int K, hipStre
 }
 
 // ``parts``: of x by ns_split_rows without scales; ``w_parts``: of w by ns_split_rows with ``w_scales``, those by ns_split_scales.  ``rows``: of a tile,
-// 64, 96, 112 or 128.  ``ranges`` of K above 1: out is [ranges][M][N] (out_stride N), the sums of each.
+// 64, 96, 112 or 128.  ``segments`` of K, by one workgroup after the other (``ranges`` 1) or by one each (as many): then out is [ranges][M][N] (out_stride N), the sums of each, to be added in order.
 // K a multiple of 32 below 2^19 (a tile's parts within 31 bits of bytes), parts on 16 bytes.  What the parts do not hold is to be put right by ns_split_mend, behind the sum of the ranges.
-extern "C" int ns_gemm_split(void* out, const void* parts, const void* w_parts, const void* w_scales, int M, int N, int K, int out_stride, int rows, int ranges, hipStream_t stream) {
-  if (M <= 0 || N <= 0 || K <= 0 || out_stride < N || ranges < 1 || (ranges > 1 && out_stride != N)) return NS_ERR_BAD_ARG;
-  if (K % SPLIT_K || (((uintptr_t)parts | (uintptr_t)w_parts) & 15) || K >= 1 << 19 || ranges > K / SPLIT_K) return NS_ERR_UNSUPPORTED;
-  const SplitParams p{(float*)out, (const _Float16*)parts, (const _Float16*)w_parts, (const float*)w_scales, M, N, K, out_stride, 0, 0, ranges};
+extern "C" int ns_gemm_split(void* out, const void* parts, const void* w_parts, const void* w_scales, int M, int N, int K, int out_stride, int rows, int segments, int ranges,
+                             hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || out_stride < N || segments < 1 || (ranges != 1 && ranges != segments) || (ranges > 1 && out_stride != N)) return NS_ERR_BAD_ARG;
+  if (K % SPLIT_K || (((uintptr_t)parts | (uintptr_t)w_parts) & 15) || K >= 1 << 19 || segments > K / SPLIT_K) return NS_ERR_UNSUPPORTED;
+  const SplitParams p{(float*)out, (const _Float16*)parts, (const _Float16*)w_parts, (const float*)w_scales, M, N, K, out_stride, 0, 0, segments, ranges};
   switch (rows) {
     case 64: return launch_split<4>(p, stream);
     case 96: return launch_split<6>(p, stream);

@@ -297,18 +297,27 @@ SPLIT_COLUMNS = 128
 SPLIT_K_MULTIPLE = 32
 SPLIT_MIN_ROWS = 48
 SPLIT_MIN_K = 1024
-SPLIT_LONG_K = 4096  # from here on ranges of K are worth their sum until the units have one and a half tiles each
+SPLIT_WIDE = 15360  # ``split_segments``
+SPLIT_LONG_K = 4096  # from here on segments by workgroups of their own are worth their sum until the units have one and a half tiles each
 SPLIT_MIN_WORK = 2e9  # rows times columns times K
 SPLIT_CHUNK_ROWS = 4096  # more are taken in portions, so that the parts of x take no more than 17 KB for each of its columns
 
 
+def split_segments(n: int, k: int) -> int:
+    """Segments of K whose sums ``linear_split`` adds in order, by one workgroup or by one each: an output is the same either way.
+
+    Four, which fill the units where the tiles do not; one for wide matrices, whose tiles of 64 rows alone are ahead of ``linear_generic`` from ``SPLIT_MIN_WORK`` on (64 rows, N 16,384, K 2,048
+    39 and 42 us): a tile's sums then need half the registers (832 rows 189 us, in four segments 199)."""
+    return min(4, k // SPLIT_K_MULTIPLE) if n < SPLIT_WIDE else 1
+
+
 @functools.lru_cache(maxsize=1 << 14)
 def split_plan(m: int, n: int, k: int, units: int) -> tuple[int, int] | None:
-    """(rows of a tile, ranges of K) for ``linear_split``, or None where ``linear_generic`` is the faster one or the sizes are not taken.
+    """(rows of a tile, ranges of K) for ``linear_split``, or None where ``linear_generic`` is the faster one or the sizes are not taken.  An output of more rows is the same for any plan, so from the
+    first number of rows on that has one a matrix's results do not depend on the rows beside.
 
-    Ranges fill the units where the tiles do not, for a sum of them and the tiles' beginnings again.  us alone / beside two others: 832 rows, N 2,048, K 8,192, tiles of 128 rows
-    in one, two, four 237 / 135, 152 / 100, 122 / 102; N 3,072, K 2,048, 96 rows 66 / 35, 65 / 43, 79 / 51; N = K = 2,048, 64 rows 52 / 26, 54 / 31, 57 / 36.  Below
-    ``SPLIT_MIN_WORK`` the splitting of x and a sum of ranges cost alone what the product gains, its time over linear_generic's alone / beside: 1.1 to 1.4e9 (five sizes)
+    Ranges, a segment each, fill the units where the tiles do not, for a sum of them.  us alone, tiles in one and four: 832 rows, N 2,048, K 8,192, 128 rows a tile 214 and 125; N 3,072, K 2,048, 96 rows
+    61 and 63; 512 rows, N = K = 2,048, 64 rows 42 and 33.  Below ``SPLIT_MIN_WORK`` the splitting of x and a sum of ranges cost alone what the product gains, its time over linear_generic's alone / beside: 1.1 to 1.4e9 (five sizes)
     1.04 to 1.25 / 0.94 to 1.46, 1.7e9 0.93 / 0.73, 2 to 3e9 (four) 0.71 to 0.97 / 0.66 to 0.94, 3 to 7e9 (fourteen) 0.58 to 1.01 / 0.33 to 0.59, larger 0.40 to 0.70 / 0.31 to 0.53."""
     if m < SPLIT_MIN_ROWS or k < SPLIT_MIN_K or k % SPLIT_K_MULTIPLE or k >= 1 << 19 or m * n * k < SPLIT_MIN_WORK:
         return None
@@ -317,10 +326,11 @@ def split_plan(m: int, n: int, k: int, units: int) -> tuple[int, int] | None:
     long = k >= SPLIT_LONG_K
     if tiles(64) < 0.25 * units:
         return None
+    segments = split_segments(n, k)
     enough = 1.5 * units if long else 0.75 * units
-    fits = [t for t in SPLIT_TILES if tiles(t[0]) * (4 if long else 1) >= (units if long else enough)]
+    fits = [t for t in SPLIT_TILES if tiles(t[0]) * (segments if long else 1) >= (units if long else enough)]
     rows = min(fits, key=lambda t: -(-m // t[0]) * t[0] * t[1])[0] if fits else SPLIT_TILES[-1][0]
-    return rows, 1 if tiles(rows) >= enough else 2 if 2 * tiles(rows) >= enough else 4
+    return rows, 1 if tiles(rows) >= enough else segments
 
 
 def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -359,7 +369,7 @@ class SplitWeight:
 def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: torch.Tensor | None = None, take=None, split: SplitWeight | None = None,
                  read_rows: torch.Tensor | None = None) -> torch.Tensor:
     """float32 x @ w.T for many rows on the float16 matrix cores, each operand as the sum of two float16 values (``csrc/gemm_split.hip``), in tiles of ``rows`` rows
-    with ``ranges`` ranges of K (``split_plan`` chooses).  The outputs of rows of either that two such values do not stand for (values that lie far apart, infinities) are those of ``linear_generic``
+    with ``ranges`` ranges of K, one or each segment (``split_plan`` chooses, another number makes so many segments).  The outputs of rows of either that two such values do not stand for (values that lie far apart, infinities) are those of ``linear_generic``
     for more than 8 rows.  ``take`` (shape, dtype): scratch, 4.13 K bytes a row of x and with ranges 4 N a row and range.  ``split``: of w; it is made where not given.
     ``read_rows`` (int32 [1] on the GPU): from this row on nobody reads the result, and whatever x holds there it is zeros."""
     out = _check_linear(x, w, out, False)
@@ -384,7 +394,8 @@ def linear_split(x: torch.Tensor, w: torch.Tensor, rows: int, ranges: int, out: 
         _check(lib.ns_split_rows(_ptr(parts), _ptr(lost), call, _ptr(piece), c_void_p(0), _ptr(read_rows), c_int(s), h, c_int(k), c_int(x.stride(0)), _stream()),
                "linear_split")
         _check(lib.ns_gemm_split(_ptr(to if sums is None else sums), _ptr(parts), _ptr(split.parts), _ptr(split.scales), h, c_int(n), c_int(k),
-                                 c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges), _stream()), "linear_split")
+                                 c_int(out.stride(0) if sums is None else n), c_int(rows), c_int(ranges if ranges > 1 else split_segments(n, k)),
+                                 c_int(ranges), _stream()), "linear_split")
         if sums is not None:
             reduce_partial(PartialSums(sums, ranges, piece.shape[0], n, torch.float32), out=to)
         _check(lib.ns_split_mend(_ptr(to), _ptr(piece), _ptr(w), _ptr(lost), call, _ptr(split.lost), h, c_int(n), c_int(k), c_int(x.stride(0)), c_int(out.stride(0)), _stream()), "linear_split")

@@ -264,6 +264,22 @@ def test_linear_split_of_values_far_apart(factor, kind, ranges):
         assert torch.equal(y, ops.linear_generic(x, w))
 
 
+@pytest.mark.parametrize("n,k", [(4096, 1024), (2056, 2080), (130, 4128), (15360, 1056)])
+def test_linear_split_is_the_same_whatever_the_rows_beside(n, k):
+    """Any tile, segments by one workgroup or by one each, any rows beside and any place among them: the same results bit by bit."""
+    ops = _ops()
+    torch.manual_seed(n)
+    x, w = torch.randn(600, k, device=DEV), torch.randn(n, k, device=DEV)
+    x[7, 3] = math.inf  # (a row of the 32-bit instruction beside the others)
+    split = ops.SplitWeight(w)
+    want = ops.linear_split(x, w, 64, 1, split=split)
+    for rows in (64, 96, 112, 128):
+        for ranges in (1, ops.split_segments(n, k)):
+            assert torch.equal(ops.linear_split(x, w, rows, ranges, split=split), want)
+            assert torch.equal(ops.linear_split(x[5:305], w, rows, ranges, split=split), want[5:305])
+    assert torch.equal(ops.linear_generic(x, w)[7], want[7])
+
+
 @pytest.mark.parametrize("read", [0, 1, 16, 77, 100])
 def test_linear_split_of_rows_that_nobody_reads(read):
     """Padding rows are zeros whatever lies there, and none of them is left to the 32-bit instruction; the others are as they are without them, through the part's own door too."""

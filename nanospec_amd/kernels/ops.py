@@ -787,6 +787,13 @@ def many_f32_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     return w.shape[1] >= MANY_K_MIN and w.shape[0] % 4 == 0 and many_takes(x, w)
 
 
+def many_f32_ranges(m: int, n: int, k: int, units: int) -> int | None:
+    """Ranges of K for a float32 result by ``linear_many``: no fewer than ``linear_rows`` sums (``rows_plan``), so that no chain of sums is longer than there, in whole pieces; None where K is not
+    cut like that."""
+    least = rows_plan(n, k, m, units=units)[0]
+    return next((r for r in range(least, 17) if k % (MANY_K_MULTIPLE * r) == 0 and k // r >= 256), None)
+
+
 def many_writes(out: torch.Tensor, m: int, n: int) -> bool:
     """Whether ``linear_many`` can write a result of m rows and n columns there: whole pieces of four values."""
     return out.shape == (m, n) and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0

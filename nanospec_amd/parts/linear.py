@@ -242,10 +242,20 @@ class LinearWeight:
         if self.k % 8 or not ops.tiled_takes(x[:1], self.k):
             return ops.linear_generic(x, self.plain, out=out, out_f32=out_f32)
         m = x.shape[0]
-        if out_f32 and m >= ops.MANY_MIN_ROWS and self.plain is not None and ops.many_f32_takes(x, self.plain) and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0):
-            # (2,048 columns, K 4,096, us in blocks of 128 rows from the re-laid copy and here, alone / beside two others: 130 rows 44 / 34, 32 / 22, 508 50 / 29, 32 / 20, 2,048 83 / 68,
-            # 40 / 31; 4,096 columns, K 8,192, 130 rows 58 / 38, 54 / 27, 2,048 219 / 207, 118 / 113; two or four ranges of K are level beside others at best)
-            return ops.linear_many(x, self.plain, out if out is not None else torch.empty((m, self.n), dtype=torch.float32, device=x.device), ops.MANY_SPLIT_FORM)
+        ranges = None
+        if (out_f32 and m >= ops.MANY_MIN_ROWS and self.plain is not None and ops.many_f32_takes(x, self.plain)
+                and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0)):
+            ranges = ops.many_f32_ranges(m, self.n, self.k, ops.compute_units(x.device))
+        if ranges is not None:
+            # (us in blocks of 128 rows from the re-laid copy and here, alone / beside two others: 2,048 columns, K 4,096, 130 rows 28.8 / 24.8, 15.3 / 9.7, 508 37.7 / 30.8, 21.1 / 15.5, 2,048 71 / 66,
+            # 46 / 42; 4,096 columns, K 8,192, 508 rows 69 / 64, 44 / 40, 2,048 203 / 205, 114 / 117.  Both 1.9e-7 to 5.7e-7 from 64 bits, the same of either; in one range 35 / 34 in the third of these, but
+            # 4.0e-7 for 2.7e-7)
+            if out is None:
+                out = torch.empty((m, self.n), dtype=torch.float32, device=x.device)
+            if ranges == 1:
+                return ops.linear_many(x, self.plain, out, ops.MANY_SPLIT_FORM)
+            sums = arena.take((ranges * m * self.n,), torch.float32) if arena is not None else torch.empty(ranges * m * self.n, dtype=torch.float32, device=x.device)
+            return ops.reduce_partial(ops.linear_many(x, self.plain, sums, ops.MANY_SPLIT_FORM, ranges=ranges), out=out)
         if self.tiled is not None and WIDE_HEAD_ROWS < m <= STREAM_ROWS and out_f32 and self.n >= 8192:
             return ops.linear_wide(x, self.tiled, out=out, out_f32=True, ksplit=1, nt=1)
         if self.tiled is not None and m <= STREAM_ROWS:

@@ -244,7 +244,7 @@ class LinearWeight:
         m = x.shape[0]
         ranges = None
         if (out_f32 and m >= ops.MANY_MIN_ROWS and self.plain is not None and ops.many_f32_takes(x, self.plain)
-                and (out is None or out.is_contiguous() and out.data_ptr() % 16 == 0)):
+                and (out is None or out.dtype == torch.float32 and out.is_contiguous() and out.data_ptr() % 16 == 0)):
             ranges = ops.many_f32_ranges(m, self.n, self.k, ops.compute_units(x.device))
         if ranges is not None:
             # (us in blocks of 128 rows from the re-laid copy and here, alone / beside two others: 2,048 columns, K 4,096, 130 rows 28.8 / 24.8, 15.3 / 9.7, 508 37.7 / 30.8, 21.1 / 15.5, 2,048 71 / 66,

@@ -498,6 +498,8 @@ def test_linear_many_f32(m, n, k):
     arena, into = Arena(x.device), torch.empty(m, n, device=DEV)
     for z in (LinearWeight(w)(x, out_f32=True), LinearWeight(w)(x, out=into, out_f32=True, arena=arena)):
         assert far(z) <= (1 + 8 * (m * n) ** -0.5) * far(LinearWeight(w, keep_plain=False)(x, out_f32=True)) and bool(((z.cpu().double() - a @ b.T).abs() <= bound).all())
+    with pytest.raises(ops.KernelRefused):  # (a 32-bit result does not go into a bfloat16 tensor)
+        LinearWeight(w)(x, out=torch.empty(m, n, dtype=torch.bfloat16, device=DEV), out_f32=True)
     for bad in (dict(act="silu"), dict(add=True), dict(out=torch.empty(m, 2 * n, device=DEV)[:, :n]), dict(form=0)):
         with pytest.raises(ops.KernelRefused):
             ops.linear_many(**{**dict(x=x, w=w, out=y, form=ops.MANY_SPLIT_FORM), **bad})

@@ -50,7 +50,7 @@ __global__ void conv_silu_kernel(float* __restrict__ out, T* __restrict__ copy, 
 // 64 bytes a thread and an input is read by K tokens, for 8 bytes of new input and 16 of result.  UNITS: the first ``vectors`` runs of 4 LANES channels then become unit
 // vectors, as delta_prep_kernel makes them, while their sums of squares are at hand (C a multiple of 4 LANES): as a kernel of its own that reads and writes them again.
 // Bound by the results' bytes: 2,048 tokens of 6,144 channels, 4 taps, bfloat16, a token a thread 35.0 / 27.2 us (alone / beside two
-// others) and the unit vectors and decays behind it 38.3 / 31.8, both in a row 69.1 / 57.4; so 30.6 / 19.8 and (decays alone) 18.7 / 14.3, 46.3 / 31.5.  Strips of four or two: level.
+// others) and the unit vectors and decays behind it 38.3 / 31.8, both in a row 69.1 / 57.4; so 30.6 / 19.8 and (decays alone) 18.7 / 14.3, 46.3 / 31.5.
 template <int LANES>
 __device__ __forceinline__ float unit_scale(const float* y, bool first_half) {
   float ss = 0.f;
@@ -167,8 +167,10 @@ __global__ void conv_carry_kernel(const T* __restrict__ x, int x_stride, float* 
   }
 }
 
-#define CONV_STRIP 8
-#define CONV_STRIP_TOKENS 512  // from so many on (fewer would leave too few workgroups)
+#define CONV_STRIP 8     // tokens of a strip at most
+// Workgroups that a step's strips come to at least, else they are shorter: two a compute unit.  us with the carry, strips of 1, 2, 4 and 8: 512 tokens of 2,048 channels 7.9, 7.5, 8.0, 9.8, of 2,304
+// 8.2, 8.1, 8.6, 9.8, of 6,144 14.6, 13.4, 12.4, 13.6; 1,024 of 6,144 21.4, 18.6, 18.5, 18.2; 2,048 of 2,048 17.0, 15.2, 14.8, 14.2; of 6,144 33.5, 28.1, 26.0, 25.5.
+#define CONV_GROUPS 512
 
 // ``single``: every request brings one token (at most); one kernel then does both.  ``unit_vectors`` (an even number, or 0): so many first runs of ``unit_size`` channels become unit
 // vectors, the first half of them times unit_size^(-1/2); unit_size a power of two from 8 to 256, and sizes and addresses as the kernel in pieces wants them (NS_ERR_UNSUPPORTED).
@@ -187,8 +189,10 @@ extern "C" int ns_conv_silu_carry(float* out, void* copy, const void* x, int x_s
   if (unit_vectors && !(vec && unit_size >= 8 && unit_size <= 256 && (unit_size & (unit_size - 1)) == 0)) return NS_ERR_UNSUPPORTED;
   if (vec) {
     const ConvUnits units{unit_vectors, unit_vectors ? unit_size / 4 : 1};
-    const bool strips = n_tokens >= CONV_STRIP_TOKENS && !single;
-    const dim3 grid(strips ? (n_tokens + CONV_STRIP - 1) / CONV_STRIP : n_tokens, (C / 4 + 255) / 256);
+    const int across = (C / 4 + 255) / 256;
+    int strip = single ? 1 : CONV_STRIP;
+    while (strip > 1 && (long long)((n_tokens + strip - 1) / strip) * across < CONV_GROUPS) strip /= 2;
+    const dim3 grid((n_tokens + strip - 1) / strip, across);
     auto launch = [&](auto* in, auto taps_of, auto strip) {
       typedef typename std::remove_const<typename std::remove_pointer<decltype(in)>::type>::type T;
       conv_silu_vec_kernel<T, decltype(taps_of)::value, decltype(strip)::value><<<grid, 256, 0, stream>>>(
@@ -203,10 +207,12 @@ extern "C" int ns_conv_silu_carry(float* out, void* copy, const void* x, int x_s
         launch(in, std::integral_constant<int, 4>(), strip);
     };
     auto of_strip = [&](auto* in) {
-      if (strips)
-        of_taps(in, std::integral_constant<int, CONV_STRIP>());
-      else
-        of_taps(in, std::integral_constant<int, 1>());
+      switch (strip) {
+        case 8: return of_taps(in, std::integral_constant<int, 8>());
+        case 4: return of_taps(in, std::integral_constant<int, 4>());
+        case 2: return of_taps(in, std::integral_constant<int, 2>());
+        default: of_taps(in, std::integral_constant<int, 1>());
+      }
     };
     if (dtype == NS_DTYPE_F32)
       of_strip((const float*)x);

@@ -435,10 +435,10 @@ def test_convolution_carries_its_inputs_across_steps(K, C, pad, off):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("K", [2, 3, 4])
-@pytest.mark.parametrize("vectors,size,rest", [(2, 8, 4), (4, 128, 60), (2, 256, 8), (6, 16, 1000), (2, 32, 0)])
+@pytest.mark.parametrize("vectors,size,rest", [(2, 8, 4), (4, 128, 60), (2, 256, 8), (6, 16, 1000), (2, 32, 0), (4, 64, 1500), (4, 128, 3000), (4, 128, 7500)])
 def test_convolution_in_strips_with_unit_vectors(dtype, K, vectors, size, rest):
-    """Strips of eight tokens that requests begin and end inside of, a request shorter than the taps, a last strip that is not full, and a step too short for strips; unit vectors
-    made of the first channels behind it; then the decays alone."""
+    """Single tokens and (by the channels) strips of two, four and eight that requests begin and end inside of, a request shorter than the taps, a last strip that is not full, and a step too short for
+    strips; unit vectors made of the first channels behind it; then the decays alone."""
     from nanospec_amd.kernels import ops
 
     torch.manual_seed(K + size)

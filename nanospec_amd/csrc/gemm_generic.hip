@@ -140,10 +140,10 @@ static int launch_rows_f32(float* out, const float* x, const float* w, int M, in
   if constexpr (MT < ROWS_M)
     if (M > MT) return launch_rows_f32<MT + 1>(out, x, w, M, N, K, x_stride, out_stride, stream);
   const int blocks = (N + ROWS_N - 1) / ROWS_N;
-  // Four waves where a row is then no more than two loads a lane (the sums of a longer chain are further from 64 bits: K 8,192 1.3e-7 instead of 1.15e-7) and there are two
-  // workgroups for every compute unit: five rows, N 128,256, K 2,048 158 us, with eight waves 169; N 32,000, K 1,024 25 and 32; N 3,072, K 2,048 9.1 and 9.2; N 512 5.2 and 4.4.
+  // Four waves where a row is then one load a lane or two of every lane (the sums of a longer chain are further from 64 bits: K 8,192 1.3e-7 instead of 1.15e-7; of chains of two lengths too: K 1,536
+  // 9.37e-8 instead of 9.25e-8; K 2,048 9.49e-8 instead of 9.58e-8) and there are two workgroups for every compute unit: five rows, N 128,256, K 2,048 158 us, with eight waves 169; N 32,000, K 1,024 25 and 32; N 3,072, K 2,048 9.1 and 9.2; N 512 5.2 and 4.4.
   // (The sums depend on this choice, so it is the same for any number of rows.)
-  if (K <= 2048 && N >= 4096)
+  if ((K <= 1024 || K == 2048) && N >= 4096)
     gemm_rows_f32_kernel<MT, 4><<<blocks, 256, 0, stream>>>(out, x, w, N, K, x_stride, out_stride);
   else
     gemm_rows_f32_kernel<MT, 8><<<blocks, 512, 0, stream>>>(out, x, w, N, K, x_stride, out_stride);

@@ -128,6 +128,7 @@ struct KvRows {
   float eps;
   RopeForm form;
   int norm_q, norm_k, v_is_k;
+  int first;  // head: the queries before it stay as they are
   const T *lambda, *v_other;  // values <- (1 - lambda) values + lambda v_other
   T* v_keep;
   int v_other_stride, v_keep_stride;
@@ -265,8 +266,8 @@ __global__ __launch_bounds__(512) void head_rows_kernel(const KvRows<T> p) {
     __syncthreads();
   }
   // (a head's lanes stand in one wave and go round together)
-  for (int u = blockIdx.y * blockDim.x + threadIdx.x; u < (p.heads + p.kv_heads) * p.lanes; u += p.shares * blockDim.x) {
-    const int h = u / p.lanes;
+  for (int u = blockIdx.y * blockDim.x + threadIdx.x; u < (p.heads - p.first + p.kv_heads) * p.lanes; u += p.shares * blockDim.x) {
+    const int h = p.first + u / p.lanes;
     const bool is_q = h < p.heads, normed = is_q ? p.norm_q : p.norm_k;
     int d1, d2;
     unit_of(p, u % p.lanes, d1, d2);
@@ -353,7 +354,7 @@ static dim3 kv_rows_grid(const KvRows<T>& p) { return dim3(p.n_tokens, p.shares 
 
 template <typename T>
 static void launch_head_rows(KvRows<T> p, hipStream_t stream) {
-  const int units = (p.heads + p.kv_heads) * p.lanes;
+  const int units = (p.heads - p.first + p.kv_heads) * p.lanes;
   p.shares = p.n_tokens < FEW_TOKENS ? (units + 255) / 256 : 1;
   const int rounds = p.shares > 1 ? p.shares : (units + 511) / 512;  // (as even as whole waves allow)
   int threads = ((units + rounds - 1) / rounds + NS_WAVE - 1) / NS_WAVE * NS_WAVE;
@@ -413,7 +414,7 @@ extern "C" int ns_unit_kv_write(void* qkv, int stride, const int* positions, con
     KvRows<typename std::remove_pointer<decltype(rows)>::type> p{};
     p.qkv = rows, p.k_cache = k, p.v_cache = v, p.positions = positions, p.token_req = token_req, p.block_table = block_table;
     p.stride = stride, p.table_stride = table_stride, p.n_tokens = n_tokens, p.heads = heads, p.kv_heads = own_kv ? kv_heads : 0, p.hd = hd, p.vd = vd, p.page_size = page_size;
-    p.eps = eps, p.norm_q = p.norm_k = eps >= 0.f;
+    p.eps = eps, p.norm_q = p.norm_k = eps >= 0.f, p.first = eps >= 0.f ? 0 : heads;
     if (!kv_rows_take(p)) return false;
     if (own_kv || eps >= 0.f) launch_head_rows(p, stream);
     return true;

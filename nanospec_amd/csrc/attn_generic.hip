@@ -199,9 +199,9 @@ __device__ __forceinline__ void finish_unit(const KvRows<T>& p, T* row, int h, i
   store_piece(to + d1, a), store_piece(to + d2, b);
 }
 
-// The values of a token, or of a run of tokens by its first.
+// The values of a token, or of a run of tokens by its first; part ``part`` of ``parts`` of them.
 template <typename T>
-__device__ __forceinline__ void write_values(const KvRows<T>& p, int t) {
+__device__ __forceinline__ void write_values(const KvRows<T>& p, int t, int part, int parts) {
   constexpr int H = KvPiece<T>::H, V = 2 * H;
   typedef T run_t __attribute__((ext_vector_type(V)));
   const int lane = threadIdx.x % NS_WAVE, req = p.token_req[t], pos = p.positions[t], slot = pos % p.page_size, nq = p.heads * p.hd;
@@ -217,7 +217,7 @@ __device__ __forceinline__ void write_values(const KvRows<T>& p, int t) {
   const int at = p.v_is_k ? nq : nq + p.kv_heads * p.hd;  // of the values in a row
   const float lam = p.lambda && p.v_other ? to_f(p.lambda[0]) : 0.f;
   // (neighbouring lanes have neighbouring channels, whose runs in a page are neighbours: four channels a lane, whose stores lie 128 bytes apart, 19.9 / 13.1 us in the first line above)
-  for (int c = threadIdx.x; c < p.kv_heads * p.vd; c += blockDim.x) {
+  for (int c = part * blockDim.x + threadIdx.x; c < p.kv_heads * p.vd; c += parts * blockDim.x) {
     T* to = p.v_cache + ((size_t)page * p.kv_heads * p.vd + c) * p.page_size + slot;  // (a page's heads and their channels lie one behind the other)
     const T *from = p.qkv + (size_t)t * p.stride + at + c, *from_other = p.v_other ? p.v_other + (size_t)t * p.v_other_stride + c : nullptr;
     const float bias = p.bias ? to_f(p.bias[at + c]) : 0.f;
@@ -245,9 +245,9 @@ __device__ __forceinline__ void write_values(const KvRows<T>& p, int t) {
   }
 }
 
-// Few tokens: ``shares`` workgroups for a token's heads and one more for its values (8 tokens 6.7 -> 3.8 us, 64 tokens of 40 heads of 128 6.4 -> 5.5); many: one for all of it.
+// Few tokens: ``shares`` workgroups for a token's heads and more for its values, a value a thread (8 tokens 6.7 -> 3.8 us, 64 tokens of 40 heads of 128 6.4 -> 5.5); many: one for all of it.
 template <typename T>
-__device__ __forceinline__ bool only_values(const KvRows<T>& p) { return (int)blockIdx.y == p.shares; }
+__device__ __forceinline__ bool only_values(const KvRows<T>& p) { return (int)blockIdx.y >= p.shares; }
 template <typename T>
 __device__ __forceinline__ bool values_too(const KvRows<T>& p) { return p.kv_heads && gridDim.y == 1; }
 
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(512) void head_rows_kernel(const KvRows<T> p) {
   constexpr int H = KvPiece<T>::H;
   extern __shared__ float cs[];  // cos[rot / 2] | sin[rot / 2]
   const int t = blockIdx.x;
-  if (only_values(p)) return write_values(p, t);
+  if (only_values(p)) return write_values(p, t, blockIdx.y - p.shares, gridDim.y - p.shares);
   const int pos = p.positions[t], half = p.form.rot / 2;
   T* row = p.qkv + (size_t)t * p.stride;
   const int page = p.kv_heads ? p.block_table[(size_t)p.token_req[t] * p.table_stride + pos / p.page_size] : 0, slot = pos % p.page_size;
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(512) void head_rows_kernel(const KvRows<T> p) {
     }
     finish_unit(p, row, h, d1, d2, a, b, 1.f / sqrtf(ss / (float)p.hd + p.eps), normed, is_q ? p.qw : p.kw, cs, page, slot);
   }
-  if (values_too(p)) write_values(p, t);
+  if (values_too(p)) write_values(p, t, 0, 1);
 }
 
 // A norm over all heads of q and one over all of k; a thread keeps up to UNITS units between the sums and what follows them.
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(1024) void whole_rows_kernel(const KvRows<T> p) {
   extern __shared__ float cs[];  // cos[rot / 2] | sin[rot / 2]
   __shared__ float sums[2][16];
   const int t = blockIdx.x;
-  if (only_values(p)) return write_values(p, t);
+  if (only_values(p)) return write_values(p, t, blockIdx.y - p.shares, gridDim.y - p.shares);
   const int pos = p.positions[t], half = p.form.rot / 2, units = (p.heads + p.kv_heads) * p.lanes;
   T* row = p.qkv + (size_t)t * p.stride;
   const int page = p.block_table[(size_t)p.token_req[t] * p.table_stride + pos / p.page_size], slot = pos % p.page_size;
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(1024) void whole_rows_kernel(const KvRows<T> p) {
     const T* w = is_q ? p.qw : p.kw;
     finish_unit(p, row, h, d1, d2, a[i], b[i], is_q ? fq : fk, is_q ? p.norm_q : p.norm_k, w ? w + (size_t)(is_q ? h : h - p.heads) * p.hd : nullptr, cs, page, slot);
   }
-  if (values_too(p)) write_values(p, t);
+  if (values_too(p)) write_values(p, t, 0, 1);
 }
 
 // Whether the kernels above take these sizes and addresses; sets ``lanes``.
@@ -348,9 +348,15 @@ static bool kv_rows_take(KvRows<T>& p) {
   return p.kv_heads == 0 || ((uintptr_t)p.v_cache & 15) == 0;
 }
 
-#define FEW_TOKENS 256
+// (a workgroup that writes a run's values behind its heads is the last to end while the units have few of them: us, values behind the heads and by workgroups of their own, bfloat16, a norm a head and a
+// norm of the projection with rotation: 300 tokens of 32 heads of 128 over 8 9.8 and 6.2, 10.8 and 6.5; 700 11.7 and 9.8, 12.9 and 11.2; of 64 8.0 and 6.7, 10.0 and 6.7; 1,024 of 128 11.7 and 14.9, of 64 8.2
+// and 8.9)
+#define FEW_TOKENS 1024
 template <typename T>
-static dim3 kv_rows_grid(const KvRows<T>& p) { return dim3(p.n_tokens, p.shares + (p.kv_heads && p.n_tokens < FEW_TOKENS)); }
+static dim3 kv_rows_grid(const KvRows<T>& p, int threads) {
+  const int parts = p.n_tokens < FEW_TOKENS ? (p.kv_heads * p.vd + threads - 1) / threads : 0;  // (of a token's values; none of its own: none)
+  return dim3(p.n_tokens, p.shares + parts);
+}
 
 template <typename T>
 static void launch_head_rows(KvRows<T> p, hipStream_t stream) {
@@ -359,7 +365,7 @@ static void launch_head_rows(KvRows<T> p, hipStream_t stream) {
   const int rounds = p.shares > 1 ? p.shares : (units + 511) / 512;  // (as even as whole waves allow)
   int threads = ((units + rounds - 1) / rounds + NS_WAVE - 1) / NS_WAVE * NS_WAVE;
   if (threads < 256 && p.kv_heads * p.vd > threads) threads = p.kv_heads * p.vd < 256 ? (p.kv_heads * p.vd + NS_WAVE - 1) / NS_WAVE * NS_WAVE : 256;
-  head_rows_kernel<T><<<kv_rows_grid(p), threads, p.form.rot * sizeof(float), stream>>>(p);
+  head_rows_kernel<T><<<kv_rows_grid(p, threads), threads, p.form.rot * sizeof(float), stream>>>(p);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -545,7 +551,8 @@ extern "C" int ns_whole_norm_kv_write(void* qkv, int stride, const void* bias, c
     // few tokens: a unit a thread, if there are threads
     const int wanted = n_tokens <= 64 && units <= 1024 ? units : each;
     p.shares = 1;
-    whole_rows_kernel<T><<<kv_rows_grid(p), (wanted + NS_WAVE - 1) / NS_WAVE * NS_WAVE, rot * sizeof(float), stream>>>(p);
+    const int threads = (wanted + NS_WAVE - 1) / NS_WAVE * NS_WAVE;
+    whole_rows_kernel<T><<<kv_rows_grid(p, threads), threads, rot * sizeof(float), stream>>>(p);
     return true;
   };
   if (dtype == NS_DTYPE_F32 ? in_pieces((float*)qkv) : dtype == NS_DTYPE_BF16 && in_pieces((bf16_t*)qkv)) return ns_launch_status();

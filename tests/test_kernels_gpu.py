@@ -237,6 +237,42 @@ def test_keys_and_values_in_pieces(dtype, order, kind, H, G, D, E, page, rot, in
         assert bool((got[0][1].cpu().transpose(1, 2)[blank] == 0).all()) and bool((got[0][2].cpu().permute(0, 3, 1, 2)[blank] == 0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("n", [65, 255, 300, 1023, 1024, 1301])
+@pytest.mark.parametrize("kind,H,G,D,E,page,rot", [("unit", 6, 2, 64, 64, 16, 0), ("unit", 40, 8, 128, 96, 16, 0), ("bare", 5, 3, 32, 40, 8, 0), ("head", 6, 2, 64, 64, 16, 32),
+                                                   ("head", 40, 10, 128, 128, 32, 128), ("same", 40, 10, 64, 64, 16, 64), ("whole", 32, 8, 64, 64, 16, 64), ("whole", 64, 16, 64, 80, 4, 0)])
+def test_keys_and_values_in_pieces_of_many_tokens(dtype, n, kind, H, G, D, E, page, rot):
+    """The forms that prompts take (values by workgroups of their own and behind the heads, heads in several rounds, one unit or two a thread), two requests of odd lengths that begin inside a run of a page:
+    against the plain kernels, every place of the pages."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n + H)
+    first, starts = n // 3 | 1, (5, 3)
+    pos = torch.cat([torch.arange(first) + starts[0], torch.arange(n - first) + starts[1]]).int().to(DEV)
+    req = torch.cat([torch.zeros(first), torch.ones(n - first)]).int().to(DEV)
+    width = H * D + G * (D + (0 if kind == "same" else E))
+    make = lambda *shape: (2.0 * torch.randn(*shape, generator=g)).to(dtype).to(DEV)
+    rows, bias = make(n, width), make(width)
+    per = 1 if kind in ("head", "same") else H
+    qw, kw, inv = make(per * D), make((1 if per == 1 else G) * D), torch.rand(max(1, rot // 2), generator=g).to(DEV)
+    pages = 1 + (n + 8) // page
+    table = torch.randperm(2 * pages, generator=g).to(torch.int32).view(2, pages).to(DEV)
+    got = []
+    for extra in (0, 3):  # (rows of whole pieces; three columns more)
+        wide = torch.full((n, width + 8 * (extra > 0) + extra), 5.0, dtype=dtype, device=DEV)
+        wide[:, :width] = rows
+        kc, vc = torch.full((2 * pages, G, page, D), 3.0, dtype=dtype, device=DEV), torch.full((2 * pages, G, E, page), 3.0, dtype=dtype, device=DEV)
+        x = wide[:, : wide.shape[1] - extra] if extra else wide
+        if kind in ("unit", "bare"):
+            ops.unit_kv_write(x, pos, req, table, kc, vc, H, G, D, E, None if kind == "bare" else 1e-3, own_kv=True)
+        elif kind in ("head", "same"):
+            ops.head_norm_rope_kv_write(x, pos, req, table, inv[: rot // 2], kc, vc, H, G, D, E, 1e-3, rot, bias=bias, q_weight=qw, k_weight=kw, value_is_key=kind == "same")
+        else:
+            ops.whole_norm_kv_write(x, pos, req, table, kc, vc, H, G, D, E, 1e-3, bias=bias, q_weight=qw, k_weight=kw, inv_freq=inv if rot else None, rotary_dim=rot)
+        got.append((wide[:, :width], kc, vc))
+    tol = dict(rtol=2.0**-19, atol=2.0**-18) if dtype == torch.float32 else dict(rtol=2.0**-7, atol=2.0**-8)  # (as above)
+    assert torch.allclose(got[0][0], got[1][0], **tol) and torch.allclose(got[0][1], got[1][1], **tol) and torch.equal(got[0][2], got[1][2])
+
+
 @pytest.mark.parametrize("spread", [12, 24])
 def test_linear_split_of_wide_rows(spread):
     """Values over many powers of two within a block of x and a row of w: the parts of the small ones lie below the float16 numbers of full precision, not below all of them."""

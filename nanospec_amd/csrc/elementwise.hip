@@ -695,9 +695,12 @@ extern "C" int ns_fill_u32(void* p, uint32_t value, size_t n_words, hipStream_t 
 __global__ __launch_bounds__(256) void clear_slots_kernel(const uint64_t* __restrict__ table, int slot) {
   const uint64_t bytes = table[2 * blockIdx.y + 1], from = table[2 * blockIdx.y] + bytes * slot;
   const uint64_t first = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
-  const uint64_t whole = (from & 15) ? 0 : bytes / 16;
-  for (uint64_t i = first; i < whole; i += step) reinterpret_cast<int4*>(from)[i] = int4{0, 0, 0, 0};
-  for (uint64_t i = 16 * whole + first; i < bytes; i += step) reinterpret_cast<char*>(from)[i] = 0;
+  // (a slot may begin and end inside of 16 bytes)
+  const uint64_t before = min(-from & 15, bytes), whole = (bytes - before) / 16, behind = bytes - before - 16 * whole;
+  int4* middle = reinterpret_cast<int4*>(from + before);
+  for (uint64_t i = first; i < whole; i += step) middle[i] = int4{0, 0, 0, 0};
+  if (first < before) reinterpret_cast<char*>(from)[first] = 0;
+  if (first < behind) reinterpret_cast<char*>(middle + whole)[first] = 0;
 }
 // ``most``: the largest slot's bytes (how many workgroups share a tensor).
 extern "C" int ns_clear_slots(const void* table, int count, int slot, size_t most, hipStream_t stream) {

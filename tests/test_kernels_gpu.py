@@ -369,7 +369,7 @@ def test_linear_weight_f32_of_many_rows(keep_plain):
     assert float((y - ref).norm() / ref.norm()) <= (3e-7 if keep_plain else 6e-7)  # 1.8e-7 and 4.1e-7 measured at K 2,048
 
 
-@pytest.mark.parametrize("shapes", [[(1,)], [(3, 5), (1,), (7,)], [(16, 128, 257), (2, 2048), (1,), (13,)]])
+@pytest.mark.parametrize("shapes", [[(1,)], [(3, 5), (1,), (7,)], [(16, 128, 257), (2, 2048), (1,), (13,)], [(9,), (8 * 257,), (65, 1023), (4, 3)]])
 def test_slot_tensors(shapes):
     """One slot of every tensor is cleared and nothing beside it: slots of single words, of odd numbers of values, of many blocks."""
     ops = _ops()

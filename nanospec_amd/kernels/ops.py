@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import itertools
+import math
 from ctypes import c_float, c_int, c_size_t, c_uint32, c_void_p
 
 import torch
@@ -245,7 +246,7 @@ class SlotTensors:
         if not tensors or any(not t.is_contiguous() or t.shape[0] != tensors[0].shape[0] for t in tensors):
             raise KernelRefused("SlotTensors takes contiguous tensors of one number of slots")
         self.tensors, self.slots = list(tensors), tensors[0].shape[0]
-        sizes = [t[0].numel() * t.element_size() for t in tensors]
+        sizes = [math.prod(t.shape[1:]) * t.element_size() for t in tensors]  # (there may be no slot at all)
         self.most = max(sizes)
         self.table = torch.tensor([v for t, n in zip(tensors, sizes) for v in (t.data_ptr(), n)], dtype=torch.int64).to(tensors[0].device)
 

@@ -383,6 +383,8 @@ def test_slot_tensors(shapes):
     for bad in (-1, 5):
         with pytest.raises(ops.KernelRefused):
             slots.clear(bad)
+    with pytest.raises(ops.KernelRefused):  # (no slots: nothing to clear, but a table all the same)
+        ops.SlotTensors([t[:0] for t in tensors]).clear(0)
 
 
 def test_many_f32_ranges():

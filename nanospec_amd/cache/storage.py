@@ -21,6 +21,9 @@ from ..parts.needs import PagedNeed, StateNeed, each_need
 from .manager import GroupSpec
 
 
+STEPS_SHARE = 0.1  # of the device's memory that is to be left for the steps beside weights, pages and states
+
+
 @dataclass
 class PagedView:
     group: int
@@ -58,6 +61,23 @@ def plan_groups(cache_needs: list) -> tuple[list[GroupSpec], list[PagedNeed], li
 
 class CacheStorage:
     def __init__(self, model, num_pages: list[int], page_size: int, num_slots: int, dtype, device) -> None:
+        # what a model keeps only to be faster makes room: where the pages do not fit beside it, or leave little for the steps
+        give_back = getattr(model, "give_back_second_copies", lambda: False)
+        short = False
+        try:
+            self._allocate(model, num_pages, page_size, num_slots, dtype, device)
+        except torch.OutOfMemoryError:
+            short = True
+        if short:  # (behind the handler, whose traceback holds what had been allocated)
+            self.__dict__.clear()
+            give_back()
+            self._allocate(model, num_pages, page_size, num_slots, dtype, device)
+        elif torch.device(device).type == "cuda":
+            free, total = torch.cuda.mem_get_info(device)
+            if free + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device) < STEPS_SHARE * total:
+                give_back()
+
+    def _allocate(self, model, num_pages: list[int], page_size: int, num_slots: int, dtype, device) -> None:
         self.group_specs, needs, of_entry = plan_groups(model.cache_needs)
         self.page_size = page_size
         flat = [(single, i) for i, (need, call) in enumerate(zip(model.cache_needs, model.spec.run_order)) if call.cache_from is None

@@ -103,6 +103,7 @@ class ModelRunner:
     def __init__(self, model, manager: CacheManager, storage: CacheStorage, max_requests: int, table_width: int,
                  use_graphs: bool = True) -> None:
         self.model, self.manager, self.storage = model, manager, storage
+        model.has_runner = True
         self.device, self.dtype = model.device, model.dtype
         self.page_size = manager.page_size
         self.table_width = table_width  # the most pages that a request's block table can name

@@ -119,6 +119,19 @@ def product_f32(x: torch.Tensor, w: torch.Tensor, split: "ops.SplitWeight | None
     return out
 
 
+def second_copies(part, seen: set | None = None):
+    """The weights within ``part`` that keep a second copy of a float32 matrix (``split_weight``)."""
+    seen = set() if seen is None else seen
+    if id(part) in seen:
+        return
+    seen.add(id(part))
+    if isinstance(part, (LinearWeight, GatedWeights)) and part._split is not None:
+        yield part
+    inside = part if isinstance(part, (list, tuple)) else part.values() if isinstance(part, dict) else vars(part).values() if type(part).__module__.startswith(__package__) else ()
+    for one in inside:
+        yield from second_copies(one, seen)
+
+
 class IntoResidual:
     """Asks a part to hand its output to the residual stream and the RMS norm after it in the cheapest form its last
     product has, instead of returning a finished tensor:

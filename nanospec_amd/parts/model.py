@@ -11,7 +11,7 @@ import torch
 from ..kernels import ops
 from ..weights import source as wsource
 from . import registry
-from .linear import LAYOUTS, LinearWeight
+from .linear import LAYOUTS, LinearWeight, second_copies
 from .needs import PagedNeed, StateNeed
 
 
@@ -49,6 +49,7 @@ class DecoderModel:
         self.head: LinearWeight | None = None
         self.dtype = self.device = None
         self._max_positions = "?"  # not asked yet
+        self.has_runner = False  # set by the first ``ModelRunner`` made for it
         # what every entry of the run order keeps in the cache
         self.cache_needs = [self.layers[c.layer].cache_need() if c.cache_from is None else None for c in spec.run_order]
         # the residual stream between the blocks: one tensor in the model's precision, or ``spec.streams`` copies in 32-bit
@@ -103,7 +104,7 @@ class DecoderModel:
         """Check the source against what the model wants (one error that lists everything wrong), then read
         each tensor once.  A head that is absent is the embedding table if the configuration ties them
         (reference: model/loader.py:62-70).  ``layouts``: "both" keeps every matrix in two layouts
-        (``parts.linear.LAYOUTS``), "tiled" only in the re-laid one, "auto" chooses by the memory that is free."""
+        (``parts.linear.LAYOUTS``), "tiled" only in one (in bfloat16 the re-laid one), "auto" chooses by the memory that is free."""
         spec = self.spec
         full = self.wanted()
         wanted = {k: v[0] for k, v in full.items()}
@@ -111,15 +112,16 @@ class DecoderModel:
         self.dtype, self.device = dtype, torch.device(device)
         if layouts != "auto" and layouts not in LAYOUTS:
             raise ValueError(f"layouts={layouts!r}: use 'auto', 'both' or 'tiled'")
-        if layouts == "auto":
+        # (of a float32 matrix the second copy only makes products of many rows faster: asked for or not, it is kept where there is room)
+        if layouts == "auto" or (layouts == "both" and dtype == torch.float32 and self.device.type == "cuda"):
             size = torch.finfo(dtype).bits // 8
             linear = sum(size * math.prod(d for d in shape if d is not None) for name, (shape, role) in full.items()
                          if role == "linear" and name != spec.head_name)
             free = torch.cuda.mem_get_info(self.device)[0]
             layouts = "both" if 2.2 * linear + size * 2 * spec.vocab_size * spec.hidden < 0.8 * free else "tiled"
-            if layouts == "tiled" and dtype == torch.bfloat16:
-                print(f"[nanospec_amd] {linear / 2**30:.0f} GiB of matrices, {free / 2**30:.0f} GiB free: keeping one layout; "
-                      "steps of many tokens copy matrices into plain rows first and are slower", file=sys.stderr, flush=True)
+            if layouts == "tiled":
+                slower = "copy matrices into plain rows first and are slower" if dtype == torch.bfloat16 else "run on the 32-bit matrix instructions and take twice as long"
+                print(f"[nanospec_amd] {linear / 2**30:.0f} GiB of matrices, {free / 2**30:.0f} GiB free: keeping one layout; steps of many tokens {slower}", file=sys.stderr, flush=True)
         self.layouts = layouts
         get = source.get
         self.embed = get(spec.embed_name).to(device=device, dtype=dtype).contiguous()
@@ -146,6 +148,22 @@ class DecoderModel:
         # matrices, random draws) is finished before anyone can read it
         torch.cuda.synchronize(self.device)
         return self
+
+    def give_back_second_copies(self) -> bool:
+        """For whoever needs the memory (``cache.storage``): the second copies of float32 matrices, which only make products of many rows faster, are given back.  Not once a runner has been made for
+        the model: a step under way or captured may read them."""
+        if self.has_runner:
+            return False
+        holders = list(second_copies(self))
+        if holders:
+            torch.cuda.synchronize(self.device)
+            count = sum(h._split.parts.numel() * 2 for h in holders)
+            for holder in holders:
+                holder._split = None
+            torch.cuda.empty_cache()
+            print(f"[nanospec_amd] {count / 2**30:.1f} GiB of second copies of float32 matrices given back for keys and values; steps of many tokens run on the 32-bit matrix instructions and take twice "
+                  "as long", file=sys.stderr, flush=True)
+        return bool(holders)
 
     # ------------------------------------------------------------------ positions
 

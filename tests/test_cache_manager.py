@@ -147,3 +147,31 @@ def test_freed_pages_land_scattered():
     t = m.get("probe").tables[0]
     assert any(b != a + 1 for a, b in zip(t, t[1:])), t
     m.check()
+
+
+@pytest.mark.parametrize("fails,gives", [(0, True), (1, True), (3, True), (9, True), (1, False)])
+def test_a_storage_that_does_not_fit_asks_the_model_for_room(fails, gives, monkeypatch):
+    """Pages that do not fit beside what a model keeps only to be faster: that is given back and they are asked for again, once."""
+    import torch
+    from types import SimpleNamespace
+
+    from nanospec_amd.cache.storage import CacheStorage
+    from nanospec_amd.parts.needs import PagedNeed
+
+    need = PagedNeed(2, 16)
+    given, made, zeros = [], [], torch.zeros
+
+    def short(*shape, **kw):
+        made.append(shape)
+        if len(made) == fails or (not gives and given):
+            raise torch.OutOfMemoryError("no room")
+        return zeros(*shape, **kw)
+
+    model = SimpleNamespace(cache_needs=[need], spec=SimpleNamespace(run_order=[SimpleNamespace(cache_from=None)]), give_back_second_copies=lambda: given.append(len(made)))
+    monkeypatch.setattr(torch, "zeros", short)
+    if not gives:
+        with pytest.raises(torch.OutOfMemoryError):
+            CacheStorage(model, [4], 8, 2, torch.float32, "cpu")
+        return
+    storage = CacheStorage(model, [4], 8, 2, torch.float32, "cpu")
+    assert given == ([fails] if fails in (1, 2) else []) and storage.k[0].shape == (1, 4, 2, 8, 16) and storage.views[0].v.shape == (4, 2, 16, 8)

@@ -369,6 +369,30 @@ def test_linear_weight_f32_of_many_rows(keep_plain):
     assert float((y - ref).norm() / ref.norm()) <= (3e-7 if keep_plain else 6e-7)  # 1.8e-7 and 4.1e-7 measured at K 2,048
 
 
+def test_second_copies_of_float32_matrices_are_given_back():
+    """Those of a model's parts, wherever they are kept, until a runner has been made for it; the products then run on the 32-bit instruction."""
+    from types import SimpleNamespace
+
+    from nanospec_amd.engine.arena import Arena
+    from nanospec_amd.parts.linear import GatedWeights, LinearWeight, second_copies
+    from nanospec_amd.parts.model import DecoderModel
+
+    ops = _ops()
+    torch.manual_seed(9)
+    w, x = torch.randn(2048, 2048, device=DEV), torch.randn(600, 2048, device=DEV)
+    linear, gated, small, tiled = LinearWeight(w), GatedWeights(w[:1024].contiguous(), w[1024:].contiguous()), LinearWeight(w[:64, :512].contiguous()), LinearWeight(w, keep_plain=False)
+    model = DecoderModel.__new__(DecoderModel)
+    model.device, model.has_runner, model.layers, model.other = torch.device(DEV), True, [{"first": (linear, small)}, tiled], gated
+    ctx = SimpleNamespace(arena=Arena(x.device), captured=False)
+    before = linear(x, arena=ctx.arena)
+    assert set(second_copies(model)) == {linear, gated} and not model.give_back_second_copies() and linear._split is not None
+    model.has_runner = False
+    assert model.give_back_second_copies() and not list(second_copies(model)) and not model.give_back_second_copies()
+    after = linear(x, arena=ctx.arena)
+    assert torch.equal(after, ops.linear_generic(x, w)) and not torch.equal(after, before)
+    gated(ctx, x, out=torch.empty(600, 1024, device=DEV))
+
+
 @pytest.mark.parametrize("shapes", [[(1,)], [(3, 5), (1,), (7,)], [(16, 128, 257), (2, 2048), (1,), (13,)], [(9,), (8 * 257,), (65, 1023), (4, 3)]])
 def test_slot_tensors(shapes):
     """One slot of every tensor is cleared and nothing beside it: slots of single words, of odd numbers of values, of many blocks."""

@@ -47,8 +47,8 @@ __global__ void conv_silu_kernel(float* __restrict__ out, T* __restrict__ copy, 
 
 // The same for four neighbouring channels a thread, with 16-byte accesses to taps, carried inputs and results, for the
 // usual numbers of taps (so that the taps are registers) and channels that are a multiple of four.  A thread takes STRIP tokens one after the other: taps are
-// 64 bytes a thread and an input is read by K tokens, for 8 bytes of new input and 16 of result.  UNITS: the first ``vectors`` runs of 4 LANES channels then become unit
-// vectors, as delta_prep_kernel makes them, while their sums of squares are at hand (C a multiple of 4 LANES): as a kernel of its own that reads and writes them again.
+// 64 bytes a thread and an input is read by K tokens, for 8 bytes of new input and 16 of result.  The first ``units.vectors`` runs of 4 ``units.lanes`` channels (no more
+// than C) then become unit vectors, as delta_prep_kernel makes them, while their sums of squares are at hand: a kernel of its own reads and writes them again.
 // Bound by the results' bytes: 2,048 tokens of 6,144 channels, 4 taps, bfloat16, a token a thread 35.0 / 27.2 us (alone / beside two
 // others) and the unit vectors and decays behind it 38.3 / 31.8, both in a row 69.1 / 57.4; so 30.6 / 19.8 and (decays alone) 18.7 / 14.3, 46.3 / 31.5.
 template <int LANES>

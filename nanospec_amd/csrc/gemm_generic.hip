@@ -70,6 +70,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(OutT* __restrict__ ou
 // a kernel of its own, and the addresses, which the scalar unit holds but for the lane's (in vector registers they would not leave room for 8 rows).  us, alone and a call beside two
 // others, with sums through LDS's crossbar and 1, 2, 4 or 8 rows of x, and now: five rows, N 16,384, K 2,048 32.5 / 27.0 and 24.9 / 20.8 (5.4 TB/s, 6.5); N 2,048, K 8,192 19.0 /
 // 13.6 and 16.0 / 12.8; N 2,048, K 2,048 8.7 / 6.2 and 7.2 / 5.4; N 128,256, K 2,048 212 / 215 and 158 / 158 (6.7 TB/s); eight rows 215 / 218 and 173 / 176, one row 170 / 165 and 156 / 152.
+// (Captured steps run 1, 2, 4 or 8 rows; the other numbers are those of steps outside graphs.)
 #define ROWS_M 8
 #define ROWS_N 8
 

@@ -85,9 +85,9 @@ def test_linear_generic(dtype, m, n, k):
         torch.testing.assert_close(one, out[:1], rtol=1e-5, atol=1e-4)
 
 
-@pytest.mark.parametrize("m", [1, 2, 3, 8, 9, 16, 17, 33, 515])
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 33, 515])
 @pytest.mark.parametrize("n,k", [(1, 4), (7, 2052), (33, 60), (130, 64), (700, 516), (4100, 576), (4130, 100), (65, 2500),
-                                 (250, 516), (8210, 252)])
+                                 (250, 516), (8210, 252), (4100, 2048), (4099, 1024), (4099, 1028)])
 def test_linear_f32_forms(m, n, k):
     """32-bit products of few and of many rows at the edges of their tiles (8 rows or columns, 16, 32, 64), of a stage of 64 k and of
     the stages that are in flight (three or eight, before and after a place in LDS is used again); rows of x and of the result with a stride of their own."""
@@ -275,15 +275,14 @@ def test_keys_and_values_in_pieces_of_many_tokens(dtype, n, kind, H, G, D, E, pa
 
 @pytest.mark.parametrize("spread", [12, 24])
 def test_linear_split_of_wide_rows(spread):
-    """Values over many powers of two within a block of x and a row of w: the parts of the small ones lie below the float16 numbers of full precision, not below all of them."""
+    """Values over many powers of two within a block of x and a row of w: no more is lost than of values of one size."""
     ops = _ops()
     torch.manual_seed(spread)
     small = torch.randint(-spread, 1, (2, 300, 1024)).float().exp2().to(DEV)
     x, w = torch.randn(100, 1024, device=DEV) * small[0, :100], torch.randn(300, 1024, device=DEV) * small[1]
     a, b = x.cpu().double(), w.cpu().double()
-    largest = a.abs().view(100, 32, 32).amax(2).repeat_interleave(32, 1)
-    # as above, and a part that is rounded to a multiple of 2^-24 where the largest value of the block or row is at least 2^14
-    bound = (2 + 2 + 4 + 12 + 32 + 1) * 2.0**-24 * (a.abs() @ b.abs().T) + 2.0**-39 * (largest @ b.abs().T + a.abs() @ b.abs().amax(1, keepdim=True).expand(300, 1024).T)
+    # as above: the second part has the float16 range to itself, and rows that it still does not hold are the 32-bit instruction's (four chains of 64 sums)
+    bound = (2 + 2 + 4 + 12 + 32 + 1) * 2.0**-24 * (a.abs() @ b.abs().T)
     assert bool(((ops.linear_split(x, w, 64, 1).cpu().double() - a @ b.T).abs() <= bound).all())
 
 
@@ -311,6 +310,27 @@ def test_linear_split_of_values_far_apart(factor, kind, ranges):
     assert far(y) <= max(far(ops.linear_generic(x, w)), limit)
     if factor >= 1e12 and kind != "sparse":  # every row: the 32-bit instruction's sums
         assert torch.equal(y, ops.linear_generic(x, w))
+
+
+@pytest.mark.parametrize("ranges", [1, 2])
+@pytest.mark.parametrize("m", [4097, 4200])
+def test_linear_split_in_portions(m, ranges):
+    """More rows than a portion, the last one short: rows of x and of the result with a stride of their own, a row of the 32-bit instruction in either portion."""
+    ops = _ops()
+    torch.manual_seed(m)
+    wide, w, out = torch.randn(m, 140, device=DEV), torch.randn(70, 128, device=DEV), torch.full((m, 77), 7.0, device=DEV)
+    x = wide[:, 8:136]
+    x[[5, 4096], 3] = math.inf
+    split = ops.SplitWeight(w)
+    ops.linear_split(x, w, 128, ranges, out=out[:, :70], split=split)
+    parts = torch.cat([ops.linear_split(p, w, 64, ranges, split=split) for p in (x[:4096], x[4096:])])
+    assert torch.equal(out[:, :70], parts) and bool((out[:, 70:] == 7).all())
+    a, b, fine = x.cpu().double(), w.cpu().double(), torch.isfinite(x).all(1).cpu()
+    bound = (2 + 2 + 4 + 12 + 4 + ranges) * 2.0**-24 * (a.abs() @ b.abs().T)  # (as in test_linear_split)
+    assert ((parts.cpu().double() - a @ b.T).abs()[fine] <= bound[fine]).all() and torch.equal(parts[[5, 4096]], ops.linear_generic(x, w)[[5, 4096]])
+    read = torch.tensor([4099], dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.linear_split(x, w, 128, ranges, split=split, read_rows=read)[:4099], parts[:4099])
+    assert bool((ops.linear_split(x, w, 128, ranges, split=split, read_rows=read)[4099:] == 0).all())
 
 
 @pytest.mark.parametrize("n,k", [(4096, 1024), (2056, 2080), (130, 4128), (15360, 1056)])

@@ -154,25 +154,36 @@ __global__ __launch_bounds__(256) void split_scales_kernel(float* __restrict__ s
   if (lane == 0) scales[n] = split_scale(largest);
 }
 
-// The blocks of 16 rows that have a row to mend: list[0] how many, then for each its number and the rows as bits, from the counts of ``lost`` [blocks][groups].  By all threads of a workgroup.
+// The blocks of 16 rows that have a row to mend: list[0] how many, then for each its number and the rows as bits, from the counts of ``lost`` [blocks][groups].  By all threads of a workgroup (1,024 at most).
+// In the order of the blocks: every workgroup of split_mend_kernel makes the list for itself and takes its items by their places there.
 __device__ __forceinline__ void list_lost(int* list, const unsigned* lost, int blocks, int groups) {
+  __shared__ int found[16];  // by each wave
+  const int lane = threadIdx.x % NS_WAVE, wave = threadIdx.x / NS_WAVE;
   if (threadIdx.x == 0) list[0] = 0;
   unsigned any = 0;
   for (size_t i = threadIdx.x; i < (size_t)blocks * groups; i += blockDim.x) any |= lost[i];
   if (!__syncthreads_or(any)) return;  // (all of the workgroup)
-  for (int b = threadIdx.x; b < blocks; b += blockDim.x) {
+  int count = 0;
+  for (int from = 0; from < blocks; from += blockDim.x) {
+    const int b = from + threadIdx.x;
     unsigned more = 0, once = 0;  // (bits 2 r: rows with two, rows with one so far)
-    for (int i = 0; i < groups; ++i) {
+    for (int i = 0; b < blocks && i < groups; ++i) {
       const unsigned word = lost[(size_t)b * groups + i], one = word & 0x55555555u, two = word >> 1 & 0x55555555u;
       more |= two | (once & one), once |= one;
     }
+    const unsigned long long with = __ballot(more != 0);
+    if (lane == 0) found[wave] = __popcll(with);
+    __syncthreads();
+    int at = count + __popcll(with & ((1ull << lane) - 1));
+    for (int i = 0; i < (int)blockDim.x / NS_WAVE; ++i) at += i < wave ? found[i] : 0, count += found[i];
     if (more) {
-      const int at = atomicAdd(list, 1);
       int rows = 0;
       for (int r = 0; r < 16; ++r) rows |= (int)(more >> 2 * r & 1) << r;
       list[1 + 2 * at] = b, list[2 + 2 * at] = rows;
     }
+    __syncthreads();
   }
+  if (threadIdx.x == 0) list[0] = count;
   __syncthreads();
 }
 __global__ __launch_bounds__(1024) void split_list_kernel(int* __restrict__ list, const unsigned* __restrict__ lost, int blocks, int groups) { list_lost(list, lost, blocks, groups); }

@@ -333,6 +333,22 @@ def test_linear_split_in_portions(m, ranges):
     assert bool((ops.linear_split(x, w, 128, ranges, split=split, read_rows=read)[4099:] == 0).all())
 
 
+@pytest.mark.parametrize("n", [40, 2072])
+@pytest.mark.parametrize("blocks", [[0, 70, 255], [3, 64, 65, 127, 128, 191, 254], list(range(1, 256, 3)), list(range(256))])
+def test_linear_split_mends_blocks_far_apart(blocks, n):
+    """Rows for the 32-bit instruction in blocks that different waves of a workgroup find, one block at a time and four: all of them are its results, the others' are theirs."""
+    ops = _ops()
+    torch.manual_seed(n + len(blocks))
+    x, w = torch.randn(4096, 128, device=DEV), torch.randn(n, 128, device=DEV)
+    split = ops.SplitWeight(w)
+    want = ops.linear_split(x, w, 64, 1, split=split)
+    rows = torch.tensor([16 * b + b % 16 for b in blocks], device=DEV)
+    x[rows, ::5] *= 1e12
+    want[rows] = ops.linear_generic(x, w)[rows]
+    for _ in range(3):
+        assert torch.equal(ops.linear_split(x, w, 64, 1, split=split), want)
+
+
 @pytest.mark.parametrize("n,k", [(4096, 1024), (2056, 2080), (130, 4128), (15360, 1056)])
 def test_linear_split_is_the_same_whatever_the_rows_beside(n, k):
     """Any tile, segments by one workgroup or by one each, any rows beside and any place among them: the same results bit by bit."""

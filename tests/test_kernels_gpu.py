@@ -333,6 +333,24 @@ def test_linear_split_in_portions(m, ranges):
     assert bool((ops.linear_split(x, w, 128, ranges, split=split, read_rows=read)[4099:] == 0).all())
 
 
+@pytest.mark.parametrize("blocks,kept", [(0, True), (1, True), (8, True), (9, False), (65, False)])
+def test_split_weight_of_values_far_apart(blocks, kept):
+    """A matrix of which the parts do not hold too many rows has no second copy: its products stay the 32-bit instruction's."""
+    from nanospec_amd.engine.arena import Arena
+    from nanospec_amd.parts.linear import LinearWeight
+
+    ops = _ops()
+    torch.manual_seed(blocks)
+    w, x = torch.randn(1040 - 5, 4096, device=DEV), torch.randn(600, 4096, device=DEV)
+    assert ops.split_plan(600, 1035, 4096, ops.compute_units(x.device)) is not None
+    w[0 : 16 * blocks : 16, ::5] *= 1e-12
+    weight = LinearWeight(w)
+    assert (weight._split is not None) == kept
+    y, plain = weight(x, arena=Arena(x.device)), ops.linear_generic(x, w)
+    lost = list(range(0, 16 * blocks, 16)) if kept else slice(None)
+    assert torch.equal(y[:, lost], plain[:, lost])
+
+
 @pytest.mark.parametrize("n", [40, 2072])
 @pytest.mark.parametrize("blocks", [[0, 70, 255], [3, 64, 65, 127, 128, 191, 254], list(range(1, 256, 3)), list(range(256))])
 def test_linear_split_mends_blocks_far_apart(blocks, n):

@@ -26,6 +26,7 @@
 // Bound by the power of the matrix unit: at the last size it works for 69% of the cycles and the clock sinks to 1.4 GHz.
 #include "common.h"
 #include "lds_loads.h"
+#include <type_traits>
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((__vector_size__(4 * sizeof(float))));
@@ -244,9 +245,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 acc[MI][NJ], total[MI][NJ];
   int to = 0;
-  auto stage = [&](int at, int kb) {
+  // ``behind``: loads of the next stage, which are on their way behind this one's.  The last stage but one fetches its next but one for nothing, and the compiler drops what goes to registers of that: the last waits until
+  // no more than the others are left.
+  typedef std::integral_constant<int, LOADS> Whole;
+  typedef std::integral_constant<int, XPARTS + 1> ToLds;
+  auto stage = [&](int at, int kb, auto behind) {
     // this stage has come, and every wave is done with the one before it, whose place the next but one is given (behind the last stage: that once more, not used)
-    TILE_WAIT_LOADS(LOADS);
+    TILE_WAIT_LOADS(decltype(behind)::value);
     TILE_BARRIER();
     load((at + 2) % SPLIT_STAGES, min(kb + 2, to - 1));
     __builtin_amdgcn_sched_barrier(0);
@@ -297,10 +302,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       for (int j = 0; j < NJ; ++j) acc[i][j] = zero;
     if (s) TILE_BARRIER();  // (every wave is done with the segment before)
     load(0, kb);
+    __builtin_amdgcn_sched_barrier(0);  // (in this order: the waits count loads)
     load(1, min(kb + 1, to - 1));
-    for (; kb + 2 < to; kb += 3) stage(0, kb), stage(1, kb + 1), stage(2, kb + 2);
-    if (kb < to) stage(0, kb);
-    if (kb + 1 < to) stage(1, kb + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    for (; kb + 2 < to; kb += 3) stage(0, kb, Whole()), stage(1, kb + 1, Whole()), stage(2, kb + 2, Whole());
+    if (kb < to) stage(0, kb, Whole());
+    if (kb + 1 < to) stage(1, kb + 1, ToLds());
     TILE_WAIT_LOADS(0);  // (what was fetched again behind the last stage must not come into another stage's LDS, or another workgroup's)
     if (SUMMED) {
 #pragma unroll

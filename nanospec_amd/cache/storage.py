@@ -72,7 +72,7 @@ class CacheStorage:
             self.__dict__.clear()
             give_back()
             self._allocate(model, num_pages, page_size, num_slots, dtype, device)
-        elif torch.device(device).type == "cuda":
+        elif dtype == torch.float32 and torch.device(device).type == "cuda":  # (no other models have such copies)
             free, total = torch.cuda.mem_get_info(device)
             if free + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device) < STEPS_SHARE * total:
                 give_back()

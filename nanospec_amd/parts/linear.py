@@ -99,18 +99,12 @@ def library_product(x: torch.Tensor, w_t: torch.Tensor, out: torch.Tensor | None
     return y if act is None else ops.activation(y, act)
 
 
-SPLIT_MOST_LOST = 0.125  # of the rows of a matrix, by 16, whose values may lie too far apart for the parts
-
-
 def split_weight(w: torch.Tensor) -> "ops.SplitWeight | None":
     """The second copy of a float32 matrix, for ``product_f32``, or None where that has no use for it."""
     n, k = w.shape
     if w.dtype != torch.float32 or not w.is_cuda or not ops.SPLIT_MIN_K <= k < 1 << 19 or k % ops.SPLIT_K_MULTIPLE or n > 1 << 19 or not ops.split_takes(w[:1], w):
         return None
-    split = ops.SplitWeight(w)
-    # Each 16 rows that the parts do not hold are made by the 32-bit instruction behind every product, which is slower than the 32-bit product of all alone where they are many: us, that product and the
-    # split one with none, an eighth and a quarter of them so, 832 rows, N = K = 2,048 62 and 45, 68, 67, N 2,048, K 8,192 244 and 123, 217, 225, N 16,384, K 2,048 546 and 204, 302, 376; 128 rows of the last 68 and 41, 66, 67
-    return split if int(split.lost[0]) <= SPLIT_MOST_LOST * -(-n // 16) else None
+    return ops.SplitWeight(w)
 
 
 def product_f32(x: torch.Tensor, w: torch.Tensor, split: "ops.SplitWeight | None", out: torch.Tensor | None, arena) -> torch.Tensor:
@@ -136,6 +130,20 @@ def second_copies(part, seen: set | None = None):
     inside = part if isinstance(part, (list, tuple)) else part.values() if isinstance(part, dict) else vars(part).values() if type(part).__module__.startswith(__package__) else ()
     for one in inside:
         yield from second_copies(one, seen)
+
+
+SPLIT_MOST_LOST = 0.125  # of the rows of a matrix, by 16, whose values may lie too far apart for the parts
+
+
+def drop_copies_of_little_use(part) -> None:
+    """Second copies within ``part`` that do not stand for too many of the matrix's rows are let go: each 16 such rows are made by the 32-bit instruction behind every product, which is slower than the 32-bit
+    product of all alone where they are many.  us, that product and the split one with none, an eighth and a quarter of them so: 832 rows, N = K = 2,048 62 and 45, 68, 67, N 2,048, K 8,192 244 and 123, 217, 225, N 16,384, K 2,048
+    546 and 204, 302, 376; 128 rows of the last 68 and 41, 66, 67.  (One trip to the GPU for all of them: a matrix by itself as it is split costs a model of 32 matrices a millisecond of its load.)"""
+    holders = list(second_copies(part))
+    if holders:
+        for holder, lost in zip(holders, torch.stack([h._split.lost[0] for h in holders]).tolist()):
+            if lost > SPLIT_MOST_LOST * -(-holder._split.n // 16):
+                holder._split = None
 
 
 class IntoResidual:

@@ -11,7 +11,7 @@ import torch
 from ..kernels import ops
 from ..weights import source as wsource
 from . import registry
-from .linear import LAYOUTS, LinearWeight, second_copies
+from .linear import LAYOUTS, LinearWeight, drop_copies_of_little_use, second_copies
 from .needs import PagedNeed, StateNeed
 
 
@@ -144,6 +144,7 @@ class DecoderModel:
         if spec.streams:
             self._ones = torch.ones(spec.streams, dtype=torch.float32, device=device)
             self._eye = torch.eye(spec.streams, dtype=torch.float32, device=device)
+        drop_copies_of_little_use(self)
         # whoever runs the model works on a stream of their own: everything that loading enqueued (copies, re-laying of
         # matrices, random draws) is finished before anyone can read it
         torch.cuda.synchronize(self.device)

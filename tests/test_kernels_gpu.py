@@ -335,17 +335,18 @@ def test_linear_split_in_portions(m, ranges):
 
 @pytest.mark.parametrize("blocks,kept", [(0, True), (1, True), (8, True), (9, False), (65, False)])
 def test_split_weight_of_values_far_apart(blocks, kept):
-    """A matrix of which the parts do not hold too many rows has no second copy: its products stay the 32-bit instruction's."""
+    """A matrix of which the parts do not hold too many rows keeps no second copy: its products stay the 32-bit instruction's."""
     from nanospec_amd.engine.arena import Arena
-    from nanospec_amd.parts.linear import LinearWeight
+    from nanospec_amd.parts.linear import LinearWeight, drop_copies_of_little_use
 
     ops = _ops()
     torch.manual_seed(blocks)
     w, x = torch.randn(1040 - 5, 4096, device=DEV), torch.randn(600, 4096, device=DEV)
     assert ops.split_plan(600, 1035, 4096, ops.compute_units(x.device)) is not None
     w[0 : 16 * blocks : 16, ::5] *= 1e-12
-    weight = LinearWeight(w)
-    assert (weight._split is not None) == kept
+    weight, other = LinearWeight(w), LinearWeight(torch.randn(1035, 4096, device=DEV))
+    drop_copies_of_little_use([weight, other])
+    assert (weight._split is not None) == kept and other._split is not None
     y, plain = weight(x, arena=Arena(x.device)), ops.linear_generic(x, w)
     lost = list(range(0, 16 * blocks, 16)) if kept else slice(None)
     assert torch.equal(y[:, lost], plain[:, lost])
